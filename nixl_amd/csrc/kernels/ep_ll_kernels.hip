@@ -23,7 +23,10 @@
 //                          also turns expert e's bits into layout_range, recv_count and the
 //                          statistics.
 //   3. ll_scales_kernel    fp8 only: moves the per-token scales into their column-major place
-//                          per expert, 64 rows at a time through LDS.
+//                          per expert, 64 rows at a time through LDS.  With few scales step 2
+//                          writes them itself (kIsolatedScaleWords).
+// A small call (kDirectSelections) is one launch, ll_direct_kernel, which counts rows from the
+// selection itself.
 // Step 1 moves 0.3 MB, step 3 the scales (twice 16 MB at 32 x 128 x 7168, top-8); step 2 moves the payload.
 // The order this produces is the canonical one among those the reference's atomics allow:
 // segments by source rank ascending, tokens ascending inside a segment.
@@ -274,7 +277,9 @@ struct DispatchArgs {
     LlDims d;
     int Wr;
     int round_scale;
-    int parts; // workgroups per token; each covers blockDim.x of the token's H/16 lanes
+    int parts; // workgroups per token; each covers blockDim.x of the token's lanes
+    void *recv_scales; // where the row kernel writes the scales itself, with use_ue8m0
+    int use_ue8m0;
 };
 
 // A call in which some token names an expert twice: one bit per (expert, token) cannot carry
@@ -362,10 +367,74 @@ ll_meta_kernel(DispatchArgs a) {
     if (e == 0) reduce_status(a, lane);
 }
 
-// grid = R*T*parts workgroups.  A token's row is H/16 "lanes" of 16 consecutive channels
-// (32 bytes of bf16, 16 bytes of fp8), so a 128-channel scale group is 8 neighbouring
-// lanes; a workgroup covers blockDim.x of them (a multiple of 64).
+// Lanes of a token's row, what a lane holds of it, and its fp8 form.
 template<bool FP8>
+__device__ __host__ __forceinline__ int
+row_lanes(int H) {
+    return FP8 ? H / 16 : H / 8;
+}
+
+template<bool FP8>
+__device__ __forceinline__ void
+load_row(const uint16_t *row, int lane, uint4 &raw0, uint4 &raw1) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(row) + lane * (FP8 ? 2 : 1);
+    raw0 = ld16_nt(src);
+    if constexpr (FP8) raw1 = ld16_nt(src + 1);
+}
+
+// 16 channels to 16 fp8 codes; the 8 lanes of one 128-channel group share the scale.
+__device__ __forceinline__ uint4
+quantise_group(const uint4 &raw0, const uint4 &raw1, bool round_scale, float &scale_inv) {
+    const uint32_t w[8] = {raw0.x, raw0.y, raw0.z, raw0.w, raw1.x, raw1.y, raw1.z, raw1.w};
+    float v[16];
+    float amax = 1e-4f; // floor of the maximum, kernels/nixl_ep_ll.cu:155
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        v[2 * j] = bf16_lo_to_f32(w[j]);
+        v[2 * j + 1] = bf16_hi_to_f32(w[j]);
+        amax = fmaxf(amax, fmaxf(fabsf(v[2 * j]), fabsf(v[2 * j + 1])));
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 1));
+    amax = fmaxf(amax, __shfl_xor(amax, 2));
+    amax = fmaxf(amax, __shfl_xor(amax, 4));
+    float scale;
+    fp8_scales(amax, round_scale, scale, scale_inv);
+    uint32_t out[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        out[j] = e4m3_pack4(v[4 * j] * scale, v[4 * j + 1] * scale, v[4 * j + 2] * scale, v[4 * j + 3] * scale);
+    return make_uint4(out[0], out[1], out[2], out[3]);
+}
+
+// What a token's scale becomes in packed_recv_x_scales: the float's bits, or (UE8M0) the exponent
+// bytes of four neighbouring groups in one word, complete in the first group's lanes.
+__device__ __forceinline__ uint32_t
+scale_word(float scale_inv, bool use_ue8m0) {
+    uint32_t word = __float_as_uint(scale_inv);
+    if (use_ue8m0) {
+        word = (word >> 23) & 0xffu;
+        word |= __shfl_down(word, 8) << 8;
+        word |= __shfl_down(word, 16) << 16;
+    }
+    return word;
+}
+
+// Writes a lane's word to its column of `row` = e * N + slot; lanes that hold no word do nothing.
+__device__ __forceinline__ void
+store_scale(void *recv_scales, const LlDims &d, bool use_ue8m0, int row, int lane, uint32_t word) {
+    const int shift = use_ue8m0 ? 5 : 3; // lanes per word
+    if (lane & ((1 << shift) - 1)) return;
+    const int e = row / d.N, columns = d.H / 16 >> shift;
+    static_cast<uint32_t *>(recv_scales)[(static_cast<size_t>(e) * columns + (lane >> shift)) * d.N + (row - e * d.N)] = word;
+}
+
+// grid = R*T*parts workgroups.  A lane stores 16 bytes of every row, so that the stores of a
+// wave are whole lines: a row is H/16 lanes of 16 channels as fp8 (a 128-channel scale group is
+// 8 neighbouring lanes) and H/8 lanes of 8 channels as bf16; a workgroup covers blockDim.x of
+// them (a multiple of 64).  (With 16 channels a lane for bf16 too, every store instruction left
+// half of each line to the next one: 976 tokens x 2560, top-6, took 31 us instead of 7.)
+// SCALES: the scales are written here (kIsolatedScaleWords), not by ll_scales_kernel.
+template<bool FP8, bool SCALES>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8)))
 ll_dispatch_kernel(DispatchArgs a) {
     const LlDims d = a.d;
@@ -380,18 +449,15 @@ ll_dispatch_kernel(DispatchArgs a) {
     const int sel = (wlane < d.K && t < nt) ? a.topk_idx[(static_cast<size_t>(r) * d.T + t) * d.K + wlane] : -1;
     // The row is requested next so that it travels while the rows are being located.
     const int lane = part * blockDim.x + tid; // lane of the token's row
-    const bool active = lane < d.H / 16 && t < nt;
+    const bool active = lane < row_lanes<FP8>(d.H) && t < nt;
     uint4 raw0 = make_uint4(0, 0, 0, 0), raw1 = raw0;
-    if (active) {
-        const uint4 *src = reinterpret_cast<const uint4 *>(a.x + (static_cast<size_t>(r) * d.T + t) * d.H) + lane * 2;
-        raw0 = ld16_nt(src);
-        raw1 = ld16_nt(src + 1);
-    }
+    if (active) load_row<FP8>(a.x + (static_cast<size_t>(r) * d.T + t) * d.H, lane, raw0, raw1);
 
-    // Receive-side metadata: the workgroup of token i derives it for experts i, i + R*T, ...
+    // Receive-side metadata: the waves of token i, last one first, derive it for experts
+    // i, i + R*T, ... (the first waves are busy locating rows).
     const bool repeats = call_has_repeats(a);
-    if (part == 0 && wave == n_waves - 1)
-        for (int e = token; e < d.E; e += d.R * d.T) {
+    if (part == 0)
+        for (int e = token + (n_waves - 1 - wave) * d.R * d.T; e < d.E; e += n_waves * d.R * d.T) {
             if (repeats)
                 expert_meta<true>(a, e, wlane);
             else
@@ -437,31 +503,14 @@ ll_dispatch_kernel(DispatchArgs a) {
         if (((own >> (t & 63)) & 1ull) && cnt < d.N) row = e * d.N + cnt;
         if (q0 == 0) row_of_k[k] = row;
     }
-    uint4 q = make_uint4(0, 0, 0, 0);
+    float scale_inv = 0.f;
     if constexpr (FP8) {
-        const uint32_t w[8] = {raw0.x, raw0.y, raw0.z, raw0.w, raw1.x, raw1.y, raw1.z, raw1.w};
-        float v[16];
-        float amax = 1e-4f; // floor of the maximum, kernels/nixl_ep_ll.cu:155
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            v[2 * j] = bf16_lo_to_f32(w[j]);
-            v[2 * j + 1] = bf16_hi_to_f32(w[j]);
-            amax = fmaxf(amax, fmaxf(fabsf(v[2 * j]), fabsf(v[2 * j + 1])));
-        }
-        // maximum over the 8 lanes of one 128-channel group
-        amax = fmaxf(amax, __shfl_xor(amax, 1));
-        amax = fmaxf(amax, __shfl_xor(amax, 2));
-        amax = fmaxf(amax, __shfl_xor(amax, 4));
-        float scale, scale_inv;
-        fp8_scales(amax, a.round_scale != 0, scale, scale_inv);
-        if (active && (lane & 7) == 0)
+        raw0 = quantise_group(raw0, raw1, a.round_scale != 0, scale_inv);
+        if (!SCALES && active && (lane & 7) == 0)
             a.token_scales[(static_cast<size_t>(r) * d.T + t) * (d.H / 128) + (lane >> 3)] = scale_inv;
-        uint32_t out[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            out[j] = e4m3_pack4(v[4 * j] * scale, v[4 * j + 1] * scale, v[4 * j + 2] * scale, v[4 * j + 3] * scale);
-        q = make_uint4(out[0], out[1], out[2], out[3]);
     }
+    [[maybe_unused]] uint32_t word = 0;
+    if constexpr (SCALES) word = scale_word(scale_inv, a.use_ue8m0 != 0);
     __syncthreads();
     // Publish the rows (combine reads them back as its row map).
     if (part == 0 && tid < d.K && a.rows_out) a.rows_out[(static_cast<size_t>(r) * d.T + t) * d.K + tid] = row_of_k[tid];
@@ -470,16 +519,170 @@ ll_dispatch_kernel(DispatchArgs a) {
         const int row = row_of_k[k];
         if (row < 0) continue;
         if (lane == 0) a.src_info[row] = t;
-        if (!active) continue;
-        if constexpr (FP8) {
-            st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H) + lane, q);
-        } else {
-            uint4 *dst = reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * 2) + lane * 2;
-            st16_stream(dst, raw0);
-            st16_stream(dst + 1, raw1);
-        }
+        if (active) st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
+        if constexpr (SCALES)
+            if (active) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, row, lane, word);
     }
 }
+
+// ---- 2b. the whole dispatch in one launch, for small calls -----------------------------------------
+//
+// A decode step with few tokens is launches and dependent round trips, not bytes.  While all
+// selections of the world fit in a few KiB, a token's rows can be counted from topk_idx itself:
+// every workgroup scans the selections in front of its own (a ballot and a bit count per
+// selection it looks for), so nothing has to be prepared by a kernel before this one, a repeated
+// expert needs no special case (every selection counts), and the scales go straight to their
+// column-major places, since there are too few of them for the isolated words to matter.
+// The first workgroups of the grid derive the receive-side metadata from the same scan.
+struct DirectArgs {
+    uint8_t *recv_x;
+    void *recv_scales; // [E][G][N] float, or [E][G/4][N] words of four exponent bytes
+    int *src_info;
+    long long *layout_range;
+    int *recv_count;
+    int *stats;
+    const uint16_t *x;
+    const int32_t *topk_idx;
+    int *status; // workspace header
+    int *rows_out;
+    LlDims d;
+    int round_scale, use_ue8m0;
+    int parts; // workgroups per token
+    int meta_wgs; // workgroups at the front of the grid that derive the metadata of kDirectExperts experts each
+};
+
+constexpr int kDirectExperts = 16;
+constexpr int kDirectMaxRanks = 64;
+constexpr int kDirectMaxThreads = 512;
+
+// Experts e0 .. e0 + 15: counts and first rows per source rank; workgroup 0 also looks for
+// tokens that name an expert twice.
+__device__ __forceinline__ void
+direct_meta(const DirectArgs &a, int e0) {
+    __shared__ int hist[kDirectExperts][kDirectMaxRanks + 1];
+    __shared__ int begin[kDirectExperts][kDirectMaxRanks + 1];
+    const LlDims d = a.d;
+    const int tid = threadIdx.x, n_threads = blockDim.x, per_rank = d.T * d.K;
+    const int experts = min(kDirectExperts, d.E - e0);
+    for (int i = tid; i < kDirectExperts * (kDirectMaxRanks + 1); i += n_threads)
+        (&hist[0][0])[i] = 0;
+    __syncthreads();
+    for (int p = tid; p < d.R * per_rank; p += n_threads) {
+        const int e = a.topk_idx[p] - e0;
+        if (e >= 0 && e < experts) atomicAdd(&hist[e][p / per_rank], 1);
+    }
+    int repeat = 0;
+    if (e0 == 0)
+        for (int t = tid; t < d.R * d.T; t += n_threads) {
+            const int32_t *sel = a.topk_idx + static_cast<size_t>(t) * d.K;
+            for (int k = 1; k < d.K; ++k)
+                for (int j = 0; j < k; ++j)
+                    repeat |= sel[k] == sel[j] && sel[k] >= 0 && sel[k] < d.E;
+        }
+    repeat = __syncthreads_or(repeat);
+    if (e0 == 0 && tid == 0) a.status[0] = repeat ? NIXL_AMD_EP_STATUS_DUPLICATE_EXPERT : 0;
+    if (tid < experts) {
+        int run = 0;
+        for (int r = 0; r < d.R; ++r) {
+            begin[tid][r] = run;
+            run += hist[tid][r];
+        }
+        a.recv_count[e0 + tid] = run;
+        if (a.stats) a.stats[e0 + tid] += run;
+    }
+    __syncthreads();
+    for (int i = tid; i < experts * d.R; i += n_threads) {
+        const int e = i / d.R, r = i - e * d.R;
+        a.layout_range[static_cast<size_t>(e0) * d.R + i] =
+            static_cast<long long>(static_cast<unsigned>(hist[e][r])) | (static_cast<long long>(begin[e][r]) << 32);
+    }
+}
+
+// grid = meta_wgs + R*T*parts workgroups; KP: K rounded up to what the counting loop unrolls.
+template<bool FP8, int KP>
+__global__ void __launch_bounds__(kDirectMaxThreads)
+ll_direct_kernel(DirectArgs a) {
+    __shared__ int counted[kDirectMaxThreads / kWaveSize][KP];
+    __shared__ int row_of_k[KP];
+    if (static_cast<int>(blockIdx.x) < a.meta_wgs) {
+        direct_meta(a, blockIdx.x * kDirectExperts);
+        return;
+    }
+    const LlDims d = a.d;
+    const int tid = threadIdx.x, wlane = tid & (kWaveSize - 1), wave = tid / kWaveSize, n_waves = blockDim.x / kWaveSize;
+    const int wg = blockIdx.x - a.meta_wgs, token = wg / a.parts, part = wg % a.parts;
+    int sel = wlane < d.K ? a.topk_idx[static_cast<size_t>(token) * d.K + wlane] : -1;
+    const int lane = part * blockDim.x + tid; // lane of the token's row
+    const bool active = lane < row_lanes<FP8>(d.H);
+    uint4 raw0 = make_uint4(0, 0, 0, 0), raw1 = raw0;
+    if (active) load_row<FP8>(a.x + static_cast<size_t>(token) * d.H, lane, raw0, raw1);
+
+    constexpr int kNone = static_cast<int>(0x80000000); // matches nothing that counts
+    if (sel < 0 || sel >= d.E) sel = kNone;
+    int want[KP], cnt[KP];
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+        want[k] = __builtin_amdgcn_readlane(sel, k); // lanes K.. hold kNone
+        cnt[k] = 0;
+    }
+    // Selections in front of this token's, four loads in flight a lane.
+    const int n = token * d.K;
+    for (int p0 = wave * kWaveSize; p0 < n; p0 += 4 * blockDim.x) {
+        int s[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int p = p0 + j * blockDim.x + wlane;
+            s[j] = p < n ? a.topk_idx[p] : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int k = 0; k < KP; ++k)
+                cnt[k] += __popcll(__ballot(s[j] == want[k]));
+    }
+    if (wlane == 0)
+#pragma unroll
+        for (int k = 0; k < KP; ++k)
+            counted[wave][k] = cnt[k];
+    float scale_inv = 0.f;
+    if constexpr (FP8) raw0 = quantise_group(raw0, raw1, a.round_scale != 0, scale_inv);
+    __syncthreads();
+    if (wave == 0) {
+        // this token's own selections of the same expert come in selection order
+        int slot = 0;
+        for (int k = 0; k < d.K; ++k)
+            slot += k < wlane && __builtin_amdgcn_readlane(sel, k) == sel;
+        if (wlane < d.K) {
+            for (int w = 0; w < n_waves; ++w)
+                slot += counted[w][wlane];
+            const int row = sel != kNone && slot < d.N ? sel * d.N + slot : -1; // beyond N only through repeats: dropped
+            row_of_k[wlane] = row;
+            if (part == 0) {
+                if (a.rows_out) a.rows_out[static_cast<size_t>(token) * d.K + wlane] = row;
+                if (row >= 0) a.src_info[row] = token % d.T;
+            }
+        }
+    }
+    __syncthreads();
+    [[maybe_unused]] uint32_t word = 0;
+    if constexpr (FP8) word = scale_word(scale_inv, a.use_ue8m0 != 0);
+    for (int k = 0; k < d.K; ++k) {
+        const int row = row_of_k[k];
+        if (row < 0 || !active) continue;
+        st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
+        if constexpr (FP8) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, row, lane, word);
+    }
+}
+
+template<bool FP8>
+void
+launch_direct(const DirectArgs &a, dim3 grid, dim3 block, hipStream_t s) {
+    if (a.d.K <= 8)
+        hipLaunchKernelGGL((ll_direct_kernel<FP8, 8>), grid, block, 0, s, a);
+    else
+        hipLaunchKernelGGL((ll_direct_kernel<FP8, 16>), grid, block, 0, s, a);
+}
+
 
 // ---- 3. scales, column-major per expert ------------------------------------------------------------
 //
@@ -912,6 +1115,24 @@ launch_bits(int per_lane, dim3 grid, size_t lds, hipStream_t s, const BitsArgs &
         hipLaunchKernelGGL((ll_bits_kernel<ROUTE, 16>), grid, dim3(threads), lds, s, a);
 }
 
+// Calls that ll_direct_kernel takes: few selections in all, and nothing that only the selection
+// bits know about (masked ranks, ragged ranks, separate phases and their time-outs).  GPU time of
+// a dispatch with hidden 7168, top-8 of 256 experts, fp8, one launch against two (bits and rows,
+// scales written by the rows): 128 selections 6.1 us against 11.5, 2048: 10.2 against 10.9, 4096:
+// 19.5 against 14.2 (every workgroup reads all selections in front of its own).
+constexpr int kDirectSelections = 2048;
+// Up to this many words of scales the row kernel writes them itself, one isolated word at a time,
+// which spares the third launch; beyond it ll_scales_kernel moves them through LDS tiles.  Two
+// launches against three: 1024 tokens x top-8 x 56 words (459 thousand) 21.6 us against 26.4, 524
+// thousand 25.9 against 26.5, 917 thousand 44.8 against 44.3, 1.8 million 86.3 against 71.1.
+constexpr long long kIsolatedScaleWords = 1 << 19;
+
+bool
+direct_fits(const LlDispatchCall &c, const LlDims &d) {
+    return d.T > 0 && static_cast<long long>(d.R) * d.T * d.K <= kDirectSelections && d.R <= kDirectMaxRanks && !c.mask_buffer &&
+        !c.num_tokens_per_rank && c.phases == 3 && c.timeout_us == 0;
+}
+
 int
 ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
     auto bad = [&](int code, const std::string &why) { return nixl_amd_fail(code, std::string(who) + ": " + why); };
@@ -946,6 +1167,37 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
     if (c.timeout_us > kMaxTimeoutUs) return bad(NIXL_AMD_ERR_INVALID, "the time-out may be at most 100 s");
 
     hipStream_t s = static_cast<hipStream_t>(c.stream);
+    if (direct_fits(c, d)) {
+        if (c.logits) {
+            const int routed = nixl_amd_ep_router_topk(c.logits, c.topk_idx, c.topk_weights, d.R * d.T, d.E, d.K, c.stream);
+            if (routed) return routed;
+        }
+        DirectArgs a{};
+        a.recv_x = static_cast<uint8_t *>(c.packed_recv_x);
+        a.recv_scales = c.packed_recv_x_scales;
+        a.src_info = c.packed_recv_src_info;
+        a.layout_range = reinterpret_cast<long long *>(c.packed_recv_layout_range);
+        a.recv_count = c.packed_recv_count;
+        a.stats = c.stats;
+        a.x = static_cast<const uint16_t *>(c.x);
+        a.topk_idx = c.topk_idx;
+        a.status = static_cast<int *>(c.workspace);
+        a.rows_out = c.row_map;
+        a.d = d;
+        a.round_scale = c.round_scale;
+        a.use_ue8m0 = c.use_ue8m0;
+        a.meta_wgs = (d.E + kDirectExperts - 1) / kDirectExperts;
+        const int lanes = c.use_fp8 ? row_lanes<true>(d.H) : row_lanes<false>(d.H);
+        const int most = std::min(kDirectMaxThreads, g_dispatch_lanes.load(std::memory_order_relaxed));
+        a.parts = (lanes + most - 1) / most;
+        const dim3 grid(static_cast<unsigned>(a.meta_wgs + d.R * d.T * a.parts)), block(round_up_wave((lanes + a.parts - 1) / a.parts));
+        if (c.use_fp8)
+            launch_direct<true>(a, grid, block, s);
+        else
+            launch_direct<false>(a, grid, block, s);
+        HIP_TRY(hipGetLastError());
+        return NIXL_AMD_OK;
+    }
     const int Wr = (d.T + kGroupTokens - 1) / kGroupTokens;
     const size_t groups = static_cast<size_t>(d.R) * Wr;
     auto *base = static_cast<uint8_t *>(c.workspace);
@@ -1029,17 +1281,24 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
         HIP_TRY(hipGetLastError());
         return NIXL_AMD_OK;
     }
-    const int wg = std::min(round_up_wave(d.H / 16), g_dispatch_lanes.load(std::memory_order_relaxed));
-    a.parts = (d.H / 16 + wg - 1) / wg;
+    const bool scales_here =
+        c.use_fp8 && static_cast<long long>(d.R) * d.T * d.K * (d.H / (c.use_ue8m0 ? 512 : 128)) <= kIsolatedScaleWords;
+    a.recv_scales = c.packed_recv_x_scales;
+    a.use_ue8m0 = c.use_ue8m0;
+    const int lanes = c.use_fp8 ? row_lanes<true>(d.H) : row_lanes<false>(d.H);
+    const int wg = std::min(round_up_wave(lanes), g_dispatch_lanes.load(std::memory_order_relaxed));
+    a.parts = (lanes + wg - 1) / wg;
     const dim3 grid(static_cast<unsigned>(d.R) * d.T * a.parts);
     const dim3 block(wg);
-    if (c.use_fp8)
-        hipLaunchKernelGGL(ll_dispatch_kernel<true>, grid, block, 0, s, a);
+    if (scales_here)
+        hipLaunchKernelGGL((ll_dispatch_kernel<true, true>), grid, block, 0, s, a);
+    else if (c.use_fp8)
+        hipLaunchKernelGGL((ll_dispatch_kernel<true, false>), grid, block, 0, s, a);
     else
-        hipLaunchKernelGGL(ll_dispatch_kernel<false>, grid, block, 0, s, a);
+        hipLaunchKernelGGL((ll_dispatch_kernel<false, false>), grid, block, 0, s, a);
     HIP_TRY(hipGetLastError());
 
-    if (c.use_fp8) {
+    if (c.use_fp8 && !scales_here) {
         ScalesArgs sa{};
         sa.recv_scales = c.packed_recv_x_scales;
         sa.token_scales = token_scales;

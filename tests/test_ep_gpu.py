@@ -1238,6 +1238,32 @@ def test_ll_combine_logfmt(cuda):
     assert calc_diff(torch.from_numpy(g), torch.from_numpy(ideal)) < 1e-5
 
 
+@pytest.mark.parametrize("shape,form", [
+    # selections in all: one, the most one launch takes (2048), one token more; top-9 and top-16;
+    # experts that do not fill the last metadata workgroup; 64 ranks and 65 (with room for a
+    # rank to name one expert more often than it has tokens, as repeats may); two parts a row
+    ((1, 1, 512, 1, 1, 1), "fp8"), ((4, 64, 512, 8, 24, 64), "fp8"), ((4, 65, 512, 8, 24, 65), "fp8"),
+    ((2, 20, 1024, 9, 34, 20), "ue8m0"), ((2, 64, 8192, 16, 34, 64), "fp8"), ((2, 65, 8192, 16, 34, 65), "bf16"),
+    ((64, 4, 512, 4, 64, 8), "ue8m0"), ((65, 4, 512, 4, 65, 8), "fp8"), ((2, 7, 7168, 8, 8, 16), "bf16"),
+    # 64 words of scales a row: the most the row kernel writes itself (8192 selections), and beyond
+    ((8, 128, 8192, 8, 16, 128), "fp8"), ((8, 129, 8192, 8, 16, 129), "fp8"), ((8, 129, 8192, 8, 16, 129), "ue8m0"),
+])
+def test_ll_dispatch_forms_by_size(cuda, shape, form):
+    """Dispatch takes one, two or three launches by the number of selections and of scale words:
+    every output byte equals the oracle's on both sides of each line, repeats included."""
+    R, T, H, K, E, M = shape
+    x, topk, _ = make_world(R * 11 + T, R, T, H, K, E, drop=0.05, scale=2.0)
+    if K > 1:
+        _with_repeats(np.random.default_rng(T), topk, min(T, 2))
+    fp8, ue = form != "bf16", form == "ue8m0"
+    stats = torch.zeros((R, E // R), dtype=torch.int32, device=cuda)
+    rc, got = raw_ll_dispatch(cuda, x, topk, E, M, fp8, ue, ue, stats=stats)
+    assert rc == 0, _lib.kernels_error()
+    want = eo.ll_dispatch(bits16(x).reshape(R, T, H), topk, E, M, fp8, ue, ue, fill=0x55)
+    assert_dispatch_equal(got, want, fp8, ue)
+    assert np.array_equal(stats.cpu().numpy(), want["recv_count"])
+
+
 def test_ll_narrow_workgroups_give_the_same_bytes(cuda):
     """nixl_amd_ep_ll_set_tuning: with workgroups of 64 and 128 lanes a token's row is split
     over several workgroups in dispatch and combine; results must not change."""
