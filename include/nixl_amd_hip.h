@@ -188,6 +188,47 @@ nixl_amd_copy_records_abandon(nixl_amd_copy_records_t *records);
 int
 nixl_amd_copy_block_len_fits(uint64_t len, const nixl_amd_copy_tuning_t *tuning);
 
+/* A prepared list whose entries share no stride (pieces of different lengths anywhere in a
+ * registered region), kept on the device for as long as the list lives: requests against it
+ * then bring index vectors only, as those against strided lists do.  Entries are 128 to 8176
+ * bytes, address and length multiples of 16 (NIXL_AMD_ERR_INVALID otherwise); `continues` is
+ * non-zero where an entry follows the one before it inside a dense run of equal blocks.  The
+ * entries are copied before the call returns.  Plans do not refer to the lists they were made
+ * from: a list may be destroyed whenever no call that names it is running. */
+typedef struct nixl_amd_copy_list_entry {
+    uint64_t addr;
+    uint32_t len;
+    uint32_t continues;
+} nixl_amd_copy_list_entry_t;
+
+typedef struct nixl_amd_copy_list nixl_amd_copy_list_t;
+
+int
+nixl_amd_copy_list_create(const nixl_amd_copy_list_entry_t *entries, size_t n, int device, nixl_amd_copy_list_t **out);
+
+int
+nixl_amd_copy_list_destroy(nixl_amd_copy_list_t *list);
+
+/* The device a list is kept on, or a negative status. */
+int
+nixl_amd_copy_list_device(const nixl_amd_copy_list_t *list);
+
+/* A plan for `n` pairs: entry src_index[i] of one list is copied to entry dst_index[i] of
+ * another on the same device.  A kernel checks every pair (indices inside their lists, equal
+ * lengths) and writes the records; the call waits for its verdict and returns
+ * NIXL_AMD_ERR_INVALID if a pair is bad.  `n_continued` (may be NULL) receives how many pairs
+ * continue the pair before them on both sides: the descriptors an agent that merges
+ * neighbours would not have listed (src/core/nixl_agent.cpp:799-857). */
+int
+nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
+                                 const int32_t *src_index,
+                                 const nixl_amd_copy_list_t *dst,
+                                 const int32_t *dst_index,
+                                 size_t n,
+                                 const nixl_amd_copy_tuning_t *tuning,
+                                 size_t *n_continued,
+                                 nixl_amd_copy_plan_t **out);
+
 /* Enqueue the whole plan on `stream`: the per-post work of
  * nixlUcxEngine::postXfer -> sendXferRange (src/plugins/ucx/ucx_backend.cpp:1183-1310).
  * Re-launching re-reads the current source bytes; nothing is cached at plan creation

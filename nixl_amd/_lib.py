@@ -40,6 +40,10 @@ class CopyTuning(Structure):
                 ("waves_per_workgroup", c_int), ("xcd_swizzle", c_int), ("sort_scatter", c_int)]
 
 
+class CopyListEntry(Structure):
+    _fields_ = [("addr", c_uint64), ("len", c_uint32), ("continues", c_uint32)]
+
+
 class CopyRun(Structure):
     _fields_ = [("base", c_uint64), ("stride", c_uint64), ("first_index", c_uint64), ("count", c_uint64)]
 
@@ -86,7 +90,13 @@ def kernels():
                                                            POINTER(CopyRecordFacts), POINTER(c_void_p)]
     lib.nixl_amd_copy_records_abandon.argtypes = [c_void_p]
     lib.nixl_amd_copy_block_len_fits.argtypes = [c_uint64, POINTER(CopyTuning)]
-    for fn in ("nixl_amd_copy_records_begin", "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon",
+    lib.nixl_amd_copy_list_create.argtypes = [c_void_p, c_size_t, c_int, POINTER(c_void_p)]
+    lib.nixl_amd_copy_list_destroy.argtypes = [c_void_p]
+    lib.nixl_amd_copy_list_device.argtypes = [c_void_p]
+    lib.nixl_amd_copy_plan_create_listed.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, POINTER(CopyTuning),
+                                                     POINTER(c_size_t), POINTER(c_void_p)]
+    for fn in ("nixl_amd_copy_list_create", "nixl_amd_copy_list_destroy", "nixl_amd_copy_list_device",
+               "nixl_amd_copy_plan_create_listed", "nixl_amd_copy_records_begin", "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon",
                "nixl_amd_copy_block_len_fits"):
         getattr(lib, fn).restype = c_int
     lib.nixl_amd_copy_plan_launch.argtypes = [c_void_p, c_void_p]
@@ -149,6 +159,8 @@ def kernel_symbols():
     return sorted(["nixl_amd_last_error", "nixl_amd_device_count", "nixl_amd_copy_plan_create", "nixl_amd_copy_plan_create_indexed",
                    "nixl_amd_copy_plan_create_indexed_runs", "nixl_amd_copy_records_begin",
                    "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon", "nixl_amd_copy_block_len_fits",
+                   "nixl_amd_copy_list_create", "nixl_amd_copy_list_destroy", "nixl_amd_copy_list_device",
+                   "nixl_amd_copy_plan_create_listed",
                    "nixl_amd_copy_plan_launch", "nixl_amd_copy_plan_destroy", "nixl_amd_copy_plan_status",
                    "nixl_amd_copy_plan_query", "nixl_amd_copy_plan_time", "nixl_amd_ep_ll_workspace_bytes"] + list(_EP_SIGS))
 

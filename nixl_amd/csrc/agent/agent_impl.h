@@ -137,10 +137,26 @@ class nixlDlistH {
 public:
     using descs_t = std::unordered_map<nixlBackendEngine *, std::unique_ptr<nixl_stride_dlist_t>>;
 
+    // A backend's own form of the list (see nixlAgentData::prepListFn), released with the handle.
+    struct resident {
+        void *list = nullptr;
+        void (*release)(void *) = nullptr;
+    };
+
     nixlDlistH(const std::string &remote_agent, descs_t &&d) : remoteAgent(remote_agent), descs(std::move(d)) {}
+
+    ~nixlDlistH() {
+        for (const auto &kv : residents)
+            kv.second.release(kv.second.list);
+    }
+
+    nixlDlistH(const nixlDlistH &) = delete;
+    nixlDlistH &
+    operator=(const nixlDlistH &) = delete;
 
     const std::string remoteAgent; // empty = initiator side
     const descs_t descs;
+    std::unordered_map<nixlBackendEngine *, resident> residents; // filled before the handle is handed out
 };
 
 // Storage of the descriptor lists a request made from index vectors carries.  A paged-KV
@@ -243,12 +259,21 @@ public:
     // lowered by the backend itself.  Null for plugins that do not export it.
     using prepIndexedFn = int (*)(nixlBackendEngine *, int, const nixlStrideDesc *, size_t, const int *,
                                   const nixlStrideDesc *, size_t, const int *, size_t, const char *, nixlBackendReqH **);
+    // Optional as well: lists of many runs are handed to the backend once, when they are
+    // prepared, and requests against two such lists bring index vectors.
+    using prepListFn = int (*)(nixlBackendEngine *, const nixlStrideDesc *, size_t, void **);
+    using releaseListFn = void (*)(void *);
+    using prepListedFn = int (*)(nixlBackendEngine *, int, const void *, const int *, const void *, const int *, size_t, const char *,
+                                 size_t *, size_t *, nixlBackendReqH **);
     struct engineSlot {
         nixlBackendEngine *engine = nullptr;
         const nixlLoadedPlugin *plugin = nullptr;
         std::unique_ptr<nixlBackendH> handle;
         nixl_b_params_t params;
         prepIndexedFn prepIndexed = nullptr;
+        prepListFn prepList = nullptr; // the three of them together or none
+        releaseListFn releaseList = nullptr;
+        prepListedFn prepListed = nullptr;
     };
     // Creation order is preference order.
     std::vector<std::unique_ptr<engineSlot>> engines_;

@@ -71,6 +71,9 @@ struct PieceRec {
 };
 constexpr int kPieceUnitsShift = 56;
 
+// Lengths of the entries of a list that stays on the device: what the piece kernel is made for.
+constexpr uint32_t kListMinBytes = 128, kListMaxBytes = 8176;
+
 struct GenericItem {
     uint64_t src;
     uint64_t dst;
@@ -411,6 +414,110 @@ index_records_runs_kernel(UniformRec *recs, const int32_t *src_index, const int3
     if (i < n)
         recs[i] = UniformRec{run_address(first[0], base[0], stride[0], n_src, static_cast<uint64_t>(src_index[i])),
                              run_address(first[1], base[1], stride[1], n_dst, static_cast<uint64_t>(dst_index[i]))};
+}
+
+// Records of a listed plan: pair i joins entry src_index[i] of one prepared list with entry
+// dst_index[i] of another, both resident on the device (nixl_amd_copy_list).  A thread per pair
+// checks it (indices inside their lists, equal lengths) and writes the piece records of its
+// descriptor: the first at recs[i], those of a descriptor that spans several pieces behind the
+// n first ones, in whatever order the workgroups get there (the order of records decides
+// nothing about the bytes that arrive).  The index vectors are read where they are, in pinned
+// host memory: every index is read once, so a copy to the device first would only add its
+// latency.  The totals reach the host through pinned memory, written by the workgroup that
+// finishes last; the host waits for them, because a bad pair must fail the request.
+struct ListTotals {
+    unsigned long long bytes;
+    uint32_t bad; // pairs that name no entry or join entries of different lengths
+    uint32_t continued; // pairs that continue the pair before them inside one dense run on both sides
+    uint32_t extra; // records beyond the first of their pair
+    uint32_t arrived; // workgroups that have added theirs
+};
+
+constexpr int kListThreads = 256;
+
+__global__ void __launch_bounds__(kListThreads)
+list_records_kernel(PieceRec *__restrict__ recs, // [n * pieces a descriptor can have]
+                    const nixl_amd_copy_list_entry_t *__restrict__ src,
+                    uint32_t n_src,
+                    const nixl_amd_copy_list_entry_t *__restrict__ dst,
+                    uint32_t n_dst,
+                    const int32_t *__restrict__ src_index,
+                    const int32_t *__restrict__ dst_index,
+                    uint32_t n,
+                    ListTotals *totals, // cleared
+                    ListTotals *host) {
+    constexpr int kWaves = kListThreads / kWaveSize;
+    __shared__ unsigned long long wave_bytes[kWaves];
+    __shared__ uint32_t wave_bad[kWaves], wave_continued[kWaves];
+    const uint32_t i = blockIdx.x * kListThreads + threadIdx.x;
+    const int lane = threadIdx.x & (kWaveSize - 1), wave = threadIdx.x / kWaveSize;
+    const int32_t si = i < n ? src_index[i] : 0, di = i < n ? dst_index[i] : 0;
+    // the pair before this one: the neighbour's, or for the first lane of a wave a load
+    int32_t sp = __shfl_up(si, 1), dp = __shfl_up(di, 1);
+    if (lane == 0 && i > 0 && i < n) {
+        sp = src_index[i - 1];
+        dp = dst_index[i - 1];
+    }
+    bool bad = false, continued = false;
+    unsigned long long bytes = 0;
+    if (i < n) {
+        // a negative index is a large unsigned one
+        bad = static_cast<uint32_t>(si) >= n_src || static_cast<uint32_t>(di) >= n_dst;
+        if (!bad) {
+            const nixl_amd_copy_list_entry_t s = src[si], d = dst[di];
+            bad = s.len != d.len;
+            bytes = s.len;
+            continued = i > 0 && si == sp + 1 && di == dp + 1 && s.continues && d.continues;
+            if (!bad) {
+                const uint32_t units = s.len / 16u, head = kPieceUnits - (static_cast<uint32_t>(d.addr >> 4) & 7u);
+                uint32_t count = min(units, head), more = units - count;
+                recs[i] = PieceRec{s.addr, d.addr | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
+                if (more) {
+                    uint32_t at = n + atomicAdd(&totals->extra, (more + kPieceUnits - 1) / kPieceUnits);
+                    for (uint32_t first = count; more; first += count, more -= count) {
+                        count = min(more, kPieceUnits);
+                        recs[at++] = PieceRec{s.addr + first * 16ull,
+                                              (d.addr + first * 16ull) | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
+                    }
+                }
+            }
+        }
+    }
+    const uint32_t n_bad = __popcll(__ballot(bad)), n_continued = __popcll(__ballot(continued));
+#pragma unroll
+    for (int off = kWaveSize / 2; off > 0; off >>= 1)
+        bytes += __shfl_xor(bytes, off);
+    if (lane == 0) {
+        wave_bytes[wave] = bytes;
+        wave_bad[wave] = n_bad;
+        wave_continued[wave] = n_continued;
+    }
+    __syncthreads(); // every extra record of the workgroup is counted as well
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+        uint32_t b = 0, c = 0;
+        for (int w = 0; w < kWaves; ++w) {
+            sum += wave_bytes[w];
+            b += wave_bad[w];
+            c += wave_continued[w];
+        }
+        atomicAdd(&totals->bytes, sum);
+        if (b) atomicAdd(&totals->bad, b);
+        if (c) atomicAdd(&totals->continued, c);
+        __threadfence();
+        if (atomicAdd(&totals->arrived, 1u) == gridDim.x - 1) {
+            __threadfence();
+            host->bytes = __hip_atomic_load(&totals->bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            host->bad = __hip_atomic_load(&totals->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            host->continued = __hip_atomic_load(&totals->continued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            host->extra = __hip_atomic_load(&totals->extra, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+__global__ void __launch_bounds__(kWaveSize)
+clear_totals_kernel(ListTotals *totals) {
+    if (threadIdx.x == 0) *totals = ListTotals{};
 }
 
 // Records of a plan whose runs of uniform chunks differ in length: run r covers chunks
@@ -1441,6 +1548,161 @@ nixl_amd_copy_plan_create_indexed(uint64_t src_base,
                                   nixl_amd_copy_plan_t **out) {
     const nixl_amd_copy_run_t src{src_base, src_stride, 0, 0}, dst{dst_base, dst_stride, 0, 0};
     return nixl_amd_copy_plan_create_indexed_runs(&src, 1, src_index, &dst, 1, dst_index, n, len, device, tuning, out);
+}
+
+// A prepared list on the device, see nixl_amd_copy_list_create.
+struct nixl_amd_copy_list {
+    int device = 0;
+    nixl_amd_copy_list_entry_t *entries = nullptr;
+    size_t cap = 0; // size of the block the entries lie in
+    uint32_t n = 0;
+    uint32_t max_len = 0;
+};
+
+int
+nixl_amd_copy_list_create(const nixl_amd_copy_list_entry_t *entries, size_t n, int device, nixl_amd_copy_list_t **out) {
+    if (!out) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "list_create: out is null");
+    *out = nullptr;
+    if (!entries || n == 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "list_create: no entries");
+    if (n >= (1ull << 30)) return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "list_create: more than 2^30 entries");
+    uint64_t address_bits = 0;
+    uint32_t len_bits = 0, min_len = ~0u, max_len = 0, wraps = 0;
+    for (size_t i = 0; i < n; ++i) {
+        const nixl_amd_copy_list_entry_t &e = entries[i];
+        address_bits |= e.addr;
+        len_bits |= e.len;
+        min_len = std::min(min_len, e.len);
+        max_len = std::max(max_len, e.len);
+        wraps |= static_cast<uint32_t>(e.addr == 0) | static_cast<uint32_t>(((e.addr + e.len) >> kPieceUnitsShift) != 0);
+    }
+    if (((address_bits | len_bits) & 15u) || min_len < kListMinBytes || max_len > kListMaxBytes || wraps)
+        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "list_create: entries must be 16-byte aligned and 128 to 8176 bytes long");
+    int ndev = 0;
+    if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return nixl_amd_fail(NIXL_AMD_ERR_NO_DEVICE, "list_create: no HIP device");
+    if (device < 0 || device >= ndev) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "list_create: bad device index");
+    const DeviceScope on_device(device);
+    HIP_TRY(on_device.status());
+    void *mem = nullptr;
+    size_t cap = 0;
+    HIP_TRY(arena_cache().get(device, n * sizeof(nixl_amd_copy_list_entry_t), &mem, &cap));
+    // waits for the copy: the caller's array may go away, and the first request finds the table there
+    hipStream_t up = nullptr;
+    hipError_t e = upload_stream(device, &up);
+    if (e == hipSuccess) e = hipMemcpyAsync(mem, entries, n * sizeof(nixl_amd_copy_list_entry_t), hipMemcpyHostToDevice, up);
+    if (e == hipSuccess) e = hipStreamSynchronize(up);
+    if (e != hipSuccess) {
+        if (up) (void)hipStreamSynchronize(up);
+        arena_cache().put(device, mem, cap);
+        return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("list_create: ") + hipGetErrorString(e));
+    }
+    auto *list = new nixl_amd_copy_list();
+    list->device = device;
+    list->entries = static_cast<nixl_amd_copy_list_entry_t *>(mem);
+    list->cap = cap;
+    list->n = static_cast<uint32_t>(n);
+    list->max_len = max_len;
+    *out = list;
+    return NIXL_AMD_OK;
+}
+
+int
+nixl_amd_copy_list_destroy(nixl_amd_copy_list_t *list) {
+    if (!list) return NIXL_AMD_OK;
+    // nothing on the device reads a list once plan_create_listed has returned
+    arena_cache().put(list->device, list->entries, list->cap);
+    delete list;
+    return NIXL_AMD_OK;
+}
+
+int
+nixl_amd_copy_list_device(const nixl_amd_copy_list_t *list) {
+    return list ? list->device : nixl_amd_fail(NIXL_AMD_ERR_INVALID, "list_device: list is null");
+}
+
+int
+nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
+                                 const int32_t *src_index,
+                                 const nixl_amd_copy_list_t *dst,
+                                 const int32_t *dst_index,
+                                 size_t n,
+                                 const nixl_amd_copy_tuning_t *tuning,
+                                 size_t *n_continued,
+                                 nixl_amd_copy_plan_t **out) {
+    if (!out) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: out is null");
+    *out = nullptr;
+    if (!src || !dst || !src_index || !dst_index || n == 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: null argument");
+    if (src->device != dst->device) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: lists on different devices");
+    Tuning t;
+    if (const int rc = parse_tuning(tuning, t, "plan_create_listed")) return rc;
+    // pieces a descriptor can have: its first line may hold back seven units of the first one
+    const size_t max_units = std::min(src->max_len, dst->max_len) / 16u;
+    const size_t per_desc = 1 + (max_units + 6) / kPieceUnits;
+    if (n > (1ull << 31) / per_desc - 1) return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "plan_create_listed: too many pairs");
+    const int device = src->device;
+    const DeviceScope on_device(device);
+    HIP_TRY(on_device.status());
+
+    const size_t index_bytes = n * sizeof(int32_t);
+    const size_t totals_at = (2 * index_bytes + 15) & ~size_t(15); // the host's totals follow the index vectors
+    void *staging = nullptr;
+    size_t staging_cap = 0;
+    reap_uploads(device);
+    hipError_t e = upload_cache().get(device, totals_at + sizeof(ListTotals), &staging, &staging_cap);
+    if (e != hipSuccess)
+        return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
+    auto *up_src = static_cast<int32_t *>(staging), *up_dst = up_src + n;
+    std::memcpy(up_src, src_index, index_bytes);
+    std::memcpy(up_dst, dst_index, index_bytes);
+    auto *host = reinterpret_cast<ListTotals *>(static_cast<uint8_t *>(staging) + totals_at);
+    *host = ListTotals{0, ~0u, 0, 0, 0}; // every pair bad until the kernel has said otherwise
+
+    auto *plan = new nixl_amd_copy_plan();
+    plan->device = device;
+    plan->upl = t.upl;
+    plan->waves = t.waves;
+    plan->swizzle = t.swizzle;
+    plan->max_wgs = t.max_wgs;
+    plan->policy = t.nt ? t.nt : kPolNtSc1Nt;
+    if (t.nt) plan->piece_policy = t.nt;
+    // one arena: the totals, then the records
+    constexpr size_t kRecsAt = 256;
+    hipStream_t up = nullptr;
+    e = arena_cache().get(device, kRecsAt + n * per_desc * sizeof(PieceRec), &plan->arena, &plan->arena_cap);
+    if (e == hipSuccess) e = upload_stream(device, &up);
+    auto *totals = static_cast<ListTotals *>(plan->arena);
+    auto *recs = reinterpret_cast<PieceRec *>(static_cast<uint8_t *>(plan->arena) + kRecsAt);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(clear_totals_kernel, dim3(1), dim3(kWaveSize), 0, up, totals);
+        hipLaunchKernelGGL(list_records_kernel, dim3(static_cast<uint32_t>((n + kListThreads - 1) / kListThreads)), dim3(kListThreads),
+                           0, up, recs, src->entries, src->n, dst->entries, dst->n, up_src, up_dst, static_cast<uint32_t>(n), totals,
+                           host);
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+    if (e == hipSuccess) e = settle_upload(plan, true);
+    if (e != hipSuccess && up) (void)hipStreamSynchronize(up); // whatever was queued reads the buffers given back below
+    const ListTotals got = *host;
+    upload_cache().put(device, staging, staging_cap);
+    if (e != hipSuccess || got.bad) {
+        if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
+        if (plan->arena) arena_cache().put(device, plan->arena, plan->arena_cap);
+        delete plan;
+        if (e != hipSuccess) return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("plan_create_listed: ") + hipGetErrorString(e));
+        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: " + std::to_string(got.bad) +
+                                                       " pairs name no entry or join entries of different lengths");
+    }
+    plan->arena_bytes = kRecsAt + (n + got.extra) * sizeof(PieceRec);
+    plan->piece_recs = recs;
+    plan->n_pieces = static_cast<uint32_t>(n + got.extra);
+    plan->info.payload_bytes = got.bytes;
+    plan->info.vec_descs = n;
+    plan->info.plan_device_bytes = plan->arena_bytes;
+    plan->info.piece_items = plan->n_pieces;
+    plan->info.units_per_lane = static_cast<uint32_t>(t.upl);
+    if (n_continued) *n_continued = got.continued;
+    *out = plan;
+    return NIXL_AMD_OK;
 }
 
 int

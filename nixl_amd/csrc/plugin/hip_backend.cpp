@@ -91,6 +91,9 @@ struct PublicRegion {
 constexpr uint64_t kRegionMagic = 0x324e474552504948ull; // "HIPREGN2"
 constexpr const char *kConnPrefix = "HIP2:pid=";
 constexpr const char *kConnMailbox = ";mbox=";
+// Pairs from which a request against two device-resident lists is lowered on the device: below,
+// the wait for the kernel's verdict costs more than the host's 27 ns a pair.
+constexpr size_t kListedFrom = 1024;
 // Allocations of 2 GiB and more are not shared between processes: opening such a mapping has
 // been seen not to return.
 constexpr size_t kMaxIpcAllocation = (size_t{2} << 30) - 1;
@@ -756,6 +759,79 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
 }
 
 nixl_status_t
+nixlHipEngine::prepList(const nixlStrideDesc *runs, size_t n_runs, nixl_amd_copy_list_t *&list) const {
+    list = nullptr;
+    if (!indexedPrep_) return NIXL_ERR_NOT_SUPPORTED;
+    if (!runs || n_runs == 0) return NIXL_ERR_INVALID_PARAM;
+    constexpr size_t kMinBytes = 128, kMaxBytes = 8176; // what the kernels library takes
+    std::vector<nixl_amd_copy_list_entry_t> entries;
+    entries.reserve(runs[n_runs - 1].start_idx + runs[n_runs - 1].count);
+    int device = -1;
+    for (size_t r = 0; r < n_runs; ++r) {
+        const nixlStrideDesc &run = runs[r];
+        if (run.len < kMinBytes || run.len > kMaxBytes || ((run.addr | run.len | (run.count > 1 ? run.stride : 0)) & 15u))
+            return NIXL_ERR_NOT_SUPPORTED;
+        if (run.count == 0 || run.start_idx != entries.size()) return NIXL_ERR_NOT_SUPPORTED;
+        const auto *md = static_cast<const nixlHipMD *>(run.metadataP);
+        size_t span = 0;
+        const bool fits = md && !__builtin_mul_overflow(run.count - 1, run.stride, &span) &&
+            !__builtin_add_overflow(span, run.len, &span) && md->contains(run.addr, span);
+        if (!fits) return NIXL_ERR_NOT_SUPPORTED; // a request that names the entry says so
+        // one device throughout, host memory anywhere: a list of host memory alone has no device to stay on
+        if (md->mem == VRAM_SEG) {
+            if (device < 0) device = md->device;
+            if (md->device != device) return NIXL_ERR_NOT_SUPPORTED;
+        }
+        const uintptr_t base = md->here(run.addr);
+        const bool dense = run.stride == run.len;
+        for (size_t j = 0; j < run.count; ++j)
+            entries.push_back(nixl_amd_copy_list_entry_t{base + j * run.stride, static_cast<uint32_t>(run.len), dense && j > 0});
+    }
+    if (device < 0) return NIXL_ERR_NOT_SUPPORTED;
+    if (nixl_amd_copy_list_create(entries.data(), entries.size(), device, &list) != NIXL_AMD_OK) {
+        NIXL_DEBUG << "HIP backend: the list stays on the host: " << nixl_amd_last_error();
+        return NIXL_ERR_NOT_SUPPORTED;
+    }
+    return NIXL_SUCCESS;
+}
+
+nixl_status_t
+nixlHipEngine::prepXferListed(const nixl_xfer_op_t &operation,
+                              const nixl_amd_copy_list_t *local,
+                              const int *local_indices,
+                              const nixl_amd_copy_list_t *remote,
+                              const int *remote_indices,
+                              size_t count,
+                              const std::string &remote_agent,
+                              size_t &bytes,
+                              size_t &merged,
+                              nixlBackendReqH *&handle) const {
+    handle = nullptr;
+    if (count < kListedFrom) return NIXL_ERR_NOT_SUPPORTED;
+    reapRetired(false);
+    if (!knowsAgent(remote_agent)) return NIXL_ERR_NOT_FOUND;
+    if (operation != NIXL_READ && operation != NIXL_WRITE) return NIXL_ERR_INVALID_PARAM;
+    const bool write = (operation == NIXL_WRITE);
+    auto req = std::make_unique<nixlHipReqH>();
+    size_t continued = 0;
+    if (nixl_amd_copy_plan_create_listed(write ? local : remote, write ? local_indices : remote_indices, write ? remote : local,
+                                         write ? remote_indices : local_indices, count, &tuning_, &continued,
+                                         &req->plan) != NIXL_AMD_OK) {
+        NIXL_DEBUG << "HIP backend: " << nixl_amd_last_error();
+        return NIXL_ERR_NOT_SUPPORTED;
+    }
+    nixl_amd_copy_plan_info_t info{};
+    (void)nixl_amd_copy_plan_query(req->plan, &info);
+    req->device = nixl_amd_copy_list_device(local);
+    req->bytes = bytes = info.payload_bytes;
+    merged = count - continued;
+    req->stream = pickStream(req->device);
+    if (!req->stream && !useExternalStream_) return NIXL_ERR_BACKEND;
+    handle = req.release();
+    return NIXL_SUCCESS;
+}
+
+nixl_status_t
 nixlHipEngine::postXfer(const nixl_xfer_op_t &,
                         const nixl_meta_dlist_t &,
                         const nixl_meta_dlist_t &,
@@ -1348,6 +1424,50 @@ nixl_hip_prep_xfer_indexed(nixlBackendEngine *engine,
         return static_cast<nixlHipEngine *>(engine)->prepXferIndexed(static_cast<nixl_xfer_op_t>(operation), local_runs,
                                                                      n_local_runs, local_indices, remote_runs, n_remote_runs,
                                                                      remote_indices, count, remote_agent, *handle);
+    } catch (const std::exception &e) {
+        NIXL_ERROR << "HIP backend: " << e.what();
+        return NIXL_ERR_BACKEND;
+    }
+}
+
+// Optional entries of this plugin for lists that share no stride: see nixlHipEngine::prepList.
+extern "C" NIXL_PLUGIN_EXPORT int
+nixl_hip_prep_list(nixlBackendEngine *engine, const nixlStrideDesc *runs, size_t n_runs, void **list) {
+    if (!engine || !runs || !list) return NIXL_ERR_INVALID_PARAM;
+    try {
+        nixl_amd_copy_list_t *made = nullptr;
+        const nixl_status_t st = static_cast<nixlHipEngine *>(engine)->prepList(runs, n_runs, made);
+        *list = made;
+        return st;
+    } catch (const std::exception &e) {
+        NIXL_ERROR << "HIP backend: " << e.what();
+        return NIXL_ERR_BACKEND;
+    }
+}
+
+extern "C" NIXL_PLUGIN_EXPORT void
+nixl_hip_release_list(void *list) {
+    (void)nixl_amd_copy_list_destroy(static_cast<nixl_amd_copy_list_t *>(list));
+}
+
+extern "C" NIXL_PLUGIN_EXPORT int
+nixl_hip_prep_xfer_listed(nixlBackendEngine *engine,
+                          int operation,
+                          const void *local,
+                          const int *local_indices,
+                          const void *remote,
+                          const int *remote_indices,
+                          size_t count,
+                          const char *remote_agent,
+                          size_t *bytes,
+                          size_t *merged,
+                          nixlBackendReqH **handle) {
+    if (!engine || !local || !local_indices || !remote || !remote_indices || !remote_agent || !bytes || !merged || !handle)
+        return NIXL_ERR_INVALID_PARAM;
+    try {
+        return static_cast<nixlHipEngine *>(engine)->prepXferListed(
+            static_cast<nixl_xfer_op_t>(operation), static_cast<const nixl_amd_copy_list_t *>(local), local_indices,
+            static_cast<const nixl_amd_copy_list_t *>(remote), remote_indices, count, remote_agent, *bytes, *merged, *handle);
     } catch (const std::exception &e) {
         NIXL_ERROR << "HIP backend: " << e.what();
         return NIXL_ERR_BACKEND;

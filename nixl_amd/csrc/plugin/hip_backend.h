@@ -190,6 +190,27 @@ public:
                     const std::string &remote_agent,
                     nixlBackendReqH *&handle) const;
 
+    // The same for lists that share no stride: a list is handed over once, when it is prepared
+    // (entries of 128 to 8176 bytes, 16-byte aligned, on one device; NIXL_ERR_NOT_SUPPORTED
+    // otherwise), and stays on the device; requests against two such lists bring their index
+    // vectors, which a kernel checks and lowers.  `bytes` and `merged` receive the request's
+    // size and the number of its descriptors after merging.  NIXL_ERR_NOT_SUPPORTED means "take
+    // the ordinary path", which also names the pair when one is bad.  Reached through
+    // nixl_hip_prep_list, nixl_hip_release_list and nixl_hip_prep_xfer_listed.
+    nixl_status_t
+    prepList(const nixlStrideDesc *runs, size_t n_runs, nixl_amd_copy_list_t *&list) const;
+    nixl_status_t
+    prepXferListed(const nixl_xfer_op_t &operation,
+                   const nixl_amd_copy_list_t *local,
+                   const int *local_indices,
+                   const nixl_amd_copy_list_t *remote,
+                   const int *remote_indices,
+                   size_t count,
+                   const std::string &remote_agent,
+                   size_t &bytes,
+                   size_t &merged,
+                   nixlBackendReqH *&handle) const;
+
     // Memory views for kernels that move data themselves: the handle is a device pointer
     // to a table of {address, length} entries (layout in nixl_amd_device.h), checked here
     // against the registrations (shape of src/plugins/ucx/ucx_backend.cpp prepMemView).

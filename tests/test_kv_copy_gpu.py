@@ -809,6 +809,62 @@ def test_more_pieces_than_one_launch_takes(cuda):
     assert bool((dst[:, :16] == 0xC3).all())
 
 
+@pytest.mark.parametrize("count", [1023, 1024, 1025, 3001])
+@pytest.mark.parametrize("op", ["WRITE", "READ"])
+def test_lists_without_a_stride_stay_on_the_device(cuda, op, count):
+    """Prepared lists of unequal pieces (128 B to 8176 B, any 16-byte address, so that one, two
+    or three records come of a piece) at the pair counts around the one from which the device
+    lowers them: every byte against the per-descriptor oracle; a repost moves the current bytes;
+    a bad index and a pair of unequal lengths are refused as on the host."""
+    import torch
+    from nixl_amd.agent import NixlError
+    rng = np.random.default_rng(count)
+    n = 4000
+    lens = rng.choice([128, 144, 1008, 3968, 3984, 4080, 4096, 4112, 8064, 8176], n).astype(np.int64)
+    half = n * 8448
+    so = np.arange(n) * 8448 + rng.integers(0, 16, n) * 16
+    do = half + rng.permutation(n) * 8448 + rng.integers(0, 16, n) * 16
+    host = rng.integers(0, 256, 2 * half, dtype=np.uint8)
+    mem = torch.from_numpy(host.copy()).to(cuda)
+    agent = nixl_agent(f"listed{op}{count}", nixl_agent_config(backends=("HIP",)))
+    try:
+        agent.register_memory([mem])
+
+        def handle(offsets, who):
+            triples = np.stack([np.uint64(mem.data_ptr()) + offsets.astype(np.uint64), lens.astype(np.uint64), np.zeros(n, np.uint64)], 1)
+            return agent.prep_xfer_dlist(who, triples, "VRAM")
+
+        # READ: the local side is the destination
+        local, remote = (handle(so, ""), handle(do, agent.name)) if op == "WRITE" else (handle(do, ""), handle(so, agent.name))
+        idx = rng.permutation(n)[:count].astype(np.int32)
+        req = agent.make_prepped_xfer(op, local, idx, remote, idx)
+        for _ in range(2):
+            torch.cuda.synchronize()
+            state = agent.transfer(req)
+            while state == "PROC":
+                state = agent.check_xfer_state(req)
+            assert state == "DONE"
+            host = ko.copy_descs(host, so[idx], do[idx], lens[idx])
+            assert np.array_equal(mem.cpu().numpy(), host)
+            host[:half] ^= 0x5A
+            mem[:half] ^= 0x5A
+        req.release()
+        bad = idx.copy()
+        bad[count // 2] = n
+        with pytest.raises(NixlError):
+            agent.make_prepped_xfer(op, local, bad, remote, idx)
+        bad[count // 2] = -1
+        with pytest.raises(NixlError):
+            agent.make_prepped_xfer(op, local, idx, remote, bad)
+        bad[count // 2] = int(np.argmax(lens != lens[idx[count // 2]]))
+        with pytest.raises(NixlError):
+            agent.make_prepped_xfer(op, local, bad, remote, idx)
+        for h in (local, remote):
+            h.release()
+    finally:
+        agent.close()
+
+
 def test_golden_descriptor_list(cuda):
     """Committed vector (tests/golden/kv_descs.npz): mixed aligned / unaligned / empty
     descriptors, destination pre-filled with a canary byte."""
