@@ -57,6 +57,11 @@ typedef struct nixl_amd_copy_tuning {
     int xcd_swizzle; /* 1 = each accelerator die walks a contiguous slice of the chunk list, 2 = off */
     int sort_scatter; /* a plan that scatters consecutive memory over irregular destinations has its records put
                        * into ascending destination order inside windows of 1024 (on the device): 1 = on, 2 = off */
+    /* The HIP stream the plan will be launched on, or NULL.  While that stream is idle the
+     * kernels that write the plan's arrays are queued on it, so that a launch needs no wait; the
+     * stream must then outlive the plan and must not be under capture when the plan is first
+     * launched on it.  NULL, or a busy stream: they run on a stream of the library's. */
+    void *stream;
 } nixl_amd_copy_tuning_t;
 
 typedef struct nixl_amd_copy_plan nixl_amd_copy_plan_t;

@@ -34,6 +34,7 @@
 #include <algorithm>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <vector>
 
@@ -158,6 +159,34 @@ copy_uniform_kernel(const UniformRec *recs, uint32_t first_chunk, uint32_t n_chu
 #pragma unroll
     for (int k = 0; k < UPL; ++k)
         store16<POL>(d + k * (kWaveSize * 16u), v[k]);
+}
+
+// The same for a request of a few blocks, whose records travel as the kernel's arguments: nothing
+// is uploaded, so nothing has to be waited for between the making of the request and its copy.
+// 64 blocks of 32 KiB, from the making of the request to its end: 51 us with uploaded records, 19
+// with these.  128 records are 2 KiB of the 4 KiB a launch can carry.
+constexpr uint32_t kInlineRecs = 128;
+
+struct InlineRecs {
+    UniformRec rec[kInlineRecs];
+};
+
+template<int POL>
+__global__ void __launch_bounds__(kWaveSize)
+copy_inline_kernel(InlineRecs recs, uint32_t chunks_per_rec) {
+    const uint32_t r = blockIdx.x / chunks_per_rec;
+    const uint64_t off = static_cast<uint64_t>(blockIdx.x % chunks_per_rec) * (kWaveSize * 16u) + threadIdx.x * 16u;
+    store16<POL>(recs.rec[r].dst + off, load16<POL>(recs.rec[r].src + off));
+}
+
+// Moves the arrays of a plan from the pinned buffer they were built in to the device, 16 bytes a
+// lane.  A copy engine is slower for all but large plans: it has to be started and its end
+// signalled to the kernels behind it (90 KB: 6.5 us here, 8.5 there and the signal on top), while
+// beyond a MiB it moves 63 GB/s and lanes reading over the bus 26.
+__global__ void __launch_bounds__(256)
+upload_kernel(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t n) {
+    for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * blockDim.x)
+        dst[i] = src[i];
 }
 
 // One wavefront per piece: the descriptor's own {src, dst, units} record, up to
@@ -724,6 +753,18 @@ upload_cache() {
     return *c;
 }
 
+// Queues the copy of `bytes` of a pinned block to a device block on `up`; both blocks are powers
+// of two from 4 KiB, so whole 16-byte units of the last one lie inside them.
+hipError_t
+upload(hipStream_t up, void *dst, const void *staging, size_t bytes) {
+    constexpr size_t kByKernel = 1u << 20;
+    if (bytes > kByKernel) return hipMemcpyAsync(dst, staging, bytes, hipMemcpyHostToDevice, up);
+    const size_t units = (bytes + 15) / 16;
+    const dim3 grid(static_cast<unsigned>(std::min<size_t>((units + 255) / 256, 1024)));
+    hipLaunchKernelGGL(upload_kernel, grid, dim3(256), 0, up, static_cast<uint4 *>(dst), static_cast<const uint4 *>(staging), units);
+    return hipGetLastError();
+}
+
 } // namespace
 
 struct nixl_amd_copy_plan {
@@ -742,6 +783,7 @@ struct nixl_amd_copy_plan {
     uint32_t n_uniform = 0; // uniform chunks
     uint32_t chunks_per_rec = 1;
     uint32_t uniform_wgs = 0;
+    std::unique_ptr<InlineRecs> inline_recs; // instead of uniform_recs: a plan of a few blocks, nothing on the device
     MixedArgs mixed_args{};
     uint32_t mixed_wgs = 0;
     const PieceRec *piece_recs = nullptr;
@@ -751,10 +793,15 @@ struct nixl_amd_copy_plan {
     uint32_t generic_wgs = 0;
     nixl_amd_copy_plan_info_t info{};
     hipEvent_t ev0 = nullptr, ev1 = nullptr; // timing events, created on first use
-    // A plan built from index vectors returns before its records exist: they are written by
-    // kernels queued on the upload stream, `uploaded` is recorded behind them, and the first
-    // launches wait for it on their own stream.
+    // A plan is returned before its arrays are on the device: they are written by kernels queued
+    // on a stream.  On the library's upload stream `uploaded` is recorded behind them, and the
+    // first launches wait for it on their own stream.  On the stream the caller named (where the
+    // launch is going to follow) nothing has to be waited for; the pinned buffer that the kernels
+    // read then stays with the plan.
     hipEvent_t uploaded = nullptr;
+    hipStream_t built_on = nullptr; // the caller's stream, until a launch is known to be behind the build
+    void *staging = nullptr;
+    size_t staging_cap = 0;
     // Recorded behind the kernels of every launch (not on a capturing stream): destroying the
     // plan while it has not completed is refused, because the arena would go back to the pool
     // and the next plan's upload would overwrite records a running kernel still reads.
@@ -769,6 +816,8 @@ struct PendingUpload {
     hipEvent_t done;
     void *staging;
     size_t cap;
+    void *arena; // of a plan destroyed before it was launched, or null
+    size_t arena_cap;
 };
 static std::mutex g_pending_mutex;
 static std::map<int, std::vector<PendingUpload>> g_pending; // by device
@@ -786,25 +835,27 @@ reap_uploads(int device) {
         }
         (void)hipEventDestroy(list[i].done);
         upload_cache().put(device, list[i].staging, list[i].cap);
+        if (list[i].arena) arena_cache().put(device, list[i].arena, list[i].arena_cap);
         list[i] = list.back();
         list.pop_back();
     }
 }
 
-// Hands `staging` over: recycled when everything queued on `up` so far has run.  Without an
-// event to watch, the stream is waited for instead.
+// Hands `staging` (and `arena`) over: recycled when everything queued on `up` so far has run.
+// Without an event to watch, the stream is waited for instead.
 static void
-recycle_after(int device, hipStream_t up, void *staging, size_t cap) {
+recycle_after(int device, hipStream_t up, void *staging, size_t cap, void *arena = nullptr, size_t arena_cap = 0) {
     hipEvent_t done = nullptr;
     if (hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess && hipEventRecord(done, up) == hipSuccess) {
         std::lock_guard<std::mutex> lock(g_pending_mutex);
-        g_pending[device].push_back(PendingUpload{done, staging, cap});
+        g_pending[device].push_back(PendingUpload{done, staging, cap, arena, arena_cap});
         return;
     }
     (void)hipGetLastError();
     if (done) (void)hipEventDestroy(done);
     (void)hipStreamSynchronize(up);
     upload_cache().put(device, staging, cap);
+    if (arena) arena_cache().put(device, arena, arena_cap);
 }
 
 // The plan's records are in place (or `wait` and they are not yet: block until they are).
@@ -825,6 +876,7 @@ settle_upload(nixl_amd_copy_plan *plan, bool wait) {
 struct Tuning {
     int upl = 1, nt = 0, waves = 1, swizzle = 0, sort_scatter = 0;
     uint32_t max_wgs = 0;
+    hipStream_t stream = nullptr;
 };
 
 // Defaults from a sweep on MI355X: the smallest chunk (one 128-bit load and store per lane,
@@ -839,6 +891,7 @@ parse_tuning(const nixl_amd_copy_tuning_t *tuning, Tuning &t, const char *who) {
         if (tuning->waves_per_workgroup) t.waves = tuning->waves_per_workgroup;
         if (tuning->xcd_swizzle) t.swizzle = tuning->xcd_swizzle == 1 ? 1 : 0;
         t.sort_scatter = tuning->sort_scatter;
+        t.stream = static_cast<hipStream_t>(tuning->stream);
     }
     if (t.upl != 1 && t.upl != 2 && t.upl != 4 && t.upl != 8 && t.upl != 16)
         return nixl_amd_fail(NIXL_AMD_ERR_INVALID, std::string(who) + ": units_per_lane must be 1, 2, 4, 8 or 16");
@@ -854,6 +907,64 @@ static bool
 block_len_fits(uint64_t len, const Tuning &t) {
     const uint64_t chunk_bytes = static_cast<uint64_t>(kWaveSize) * t.upl * 16u;
     return len >= 8192 && len % chunk_bytes == 0;
+}
+
+// Whether a plan of `n` equal blocks can carry its records as kernel arguments: few enough, and
+// the launch shape the inline kernel has.
+static bool
+fits_inline(size_t n, uint64_t len, const Tuning &t) {
+    return n <= kInlineRecs && t.upl == 1 && t.waves == 1 && !t.swizzle && n * (len / (kWaveSize * 16u)) <= kMaxGrid;
+}
+
+// The members a plan of `n_recs` equal blocks has wherever its records are.
+static void
+describe_blocks(nixl_amd_copy_plan &plan, const Tuning &t, size_t n_recs, uint64_t len, size_t n_descs) {
+    const uint64_t chunk_bytes = static_cast<uint64_t>(kWaveSize) * t.upl * 16u;
+    plan.chunks_per_rec = static_cast<uint32_t>(len / chunk_bytes);
+    plan.n_uniform = static_cast<uint32_t>(n_recs * plan.chunks_per_rec);
+    plan.uniform_wgs = (plan.n_uniform + static_cast<uint32_t>(t.waves) - 1) / static_cast<uint32_t>(t.waves);
+    plan.info.payload_bytes = n_recs * len;
+    plan.info.vec_descs = n_descs;
+    plan.info.plan_device_bytes = plan.arena_bytes;
+    plan.info.vec_chunks = plan.n_uniform;
+    plan.info.uniform_chunks = plan.n_uniform;
+    plan.info.units_per_lane = static_cast<uint32_t>(t.upl);
+    plan.info.uniform_workgroups = plan.uniform_wgs;
+}
+
+// The stream a plan's arrays are written on: the one its launches will follow on, if the caller
+// named it and it is idle.  A launch right behind the making then needs no event, no wait of one
+// stream for another and no recycling in between (20 us of host time between make and kernel
+// became 5); behind a transfer that is still running, the library's own stream writes the arrays
+// meanwhile.
+static hipError_t
+build_stream(int device, const Tuning &t, hipStream_t *out) {
+    if (t.stream) {
+        const hipError_t idle = hipStreamQuery(t.stream);
+        if (idle == hipSuccess) {
+            *out = t.stream;
+            return hipSuccess;
+        }
+        (void)hipGetLastError();
+    }
+    return upload_stream(device, out);
+}
+
+// Everything that writes the plan's arrays is queued on `up`: what later launches and the pinned
+// buffer's next user wait for.  The buffer is taken over if this succeeds.
+static hipError_t
+end_build(nixl_amd_copy_plan *plan, const Tuning &t, hipStream_t up, void *staging, size_t staging_cap) {
+    if (t.stream && up == t.stream) {
+        plan->built_on = up;
+        plan->staging = staging;
+        plan->staging_cap = staging_cap;
+        return hipSuccess;
+    }
+    // No wait here: the event goes behind the kernels, launches wait for it on their stream.
+    hipError_t e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+    if (e == hipSuccess) recycle_after(plan->device, up, staging, staging_cap);
+    return e;
 }
 
 constexpr int kNotBlocks = 1; // build_block_plan: the records are not what a block plan takes (no error recorded)
@@ -915,18 +1026,24 @@ build_block_plan(int device, const Tuning &t, void *staging, size_t staging_cap,
     // a scatter out of consecutive memory is put into ascending destination order, window by window
     const bool sort = scattered && t.sort_scatter != 2 && 2 * src_follows >= steps && n_recs >= kSortWindow;
     plan->policy = t.nt ? t.nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
+    if (fits_inline(n_recs, len, t)) {
+        plan->inline_recs = std::make_unique<InlineRecs>();
+        std::memcpy(plan->inline_recs->rec, recs, bytes);
+        upload_cache().put(device, staging, staging_cap);
+        describe_blocks(*plan, t, n_recs, len, n_descs);
+        *out = plan;
+        return NIXL_AMD_OK;
+    }
     hipStream_t up = nullptr;
     hipError_t e = arena_cache().get(device, bytes, &plan->arena, &plan->arena_cap);
-    if (e == hipSuccess) e = upload_stream(device, &up);
-    if (e == hipSuccess) e = hipMemcpyAsync(plan->arena, staging, bytes, hipMemcpyHostToDevice, up);
+    if (e == hipSuccess) e = build_stream(device, t, &up);
+    if (e == hipSuccess) e = upload(up, plan->arena, staging, bytes);
     if (e == hipSuccess && sort) {
         hipLaunchKernelGGL(sort_records_kernel, dim3(static_cast<uint32_t>((n_recs + kSortWindow - 1) / kSortWindow)),
                            dim3(kSortWindow / 2), 0, up, static_cast<UniformRec *>(plan->arena), static_cast<uint32_t>(n_recs));
         e = hipGetLastError();
     }
-    // No wait here: the event goes behind the copy, launches wait for it on their stream.
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+    if (e == hipSuccess) e = end_build(plan, t, up, staging, staging_cap);
     if (e != hipSuccess) {
         if (up) (void)hipStreamSynchronize(up); // whatever was queued reads the buffers given back below
         if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -935,19 +1052,9 @@ build_block_plan(int device, const Tuning &t, void *staging, size_t staging_cap,
         delete plan;
         return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("plan upload: ") + hipGetErrorString(e));
     }
-    recycle_after(device, up, staging, staging_cap);
     plan->arena_bytes = bytes;
     plan->uniform_recs = static_cast<const UniformRec *>(plan->arena);
-    plan->chunks_per_rec = static_cast<uint32_t>(len / chunk_bytes);
-    plan->n_uniform = static_cast<uint32_t>(n_recs * plan->chunks_per_rec);
-    plan->uniform_wgs = (plan->n_uniform + static_cast<uint32_t>(t.waves) - 1) / static_cast<uint32_t>(t.waves);
-    plan->info.payload_bytes = n_recs * len;
-    plan->info.vec_descs = n_descs;
-    plan->info.plan_device_bytes = bytes;
-    plan->info.vec_chunks = plan->n_uniform;
-    plan->info.uniform_chunks = plan->n_uniform;
-    plan->info.units_per_lane = static_cast<uint32_t>(t.upl);
-    plan->info.uniform_workgroups = plan->uniform_wgs;
+    describe_blocks(*plan, t, n_recs, len, n_descs);
     *out = plan;
     return NIXL_AMD_OK;
 }
@@ -1247,13 +1354,11 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             delete plan;
             return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipMalloc(plan arena): ") + hipGetErrorString(e));
         }
-        // No wait here either: the event goes behind the copy, launches wait for it on their
-        // stream, and the pinned buffer is recycled once the copy has completed.
         hipStream_t up = nullptr;
-        e = upload_stream(device, &up);
+        e = build_stream(device, t, &up);
         auto *arena = static_cast<uint8_t *>(plan->arena);
         if (e == hipSuccess && total > upload_from)
-            e = hipMemcpyAsync(arena + upload_from, staging, total - upload_from, hipMemcpyHostToDevice, up);
+            e = upload(up, arena + upload_from, staging, total - upload_from);
         if (e == hipSuccess && expand) {
             const uint32_t wgs = static_cast<uint32_t>(std::min<uint64_t>((static_cast<uint64_t>(n_uniform_chunks) + 255) / 256, 1u << 20));
             hipLaunchKernelGGL(expand_runs_kernel, dim3(wgs), dim3(256), 0, up, reinterpret_cast<UniformRec *>(arena + off_uni),
@@ -1262,8 +1367,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
                                n_uniform_chunks, static_cast<uint32_t>(chunk_units * 16u));
             e = hipGetLastError();
         }
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+        if (e == hipSuccess) e = end_build(plan, t, up, staging, staging_cap);
         if (e != hipSuccess) {
             if (up) (void)hipStreamSynchronize(up); // a queued copy still reads the buffer given back below
             if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -1272,7 +1376,6 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             delete plan;
             return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipMemcpy(plan arena): ") + hipGetErrorString(e));
         }
-        recycle_after(device, up, staging, staging_cap);
         plan->arena_bytes = total;
         auto *base = static_cast<uint8_t *>(plan->arena);
         plan->uniform_recs = reinterpret_cast<const UniformRec *>(base + off_uni);
@@ -1432,22 +1535,26 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     const DeviceScope on_device(device);
     HIP_TRY(on_device.status());
 
-    // Destination pattern (cache policy, record order) and source pattern from the index
-    // vectors, while they are copied into the pinned upload buffer.
+    // The index vectors (and run tables) go into a pinned buffer, where the records kernel reads
+    // them: every index is read once, so a copy to the device first would only add its latency.
+    // The records of a few blocks are made right here instead.
     const size_t index_bytes = n * sizeof(int32_t);
+    const bool inlined = fits_inline(n, len, t);
     void *staging = nullptr;
     size_t staging_cap = 0;
     const bool tables = n_src_runs > 1 || n_dst_runs > 1;
     const size_t table_at = (2 * index_bytes + 15) & ~size_t(15); // the run tables follow the index vectors
     const size_t table_bytes = tables ? (n_src_runs + n_dst_runs) * sizeof(nixl_amd_copy_run_t) : 0;
-    const size_t upload_bytes = tables ? table_at + table_bytes : 2 * index_bytes;
-    reap_uploads(device);
-    hipError_t e = upload_cache().get(device, upload_bytes, &staging, &staging_cap);
-    if (e != hipSuccess)
-        return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
-    auto *up_src = static_cast<int32_t *>(staging), *up_dst = up_src + n;
-    std::memcpy(up_src, src_index, index_bytes);
-    std::memcpy(up_dst, dst_index, index_bytes);
+    hipError_t e = hipSuccess;
+    if (!inlined) {
+        reap_uploads(device);
+        e = upload_cache().get(device, table_at + table_bytes, &staging, &staging_cap);
+        if (e != hipSuccess)
+            return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
+        std::memcpy(staging, src_index, index_bytes);
+        std::memcpy(static_cast<int32_t *>(staging) + n, dst_index, index_bytes);
+    }
+    // Destination pattern (cache policy, record order) and source pattern from the index vectors.
     // How many destination steps are regular (one block on in dense lists, or the same step as
     // the one before) and how many source steps go one block on: differences taken modulo 2^32
     // and without a value carried from one iteration to the next, so that the loop vectorises.
@@ -1464,7 +1571,7 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
         regular += (static_cast<uint32_t>(step == 1u) & dst_dense) | static_cast<uint32_t>(step == before);
         src_follows += static_cast<uint32_t>((sv[i] - sv[i - 1]) == 1u) & src_dense;
     }
-    if (tables) {
+    if (tables && !inlined) {
         auto *up_runs = reinterpret_cast<nixl_amd_copy_run_t *>(static_cast<uint8_t *>(staging) + table_at);
         std::memcpy(up_runs, src_runs, n_src_runs * sizeof(nixl_amd_copy_run_t));
         std::memcpy(up_runs + n_src_runs, dst_runs, n_dst_runs * sizeof(nixl_amd_copy_run_t));
@@ -1478,26 +1585,34 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     plan->waves = waves;
     plan->swizzle = swizzle;
     plan->policy = nt ? nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
-    // one arena: the records, then the two index vectors (and run tables) the records are built from
-    const size_t rec_bytes = (n * sizeof(UniformRec) + 255) & ~size_t(255);
+    if (inlined) {
+        const auto address = [](const nixl_amd_copy_run_t *runs, size_t n_runs, uint64_t index) {
+            const auto *run = std::upper_bound(runs, runs + n_runs, index, [](uint64_t i, const nixl_amd_copy_run_t &r) { return i < r.first_index; }) - 1;
+            return run->base + (index - run->first_index) * run->stride;
+        };
+        plan->inline_recs = std::make_unique<InlineRecs>();
+        for (size_t i = 0; i < n; ++i)
+            plan->inline_recs->rec[i] = UniformRec{address(src_runs, n_src_runs, static_cast<uint64_t>(src_index[i])),
+                                                   address(dst_runs, n_dst_runs, static_cast<uint64_t>(dst_index[i]))};
+        describe_blocks(*plan, t, n, len, n);
+        *out = plan;
+        return NIXL_AMD_OK;
+    }
+    const size_t rec_bytes = n * sizeof(UniformRec);
     hipStream_t up = nullptr;
-    e = arena_cache().get(device, rec_bytes + upload_bytes, &plan->arena, &plan->arena_cap);
-    if (e == hipSuccess) e = upload_stream(device, &up);
+    e = arena_cache().get(device, rec_bytes, &plan->arena, &plan->arena_cap);
+    if (e == hipSuccess) e = build_stream(device, t, &up);
     auto *recs = static_cast<UniformRec *>(plan->arena);
-    auto *dev_index = reinterpret_cast<int32_t *>(static_cast<uint8_t *>(plan->arena) + rec_bytes);
-    if (e == hipSuccess) e = hipMemcpyAsync(dev_index, staging, upload_bytes, hipMemcpyHostToDevice, up);
+    const auto *index = static_cast<const int32_t *>(staging);
     if (e == hipSuccess) {
         const dim3 grid(static_cast<uint32_t>((n + 255) / 256));
         if (tables) {
-            const auto *dev_runs =
-                reinterpret_cast<const nixl_amd_copy_run_t *>(reinterpret_cast<const uint8_t *>(dev_index) + table_at);
-            hipLaunchKernelGGL(index_records_runs_kernel, grid, dim3(256), 0, up, recs, dev_index, dev_index + n,
-                               static_cast<uint32_t>(n), dev_runs, static_cast<uint32_t>(n_src_runs), dev_runs + n_src_runs,
-                               static_cast<uint32_t>(n_dst_runs));
+            const auto *runs = reinterpret_cast<const nixl_amd_copy_run_t *>(static_cast<const uint8_t *>(staging) + table_at);
+            hipLaunchKernelGGL(index_records_runs_kernel, grid, dim3(256), 0, up, recs, index, index + n, static_cast<uint32_t>(n),
+                               runs, static_cast<uint32_t>(n_src_runs), runs + n_src_runs, static_cast<uint32_t>(n_dst_runs));
         } else {
-            hipLaunchKernelGGL(index_records_kernel, grid, dim3(256), 0, up, recs, dev_index, dev_index + n,
-                               static_cast<uint32_t>(n), src_runs[0].base, src_runs[0].stride, dst_runs[0].base,
-                               dst_runs[0].stride);
+            hipLaunchKernelGGL(index_records_kernel, grid, dim3(256), 0, up, recs, index, index + n, static_cast<uint32_t>(n),
+                               src_runs[0].base, src_runs[0].stride, dst_runs[0].base, dst_runs[0].stride);
         }
         e = hipGetLastError();
     }
@@ -1506,9 +1621,7 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
                            dim3(kSortWindow / 2), 0, up, recs, static_cast<uint32_t>(n));
         e = hipGetLastError();
     }
-    // No wait here: the event goes behind the kernels, launches wait for it on their stream.
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+    if (e == hipSuccess) e = end_build(plan, t, up, staging, staging_cap);
     if (e != hipSuccess) {
         if (up) (void)hipStreamSynchronize(up); // whatever was queued reads the buffers given back below
         if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -1517,19 +1630,9 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
         delete plan;
         return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("plan upload: ") + hipGetErrorString(e));
     }
-    recycle_after(device, up, staging, staging_cap);
-    plan->arena_bytes = rec_bytes + upload_bytes;
+    plan->arena_bytes = rec_bytes;
     plan->uniform_recs = recs;
-    plan->chunks_per_rec = static_cast<uint32_t>(len / chunk_bytes);
-    plan->n_uniform = static_cast<uint32_t>(n * plan->chunks_per_rec);
-    plan->uniform_wgs = (plan->n_uniform + static_cast<uint32_t>(waves) - 1) / static_cast<uint32_t>(waves);
-    plan->info.payload_bytes = n * len;
-    plan->info.vec_descs = n;
-    plan->info.plan_device_bytes = plan->arena_bytes;
-    plan->info.vec_chunks = plan->n_uniform;
-    plan->info.uniform_chunks = plan->n_uniform;
-    plan->info.units_per_lane = static_cast<uint32_t>(upl);
-    plan->info.uniform_workgroups = plan->uniform_wgs;
+    describe_blocks(*plan, t, n, len, n);
     *out = plan;
     return NIXL_AMD_OK;
 }
@@ -1711,13 +1814,28 @@ nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream) {
     const DeviceScope on_device(plan->device);
     HIP_TRY(on_device.status());
     hipStream_t s = static_cast<hipStream_t>(stream);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
+    if (plan->built_on && plan->launched_valid) {
+        // an earlier launch followed the build: once it has run, so has the build
+        if (hipEventQuery(plan->launched) == hipSuccess)
+            plan->built_on = nullptr;
+        else
+            (void)hipGetLastError();
+    }
+    if (plan->built_on && s == plan->built_on && capture != hipStreamCaptureStatusNone)
+        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_launch: the stream a plan was made on may not be captured at its first launch");
+    if (plan->built_on && s != plan->built_on) {
+        // not where the caller said: from here on the build is one on a stream of its own
+        if (!plan->uploaded) HIP_TRY(hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming));
+        HIP_TRY(hipEventRecord(plan->uploaded, plan->built_on));
+        plan->built_on = nullptr;
+    }
     if (plan->uploaded) {
         hipError_t e = settle_upload(plan, false);
         if (e == hipErrorNotReady) {
             // A stream under graph capture must not be made to depend on work outside the
             // graph: the host waits instead, and the graph holds the launch alone.
-            hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-            if (s && hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
             e = capture == hipStreamCaptureStatusNone ? hipStreamWaitEvent(s, plan->uploaded, 0) : hipErrorNotReady;
             if (e != hipSuccess) {
                 (void)hipGetLastError();
@@ -1726,7 +1844,13 @@ nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream) {
         }
         HIP_TRY(e);
     }
-    if (plan->uniform_wgs) {
+    if (plan->inline_recs) {
+        with_policy(plan->policy, [&]<int POL>() {
+            hipLaunchKernelGGL(copy_inline_kernel<POL>, dim3(plan->n_uniform), dim3(kWaveSize), 0, s, *plan->inline_recs,
+                               plan->chunks_per_rec);
+        });
+        HIP_TRY(hipGetLastError());
+    } else if (plan->uniform_wgs) {
         // One launch per kMaxGrid workgroups.  With the die swizzle each launch's grid is
         // rounded up to a multiple of 8 so that every die owns an equally long slice; surplus
         // workgroups exit at once.
@@ -1767,8 +1891,6 @@ nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream) {
     }
     // What nixl_amd_copy_plan_destroy looks at.  A stream under graph capture gets no event: the
     // graph's owner keeps the plan alive for as long as the graph may be replayed.
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (s && hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
     if (capture == hipStreamCaptureStatusNone) {
         if (!plan->launched) HIP_TRY(hipEventCreateWithFlags(&plan->launched, hipEventDisableTiming));
         HIP_TRY(hipEventRecord(plan->launched, s));
@@ -1804,10 +1926,16 @@ nixl_amd_copy_plan_destroy(nixl_amd_copy_plan_t *plan) {
             return nixl_amd_fail(NIXL_AMD_ERR_BUSY, "plan_destroy: a launch of this plan has not completed");
         }
     }
+    if (plan->built_on && !plan->launched_valid) {
+        // never launched: the build itself may still run, behind whatever is in front of it
+        recycle_after(plan->device, plan->built_on, plan->staging, plan->staging_cap, plan->arena, plan->arena_cap);
+        plan->staging = plan->arena = nullptr;
+    }
     (void)settle_upload(plan, true); // the arena and the upload buffer go back only when nothing writes or reads them
     if (plan->launched) (void)hipEventDestroy(plan->launched);
     if (plan->ev0) (void)hipEventDestroy(plan->ev0);
     if (plan->ev1) (void)hipEventDestroy(plan->ev1);
+    if (plan->staging) upload_cache().put(plan->device, plan->staging, plan->staging_cap);
     if (plan->arena) arena_cache().put(plan->device, plan->arena, plan->arena_cap);
     delete plan;
     return NIXL_AMD_OK;

@@ -248,6 +248,14 @@ nixlHipEngine::pickStream(int device) const {
     return streams_[idx];
 }
 
+bool
+nixlHipEngine::chooseStream(int device, nixlHipReqH &req, nixl_amd_copy_tuning_t &tuning) const {
+    req.stream = pickStream(device);
+    tuning = tuning_;
+    if (!useExternalStream_) tuning.stream = req.stream;
+    return req.stream || useExternalStream_;
+}
+
 nixl_amd_hip::WorkerPool *
 nixlHipEngine::prepPool() const {
     std::call_once(prepPoolOnce_, [this] {
@@ -634,7 +642,12 @@ nixlHipEngine::prepXfer(const nixl_xfer_op_t &operation,
         if (!pass.blocks) {
             (void)nixl_amd_copy_records_abandon(buffer);
         } else {
-            const int rc = nixl_amd_copy_plan_create_from_records(buffer, n_records, local[0].len, device, &tuning_, &facts, &req->plan);
+            nixl_amd_copy_tuning_t tuning;
+            if (!chooseStream(device, *req, tuning)) {
+                (void)nixl_amd_copy_records_abandon(buffer);
+                return NIXL_ERR_BACKEND;
+            }
+            const int rc = nixl_amd_copy_plan_create_from_records(buffer, n_records, local[0].len, device, &tuning, &facts, &req->plan);
             if (rc == NIXL_AMD_OK)
                 path = "blocks";
             else if (rc != NIXL_AMD_ERR_INVALID) { // INVALID: not on 128-byte lines, say; the general lowering judges
@@ -651,15 +664,15 @@ nixlHipEngine::prepXfer(const nixl_xfer_op_t &operation,
         bytes = 0;
         const nixl_status_t st = lowerGeneral(write, local, remote, lowered.get(), device, bytes);
         if (st != NIXL_SUCCESS) return st;
-        if (nixl_amd_copy_plan_create(lowered.get(), static_cast<size_t>(n), device, &tuning_, &req->plan) != NIXL_AMD_OK) {
+        nixl_amd_copy_tuning_t tuning;
+        if (!chooseStream(device, *req, tuning)) return NIXL_ERR_BACKEND;
+        if (nixl_amd_copy_plan_create(lowered.get(), static_cast<size_t>(n), device, &tuning, &req->plan) != NIXL_AMD_OK) {
             NIXL_ERROR << "HIP backend: " << nixl_amd_last_error();
             return NIXL_ERR_BACKEND;
         }
     }
     req->device = device;
     req->bytes = bytes;
-    req->stream = pickStream(device);
-    if (!req->stream && !useExternalStream_) return NIXL_ERR_BACKEND;
 
     const auto t_done = std::chrono::steady_clock::now();
     const auto us = [](auto from, auto to) { return std::chrono::duration<double, std::micro>(to - from).count(); };
@@ -744,16 +757,16 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
     req->bytes = count * len;
     const int src = write ? 0 : 1, dst = 1 - src;
     const int *index_of[2] = {local_indices, remote_indices};
+    nixl_amd_copy_tuning_t tuning;
+    if (!chooseStream(device, *req, tuning)) return NIXL_ERR_BACKEND;
     const int rc = nixl_amd_copy_plan_create_indexed_runs(tables[src].data(), tables[src].size(), index_of[src],
                                                           tables[dst].data(), tables[dst].size(), index_of[dst], count, len,
-                                                          device, &tuning_, &req->plan);
+                                                          device, &tuning, &req->plan);
     if (rc == NIXL_AMD_ERR_INVALID) return NIXL_ERR_NOT_SUPPORTED; // shape or alignment: the descriptor path handles it
     if (rc != NIXL_AMD_OK) {
         NIXL_ERROR << "HIP backend: " << nixl_amd_last_error();
         return NIXL_ERR_BACKEND;
     }
-    req->stream = pickStream(device);
-    if (!req->stream && !useExternalStream_) return NIXL_ERR_BACKEND;
     handle = req.release();
     return NIXL_SUCCESS;
 }

@@ -865,6 +865,51 @@ def test_lists_without_a_stride_stay_on_the_device(cuda, op, count):
         agent.close()
 
 
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 1500])
+@pytest.mark.parametrize("n_runs", [1, 3])
+@pytest.mark.parametrize("named", ["", "same", "other", "busy"])
+def test_block_plans_inline_and_on_the_callers_stream(cuda, n, n_runs, named):
+    """Indexed plans around the count up to which their records travel as kernel arguments, over
+    lists of one run and of several, made for no stream, for the one they are launched on, for
+    another one, and for one with work in front; launched twice, and once made and destroyed
+    without a launch."""
+    import torch
+    rng = np.random.default_rng(n * 10 + n_runs)
+    blk, pool = 8192, 1800
+    src = torch.randint(0, 256, (pool, blk), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros_like(src)
+    at, to = (rng.permutation(pool)[:n].astype(np.int32) for _ in range(2))
+    cuts = [pool * r // n_runs for r in range(n_runs + 1)]
+
+    def runs(t):
+        return (_lib.CopyRun * n_runs)(*[_lib.CopyRun(t.data_ptr() + a * blk, blk, a, b - a) for a, b in zip(cuts, cuts[1:])])
+
+    lib = _lib.kernels()
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    busy = torch.zeros(64 << 20, dtype=torch.float32, device=cuda)
+    for launched in (True, False):
+        if named == "busy":
+            with torch.cuda.stream(stream):
+                for _ in range(4):
+                    busy.add_(1.0)
+        tuning = _lib.CopyTuning(stream=None if not named else other.cuda_stream if named == "other" else stream.cuda_stream)
+        plan = ctypes.c_void_p()
+        assert lib.nixl_amd_copy_plan_create_indexed_runs(runs(src), n_runs, at.ctypes.data, runs(dst), n_runs, to.ctypes.data, n, blk, 0,
+                                                          ctypes.byref(tuning), ctypes.byref(plan)) == 0, _lib.kernels_error()
+        for _ in range(2 if launched else 0):
+            want = torch.zeros_like(dst)
+            want[torch.from_numpy(to).to(cuda).long()] = src[torch.from_numpy(at).to(cuda).long()]
+            dst.zero_()
+            torch.cuda.synchronize()
+            assert lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+            torch.cuda.synchronize()
+            assert torch.equal(dst, want)
+            src ^= 0x3C
+        assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+    torch.cuda.synchronize()
+
+
 def test_golden_descriptor_list(cuda):
     """Committed vector (tests/golden/kv_descs.npz): mixed aligned / unaligned / empty
     descriptors, destination pre-filled with a canary byte."""
