@@ -21,7 +21,9 @@
 //       chunk touches (span[m] = {first, last} for the m-th listed chunk; src[j], dst[j], prefix[j] = first unit of
 //       descriptor j, prefix[n] = total) in a per-wave LDS slice and walks them.
 //   Descriptors that are not 16-byte aligned in src, dst and len are cut into byte-range
-//   work items handled by a third, byte-exact kernel.
+//   work items of at most 4 KiB handled by a third, byte-exact kernel; of a long one whose
+//   source and destination lie alike inside their 128-byte lines only the ends are, and the
+//   whole chunks between them join the virtual stream.
 //   Lists of equal-length, line-aligned descriptors of whole chunks (KV blocks) take none of
 //   these steps: one pass writes their records, or, when the request is two index vectors
 //   into two strided runs, a kernel writes them from the indices on the device.  Arenas and
@@ -44,7 +46,8 @@ namespace {
 
 constexpr int kMixedWaves = 4; // waves per workgroup of the mixed and byte-path kernels
 constexpr int kMixedThreads = kWaveSize * kMixedWaves;
-constexpr uint32_t kGenericItemBytes = 16384; // byte-path work item size
+constexpr int kGenericLoads = 4; // 16-byte loads a lane keeps in flight for a byte-path work item
+constexpr uint32_t kGenericItemBytes = kWaveSize * kGenericLoads * 16; // reach of an item, from the destination line it starts in
 constexpr int kMaxLdsDescs = 64; // descriptors a wave stages in LDS for one chunk
 constexpr int kNumXcd = 8; // accelerator dies; workgroup i is dispatched to die i % 8
 
@@ -75,11 +78,11 @@ constexpr int kPieceUnitsShift = 56;
 // Lengths of the entries of a list that stays on the device: what the piece kernel is made for.
 constexpr uint32_t kListMinBytes = 128, kListMaxBytes = 8176;
 
+// A byte range of at most kGenericItemBytes, 16 bytes a record like a piece: the length, less
+// one, rides in the top bytes of the two addresses (low eight bits in dst's).
 struct GenericItem {
-    uint64_t src;
-    uint64_t dst;
-    uint32_t len; // <= kGenericItemBytes
-    uint32_t pad;
+    uint64_t src_len; // src | (len - 1) >> 8 << 56
+    uint64_t dst_len; // dst | ((len - 1) & 255) << 56
 };
 
 // 16-byte vector in the global address space, so that accesses compile to
@@ -315,44 +318,58 @@ copy_mixed_kernel(MixedArgs a) {
     }
 }
 
-struct __attribute__((packed, aligned(1))) unaligned16 {
-    uint32_t w[4];
-};
+// One wavefront per byte-range work item; correct for any alignment and length.  An item ends
+// at most kGenericItemBytes behind the destination line it starts in (the plan cuts them so), so
+// its body of whole 16-byte units is at most kGenericLoads instructions wide with lane 0 of each
+// on a destination line, as in the piece kernel; loads take their 16 bytes from any address.
+// All loads of an item (body, up to 15 head and 15 tail bytes) are in flight before the first
+// store: what bounds a list of a few thousand such descriptors is that round trip and the
+// number of waves sharing it, not bytes (3000 descriptors of up to 64 KiB, 18 MB: 7 us; with items
+// of 16 KiB whose lanes had one load in flight a 64 KiB descriptor alone was 64 of those trips
+// in a row on four waves).
+using v4u_any = __attribute__((__vector_size__(4 * sizeof(unsigned)), __aligned__(1))) unsigned;
 
-// One wavefront per byte-range work item; correct for any alignment and length.
 __global__ void __launch_bounds__(kMixedThreads)
 copy_generic_kernel(const GenericItem *items, uint32_t n_items) {
+    using any_cptr = const __attribute__((address_space(1))) v4u_any *;
+    using byte_ptr = __attribute__((address_space(1))) uint8_t *;
+    using byte_cptr = const __attribute__((address_space(1))) uint8_t *;
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
     const uint32_t wave = threadIdx.x / kWaveSize;
     const uint32_t n_waves = gridDim.x * kMixedWaves;
     for (uint32_t it = uniform(blockIdx.x * kMixedWaves + wave); it < n_items; it += n_waves) {
-        const uint64_t src = uniform64(items[it].src);
-        const uint64_t dst = uniform64(items[it].dst);
-        const uint32_t len = uniform(items[it].len);
-        const uint8_t *s = reinterpret_cast<const uint8_t *>(src);
-        uint8_t *d = reinterpret_cast<uint8_t *>(dst);
-
-        // Head: bytes until dst is 16-byte aligned (at most 15).
-        uint32_t head = static_cast<uint32_t>((16u - (dst & 15u)) & 15u);
-        if (head > len) head = len;
-        if (lane < head) d[lane] = s[lane];
+        const uint64_t src_len = uniform64(items[it].src_len), dst_len = uniform64(items[it].dst_len);
+        constexpr uint64_t kAddress = (1ull << kPieceUnitsShift) - 1ull;
+        const uint64_t src = src_len & kAddress, dst = dst_len & kAddress;
+        const uint32_t len = (static_cast<uint32_t>(src_len >> kPieceUnitsShift) << 8 | static_cast<uint32_t>(dst_len >> kPieceUnitsShift)) + 1u;
+        // bytes until dst is 16-byte aligned (at most 15), whole units, the rest
+        const uint32_t head = min(static_cast<uint32_t>(-dst) & 15u, len);
         const uint32_t body = (len - head) / 16u;
-        const uint8_t *sb = s + head;
-        uint4 *db = reinterpret_cast<uint4 *>(d + head);
-        if (((src + head) & 15u) == 0) {
-            const uint4 *sv = reinterpret_cast<const uint4 *>(sb);
-            for (uint32_t i = lane; i < body; i += kWaveSize)
-                db[i] = sv[i];
-        } else {
-            const unaligned16 *sv = reinterpret_cast<const unaligned16 *>(sb);
-            for (uint32_t i = lane; i < body; i += kWaveSize) {
-                const unaligned16 t = sv[i];
-                db[i] = make_uint4(t.w[0], t.w[1], t.w[2], t.w[3]);
-            }
-        }
         const uint32_t done = head + body * 16u;
         const uint32_t tail = len - done; // < 16
-        if (lane < tail) d[done + lane] = s[done + lane];
+        const uint32_t shift = (static_cast<uint32_t>(dst + head) >> 4) & 7u; // body's offset inside its line
+
+        uint8_t first = 0, last = 0;
+        if (lane < head) first = *(byte_cptr)(src + lane);
+        if (lane < tail) last = *(byte_cptr)(src + done + lane);
+        v4u v[kGenericLoads];
+        if (body) {
+            // unconditional, as in the piece kernel: a lane outside the body re-reads its first
+            // or last unit
+#pragma unroll
+            for (int k = 0; k < kGenericLoads; ++k) {
+                const uint32_t at = k * kWaveSize + lane;
+                const uint32_t u = min(at < shift ? 0u : at - shift, body - 1);
+                v[k] = *(any_cptr)(src + head + u * 16ull);
+            }
+#pragma unroll
+            for (int k = 0; k < kGenericLoads; ++k) {
+                const uint32_t at = k * kWaveSize + lane;
+                if (at >= shift && at - shift < body) store16<kPolNtNt>(dst + head + (at - shift) * 16ull, v[k]);
+            }
+        }
+        if (lane < head) *(byte_ptr)(dst + lane) = first;
+        if (lane < tail) *(byte_ptr)(dst + done + lane) = last;
     }
 }
 
@@ -1146,11 +1163,12 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     // start on a 128-byte line, go to the piece kernel: measured faster there (fewer lines
     // split between wavefronts); line-aligned long descriptors stream best in 1 KiB chunks.
     constexpr uint64_t kPieceMinUnits = 16, kPieceMaxDescUnits = 512;
+    constexpr uint64_t kSplitFromBytes = 64 * 1024; // at least two chunks of the largest size besides a first line
     vsrc.reserve(n);
     vdst.reserve(n);
     vprefix.reserve(n + 1);
     pieces.reserve(n);
-    uint64_t units = 0, payload = 0, n_generic_descs = 0, n_piece_descs = 0;
+    uint64_t units = 0, payload = 0, n_generic_descs = 0, n_piece_descs = 0, n_split = 0;
     for (size_t i = 0; i < n; ++i) {
         const nixl_amd_copy_desc_t &d = descs[i];
         if (d.len == 0) continue;
@@ -1181,12 +1199,33 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             units += d.len / 16u;
         } else {
             ++n_generic_descs;
-            for (uint64_t off = 0; off < d.len; off += kGenericItemBytes) {
-                GenericItem it{};
-                it.src = d.src + off;
-                it.dst = d.dst + off;
-                it.len = static_cast<uint32_t>(std::min<uint64_t>(kGenericItemBytes, d.len - off));
-                items.push_back(it);
+            if (((d.src + d.len) | (d.dst + d.len)) >> kPieceUnitsShift)
+                return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create: address beyond 2^56");
+            // every item but the first starts on a destination line
+            const auto byte_items = [&](uint64_t off, uint64_t end) {
+                while (off < end) {
+                    const uint64_t reach = kGenericItemBytes - ((d.dst + off) & 127u);
+                    const uint32_t len = static_cast<uint32_t>(std::min<uint64_t>(reach, end - off));
+                    items.push_back(GenericItem{(d.src + off) | static_cast<uint64_t>((len - 1) >> 8) << kPieceUnitsShift,
+                                                (d.dst + off) | static_cast<uint64_t>((len - 1) & 255u) << kPieceUnitsShift});
+                    off += len;
+                }
+            };
+            // A long one whose two ends lie at the same place inside their lines (tensors whose
+            // size is no multiple of 16) is whole chunks but for its first line and its last
+            // chunk: only those go byte by byte.
+            const uint64_t head = (0 - d.dst) & 127u;
+            if (d.len >= kSplitFromBytes && ((d.src ^ d.dst) & 127u) == 0) {
+                const uint64_t body = (d.len - head) / (chunk_units * 16u) * (chunk_units * 16u);
+                if (head) byte_items(0, head);
+                vsrc.push_back(d.src + head);
+                vdst.push_back(d.dst + head);
+                vprefix.push_back(units);
+                units += body / 16u;
+                ++n_split;
+                byte_items(head + body, d.len);
+            } else {
+                byte_items(0, d.len);
             }
         }
     }
@@ -1405,7 +1444,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->generic_wgs = wgs_for(plan->n_generic, kMixedWaves, true);
 
     plan->info.payload_bytes = payload;
-    plan->info.vec_descs = nv + n_piece_descs;
+    plan->info.vec_descs = nv - n_split + n_piece_descs;
     plan->info.generic_descs = n_generic_descs;
     plan->info.plan_device_bytes = plan->arena_bytes;
     plan->info.vec_chunks = n_chunks;

@@ -143,6 +143,24 @@ def test_unaligned_brute_force(cuda):
     assert info.generic_descs > 0
 
 
+@pytest.mark.parametrize("length", [1, 15, 16, 17, 127, 4095, 4096, 4097, 65535, 65536, 65536 + 1040, 200001])
+def test_byte_path_items_and_split_ends(cuda, length):
+    """Byte-aligned descriptors around the edges of a work item (4 KiB from the line the
+    destination starts in) and of the split that sends the whole chunks of long ones through the
+    chunk kernel: destinations at the first, second and last bytes of a line, sources at the same
+    place in theirs, at the same 16-byte place, or anywhere."""
+    import torch
+    pitch = (length + 255) // 128 * 128 + 128
+    src_off, dst_off = [], []
+    for da in (0, 1, 15, 16, 112, 113, 127):
+        for sa in (da, (da + 16) % 128, (da + 1) % 128, 127 - da):
+            src_off.append(len(src_off) * pitch + sa)
+            dst_off.append(len(dst_off) * pitch + da)
+    half = (len(src_off) * pitch + 4095) // 4096 * 4096
+    dst_off = [d + half for d in dst_off]
+    _check_against_oracle(torch, cuda, 2 * half, src_off, dst_off, [length] * len(src_off), seed=length)
+
+
 @pytest.mark.parametrize("seed", [1, 2, 3])
 def test_random_mixture_of_every_descriptor_class(cuda, seed):
     """One request that mixes everything the planner tells apart: lengths log-uniform from
