@@ -48,10 +48,16 @@ block_exclusive_scan(V v, V *wave_sums, V &total) {
 }
 
 // ---- layout (kernels/layout.cu:31-138) ----------------------------------------------------
-// grid = R source ranks x chunks of kLayoutTokens tokens, one token per thread; LDS: E + R
+// grid = R source ranks x chunks of blockDim.x tokens, one token per thread; LDS: E + R
 // counters per workgroup, added to the (zeroed) outputs at the end.  Integer sums: the
-// result does not depend on the order of the additions.
+// result does not depend on the order of the additions.  A rank of at most kLayoutWhole tokens
+// and kLayoutWholeSelections selections is one chunk, whose counters are the result: nothing to
+// clear and nothing to add (8 x 1024 tokens top-4: 6.1 -> 4.6 us, 4 x 333 top-6: 6.7 -> 4.1).
+// Beyond, the LDS atomics of a single workgroup cost more than a second launch: 8 x 1024 top-8
+// 5.7 us in chunks, 7.6 whole.
 constexpr int kLayoutTokens = 256;
+constexpr int kLayoutWhole = 1024;
+constexpr int kLayoutWholeSelections = 4096;
 
 __global__ void __launch_bounds__(256)
 zero_ints_kernel(int *__restrict__ a, size_t na, int *__restrict__ b, size_t nb) {
@@ -60,7 +66,7 @@ zero_ints_kernel(int *__restrict__ a, size_t na, int *__restrict__ b, size_t nb)
     if (i < nb) b[i] = 0;
 }
 
-__global__ void __launch_bounds__(kLayoutTokens)
+__global__ void __launch_bounds__(kLayoutWhole)
 layout_kernel(const int32_t *__restrict__ topk_idx,
               int *__restrict__ per_rank,
               int *__restrict__ per_expert,
@@ -70,9 +76,9 @@ layout_kernel(const int32_t *__restrict__ topk_idx,
               int R,
               int E) {
     extern __shared__ int counters[]; // [E] experts, then [R] ranks
-    const int chunks = (T + kLayoutTokens - 1) / kLayoutTokens;
+    const int chunks = (T + blockDim.x - 1) / blockDim.x;
     const int src = blockIdx.x / chunks, El = E / R;
-    const int t = (blockIdx.x % chunks) * kLayoutTokens + threadIdx.x;
+    const int t = (blockIdx.x % chunks) * blockDim.x + threadIdx.x;
     for (int i = threadIdx.x; i < E + R; i += blockDim.x)
         counters[i] = 0;
     __syncthreads();
@@ -119,6 +125,13 @@ layout_kernel(const int32_t *__restrict__ topk_idx,
         }
     }
     __syncthreads();
+    if (chunks == 1) {
+        for (int i = threadIdx.x; i < E; i += blockDim.x)
+            per_expert[static_cast<size_t>(src) * E + i] = counters[i];
+        for (int i = threadIdx.x; i < R; i += blockDim.x)
+            per_rank[static_cast<size_t>(src) * R + i] = counters[E + i];
+        return;
+    }
     for (int i = threadIdx.x; i < E; i += blockDim.x)
         if (counters[i]) atomicAdd(&per_expert[static_cast<size_t>(src) * E + i], counters[i]);
     for (int i = threadIdx.x; i < R; i += blockDim.x)
@@ -168,7 +181,8 @@ ht_scan_kernel(const uint8_t *__restrict__ in_rank,
 // not wait for each other), then scans its own.  A thread writes the R positions of its
 // token as one run, a wave consecutive runs.  The positions are stored non-temporally: the
 // row kernel that follows reads them from every XCD, and lines left dirty in the writer's L2
-// made those reads slow (+45 us on 8 x 4096 tokens).  grid = R * ceil(T / kScanThreads).
+// made those reads slow (+45 us on 8 x 4096 tokens).  grid = R * ceil(T / kScanThreads), and one
+// more workgroup where that also does part 2 (notify_from_flags).
 constexpr int kPackedScanRanks = 8;
 constexpr int kPackedScanMaxTokens = 65535;
 
@@ -191,6 +205,11 @@ packed_hits(const uint8_t *flags, int t, int R) {
             hit.lo |= static_cast<unsigned long long>(((f >> (8 * d)) & 0xffu) != 0) << (16 * d);
             hit.hi |= static_cast<unsigned long long>(((f >> (8 * (d + 4))) & 0xffu) != 0) << (16 * d);
         }
+    } else if (R == 4) {
+        const uint32_t f = *reinterpret_cast<const uint32_t *>(flags + static_cast<size_t>(t) * 4);
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+            hit.lo |= static_cast<unsigned long long>(((f >> (8 * d)) & 0xffu) != 0) << (16 * d);
     } else {
         for (int d = 0; d < R; ++d) {
             const unsigned long long bit = flags[static_cast<size_t>(t) * R + d] != 0;
@@ -203,16 +222,144 @@ packed_hits(const uint8_t *flags, int t, int R) {
     return hit;
 }
 
+// ---- notify, part 2: receive-side prefix over source ranks, aligned per-expert counts
+// (kernels/nixl_ep_ht.cu:295-314) and where each destination's rows start in the
+// concatenated outputs.  One workgroup; total_of(r, d) = tokens of source r that go to
+// destination d. ------------------------------------------------------------------------------
+struct HtNotifyOut {
+    const int *per_expert;
+    int *recv_rank_prefix;
+    int *recv_expert_count;
+    long long *row_offset;
+    int *recv_counter;
+    int alignment;
+};
+
+template<typename TotalOf>
+__device__ __forceinline__ void
+notify_prefix(const HtNotifyOut &o, int R, int E, const TotalOf &total_of) {
+    __shared__ int wave_sums[kScanThreads / kWaveSize];
+    const int tid = threadIdx.x;
+    // Loads go out eight at a time before anything depends on them: issued one by one, the
+    // round trips of this single workgroup add up to most of the kernel's time.
+    constexpr int kBatch = 8;
+    for (int e = tid; e < E; e += kScanThreads) {
+        int n = 0;
+        for (int r0 = 0; r0 < R; r0 += kBatch) {
+            int v[kBatch];
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j)
+                v[j] = r0 + j < R ? o.per_expert[static_cast<size_t>(r0 + j) * E + e] : 0;
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j)
+                n += v[j];
+        }
+        o.recv_expert_count[e] = (n + o.alignment - 1) / o.alignment * o.alignment;
+    }
+    // R <= kScanThreads: thread d owns destination d
+    int total = 0;
+    if (tid < R) {
+        for (int r0 = 0; r0 < R; r0 += kBatch) {
+            int v[kBatch];
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j)
+                v[j] = r0 + j < R ? total_of(r0 + j, tid) : 0;
+#pragma unroll
+            for (int j = 0; j < kBatch; ++j)
+                if (r0 + j < R) {
+                    total += v[j];
+                    o.recv_rank_prefix[tid * R + r0 + j] = total;
+                }
+        }
+        if (o.recv_counter) o.recv_counter[tid] = total;
+    }
+    if (o.row_offset) {
+        // exclusive prefix of the per-destination totals in 64 bits
+        long long incl = total;
+        const int lane = tid & (kWaveSize - 1), wave = tid / kWaveSize;
+#pragma unroll
+        for (int off = 1; off < kWaveSize; off <<= 1) {
+            const long long up = __shfl_up(incl, off);
+            if (lane >= off) incl += up;
+        }
+        // wave totals fit in 32 bits each only if R * T does; check_ht bounds R * T by 2^30
+        if (lane == kWaveSize - 1) wave_sums[wave] = static_cast<int>(incl);
+        __syncthreads();
+        long long before = 0;
+        for (int w = 0; w < wave; ++w)
+            before += wave_sums[w];
+        if (tid < R) o.row_offset[tid + 1] = before + incl;
+        if (tid == 0) o.row_offset[0] = 0;
+    }
+}
+
+__global__ void __launch_bounds__(kScanThreads)
+ht_prefix_kernel(const int *__restrict__ channel_prefix, HtNotifyOut o, int R, int E, int C) {
+    notify_prefix(o, R, E, [&](int r, int d) { return channel_prefix[(static_cast<size_t>(r) * R + d) * C + (C - 1)]; });
+}
+
+// The same without a launch of its own, for up to kNotifyFlags flags and 8 ranks: one more
+// workgroup behind those of the scan counts the flags itself instead of waiting for their
+// counts.  Both steps take 5.3 us instead of 7.8 at 4 x 333 tokens, called again and again on the
+// same flags, and 6.1 instead of 8.1 at 8 x 512 (32 768 flags).  With more flags that one
+// workgroup is what the call waits for, the sooner since flags that another kernel has just
+// written come from memory: 8 x 1024, 7.9 us instead of 8.5 on the same flags but 11.7 instead of
+// 5.4 + 4.0 behind the layout kernel; 8 x 4096, 15 instead of 9.1.
+constexpr int kNotifyFlags = 32768; // R * T * R
+constexpr int kNotifyPerLane = 16; // tokens a lane counts at a time, their loads together
+
+__device__ __forceinline__ void
+notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int R, int E) {
+    __shared__ int hits[kPackedScanRanks * kPackedScanRanks]; // [source][destination]
+    constexpr int kWaves = kScanThreads / kWaveSize, kUnit = kWaveSize * kNotifyPerLane;
+    const int tid = threadIdx.x, lane = tid & (kWaveSize - 1);
+    if (tid < kPackedScanRanks * kPackedScanRanks) hits[tid] = 0;
+    __syncthreads();
+    const int units = (T + kUnit - 1) / kUnit;
+    for (int u = tid / kWaveSize; u < R * units; u += kWaves) {
+        const int r = u / units, t0 = (u % units) * kUnit + lane;
+        const uint8_t *flags = in_rank + static_cast<size_t>(r) * T * R;
+        PackedCounts h[kNotifyPerLane];
+#pragma unroll
+        for (int j = 0; j < kNotifyPerLane; ++j) {
+            const int t = t0 + j * kWaveSize;
+            h[j] = t < T ? packed_hits(flags, t, R) : PackedCounts{0, 0};
+        }
+        PackedCounts sum{0, 0}; // at most 1024 to a field
+#pragma unroll
+        for (int j = 0; j < kNotifyPerLane; ++j) {
+            sum.lo += h[j].lo;
+            sum.hi += h[j].hi;
+        }
+#pragma unroll
+        for (int off = kWaveSize / 2; off > 0; off >>= 1) {
+            sum.lo += __shfl_xor(sum.lo, off);
+            sum.hi += __shfl_xor(sum.hi, off);
+        }
+        if (lane < R) atomicAdd(&hits[r * kPackedScanRanks + lane], packed_field(sum, lane));
+    }
+    __syncthreads();
+    notify_prefix(o, R, E, [&](int r, int d) { return hits[r * kPackedScanRanks + d]; });
+}
+
+// NOTIFY: the launch has that workgroup.
+template<bool NOTIFY>
 __global__ void __launch_bounds__(kScanThreads)
 ht_scan_packed_kernel(const uint8_t *__restrict__ in_rank,
                       int *__restrict__ send_head,
                       int *__restrict__ channel_prefix,
                       int T,
                       int R,
-                      int C) {
+                      int C,
+                      int E,
+                      HtNotifyOut notify) {
     constexpr int kWaves = kScanThreads / kWaveSize;
     __shared__ PackedCounts wave_sums[kWaves], wave_before[kWaves];
     const int chunks = (T + kScanThreads - 1) / kScanThreads;
+    if (NOTIFY && static_cast<int>(blockIdx.x) == R * chunks) {
+        notify_from_flags(in_rank, notify, T, R, E);
+        return;
+    }
     const int src = blockIdx.x / chunks, base = (blockIdx.x % chunks) * kScanThreads;
     const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), wave = tid / kWaveSize;
     const int per_channel = (T + C - 1) / C;
@@ -302,75 +449,6 @@ ht_scan_packed_kernel(const uint8_t *__restrict__ in_rank,
                 channel_prefix[(static_cast<size_t>(src) * R + d) * C + c] = packed_field(total, d);
 }
 
-// ---- notify, part 2: receive-side prefix over source ranks, aligned per-expert counts
-// (kernels/nixl_ep_ht.cu:295-314) and where each destination's rows start in the
-// concatenated outputs.  One workgroup. ------------------------------------------------------
-__global__ void __launch_bounds__(kScanThreads)
-ht_prefix_kernel(const int *__restrict__ channel_prefix,
-                 const int *__restrict__ per_expert,
-                 int *__restrict__ recv_rank_prefix,
-                 int *__restrict__ recv_expert_count,
-                 long long *__restrict__ row_offset,
-                 int *__restrict__ recv_counter,
-                 int R,
-                 int E,
-                 int C,
-                 int alignment) {
-    __shared__ int wave_sums[kScanThreads / kWaveSize];
-    const int tid = threadIdx.x;
-    // Loads go out eight at a time before anything depends on them: issued one by one, the
-    // round trips of this single workgroup add up to most of the kernel's time.
-    constexpr int kBatch = 8;
-    for (int e = tid; e < E; e += kScanThreads) {
-        int n = 0;
-        for (int r0 = 0; r0 < R; r0 += kBatch) {
-            int v[kBatch];
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j)
-                v[j] = r0 + j < R ? per_expert[static_cast<size_t>(r0 + j) * E + e] : 0;
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j)
-                n += v[j];
-        }
-        recv_expert_count[e] = (n + alignment - 1) / alignment * alignment;
-    }
-    // R <= kScanThreads: thread d owns destination d
-    int total = 0;
-    if (tid < R) {
-        for (int r0 = 0; r0 < R; r0 += kBatch) {
-            int v[kBatch];
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j)
-                v[j] = r0 + j < R ? channel_prefix[(static_cast<size_t>(r0 + j) * R + tid) * C + (C - 1)] : 0;
-#pragma unroll
-            for (int j = 0; j < kBatch; ++j)
-                if (r0 + j < R) {
-                    total += v[j];
-                    recv_rank_prefix[tid * R + r0 + j] = total;
-                }
-        }
-        if (recv_counter) recv_counter[tid] = total;
-    }
-    if (row_offset) {
-        // exclusive prefix of the per-destination totals in 64 bits
-        long long incl = total;
-        const int lane = tid & (kWaveSize - 1), wave = tid / kWaveSize;
-#pragma unroll
-        for (int off = 1; off < kWaveSize; off <<= 1) {
-            const long long up = __shfl_up(incl, off);
-            if (lane >= off) incl += up;
-        }
-        // wave totals fit in 32 bits each only if R * T does; check_ht bounds R * T by 2^30
-        if (lane == kWaveSize - 1) wave_sums[wave] = static_cast<int>(incl);
-        __syncthreads();
-        long long before = 0;
-        for (int w = 0; w < wave; ++w)
-            before += wave_sums[w];
-        if (tid < R) row_offset[tid + 1] = before + incl;
-        if (tid == 0) row_offset[0] = 0;
-    }
-}
-
 struct HtDims {
     int R, T, H, K, E;
 };
@@ -381,77 +459,96 @@ recv_row(const int *prefix, const int *send_head, const long long *row_offset, c
     return row_offset[dst] + seg + send_head[(static_cast<size_t>(r) * d.T + t) * d.R + dst];
 }
 
-constexpr int kMaxHtRanks = 1024;
 constexpr int kHtBatch = 8; // row loads a lane keeps in flight in combine
 
-// The rows of token (r, t) at the destination ranks that hold it, in ascending rank order,
-// gathered into LDS by the first wave (64 destinations per step, compacted with a ballot).
-// Every thread of the workgroup calls this; the return value is the number of rows.
-__device__ __forceinline__ int
-collect_rows(const uint8_t *in_rank,
-             const int *prefix,
-             const int *send_head,
-             const long long *row_offset,
-             const HtDims &d,
-             int r,
-             int t,
-             long long *rows,
-             int *dsts,
-             int *n_rows) {
-    if (threadIdx.x < kWaveSize) {
-        const int lane = threadIdx.x;
-        const size_t tok = static_cast<size_t>(r) * d.T + t;
-        int n = 0;
-        for (int d0 = 0; d0 < d.R; d0 += kWaveSize) {
-            const int dst = d0 + lane;
-            bool hit = dst < d.R && in_rank[tok * d.R + dst] != 0;
-            long long row = hit ? recv_row(prefix, send_head, row_offset, d, r, t, dst) : 0;
-            // the handle comes from the caller: a row outside the destination's range is dropped
-            if (hit && (row < row_offset[dst] || row >= row_offset[dst + 1])) hit = false;
-            const unsigned long long m = __ballot(hit);
-            if (hit) {
-                const int p = n + __popcll(m & ((1ull << lane) - 1ull));
-                rows[p] = row;
-                dsts[p] = dst;
-            }
-            n += __popcll(m);
+// The rows of token (r, t) at destinations d0 .. d0 + 63, found by one wave, lane = destination
+// - d0: no LDS and no barrier, so that waves of a workgroup need not serve the same token.
+// EAGER: positions are loaded beside the flags instead of behind them.
+struct WaveRows {
+    unsigned long long hits; // destinations that hold the token
+    long long mine; // the row at this lane's
+};
+
+template<bool EAGER>
+__device__ __forceinline__ WaveRows
+wave_rows(const uint8_t *in_rank,
+          const int *prefix,
+          const int *send_head,
+          const long long *row_offset,
+          const HtDims &d,
+          int r,
+          int t,
+          int d0) {
+    const int dst = d0 + (threadIdx.x & (kWaveSize - 1));
+    const size_t tok = static_cast<size_t>(r) * d.T + t;
+    bool hit = false;
+    long long row = 0;
+    // the handle comes from the caller: a row outside the destination's range is dropped
+    if (EAGER) {
+        if (dst < d.R) {
+            const uint8_t flag = in_rank[tok * d.R + dst];
+            const int head = send_head[tok * d.R + dst], seg = r == 0 ? 0 : prefix[dst * d.R + r - 1];
+            const long long lo = row_offset[dst], hi = row_offset[dst + 1];
+            row = lo + seg + head;
+            hit = flag != 0 && row >= lo && row < hi;
         }
-        if (lane == 0) *n_rows = n;
+    } else {
+        hit = dst < d.R && in_rank[tok * d.R + dst] != 0;
+        if (hit) {
+            row = recv_row(prefix, send_head, row_offset, d, r, t, dst);
+            hit = row >= row_offset[dst] && row < row_offset[dst + 1];
+        }
     }
-    __syncthreads();
-    return *n_rows;
+    return {__ballot(hit), row};
+}
+
+// Row of the lowest destination in `hits`, which leaves the set.
+__device__ __forceinline__ long long
+next_row(const WaveRows &w, unsigned long long &hits) {
+    const int lane = __builtin_ctzll(hits);
+    hits &= hits - 1;
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(w.mine), lane);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(w.mine >> 32), lane);
+    return static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo);
 }
 
 // ---- dispatch (result of kernels/nixl_ep_ht.cu:1109-1243) -------------------------------------
-// Rows: grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x
-// of them.  Narrow workgroups (one wave) measured fastest for this write-dominated scatter.
-// Dynamic LDS: R * 12 bytes (rows, then destination ranks).
-constexpr int kHtDispatchLanes = 64;
+// Rows, scales and metadata in one launch (ht_dispatch_kernel below); these are its three parts.
+//
+// Rows: a wave owns 1 KiB of a row (`parts` waves a row), holds it in registers and stores it to
+// every row of the token.  Bound by the writes.  The loads are ordinary ones, since a layer's
+// input is usually still in the last-level cache that its producer filled, and the stores carry
+// device scope: against non-temporal loads and stores 8 x 4096 x 7168 bf16 (5.23 rows a token, inputs of
+// other calls in between) takes 469 us instead of 547, 8 x 1024 x 4096 (3.38) 49.5 instead of
+// 53; non-temporal stores behind ordinary loads 554 and 52, the other way round 502 and 49.4.
+struct HtRows {
+    uint16_t *recv_x;
+    const uint16_t *x;
+    const uint8_t *in_rank;
+    const int *prefix;
+    const int *send_head;
+    const long long *row_offset;
+    HtDims d;
+    int parts;
+    uint32_t first; // piece the first row workgroup of the launch starts at
+};
 
-__global__ void __launch_bounds__(1024)
-ht_dispatch_kernel(uint16_t *__restrict__ recv_x,
-                   const uint16_t *__restrict__ x,
-                   const uint8_t *__restrict__ in_rank,
-                   const int *__restrict__ prefix,
-                   const int *__restrict__ send_head,
-                   const long long *__restrict__ row_offset,
-                   HtDims d,
-                   int parts) {
-    extern __shared__ long long rows[]; // [R] rows, then [R] int destination ranks
-    int *dsts = reinterpret_cast<int *>(rows + d.R);
-    __shared__ int n_rows;
-    const int tid = threadIdx.x;
-    const int token = blockIdx.x / parts, part = blockIdx.x % parts;
-    const int r = token / d.T, t = token % d.T;
-    const size_t tok = static_cast<size_t>(r) * d.T + t;
-    const int col = part * blockDim.x + tid;
-    const bool active = col < d.H / 8;
+__device__ __forceinline__ void
+dispatch_piece(const HtRows &a, uint32_t piece) {
+    const uint32_t token = piece / a.parts, part = piece % a.parts;
+    if (token >= static_cast<uint32_t>(a.d.R) * a.d.T) return;
+    const int r = token / a.d.T, t = token % a.d.T;
+    const int col = part * kWaveSize + (threadIdx.x & (kWaveSize - 1));
+    const bool active = col < a.d.H / 8;
     uint4 v = make_uint4(0, 0, 0, 0);
-    if (active) v = ld16_nt(reinterpret_cast<const uint4 *>(x + tok * d.H) + col);
-    const int n = collect_rows(in_rank, prefix, send_head, row_offset, d, r, t, rows, dsts, &n_rows);
-    if (!active) return;
-    for (int i = 0; i < n; ++i)
-        st16_nt(reinterpret_cast<uint4 *>(recv_x + static_cast<size_t>(rows[i]) * d.H) + col, v);
+    if (active) v = *(reinterpret_cast<const uint4 *>(a.x + static_cast<size_t>(token) * a.d.H) + col);
+    for (int d0 = 0; d0 < a.d.R; d0 += kWaveSize) {
+        const WaveRows w = wave_rows<true>(a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, r, t, d0);
+        for (unsigned long long hits = w.hits; hits;) {
+            const long long row = next_row(w, hits);
+            if (active) st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * a.d.H) + col, v);
+        }
+    }
 }
 
 // Per-row metadata: rebased top-k indices, weights of the local selections, source rank and
@@ -463,22 +560,32 @@ constexpr int kHtMetaThreads = 256;
 
 // VEC: selections moved four at a time and the (rank, token) pair in one store; the host
 // picks it when K is a multiple of 4 and every pointer is 16-byte aligned.
-template <bool VEC>
-__global__ void __launch_bounds__(kHtMetaThreads)
-ht_meta_kernel(int32_t *__restrict__ recv_topk_idx,
-               float *__restrict__ recv_topk_weights,
-               int32_t *__restrict__ recv_src_meta,
-               const int32_t *__restrict__ topk_idx,
-               const float *__restrict__ topk_weights,
-               const uint8_t *__restrict__ in_rank,
-               const int *__restrict__ prefix,
-               const int *__restrict__ send_head,
-               const long long *__restrict__ row_offset,
-               HtDims d) {
+struct HtMeta {
+    int32_t *recv_topk_idx;
+    float *recv_topk_weights;
+    int32_t *recv_src_meta;
+    const int32_t *topk_idx;
+    const float *topk_weights;
+};
+
+template<bool VEC>
+__device__ __forceinline__ void
+meta_block(const HtMeta &m,
+           const uint8_t *__restrict__ in_rank,
+           const int *__restrict__ prefix,
+           const int *__restrict__ send_head,
+           const long long *__restrict__ row_offset,
+           const HtDims &d,
+           uint32_t block) {
+    int32_t *__restrict__ recv_topk_idx = m.recv_topk_idx;
+    float *__restrict__ recv_topk_weights = m.recv_topk_weights;
+    int32_t *__restrict__ recv_src_meta = m.recv_src_meta;
+    const int32_t *__restrict__ topk_idx = m.topk_idx;
+    const float *__restrict__ topk_weights = m.topk_weights;
     const int blocks_per_pair = (d.T + kHtMetaThreads - 1) / kHtMetaThreads;
-    const int pair = blockIdx.x / blocks_per_pair;
+    const int pair = block / blocks_per_pair;
     const int r = pair / d.R, dst = pair % d.R;
-    const int t = (blockIdx.x % blocks_per_pair) * kHtMetaThreads + threadIdx.x;
+    const int t = (block % blocks_per_pair) * kHtMetaThreads + threadIdx.x;
     if (t >= d.T) return;
     const size_t tok = static_cast<size_t>(r) * d.T + t;
     if (!in_rank[tok * d.R + dst]) return;
@@ -532,25 +639,34 @@ constexpr int kHtScaleTokens = 64;
 constexpr int kHtScaleTile = 64;
 constexpr int kHtScaleThreads = 256;
 
-__global__ void __launch_bounds__(kHtScaleThreads)
-ht_row_scales_kernel(uint32_t *__restrict__ recv_scales,
-                     const uint32_t *__restrict__ scales,
-                     const uint8_t *__restrict__ in_rank,
-                     const int *__restrict__ prefix,
-                     const int *__restrict__ send_head,
-                     const long long *__restrict__ row_offset,
-                     HtDims d,
-                     int S,
-                     long long rank_stride,
-                     long long token_stride,
-                     long long scale_stride,
-                     int wide) {
+struct HtScales {
+    uint32_t *recv;
+    const uint32_t *scales;
+    int S;
+    int wide; // S is a multiple of 4 and recv is 16-byte aligned
+    long long rank_stride;
+    long long token_stride;
+    long long scale_stride;
+};
+
+__device__ __forceinline__ void
+scales_block(const HtScales &a,
+             const uint8_t *__restrict__ in_rank,
+             const int *__restrict__ prefix,
+             const int *__restrict__ send_head,
+             const long long *__restrict__ row_offset,
+             const HtDims &d,
+             uint32_t block) {
+    uint32_t *__restrict__ recv_scales = a.recv;
+    const uint32_t *__restrict__ scales = a.scales;
+    const int S = a.S, wide = a.wide;
+    const long long rank_stride = a.rank_stride, token_stride = a.token_stride, scale_stride = a.scale_stride;
     __shared__ long long rows[kHtScaleTokens];
     __shared__ uint32_t tile[kHtScaleTokens][kHtScaleTile + 1]; // odd pitch: no bank conflicts either way
     const int blocks_per_pair = (d.T + kHtScaleTokens - 1) / kHtScaleTokens;
-    const int pair = blockIdx.x / blocks_per_pair;
+    const int pair = block / blocks_per_pair;
     const int r = pair / d.R, dst = pair % d.R;
-    const int t0 = (blockIdx.x % blocks_per_pair) * kHtScaleTokens;
+    const int t0 = (block % blocks_per_pair) * kHtScaleTokens;
     const int tid = threadIdx.x;
     if (tid < kHtScaleTokens) {
         const int t = t0 + tid;
@@ -609,11 +725,49 @@ ht_row_scales_kernel(uint32_t *__restrict__ recv_scales,
     }
 }
 
-// ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
-// grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x of them.
-constexpr int kHtCombineLanes = 128;
+// One launch for the three: workgroups of the scales and of the metadata first, whose short
+// writes then run beside the rows', four pieces of rows to a workgroup behind them.  Launched one
+// after the other, the three took 14.6 us at 4 x 333 x 4096 fp8 (now 6.9), 157 at 8 x 2048 x 7168
+// fp8 (145, and 132 with the loads and stores described at the rows), 55.3 at 8 x 1024 x 4096
+// bf16 (52.9 and 49.5).  A launch holds fewer than 2^24 such workgroups; a call of more is launched part
+// by part.
+constexpr int kHtThreads = 256;
+constexpr int kHtWaves = kHtThreads / kWaveSize;
+constexpr long long kHtMaxGrid = (1ll << 24) - 1;
+static_assert(kHtThreads == kHtMetaThreads && kHtThreads == kHtScaleThreads);
 
-__global__ void __launch_bounds__(1024)
+template<bool VEC, bool SCALES>
+__global__ void __launch_bounds__(kHtThreads)
+ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint32_t meta_blocks) {
+    uint32_t block = blockIdx.x;
+    if (SCALES) {
+        if (block < scale_blocks) {
+            scales_block(sc, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, block);
+            return;
+        }
+        block -= scale_blocks;
+    }
+    if (block < meta_blocks) {
+        meta_block<VEC>(m, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, block);
+        return;
+    }
+    dispatch_piece(a, a.first + (block - meta_blocks) * kHtWaves + uniform(threadIdx.x / kWaveSize));
+}
+
+// ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
+// grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x of them,
+// every wave for itself.  Two forms: up to kHtCombineEager values of output, four waves a
+// workgroup and positions loaded beside the flags (EAGER), which shortens the chain of loads
+// (8 x 1024 x 4096: 52.8 -> 48.8 us, 2 x 4096 x 4096: 40.4 -> 36.2, 4 x 1500 x 4096: 36.6 ->
+// 32.7 against a workgroup whose first wave finds the rows for both).  Beyond, that many rows
+// in flight cost bandwidth (8 x 2048 x 7168: 247 us, 8 x 4096: 494): one wave a workgroup and
+// positions behind the flags, 231 and 457, is what those calls took with the shared look-up as
+// well (8 x 1024 x 7168: 112 -> 109, 4 x 4096: 181 -> 175).
+constexpr int kHtCombineEagerLanes = 256;
+constexpr long long kHtCombineEager = 1ll << 25;
+
+template<bool EAGER>
+__global__ void __launch_bounds__(kHtCombineEagerLanes)
 ht_combine_kernel(uint16_t *__restrict__ combined,
                   float *__restrict__ combined_w,
                   const uint16_t *__restrict__ x,
@@ -626,9 +780,6 @@ ht_combine_kernel(uint16_t *__restrict__ combined,
                   const long long *__restrict__ row_offset,
                   HtDims d,
                   int parts) {
-    __shared__ long long rows[kMaxHtRanks];
-    __shared__ int dsts[kMaxHtRanks];
-    __shared__ int n_rows;
     const int tid = threadIdx.x;
     const int token = blockIdx.x / parts, part = blockIdx.x % parts;
     const int r = token / d.T, t = token % d.T;
@@ -641,7 +792,6 @@ ht_combine_kernel(uint16_t *__restrict__ combined,
         if (bias0) b0 = ld16_nt(reinterpret_cast<const uint4 *>(bias0 + tok * d.H) + col);
         if (bias1) b1 = ld16_nt(reinterpret_cast<const uint4 *>(bias1 + tok * d.H) + col);
     }
-    const int n = collect_rows(in_rank, prefix, send_head, row_offset, d, r, t, rows, dsts, &n_rows);
     float acc[8];
     {
         const uint32_t u0[4] = {b0.x, b0.y, b0.z, b0.w}, u1[4] = {b1.x, b1.y, b1.z, b1.w};
@@ -652,30 +802,34 @@ ht_combine_kernel(uint16_t *__restrict__ combined,
         }
     }
     float wsum = 0.f;
-    for (int i0 = 0; i0 < n; i0 += kHtBatch) {
-        // all loads of the batch first, then the additions in ascending rank order
-        uint4 v[kHtBatch];
-        float wv[kHtBatch];
+    for (int d0 = 0; d0 < d.R; d0 += kWaveSize) {
+        const WaveRows w = wave_rows<EAGER>(in_rank, prefix, send_head, row_offset, d, r, t, d0);
+        for (unsigned long long hits = w.hits; hits;) {
+            // all loads of the batch first, then the additions in ascending rank order
+            const int n = __popcll(hits);
+            uint4 v[kHtBatch];
+            float wv[kHtBatch];
 #pragma unroll
-        for (int j = 0; j < kHtBatch; ++j) {
-            v[j] = make_uint4(0, 0, 0, 0);
-            wv[j] = 0.f;
-            if (i0 + j < n) {
-                const long long row = rows[i0 + j];
-                if (active) v[j] = ld16_nt(reinterpret_cast<const uint4 *>(x + static_cast<size_t>(row) * d.H) + col);
-                if (topk_weights && weights) wv[j] = topk_weights[row * d.K + tid];
+            for (int j = 0; j < kHtBatch; ++j) {
+                v[j] = make_uint4(0, 0, 0, 0);
+                wv[j] = 0.f;
+                if (j < n) {
+                    const long long row = next_row(w, hits);
+                    if (active) v[j] = ld16_nt(reinterpret_cast<const uint4 *>(x + static_cast<size_t>(row) * d.H) + col);
+                    if (topk_weights && weights) wv[j] = topk_weights[row * d.K + tid];
+                }
             }
-        }
 #pragma unroll
-        for (int j = 0; j < kHtBatch; ++j) {
-            if (i0 + j >= n) continue;
-            const uint32_t u[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
+            for (int j = 0; j < kHtBatch; ++j) {
+                if (j >= n) continue;
+                const uint32_t u[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                acc[2 * c] += bf16_lo_to_f32(u[c]);
-                acc[2 * c + 1] += bf16_hi_to_f32(u[c]);
+                for (int c = 0; c < 4; ++c) {
+                    acc[2 * c] += bf16_lo_to_f32(u[c]);
+                    acc[2 * c + 1] += bf16_hi_to_f32(u[c]);
+                }
+                wsum += wv[j];
             }
-            wsum += wv[j];
         }
     }
     if (active) {
@@ -774,6 +928,13 @@ nixl_amd_ep_get_dispatch_layout(const int32_t *topk_idx,
     const size_t lds = static_cast<size_t>(num_experts + num_ranks) * sizeof(int);
     if (lds > 48 * 1024) return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "get_dispatch_layout: too many experts");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (num_tokens <= kLayoutWhole && num_tokens * num_topk <= kLayoutWholeSelections) {
+        hipLaunchKernelGGL(layout_kernel, dim3(static_cast<unsigned>(num_ranks)), dim3(round_up_wave(num_tokens)), lds, s, topk_idx,
+                           num_tokens_per_rank, num_tokens_per_expert, is_token_in_rank, num_tokens, num_topk, num_ranks,
+                           num_experts);
+        HIP_TRY(hipGetLastError());
+        return NIXL_AMD_OK;
+    }
     // the counts are accumulated with atomics; cleared by a kernel, not a memset, so that a
     // caller may capture the call into a graph
     const size_t n_rank = static_cast<size_t>(num_ranks) * num_ranks, n_expert = static_cast<size_t>(num_ranks) * num_experts;
@@ -813,19 +974,25 @@ nixl_amd_ep_ht_notify_dispatch(const uint8_t *is_token_in_rank,
     hipStream_t s = static_cast<hipStream_t>(stream);
     // the packed kernel reads 8 flag bytes and writes 16-byte pieces at a time
     const bool aligned = reinterpret_cast<uintptr_t>(is_token_in_rank) % 8 == 0 && reinterpret_cast<uintptr_t>(send_head) % 16 == 0;
-    if (num_ranks <= kPackedScanRanks && num_tokens <= kPackedScanMaxTokens && aligned)
-        hipLaunchKernelGGL(ht_scan_packed_kernel,
-                           dim3(static_cast<unsigned>(num_ranks) * ((num_tokens + kScanThreads - 1) / kScanThreads)),
-                           dim3(kScanThreads), 0, s,
-                           is_token_in_rank, send_head, gbl_channel_prefix_matrix, num_tokens, num_ranks, num_channels);
-    else
+    const HtNotifyOut notify{num_tokens_per_expert, recv_gbl_rank_prefix_sum, recv_expert_count,
+                             reinterpret_cast<long long *>(recv_row_offset), recv_counter, expert_alignment};
+    if (num_ranks <= kPackedScanRanks && num_tokens <= kPackedScanMaxTokens && aligned) {
+        const bool one_launch = static_cast<long long>(num_ranks) * num_ranks * num_tokens <= kNotifyFlags;
+        hipLaunchKernelGGL(one_launch ? ht_scan_packed_kernel<true> : ht_scan_packed_kernel<false>,
+                           dim3(static_cast<unsigned>(num_ranks) * ((num_tokens + kScanThreads - 1) / kScanThreads) + one_launch),
+                           dim3(kScanThreads), 0, s, is_token_in_rank, send_head, gbl_channel_prefix_matrix, num_tokens, num_ranks,
+                           num_channels, num_experts, notify);
+        if (one_launch) {
+            HIP_TRY(hipGetLastError());
+            return NIXL_AMD_OK;
+        }
+    } else {
         hipLaunchKernelGGL(ht_scan_kernel, dim3(static_cast<unsigned>(num_ranks) * num_ranks), dim3(kScanThreads), 0, s,
                            is_token_in_rank, send_head, gbl_channel_prefix_matrix, num_tokens, num_ranks, num_channels);
+    }
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(ht_prefix_kernel, dim3(1), dim3(kScanThreads), 0, s, gbl_channel_prefix_matrix,
-                       num_tokens_per_expert, recv_gbl_rank_prefix_sum, recv_expert_count,
-                       reinterpret_cast<long long *>(recv_row_offset), recv_counter, num_ranks, num_experts,
-                       num_channels, expert_alignment);
+    hipLaunchKernelGGL(ht_prefix_kernel, dim3(1), dim3(kScanThreads), 0, s, gbl_channel_prefix_matrix, notify, num_ranks, num_experts,
+                       num_channels);
     HIP_TRY(hipGetLastError());
     return NIXL_AMD_OK;
 }
@@ -874,41 +1041,47 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
     if (x_scales && (scale_rank_stride < 0 || scale_token_stride < 0 || scale_hidden_stride < 0))
         return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_dispatch: negative scale stride");
     const HtDims d{num_ranks, num_tokens, static_cast<int>(row_halves), num_topk, num_experts};
-    const int lanes = round_up_wave(d.H / 8);
-    const int parts = (lanes + kHtDispatchLanes - 1) / kHtDispatchLanes;
+    const int parts = round_up_wave(d.H / 8) / kWaveSize;
     if (static_cast<long long>(num_ranks) * num_tokens * parts >= (1ll << 31))
         return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_dispatch: too many tokens");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(ht_dispatch_kernel, dim3(static_cast<unsigned>(num_ranks) * num_tokens * parts), dim3(kHtDispatchLanes),
-                       static_cast<size_t>(num_ranks) * 12, s, static_cast<uint16_t *>(recv_x),
-                       static_cast<const uint16_t *>(x), is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
-                       reinterpret_cast<const long long *>(recv_row_offset), d, parts);
-    HIP_TRY(hipGetLastError());
-    if (x_scales) {
-        const long long blocks = static_cast<long long>(num_ranks) * num_ranks * ((num_tokens + kHtScaleTokens - 1) / kHtScaleTokens);
-        if (blocks >= (1ll << 31)) return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_dispatch: too many ranks and tokens");
-        hipLaunchKernelGGL(ht_row_scales_kernel, dim3(static_cast<unsigned>(blocks)), dim3(kHtScaleThreads), 0, s,
-                           static_cast<uint32_t *>(recv_x_scales), static_cast<const uint32_t *>(x_scales), is_token_in_rank,
-                           recv_gbl_rank_prefix_sum, send_head, reinterpret_cast<const long long *>(recv_row_offset), d,
-                           num_scales, static_cast<long long>(scale_rank_stride), static_cast<long long>(scale_token_stride),
-                           static_cast<long long>(scale_hidden_stride),
-                           (num_scales % 4 == 0 && reinterpret_cast<uintptr_t>(recv_x_scales) % 16 == 0) ? 1 : 0);
+    const long long scale_blocks =
+        x_scales ? static_cast<long long>(num_ranks) * num_ranks * ((num_tokens + kHtScaleTokens - 1) / kHtScaleTokens) : 0;
+    const long long meta_blocks = recv_topk_idx || recv_src_meta ?
+        static_cast<long long>(num_ranks) * num_ranks * ((num_tokens + kHtMetaThreads - 1) / kHtMetaThreads) : 0;
+    if (scale_blocks >= (1ll << 31) || meta_blocks >= (1ll << 31))
+        return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_dispatch: too many ranks and tokens");
+    const long long *offsets = reinterpret_cast<const long long *>(recv_row_offset);
+    const int *prefix = recv_gbl_rank_prefix_sum;
+    HtRows rows{static_cast<uint16_t *>(recv_x), static_cast<const uint16_t *>(x), is_token_in_rank, prefix, send_head, offsets, d,
+                parts, 0};
+    const HtMeta meta{recv_topk_idx, recv_topk_weights, recv_src_meta, topk_idx, topk_weights};
+    const HtScales sc{static_cast<uint32_t *>(recv_x_scales), static_cast<const uint32_t *>(x_scales), num_scales,
+                      num_scales % 4 == 0 && reinterpret_cast<uintptr_t>(recv_x_scales) % 16 == 0, scale_rank_stride,
+                      scale_token_stride, scale_hidden_stride};
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(recv_topk_idx) | reinterpret_cast<uintptr_t>(recv_topk_weights) |
+                           reinterpret_cast<uintptr_t>(recv_src_meta) | reinterpret_cast<uintptr_t>(topk_idx) |
+                           reinterpret_cast<uintptr_t>(topk_weights);
+    const bool vec = num_topk % 4 == 0 && bits % 16 == 0;
+    const long long pieces = static_cast<long long>(num_ranks) * num_tokens * parts;
+    const long long row_blocks = (pieces + kHtWaves - 1) / kHtWaves;
+    const auto kernel = x_scales ? (vec ? ht_dispatch_kernel<true, true> : ht_dispatch_kernel<false, true>)
+                                 : (vec ? ht_dispatch_kernel<true, false> : ht_dispatch_kernel<false, false>);
+    const auto launch = [&](long long n_scale, long long n_meta, long long n_row) -> int {
+        const long long blocks = n_scale + n_meta + n_row;
+        if (blocks == 0) return NIXL_AMD_OK;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kHtThreads), 0, s, rows, meta, sc,
+                           static_cast<uint32_t>(n_scale), static_cast<uint32_t>(n_meta));
         HIP_TRY(hipGetLastError());
+        return NIXL_AMD_OK;
+    };
+    if (scale_blocks + meta_blocks + row_blocks <= kHtMaxGrid) return launch(scale_blocks, meta_blocks, row_blocks);
+    for (long long at = 0; at < row_blocks; at += kHtMaxGrid) {
+        rows.first = static_cast<uint32_t>(at * kHtWaves);
+        if (const int status = launch(0, 0, std::min(kHtMaxGrid, row_blocks - at))) return status;
     }
-    if (recv_topk_idx || recv_src_meta) {
-        const long long blocks = static_cast<long long>(num_ranks) * num_ranks * ((num_tokens + kHtMetaThreads - 1) / kHtMetaThreads);
-        if (blocks >= (1ll << 31)) return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_dispatch: too many ranks and tokens");
-        const dim3 grid(static_cast<unsigned>(blocks));
-        const uintptr_t bits = reinterpret_cast<uintptr_t>(recv_topk_idx) | reinterpret_cast<uintptr_t>(recv_topk_weights) |
-                               reinterpret_cast<uintptr_t>(recv_src_meta) | reinterpret_cast<uintptr_t>(topk_idx) |
-                               reinterpret_cast<uintptr_t>(topk_weights);
-        const auto kernel = (num_topk % 4 == 0 && bits % 16 == 0) ? ht_meta_kernel<true> : ht_meta_kernel<false>;
-        hipLaunchKernelGGL(kernel, grid, dim3(kHtMetaThreads), 0, s, recv_topk_idx, recv_topk_weights, recv_src_meta,
-                           topk_idx, topk_weights, is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
-                           reinterpret_cast<const long long *>(recv_row_offset), d);
-    }
-    HIP_TRY(hipGetLastError());
-    return NIXL_AMD_OK;
+    if (const int status = launch(scale_blocks, 0, 0)) return status;
+    return launch(0, meta_blocks, 0);
 }
 
 int
@@ -956,15 +1129,14 @@ nixl_amd_ep_ht_combine(void *combined_x,
     if (!combined_x || !x || !is_token_in_rank || !recv_gbl_rank_prefix_sum || !send_head || !recv_row_offset)
         return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_combine: null pointer argument");
     const HtDims d{num_ranks, num_tokens, hidden, num_topk, num_ranks};
-    // Two-wave workgroups over 2 KiB pieces of a row: more workgroups resident, so that the
-    // look-ups of some overlap the row loads of others (485 us against 510 for a workgroup per
-    // row at 8 x 4096 x 7168; one wave: 575, four: 514).
-    const int lanes = std::min(kHtCombineLanes, round_up_wave(hidden / 8));
-    const int parts = (round_up_wave(hidden / 8) + lanes - 1) / lanes;
+    // the lanes of a row dealt evenly to workgroups of at most four waves, or of one
+    const bool eager = static_cast<long long>(num_ranks) * num_tokens * hidden <= kHtCombineEager;
+    const int row_lanes = round_up_wave(hidden / 8), most = eager ? kHtCombineEagerLanes : kWaveSize;
+    const int parts = (row_lanes + most - 1) / most, lanes = round_up_wave((row_lanes + parts - 1) / parts);
     if (static_cast<long long>(num_ranks) * num_tokens * parts >= (1ll << 31))
         return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_combine: too many tokens");
-    hipLaunchKernelGGL(ht_combine_kernel, dim3(static_cast<unsigned>(num_ranks) * num_tokens * parts), dim3(lanes),
-                       0, static_cast<hipStream_t>(stream), static_cast<uint16_t *>(combined_x), combined_topk_weights,
+    hipLaunchKernelGGL(eager ? ht_combine_kernel<true> : ht_combine_kernel<false>,
+                       dim3(static_cast<unsigned>(num_ranks) * num_tokens * parts), dim3(lanes), 0, static_cast<hipStream_t>(stream), static_cast<uint16_t *>(combined_x), combined_topk_weights,
                        static_cast<const uint16_t *>(x), topk_weights, static_cast<const uint16_t *>(bias_0),
                        static_cast<const uint16_t *>(bias_1), is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
                        reinterpret_cast<const long long *>(recv_row_offset), d, parts);

@@ -476,6 +476,16 @@ def test_ht_pipeline_matches_oracle(cuda, shape):
         assert np.array_equal(comb_w.cpu().numpy(), want_w)
 
 
+# 4096 selections a rank are counted by one workgroup, 4104 and 1025 tokens by several; 32 768
+# flags are counted beside the scan, 32 832 behind it; 66 ranks take two steps of 64 in every
+# wave, and 33 lanes leave a wave half idle; 33.7 million values are combined in the form for
+# large calls.
+@pytest.mark.parametrize("shape", [(8, 512, 128, 8, 16, 4, 1), (8, 513, 128, 8, 16, 4, 1), (1, 1024, 256, 4, 4, 2, 1),
+                                   (2, 1025, 256, 2, 4, 2, 1), (66, 5, 264, 4, 66, 2, 1), (4, 1030, 8192, 2, 8, 4, 1)])
+def test_ht_pipeline_at_the_edges_of_its_launch_forms(cuda, shape):
+    test_ht_pipeline_matches_oracle(cuda, shape)
+
+
 @pytest.mark.parametrize("scale_dtype", [np.float32, np.int32])
 def test_ht_dispatch_fp8_rows_with_scales(cuda, scale_dtype):
     """The (x, x_scales) form of normal-mode dispatch.  The reference's test passes fp8 rows
