@@ -883,6 +883,46 @@ def test_lists_without_a_stride_stay_on_the_device(cuda, op, count):
         agent.close()
 
 
+@pytest.mark.parametrize("count", [65535, 65536, 65537, 131072 + 300])
+def test_listed_requests_lowered_in_slices(cuda, count):
+    """Pairs against device-resident lists around the number one launch of the records kernel
+    takes: every byte against the per-descriptor oracle, a bad pair refused wherever it lies."""
+    import torch
+    from nixl_amd.agent import NixlError
+    rng = np.random.default_rng(count)
+    n, slot = count + 5, 288
+    lens = rng.choice([128, 144, 256], n).astype(np.int64)
+    half = n * slot
+    so = np.arange(n) * slot + rng.integers(0, 3, n) * 16
+    do = half + rng.permutation(n) * slot + rng.integers(0, 3, n) * 16
+    host = rng.integers(0, 256, 2 * half, dtype=np.uint8)
+    mem = torch.from_numpy(host.copy()).to(cuda)
+    torch.cuda.synchronize()
+    agent = nixl_agent(f"slices{count}", nixl_agent_config(backends=("HIP",)))
+    try:
+        agent.register_memory([mem])
+        local, remote = (agent.prep_xfer_dlist(who, np.stack([np.uint64(mem.data_ptr()) + o.astype(np.uint64), lens.astype(np.uint64),
+                                                              np.zeros(n, np.uint64)], 1), "VRAM")
+                         for o, who in ((so, ""), (do, agent.name)))
+        idx = rng.permutation(n)[:count].astype(np.int32)
+        req = agent.make_prepped_xfer("WRITE", local, idx, remote, idx)
+        state = agent.transfer(req)
+        while state == "PROC":
+            state = agent.check_xfer_state(req)
+        assert state == "DONE"
+        assert np.array_equal(mem.cpu().numpy(), ko.copy_descs(host, so[idx], do[idx], lens[idx]))
+        req.release()
+        for at in (0, min(65536, count - 1), count - 1):
+            bad = idx.copy()
+            bad[at] = n
+            with pytest.raises(NixlError):
+                agent.make_prepped_xfer("WRITE", local, bad, remote, idx)
+        for h in (local, remote):
+            h.release()
+    finally:
+        agent.close()
+
+
 @pytest.mark.parametrize("n", [1, 127, 128, 129, 1500])
 @pytest.mark.parametrize("n_runs", [1, 3])
 @pytest.mark.parametrize("named", ["", "same", "other", "busy"])
