@@ -481,7 +481,8 @@ struct ListTotals {
 
 constexpr int kListThreads = 256;
 // Pairs a launch: while it reads them over the bus the host copies the next ones into the pinned
-// buffer.  262 144 pairs made, posted and waited for: 443 us in one launch, 382 in four.
+// buffer.  262 144 pairs made, posted and waited for: 443 us in one launch, 382 in four, the
+// same in eight.
 constexpr size_t kListSlice = 65536;
 static_assert(kListSlice % kListThreads == 0);
 
@@ -1599,38 +1600,42 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
         std::memcpy(staging, src_index, index_bytes);
         std::memcpy(static_cast<int32_t *>(staging) + n, dst_index, index_bytes);
     }
-    // Destination pattern (cache policy, record order) and source pattern from the index vectors.
-    // How many destination steps are regular (one block on in dense lists, or the same step as
-    // the one before) and how many source steps go one block on: differences taken modulo 2^32
-    // and without a value carried from one iteration to the next, so that the loop vectorises.
-    uint32_t regular = 0, src_follows = 0; // n < 2^31
-    const uint32_t dst_dense = dst_all_dense ? 1u : 0u, src_dense = src_all_dense ? 1u : 0u;
-    const auto *sv = reinterpret_cast<const uint32_t *>(src_index);
-    const auto *dv = reinterpret_cast<const uint32_t *>(dst_index);
-    if (n > 1) {
-        regular += ((dv[1] - dv[0]) == 1u) & dst_dense;
-        src_follows += ((sv[1] - sv[0]) == 1u) & src_dense;
-    }
-    for (size_t i = 2; i < n; ++i) {
-        const uint32_t step = dv[i] - dv[i - 1], before = dv[i - 1] - dv[i - 2];
-        regular += (static_cast<uint32_t>(step == 1u) & dst_dense) | static_cast<uint32_t>(step == before);
-        src_follows += static_cast<uint32_t>((sv[i] - sv[i - 1]) == 1u) & src_dense;
-    }
     if (tables && !inlined) {
         auto *up_runs = reinterpret_cast<nixl_amd_copy_run_t *>(static_cast<uint8_t *>(staging) + table_at);
         std::memcpy(up_runs, src_runs, n_src_runs * sizeof(nixl_amd_copy_run_t));
         std::memcpy(up_runs + n_src_runs, dst_runs, n_dst_runs * sizeof(nixl_amd_copy_run_t));
     }
-    const bool scattered = !(n == 1 || 2 * static_cast<uint64_t>(regular) >= n - 1);
-    const bool sort = scattered && sort_scatter != 2 && 2 * static_cast<uint64_t>(src_follows) >= n - 1 && n >= kSortWindow;
-
     auto *plan = new nixl_amd_copy_plan();
     plan->device = device;
     plan->upl = upl;
     plan->waves = waves;
     plan->swizzle = swizzle;
-    plan->policy = nt ? nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
+    // Destination pattern (cache policy, record order) and source pattern from the index vectors.
+    // How many destination steps are regular (one block on in dense lists, or the same step as
+    // the one before) and how many source steps go one block on: differences taken modulo 2^32
+    // and without a value carried from one iteration to the next, so that the loop vectorises.
+    // Sets the policy and says whether the records are to be sorted.
+    const auto study_pattern = [&] {
+        uint32_t regular = 0, src_follows = 0; // n < 2^31
+        const uint32_t dst_dense = dst_all_dense ? 1u : 0u, src_dense = src_all_dense ? 1u : 0u;
+        const auto *sv = reinterpret_cast<const uint32_t *>(src_index);
+        const auto *dv = reinterpret_cast<const uint32_t *>(dst_index);
+        if (n > 1) {
+            regular += ((dv[1] - dv[0]) == 1u) & dst_dense;
+            src_follows += ((sv[1] - sv[0]) == 1u) & src_dense;
+        }
+        for (size_t i = 2; i < n; ++i) {
+            const uint32_t step = dv[i] - dv[i - 1], before = dv[i - 1] - dv[i - 2];
+            regular += (static_cast<uint32_t>(step == 1u) & dst_dense) | static_cast<uint32_t>(step == before);
+            src_follows += static_cast<uint32_t>((sv[i] - sv[i - 1]) == 1u) & src_dense;
+        }
+        const bool scattered = !(n == 1 || 2 * static_cast<uint64_t>(regular) >= n - 1);
+        const bool sort = scattered && sort_scatter != 2 && 2 * static_cast<uint64_t>(src_follows) >= n - 1 && n >= kSortWindow;
+        plan->policy = nt ? nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
+        return sort;
+    };
     if (inlined) {
+        (void)study_pattern();
         const auto address = [](const nixl_amd_copy_run_t *runs, size_t n_runs, uint64_t index) {
             const auto *run = std::upper_bound(runs, runs + n_runs, index, [](uint64_t i, const nixl_amd_copy_run_t &r) { return i < r.first_index; }) - 1;
             return run->base + (index - run->first_index) * run->stride;
@@ -1661,7 +1666,9 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
         }
         e = hipGetLastError();
     }
-    if (e == hipSuccess && sort) {
+    // after the launch: the kernel reads the indices over the bus meanwhile (65 536 blocks there and
+    // back 848 us with the pattern first, 831 so; 15 250 blocks 75.5 and 73.1)
+    if (e == hipSuccess && study_pattern()) {
         hipLaunchKernelGGL(sort_records_kernel, dim3(static_cast<uint32_t>((n + kSortWindow - 1) / kSortWindow)),
                            dim3(kSortWindow / 2), 0, up, recs, static_cast<uint32_t>(n));
         e = hipGetLastError();
