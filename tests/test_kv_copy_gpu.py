@@ -520,6 +520,53 @@ def test_many_requests_leave_memory_where_it_was(hip_agent, cuda):
         h.release()
 
 
+@pytest.mark.parametrize("posted", [False, True])
+def test_kept_requests_do_not_keep_pinned_memory(hip_agent, cuda, posted):
+    """Requests that a program makes and keeps (posted and done, or not posted yet): the pinned
+    buffers that their plans were written from go back to the cache, all but a few.  Each is an
+    allocation of its own, so 300 of them would be 300 more mappings of the process; a third of
+    that leaves room for the plans' device memory, of which an allocation holds many."""
+    import torch
+    a = hip_agent
+    blk, n_pool, n, kept = 8192, 8192, 4096, 300
+    mem = torch.randint(0, 256, (2 * n_pool * blk,), dtype=torch.uint8, device=cuda)
+    a.register_memory([mem])
+    h_l = a.prep_xfer_dlist("", _descs(mem, np.arange(n_pool) * blk, [blk] * n_pool), "VRAM")
+    h_r = a.prep_xfer_dlist("agent", _descs(mem, (n_pool + np.arange(n_pool)) * blk, [blk] * n_pool), "VRAM")
+    rng = np.random.default_rng(29)
+    torch.cuda.synchronize()
+
+    def make():
+        li, ri = (rng.permutation(n_pool)[:n].astype(np.int32) for _ in range(2))
+        req = a.make_prepped_xfer("WRITE", h_l, li, h_r, ri)
+        if posted:
+            _wait(a, req)
+        return req, li, ri
+
+    def mappings():
+        with open("/proc/self/maps") as f:
+            return sum(1 for _ in f)
+
+    for _ in range(50):
+        make()[0].release()
+    before = mappings()
+    requests = [make() for _ in range(kept)]
+    grown = mappings() - before
+    # every one of them still moves its own blocks, buffers given back or not
+    for req, li, ri in requests[::23] + requests[-1:]:
+        mem[n_pool * blk:].zero_()
+        torch.cuda.synchronize()
+        _wait(a, req)
+        blocks = mem.view(2, n_pool, blk)
+        li, ri = (torch.from_numpy(i).to(cuda).long() for i in (li, ri))
+        assert torch.equal(blocks[1][ri], blocks[0][li])
+    for req, _, _ in requests:
+        req.release()
+    for h in (h_l, h_r):
+        h.release()
+    assert grown < kept // 3, f"{grown} more mappings with {kept} requests kept"
+
+
 def test_write_zero_read_roundtrip_and_repost(hip_agent, cuda):
     # transfer_handler round trip (test/gtest/plugins/transfer_handler.h:182-209 with
     # memory_handler.h:42-58): WRITE, clear the source, READ back, expect the increasing
