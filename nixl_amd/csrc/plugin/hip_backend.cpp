@@ -250,7 +250,8 @@ nixlHipEngine::pickStream(int device) const {
 
 bool
 nixlHipEngine::chooseStream(int device, nixlHipReqH &req, nixl_amd_copy_tuning_t &tuning) const {
-    req.stream = pickStream(device);
+    if (!req.stream || req.device != device) req.stream = pickStream(device);
+    req.device = device;
     tuning = tuning_;
     if (!useExternalStream_) tuning.stream = req.stream;
     return req.stream || useExternalStream_;
@@ -711,6 +712,7 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
     const nixlHipMD *first_md = nullptr;
     std::vector<nixl_amd_copy_run_t> tables[2];
     size_t flat[2] = {0, 0};
+    uint64_t address_bits = 0;
     for (int side = 0; side < 2; ++side) {
         const nixlStrideDesc *runs = side ? remote_runs : local_runs;
         const size_t n_runs = side ? n_remote_runs : n_local_runs;
@@ -734,6 +736,7 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
                 if (md->device != device) return NIXL_ERR_NOT_SUPPORTED;
             }
             tables[side].push_back(nixl_amd_copy_run_t{md->here(run.addr), run.stride, flat[side], run.count});
+            address_bits |= tables[side].back().base | run.stride;
             flat[side] += run.count;
         }
     }
@@ -751,9 +754,14 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
         return NIXL_ERR_INVALID_PARAM;
     }
 
+    // Whole chunks on 128-byte lines are what such plans are made of.  Decided here and not by
+    // the plan's refusal, so that a request which goes on to the descriptor path has taken no
+    // turn on the engine's streams yet.
+    const uint64_t chunk = 1024u * static_cast<uint64_t>(std::max(tuning_.units_per_lane, 1));
+    if ((address_bits & 127u) || len % chunk != 0) return NIXL_ERR_NOT_SUPPORTED;
+
     const bool write = (operation == NIXL_WRITE);
     auto req = std::make_unique<nixlHipReqH>();
-    req->device = device;
     req->bytes = count * len;
     const int src = write ? 0 : 1, dst = 1 - src;
     const int *index_of[2] = {local_indices, remote_indices};
@@ -762,7 +770,7 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
     const int rc = nixl_amd_copy_plan_create_indexed_runs(tables[src].data(), tables[src].size(), index_of[src],
                                                           tables[dst].data(), tables[dst].size(), index_of[dst], count, len,
                                                           device, &tuning, &req->plan);
-    if (rc == NIXL_AMD_ERR_INVALID) return NIXL_ERR_NOT_SUPPORTED; // shape or alignment: the descriptor path handles it
+    if (rc == NIXL_AMD_ERR_INVALID) return NIXL_ERR_NOT_SUPPORTED; // the descriptor path handles it
     if (rc != NIXL_AMD_OK) {
         NIXL_ERROR << "HIP backend: " << nixl_amd_last_error();
         return NIXL_ERR_BACKEND;

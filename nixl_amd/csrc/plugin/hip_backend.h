@@ -243,8 +243,9 @@ public:
                      const nixl_opt_args_t *extra_params = nullptr) const override;
 
 private:
-    // The stream of a request on `device`, and the tuning that names it to the kernels library
-    // (a stream of the application's is not named: the application may capture it).
+    // The stream of a request on `device` (a request takes one turn, however many forms of plan
+    // are tried for it), and the tuning that names it to the kernels library (a stream of the
+    // application's is not named: the application may capture it).
     bool
     chooseStream(int device, nixlHipReqH &req, nixl_amd_copy_tuning_t &tuning) const;
     // The two passes of prepXfer over a request's descriptor lists (hip_backend.cpp).

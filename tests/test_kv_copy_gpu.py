@@ -1067,6 +1067,19 @@ def test_raw_south_bound_api_from_cpp(cuda):
     assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
 
 
+def test_requests_take_the_streams_in_turn(cuda):
+    """num_streams: requests go to the engine's streams one after the other, whichever form of plan
+    they end up with.  The program is tests/cpp/stream_turns_check.cpp."""
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = os.path.join(root, "tests", "cpp", "_build", "stream_turns_check")
+    if not os.path.exists(exe):
+        pytest.fail(f"{exe} missing: run __graft_entry__.build() first")
+    proc = subprocess.run([exe, os.path.join(_lib.PLUGIN_DIR, "libplugin_HIP.so")], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
+
+
 def test_device_memory_view_calls_from_hip(cuda):
     """Memory views and the device-side put / counter add / get-pointer calls over them,
     driven from a HIP program through nixlAgent (tests/cpp/mem_view_device_api.hip; the
