@@ -59,8 +59,10 @@ typedef struct nixl_amd_copy_tuning {
                        * into ascending destination order inside windows of 1024 (on the device): 1 = on, 2 = off */
     /* The HIP stream the plan will be launched on, or NULL.  While that stream is idle the
      * kernels that write the plan's arrays are queued on it, so that a launch needs no wait; the
-     * stream must then outlive the plan and must not be under capture when the plan is first
-     * launched on it.  NULL, or a busy stream: they run on a stream of the library's. */
+     * stream must then outlive the plan, and while it is under capture the plan can be launched
+     * on it only after nixl_amd_copy_plan_status has seen an earlier launch complete
+     * (NIXL_AMD_ERR_INVALID otherwise; the capture goes on).  NULL, a busy stream or one under
+     * capture: they run on a stream of the library's. */
     void *stream;
 } nixl_amd_copy_tuning_t;
 
@@ -256,7 +258,8 @@ nixl_amd_copy_plan_status(nixl_amd_copy_plan_t *plan, int wait);
  * returns NIXL_AMD_ERR_BUSY and leaves the plan as it is (its arrays would go back to a pool
  * that the next plan's upload writes into): wait for the launch, then destroy again.  Launches
  * recorded into a HIP graph are not tracked: their owner keeps the plan for as long as the
- * graph may be replayed. */
+ * graph may be replayed.  BUSY is also the answer for a plan that was never launched while the
+ * stream it names (nixl_amd_copy_tuning_t) is under capture. */
 int
 nixl_amd_copy_plan_destroy(nixl_amd_copy_plan_t *plan);
 

@@ -757,11 +757,11 @@ arena_cache() {
 
 // Plans are uploaded on a stream of their own that does not synchronise with the default
 // stream, so that preparing one request does not wait for another that is still copying.
+constexpr int kMaxDevices = 64;
+
 hipError_t
-upload_stream(int device, hipStream_t *out) {
-    constexpr int kMaxDevices = 64;
+library_stream(hipStream_t (&streams)[kMaxDevices], int device, hipStream_t *out) {
     static std::mutex mutex;
-    static hipStream_t streams[kMaxDevices] = {};
     if (device < 0 || device >= kMaxDevices) return hipErrorInvalidDevice;
     std::lock_guard<std::mutex> lock(mutex);
     if (!streams[device]) {
@@ -770,6 +770,20 @@ upload_stream(int device, hipStream_t *out) {
     }
     *out = streams[device];
     return hipSuccess;
+}
+
+hipError_t
+upload_stream(int device, hipStream_t *out) {
+    static hipStream_t streams[kMaxDevices] = {};
+    return library_stream(streams, device, out);
+}
+
+// A stream on which nothing but events lie, each behind the caller's stream of a plan that was
+// destroyed before its launch (recycle_after).
+hipError_t
+recycle_stream(int device, hipStream_t *out) {
+    static hipStream_t streams[kMaxDevices] = {};
+    return library_stream(streams, device, out);
 }
 
 BlockCache &
@@ -825,6 +839,8 @@ struct nixl_amd_copy_plan {
     // read then stays with the plan until a launch behind them is known to have run (see end_build).
     hipEvent_t uploaded = nullptr;
     hipStream_t built_on = nullptr; // the caller's stream, until a launch is known to be behind the build
+    std::atomic<bool> seen_done{false}; // nixl_amd_copy_plan_status has seen a launch complete
+    bool reserved = false; // one of kMaxHeldStaging is this plan's, its buffer not handed over yet
     std::atomic<void *> staging{nullptr}; // taken out by whoever gives it back: the status may be asked from any thread
     size_t staging_cap = 0;
     // Recorded behind the kernels of every launch (not on a capturing stream): destroying the
@@ -832,6 +848,8 @@ struct nixl_amd_copy_plan {
     // and the next plan's upload would overwrite records a running kernel still reads.
     hipEvent_t launched = nullptr;
     bool launched_valid = false;
+
+    ~nixl_amd_copy_plan();
 };
 
 // Pinned buffers whose contents are still travelling to the device: each goes back to the
@@ -866,12 +884,30 @@ reap_uploads(int device) {
     }
 }
 
+// Records `done` behind everything queued on `up` so far: on `up` itself if that is a stream of the
+// library's, on one of its own if it is a caller's.  An event that lies on a caller's stream may
+// not even be asked for while that stream is captured, which would break a capture that has
+// nothing to do with it.
+static hipError_t
+record_behind(int device, hipStream_t up, bool of_caller, hipEvent_t done) {
+    if (!of_caller) return hipEventRecord(done, up);
+    hipStream_t aside = nullptr;
+    hipEvent_t joint = nullptr;
+    hipError_t e = recycle_stream(device, &aside);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&joint, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(joint, up);
+    if (e == hipSuccess) e = hipStreamWaitEvent(aside, joint, 0);
+    if (e == hipSuccess) e = hipEventRecord(done, aside);
+    if (joint) (void)hipEventDestroy(joint);
+    return e;
+}
+
 // Hands `staging` and `arena` (either may be null) over: recycled when everything queued on `up` so far has run.
 // Without an event to watch, the stream is waited for instead.
 static void
-recycle_after(int device, hipStream_t up, void *staging, size_t cap, void *arena = nullptr, size_t arena_cap = 0) {
+recycle_after(int device, hipStream_t up, bool of_caller, void *staging, size_t cap, void *arena = nullptr, size_t arena_cap = 0) {
     hipEvent_t done = nullptr;
-    if (hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess && hipEventRecord(done, up) == hipSuccess) {
+    if (hipEventCreateWithFlags(&done, hipEventDisableTiming) == hipSuccess && record_behind(device, up, of_caller, done) == hipSuccess) {
         std::lock_guard<std::mutex> lock(g_pending_mutex);
         g_pending[device].push_back(PendingUpload{done, staging, cap, arena, arena_cap});
         return;
@@ -887,6 +923,10 @@ recycle_after(int device, hipStream_t up, void *staging, size_t cap, void *arena
 // requests and keep them, so only a few may.
 constexpr int kMaxHeldStaging = 16;
 static std::atomic<int> g_held_staging{0};
+
+nixl_amd_copy_plan::~nixl_amd_copy_plan() {
+    if (reserved) g_held_staging.fetch_sub(1, std::memory_order_relaxed);
+}
 
 // The kernels that read the plan's pinned buffer have run: back into the cache with it.
 static void
@@ -975,43 +1015,45 @@ describe_blocks(nixl_amd_copy_plan &plan, const Tuning &t, size_t n_recs, uint64
 // named it and it is idle.  A launch right behind the making then needs no event, no wait of one
 // stream for another and no recycling in between (20 us of host time between make and kernel
 // became 5); behind a transfer that is still running, the library's own stream writes the arrays
-// meanwhile.
+// meanwhile.  It does so, too, for a stream under capture (which may not be asked whether it is
+// idle, and whose graph these kernels do not belong in), and for requests that are made and kept:
+// the pinned buffer of a plan built on the caller's stream waits with the plan for its first
+// launch to be seen done, and only kMaxHeldStaging plans may do that.  (1000 requests of 4096
+// blocks made, posted and kept, each with a pinned buffer until its end: 204 us a request, 40 with
+// buffers that come back.)
 static hipError_t
-build_stream(int device, const Tuning &t, hipStream_t *out) {
+build_stream(nixl_amd_copy_plan *plan, const Tuning &t, hipStream_t *out) {
     if (t.stream) {
-        const hipError_t idle = hipStreamQuery(t.stream);
-        if (idle == hipSuccess) {
-            *out = t.stream;
-            return hipSuccess;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        const bool may_ask = hipStreamIsCapturing(t.stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+        if (may_ask && hipStreamQuery(t.stream) == hipSuccess) {
+            if (g_held_staging.fetch_add(1, std::memory_order_relaxed) < kMaxHeldStaging) {
+                plan->reserved = true;
+                *out = t.stream;
+                return hipSuccess;
+            }
+            g_held_staging.fetch_sub(1, std::memory_order_relaxed);
         }
         (void)hipGetLastError();
     }
-    return upload_stream(device, out);
+    return upload_stream(plan->device, out);
 }
 
 // Everything that writes the plan's arrays is queued on `up`: what later launches and the pinned
-// buffer's next user wait for.  The buffer is taken over if this succeeds.  On the caller's stream
-// it waits with the plan for the first launch to be seen done, which spares a request that is
-// posted at once an event of its own; when kMaxHeldStaging plans hold one already (requests made
-// and kept), an event is recorded after all.  (1000 requests of 4096 blocks made, posted and kept,
-// each with a pinned buffer until its end: 204 us a request, 40 with buffers that come back.)
+// buffer's next user wait for.  The buffer is taken over if this succeeds.
 static hipError_t
-end_build(nixl_amd_copy_plan *plan, const Tuning &t, hipStream_t up, void *staging, size_t staging_cap) {
-    if (t.stream && up == t.stream) {
+end_build(nixl_amd_copy_plan *plan, hipStream_t up, void *staging, size_t staging_cap) {
+    if (plan->reserved) {
         plan->built_on = up;
-        if (g_held_staging.fetch_add(1, std::memory_order_relaxed) < kMaxHeldStaging) {
-            plan->staging_cap = staging_cap;
-            plan->staging = staging;
-        } else {
-            g_held_staging.fetch_sub(1, std::memory_order_relaxed);
-            recycle_after(plan->device, up, staging, staging_cap);
-        }
+        plan->staging_cap = staging_cap;
+        plan->staging = staging;
+        plan->reserved = false; // from here on the buffer stands for it
         return hipSuccess;
     }
     // No wait here: the event goes behind the kernels, launches wait for it on their stream.
     hipError_t e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
-    if (e == hipSuccess) recycle_after(plan->device, up, staging, staging_cap);
+    if (e == hipSuccess) recycle_after(plan->device, up, false, staging, staging_cap);
     return e;
 }
 
@@ -1084,14 +1126,14 @@ build_block_plan(int device, const Tuning &t, void *staging, size_t staging_cap,
     }
     hipStream_t up = nullptr;
     hipError_t e = arena_cache().get(device, bytes, &plan->arena, &plan->arena_cap);
-    if (e == hipSuccess) e = build_stream(device, t, &up);
+    if (e == hipSuccess) e = build_stream(plan, t, &up);
     if (e == hipSuccess) e = upload(up, plan->arena, staging, bytes);
     if (e == hipSuccess && sort) {
         hipLaunchKernelGGL(sort_records_kernel, dim3(static_cast<uint32_t>((n_recs + kSortWindow - 1) / kSortWindow)),
                            dim3(kSortWindow / 2), 0, up, static_cast<UniformRec *>(plan->arena), static_cast<uint32_t>(n_recs));
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = end_build(plan, t, up, staging, staging_cap);
+    if (e == hipSuccess) e = end_build(plan, up, staging, staging_cap);
     if (e != hipSuccess) {
         if (up) (void)hipStreamSynchronize(up); // whatever was queued reads the buffers given back below
         if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -1425,7 +1467,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipMalloc(plan arena): ") + hipGetErrorString(e));
         }
         hipStream_t up = nullptr;
-        e = build_stream(device, t, &up);
+        e = build_stream(plan, t, &up);
         auto *arena = static_cast<uint8_t *>(plan->arena);
         if (e == hipSuccess && total > upload_from)
             e = upload(up, arena + upload_from, staging, total - upload_from);
@@ -1437,7 +1479,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
                                n_uniform_chunks, static_cast<uint32_t>(chunk_units * 16u));
             e = hipGetLastError();
         }
-        if (e == hipSuccess) e = end_build(plan, t, up, staging, staging_cap);
+        if (e == hipSuccess) e = end_build(plan, up, staging, staging_cap);
         if (e != hipSuccess) {
             if (up) (void)hipStreamSynchronize(up); // a queued copy still reads the buffer given back below
             if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -1675,7 +1717,7 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     const size_t rec_bytes = n * sizeof(UniformRec);
     hipStream_t up = nullptr;
     e = arena_cache().get(device, rec_bytes, &plan->arena, &plan->arena_cap);
-    if (e == hipSuccess) e = build_stream(device, t, &up);
+    if (e == hipSuccess) e = build_stream(plan, t, &up);
     auto *recs = static_cast<UniformRec *>(plan->arena);
     const auto *index = static_cast<const int32_t *>(staging);
     if (e == hipSuccess) {
@@ -1697,7 +1739,7 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
                            dim3(kSortWindow / 2), 0, up, recs, static_cast<uint32_t>(n));
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = end_build(plan, t, up, staging, staging_cap);
+    if (e == hipSuccess) e = end_build(plan, up, staging, staging_cap);
     if (e != hipSuccess) {
         if (up) (void)hipStreamSynchronize(up); // whatever was queued reads the buffers given back below
         if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -1901,16 +1943,23 @@ nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (s && hipStreamIsCapturing(s, &capture) != hipSuccess) (void)hipGetLastError();
     if (plan->built_on && plan->launched_valid) {
-        // an earlier launch followed the build: once it has run, so has the build
-        if (hipEventQuery(plan->launched) == hipSuccess) {
+        // An earlier launch followed the build: once it has run, so has the build.  Its event lies
+        // on built_on: asking for it while that stream is captured would end the capture.
+        if (plan->seen_done) {
             plan->built_on = nullptr;
-            give_back_staging(plan);
-        } else {
-            (void)hipGetLastError();
+        } else if (capture == hipStreamCaptureStatusNone) {
+            if (hipEventQuery(plan->launched) == hipSuccess) {
+                plan->built_on = nullptr;
+                give_back_staging(plan);
+            } else {
+                (void)hipGetLastError();
+            }
         }
     }
     if (plan->built_on && s == plan->built_on && capture != hipStreamCaptureStatusNone)
-        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_launch: the stream a plan was made on may not be captured at its first launch");
+        return nixl_amd_fail(NIXL_AMD_ERR_INVALID,
+                             "plan_launch: the stream a plan was made on is under capture and no launch of the plan has been seen "
+                             "complete (nixl_amd_copy_plan_status)");
     if (plan->built_on && s != plan->built_on) {
         // not where the caller said: from here on the build is one on a stream of its own
         if (!plan->uploaded) HIP_TRY(hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming));
@@ -1992,6 +2041,7 @@ nixl_amd_copy_plan_status(nixl_amd_copy_plan_t *plan, int wait) {
     const DeviceScope on_device(plan->device);
     const hipError_t state = wait ? hipEventSynchronize(plan->launched) : hipEventQuery(plan->launched);
     if (state == hipSuccess) {
+        plan->seen_done = true;
         give_back_staging(plan);
         return NIXL_AMD_OK;
     }
@@ -2017,9 +2067,13 @@ nixl_amd_copy_plan_destroy(nixl_amd_copy_plan_t *plan) {
     }
     if (plan->built_on && !plan->launched_valid) {
         // never launched: the build itself may still run, behind whatever is in front of it
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(plan->built_on, &capture) != hipSuccess) (void)hipGetLastError();
+        if (capture != hipStreamCaptureStatusNone)
+            return nixl_amd_fail(NIXL_AMD_ERR_BUSY, "plan_destroy: the stream the plan was made on is under capture");
         void *staging = plan->staging.exchange(nullptr);
         if (staging) g_held_staging.fetch_sub(1, std::memory_order_relaxed);
-        recycle_after(plan->device, plan->built_on, staging, plan->staging_cap, plan->arena, plan->arena_cap);
+        recycle_after(plan->device, plan->built_on, true, staging, plan->staging_cap, plan->arena, plan->arena_cap);
         plan->arena = nullptr;
     }
     (void)settle_upload(plan, true); // the arena and the upload buffer go back only when nothing writes or reads them

@@ -1015,6 +1015,80 @@ def test_block_plans_inline_and_on_the_callers_stream(cuda, n, n_runs, named):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("made", ["seen", "unseen", "other", "during"])
+def test_captured_launches_of_plans_that_name_a_stream(cuda, made):
+    """A plan that names a stream is launched into a graph captured from that stream: made before
+    and launched once, with that launch seen complete (taken) or not (refused, and the capture goes
+    on); made while the stream is under capture; or captured from another stream.  Plans made and
+    dropped meanwhile do not disturb the capture.  Every replay copies the bytes of its time."""
+    import torch
+    rng = np.random.default_rng(71)
+    n, blk, pool = 1500, 8192, 1800
+    src = torch.randint(0, 256, (pool, blk), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros_like(src)
+    at, to = (rng.permutation(pool)[:n].astype(np.int32) for _ in range(2))
+    run_s, run_d = (_lib.CopyRun(t.data_ptr(), blk, 0, pool) for t in (src, dst))
+    lib = _lib.kernels()
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def make():
+        plan = ctypes.c_void_p()
+        tuning = _lib.CopyTuning(stream=stream.cuda_stream)
+        assert lib.nixl_amd_copy_plan_create_indexed_runs(ctypes.byref(run_s), 1, at.ctypes.data, ctypes.byref(run_d), 1, to.ctypes.data,
+                                                          n, blk, 0, ctypes.byref(tuning), ctypes.byref(plan)) == 0, _lib.kernels_error()
+        return plan
+
+    # plans destroyed after a launch, without one, and an unlaunched one that is still there: the
+    # cache holds the memory of the ones made under capture
+    spare = []
+    for _ in range(4):
+        torch.cuda.synchronize()  # the named stream is idle: built there
+        spare.append(make())
+    assert lib.nixl_amd_copy_plan_launch(spare[0], stream.cuda_stream) == 0
+    torch.cuda.synchronize()
+    for p in spare[:3]:
+        assert lib.nixl_amd_copy_plan_destroy(p) == 0
+    torch.cuda.synchronize()
+    plan = make()
+    if made in ("seen", "unseen"):
+        assert lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+        if made == "seen":
+            assert lib.nixl_amd_copy_plan_status(plan, 1) == 0
+    torch.cuda.synchronize()
+    captured = other if made == "other" else stream
+    graph, late = torch.cuda.CUDAGraph(), None
+    with torch.cuda.stream(captured):
+        # relaxed: calls that concern other streams are allowed meanwhile (a plan's upload is waited
+        # for); what would end the capture is a question about work on the captured stream itself
+        graph.capture_begin(capture_error_mode="relaxed")
+        try:
+            dst.zero_()
+            late = make()
+            if made != "other":
+                assert lib.nixl_amd_copy_plan_destroy(spare[3]) == -4  # its stream is captured: later
+            rc = lib.nixl_amd_copy_plan_launch(plan, captured.cuda_stream)
+            if made in ("unseen", "during"):
+                assert rc == -1 and "capture" in _lib.kernels_error()
+                assert lib.nixl_amd_copy_plan_launch(late, captured.cuda_stream) == 0, _lib.kernels_error()
+            else:
+                assert rc == 0, _lib.kernels_error()
+        finally:
+            graph.capture_end()
+    at_t, to_t = (torch.from_numpy(i).to(cuda).long() for i in (at, to))
+    for _ in range(4):
+        src ^= 0x5A
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = torch.zeros_like(dst)
+        want[to_t] = src[at_t]
+        assert torch.equal(dst, want)
+    for p in (plan, late, spare[3]):
+        assert lib.nixl_amd_copy_plan_status(p, 1) == 0
+        assert lib.nixl_amd_copy_plan_destroy(p) == 0
+    torch.cuda.synchronize()
+
+
 def test_golden_descriptor_list(cuda):
     """Committed vector (tests/golden/kv_descs.npz): mixed aligned / unaligned / empty
     descriptors, destination pre-filled with a canary byte."""
