@@ -1274,6 +1274,36 @@ def test_ll_dispatch_forms_by_size(cuda, shape, form):
     assert np.array_equal(stats.cpu().numpy(), want["recv_count"])
 
 
+@pytest.mark.parametrize("hidden,topk", [(512, 16), (1024, 8), (2048, 16)])
+def test_ll_one_launch_is_no_slower_than_two(cuda, hidden, topk):
+    """The largest calls that take one launch (2048 selections) against the smallest ones that take
+    two (one token a rank more): the rows' width and the number of selections a token must not make
+    the one launch the slower of the two.  Medians of 40 calls in turn; a tenth for their spread."""
+    R, E, T = 2, 64, 1024 // topk
+    buf = Buffer(R, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(hidden + topk)
+
+    def call(tokens):
+        x = torch.empty((R, tokens, hidden), dtype=torch.bfloat16, device=cuda).normal_(generator=g)
+        idx = torch.topk(torch.rand((R * tokens, E), generator=g, device=cuda), topk, dim=1)[1].to(torch.int32).view(R, tokens, topk)
+        idx = idx.contiguous()
+        return lambda: buf.dispatch(x, idx, tokens, E, use_fp8=True)
+
+    calls = [call(T), call(T + 1)]
+    times = [[], []]
+    for i in range(50):
+        for f, ts in zip(calls, times):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            f()
+            b.record()
+            b.synchronize()
+            if i >= 10:
+                ts.append(a.elapsed_time(b))
+    one, two = (float(np.median(ts)) for ts in times)
+    assert one <= 1.1 * two, f"one launch {one * 1e3:.1f} us, two {two * 1e3:.1f} us"
+
+
 def test_ll_narrow_workgroups_give_the_same_bytes(cuda):
     """nixl_amd_ep_ll_set_tuning: with workgroups of 64 and 128 lanes a token's row is split
     over several workgroups in dispatch and combine; results must not change."""
