@@ -530,7 +530,6 @@ struct HtRows {
     const long long *row_offset;
     HtDims d;
     int parts;
-    uint32_t first; // piece the first row workgroup of the launch starts at
 };
 
 __device__ __forceinline__ void
@@ -729,8 +728,8 @@ scales_block(const HtScales &a,
 // writes then run beside the rows', four pieces of rows to a workgroup behind them.  Launched one
 // after the other, the three took 14.6 us at 4 x 333 x 4096 fp8 (now 6.9), 157 at 8 x 2048 x 7168
 // fp8 (145, and 132 with the loads and stores described at the rows), 55.3 at 8 x 1024 x 4096
-// bf16 (52.9 and 49.5).  A launch holds fewer than 2^24 such workgroups; a call of more is launched part
-// by part.
+// bf16 (52.9 and 49.5).  A launch holds fewer than 2^24 such workgroups (2^32 threads); a call of
+// more is launched part by part, each part from its workgroup `first` on.
 constexpr int kHtThreads = 256;
 constexpr int kHtWaves = kHtThreads / kWaveSize;
 constexpr long long kHtMaxGrid = (1ll << 24) - 1;
@@ -738,20 +737,20 @@ static_assert(kHtThreads == kHtMetaThreads && kHtThreads == kHtScaleThreads);
 
 template<bool VEC, bool SCALES>
 __global__ void __launch_bounds__(kHtThreads)
-ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint32_t meta_blocks) {
+ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint32_t meta_blocks, uint32_t first) {
     uint32_t block = blockIdx.x;
     if (SCALES) {
         if (block < scale_blocks) {
-            scales_block(sc, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, block);
+            scales_block(sc, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, first + block);
             return;
         }
         block -= scale_blocks;
     }
     if (block < meta_blocks) {
-        meta_block<VEC>(m, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, block);
+        meta_block<VEC>(m, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, first + block);
         return;
     }
-    dispatch_piece(a, a.first + (block - meta_blocks) * kHtWaves + uniform(threadIdx.x / kWaveSize));
+    dispatch_piece(a, (first + block - meta_blocks) * kHtWaves + uniform(threadIdx.x / kWaveSize));
 }
 
 // ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
@@ -1053,8 +1052,8 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
         return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_dispatch: too many ranks and tokens");
     const long long *offsets = reinterpret_cast<const long long *>(recv_row_offset);
     const int *prefix = recv_gbl_rank_prefix_sum;
-    HtRows rows{static_cast<uint16_t *>(recv_x), static_cast<const uint16_t *>(x), is_token_in_rank, prefix, send_head, offsets, d,
-                parts, 0};
+    const HtRows rows{static_cast<uint16_t *>(recv_x), static_cast<const uint16_t *>(x), is_token_in_rank, prefix, send_head, offsets, d,
+                      parts};
     const HtMeta meta{recv_topk_idx, recv_topk_weights, recv_src_meta, topk_idx, topk_weights};
     const HtScales sc{static_cast<uint32_t *>(recv_x_scales), static_cast<const uint32_t *>(x_scales), num_scales,
                       num_scales % 4 == 0 && reinterpret_cast<uintptr_t>(recv_x_scales) % 16 == 0, scale_rank_stride,
@@ -1067,21 +1066,22 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
     const long long row_blocks = (pieces + kHtWaves - 1) / kHtWaves;
     const auto kernel = x_scales ? (vec ? ht_dispatch_kernel<true, true> : ht_dispatch_kernel<false, true>)
                                  : (vec ? ht_dispatch_kernel<true, false> : ht_dispatch_kernel<false, false>);
-    const auto launch = [&](long long n_scale, long long n_meta, long long n_row) -> int {
+    const auto launch = [&](long long n_scale, long long n_meta, long long n_row, long long first) -> int {
         const long long blocks = n_scale + n_meta + n_row;
         if (blocks == 0) return NIXL_AMD_OK;
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(kHtThreads), 0, s, rows, meta, sc,
-                           static_cast<uint32_t>(n_scale), static_cast<uint32_t>(n_meta));
+                           static_cast<uint32_t>(n_scale), static_cast<uint32_t>(n_meta), static_cast<uint32_t>(first));
         HIP_TRY(hipGetLastError());
         return NIXL_AMD_OK;
     };
-    if (scale_blocks + meta_blocks + row_blocks <= kHtMaxGrid) return launch(scale_blocks, meta_blocks, row_blocks);
-    for (long long at = 0; at < row_blocks; at += kHtMaxGrid) {
-        rows.first = static_cast<uint32_t>(at * kHtWaves);
-        if (const int status = launch(0, 0, std::min(kHtMaxGrid, row_blocks - at))) return status;
-    }
-    if (const int status = launch(scale_blocks, 0, 0)) return status;
-    return launch(0, meta_blocks, 0);
+    if (scale_blocks + meta_blocks + row_blocks <= kHtMaxGrid) return launch(scale_blocks, meta_blocks, row_blocks, 0);
+    const long long part_blocks[3] = {row_blocks, scale_blocks, meta_blocks};
+    for (int part = 0; part < 3; ++part)
+        for (long long at = 0; at < part_blocks[part]; at += kHtMaxGrid) {
+            const long long n = std::min(kHtMaxGrid, part_blocks[part] - at);
+            if (const int status = launch(part == 1 ? n : 0, part == 2 ? n : 0, part == 0 ? n : 0, at)) return status;
+        }
+    return NIXL_AMD_OK;
 }
 
 int

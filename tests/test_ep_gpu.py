@@ -546,6 +546,35 @@ def test_ht_dispatch_fp8_rows_with_scales(cuda, scale_dtype):
                         num_tokens_per_expert=per_expert, topk_idx=td, num_channels=C)
 
 
+@pytest.mark.parametrize("R,T", [(1, (1 << 26) + 5), (1024, 1024)])
+def test_ht_dispatch_of_more_workgroups_than_a_launch_holds(cuda, R, T):
+    """A launch holds fewer than 2^24 workgroups of 256 threads.  One rank of 2^26 + 5 tokens has
+    more workgroups of rows than that, 1024 ranks of 1024 tokens have 2^24 of scales: rows, scales
+    and metadata arrive as from one launch.  A token names one expert or none, so that destination
+    d's rows are its tokens in order."""
+    H, E = 16, R
+    g = torch.Generator(device=cuda).manual_seed(R)
+    topk = torch.randint(0, E, (R, T, 1), generator=g, device=cuda, dtype=torch.int32)
+    topk[torch.rand((R, T, 1), generator=g, device=cuda) < 0.1] = -1
+    topk[-1, -1, 0] = E - 1  # the last workgroup of each part has work
+    w = torch.rand((R, T, 1), generator=g, device=cuda)
+    x = torch.randint(0, 256, (R, T, H), generator=g, device=cuda, dtype=torch.uint8)
+    scales = torch.rand((R, T, 1), generator=g, device=cuda)
+    buf = Buffer(R, low_latency_mode=False, device=cuda)
+    per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk, E)
+    (rows, row_scales), idx, weights, counts, handle, _ = buf.ht_dispatch(
+        (x.view(torch.float8_e4m3fn), scales), num_tokens_per_rank=per_rank, is_token_in_rank=in_rank,
+        num_tokens_per_expert=per_expert, topk_idx=topk, topk_weights=w, num_channels=1)
+    torch.cuda.synchronize()
+    dst = topk.view(-1)
+    order = torch.argsort(torch.where(dst < 0, E, dst), stable=True)[:int((dst >= 0).sum())]
+    assert rows.shape[0] == order.numel() == sum(sum(c) for c in counts)
+    assert torch.equal(rows.view(torch.uint8), x.view(R * T, H)[order])
+    assert torch.equal(row_scales, scales.view(R * T, 1)[order])
+    assert not idx.any() and torch.equal(weights, w.view(R * T, 1)[order])
+    assert torch.equal(handle[3], torch.stack([order // T, order % T], 1).to(torch.int32))
+
+
 def test_ht_calls_honour_previous_event_and_async_finish(cuda):
     """previous_event / async_finish as the reference defines them (csrc/nixl_ep.cpp:558-571,
     596-611; its test passes buffer.capture() and waits on the returned event,
