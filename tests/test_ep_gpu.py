@@ -1284,8 +1284,11 @@ def test_ll_combine_logfmt(cuda):
     ((1, 1, 512, 1, 1, 1), "fp8"), ((4, 64, 512, 8, 24, 64), "fp8"), ((4, 65, 512, 8, 24, 65), "fp8"),
     ((2, 20, 1024, 9, 34, 20), "ue8m0"), ((2, 64, 8192, 16, 34, 64), "fp8"), ((2, 65, 8192, 16, 34, 65), "bf16"),
     ((64, 4, 512, 4, 64, 8), "ue8m0"), ((65, 4, 512, 4, 65, 8), "fp8"), ((2, 7, 7168, 8, 8, 16), "bf16"),
-    # 64 words of scales a row: the most the row kernel writes itself (8192 selections), and beyond
+    # 64 words of scales a row (16 as UE8M0): the most words the row kernel writes itself (2^19), and
+    # beyond, where the third launch moves them; the same call as UE8M0 stays below that line
     ((8, 128, 8192, 8, 16, 128), "fp8"), ((8, 129, 8192, 8, 16, 129), "fp8"), ((8, 129, 8192, 8, 16, 129), "ue8m0"),
+    # the third launch for UE8M0 words, and for row counts an expert that are no multiple of 4
+    ((8, 257, 8192, 16, 16, 257), "ue8m0"), ((7, 131, 8192, 10, 14, 131), "fp8"), ((7, 293, 8192, 16, 21, 293), "ue8m0"),
 ])
 def test_ll_dispatch_forms_by_size(cuda, shape, form):
     """Dispatch takes one, two or three launches by the number of selections and of scale words:
@@ -1301,6 +1304,25 @@ def test_ll_dispatch_forms_by_size(cuda, shape, form):
     want = eo.ll_dispatch(bits16(x).reshape(R, T, H), topk, E, M, fp8, ue, ue, fill=0x55)
     assert_dispatch_equal(got, want, fp8, ue)
     assert np.array_equal(stats.cpu().numpy(), want["recv_count"])
+
+
+@pytest.mark.parametrize("shape,form", [((7, 131, 8192, 10, 14, 131), "fp8"), ((8, 257, 8192, 16, 16, 257), "ue8m0")])
+def test_ll_scales_of_large_ragged_and_masked_calls(cuda, shape, form):
+    """More than 2^19 words of scales, so that ll_scales_kernel moves them: ranks with fewer tokens
+    than the others (one with none) and a masked pair of ranks leave the scales of the rows that
+    do not come untouched."""
+    R, T, H, K, E, M = shape
+    ue = form == "ue8m0"
+    assert R * T * K * (H // (512 if ue else 128)) > 1 << 19
+    x, topk, _ = make_world(R * 13 + T, R, T, H, K, E, drop=0.05, scale=2.0)
+    nt = np.random.default_rng(T).integers(1, T + 1, R).astype(np.int32)
+    nt[0], nt[2] = T, 0
+    mask = np.zeros((R, R), np.int32)
+    mask[0, R - 1] = mask[3, 1] = 1
+    rc, got = raw_ll_dispatch(cuda, x, topk, E, M, True, ue, ue, num_tokens=nt, mask=mask)
+    assert rc == 0, _lib.kernels_error()
+    want = eo.ll_dispatch(bits16(x).reshape(R, T, H), topk, E, M, True, ue, ue, num_tokens=nt, mask=mask, fill=0x55)
+    assert_dispatch_equal(got, want, True, ue)
 
 
 @pytest.mark.parametrize("hidden,topk", [(512, 16), (1024, 8), (2048, 16)])
