@@ -792,6 +792,14 @@ upload_cache() {
     return *c;
 }
 
+// Memory of the lists that stay on the device.  A cache of its own: a list is far larger than a
+// request's records, and one that is released would push those out of theirs.
+BlockCache &
+list_cache() {
+    static BlockCache *c = new BlockCache(false);
+    return *c;
+}
+
 // Queues the copy of `bytes` of a pinned block to a device block on `up`; both blocks are powers
 // of two from 4 KiB, so whole 16-byte units of the last one lie inside them.
 hipError_t
@@ -1805,7 +1813,7 @@ nixl_amd_copy_list_create(const nixl_amd_copy_list_entry_t *entries, size_t n, i
     HIP_TRY(on_device.status());
     void *mem = nullptr;
     size_t cap = 0;
-    HIP_TRY(arena_cache().get(device, n * sizeof(nixl_amd_copy_list_entry_t), &mem, &cap));
+    HIP_TRY(list_cache().get(device, n * sizeof(nixl_amd_copy_list_entry_t), &mem, &cap));
     // waits for the copy: the caller's array may go away, and the first request finds the table there
     hipStream_t up = nullptr;
     hipError_t e = upload_stream(device, &up);
@@ -1813,7 +1821,7 @@ nixl_amd_copy_list_create(const nixl_amd_copy_list_entry_t *entries, size_t n, i
     if (e == hipSuccess) e = hipStreamSynchronize(up);
     if (e != hipSuccess) {
         if (up) (void)hipStreamSynchronize(up);
-        arena_cache().put(device, mem, cap);
+        list_cache().put(device, mem, cap);
         return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("list_create: ") + hipGetErrorString(e));
     }
     auto *list = new nixl_amd_copy_list();
@@ -1830,7 +1838,7 @@ int
 nixl_amd_copy_list_destroy(nixl_amd_copy_list_t *list) {
     if (!list) return NIXL_AMD_OK;
     // nothing on the device reads a list once plan_create_listed has returned
-    arena_cache().put(list->device, list->entries, list->cap);
+    list_cache().put(list->device, list->entries, list->cap);
     delete list;
     return NIXL_AMD_OK;
 }

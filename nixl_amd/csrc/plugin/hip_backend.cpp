@@ -94,6 +94,9 @@ constexpr const char *kConnMailbox = ";mbox=";
 // Pairs from which a request against two device-resident lists is lowered on the device: below,
 // the wait for the kernel's verdict costs more than the host's 27 ns a pair.
 constexpr size_t kListedFrom = 1024;
+// Entries up to which a list stays on the device, at 16 bytes each there and, while it is made, on
+// the host: 64 MiB.  A longer one is lowered on the host, request by request.
+constexpr size_t kMaxListed = size_t{1} << 22;
 // Allocations of 2 GiB and more are not shared between processes: opening such a mapping has
 // been seen not to return.
 constexpr size_t kMaxIpcAllocation = (size_t{2} << 30) - 1;
@@ -785,8 +788,10 @@ nixlHipEngine::prepList(const nixlStrideDesc *runs, size_t n_runs, nixl_amd_copy
     if (!indexedPrep_) return NIXL_ERR_NOT_SUPPORTED;
     if (!runs || n_runs == 0) return NIXL_ERR_INVALID_PARAM;
     constexpr size_t kMinBytes = 128, kMaxBytes = 8176; // what the kernels library takes
+    const nixlStrideDesc &last = runs[n_runs - 1];
+    if (last.start_idx >= kMaxListed || last.count > kMaxListed - last.start_idx) return NIXL_ERR_NOT_SUPPORTED;
     std::vector<nixl_amd_copy_list_entry_t> entries;
-    entries.reserve(runs[n_runs - 1].start_idx + runs[n_runs - 1].count);
+    entries.reserve(last.start_idx + last.count);
     int device = -1;
     for (size_t r = 0; r < n_runs; ++r) {
         const nixlStrideDesc &run = runs[r];

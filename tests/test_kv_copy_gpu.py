@@ -930,6 +930,74 @@ def test_lists_without_a_stride_stay_on_the_device(cuda, op, count):
         agent.close()
 
 
+def test_lists_beyond_the_longest_stay_on_the_host(cuda):
+    """A list of more than 2^22 entries takes no device memory (16 bytes an entry, rounded up to a
+    power of two, would be 128 MiB), and its requests are lowered on the host as before."""
+    import torch
+    rng = np.random.default_rng(11)
+    n, count = (1 << 22) + 1000, 2000
+    mem = torch.randint(0, 256, (2 * 160 * n,), dtype=torch.uint8, device=cuda)
+    offsets = np.arange(n, dtype=np.uint64) * np.uint64(160)
+    lens = np.where(np.arange(n) % 5000 < 2500, 128, 144).astype(np.uint64)  # no stride holds for more than 2500 entries
+    agent = nixl_agent("longlist", nixl_agent_config(backends=("HIP",)))
+    try:
+        agent.register_memory([mem])
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        local, remote = (agent.prep_xfer_dlist(who, np.stack([np.uint64(mem.data_ptr() + at) + offsets, lens, np.zeros(n, np.uint64)], 1), "VRAM")
+                         for who, at in (("", 0), (agent.name, 160 * n)))
+        assert free - torch.cuda.mem_get_info()[0] < 64 << 20
+        idx = rng.permutation(n)[:count].astype(np.int32)
+        want = mem.clone()
+        for i in idx:
+            o, b = 160 * int(i), int(lens[i])
+            want[160 * n + o:160 * n + o + b] = mem[o:o + b]
+        torch.cuda.synchronize()
+        req = agent.make_prepped_xfer("WRITE", local, idx, remote, idx)
+        _wait(agent, req)
+        assert torch.equal(mem, want)
+        req.release()
+        for h in (local, remote):
+            h.release()
+    finally:
+        agent.close()
+
+
+def test_released_lists_leave_the_memory_of_requests_in_its_cache(cuda):
+    """Device-resident lists come and go (five of 64 MiB): the device memory that a request gave
+    back is still there for the next one of its size, and nothing is allocated for it."""
+    import torch
+    lib = _lib.kernels()
+    mem = torch.zeros(8192, dtype=torch.uint8, device=cuda)
+    n, entries = (1 << 20) + 1, (1 << 21) + 1  # 32 MiB of records, 64 MiB of entries
+    run = _lib.CopyRun(mem.data_ptr(), 8192, 0, 1)
+    idx = np.zeros(n, np.int32)
+    table = np.zeros(entries, dtype=[("addr", "<u8"), ("len", "<u4"), ("continues", "<u4")])
+    table["addr"], table["len"] = mem.data_ptr(), 128
+
+    def make_plan():
+        plan = ctypes.c_void_p()
+        rc = lib.nixl_amd_copy_plan_create_indexed_runs(ctypes.byref(run), 1, idx.ctypes.data, ctypes.byref(run), 1, idx.ctypes.data, n, 8192,
+                                                        0, None, ctypes.byref(plan))
+        assert rc == 0, _lib.kernels_error()
+        torch.cuda.synchronize()
+        return plan
+
+    assert lib.nixl_amd_copy_plan_destroy(make_plan()) == 0
+    lists = []
+    for _ in range(5):
+        lists.append(ctypes.c_void_p())
+        assert lib.nixl_amd_copy_list_create(table.ctypes.data, entries, 0, ctypes.byref(lists[-1])) == 0, _lib.kernels_error()
+    for one in lists:
+        assert lib.nixl_amd_copy_list_destroy(one) == 0
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    plan = make_plan()
+    taken = free - torch.cuda.mem_get_info()[0]
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+    assert taken < 16 << 20
+
+
 @pytest.mark.parametrize("count", [65535, 65536, 65537, 131072 + 300])
 def test_listed_requests_lowered_in_slices(cuda, count):
     """Pairs against device-resident lists around the number one launch of the records kernel
