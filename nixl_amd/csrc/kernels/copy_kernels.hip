@@ -48,7 +48,9 @@ namespace {
 constexpr int kMixedWaves = 4; // waves per workgroup of the mixed and byte-path kernels
 constexpr int kMixedThreads = kWaveSize * kMixedWaves;
 constexpr int kGenericLoads = 4; // 16-byte loads a lane keeps in flight for a byte-path work item
-constexpr uint32_t kGenericItemBytes = kWaveSize * kGenericLoads * 16; // reach of an item, from the destination line it starts in
+// Reach of an item, from the destination line it starts in: one round of those loads, or (a few
+// long tensors, where the items are what the plan's making costs) four.
+constexpr uint32_t kGenericRound = kWaveSize * kGenericLoads * 16, kGenericItemBytes = 4 * kGenericRound;
 constexpr int kMaxLdsDescs = 64; // descriptors a wave stages in LDS for one chunk
 constexpr int kNumXcd = 8; // accelerator dies; workgroup i is dispatched to die i % 8
 
@@ -320,10 +322,11 @@ copy_mixed_kernel(MixedArgs a) {
 }
 
 // One wavefront per byte-range work item; correct for any alignment and length.  An item ends
-// at most kGenericItemBytes behind the destination line it starts in (the plan cuts them so), so
-// its body of whole 16-byte units is at most kGenericLoads instructions wide with lane 0 of each
-// on a destination line, as in the piece kernel; loads take their 16 bytes from any address.
-// All loads of an item (body, up to 15 head and 15 tail bytes) are in flight before the first
+// at most kGenericRound (or kGenericItemBytes) behind the destination line it starts in (the plan
+// cuts them so), so its body of whole 16-byte units is one round (or four) of kGenericLoads
+// instructions with lane 0 of each on a destination line, as in the piece kernel; loads take
+// their 16 bytes from any address.
+// All loads of a round (body, up to 15 head and 15 tail bytes) are in flight before its first
 // store: what bounds a list of a few thousand such descriptors is that round trip and the
 // number of waves sharing it, not bytes (3000 descriptors of up to 64 KiB, 18 MB: 7 us; with items
 // of 16 KiB whose lanes had one load in flight a 64 KiB descriptor alone was 64 of those trips
@@ -353,19 +356,20 @@ copy_generic_kernel(const GenericItem *items, uint32_t n_items) {
         uint8_t first = 0, last = 0;
         if (lane < head) first = *(byte_cptr)(src + lane);
         if (lane < tail) last = *(byte_cptr)(src + done + lane);
-        v4u v[kGenericLoads];
-        if (body) {
-            // unconditional, as in the piece kernel: a lane outside the body re-reads its first
-            // or last unit
+        // unconditional, as in the piece kernel: a lane outside the body re-reads its first or last
+        // unit (an item without a body has no round)
+        const uint32_t end = body ? body + shift : 0;
+        for (uint32_t round = 0; round < end; round += kGenericLoads * kWaveSize) {
+            v4u v[kGenericLoads];
 #pragma unroll
             for (int k = 0; k < kGenericLoads; ++k) {
-                const uint32_t at = k * kWaveSize + lane;
+                const uint32_t at = round + k * kWaveSize + lane;
                 const uint32_t u = min(at < shift ? 0u : at - shift, body - 1);
                 v[k] = *(any_cptr)(src + head + u * 16ull);
             }
 #pragma unroll
             for (int k = 0; k < kGenericLoads; ++k) {
-                const uint32_t at = k * kWaveSize + lane;
+                const uint32_t at = round + k * kWaveSize + lane;
                 if (at >= shift && at - shift < body) store16<kPolNtNt>(dst + head + (at - shift) * 16ull, v[k]);
             }
         }
@@ -1065,6 +1069,30 @@ end_build(nixl_amd_copy_plan *plan, hipStream_t up, void *staging, size_t stagin
     return e;
 }
 
+static GenericItem
+generic_item(uint64_t src, uint64_t dst, uint64_t len) {
+    return GenericItem{src | (len - 1) >> 8 << kPieceUnitsShift, dst | ((len - 1) & 255u) << kPieceUnitsShift};
+}
+
+// Byte-range items while a plan is made.  Room for all items of a descriptor is made before the
+// first of them is written: appended one by one to a vector, making a plan took 106 us for
+// 14 394 descriptors of up to 16 KiB (61 with this), 24 for 3000 of up to 64 KiB (19).
+struct GenericItems {
+    std::unique_ptr<GenericItem[]> at;
+    size_t n = 0, cap = 0;
+
+    GenericItem *
+    room(size_t more, size_t expected) {
+        if (cap - n < more) {
+            cap = std::max(2 * cap, n + more + expected);
+            std::unique_ptr<GenericItem[]> grown(new GenericItem[cap]);
+            if (n) std::memcpy(grown.get(), at.get(), n * sizeof(GenericItem));
+            at = std::move(grown);
+        }
+        return at.get() + n;
+    }
+};
+
 constexpr int kNotBlocks = 1; // build_block_plan: the records are not what a block plan takes (no error recorded)
 
 // A plan of `n_recs` equal blocks of `len` bytes whose {src, dst} records the host has written
@@ -1238,20 +1266,42 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
 
     // ---- host-side lowering ------------------------------------------------------
     std::vector<uint64_t> vsrc, vdst, vprefix;
-    std::vector<GenericItem> items;
+    GenericItems items;
     std::vector<PieceRec> pieces;
     // Descriptors of 256 B to 8 KiB, and longer ones whose source or destination does not
     // start on a 128-byte line, go to the piece kernel: measured faster there (fewer lines
     // split between wavefronts); line-aligned long descriptors stream best in 1 KiB chunks.
     constexpr uint64_t kPieceMinUnits = 16, kPieceMaxDescUnits = 512;
+    // Long byte descriptors: see where they are placed.  Beyond kLongItemsFrom of them the items take
+    // four rounds each, as making four times as many costs more than the copy gains (64 MiB in
+    // tensors of 1 MiB, 6 bytes off: 38 us to make and 20.3 to copy with short items, 11.6 and 21.8 with long).
+    constexpr uint64_t kLongItemsFrom = 8ull << 20;
     constexpr uint64_t kSplitFromBytes = 64 * 1024; // at least two chunks of the largest size besides a first line
     vsrc.reserve(n);
     vdst.reserve(n);
     vprefix.reserve(n + 1);
     pieces.reserve(n);
-    uint64_t units = 0, payload = 0, n_generic_descs = 0, n_piece_descs = 0, n_split = 0;
+    uint64_t units = 0, payload = 0, n_generic_descs = 0, n_piece_descs = 0;
+    std::vector<uint32_t> long_bytes; // byte descriptors of kSplitFromBytes and more, placed when the others are known
+    uint64_t long_total = 0, splittable_total = 0;
+    uint64_t item_bytes = kGenericRound;
+    const auto splittable = [](const nixl_amd_copy_desc_t &d) { return ((d.src ^ d.dst) & 127u) == 0; };
+    // Byte-range items of `len` bytes; every one but the first starts on a destination line.
+    // (Inlined by force: called, the state it shares with the loop goes through memory, 3 ns a descriptor.)
+    const auto byte_items = [&](uint64_t src, uint64_t dst, uint64_t len) __attribute__((always_inline)) {
+        if (len == 0) return;
+        GenericItem *at = items.room(len / item_bytes + 2, 2 * n);
+        for (uint64_t reach = item_bytes - (dst & 127u); len > reach; reach = item_bytes) {
+            *at++ = generic_item(src, dst, reach);
+            src += reach;
+            dst += reach;
+            len -= reach;
+        }
+        *at++ = generic_item(src, dst, len);
+        items.n = static_cast<size_t>(at - items.at.get());
+    };
     for (size_t i = 0; i < n; ++i) {
-        const nixl_amd_copy_desc_t &d = descs[i];
+        const nixl_amd_copy_desc_t d = descs[i]; // a copy: what is written below may not be taken to change it
         if (d.len == 0) continue;
         if (d.src == 0 || d.dst == 0)
             return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create: null address in descriptor " + std::to_string(i));
@@ -1282,38 +1332,39 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             ++n_generic_descs;
             if (((d.src + d.len) | (d.dst + d.len)) >> kPieceUnitsShift)
                 return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create: address beyond 2^56");
-            // every item but the first starts on a destination line
-            const auto byte_items = [&](uint64_t off, uint64_t end) {
-                while (off < end) {
-                    const uint64_t reach = kGenericItemBytes - ((d.dst + off) & 127u);
-                    const uint32_t len = static_cast<uint32_t>(std::min<uint64_t>(reach, end - off));
-                    items.push_back(GenericItem{(d.src + off) | static_cast<uint64_t>((len - 1) >> 8) << kPieceUnitsShift,
-                                                (d.dst + off) | static_cast<uint64_t>((len - 1) & 255u) << kPieceUnitsShift});
-                    off += len;
-                }
-            };
-            // A long one whose two ends lie at the same place inside their lines (tensors whose
-            // size is no multiple of 16) is whole chunks but for its first line and its last
-            // chunk: only those go byte by byte.
-            const uint64_t head = (0 - d.dst) & 127u;
-            if (d.len >= kSplitFromBytes && ((d.src ^ d.dst) & 127u) == 0) {
-                const uint64_t body = (d.len - head) / (chunk_units * 16u) * (chunk_units * 16u);
-                if (head) byte_items(0, head);
-                vsrc.push_back(d.src + head);
-                vdst.push_back(d.dst + head);
-                vprefix.push_back(units);
-                units += body / 16u;
-                ++n_split;
-                byte_items(head + body, d.len);
+            if (d.len >= kSplitFromBytes) {
+                long_bytes.push_back(static_cast<uint32_t>(i));
+                long_total += d.len;
+                if (splittable(d)) splittable_total += d.len;
             } else {
-                byte_items(0, d.len);
+                byte_items(d.src, d.dst, d.len);
             }
         }
+    }
+    // A long byte descriptor whose two ends lie at the same place inside their lines (tensors whose
+    // size is no multiple of 16) is whole chunks but for its first line and its last chunk: only
+    // those go byte by byte.
+    if (long_total - splittable_total > kLongItemsFrom) item_bytes = kGenericItemBytes;
+    size_t n_split = 0;
+    for (const uint32_t i : long_bytes) {
+        const nixl_amd_copy_desc_t &d = descs[i];
+        if (!splittable(d)) {
+            byte_items(d.src, d.dst, d.len);
+            continue;
+        }
+        const uint64_t head = (0 - d.dst) & 127u, body = (d.len - head) / (chunk_units * 16u) * (chunk_units * 16u);
+        byte_items(d.src, d.dst, head);
+        byte_items(d.src + head + body, d.dst + head + body, d.len - head - body);
+        vsrc.push_back(d.src + head);
+        vdst.push_back(d.dst + head);
+        vprefix.push_back(units);
+        units += body / 16u;
+        ++n_split;
     }
     vprefix.push_back(units);
     const size_t nv = vsrc.size();
     const uint64_t n_chunks64 = (units + chunk_units - 1) / chunk_units;
-    if (n_chunks64 >= (1ull << 32) || items.size() >= (1ull << 32) || pieces.size() >= (1ull << 31))
+    if (n_chunks64 >= (1ull << 32) || items.n >= (1ull << 32) || pieces.size() >= (1ull << 31))
         return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "plan_create: request too large for 32-bit chunk index");
     const uint32_t n_chunks = static_cast<uint32_t>(n_chunks64);
 
@@ -1411,7 +1462,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     const size_t off_mixed = off_span + (need_desc_arrays ? align256(span.size() * sizeof(uint2)) : 0);
     const size_t off_pieces = off_mixed + align256(mixed.size() * sizeof(uint32_t));
     const size_t off_items = off_pieces + align256(pieces.size() * sizeof(PieceRec));
-    const size_t off_runs = off_items + align256(items.size() * sizeof(GenericItem));
+    const size_t off_runs = off_items + align256(items.n * sizeof(GenericItem));
     const size_t off_first = off_runs + (expand ? align256(uni.size() * sizeof(UniformRec)) : 0);
     const size_t total = off_first + (expand ? align256(first_chunk.size() * sizeof(uint32_t)) : 0);
     const size_t upload_from = expand ? off_src : 0;
@@ -1467,7 +1518,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             std::memcpy(host(off_mixed), mixed.data(), mixed.size() * sizeof(uint32_t));
         }
         if (!pieces.empty()) std::memcpy(host(off_pieces), pieces.data(), pieces.size() * sizeof(PieceRec));
-        if (!items.empty()) std::memcpy(host(off_items), items.data(), items.size() * sizeof(GenericItem));
+        if (items.n) std::memcpy(host(off_items), items.at.get(), items.n * sizeof(GenericItem));
         e = arena_cache().get(device, total, &plan->arena, &plan->arena_cap);
         if (e != hipSuccess) {
             upload_cache().put(device, staging, staging_cap);
@@ -1512,7 +1563,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->chunks_per_rec = chunks_per_rec;
     plan->mixed_args.total_units = units;
     plan->mixed_args.n_mixed = static_cast<uint32_t>(mixed.size());
-    plan->n_generic = static_cast<uint32_t>(items.size());
+    plan->n_generic = static_cast<uint32_t>(items.n);
 
     auto wgs_for = [&](uint32_t n_waves, uint32_t waves_per_wg, bool cap) {
         uint32_t w = (n_waves + waves_per_wg - 1) / waves_per_wg;

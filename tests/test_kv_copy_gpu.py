@@ -222,6 +222,29 @@ def test_runs_of_different_lengths_are_expanded_on_the_device(cuda):
     assert info.plan_device_bytes >= info.uniform_chunks * 16
 
 
+@pytest.mark.parametrize("copies,reach", [(1, 4096), (6, 16384)])
+def test_items_of_long_byte_descriptors(cuda, copies, reach):
+    """Long descriptors whose two sides lie differently inside their lines: byte-range items of one
+    round of the kernel's loads while the request has no more than 8 MiB of them, of four beyond
+    (that many short items took 160 us to make for 256 MiB).  Lengths around whole items at several
+    destination offsets; every byte against the oracle, and the number of items."""
+    import torch
+    lens, src_off, dst_off, at = [], [], [], 0
+    for c in range(copies):
+        for k in (4, 5, 6):
+            for extra in (0, 1, 15, 16, 17, 112, 127, 128, 129):
+                lens.append(16384 * k + extra)
+                dst_off.append(at + (7, 0, 16, 113, 127, 64)[c])
+                src_off.append(at + (7, 0, 16, 113, 127, 64)[c] + 1 + (extra + c) % 64)
+                at += 16384 * k + 512
+    half = at
+    info = _check_against_oracle(torch, cuda, 2 * half, src_off, [half + d for d in dst_off], lens, seed=copies)
+    assert (sum(lens) > 8 << 20) == (reach == 16384) and half % 128 == 0
+    assert info.generic_descs == len(lens) and info.uniform_chunks == 0
+    first = [reach - d % 128 for d in dst_off]  # the memory starts on a line
+    assert info.generic_items == sum(1 + -(-max(0, n - f) // reach) for n, f in zip(lens, first))
+
+
 def test_zero_length_and_empty(cuda):
     import torch
     dev = torch.zeros(4096, dtype=torch.uint8, device=cuda)
