@@ -1274,8 +1274,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     constexpr uint64_t kPieceMinUnits = 16, kPieceMaxDescUnits = 512;
     // Long byte descriptors: see where they are placed.  Beyond kLongItemsFrom of them the items take
     // four rounds each, as making four times as many costs more than the copy gains (64 MiB in
-    // tensors of 1 MiB, 6 bytes off: 38 us to make and 20.3 to copy with short items, 11.6 and 21.8 with long).
-    constexpr uint64_t kLongItemsFrom = 8ull << 20;
+    // tensors of 1 MiB + 2 B: 24 us to make and 20.6 to copy with short items, 10.7 and 22.0 with long).
+    constexpr uint64_t kSplitFromTotal = 128ull << 20, kLongItemsFrom = 8ull << 20;
     constexpr uint64_t kSplitFromBytes = 64 * 1024; // at least two chunks of the largest size besides a first line
     vsrc.reserve(n);
     vdst.reserve(n);
@@ -1284,6 +1284,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     uint64_t units = 0, payload = 0, n_generic_descs = 0, n_piece_descs = 0;
     std::vector<uint32_t> long_bytes; // byte descriptors of kSplitFromBytes and more, placed when the others are known
     uint64_t long_total = 0, splittable_total = 0;
+    bool whole_chunks = false; // some descriptor brings the stream whole chunks whatever becomes of those
     uint64_t item_bytes = kGenericRound;
     const auto splittable = [](const nixl_amd_copy_desc_t &d) { return ((d.src ^ d.dst) & 127u) == 0; };
     // Byte-range items of `len` bytes; every one but the first starts on a destination line.
@@ -1324,6 +1325,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             }
             ++n_piece_descs;
         } else if (aligned16) {
+            whole_chunks |= du >= kPieceMaxDescUnits;
             vsrc.push_back(d.src);
             vdst.push_back(d.dst);
             vprefix.push_back(units);
@@ -1343,23 +1345,37 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     }
     // A long byte descriptor whose two ends lie at the same place inside their lines (tensors whose
     // size is no multiple of 16) is whole chunks but for its first line and its last chunk: only
-    // those go byte by byte.
-    if (long_total - splittable_total > kLongItemsFrom) item_bytes = kGenericItemBytes;
-    size_t n_split = 0;
+    // those go byte by byte.  These chunks go in front of the stream, where they lie on their own
+    // lines and move nobody else's.  Without chunks of other descriptors that is one launch more, and
+    // up to kSplitFromTotal (both sides in the 256 MB last-level cache) the byte kernel alone is as
+    // fast or faster: 32 tensors of 1 MiB + 2 B 12.3 us instead of 15.0, 128 of them 36.9 and 45.4;
+    // 256 of them 90 us and a plan that takes 25 us to make, instead of 84 and 9.
+    const bool join = whole_chunks || splittable_total >= kSplitFromTotal;
+    if (long_total - (join ? splittable_total : 0) > kLongItemsFrom) item_bytes = kGenericItemBytes;
+    std::vector<uint64_t> front_src, front_dst, front_prefix;
+    uint64_t front_units = 0;
     for (const uint32_t i : long_bytes) {
         const nixl_amd_copy_desc_t &d = descs[i];
-        if (!splittable(d)) {
+        if (!join || !splittable(d)) {
             byte_items(d.src, d.dst, d.len);
             continue;
         }
         const uint64_t head = (0 - d.dst) & 127u, body = (d.len - head) / (chunk_units * 16u) * (chunk_units * 16u);
         byte_items(d.src, d.dst, head);
         byte_items(d.src + head + body, d.dst + head + body, d.len - head - body);
-        vsrc.push_back(d.src + head);
-        vdst.push_back(d.dst + head);
-        vprefix.push_back(units);
-        units += body / 16u;
-        ++n_split;
+        front_src.push_back(d.src + head);
+        front_dst.push_back(d.dst + head);
+        front_prefix.push_back(front_units);
+        front_units += body / 16u;
+    }
+    const size_t n_split = front_src.size();
+    if (n_split) {
+        vsrc.insert(vsrc.begin(), front_src.begin(), front_src.end());
+        vdst.insert(vdst.begin(), front_dst.begin(), front_dst.end());
+        for (uint64_t &p : vprefix)
+            p += front_units;
+        vprefix.insert(vprefix.begin(), front_prefix.begin(), front_prefix.end());
+        units += front_units;
     }
     vprefix.push_back(units);
     const size_t nv = vsrc.size();

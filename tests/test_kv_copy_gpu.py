@@ -245,6 +245,37 @@ def test_items_of_long_byte_descriptors(cuda, copies, reach):
     assert info.generic_items == sum(1 + -(-max(0, n - f) // reach) for n, f in zip(lens, first))
 
 
+def test_split_tensors_keep_to_their_lines_and_others_to_theirs(cuda):
+    """Long tensors of odd lengths beside aligned ones that are no whole number of chunks: the odd
+    ones' chunks start on their own lines, so that no chunk more than without them has to be put
+    together from several descriptors.  Alone and small, they are not split (no launch for a few
+    chunks); alone and large, they are."""
+    import torch
+
+    def place(lens):
+        offs = np.concatenate([[0], np.cumsum([(n + 1023) // 128 * 128 for n in lens])])
+        half = int(offs[-1])
+        return 2 * half, offs[:-1] + 2, half + offs[:-1] + 2
+
+    aligned, odd = [4120416, 1048576 + 48, 300016], [1048578, 300002, 65536 + 126, 2097151]
+    mem, so, do = place(aligned)
+    base = _check_against_oracle(torch, cuda, mem, so - 2, do - 2, aligned, seed=1)
+    assert base.mixed_chunks > 0
+    for lens in (aligned + odd, odd + aligned, [aligned[0], odd[0], aligned[1], odd[1], aligned[2], odd[2], odd[3]]):
+        mem, so, do = place(lens)
+        shift = np.array([2 if n in odd else 0 for n in lens])  # the odd ones start two bytes into a line
+        info = _check_against_oracle(torch, cuda, mem, so - 2 + shift, do - 2 + shift, lens, seed=2)
+        assert info.mixed_chunks == base.mixed_chunks
+        assert info.uniform_chunks == base.uniform_chunks + sum((n - 126) // 1024 for n in odd)
+    mem, so, do = place(odd)
+    info = _check_against_oracle(torch, cuda, mem, so, do, odd, seed=3)
+    assert info.uniform_chunks == 0 and info.mixed_chunks == 0 and info.generic_descs == len(odd)
+    large = [(64 << 20) + 2] * 2
+    mem, so, do = place(large)
+    info = _check_against_oracle(torch, cuda, mem, so, do, large, seed=4)
+    assert info.uniform_chunks == 2 * (((64 << 20) - 124) // 1024) and info.mixed_chunks == 0
+
+
 def test_zero_length_and_empty(cuda):
     import torch
     dev = torch.zeros(4096, dtype=torch.uint8, device=cuda)
