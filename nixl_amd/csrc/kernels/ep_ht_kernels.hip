@@ -753,6 +753,26 @@ ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint3
     dispatch_piece(a, (first + block - meta_blocks) * kHtWaves + uniform(threadIdx.x / kWaveSize));
 }
 
+// From this many ranks on, the metadata has a launch of its own: a workgroup of it finds one token in
+// R / K of its own and is soon gone, and the three kinds' arguments and branches in front
+// of it cost more than the launch.  Metadata alone at 64 ranks x 4096 tokens, top-4: 79 us by its own
+// kernel, 129 by the common one; whole dispatches there 1286 -> 1254 us, 64 x 3000 x 512 fp8
+// 1121 -> 1080, 128 x 3000 x 512 4510 -> 4370, 32 x 3000 x 512 325 -> 317; 24 x 4096 256 -> 262,
+// 16 x 4096 141 -> 142, 8 x 4096 61 -> 67.
+constexpr int kHtMetaApartRanks = 32;
+
+template<bool VEC>
+__global__ void __launch_bounds__(kHtMetaThreads)
+ht_meta_kernel(HtMeta m,
+               const uint8_t *__restrict__ in_rank,
+               const int *__restrict__ prefix,
+               const int *__restrict__ send_head,
+               const long long *__restrict__ row_offset,
+               HtDims d,
+               uint32_t first) {
+    meta_block<VEC>(m, in_rank, prefix, send_head, row_offset, d, first + blockIdx.x);
+}
+
 // ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
 // grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x of them,
 // every wave for itself.  Two forms: up to kHtCombineEager values of output, four waves a
@@ -1074,13 +1094,24 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
         HIP_TRY(hipGetLastError());
         return NIXL_AMD_OK;
     };
-    if (scale_blocks + meta_blocks + row_blocks <= kHtMaxGrid) return launch(scale_blocks, meta_blocks, row_blocks, 0);
-    const long long part_blocks[3] = {row_blocks, scale_blocks, meta_blocks};
-    for (int part = 0; part < 3; ++part)
-        for (long long at = 0; at < part_blocks[part]; at += kHtMaxGrid) {
-            const long long n = std::min(kHtMaxGrid, part_blocks[part] - at);
-            if (const int status = launch(part == 1 ? n : 0, part == 2 ? n : 0, part == 0 ? n : 0, at)) return status;
-        }
+    const bool meta_apart = num_ranks >= kHtMetaApartRanks;
+    const long long with_rows = meta_apart ? 0 : meta_blocks;
+    if (scale_blocks + with_rows + row_blocks <= kHtMaxGrid) {
+        if (const int status = launch(scale_blocks, with_rows, row_blocks, 0)) return status;
+    } else {
+        const long long part_blocks[3] = {row_blocks, scale_blocks, with_rows};
+        for (int part = 0; part < 3; ++part)
+            for (long long at = 0; at < part_blocks[part]; at += kHtMaxGrid) {
+                const long long n = std::min(kHtMaxGrid, part_blocks[part] - at);
+                if (const int status = launch(part == 1 ? n : 0, part == 2 ? n : 0, part == 0 ? n : 0, at)) return status;
+            }
+    }
+    for (long long at = 0; at < meta_blocks - with_rows; at += kHtMaxGrid) {
+        hipLaunchKernelGGL(vec ? ht_meta_kernel<true> : ht_meta_kernel<false>,
+                           dim3(static_cast<unsigned>(std::min(kHtMaxGrid, meta_blocks - at))), dim3(kHtMetaThreads), 0, s, meta,
+                           is_token_in_rank, prefix, send_head, offsets, d, static_cast<uint32_t>(at));
+        HIP_TRY(hipGetLastError());
+    }
     return NIXL_AMD_OK;
 }
 
