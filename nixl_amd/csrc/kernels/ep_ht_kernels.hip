@@ -52,12 +52,18 @@ block_exclusive_scan(V v, V *wave_sums, V &total) {
 // counters per workgroup, added to the (zeroed) outputs at the end.  Integer sums: the
 // result does not depend on the order of the additions.  A rank of at most kLayoutWhole tokens
 // and kLayoutWholeSelections selections is one chunk, whose counters are the result: nothing to
-// clear and nothing to add (8 x 1024 tokens top-4: 6.1 -> 4.6 us, 4 x 333 top-6: 6.7 -> 4.1).
-// Beyond, the LDS atomics of a single workgroup cost more than a second launch: 8 x 1024 top-8
-// 5.7 us in chunks, 7.6 whole.
+// clear and nothing to add (GPU time, one chunk against several: 8 x 1024 tokens top-4 4.1 and 4.7 us,
+// 4 x 512 top-2 2.8 and 4.4, 8 x 512 top-8 4.8 and 5.4; top-6 of 1024 is even, 4.8 and 5.2).  Beyond, the
+// LDS atomics of a single workgroup cost more than a second launch: 8 x 1024 top-8 7.6 and 5.5, 8 x 512
+// top-16 7.7 and 7.2.  So do the flags of many ranks, R bytes a token by one thread, beyond
+// kLayoutWholeFlags a rank: 32 x 768 tokens 5.0 and 5.1 us, 32 x 1024 5.9 and 5.1, 64 x 384 5.5 and 7.0, 64 x 768
+// 8.7 and 8.1, 128 x 384 42 and 37; a single chunk of kLayoutTokens tokens is one workgroup either way, and
+// from 256 ranks on one workgroup a rank fills the chip (256 x 384 121 and 159, 256 x 1024 327 and 592).
 constexpr int kLayoutTokens = 256;
 constexpr int kLayoutWhole = 1024;
 constexpr int kLayoutWholeSelections = 4096;
+constexpr int kLayoutWholeFlags = 24576;
+constexpr int kLayoutWholeRanks = 256;
 
 __global__ void __launch_bounds__(256)
 zero_ints_kernel(int *__restrict__ a, size_t na, int *__restrict__ b, size_t nb) {
@@ -776,12 +782,15 @@ ht_meta_kernel(HtMeta m,
 // ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
 // grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x of them,
 // every wave for itself.  Two forms: up to kHtCombineEager values of output, four waves a
-// workgroup and positions loaded beside the flags (EAGER), which shortens the chain of loads
-// (8 x 1024 x 4096: 52.8 -> 48.8 us, 2 x 4096 x 4096: 40.4 -> 36.2, 4 x 1500 x 4096: 36.6 ->
-// 32.7 against a workgroup whose first wave finds the rows for both).  Beyond, that many rows
-// in flight cost bandwidth (8 x 2048 x 7168: 247 us, 8 x 4096: 494): one wave a workgroup and
-// positions behind the flags, 231 and 457, is what those calls took with the shared look-up as
-// well (8 x 1024 x 7168: 112 -> 109, 4 x 4096: 181 -> 175).
+// workgroup and positions loaded beside the flags (EAGER), which shortens the chain of loads;
+// beyond, one wave a workgroup and positions behind the flags.  Which is faster depends on the
+// rows a token gathers more than on the size: with few of them the eager form at every size (2 ranks
+// x 4096 x 4096 35.3 us against 41.6, 2 x 16 384 130 and 157; 8 x 1024 top-4 48.4 and 52.4, 8 x 4096 182 and 200),
+// with 5.3 a token the other one from 2^24 values on, ever more so (8 x 206 x 7168 top-8 27.8 and 27.0, 8 x 585
+// 71 and 68, 8 x 2340 283 and 261; 16 x 512 x 4096 85.5 and 84.6, 16 x 2048 352 and 340).  The number of
+// rows is not known here.  With the line at 2^25 values, calls below it that gather many rows lose up
+// to 4 % and calls above it that gather few up to 17 %, against the other form; neither is slower than
+// the look-up shared by two waves that came before both (8 x 1024 x 4096 52.8, 2 x 4096 x 4096 40.4).
 constexpr int kHtCombineEagerLanes = 256;
 constexpr long long kHtCombineEager = 1ll << 25;
 
@@ -947,7 +956,9 @@ nixl_amd_ep_get_dispatch_layout(const int32_t *topk_idx,
     const size_t lds = static_cast<size_t>(num_experts + num_ranks) * sizeof(int);
     if (lds > 48 * 1024) return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "get_dispatch_layout: too many experts");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (num_tokens <= kLayoutWhole && num_tokens * num_topk <= kLayoutWholeSelections) {
+    const bool flags_fit = num_tokens <= kLayoutTokens || num_ranks >= kLayoutWholeRanks ||
+                           static_cast<long long>(num_tokens) * num_ranks <= kLayoutWholeFlags;
+    if (num_tokens <= kLayoutWhole && num_tokens * num_topk <= kLayoutWholeSelections && flags_fit) {
         hipLaunchKernelGGL(layout_kernel, dim3(static_cast<unsigned>(num_ranks)), dim3(round_up_wave(num_tokens)), lds, s, topk_idx,
                            num_tokens_per_rank, num_tokens_per_expert, is_token_in_rank, num_tokens, num_topk, num_ranks,
                            num_experts);

@@ -480,10 +480,12 @@ def test_ht_pipeline_matches_oracle(cuda, shape):
 # flags are counted beside the scan, 32 832 behind it; 66 ranks take two steps of 64 in every
 # wave, and 33 lanes leave a wave half idle; 33.7 million values are combined in the form for
 # large calls.  From 32 ranks on the metadata has a launch of its own (31 and 32; 257 tokens leave
-# one to its second workgroup; selections by fours and one by one).
+# one to its second workgroup; selections by fours and one by one), and 24 576 flags a rank are
+# the most that one workgroup writes: 768 tokens of 32 ranks, 769 of them by several.
 @pytest.mark.parametrize("shape", [(8, 512, 128, 8, 16, 4, 1), (8, 513, 128, 8, 16, 4, 1), (1, 1024, 256, 4, 4, 2, 1),
                                    (2, 1025, 256, 2, 4, 2, 1), (66, 5, 264, 4, 66, 2, 1), (4, 1030, 8192, 2, 8, 4, 1),
-                                   (31, 9, 256, 4, 62, 2, 1), (32, 9, 256, 4, 64, 2, 1), (32, 257, 128, 3, 32, 2, 1)])
+                                   (31, 9, 256, 4, 62, 2, 1), (32, 9, 256, 4, 64, 2, 1), (32, 257, 128, 3, 32, 2, 1),
+                                   (32, 768, 128, 2, 32, 2, 1), (32, 769, 128, 2, 32, 2, 1)])
 def test_ht_pipeline_at_the_edges_of_its_launch_forms(cuda, shape):
     test_ht_pipeline_matches_oracle(cuda, shape)
 
