@@ -1137,6 +1137,50 @@ def test_block_plans_inline_and_on_the_callers_stream(cuda, n, n_runs, named):
     torch.cuda.synchronize()
 
 
+def test_threads_make_and_launch_plans_on_one_stream(cuda):
+    """Four threads make plans that name the same stream and launch them on it, each waiting for
+    its own: plans are built there or, while another thread's work keeps it busy, on the library's
+    stream, and pinned buffers change hands between the threads.  Every thread checks its bytes
+    after every launch; every fourth plan is dropped without one."""
+    import threading
+    import torch
+    lib = _lib.kernels()
+    n, blk, pool, rounds = 1500, 8192, 1600, 40
+    stream = torch.cuda.Stream()
+    faults = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        src = torch.randint(0, 256, (pool, blk), dtype=torch.uint8, device=cuda)
+        dst = torch.zeros_like(src)
+        torch.cuda.synchronize()
+        run_s, run_d = (_lib.CopyRun(m.data_ptr(), blk, 0, pool) for m in (src, dst))
+        for i in range(rounds):
+            at, to = (rng.permutation(pool)[:n].astype(np.int32) for _ in range(2))
+            plan = ctypes.c_void_p()
+            tuning = _lib.CopyTuning(stream=stream.cuda_stream)
+            rc = lib.nixl_amd_copy_plan_create_indexed_runs(ctypes.byref(run_s), 1, at.ctypes.data, ctypes.byref(run_d), 1, to.ctypes.data,
+                                                            n, blk, 0, ctypes.byref(tuning), ctypes.byref(plan))
+            if rc == 0 and i % 4 != 3:
+                rc = lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream) or lib.nixl_amd_copy_plan_status(plan, 1)
+                at_t, to_t = (torch.from_numpy(x).to(cuda).long() for x in (at, to))
+                if rc == 0 and not torch.equal(dst[to_t], src[at_t]):
+                    rc = "wrong bytes"
+            if rc == 0:
+                rc = lib.nixl_amd_copy_plan_destroy(plan)
+            if rc != 0:
+                faults.append((seed, i, rc, _lib.kernels_error()))
+                return
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not faults
+
+
 @pytest.mark.parametrize("made", ["seen", "unseen", "other", "during"])
 def test_captured_launches_of_plans_that_name_a_stream(cuda, made):
     """A plan that names a stream is launched into a graph captured from that stream: made before
