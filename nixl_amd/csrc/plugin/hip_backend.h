@@ -191,8 +191,8 @@ public:
                     nixlBackendReqH *&handle) const;
 
     // The same for lists that share no stride: a list is handed over once, when it is prepared
-    // (entries of 128 to 8176 bytes, 16-byte aligned, on one device; NIXL_ERR_NOT_SUPPORTED
-    // otherwise), and stays on the device; requests against two such lists bring their index
+    // (at most 2^22 entries of 128 to 8176 bytes, 16-byte aligned, on one device;
+    // NIXL_ERR_NOT_SUPPORTED otherwise), and stays on the device; requests against two such lists bring their index
     // vectors, which a kernel checks and lowers.  `bytes` and `merged` receive the request's
     // size and the number of its descriptors after merging.  NIXL_ERR_NOT_SUPPORTED means "take
     // the ordinary path", which also names the pair when one is bad.  Reached through
