@@ -522,11 +522,18 @@ next_row(const WaveRows &w, unsigned long long &hits) {
 // Rows, scales and metadata in one launch (ht_dispatch_kernel below); these are its three parts.
 //
 // Rows: a wave owns 1 KiB of a row (`parts` waves a row), holds it in registers and stores it to
-// every row of the token.  Bound by the writes.  The loads are ordinary ones, since a layer's
-// input is usually still in the last-level cache that its producer filled, and the stores carry
-// device scope: against non-temporal loads and stores 8 x 4096 x 7168 bf16 (5.23 rows a token, inputs of
-// other calls in between) takes 469 us instead of 547, 8 x 1024 x 4096 (3.38) 49.5 instead of
-// 53; non-temporal stores behind ordinary loads 554 and 52, the other way round 502 and 49.4.
+// every row of the token.  Bound by the writes, which carry device scope.  Inputs of more than
+// kHtStreamFrom (half the last-level cache) are loaded non-temporally, smaller ones ordinarily:
+// what a large call loads pushes lines out of the cache that the kernel which made the input left
+// there.  8 x 4096 x 7168 bf16 with combine, one pass after another, us a pass with ordinary and with
+// non-temporal loads (and with non-temporal stores as well, before rows and metadata shared a
+// launch): an element-wise kernel on the input in front of every pass 1159 and 1106 (1116), one
+// that writes it from another tensor 1128 and 1118 (1131), a 512 MB fill 1103 and 1068 (1075), nothing
+// 957 and 979 (1012).  Dispatch alone behind the fill 568 and 525 (513), of fp8 rows with scales 305 and
+// 277 (289).  8 x 1024 x 4096 (67 MB) is the same either way behind a producer, and a dispatch
+// again and again takes 44 us with ordinary loads and 54 without.
+constexpr long long kHtStreamFrom = 128ll << 20;
+
 struct HtRows {
     uint16_t *recv_x;
     const uint16_t *x;
@@ -536,6 +543,7 @@ struct HtRows {
     const long long *row_offset;
     HtDims d;
     int parts;
+    int streamed; // rows are loaded non-temporally
 };
 
 __device__ __forceinline__ void
@@ -546,7 +554,10 @@ dispatch_piece(const HtRows &a, uint32_t piece) {
     const int col = part * kWaveSize + (threadIdx.x & (kWaveSize - 1));
     const bool active = col < a.d.H / 8;
     uint4 v = make_uint4(0, 0, 0, 0);
-    if (active) v = *(reinterpret_cast<const uint4 *>(a.x + static_cast<size_t>(token) * a.d.H) + col);
+    if (active) {
+        const uint4 *from = reinterpret_cast<const uint4 *>(a.x + static_cast<size_t>(token) * a.d.H) + col;
+        v = a.streamed ? ld16_nt(from) : *from;
+    }
     for (int d0 = 0; d0 < a.d.R; d0 += kWaveSize) {
         const WaveRows w = wave_rows<true>(a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, r, t, d0);
         for (unsigned long long hits = w.hits; hits;) {
@@ -1084,7 +1095,7 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
     const long long *offsets = reinterpret_cast<const long long *>(recv_row_offset);
     const int *prefix = recv_gbl_rank_prefix_sum;
     const HtRows rows{static_cast<uint16_t *>(recv_x), static_cast<const uint16_t *>(x), is_token_in_rank, prefix, send_head, offsets, d,
-                      parts};
+                      parts, static_cast<long long>(num_ranks) * num_tokens * d.H * 2 > kHtStreamFrom};
     const HtMeta meta{recv_topk_idx, recv_topk_weights, recv_src_meta, topk_idx, topk_weights};
     const HtScales sc{static_cast<uint32_t *>(recv_x_scales), static_cast<const uint32_t *>(x_scales), num_scales,
                       num_scales % 4 == 0 && reinterpret_cast<uintptr_t>(recv_x_scales) % 16 == 0, scale_rank_stride,
