@@ -773,7 +773,7 @@ ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint3
 // From this many ranks on, the metadata has a launch of its own: a workgroup of it finds one token in
 // R / K of its own and is soon gone, and the three kinds' arguments and branches in front
 // of it cost more than the launch.  Metadata alone at 64 ranks x 4096 tokens, top-4: 79 us by its own
-// kernel, 129 by the common one; whole dispatches there 1286 -> 1254 us, 64 x 3000 x 512 fp8
+// kernel, 129 by the common one; whole dispatches there, rows loaded ordinarily, 1286 -> 1254 us, 64 x 3000 x 512 fp8
 // 1121 -> 1080, 128 x 3000 x 512 4510 -> 4370, 32 x 3000 x 512 325 -> 317; 24 x 4096 256 -> 262,
 // 16 x 4096 141 -> 142, 8 x 4096 61 -> 67.
 constexpr int kHtMetaApartRanks = 32;
