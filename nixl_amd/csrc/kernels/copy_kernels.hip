@@ -42,6 +42,10 @@
 #include <mutex>
 #include <vector>
 
+#if defined(__x86_64__)
+#include <immintrin.h>
+#endif
+
 #include "common.h"
 
 namespace {
@@ -473,104 +477,179 @@ index_records_runs_kernel(UniformRec *recs, const int32_t *src_index, const int3
 // checks it (indices inside their lists, equal lengths) and writes the piece records of its
 // descriptor: the first at recs[i], those of a descriptor that spans several pieces behind the
 // n first ones, in whatever order the workgroups get there (the order of records decides
-// nothing about the bytes that arrive).  The index vectors are read where they are, in pinned
-// host memory: every index is read once, so a copy to the device first would only add its
-// latency.  The totals reach the host through pinned memory, written by the workgroup that
-// finishes last; the host waits for them, because a bad pair must fail the request.
-struct ListTotals {
-    unsigned long long bytes;
-    uint32_t bad; // pairs that name no entry or join entries of different lengths
-    uint32_t continued; // pairs that continue the pair before them inside one dense run on both sides
-    uint32_t extra; // records beyond the first of their pair
-    uint32_t arrived; // workgroups that have added theirs
+// nothing about the bytes that arrive).
+//
+// What bounds it is the way of the pairs over the bus, so they come in one of two forms, both read
+// where they are in pinned host memory (every word is read once, a copy to the device first would
+// only add its latency).  RUNS: stretches of pairs whose indices advance by one on both sides, as
+// those of a request that names blocks of consecutive entries, are 16 bytes each, and a workgroup
+// bisects the few that its pairs lie in; else the two vectors as they came, 8 bytes a pair.
+//
+// The verdict reaches the host through pinned memory, written by the workgroup that finishes last;
+// the host waits for it, because a bad pair must fail the request.  A workgroup adds to the totals
+// with two atomics (all dies add to one line).  Kernel time: 65 536 pairs as vectors 22.5 us with an
+// atomic for every descriptor of several pieces and four a workgroup of 256 pairs, 19.2 now; as
+// runs of 64 pairs 9.9, and 262 144 pairs 14.8 (as vectors in four launches 77).
+struct IndexRun {
+    uint32_t first; // pair the run starts with; it ends where the next one starts
+    uint32_t src, dst; // indices of that pair
+    uint32_t unused;
 };
 
-constexpr int kListThreads = 256;
-// Pairs a launch: while it reads them over the bus the host copies the next ones into the pinned
-// buffer.  262 144 pairs made, posted and waited for: 443 us in one launch, 382 in four, the
-// same in eight.
+// n < 2^31 pairs over the records a pair can have (plan_create_listed), so that a request's bytes stay
+// below 2^43 and its workgroups below or at 2^21.
+constexpr int kListBytesBits = 43;
+
+struct ListTotals {
+    unsigned long long bytes_arrived; // bytes of the good pairs | workgroups that have added theirs << kListBytesBits
+    // records beyond the first of their pair | pairs that continue the pair before them inside one
+    // dense run on both sides << 32
+    unsigned long long extra_continued;
+    uint32_t bad; // pairs that name no entry or join entries of different lengths
+};
+
+struct ListVerdict {
+    unsigned long long bytes;
+    uint32_t bad, continued, extra;
+    uint32_t there; // set last
+};
+
+constexpr int kListThreads = 1024;
+// Pairs a launch, where the vectors are sent as they came: while it reads them over the bus the host
+// copies the next ones into the pinned buffer.
 constexpr size_t kListSlice = 65536;
 static_assert(kListSlice % kListThreads == 0);
 
+struct ListArgs {
+    PieceRec *recs; // [n * pieces a descriptor can have]
+    const nixl_amd_copy_list_entry_t *src, *dst;
+    uint32_t n_src, n_dst;
+    const int32_t *src_index, *dst_index; // [n]
+    const IndexRun *runs; // instead
+    const uint32_t *run_of; // [n_workgroups + 1]: run that workgroup b's first pair lies in, then the last run
+    uint32_t first_workgroup; // of this launch; a plan's pairs may come in several
+    uint32_t n;
+    uint32_t n_workgroups; // of all launches together
+    ListTotals *totals; // cleared
+    ListVerdict *verdict;
+};
+
+template<bool RUNS>
 __global__ void __launch_bounds__(kListThreads)
-list_records_kernel(PieceRec *__restrict__ recs, // [n * pieces a descriptor can have]
-                    const nixl_amd_copy_list_entry_t *__restrict__ src,
-                    uint32_t n_src,
-                    const nixl_amd_copy_list_entry_t *__restrict__ dst,
-                    uint32_t n_dst,
-                    const int32_t *__restrict__ src_index,
-                    const int32_t *__restrict__ dst_index,
-                    uint32_t first_pair, // of this launch; a plan's pairs may come in several
-                    uint32_t n,
-                    uint32_t n_workgroups, // of all launches together
-                    ListTotals *totals, // cleared
-                    ListTotals *host) {
+list_records_kernel(ListArgs a) {
     constexpr int kWaves = kListThreads / kWaveSize;
     __shared__ unsigned long long wave_bytes[kWaves];
-    __shared__ uint32_t wave_bad[kWaves], wave_continued[kWaves];
-    const uint32_t i = first_pair + blockIdx.x * kListThreads + threadIdx.x;
+    __shared__ uint32_t wave_bad[kWaves], wave_continued[kWaves], wave_extra[kWaves], extra_at;
+    __shared__ IndexRun runs[RUNS ? kListThreads + 1 : 1];
+    __shared__ uint2 last[RUNS ? 1 : kWaves];
+    const uint32_t workgroup = a.first_workgroup + blockIdx.x, i = workgroup * kListThreads + threadIdx.x;
     const int lane = threadIdx.x & (kWaveSize - 1), wave = threadIdx.x / kWaveSize;
-    const int32_t si = i < n ? src_index[i] : 0, di = i < n ? dst_index[i] : 0;
-    // the pair before this one: the neighbour's, or for the first lane of a wave a load
-    int32_t sp = __shfl_up(si, 1), dp = __shfl_up(di, 1);
-    if (lane == 0 && i > 0 && i < n) {
-        sp = src_index[i - 1];
-        dp = dst_index[i - 1];
-    }
-    bool bad = false, continued = false;
-    unsigned long long bytes = 0;
-    if (i < n) {
-        // a negative index is a large unsigned one
-        bad = static_cast<uint32_t>(si) >= n_src || static_cast<uint32_t>(di) >= n_dst;
-        if (!bad) {
-            const nixl_amd_copy_list_entry_t s = src[si], d = dst[di];
-            bad = s.len != d.len;
-            bytes = s.len;
-            continued = i > 0 && si == sp + 1 && di == dp + 1 && s.continues && d.continues;
-            if (!bad) {
-                const uint32_t units = s.len / 16u, head = kPieceUnits - (static_cast<uint32_t>(d.addr >> 4) & 7u);
-                uint32_t count = min(units, head), more = units - count;
-                recs[i] = PieceRec{s.addr, d.addr | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
-                if (more) {
-                    uint32_t at = n + atomicAdd(&totals->extra, (more + kPieceUnits - 1) / kPieceUnits);
-                    for (uint32_t first = count; more; first += count, more -= count) {
-                        count = min(more, kPieceUnits);
-                        recs[at++] = PieceRec{s.addr + first * 16ull,
-                                              (d.addr + first * 16ull) | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
-                    }
-                }
-            }
+    uint32_t si = 0, di = 0;
+    bool follows; // the pair before this one names the entries before this one's
+    if constexpr (RUNS) {
+        const uint32_t r0 = a.run_of[workgroup], n_runs = a.run_of[workgroup + 1] - r0 + 1; // at most a run a pair and the next
+        if (threadIdx.x < n_runs) runs[threadIdx.x] = a.runs[r0 + threadIdx.x];
+        if (threadIdx.x == 0 && n_runs > kListThreads) runs[kListThreads] = a.runs[r0 + kListThreads];
+        __syncthreads();
+        uint32_t lo = 0, hi = n_runs; // runs[lo].first <= i < runs[hi].first
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (runs[mid].first <= i) lo = mid;
+            else hi = mid;
         }
+        si = runs[lo].src + (i - runs[lo].first);
+        di = runs[lo].dst + (i - runs[lo].first);
+        follows = i != runs[lo].first;
+    } else {
+        if (i < a.n) {
+            si = static_cast<uint32_t>(a.src_index[i]);
+            di = static_cast<uint32_t>(a.dst_index[i]);
+        }
+        // the pair before this one: the neighbour's, for the first lane of a wave by LDS and for that of
+        // the workgroup a load (one a wave is a quarter more requests over the bus)
+        uint32_t sp = __shfl_up(si, 1), dp = __shfl_up(di, 1);
+        uint32_t first_sp = 0, first_dp = 0;
+        if (threadIdx.x == 0 && i > 0) {
+            first_sp = static_cast<uint32_t>(a.src_index[i - 1]);
+            first_dp = static_cast<uint32_t>(a.dst_index[i - 1]);
+        }
+        if (lane == kWaveSize - 1) last[wave] = make_uint2(si, di);
+        __syncthreads();
+        if (lane == 0) {
+            sp = wave ? last[wave - 1].x : first_sp;
+            dp = wave ? last[wave - 1].y : first_dp;
+        }
+        follows = i > 0 && si == sp + 1 && di == dp + 1;
     }
-    const uint32_t n_bad = __popcll(__ballot(bad)), n_continued = __popcll(__ballot(continued));
+    const bool here = i < a.n;
+    const bool named = here && si < a.n_src && di < a.n_dst; // a negative index is a large unsigned one
+    nixl_amd_copy_list_entry_t s{}, d{};
+    if (named) {
+        s = a.src[si];
+        d = a.dst[di];
+    }
+    const bool good = named && s.len == d.len;
+    const uint32_t units = s.len / 16u, head = kPieceUnits - (static_cast<uint32_t>(d.addr >> 4) & 7u);
+    uint32_t count = min(units, head), more = good ? units - count : 0;
+    const uint32_t mine = (more + kPieceUnits - 1) / kPieceUnits; // records beyond the first
+    if (good) a.recs[i] = PieceRec{s.addr, d.addr | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
+
+    const uint32_t n_bad = __popcll(__ballot(here && !good));
+    const uint32_t n_continued = __popcll(__ballot(good && follows && s.continues && d.continues));
+    unsigned long long bytes = good ? s.len : 0;
+    uint32_t incl = mine;
 #pragma unroll
-    for (int off = kWaveSize / 2; off > 0; off >>= 1)
+    for (int off = 1; off < kWaveSize; off <<= 1) {
         bytes += __shfl_xor(bytes, off);
-    if (lane == 0) {
+        const uint32_t up = __shfl_up(incl, off);
+        if (lane >= off) incl += up;
+    }
+    if (lane == kWaveSize - 1) {
         wave_bytes[wave] = bytes;
         wave_bad[wave] = n_bad;
         wave_continued[wave] = n_continued;
+        wave_extra[wave] = incl;
     }
-    __syncthreads(); // every extra record of the workgroup is counted as well
-    if (threadIdx.x == 0) {
-        unsigned long long sum = 0;
-        uint32_t b = 0, c = 0;
-        for (int w = 0; w < kWaves; ++w) {
-            sum += wave_bytes[w];
-            b += wave_bad[w];
-            c += wave_continued[w];
+    __syncthreads();
+    if (wave == 0) {
+        unsigned long long sum = lane < kWaves ? wave_bytes[lane] : 0;
+        uint32_t b = lane < kWaves ? wave_bad[lane] : 0, c = lane < kWaves ? wave_continued[lane] : 0;
+        const uint32_t x = lane < kWaves ? wave_extra[lane] : 0;
+        uint32_t run = x;
+#pragma unroll
+        for (int off = 1; off < kWaves; off <<= 1) {
+            sum += __shfl_xor(sum, off);
+            b += __shfl_xor(b, off);
+            c += __shfl_xor(c, off);
+            const uint32_t up = __shfl_up(run, off);
+            if (lane >= off) run += up;
         }
-        atomicAdd(&totals->bytes, sum);
-        if (b) atomicAdd(&totals->bad, b);
-        if (c) atomicAdd(&totals->continued, c);
-        __threadfence();
-        if (atomicAdd(&totals->arrived, 1u) == n_workgroups - 1) {
+        if (lane < kWaves) wave_extra[lane] = run - x; // records of the waves before
+        const uint32_t extra = __shfl(run, kWaves - 1);
+        if (lane == 0) {
+            const unsigned long long packed = extra | static_cast<unsigned long long>(c) << 32;
+            if (packed) extra_at = static_cast<uint32_t>(atomicAdd(&a.totals->extra_continued, packed));
+            if (b) atomicAdd(&a.totals->bad, b);
             __threadfence();
-            host->bytes = __hip_atomic_load(&totals->bytes, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            host->bad = __hip_atomic_load(&totals->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            host->continued = __hip_atomic_load(&totals->continued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            host->extra = __hip_atomic_load(&totals->extra, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long before = atomicAdd(&a.totals->bytes_arrived, sum | 1ull << kListBytesBits);
+            if (before >> kListBytesBits == a.n_workgroups - 1) {
+                __threadfence();
+                const unsigned long long both = __hip_atomic_load(&a.totals->extra_continued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                a.verdict->bytes = (before & ((1ull << kListBytesBits) - 1)) + sum;
+                a.verdict->bad = __hip_atomic_load(&a.totals->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                a.verdict->continued = static_cast<uint32_t>(both >> 32);
+                a.verdict->extra = static_cast<uint32_t>(both);
+                __hip_atomic_store(&a.verdict->there, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
+    }
+    __syncthreads();
+    if (!more) return;
+    uint32_t at = a.n + extra_at + wave_extra[wave] + (incl - mine);
+    for (uint32_t first = count; more; first += count, more -= count) {
+        count = min(more, kPieceUnits);
+        a.recs[at++] =
+            PieceRec{s.addr + first * 16ull, (d.addr + first * 16ull) | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
     }
 }
 
@@ -963,6 +1042,78 @@ settle_upload(nixl_amd_copy_plan *plan, bool wait) {
     (void)hipEventDestroy(plan->uploaded);
     plan->uploaded = nullptr;
     return e;
+}
+
+// The records kernels of a listed plan, queued on `up`, have written their verdict.  The word is
+// watched for some hundred microseconds (it is there about 5 us before an event behind the kernels
+// is seen complete); an end of the kernels without it is an error of theirs.
+static hipError_t
+await_verdict(const ListVerdict &verdict, hipStream_t up) {
+    const auto there = [&] { return __atomic_load_n(&verdict.there, __ATOMIC_ACQUIRE) != 0; };
+    for (int spins = 0; spins < 10000; ++spins) {
+        if (there()) return hipSuccess;
+        __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamSynchronize(up);
+    return e != hipSuccess || there() ? e : hipErrorUnknown;
+}
+
+// Requests of at least so many pairs a run are sent as runs.  Making a request of 65 536 and of 262 144
+// pairs, us: vectors 45 and 150, runs of 16 pairs 36 and 141, of 64 pairs 34 and 120.
+constexpr size_t kMinIndexRun = 16;
+
+#if defined(__x86_64__)
+// One bit a pair of the 64 from `i` on: it does not continue the pair before it on both sides.
+__attribute__((target("avx2"))) static uint64_t
+index_breaks(const int32_t *src, const int32_t *dst, size_t i, size_t n) {
+    uint64_t breaks = 0;
+    if (i > 0 && i + 64 <= n) {
+        const __m256i one = _mm256_set1_epi32(1);
+        for (size_t j = 0; j < 64; j += 8) {
+            const auto *s = reinterpret_cast<const __m256i_u *>(src + i + j), *s1 = reinterpret_cast<const __m256i_u *>(src + i + j - 1);
+            const auto *d = reinterpret_cast<const __m256i_u *>(dst + i + j), *d1 = reinterpret_cast<const __m256i_u *>(dst + i + j - 1);
+            const __m256i follows =
+                _mm256_and_si256(_mm256_cmpeq_epi32(_mm256_sub_epi32(_mm256_loadu_si256(s), _mm256_loadu_si256(s1)), one),
+                                 _mm256_cmpeq_epi32(_mm256_sub_epi32(_mm256_loadu_si256(d), _mm256_loadu_si256(d1)), one));
+            breaks |= static_cast<uint64_t>(~static_cast<uint32_t>(_mm256_movemask_ps(_mm256_castsi256_ps(follows))) & 0xffu) << j;
+        }
+        return breaks;
+    }
+    for (size_t j = i; j < std::min(i + 64, n); ++j)
+        breaks |= static_cast<uint64_t>(j == 0 || static_cast<uint32_t>(src[j]) - static_cast<uint32_t>(src[j - 1]) != 1u ||
+                                        static_cast<uint32_t>(dst[j]) - static_cast<uint32_t>(dst[j - 1]) != 1u)
+            << (j - i);
+    return breaks;
+}
+#endif
+
+// Cuts `n` pairs into runs whose indices advance by one on both sides, and notes for every
+// kListThreads pairs the run that their first one lies in, and at the end the last run.  False
+// when more than a run for every kMinIndexRun pairs comes of it, looked at in stretches (vectors
+// that are no runs are found out at their start), or where the pairs cannot be looked at eight at
+// a time.  `runs` has room for n / kMinIndexRun + 1.
+static bool
+index_runs(const int32_t *src, const int32_t *dst, size_t n, IndexRun *runs, uint32_t *run_of) {
+#if defined(__x86_64__)
+    if (!__builtin_cpu_supports("avx2")) return false;
+    constexpr size_t kStretch = 4096;
+    static_assert(kListThreads % 64 == 0);
+    size_t n_runs = 0;
+    for (size_t i = 0; i < n; i += 64) {
+        const uint64_t breaks = index_breaks(src, dst, i, n);
+        if (i % kListThreads == 0) run_of[i / kListThreads] = static_cast<uint32_t>(n_runs - 1 + (breaks & 1));
+        const size_t allowed = std::min(n, (i / kStretch + 1) * kStretch) / kMinIndexRun + 1;
+        if (n_runs + static_cast<size_t>(__builtin_popcountll(breaks)) > allowed) return false;
+        for (uint64_t left = breaks; left; left &= left - 1) {
+            const size_t at = i + static_cast<size_t>(__builtin_ctzll(left));
+            runs[n_runs++] = IndexRun{static_cast<uint32_t>(at), static_cast<uint32_t>(src[at]), static_cast<uint32_t>(dst[at]), 0};
+        }
+    }
+    run_of[(n + kListThreads - 1) / kListThreads] = static_cast<uint32_t>(n_runs - 1);
+    return true;
+#else
+    return false;
+#endif
 }
 
 struct Tuning {
@@ -2005,19 +2156,24 @@ nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
     HIP_TRY(on_device.status());
 
     const size_t index_bytes = n * sizeof(int32_t);
-    // both vectors start on a line and so does every slice of them: no line is written by the
-    // host after a kernel has read it
+    const uint32_t workgroups = static_cast<uint32_t>((n + kListThreads - 1) / kListThreads);
+    // The two vectors, each starting on a line as every slice of them does (no line is written by the
+    // host after a kernel has read it), or in their place the runs and the run of every workgroup
+    // (which take less: 16 bytes for kMinIndexRun pairs and more); then the verdict.
     const size_t dst_at = (index_bytes + 127) & ~size_t(127);
-    const size_t totals_at = dst_at + dst_at; // the host's totals follow the index vectors
+    const size_t verdict_at = 2 * dst_at + 128;
+    static_assert(sizeof(IndexRun) <= kMinIndexRun * sizeof(int32_t) && kListThreads >= 64);
     void *staging = nullptr;
     size_t staging_cap = 0;
     reap_uploads(device);
-    hipError_t e = upload_cache().get(device, totals_at + sizeof(ListTotals), &staging, &staging_cap);
+    hipError_t e = upload_cache().get(device, verdict_at + sizeof(ListVerdict), &staging, &staging_cap);
     if (e != hipSuccess)
         return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
     auto *up_src = static_cast<int32_t *>(staging), *up_dst = up_src + dst_at / sizeof(int32_t);
-    auto *host = reinterpret_cast<ListTotals *>(static_cast<uint8_t *>(staging) + totals_at);
-    *host = ListTotals{0, ~0u, 0, 0, 0}; // every pair bad until the kernel has said otherwise
+    auto *up_runs = static_cast<IndexRun *>(staging);
+    auto *up_run_of = reinterpret_cast<uint32_t *>(up_dst);
+    auto *verdict = reinterpret_cast<ListVerdict *>(static_cast<uint8_t *>(staging) + verdict_at);
+    *verdict = ListVerdict{};
 
     auto *plan = new nixl_amd_copy_plan();
     plan->device = device;
@@ -2031,28 +2187,42 @@ nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
     constexpr size_t kRecsAt = 256;
     hipStream_t up = nullptr;
     e = arena_cache().get(device, kRecsAt + n * per_desc * sizeof(PieceRec), &plan->arena, &plan->arena_cap);
-    if (e == hipSuccess) e = upload_stream(device, &up);
+    if (e == hipSuccess) e = build_stream(plan, t, &up);
     auto *totals = static_cast<ListTotals *>(plan->arena);
     auto *recs = reinterpret_cast<PieceRec *>(static_cast<uint8_t *>(plan->arena) + kRecsAt);
     if (e == hipSuccess) {
         hipLaunchKernelGGL(clear_totals_kernel, dim3(1), dim3(kWaveSize), 0, up, totals);
         e = hipGetLastError();
     }
-    const uint32_t workgroups = static_cast<uint32_t>((n + kListThreads - 1) / kListThreads);
-    for (size_t at = 0; at < n && e == hipSuccess; at += kListSlice) {
-        const size_t count = std::min(kListSlice, n - at);
-        std::memcpy(up_src + at, src_index + at, count * sizeof(int32_t));
-        std::memcpy(up_dst + at, dst_index + at, count * sizeof(int32_t));
-        hipLaunchKernelGGL(list_records_kernel, dim3(static_cast<uint32_t>((count + kListThreads - 1) / kListThreads)), dim3(kListThreads),
-                           0, up, recs, src->entries, src->n, dst->entries, dst->n, up_src, up_dst, static_cast<uint32_t>(at),
-                           static_cast<uint32_t>(n), workgroups, totals, host);
-        e = hipGetLastError();
+    if (e == hipSuccess) {
+        ListArgs a{recs, src->entries, dst->entries, src->n,  dst->n,
+                   up_src, up_dst,      up_runs,      up_run_of, 0,
+                   static_cast<uint32_t>(n), workgroups, totals, verdict};
+        if (index_runs(src_index, dst_index, n, up_runs, up_run_of)) {
+            hipLaunchKernelGGL(list_records_kernel<true>, dim3(workgroups), dim3(kListThreads), 0, up, a);
+            e = hipGetLastError();
+        } else {
+            for (size_t at = 0; at < n && e == hipSuccess; at += kListSlice) {
+                const size_t count = std::min(kListSlice, n - at);
+                std::memcpy(up_src + at, src_index + at, count * sizeof(int32_t));
+                std::memcpy(up_dst + at, dst_index + at, count * sizeof(int32_t));
+                a.first_workgroup = static_cast<uint32_t>(at / kListThreads);
+                hipLaunchKernelGGL(list_records_kernel<false>, dim3(static_cast<uint32_t>((count + kListThreads - 1) / kListThreads)),
+                                   dim3(kListThreads), 0, up, a);
+                e = hipGetLastError();
+            }
+        }
     }
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
-    if (e == hipSuccess) e = settle_upload(plan, true);
-    if (e != hipSuccess && up) (void)hipStreamSynchronize(up); // whatever was queued reads the buffers given back below
-    const ListTotals got = *host;
+    if (e == hipSuccess) e = await_verdict(*verdict, up);
+    const ListVerdict got = *verdict;
+    // The records are complete when the last kernel ends, which comes behind its verdict: a launch
+    // follows on the same stream, or it waits for the event.
+    if (e == hipSuccess && !plan->reserved && !got.bad) {
+        e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+    }
+    if ((e != hipSuccess || got.bad) && up) (void)hipStreamSynchronize(up); // whatever is queued uses the buffers given back below
+    // the verdict is the last thing that is written there, and everything else has been read by then
     upload_cache().put(device, staging, staging_cap);
     if (e != hipSuccess || got.bad) {
         if (plan->uploaded) (void)hipEventDestroy(plan->uploaded);
@@ -2061,6 +2231,11 @@ nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
         if (e != hipSuccess) return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("plan_create_listed: ") + hipGetErrorString(e));
         return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: " + std::to_string(got.bad) +
                                                        " pairs name no entry or join entries of different lengths");
+    }
+    if (plan->reserved) {
+        plan->built_on = up;
+        plan->reserved = false; // no buffer waits with the plan
+        g_held_staging.fetch_sub(1, std::memory_order_relaxed);
     }
     plan->arena_bytes = kRecsAt + (n + got.extra) * sizeof(PieceRec);
     plan->piece_recs = recs;

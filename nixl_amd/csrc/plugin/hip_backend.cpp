@@ -839,20 +839,19 @@ nixlHipEngine::prepXferListed(const nixl_xfer_op_t &operation,
     if (operation != NIXL_READ && operation != NIXL_WRITE) return NIXL_ERR_INVALID_PARAM;
     const bool write = (operation == NIXL_WRITE);
     auto req = std::make_unique<nixlHipReqH>();
+    nixl_amd_copy_tuning_t tuning;
+    if (!chooseStream(nixl_amd_copy_list_device(local), *req, tuning)) return NIXL_ERR_BACKEND;
     size_t continued = 0;
     if (nixl_amd_copy_plan_create_listed(write ? local : remote, write ? local_indices : remote_indices, write ? remote : local,
-                                         write ? remote_indices : local_indices, count, &tuning_, &continued,
+                                         write ? remote_indices : local_indices, count, &tuning, &continued,
                                          &req->plan) != NIXL_AMD_OK) {
         NIXL_DEBUG << "HIP backend: " << nixl_amd_last_error();
         return NIXL_ERR_NOT_SUPPORTED;
     }
     nixl_amd_copy_plan_info_t info{};
     (void)nixl_amd_copy_plan_query(req->plan, &info);
-    req->device = nixl_amd_copy_list_device(local);
     req->bytes = bytes = info.payload_bytes;
     merged = count - continued;
-    req->stream = pickStream(req->device);
-    if (!req->stream && !useExternalStream_) return NIXL_ERR_BACKEND;
     handle = req.release();
     return NIXL_SUCCESS;
 }

@@ -1092,6 +1092,54 @@ def test_listed_requests_lowered_in_slices(cuda, count):
         agent.close()
 
 
+@pytest.mark.parametrize("cut", ["block", "at_1024", "one", "mixed", "short"])
+def test_listed_requests_of_consecutive_entries(cuda, cut):
+    """Index pairs that advance by one on both sides, cut into runs of 64, at and around the 1024
+    pairs of a workgroup, not at all, of any length, and so short that the vectors are sent as they
+    are: every byte against the per-descriptor oracle, the descriptors that neighbours merge into
+    counted; a run that leaves its list or meets other lengths on its way is refused."""
+    import torch
+    from nixl_amd.agent import NixlError
+    rng = np.random.default_rng(len(cut))
+    n_runs, per = 640, 24  # dense runs of equal pieces, so many that the list has no strides to speak of
+    lens = np.repeat(rng.choice([128, 256, 144, 4000], n_runs), per).astype(np.int64)
+    n = lens.size
+    starts = np.concatenate([[0], np.cumsum(lens)])[:-1] + np.repeat(np.arange(n_runs) * 48, per)
+    half = int(starts[-1] + lens[-1] + 4096) // 128 * 128 + 128
+    so, do = starts, half + starts + 32
+    pairs = {"block": [(64 * i, 64) for i in rng.permutation(n // 64)], "one": [(5, n - 9)],
+             "at_1024": [(0, 1024), (2048, 1023), (6000, 1025), (9000, 1), (10240, 1023), (12000, 1024), (4096, 17)],
+             "mixed": [(int(a), int(b)) for a, b in zip(np.sort(rng.choice(n // 512, 24, replace=False)) * 512, rng.integers(17, 512, 24))],
+             "short": [(12 * i, 12) for i in rng.permutation(n // 12)[:400]]}[cut]
+    idx = np.concatenate([np.arange(a, a + b) for a, b in pairs]).astype(np.int32)
+    host = rng.integers(0, 256, 2 * half, dtype=np.uint8)
+    mem = torch.from_numpy(host.copy()).to(cuda)
+    torch.cuda.synchronize()
+    agent = nixl_agent(f"runs{cut}", nixl_agent_config(backends=("HIP",), capture_telemetry=True))
+    try:
+        agent.register_memory([mem])
+        local, remote = (agent.prep_xfer_dlist(who, np.stack([np.uint64(mem.data_ptr()) + o.astype(np.uint64), lens.astype(np.uint64),
+                                                              np.zeros(n, np.uint64)], 1), "VRAM")
+                         for o, who in ((so, ""), (do, agent.name)))
+        req = agent.make_prepped_xfer("WRITE", local, idx, remote, idx)
+        _wait(agent, req)
+        assert np.array_equal(mem.cpu().numpy(), ko.copy_descs(host, so[idx], do[idx], lens[idx]))
+        follows = (np.diff(idx) == 1) & (idx[1:] % per != 0) & (lens[idx[1:]] == lens[idx[:-1]])
+        # neighbours of equal length in adjoining runs are one run of the prepared list only if they adjoin in memory, and these do not
+        assert agent.get_xfer_telemetry(req).desc_count == idx.size - int(follows.sum())
+        req.release()
+        off = idx.copy()  # one place further on one side: other lengths somewhere, and at the end no entry
+        off[-16:] = np.arange(n - 15, n + 1)
+        with pytest.raises(NixlError):
+            agent.make_prepped_xfer("WRITE", local, off, remote, idx)
+        with pytest.raises(NixlError):
+            agent.make_prepped_xfer("WRITE", local, idx, remote, off)
+        for h in (local, remote):
+            h.release()
+    finally:
+        agent.close()
+
+
 @pytest.mark.parametrize("n", [1, 127, 128, 129, 1500])
 @pytest.mark.parametrize("n_runs", [1, 3])
 @pytest.mark.parametrize("named", ["", "same", "other", "busy"])
