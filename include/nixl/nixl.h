@@ -67,6 +67,17 @@ public:
                 const std::vector<int> &remote_indices,
                 nixlXferReqH *&req_hndl,
                 const nixl_opt_args_t *extra_params = nullptr) const;
+    // The same with the indices where the caller keeps them (no reference counterpart).
+    nixl_status_t
+    makeXferReq(const nixl_xfer_op_t &operation,
+                const nixlDlistH *local_side,
+                const int *local_indices,
+                size_t local_count,
+                const nixlDlistH *remote_side,
+                const int *remote_indices,
+                size_t remote_count,
+                nixlXferReqH *&req_hndl,
+                const nixl_opt_args_t *extra_params = nullptr) const;
     nixl_status_t
     createXferReq(const nixl_xfer_op_t &operation,
                   const nixl_xfer_dlist_t &local_descs,

@@ -31,7 +31,8 @@ enum nixl_amd_status {
     NIXL_AMD_ERR_HIP = -2, /* a HIP runtime call failed; see nixl_amd_last_error() */
     NIXL_AMD_ERR_NO_DEVICE = -3, /* no gfx950-class device visible */
     NIXL_AMD_ERR_BUSY = -4, /* plan destroyed while one of its launches has not completed */
-    NIXL_AMD_ERR_TOO_LARGE = -5 /* request exceeds a documented fixed limit */
+    NIXL_AMD_ERR_TOO_LARGE = -5, /* request exceeds a documented fixed limit */
+    NIXL_AMD_ERR_INDEX = -6 /* an index names no entry of its list */
 };
 
 /* One span to copy: `len` bytes from device address `src` to device address `dst`.
@@ -140,6 +141,24 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
                                        int device,
                                        const nixl_amd_copy_tuning_t *tuning,
                                        nixl_amd_copy_plan_t **out);
+
+/* The same for a caller that has not looked at the indices: the two lists have src_entries and
+ * dst_entries entries, and an index outside its list is refused (NIXL_AMD_ERR_INDEX).  The
+ * arrays are read once, bounds and patterns are found out on the copy that the device reads. */
+int
+nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
+                                        size_t n_src_runs,
+                                        const int32_t *src_index,
+                                        uint64_t src_entries,
+                                        const nixl_amd_copy_run_t *dst_runs,
+                                        size_t n_dst_runs,
+                                        const int32_t *dst_index,
+                                        uint64_t dst_entries,
+                                        size_t n,
+                                        uint64_t len,
+                                        int device,
+                                        const nixl_amd_copy_tuning_t *tuning,
+                                        nixl_amd_copy_plan_t **out);
 
 /* A plan of equal blocks from records the CALLER writes: what a backend's prepXfer does when
  * it checks the two nixl_meta_dlist_t of a request (src/api/cpp/backend/backend_engine.h:135-141)

@@ -158,7 +158,7 @@ def ep_kernels():
 
 def kernel_symbols():
     return sorted(["nixl_amd_last_error", "nixl_amd_device_count", "nixl_amd_copy_plan_create", "nixl_amd_copy_plan_create_indexed",
-                   "nixl_amd_copy_plan_create_indexed_runs", "nixl_amd_copy_records_begin",
+                   "nixl_amd_copy_plan_create_indexed_runs", "nixl_amd_copy_plan_create_indexed_lists", "nixl_amd_copy_records_begin",
                    "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon", "nixl_amd_copy_block_len_fits",
                    "nixl_amd_copy_list_create", "nixl_amd_copy_list_destroy", "nixl_amd_copy_list_device",
                    "nixl_amd_copy_plan_create_listed",

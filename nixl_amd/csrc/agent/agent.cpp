@@ -915,13 +915,29 @@ expandIndexPairs(const nixl_stride_dlist_t &lruns,
 
 } // namespace
 
-// reference: src/core/nixl_agent.cpp:696-887
 nixl_status_t
 nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
                        const nixlDlistH *local_side,
                        const std::vector<int> &local_indices,
                        const nixlDlistH *remote_side,
                        const std::vector<int> &remote_indices,
+                       nixlXferReqH *&req_hndl,
+                       const nixl_opt_args_t *extra_params) const {
+    return makeXferReq(operation, local_side, local_indices.data(), local_indices.size(), remote_side, remote_indices.data(),
+                       remote_indices.size(), req_hndl, extra_params);
+}
+
+// reference: src/core/nixl_agent.cpp:696-887
+// A backend that takes index vectors reads every index once and checks what it has read; only the
+// expansion into descriptors, which looks at them twice, works on copies.
+nixl_status_t
+nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
+                       const nixlDlistH *local_side,
+                       const int *local_indices,
+                       size_t local_count,
+                       const nixlDlistH *remote_side,
+                       const int *remote_indices,
+                       size_t remote_count,
                        nixlXferReqH *&req_hndl,
                        const nixl_opt_args_t *extra_params) const {
     req_hndl = nullptr;
@@ -933,10 +949,10 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
         NIXL_ERROR_FUNC << "invalid sides (local must be local, remote must be remote)";
         return NIXL_ERR_INVALID_PARAM;
     }
-    const size_t count = local_indices.size();
-    if (count == 0 || count != remote_indices.size()) {
+    const size_t count = local_count;
+    if (count == 0 || count != remote_count) {
         NIXL_ERROR_FUNC << "different number of indices for local (" << count << "), remote ("
-                        << remote_indices.size() << ")";
+                        << remote_count << ")";
         return NIXL_ERR_INVALID_PARAM;
     }
 
@@ -970,8 +986,8 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
         if (slot && slot->prepIndexed && slot->engine == backend) {
             const nixl_status_t st = static_cast<nixl_status_t>(
                 slot->prepIndexed(backend, static_cast<int>(req->backendOp), &lruns[0], static_cast<size_t>(lruns.descCount()),
-                                  local_indices.data(), &rruns[0], static_cast<size_t>(rruns.descCount()),
-                                  remote_indices.data(), count, req->remoteAgent.c_str(), &req->backendHandle));
+                                  local_indices, &rruns[0], static_cast<size_t>(rruns.descCount()),
+                                  remote_indices, count, req->remoteAgent.c_str(), &req->backendHandle));
             if (st == NIXL_SUCCESS) {
                 req->engine = backend;
                 req->notifMsg = opt.notifMsg;
@@ -995,7 +1011,7 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
         const nixl_status_t st = !slot || slot->engine != backend ?
             NIXL_ERR_NOT_SUPPORTED :
             static_cast<nixl_status_t>(slot->prepListed(backend, static_cast<int>(req->backendOp), lres->second.list,
-                                                        local_indices.data(), rres->second.list, remote_indices.data(), count,
+                                                        local_indices, rres->second.list, remote_indices, count,
                                                         req->remoteAgent.c_str(), &bytes, &merged, &req->backendHandle));
         if (st == NIXL_SUCCESS) {
             req->engine = backend;
@@ -1013,7 +1029,8 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
     }
     size_t total = 0;
     const auto t_expand = std::chrono::steady_clock::now();
-    const nixl_status_t expanded = expandIndexPairs(lruns, rruns, local_indices, remote_indices,
+    const nixl_status_t expanded = expandIndexPairs(lruns, rruns, std::vector<int>(local_indices, local_indices + count),
+                                                    std::vector<int>(remote_indices, remote_indices + count),
                                                     !(extra_params && extra_params->skipDescMerge), req->initiatorDescs,
                                                     req->targetDescs, total);
     if (expanded != NIXL_SUCCESS) return expanded;

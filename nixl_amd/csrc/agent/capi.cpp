@@ -363,11 +363,10 @@ nixl_capi_make_xfer_req(nixl_capi_agent_t agent,
         (!remote_indices && remote_indices_count))
         return NIXL_CAPI_ERROR_INVALID_PARAM;
     return guarded([&] {
-        const std::vector<int> li(local_indices, local_indices + local_indices_count);
-        const std::vector<int> ri(remote_indices, remote_indices + remote_indices_count);
         nixlXferReqH *req = nullptr;
-        const nixl_status_t st = agent->inner->makeXferReq(static_cast<nixl_xfer_op_t>(operation), local_descs->handle, li,
-                                                          remote_descs->handle, ri, req, opt_args ? &opt_args->args : nullptr);
+        const nixl_status_t st = agent->inner->makeXferReq(static_cast<nixl_xfer_op_t>(operation), local_descs->handle, local_indices,
+                                                          local_indices_count, remote_descs->handle, remote_indices,
+                                                          remote_indices_count, req, opt_args ? &opt_args->args : nullptr);
         if (st != NIXL_SUCCESS) return fold(st);
         *req_hndl = new nixl_capi_xfer_req_s{req};
         return fold(st);

@@ -423,14 +423,25 @@ sort_records_kernel(UniformRec *recs, uint32_t n) {
 
 // Records of an indexed plan: block i goes from src_base + src_index[i] * src_stride to
 // dst_base + dst_index[i] * dst_stride.  The index vectors are the only per-request data
-// that crosses the bus (8 bytes per block instead of 16, and no host loop over descriptors).
+// that crosses the bus, at most 8 bytes per block: one whose indices are consecutive (the staging
+// side of a gather or a scatter) stays where it is.  65 536 pairs, both
+// vectors read 15 us, one 8.5.
+struct IndexVector {
+    const int32_t *at; // null: first, first + 1, ...
+    int32_t first;
+};
+
+__device__ __forceinline__ uint64_t
+index_at(const IndexVector &v, uint32_t i) {
+    return static_cast<uint64_t>(v.at ? v.at[i] : static_cast<int32_t>(v.first + i));
+}
+
 __global__ void __launch_bounds__(256)
-index_records_kernel(UniformRec *recs, const int32_t *src_index, const int32_t *dst_index, uint32_t n, uint64_t src_base,
+index_records_kernel(UniformRec *recs, IndexVector src_index, IndexVector dst_index, uint32_t n, uint64_t src_base,
                      uint64_t src_stride, uint64_t dst_base, uint64_t dst_stride) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n)
-        recs[i] = UniformRec{src_base + static_cast<uint64_t>(src_index[i]) * src_stride,
-                             dst_base + static_cast<uint64_t>(dst_index[i]) * dst_stride};
+        recs[i] = UniformRec{src_base + index_at(src_index, i) * src_stride, dst_base + index_at(dst_index, i) * dst_stride};
 }
 
 // The same for lists of several runs (a pool registered as several regions): index i of a
@@ -451,7 +462,7 @@ run_address(const uint64_t *first, const uint64_t *base, const uint64_t *stride,
 }
 
 __global__ void __launch_bounds__(256)
-index_records_runs_kernel(UniformRec *recs, const int32_t *src_index, const int32_t *dst_index, uint32_t n,
+index_records_runs_kernel(UniformRec *recs, IndexVector src_index, IndexVector dst_index, uint32_t n,
                           const nixl_amd_copy_run_t *src_runs, uint32_t n_src, const nixl_amd_copy_run_t *dst_runs,
                           uint32_t n_dst) {
     __shared__ uint64_t first[2][kMaxIndexRuns], base[2][kMaxIndexRuns], stride[2][kMaxIndexRuns];
@@ -468,8 +479,8 @@ index_records_runs_kernel(UniformRec *recs, const int32_t *src_index, const int3
     __syncthreads();
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n)
-        recs[i] = UniformRec{run_address(first[0], base[0], stride[0], n_src, static_cast<uint64_t>(src_index[i])),
-                             run_address(first[1], base[1], stride[1], n_dst, static_cast<uint64_t>(dst_index[i]))};
+        recs[i] = UniformRec{run_address(first[0], base[0], stride[0], n_src, index_at(src_index, i)),
+                             run_address(first[1], base[1], stride[1], n_dst, index_at(dst_index, i))};
 }
 
 // Records of a listed plan: pair i joins entry src_index[i] of one prepared list with entry
@@ -1058,9 +1069,70 @@ await_verdict(const ListVerdict &verdict, hipStream_t up) {
     return e != hipSuccess || there() ? e : hipErrorUnknown;
 }
 
+// What one pass over an index vector tells.
+struct IndexFacts {
+    uint32_t highest = 0; // a negative index is a large one
+    uint32_t ones = 0; // steps to the index behind the one before
+    uint32_t regular = 0; // steps like the one before, or of one where that is dense
+};
+
+// v[i] for begin <= i < end, v[i - 1] and v[i - 2] being those before it: differences modulo 2^32 and no
+// value carried from one iteration to the next, so that the loop vectorises.
+static __attribute__((always_inline)) inline void
+study_indices(const uint32_t *v, size_t begin, size_t end, uint32_t dense, IndexFacts &f) {
+    uint32_t highest = f.highest, ones = 0, regular = 0;
+    for (size_t i = begin; i < end; ++i) {
+        const uint32_t step = v[i] - v[i - 1], before = v[i - 1] - v[i - 2];
+        highest = std::max(highest, v[i]);
+        ones += step == 1u;
+        regular += (static_cast<uint32_t>(step == 1u) & dense) | static_cast<uint32_t>(step == before);
+    }
+    f.highest = highest;
+    f.ones += ones;
+    f.regular += regular;
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) static void
+study_indices_avx2(const uint32_t *v, size_t begin, size_t end, uint32_t dense, IndexFacts &f) {
+    study_indices(v, begin, end, dense, f);
+}
+#endif
+
+// Copies `n` indices and studies the copy, a stretch that the first-level cache holds at a time: what
+// is found out holds for what the kernel will read, whatever becomes of the caller's array.
+static IndexFacts
+take_indices(const int32_t *from, size_t n, int32_t *to, bool dense) {
+#if defined(__x86_64__)
+    const bool wide = __builtin_cpu_supports("avx2");
+#endif
+    IndexFacts f;
+    const auto *v = reinterpret_cast<const uint32_t *>(to);
+    constexpr size_t kStretch = 4096;
+    for (size_t begin = 0; begin < n; begin += kStretch) {
+        const size_t end = std::min(n, begin + kStretch);
+        std::memcpy(to + begin, from + begin, (end - begin) * sizeof(int32_t));
+        size_t i = begin;
+        for (; i < std::min<size_t>(end, 2); ++i) { // no step, and one without a step before it
+            const bool one = i == 1 && v[1] - v[0] == 1u;
+            f.highest = std::max(f.highest, v[i]);
+            f.ones += one;
+            f.regular += one && dense;
+        }
+#if defined(__x86_64__)
+        if (wide) {
+            study_indices_avx2(v, i, end, dense, f);
+            continue;
+        }
+#endif
+        study_indices(v, i, end, dense, f);
+    }
+    return f;
+}
+
 // Requests of at least so many pairs a run are sent as runs.  Making a request of 65 536 and of 262 144
-// pairs, us: vectors 45 and 150, runs of 16 pairs 36 and 141, of 64 pairs 34 and 120.
-constexpr size_t kMinIndexRun = 16;
+// pairs, us: vectors 34 and 88, runs of 8 pairs 34 and 86, of 16 pairs 29 and 65, of 64 pairs 26 and 50.
+constexpr size_t kMinIndexRun = 8;
 
 #if defined(__x86_64__)
 // One bit a pair of the 64 from `i` on: it does not continue the pair before it on both sides.
@@ -1895,17 +1967,19 @@ nixl_amd_copy_plan_create_from_records(nixl_amd_copy_records_t *records,
 }
 
 int
-nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
-                                       size_t n_src_runs,
-                                       const int32_t *src_index,
-                                       const nixl_amd_copy_run_t *dst_runs,
-                                       size_t n_dst_runs,
-                                       const int32_t *dst_index,
-                                       size_t n,
-                                  uint64_t len,
-                                  int device,
-                                  const nixl_amd_copy_tuning_t *tuning,
-                                  nixl_amd_copy_plan_t **out) {
+nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
+                                        size_t n_src_runs,
+                                        const int32_t *src_index,
+                                        uint64_t src_entries,
+                                        const nixl_amd_copy_run_t *dst_runs,
+                                        size_t n_dst_runs,
+                                        const int32_t *dst_index,
+                                        uint64_t dst_entries,
+                                        size_t n,
+                                        uint64_t len,
+                                        int device,
+                                        const nixl_amd_copy_tuning_t *tuning,
+                                        nixl_amd_copy_plan_t **out) {
     if (!out) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_indexed: out is null");
     *out = nullptr;
     if (!src_index || !dst_index || n == 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_indexed: no indices");
@@ -1944,6 +2018,7 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     // The records of a few blocks are made right here instead.
     const size_t index_bytes = n * sizeof(int32_t);
     const bool inlined = fits_inline(n, len, t);
+    int32_t few[2 * kInlineRecs];
     void *staging = nullptr;
     size_t staging_cap = 0;
     const bool tables = n_src_runs > 1 || n_dst_runs > 1;
@@ -1955,9 +2030,18 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
         e = upload_cache().get(device, table_at + table_bytes, &staging, &staging_cap);
         if (e != hipSuccess)
             return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
-        std::memcpy(staging, src_index, index_bytes);
-        std::memcpy(static_cast<int32_t *>(staging) + n, dst_index, index_bytes);
     }
+    // One pass over each vector on its way there: bounds, and the patterns that decide cache policy and
+    // record order.  A request of 65 536 blocks made, one of whose vectors is consecutive: 51 us with a
+    // pass each for a copy, bounds, the pinned copy and the pattern, 23 so.
+    int32_t *const si = inlined ? few : static_cast<int32_t *>(staging), *const di = si + n;
+    const IndexFacts src_facts = take_indices(src_index, n, si, src_all_dense), dst_facts = take_indices(dst_index, n, di, dst_all_dense);
+    if (src_facts.highest >= src_entries || dst_facts.highest >= dst_entries) {
+        if (staging) upload_cache().put(device, staging, staging_cap);
+        return nixl_amd_fail(NIXL_AMD_ERR_INDEX, "plan_create_indexed: an index names no entry of its list");
+    }
+    const bool scattered = !(n == 1 || 2 * static_cast<uint64_t>(dst_facts.regular) >= n - 1);
+    const bool sort = scattered && sort_scatter != 2 && src_all_dense && 2 * static_cast<uint64_t>(src_facts.ones) >= n - 1 && n >= kSortWindow;
     if (tables && !inlined) {
         auto *up_runs = reinterpret_cast<nixl_amd_copy_run_t *>(static_cast<uint8_t *>(staging) + table_at);
         std::memcpy(up_runs, src_runs, n_src_runs * sizeof(nixl_amd_copy_run_t));
@@ -1968,40 +2052,16 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     plan->upl = upl;
     plan->waves = waves;
     plan->swizzle = swizzle;
-    // Destination pattern (cache policy, record order) and source pattern from the index vectors.
-    // How many destination steps are regular (one block on in dense lists, or the same step as
-    // the one before) and how many source steps go one block on: differences taken modulo 2^32
-    // and without a value carried from one iteration to the next, so that the loop vectorises.
-    // Sets the policy and says whether the records are to be sorted.
-    const auto study_pattern = [&] {
-        uint32_t regular = 0, src_follows = 0; // n < 2^31
-        const uint32_t dst_dense = dst_all_dense ? 1u : 0u, src_dense = src_all_dense ? 1u : 0u;
-        const auto *sv = reinterpret_cast<const uint32_t *>(src_index);
-        const auto *dv = reinterpret_cast<const uint32_t *>(dst_index);
-        if (n > 1) {
-            regular += ((dv[1] - dv[0]) == 1u) & dst_dense;
-            src_follows += ((sv[1] - sv[0]) == 1u) & src_dense;
-        }
-        for (size_t i = 2; i < n; ++i) {
-            const uint32_t step = dv[i] - dv[i - 1], before = dv[i - 1] - dv[i - 2];
-            regular += (static_cast<uint32_t>(step == 1u) & dst_dense) | static_cast<uint32_t>(step == before);
-            src_follows += static_cast<uint32_t>((sv[i] - sv[i - 1]) == 1u) & src_dense;
-        }
-        const bool scattered = !(n == 1 || 2 * static_cast<uint64_t>(regular) >= n - 1);
-        const bool sort = scattered && sort_scatter != 2 && 2 * static_cast<uint64_t>(src_follows) >= n - 1 && n >= kSortWindow;
-        plan->policy = nt ? nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
-        return sort;
-    };
+    plan->policy = nt ? nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
     if (inlined) {
-        (void)study_pattern();
         const auto address = [](const nixl_amd_copy_run_t *runs, size_t n_runs, uint64_t index) {
             const auto *run = std::upper_bound(runs, runs + n_runs, index, [](uint64_t i, const nixl_amd_copy_run_t &r) { return i < r.first_index; }) - 1;
             return run->base + (index - run->first_index) * run->stride;
         };
         plan->inline_recs = std::make_unique<InlineRecs>();
         for (size_t i = 0; i < n; ++i)
-            plan->inline_recs->rec[i] = UniformRec{address(src_runs, n_src_runs, static_cast<uint64_t>(src_index[i])),
-                                                   address(dst_runs, n_dst_runs, static_cast<uint64_t>(dst_index[i]))};
+            plan->inline_recs->rec[i] = UniformRec{address(src_runs, n_src_runs, static_cast<uint64_t>(si[i])),
+                                                   address(dst_runs, n_dst_runs, static_cast<uint64_t>(di[i]))};
         describe_blocks(*plan, t, n, len, n);
         *out = plan;
         return NIXL_AMD_OK;
@@ -2011,22 +2071,20 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     e = arena_cache().get(device, rec_bytes, &plan->arena, &plan->arena_cap);
     if (e == hipSuccess) e = build_stream(plan, t, &up);
     auto *recs = static_cast<UniformRec *>(plan->arena);
-    const auto *index = static_cast<const int32_t *>(staging);
     if (e == hipSuccess) {
         const dim3 grid(static_cast<uint32_t>((n + 255) / 256));
+        const IndexVector src_at{src_facts.ones == n - 1 ? nullptr : si, si[0]}, dst_at{dst_facts.ones == n - 1 ? nullptr : di, di[0]};
         if (tables) {
             const auto *runs = reinterpret_cast<const nixl_amd_copy_run_t *>(static_cast<const uint8_t *>(staging) + table_at);
-            hipLaunchKernelGGL(index_records_runs_kernel, grid, dim3(256), 0, up, recs, index, index + n, static_cast<uint32_t>(n),
-                               runs, static_cast<uint32_t>(n_src_runs), runs + n_src_runs, static_cast<uint32_t>(n_dst_runs));
+            hipLaunchKernelGGL(index_records_runs_kernel, grid, dim3(256), 0, up, recs, src_at, dst_at, static_cast<uint32_t>(n), runs,
+                               static_cast<uint32_t>(n_src_runs), runs + n_src_runs, static_cast<uint32_t>(n_dst_runs));
         } else {
-            hipLaunchKernelGGL(index_records_kernel, grid, dim3(256), 0, up, recs, index, index + n, static_cast<uint32_t>(n),
+            hipLaunchKernelGGL(index_records_kernel, grid, dim3(256), 0, up, recs, src_at, dst_at, static_cast<uint32_t>(n),
                                src_runs[0].base, src_runs[0].stride, dst_runs[0].base, dst_runs[0].stride);
         }
         e = hipGetLastError();
     }
-    // after the launch: the kernel reads the indices over the bus meanwhile (65 536 blocks there and
-    // back 848 us with the pattern first, 831 so; 15 250 blocks 75.5 and 73.1)
-    if (e == hipSuccess && study_pattern()) {
+    if (e == hipSuccess && sort) {
         hipLaunchKernelGGL(sort_records_kernel, dim3(static_cast<uint32_t>((n + kSortWindow - 1) / kSortWindow)),
                            dim3(kSortWindow / 2), 0, up, recs, static_cast<uint32_t>(n));
         e = hipGetLastError();
@@ -2045,6 +2103,22 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
     describe_blocks(*plan, t, n, len, n);
     *out = plan;
     return NIXL_AMD_OK;
+}
+
+int
+nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
+                                       size_t n_src_runs,
+                                       const int32_t *src_index,
+                                       const nixl_amd_copy_run_t *dst_runs,
+                                       size_t n_dst_runs,
+                                       const int32_t *dst_index,
+                                       size_t n,
+                                       uint64_t len,
+                                       int device,
+                                       const nixl_amd_copy_tuning_t *tuning,
+                                       nixl_amd_copy_plan_t **out) {
+    return nixl_amd_copy_plan_create_indexed_lists(src_runs, n_src_runs, src_index, UINT64_MAX, dst_runs, n_dst_runs, dst_index, UINT64_MAX,
+                                                   n, len, device, tuning, out);
 }
 
 int

@@ -744,19 +744,6 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
         }
     }
     if (device < 0) device = first_md->device;
-    // every index must name a block of its list: one pass over each vector
-    int lmin = local_indices[0], lmax = lmin, rmin = remote_indices[0], rmax = rmin;
-    for (size_t i = 1; i < count; ++i) {
-        lmin = std::min(lmin, local_indices[i]);
-        lmax = std::max(lmax, local_indices[i]);
-        rmin = std::min(rmin, remote_indices[i]);
-        rmax = std::max(rmax, remote_indices[i]);
-    }
-    if (lmin < 0 || static_cast<size_t>(lmax) >= flat[0] || rmin < 0 || static_cast<size_t>(rmax) >= flat[1]) {
-        NIXL_ERROR << "HIP backend: index outside its prepared list";
-        return NIXL_ERR_INVALID_PARAM;
-    }
-
     // Whole chunks on 128-byte lines are what such plans are made of.  Decided here and not by
     // the plan's refusal, so that a request which goes on to the descriptor path has taken no
     // turn on the engine's streams yet.
@@ -770,9 +757,13 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
     const int *index_of[2] = {local_indices, remote_indices};
     nixl_amd_copy_tuning_t tuning;
     if (!chooseStream(device, *req, tuning)) return NIXL_ERR_BACKEND;
-    const int rc = nixl_amd_copy_plan_create_indexed_runs(tables[src].data(), tables[src].size(), index_of[src],
-                                                          tables[dst].data(), tables[dst].size(), index_of[dst], count, len,
-                                                          device, &tuning, &req->plan);
+    const int rc = nixl_amd_copy_plan_create_indexed_lists(tables[src].data(), tables[src].size(), index_of[src], flat[src],
+                                                           tables[dst].data(), tables[dst].size(), index_of[dst], flat[dst], count, len,
+                                                           device, &tuning, &req->plan);
+    if (rc == NIXL_AMD_ERR_INDEX) {
+        NIXL_ERROR << "HIP backend: index outside its prepared list";
+        return NIXL_ERR_INVALID_PARAM;
+    }
     if (rc == NIXL_AMD_ERR_INVALID) return NIXL_ERR_NOT_SUPPORTED; // the descriptor path handles it
     if (rc != NIXL_AMD_OK) {
         NIXL_ERROR << "HIP backend: " << nixl_amd_last_error();

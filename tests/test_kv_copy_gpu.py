@@ -1092,6 +1092,51 @@ def test_listed_requests_lowered_in_slices(cuda, count):
         agent.close()
 
 
+@pytest.mark.parametrize("n", [1, 2, 129, 4096, 4097, 8195])
+@pytest.mark.parametrize("consecutive", ["neither", "source", "destination", "both"])
+@pytest.mark.parametrize("n_runs", [1, 3])
+def test_index_vectors_read_once(cuda, n, consecutive, n_runs):
+    """Requests by index around the stretches in which the vectors are read, with vectors that are
+    consecutive and so do not travel: every block; an index outside its list is refused wherever it
+    stands, on either side, and the agent goes on."""
+    import torch
+    from nixl_amd.agent import NixlError
+    rng = np.random.default_rng(n)
+    pool, blk = 8300, 8192
+    src = torch.randint(0, 256, (pool, blk), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros_like(src)
+    torch.cuda.synchronize()
+    # n_runs lists that no single stride describes: the second third of a pool starts a block late
+    order = np.concatenate([np.arange(a, b) for a, b in ((0, 2000), (2001, 5000), (5002, pool))]) if n_runs > 1 else np.arange(pool)
+    agent = nixl_agent(f"once{n}{consecutive}{n_runs}", nixl_agent_config(backends=("HIP",)))
+    try:
+        agent.register_memory([src, dst])
+        local, remote = (agent.prep_xfer_dlist(who, np.stack([np.uint64(t.data_ptr()) + order.astype(np.uint64) * np.uint64(blk),
+                                                              np.full(order.size, blk, np.uint64), np.zeros(order.size, np.uint64)], 1), "VRAM")
+                         for t, who in ((src, ""), (dst, agent.name)))
+        row = np.arange(n, dtype=np.int32) + 3
+        at = row if consecutive in ("source", "both") else rng.permutation(order.size)[:n].astype(np.int32)
+        to = row if consecutive in ("destination", "both") else rng.permutation(order.size)[:n].astype(np.int32)
+        for where in sorted({0, 1, 4095, 4096, n - 2, n - 1}):
+            for value in (-1, order.size, -(1 << 31)):
+                if 0 <= where < n:
+                    bad = at.copy()
+                    bad[where] = value
+                    with pytest.raises(NixlError):
+                        agent.make_prepped_xfer("WRITE", local, bad, remote, to)
+                    with pytest.raises(NixlError):
+                        agent.make_prepped_xfer("READ", local, at, remote, bad)
+        req = agent.make_prepped_xfer("WRITE", local, at, remote, to)
+        _wait(agent, req)
+        want = torch.zeros_like(dst)
+        want[torch.from_numpy(order[to]).to(cuda)] = src[torch.from_numpy(order[at]).to(cuda)]
+        assert torch.equal(dst, want)
+        for h in (req, local, remote):
+            h.release()
+    finally:
+        agent.close()
+
+
 @pytest.mark.parametrize("cut", ["block", "at_1024", "one", "mixed", "short"])
 def test_listed_requests_of_consecutive_entries(cuda, cut):
     """Index pairs that advance by one on both sides, cut into runs of 64, at and around the 1024
