@@ -45,7 +45,9 @@ def _ptr(t):
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The handle of the current device's current stream: 0.1 us, where building the Stream object of
+    torch.cuda.current_stream() takes 2.9 (a small dispatch and combine together: 35 us)."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
 
 
 def _check(rc, what):
