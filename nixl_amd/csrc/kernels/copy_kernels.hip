@@ -129,7 +129,10 @@ store16(uint64_t addr, const v4u &v) {
     else if constexpr (POL == kPolPlain)
         *g = v;
     else
-        asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" : : "v"(g), "v"(v) : "memory");
+        // The compiler does not see that this is a store of more than two registers, after which they
+        // may not be written for two wait states: chunks of two units a lane lost half of a lane's
+        // 16 bytes to the address of the next store.
+        asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(g), "v"(v) : "memory");
 }
 
 // Workgroups are handed to the 8 dies round-robin.  With the swizzle on, die x works

@@ -101,11 +101,13 @@ st16_nt(void *p, const uint4 &x) {
 }
 
 // Streaming store with device scope ("sc1 nt"): measured a little faster than the plain
-// non-temporal store for rows that are written once and read by a later kernel.
+// non-temporal store for rows that are written once and read by a later kernel.  The two wait states
+// behind it are those in which the registers of such a store may not be written; the compiler
+// keeps to them only for stores that it sees.
 __device__ __forceinline__ void
 st16_stream(void *p, const uint4 &x) {
     const ep_v4u v = {x.x, x.y, x.z, x.w};
-    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt"
+    asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1"
                  :
                  : "v"((__attribute__((address_space(1))) ep_v4u *)(reinterpret_cast<uintptr_t>(p))), "v"(v)
                  : "memory");

@@ -73,6 +73,20 @@ def test_aligned_descriptors_match_oracle(cuda, upl, nt):
     assert info.payload_bytes == sum(lens)
 
 
+@pytest.mark.parametrize("upl", [1, 2, 4, 8, 16])
+@pytest.mark.parametrize("nt", [0, 1, 2, 3, 4])
+def test_blocks_at_every_chunk_size_and_cache_policy(cuda, upl, nt):
+    """Equal blocks on lines, which take the kernel of whole chunks, at every chunk size it is built for
+    and with every form of its loads and stores."""
+    import torch
+    rng = np.random.default_rng(upl + nt)
+    blk, n = 32768, 96
+    at = rng.permutation(n) * blk
+    to = n * blk + rng.permutation(n) * blk
+    info = _check_against_oracle(torch, cuda, 2 * n * blk, at, to, [blk] * n, (upl, nt, 0, 0, 0), seed=upl)
+    assert info.uniform_chunks == n * blk // (1024 * upl) and info.piece_items == 0 and info.mixed_chunks == 0
+
+
 @pytest.mark.parametrize("sort_scatter", [0, 2])
 @pytest.mark.parametrize("n", [1024, 3000, 5121])
 def test_scatter_of_consecutive_memory_matches_oracle(cuda, n, sort_scatter):
