@@ -7,24 +7,22 @@
 //   16-byte record {src, dst | (units - 1) << 56} and one wavefront each
 //   (wavefront-per-descriptor for anything up to 4 KiB); pieces after the first start on a
 //   destination line.
-//   The other 16-byte-aligned descriptors (long and line-aligned, or tiny) are
-//   concatenated, in request order, into one virtual stream measured in 16-byte units.  The stream is cut into chunks of
-//   64*UPL units; one wavefront moves one chunk: lane l moves units k*64 + l of the chunk,
-//   k < UPL, so every load/store instruction of a wave touches 1 KiB of consecutive bytes
-//   unless a descriptor boundary falls inside it.  Chunks are classified on the host:
-//     * a full chunk that lies inside one descriptor becomes a 16-byte record
-//       {src address, dst address} in `uniform[]`; the uniform kernel reads its record
-//       with one scalar load and issues UPL 128-bit loads and UPL 128-bit stores per lane
-//       with wave-uniform base addresses — no search, no LDS, few registers;
-//     * any other chunk (it crosses descriptor boundaries, or it is the short last chunk)
-//       is listed by chunk index in `mixed[]`; the mixed kernel stages the descriptors the
-//       chunk touches (span[m] = {first, last} for the m-th listed chunk; src[j], dst[j], prefix[j] = first unit of
-//       descriptor j, prefix[n] = total) in a per-wave LDS slice and walks them.
+//   Longer line-aligned ones are chunks of 64*UPL 16-byte units; one wavefront moves one
+//   chunk: lane l moves units k*64 + l of the chunk, k < UPL, so every load/store instruction
+//   of a wave touches 1 KiB of consecutive bytes.  A chunk is a 16-byte record {src address,
+//   dst address} in `uniform[]`; the uniform kernel reads its record with one scalar load and
+//   issues UPL 128-bit loads and UPL 128-bit stores per lane with wave-uniform base addresses —
+//   no search, no LDS, few registers.  The end of a descriptor that is no whole number of
+//   chunks is one more chunk, which lies over the one before it.
+//   Tiny ones (below 256 B) are concatenated, in request order, into one virtual stream measured
+//   in 16-byte units and cut into such chunks, listed by chunk index in `mixed[]`; the mixed kernel
+//   stages the descriptors a chunk touches (span[m] = {first, last} for the m-th listed chunk; src[j],
+//   dst[j], prefix[j] = first unit of descriptor j, prefix[n] = total) in a per-wave LDS slice and
+//   walks them.
 //   Descriptors that are not 16-byte aligned in src, dst and len are cut into byte-range
-//   work items of at most 4 KiB (16 of many long ones) handled by a third, byte-exact kernel; of a
-//   long one whose source and destination lie alike inside their 128-byte lines only the ends are,
-//   and the whole chunks between them stand in front of the virtual stream, unless the request is
-//   small and brings no other chunks.
+//   work items of at most 4 KiB (16 of many long ones) handled by a third, byte-exact kernel; a
+//   long one whose source and destination lie alike inside their 128-byte lines is chunks as well,
+//   unless the request is small and brings no other chunks.
 //   Lists of equal-length, line-aligned descriptors of whole chunks (KV blocks) take none of
 //   these steps: one pass writes their records, or, when the request is two index vectors
 //   into two strided runs, a kernel writes them from the indices on the device.  Arenas and
@@ -698,25 +696,41 @@ clear_totals_kernel(ListTotals *totals) {
     if (threadIdx.x == 0) *totals = ListTotals{};
 }
 
-// Records of a plan whose runs of uniform chunks differ in length: run r covers chunks
-// first_chunk[r] .. first_chunk[r + 1] - 1 and chunk c of it lies c - first_chunk[r] chunks
-// behind the run's start on both sides.  A thread per chunk finds its run by bisection (the
+// A long descriptor as chunks of its own: chunk k starts k chunks behind the place `back` bytes in
+// front of the descriptor, but not before the descriptor and not so late that it would reach
+// beyond it.  With a whole number of chunks and back = 0 that is all there is to it; else the last chunk
+// (and, with a `back` that puts the others on the destination's lines, the first) lies partly over
+// its neighbour, and both write the same bytes there.  So every chunk is whole and belongs to one
+// descriptor, whatever the length, and no descriptor moves another one's chunks off the lines.
+// Cut from one stream of all descriptors, chunks behind one that is no whole number of them started
+// anywhere in a line and those on a border were put together by another kernel: 40 tensors of 1 to
+// 128 MiB in multiples of 16 bytes 393 us, 348 so; 512 of 2 MiB + 16 B to 48 B 397 and 315; 64 of 1 MiB + 16 to 48 B
+// 31.2 and 24.1; 64 165 descriptors of 8 to 64 KiB in multiples of 16 bytes 897 and 805.  Odd tensors, whose ends
+// the byte kernel moved, 358 and 348.  On the grid of whole KiB of the destination they are no faster (351).
+struct ChunkRun {
+    uint64_t src, dst, len; // len >= a chunk
+    uint32_t first; // chunk of the plan that the run starts with
+    uint32_t back; // less than a chunk
+};
+
+// Records of a plan of such runs: a thread per chunk finds its run by bisection (the
 // table stays in the L2), so that one long run among short ones costs no more than any other;
-// 16 bytes per run cross the bus instead of 16 per chunk.
+// 32 bytes per run cross the bus instead of 16 per chunk.
 __global__ void __launch_bounds__(256)
-expand_runs_kernel(UniformRec *recs, const UniformRec *runs, const uint32_t *first_chunk, uint32_t n_runs, uint32_t n_chunks,
-                   uint32_t chunk_bytes) {
+expand_runs_kernel(UniformRec *recs, const ChunkRun *runs, uint32_t n_runs, uint32_t n_chunks, uint32_t chunk_bytes) {
     for (uint64_t c64 = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; c64 < n_chunks;
          c64 += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
         const uint32_t c = static_cast<uint32_t>(c64);
-        uint32_t lo = 0, hi = n_runs; // first_chunk[lo] <= c < first_chunk[hi]
+        uint32_t lo = 0, hi = n_runs; // runs[lo].first <= c < runs[hi].first
         while (hi - lo > 1) {
             const uint32_t mid = lo + (hi - lo) / 2;
-            if (first_chunk[mid] <= c) lo = mid;
+            if (runs[mid].first <= c) lo = mid;
             else hi = mid;
         }
-        const uint64_t off = static_cast<uint64_t>(c - first_chunk[lo]) * chunk_bytes;
-        recs[c] = UniformRec{runs[lo].src + off, runs[lo].dst + off};
+        const ChunkRun run = runs[lo];
+        const uint64_t at = static_cast<uint64_t>(c - run.first) * chunk_bytes;
+        const uint64_t off = min(at > run.back ? at - run.back : 0, run.len - chunk_bytes);
+        recs[c] = UniformRec{run.src + off, run.dst + off};
     }
 }
 
@@ -1362,6 +1376,26 @@ private:
 // items, 10.7 and 22.0 with long).
 constexpr uint64_t kSplitFromBytes = 64 * 1024, kSplitFromTotal = 128ull << 20, kLongItemsFrom = 8ull << 20;
 
+// Long descriptors, which become chunks of their own (ChunkRun).
+struct LongDescs {
+    explicit LongDescs(uint64_t chunk) : chunk_bytes(chunk) {}
+
+    const uint64_t chunk_bytes;
+    std::vector<ChunkRun> runs;
+    uint64_t n = 0, edges = 0; // chunks, and how many of them lie over their neighbours
+    bool equal = true; // as many chunks in every run, none of them over another
+
+    // len >= chunk_bytes > back, and len + back > chunk_bytes if there is a back
+    void
+    add(uint64_t src, uint64_t dst, uint64_t len, uint64_t back) {
+        const uint64_t reach = len + back;
+        equal = equal && reach % chunk_bytes == 0 && back == 0 && (runs.empty() || runs[0].len == len);
+        edges += static_cast<uint64_t>(back != 0) + static_cast<uint64_t>(reach % chunk_bytes != 0);
+        runs.push_back(ChunkRun{src, dst, len, static_cast<uint32_t>(n), static_cast<uint32_t>(back)});
+        n += (reach + chunk_bytes - 1) / chunk_bytes;
+    }
+};
+
 // The descriptors of a request that are not 16-byte aligned.  Their loop is apart from that over
 // the others: in one loop, with items appended one by one to a vector, making a plan took 106 us for
 // 14 394 descriptors of up to 16 KiB and 24 for 3000 of up to 64 KiB (54 and 18 so), and code
@@ -1558,7 +1592,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     const DeviceScope on_device(device);
     HIP_TRY(on_device.status());
 
-    const uint64_t chunk_units = static_cast<uint64_t>(kWaveSize) * upl;
+    const uint64_t chunk_units = static_cast<uint64_t>(kWaveSize) * upl, chunk_bytes = chunk_units * 16u;
 
     // ---- fast path: equal-length, line-aligned descriptors of whole chunks (KV blocks) ----
     // One pass over the descriptors writes the {src, dst} records straight into the pinned
@@ -1615,8 +1649,9 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     vdst.reserve(n);
     vprefix.reserve(n + 1);
     uint64_t units = 0, payload = 0, n_piece_descs = 0;
+    LongDescs chunks(chunk_bytes);
     ByteDescs bytes;
-    bool whole_chunks = false; // some descriptor brings the stream whole chunks whatever becomes of those
+    bool whole_chunks = false; // there are chunks of some aligned descriptor whatever becomes of those
     for (size_t i = 0; i < n; ++i) {
         const nixl_amd_copy_desc_t &d = descs[i];
         if (d.len == 0) continue;
@@ -1652,6 +1687,10 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             ++n_piece_descs;
         } else {
             whole_chunks |= du >= kPieceMaxDescUnits;
+            if (du >= std::max(kPieceMaxDescUnits, chunk_units)) {
+                chunks.add(d.src, d.dst, d.len, 0);
+                continue;
+            }
             vsrc.push_back(d.src);
             vdst.push_back(d.dst);
             vprefix.push_back(units);
@@ -1660,132 +1699,56 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     }
     payload += bytes.payload;
     // A long byte descriptor whose two ends lie at the same place inside their lines (tensors whose
-    // size is no multiple of 16) is whole chunks but for its first line and its last chunk: only
-    // those go byte by byte.  These chunks go in front of the stream, where they lie on their own
-    // lines and move nobody else's.  Without chunks of other descriptors that is one launch more, and
-    // up to kSplitFromTotal (both sides in the 256 MB last-level cache) the byte kernel alone is as
-    // fast or faster: 32 tensors of 1 MiB + 2 B 12.3 us instead of 15.0, 128 of them 36.9 and 45.4;
-    // 256 of them 90 us and a plan that takes 25 us to make, instead of 84 and 9.
+    // size is no multiple of 16) is chunks but for its two ends, and those are chunks as well that lie
+    // over their neighbours (their lanes' 16 bytes start anywhere).  Without chunks of other
+    // descriptors and up to kSplitFromTotal (both sides in the 256 MB last-level cache) the byte kernel
+    // is as fast or faster: 32 tensors of 1 MiB + 2 B 12.3 us instead of 15.0, 128 of them 36.9 and
+    // 45.4; 256 of them 90 us and a plan that takes 25 us to make, instead of 84 and 9.
     const bool join = whole_chunks || bytes.splittable_total >= kSplitFromTotal;
     if (bytes.long_total - (join ? bytes.splittable_total : 0) > kLongItemsFrom) bytes.reach = kGenericItemBytes;
-    std::vector<uint64_t> front_src, front_dst, front_prefix;
-    uint64_t front_units = 0;
+    const size_t n_aligned_runs = chunks.runs.size(), n_aligned_edges = chunks.edges;
     for (const uint32_t i : bytes.longs) {
         const nixl_amd_copy_desc_t &d = descs[i];
         if (!join || !ByteDescs::splittable(d)) {
             bytes.add(d.src, d.dst, d.len);
             continue;
         }
-        const uint64_t head = (0 - d.dst) & 127u, body = (d.len - head) / (chunk_units * 16u) * (chunk_units * 16u);
-        bytes.add(d.src, d.dst, head);
-        bytes.add(d.src + head + body, d.dst + head + body, d.len - head - body);
-        front_src.push_back(d.src + head);
-        front_dst.push_back(d.dst + head);
-        front_prefix.push_back(front_units);
-        front_units += body / 16u;
-    }
-    const size_t n_split = front_src.size();
-    if (n_split) {
-        vsrc.insert(vsrc.begin(), front_src.begin(), front_src.end());
-        vdst.insert(vdst.begin(), front_dst.begin(), front_dst.end());
-        for (uint64_t &p : vprefix)
-            p += front_units;
-        vprefix.insert(vprefix.begin(), front_prefix.begin(), front_prefix.end());
-        units += front_units;
+        // the chunks between the ends start on a line
+        chunks.add(d.src, d.dst, d.len, (0 - ((0 - d.dst) & 127u)) % chunk_bytes);
     }
     vprefix.push_back(units);
     const size_t nv = vsrc.size();
-    const uint64_t n_chunks64 = (units + chunk_units - 1) / chunk_units;
-    if (n_chunks64 >= (1ull << 32) || bytes.items.n >= (1ull << 32) || pieces.n >= (1ull << 31))
+    const uint64_t n_stream64 = (units + chunk_units - 1) / chunk_units;
+    if (n_stream64 + chunks.n >= (1ull << 32) || bytes.items.n >= (1ull << 32) || pieces.n >= (1ull << 31))
         return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "plan_create: request too large for 32-bit chunk index");
-    const uint32_t n_chunks = static_cast<uint32_t>(n_chunks64);
+    const uint32_t n_stream = static_cast<uint32_t>(n_stream64), n_uniform_chunks = static_cast<uint32_t>(chunks.n);
 
-    // Walk the stream by descriptor: the chunks that lie wholly inside one descriptor form a
-    // run of uniform chunks (one step for the whole run, however long); a chunk that holds a
-    // descriptor boundary, or the short last chunk, is "mixed" and remembers the first and
-    // last descriptor it touches.  If all runs have the same length L, one record per run is
-    // kept and the kernel derives the rest; otherwise every uniform chunk gets its record.
-    struct Run {
-        uint64_t src, dst;
-        uint32_t chunks;
-    };
-    std::vector<Run> runs;
-    std::vector<uint32_t> mixed;
-    std::vector<uint2> span; // per mixed chunk: first and last descriptor
-    uint32_t n_uniform_chunks = 0, common_run = 0;
-    bool runs_equal = true;
-    // Equal-length descriptors that are whole numbers of chunks (KV blocks): every descriptor
-    // is one run, nothing is mixed, and the walk below is not needed.
-    const uint64_t chunk_bytes_all = chunk_units * 16u;
-    bool all_whole = nv > 0;
-    for (size_t j = 0; j < nv && all_whole; ++j)
-        all_whole = (vprefix[j + 1] - vprefix[j]) * 16u == (vprefix[1] - vprefix[0]) * 16u;
-    all_whole = all_whole && ((vprefix[1] - vprefix[0]) * 16u) % chunk_bytes_all == 0;
-    if (all_whole) {
-        common_run = static_cast<uint32_t>((vprefix[1] - vprefix[0]) * 16u / chunk_bytes_all);
-        n_uniform_chunks = n_chunks;
-    } else {
-        size_t j = 0;
-        for (uint32_t c = 0; c < n_chunks;) {
-            const uint64_t first = static_cast<uint64_t>(c) * chunk_units;
-            while (vprefix[j + 1] <= first)
-                ++j;
-            const uint64_t inside = (vprefix[j + 1] - first) / chunk_units; // whole chunks left in descriptor j
-            if (inside > 0) {
-                const uint32_t len = static_cast<uint32_t>(inside);
-                const uint64_t off = (first - vprefix[j]) * 16u;
-                runs.push_back(Run{vsrc[j] + off, vdst[j] + off, len});
-                if (common_run == 0)
-                    common_run = len;
-                else if (common_run != len)
-                    runs_equal = false;
-                n_uniform_chunks += len;
-                c += len;
-                continue;
-            }
-            const uint64_t last = std::min(units, first + chunk_units) - 1;
-            size_t jl = j;
-            while (vprefix[jl + 1] <= last)
-                ++jl;
-            mixed.push_back(c);
-            span.push_back(make_uint2(static_cast<uint32_t>(j), static_cast<uint32_t>(jl)));
-            ++c;
-        }
+    // The stream: descriptors shorter than a chunk.  Every chunk of it remembers the first and the
+    // last descriptor that it touches.
+    std::vector<uint32_t> mixed(n_stream);
+    std::vector<uint2> span(n_stream);
+    for (size_t c = 0, j = 0; c < n_stream; ++c) {
+        const uint64_t first = c * chunk_units, last = std::min(units, first + chunk_units) - 1;
+        while (vprefix[j + 1] <= first)
+            ++j;
+        size_t jl = j;
+        while (vprefix[jl + 1] <= last)
+            ++jl;
+        mixed[c] = static_cast<uint32_t>(c);
+        span[c] = make_uint2(static_cast<uint32_t>(j), static_cast<uint32_t>(jl));
     }
-    std::vector<UniformRec> uni;
-    std::vector<uint32_t> first_chunk; // runs of different lengths: run r starts at uniform chunk first_chunk[r]
-    uint32_t chunks_per_rec = 1;
-    if (all_whole) {
-        chunks_per_rec = common_run;
-        uni.resize(nv);
-        for (size_t j = 0; j < nv; ++j)
-            uni[j] = UniformRec{vsrc[j], vdst[j]};
-    } else if (runs_equal && common_run > 1) {
-        chunks_per_rec = common_run;
-        uni.reserve(runs.size());
-        for (const Run &r : runs)
-            uni.push_back(UniformRec{r.src, r.dst});
-    } else if (!runs.empty()) {
-        // a record per chunk, written on the device from a record per run
-        uni.reserve(runs.size());
-        first_chunk.reserve(runs.size() + 1);
-        uint32_t at = 0;
-        for (const Run &r : runs) {
-            uni.push_back(UniformRec{r.src, r.dst});
-            first_chunk.push_back(at);
-            at += r.chunks;
-        }
-        first_chunk.push_back(at);
-    }
-    const bool expand = !first_chunk.empty();
-    const size_t n_uniform_recs = expand ? n_uniform_chunks : uni.size();
+    // Runs of the same whole number of chunks share a record each; else every chunk gets its own,
+    // written on the device from the runs.
+    const bool expand = !chunks.equal;
+    const uint32_t chunks_per_rec = expand || chunks.runs.empty() ? 1 : static_cast<uint32_t>(chunks.runs[0].len / chunk_bytes);
+    const size_t n_uniform_recs = expand ? n_uniform_chunks : chunks.runs.size();
 
     // ---- one device arena for all plan arrays --------------------------------------
     auto align256 = [](size_t x) { return (x + 255) & ~size_t(255); };
     const bool need_desc_arrays = !mixed.empty();
     // The arena starts with the records the copy kernel reads.  When they are expanded on the
-    // device, that stretch is not uploaded: the upload starts behind it, and the records per run
-    // and their first chunks travel at the arena's end.
+    // device, that stretch is not uploaded: the upload starts behind it, and the runs
+    // travel at the arena's end.
     const size_t off_uni = 0;
     const size_t off_src = off_uni + align256(n_uniform_recs * sizeof(UniformRec));
     const size_t off_dst = off_src + (need_desc_arrays ? align256(nv * 8) : 0);
@@ -1795,8 +1758,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     const size_t off_pieces = off_mixed + align256(mixed.size() * sizeof(uint32_t));
     const size_t off_items = off_pieces + align256(pieces.n * sizeof(PieceRec));
     const size_t off_runs = off_items + align256(bytes.items.n * sizeof(GenericItem));
-    const size_t off_first = off_runs + (expand ? align256(uni.size() * sizeof(UniformRec)) : 0);
-    const size_t total = off_first + (expand ? align256(first_chunk.size() * sizeof(uint32_t)) : 0);
+    const size_t total = off_runs + (expand ? align256(chunks.runs.size() * sizeof(ChunkRun)) : 0);
     const size_t upload_from = expand ? off_src : 0;
 
     auto *plan = new nixl_amd_copy_plan();
@@ -1838,10 +1800,12 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         // the pinned buffer mirrors the arena from upload_from on
         const auto host = [&](size_t arena_offset) { return static_cast<uint8_t *>(staging) + (arena_offset - upload_from); };
         if (expand) {
-            std::memcpy(host(off_runs), uni.data(), uni.size() * sizeof(UniformRec));
-            std::memcpy(host(off_first), first_chunk.data(), first_chunk.size() * sizeof(uint32_t));
-        } else if (!uni.empty())
-            std::memcpy(host(off_uni), uni.data(), uni.size() * sizeof(UniformRec));
+            std::memcpy(host(off_runs), chunks.runs.data(), chunks.runs.size() * sizeof(ChunkRun));
+        } else {
+            auto *recs = reinterpret_cast<UniformRec *>(host(off_uni));
+            for (const ChunkRun &run : chunks.runs)
+                *recs++ = UniformRec{run.src, run.dst};
+        }
         if (need_desc_arrays) {
             std::memcpy(host(off_src), vsrc.data(), nv * 8);
             std::memcpy(host(off_dst), vdst.data(), nv * 8);
@@ -1865,9 +1829,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         if (e == hipSuccess && expand) {
             const uint32_t wgs = static_cast<uint32_t>(std::min<uint64_t>((static_cast<uint64_t>(n_uniform_chunks) + 255) / 256, 1u << 20));
             hipLaunchKernelGGL(expand_runs_kernel, dim3(wgs), dim3(256), 0, up, reinterpret_cast<UniformRec *>(arena + off_uni),
-                               reinterpret_cast<const UniformRec *>(arena + off_runs),
-                               reinterpret_cast<const uint32_t *>(arena + off_first), static_cast<uint32_t>(uni.size()),
-                               n_uniform_chunks, static_cast<uint32_t>(chunk_units * 16u));
+                               reinterpret_cast<const ChunkRun *>(arena + off_runs), static_cast<uint32_t>(chunks.runs.size()),
+                               n_uniform_chunks, static_cast<uint32_t>(chunk_bytes));
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = end_build(plan, up, staging, staging_cap);
@@ -1908,12 +1871,13 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->generic_wgs = wgs_for(plan->n_generic, kMixedWaves, true);
 
     plan->info.payload_bytes = payload;
-    plan->info.vec_descs = nv - n_split + n_piece_descs;
+    plan->info.vec_descs = nv + n_aligned_runs + n_piece_descs;
     plan->info.generic_descs = bytes.n;
     plan->info.plan_device_bytes = plan->arena_bytes;
-    plan->info.vec_chunks = n_chunks;
-    plan->info.uniform_chunks = plan->n_uniform;
-    plan->info.mixed_chunks = plan->mixed_args.n_mixed;
+    plan->info.vec_chunks = n_stream + n_uniform_chunks;
+    // chunks that are their descriptor's alone, and those in which something else is written as well
+    plan->info.uniform_chunks = static_cast<uint32_t>(chunks.n - chunks.edges);
+    plan->info.mixed_chunks = n_stream + static_cast<uint32_t>(n_aligned_edges);
     plan->info.generic_items = plan->n_generic;
     plan->info.piece_items = plan->n_pieces;
     plan->info.units_per_lane = static_cast<uint32_t>(upl);

@@ -236,6 +236,27 @@ def test_runs_of_different_lengths_are_expanded_on_the_device(cuda):
     assert info.plan_device_bytes >= info.uniform_chunks * 16
 
 
+@pytest.mark.parametrize("upl", [1, 2, 16])
+@pytest.mark.parametrize("nt", [0, 1, 2, 3])
+def test_chunks_that_lie_over_their_neighbours(cuda, upl, nt):
+    """Long descriptors of every remainder: aligned ones that start on a line anywhere in a chunk, odd
+    ones whose two sides start at the same byte of a line.  Every byte, those around the descriptors included; the
+    ends of the aligned ones are counted."""
+    import torch
+    chunk, large = 1024 * upl, 4 << 20
+    aligned = [16384, 16400, 16384 + chunk - 16, 5 * chunk + 16384, 65536 + 112, large - 16, large, large + 16, large + 1024, large + chunk + 1008]
+    odd = [65537, 65536 + 127, 65536 + 1040, 8 * chunk + 65536 + 1, large - 1, large + 1, large + 1023, large + 1041]
+    lens, so, do, at = aligned + odd, [], [], 0
+    for i, n in enumerate(lens):
+        inside = 0 if i < len(aligned) else (1, 2, 15, 64, 127, 0, 16, 126)[i - len(aligned)]
+        so.append(at + 128 * (i % 7) + inside)
+        do.append(at + 128 * (i * 5 % 8) + inside)
+        at = (at + n + 2047) // 1024 * 1024 + 1024
+    info = _check_against_oracle(torch, cuda, 2 * at, so, [at + d for d in do], lens, (upl, nt, 0, 0, 0), seed=upl)
+    assert info.vec_descs == len(aligned) and info.generic_descs == len(odd) and info.generic_items == 0 and info.piece_items == 0
+    assert info.mixed_chunks == sum(n % chunk != 0 for n in aligned)
+
+
 @pytest.mark.parametrize("copies,reach", [(1, 4096), (6, 16384)])
 def test_items_of_long_byte_descriptors(cuda, copies, reach):
     """Long descriptors whose two sides lie differently inside their lines: byte-range items of one
