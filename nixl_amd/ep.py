@@ -41,13 +41,14 @@ class EventOverlap:
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    # a plain integer: the entry points' argument types make the pointer of it (a call takes up to 33)
+    return None if t is None else t.data_ptr()
 
 
 def _stream():
     """The handle of the current device's current stream: 0.1 us, where building the Stream object of
     torch.cuda.current_stream() takes 2.9 (a small dispatch and combine together: 35 us)."""
-    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice()))
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _check(rc, what):
@@ -603,8 +604,8 @@ class Buffer:
         # below, as in the reference (csrc/nixl_ep.cpp:762-800).
         mapped = self._mapped_counts(R + R * El)
         mapped.fill(-1)
-        recv_counter_ptr = ctypes.c_void_p(self._mapped_tensor.data_ptr())
-        expert_count_ptr = ctypes.c_void_p(self._mapped_tensor.data_ptr() + 4 * R)
+        recv_counter_ptr = self._mapped_tensor.data_ptr()
+        expert_count_ptr = recv_counter_ptr + 4 * R
         _check(self._k.nixl_amd_ep_ht_notify_dispatch(_ptr(is_token_in_rank), _ptr(num_tokens_per_expert), _ptr(prefix),
                                                       expert_count_ptr, _ptr(chan), _ptr(send_head), _ptr(row_offset),
                                                       recv_counter_ptr, T, R, E, num_channels, expert_alignment,
