@@ -304,45 +304,68 @@ ht_prefix_kernel(const int *__restrict__ channel_prefix, HtNotifyOut o, int R, i
     notify_prefix(o, R, E, [&](int r, int d) { return channel_prefix[(static_cast<size_t>(r) * R + d) * C + (C - 1)]; });
 }
 
-// The same without a launch of its own, for up to kNotifyFlags flags and 8 ranks: one more
-// workgroup behind those of the scan counts the flags itself instead of waiting for their
-// counts.  Both steps take 5.3 us instead of 7.8 at 4 x 333 tokens, called again and again on the
-// same flags, and 6.1 instead of 8.1 at 8 x 512 (32 768 flags).  With more flags that one
-// workgroup is what the call waits for, the sooner since flags that another kernel has just
-// written come from memory: 8 x 1024, 7.9 us instead of 8.5 on the same flags but 11.7 instead of
-// 5.4 + 4.0 behind the layout kernel; 8 x 4096, 15 instead of 9.1.
-constexpr int kNotifyFlags = 32768; // R * T * R
-constexpr int kNotifyPerLane = 16; // tokens a lane counts at a time, their loads together
+// The same without a launch of its own, for up to 8 ranks: one more workgroup behind those of the
+// scan counts the flags itself instead of waiting for their counts.  What bounds it is one workgroup's
+// way to flags that another kernel has just written, so every wave has a share of a rank's tokens, eight
+// loads in flight a lane, and counts bytes (eight destinations an addition) that are widened once a
+// step.  Layout, scan and this behind one another, us, against two launches (and the first form, which
+// counted 16-bit fields with half of the waves, up to 32 768 flags): 4 x 333 tokens 8.6 and 11.6 (10.1), 8 x 256 7.9 and
+// 11.1 (9.3), 8 x 512 10.0 and 13.3 (13.0), 8 x 1024 9.6 and 12.7, 8 x 2048 12.1 and 14.8, 8 x 4096 15.0 and 16.0, 8 x 6000
+// 17.5 and 17.3, 8 x 8192 20.0 and 18.6; 4 x 4096 13.1 and 15.7, 4 x 16 384 19.3 and 22.0.  Where a token's flags are
+// no word that one load takes, the line lies lower: 6 x 300 11.5 and 11.6, 6 x 600 14.0 and 12.5, 7 x 400 13.5 and 11.8, 2 x 3000 13.7
+// and 14.2, 2 x 4500 16.2 and 15.5, 1 x 4000 11.2 and 14.1.
+constexpr int kNotifyTokensOf8 = 40960, kNotifyTokensOf4 = 65536; // R * T
+constexpr int kNotifyFlags = 12288; // R * T * R, other numbers of ranks
+constexpr int kNotifyPerLane = 8; // tokens a lane counts at a time, their loads together
 
+// The flags of a token, a byte a destination (R <= 8).
+template<int RANKS>
+__device__ __forceinline__ unsigned long long
+token_flags(const uint8_t *flags, int t, int R) {
+    const uint8_t *at = flags + static_cast<size_t>(t) * R;
+    if constexpr (RANKS == 8) return *reinterpret_cast<const unsigned long long *>(at);
+    if constexpr (RANKS == 4) return *reinterpret_cast<const uint32_t *>(at);
+    unsigned long long f = 0;
+    for (int d = 0; d < R; ++d)
+        f |= static_cast<unsigned long long>(at[d]) << (8 * d);
+    return f;
+}
+
+// RANKS: the number of ranks, or 0 where it is known at run time only.
+template<int RANKS>
 __device__ __forceinline__ void
-notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int R, int E) {
+notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int n_ranks, int E) {
+    const int R = RANKS ? RANKS : n_ranks;
     __shared__ int hits[kPackedScanRanks * kPackedScanRanks]; // [source][destination]
     constexpr int kWaves = kScanThreads / kWaveSize, kUnit = kWaveSize * kNotifyPerLane;
-    const int tid = threadIdx.x, lane = tid & (kWaveSize - 1);
+    constexpr unsigned long long kLow7 = 0x7f7f7f7f7f7f7f7full, kOnes = 0x0101010101010101ull, kEven = 0x00ff00ff00ff00ffull;
+    const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), wave = tid / kWaveSize;
     if (tid < kPackedScanRanks * kPackedScanRanks) hits[tid] = 0;
     __syncthreads();
-    const int units = (T + kUnit - 1) / kUnit;
-    for (int u = tid / kWaveSize; u < R * units; u += kWaves) {
-        const int r = u / units, t0 = (u % units) * kUnit + lane;
+    // as many waves to a rank as there are; a wave adds up what it counts in 16-bit fields (T < 65 536)
+    const int per_rank = kWaves / R, r = wave / per_rank;
+    if (r < R) {
         const uint8_t *flags = in_rank + static_cast<size_t>(r) * T * R;
-        PackedCounts h[kNotifyPerLane];
+        unsigned long long even = 0, odd = 0; // destinations 0, 2, 4, 6 and 1, 3, 5, 7
+        for (int t0 = (wave % per_rank) * kUnit + lane; t0 - lane < T; t0 += per_rank * kUnit) {
+            unsigned long long f[kNotifyPerLane], sum = 0;
 #pragma unroll
-        for (int j = 0; j < kNotifyPerLane; ++j) {
-            const int t = t0 + j * kWaveSize;
-            h[j] = t < T ? packed_hits(flags, t, R) : PackedCounts{0, 0};
-        }
-        PackedCounts sum{0, 0}; // at most 1024 to a field
+            for (int j = 0; j < kNotifyPerLane; ++j) {
+                const int t = t0 + j * kWaveSize;
+                f[j] = t < T ? token_flags<RANKS>(flags, t, R) : 0;
+            }
 #pragma unroll
-        for (int j = 0; j < kNotifyPerLane; ++j) {
-            sum.lo += h[j].lo;
-            sum.hi += h[j].hi;
+            for (int j = 0; j < kNotifyPerLane; ++j)
+                sum += ((((f[j] & kLow7) + kLow7) | f[j]) >> 7) & kOnes; // one in every byte that is not zero
+            even += sum & kEven;
+            odd += (sum >> 8) & kEven;
         }
 #pragma unroll
         for (int off = kWaveSize / 2; off > 0; off >>= 1) {
-            sum.lo += __shfl_xor(sum.lo, off);
-            sum.hi += __shfl_xor(sum.hi, off);
+            even += __shfl_xor(even, off);
+            odd += __shfl_xor(odd, off);
         }
-        if (lane < R) atomicAdd(&hits[r * kPackedScanRanks + lane], packed_field(sum, lane));
+        if (lane < R) atomicAdd(&hits[r * kPackedScanRanks + lane], static_cast<int>(((lane & 1 ? odd : even) >> (8 * (lane & 6))) & 0xffffu));
     }
     __syncthreads();
     notify_prefix(o, R, E, [&](int r, int d) { return hits[r * kPackedScanRanks + d]; });
@@ -363,7 +386,12 @@ ht_scan_packed_kernel(const uint8_t *__restrict__ in_rank,
     __shared__ PackedCounts wave_sums[kWaves], wave_before[kWaves];
     const int chunks = (T + kScanThreads - 1) / kScanThreads;
     if (NOTIFY && static_cast<int>(blockIdx.x) == R * chunks) {
-        notify_from_flags(in_rank, notify, T, R, E);
+        if (R == 8)
+            notify_from_flags<8>(in_rank, notify, T, R, E);
+        else if (R == 4)
+            notify_from_flags<4>(in_rank, notify, T, R, E);
+        else
+            notify_from_flags<0>(in_rank, notify, T, R, E);
         return;
     }
     const int src = blockIdx.x / chunks, base = (blockIdx.x % chunks) * kScanThreads;
@@ -1018,7 +1046,10 @@ nixl_amd_ep_ht_notify_dispatch(const uint8_t *is_token_in_rank,
     const HtNotifyOut notify{num_tokens_per_expert, recv_gbl_rank_prefix_sum, recv_expert_count,
                              reinterpret_cast<long long *>(recv_row_offset), recv_counter, expert_alignment};
     if (num_ranks <= kPackedScanRanks && num_tokens <= kPackedScanMaxTokens && aligned) {
-        const bool one_launch = static_cast<long long>(num_ranks) * num_ranks * num_tokens <= kNotifyFlags;
+        const long long tokens = static_cast<long long>(num_ranks) * num_tokens;
+        const bool one_launch = num_ranks == 8 ? tokens <= kNotifyTokensOf8 :
+            num_ranks == 4                     ? tokens <= kNotifyTokensOf4 :
+                                                 tokens * num_ranks <= kNotifyFlags;
         hipLaunchKernelGGL(one_launch ? ht_scan_packed_kernel<true> : ht_scan_packed_kernel<false>,
                            dim3(static_cast<unsigned>(num_ranks) * ((num_tokens + kScanThreads - 1) / kScanThreads) + one_launch),
                            dim3(kScanThreads), 0, s, is_token_in_rank, send_head, gbl_channel_prefix_matrix, num_tokens, num_ranks,

@@ -1390,3 +1390,38 @@ def test_ll_narrow_workgroups_give_the_same_bytes(cuda):
                         assert np.array_equal(bits16(out).reshape(R, T, H), ref)
     finally:
         assert k.nixl_amd_ep_ll_set_tuning(-1, -1) == 0  # back to the built-in choice
+
+
+@pytest.mark.parametrize("R,T", [(1, 1), (1, 12288), (1, 12289), (2, 513), (2, 3072), (2, 3073), (3, 1365), (3, 1366), (4, 511), (4, 512), (4, 1025),
+                                 (4, 16384), (4, 16385), (5, 64), (6, 341), (6, 342), (7, 250), (7, 251), (8, 1), (8, 511), (8, 513), (8, 1024), (8, 2049),
+                                 (8, 5120), (8, 5121)])
+def test_notify_counts_flags(cuda, R, T):
+    """What a dispatch is told before its rows travel, from flags of any density (a rank that gets nothing, one
+    that gets every token, flags that are other than one): around the number of tokens from which the counts have a
+    launch of their own, and at the steps in which they are counted."""
+    import torch
+    g = torch.Generator(device="cpu").manual_seed(R * 100003 + T)
+    density = torch.linspace(0, 1, R) if R > 1 else torch.tensor([0.5])
+    hit = torch.rand((R, T, R), generator=g) < density
+    flags = (hit * torch.randint(1, 256, hit.shape, generator=g)).to(torch.uint8).to(cuda)
+    E, C, align = 4 * R, 3, 4
+    per_expert = torch.randint(0, 9, (R, E), generator=g, dtype=torch.int32)
+    dev = {k: torch.full(shape, -7, dtype=dt, device=cuda) for k, shape, dt in
+           (("prefix", (R, R), torch.int32), ("experts", (E,), torch.int32), ("channels", (R, R, C), torch.int32),
+            ("head", (R, T, R), torch.int32), ("offset", (R + 1,), torch.int64), ("counter", (R,), torch.int32))}
+    experts = per_expert.to(cuda)
+    k = _lib.ep_kernels()
+    rc = k.nixl_amd_ep_ht_notify_dispatch(flags.data_ptr(), experts.data_ptr(), dev["prefix"].data_ptr(), dev["experts"].data_ptr(),
+                                          dev["channels"].data_ptr(), dev["head"].data_ptr(), dev["offset"].data_ptr(),
+                                          dev["counter"].data_ptr(), T, R, E, C, align, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _lib.kernels_error()
+    before = hit.int().cumsum(1)
+    count = before[:, -1]  # [source, destination]
+    assert torch.equal(dev["head"].cpu(), torch.where(hit, before - 1, -1).int())
+    assert torch.equal(dev["prefix"].cpu(), count.t().cumsum(1).int())
+    assert torch.equal(dev["counter"].cpu(), count.sum(0).int())
+    assert dev["offset"].tolist() == [0] + count.sum(0).cumsum(0).tolist()
+    assert torch.equal(dev["experts"].cpu(), ((per_expert.sum(0) + align - 1) // align * align).int())
+    per_channel = -(-T // C)
+    ends = [min((c + 1) * per_channel, T) - 1 for c in range(C)]
+    assert torch.equal(dev["channels"].cpu(), before[:, ends].permute(0, 2, 1).int())
