@@ -1142,15 +1142,51 @@ study_indices_avx2(const uint32_t *v, size_t begin, size_t end, uint32_t dense, 
 }
 #endif
 
+// How many of `n` indices follow the first one by one each, looked at in stretches of 1024.
+static __attribute__((always_inline)) inline size_t
+count_consecutive(const uint32_t *v, uint32_t first, size_t n) {
+    size_t i = 0;
+    while (i < n) {
+        const size_t end = std::min<size_t>(n, i + 1024);
+        uint32_t off = 0;
+        for (size_t j = i; j < end; ++j)
+            off |= v[j] ^ (first + static_cast<uint32_t>(j));
+        if (off) break;
+        i = end;
+    }
+    return i;
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) static size_t
+count_consecutive_avx2(const uint32_t *v, uint32_t first, size_t n) {
+    return count_consecutive(v, first, n);
+}
+#endif
+
 // Copies `n` indices and studies the copy, a stretch that the first-level cache holds at a time: what
-// is found out holds for what the kernel will read, whatever becomes of the caller's array.
+// is found out holds for what the kernel will read, whatever becomes of the caller's array.  Consecutive
+// indices, of which the kernel needs the first, are not copied but for that one unless `whole` says so.
 static IndexFacts
-take_indices(const int32_t *from, size_t n, int32_t *to, bool dense) {
+take_indices(const int32_t *from, size_t n, int32_t *to, bool dense, bool whole) {
 #if defined(__x86_64__)
     const bool wide = __builtin_cpu_supports("avx2");
 #endif
     IndexFacts f;
-    const auto *v = reinterpret_cast<const uint32_t *>(to);
+    const auto *v = reinterpret_cast<const uint32_t *>(to), *given = reinterpret_cast<const uint32_t *>(from);
+    const uint32_t first = given[0];
+#if defined(__x86_64__)
+    const size_t consecutive = wide ? count_consecutive_avx2(given, first, n) : count_consecutive(given, first, n);
+#else
+    const size_t consecutive = count_consecutive(given, first, n);
+#endif
+    if (!whole && consecutive == n && n - 1 <= UINT32_MAX - first) {
+        to[0] = static_cast<int32_t>(first);
+        f.highest = first + static_cast<uint32_t>(n - 1);
+        f.ones = static_cast<uint32_t>(n - 1);
+        f.regular = n < 2 ? 0 : static_cast<uint32_t>(n - 2) + (dense ? 1 : 0);
+        return f;
+    }
     constexpr size_t kStretch = 4096;
     for (size_t begin = 0; begin < n; begin += kStretch) {
         const size_t end = std::min(n, begin + kStretch);
@@ -2026,9 +2062,11 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
     }
     // One pass over each vector on its way there: bounds, and the patterns that decide cache policy and
     // record order.  A request of 65 536 blocks made, one of whose vectors is consecutive: 51 us with a
-    // pass each for a copy, bounds, the pinned copy and the pattern, 23 so.
+    // pass each for a copy, bounds, the pinned copy and the pattern, 23 in one, 16 with the consecutive
+    // one left where it is.
     int32_t *const si = inlined ? few : static_cast<int32_t *>(staging), *const di = si + n;
-    const IndexFacts src_facts = take_indices(src_index, n, si, src_all_dense), dst_facts = take_indices(dst_index, n, di, dst_all_dense);
+    const IndexFacts src_facts = take_indices(src_index, n, si, src_all_dense, inlined),
+                     dst_facts = take_indices(dst_index, n, di, dst_all_dense, inlined);
     if (src_facts.highest >= src_entries || dst_facts.highest >= dst_entries) {
         if (staging) upload_cache().put(device, staging, staging_cap);
         return nixl_amd_fail(NIXL_AMD_ERR_INDEX, "plan_create_indexed: an index names no entry of its list");
