@@ -449,6 +449,26 @@ nixl_amd_ep_ht_combine(void *combined_x,
                        int num_ranks,
                        void *stream);
 
+/* The same for a caller that knows how many rows `x` has: the kernel's form is chosen by the rows that a
+ * token gathers.  The results do not depend on it, nor on num_rows being right; -1: not known. */
+int
+nixl_amd_ep_ht_combine_rows(void *combined_x,
+                            float *combined_topk_weights,
+                            const void *x,
+                            const float *topk_weights,
+                            const void *bias_0,
+                            const void *bias_1,
+                            const uint8_t *is_token_in_rank,
+                            const int *recv_gbl_rank_prefix_sum,
+                            const int *send_head,
+                            const int64_t *recv_row_offset,
+                            int64_t num_rows,
+                            int num_tokens,
+                            int hidden,
+                            int num_topk,
+                            int num_ranks,
+                            void *stream);
+
 /*
  * Router: for every token the K largest logits (descending, ties to the lower expert
  * index) and the softmax over those K logits in fp32.  No counterpart in the reference,

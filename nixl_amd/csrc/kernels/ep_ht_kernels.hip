@@ -820,18 +820,20 @@ ht_meta_kernel(HtMeta m,
 
 // ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
 // grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x of them,
-// every wave for itself.  Two forms: up to kHtCombineEager values of output, four waves a
-// workgroup and positions loaded beside the flags (EAGER), which shortens the chain of loads;
-// beyond, one wave a workgroup and positions behind the flags.  Which is faster depends on the
-// rows a token gathers more than on the size: with few of them the eager form at every size (2 ranks
-// x 4096 x 4096 35.3 us against 41.6, 2 x 16 384 130 and 157; 8 x 1024 top-4 48.4 and 52.4, 8 x 4096 182 and 200),
-// with 5.3 a token the other one from 2^24 values on, ever more so (8 x 206 x 7168 top-8 27.8 and 27.0, 8 x 585
-// 71 and 68, 8 x 2340 283 and 261; 16 x 512 x 4096 85.5 and 84.6, 16 x 2048 352 and 340).  The number of
-// rows is not known here.  With the line at 2^25 values, calls below it that gather many rows lose up
-// to 4 % and calls above it that gather few up to 17 %, against the other form; neither is slower than
-// the look-up shared by two waves that came before both (8 x 1024 x 4096 52.8, 2 x 4096 x 4096 40.4).
+// every wave for itself.  Two forms: positions loaded beside the flags (EAGER), which shortens the chain
+// of loads, or behind them, which spares loads.  Which is faster depends on the rows that a token
+// gathers, as long as the call is so large that there are always waves to take over: us a call, eager and not,
+// 2 x 4096 x 7168 (2.0 rows a token) 62 and 72, 4 x 4096 x 7168 (3.6) 165 and 176, 8 x 4096 x 4096 (1.9) 138 and 156, (3.4) 182 and 195,
+// (3.9) 204 and 211, (4.4) 235 and 227, (5.3) 276 and 267, 8 x 4096 x 7168 (3.4) 317 and 337, (3.9) 363 and 363, (4.4) 409 and 397,
+// (5.3) 481 and 464.  Up to kHtCombineEager values the eager one is as fast or faster with any number of rows (8 x 256 x 7168 (5.3) 30.0 and
+// 30.9, 16 x 512 x 4096 (6.8) 84.1 and 84.0).  A call that does not say how many rows there are is eager up to that size.
+// A wave a workgroup, but four where a row is whole workgroups of them and tokens gather few rows: 8 x 4096 x 4096 (1.9) 134 and
+// 138 with one, 4 x 4096 x 4096 (2.8) 79.9 and 81.1, 8 x 4096 x 4096 (3.4) 182.5 and 181.9, (3.9) 208 and 205, 8 x 1024 x 4096 (3.9) 54.8 and
+// 55.3, (4.4) 58.8 and 57.9; with rows of 7168, which leave a fourth of every fourth workgroup idle, 4 x 1024 (1.8) 33.1 and 30.9, 4 x 4096
+// (3.6) 175 and 165.
 constexpr int kHtCombineEagerLanes = 256;
 constexpr long long kHtCombineEager = 1ll << 25;
+constexpr int kHtCombineManyRows = 4, kHtCombineFewRows = 3; // a token; few are as many as are not many in a small call
 
 template<bool EAGER>
 __global__ void __launch_bounds__(kHtCombineEagerLanes)
@@ -1192,6 +1194,46 @@ nixl_amd_ep_ht_dispatch(void *recv_x,
 }
 
 int
+nixl_amd_ep_ht_combine_rows(void *combined_x,
+                            float *combined_topk_weights,
+                            const void *x,
+                            const float *topk_weights,
+                            const void *bias_0,
+                            const void *bias_1,
+                            const uint8_t *is_token_in_rank,
+                            const int *recv_gbl_rank_prefix_sum,
+                            const int *send_head,
+                            const int64_t *recv_row_offset,
+                            int64_t num_rows,
+                            int num_tokens,
+                            int hidden,
+                            int num_topk,
+                            int num_ranks,
+                            void *stream) {
+    const int rc = check_ht("ht_combine", num_tokens, hidden, num_topk, num_ranks, num_ranks);
+    if (rc) return rc;
+    if (hidden == 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_combine: hidden must be positive");
+    if (!combined_x || !x || !is_token_in_rank || !recv_gbl_rank_prefix_sum || !send_head || !recv_row_offset)
+        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_combine: null pointer argument");
+    const HtDims d{num_ranks, num_tokens, hidden, num_topk, num_ranks};
+    const long long tokens = static_cast<long long>(num_ranks) * num_tokens;
+    const bool large = tokens * hidden > kHtCombineEager;
+    const bool eager = !large || (num_rows >= 0 && num_rows <= kHtCombineManyRows * tokens);
+    const int row_lanes = round_up_wave(hidden / 8);
+    const bool four_waves = eager && row_lanes % kHtCombineEagerLanes == 0 && num_rows <= (large ? kHtCombineFewRows : kHtCombineManyRows) * tokens;
+    const int lanes = four_waves ? kHtCombineEagerLanes : kWaveSize, parts = row_lanes / lanes;
+    if (static_cast<long long>(num_ranks) * num_tokens * parts >= (1ll << 31))
+        return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_combine: too many tokens");
+    hipLaunchKernelGGL(eager ? ht_combine_kernel<true> : ht_combine_kernel<false>,
+                       dim3(static_cast<unsigned>(num_ranks) * num_tokens * parts), dim3(lanes), 0, static_cast<hipStream_t>(stream), static_cast<uint16_t *>(combined_x), combined_topk_weights,
+                       static_cast<const uint16_t *>(x), topk_weights, static_cast<const uint16_t *>(bias_0),
+                       static_cast<const uint16_t *>(bias_1), is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
+                       reinterpret_cast<const long long *>(recv_row_offset), d, parts);
+    HIP_TRY(hipGetLastError());
+    return NIXL_AMD_OK;
+}
+
+int
 nixl_amd_ep_ht_combine(void *combined_x,
                        float *combined_topk_weights,
                        const void *x,
@@ -1207,25 +1249,9 @@ nixl_amd_ep_ht_combine(void *combined_x,
                        int num_topk,
                        int num_ranks,
                        void *stream) {
-    const int rc = check_ht("ht_combine", num_tokens, hidden, num_topk, num_ranks, num_ranks);
-    if (rc) return rc;
-    if (hidden == 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_combine: hidden must be positive");
-    if (!combined_x || !x || !is_token_in_rank || !recv_gbl_rank_prefix_sum || !send_head || !recv_row_offset)
-        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_combine: null pointer argument");
-    const HtDims d{num_ranks, num_tokens, hidden, num_topk, num_ranks};
-    // the lanes of a row dealt evenly to workgroups of at most four waves, or of one
-    const bool eager = static_cast<long long>(num_ranks) * num_tokens * hidden <= kHtCombineEager;
-    const int row_lanes = round_up_wave(hidden / 8), most = eager ? kHtCombineEagerLanes : kWaveSize;
-    const int parts = (row_lanes + most - 1) / most, lanes = round_up_wave((row_lanes + parts - 1) / parts);
-    if (static_cast<long long>(num_ranks) * num_tokens * parts >= (1ll << 31))
-        return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_combine: too many tokens");
-    hipLaunchKernelGGL(eager ? ht_combine_kernel<true> : ht_combine_kernel<false>,
-                       dim3(static_cast<unsigned>(num_ranks) * num_tokens * parts), dim3(lanes), 0, static_cast<hipStream_t>(stream), static_cast<uint16_t *>(combined_x), combined_topk_weights,
-                       static_cast<const uint16_t *>(x), topk_weights, static_cast<const uint16_t *>(bias_0),
-                       static_cast<const uint16_t *>(bias_1), is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
-                       reinterpret_cast<const long long *>(recv_row_offset), d, parts);
-    HIP_TRY(hipGetLastError());
-    return NIXL_AMD_OK;
+    return nixl_amd_ep_ht_combine_rows(combined_x, combined_topk_weights, x, topk_weights, bias_0, bias_1, is_token_in_rank,
+                                       recv_gbl_rank_prefix_sum, send_head, recv_row_offset, -1, num_tokens, hidden, num_topk,
+                                       num_ranks, stream);
 }
 
 int

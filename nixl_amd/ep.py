@@ -653,7 +653,7 @@ class Buffer:
         self._after(previous_event, async_finish, allocate_on_comm_stream)
         combined = torch.empty((R, T, H), dtype=torch.bfloat16, device=dev)
         combined_w = torch.empty((R, T, K), dtype=torch.float32, device=dev) if K else None
-        _check(self._k.nixl_amd_ep_ht_combine(_ptr(combined), _ptr(combined_w), _ptr(x), _ptr(topk_weights),
-                                              _ptr(bias_0), _ptr(bias_1), _ptr(in_rank), _ptr(prefix), _ptr(send_head),
-                                              _ptr(row_offset), T, H, max(K, 1), R, _stream()), "ht_combine")
+        _check(self._k.nixl_amd_ep_ht_combine_rows(_ptr(combined), _ptr(combined_w), _ptr(x), _ptr(topk_weights),
+                                                   _ptr(bias_0), _ptr(bias_1), _ptr(in_rank), _ptr(prefix), _ptr(send_head),
+                                                   _ptr(row_offset), x.shape[0], T, H, max(K, 1), R, _stream()), "ht_combine")
         return combined, combined_w, self._done(async_finish)

@@ -1425,3 +1425,42 @@ def test_notify_counts_flags(cuda, R, T):
     per_channel = -(-T // C)
     ends = [min((c + 1) * per_channel, T) - 1 for c in range(C)]
     assert torch.equal(dev["channels"].cpu(), before[:, ends].permute(0, 2, 1).int())
+
+
+@pytest.mark.parametrize("R,T,H,K", [(3, 37, 2048, 2), (3, 37, 1032, 2), (8, 300, 4096, 8), (1, 5, 8, 1), (4, 1030, 8192, 4), (66, 9, 256, 3)])
+def test_combine_in_every_form(cuda, R, T, H, K):
+    """The form of normal-mode combine follows the rows that a token gathers, the size of the call and of a row:
+    bit for bit the same results whatever number of rows the caller states, with and without biases
+    and weights, and those of a sum in double precision within a rounding to bfloat16."""
+    import torch
+    g = torch.Generator(device=cuda).manual_seed(R + T + H)
+    E = 2 * R
+    topk = torch.topk(torch.rand((R, T, E), generator=g, device=cuda), K, dim=2)[1].to(torch.int32)
+    buf = Buffer(R, low_latency_mode=False, device=cuda)
+    per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk, E)
+    x = torch.randn((R, T, H), generator=g, device=cuda).to(torch.bfloat16)
+    w = torch.rand((R, T, K), generator=g, device=cuda)
+    rows, _, row_w, _, handle, _ = buf.ht_dispatch(x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=per_expert,
+                                                   topk_idx=topk, topk_weights=w)
+    y = torch.randn(rows.shape, generator=g, device=cuda).to(torch.bfloat16)
+    bias = torch.randn((R, T, H), generator=g, device=cuda).to(torch.bfloat16)
+    in_rank, prefix, _, meta, head, offset = handle
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
+    for b, weights in ((None, row_w), (bias, None)):
+        seen = []
+        for n in (-1, 0, rows.shape[0], 3 * R * T, 4 * R * T, 4 * R * T + 1, 1 << 40):
+            out = torch.zeros((R, T, H), dtype=torch.bfloat16, device=cuda)
+            out_w = torch.zeros((R, T, K), device=cuda) if weights is not None else None
+            rc = _lib.ep_kernels().nixl_amd_ep_ht_combine_rows(ptr(out), ptr(out_w), ptr(y), ptr(weights), ptr(b), None, ptr(in_rank), ptr(prefix),
+                                                               ptr(head), ptr(offset), n, T, H, K, R, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, _lib.kernels_error()
+            seen.append((out, out_w))
+        for out, out_w in seen[1:]:
+            assert torch.equal(out.view(torch.int16), seen[0][0].view(torch.int16))
+            assert out_w is None or torch.equal(out_w, seen[0][1])
+        want = torch.zeros((R * T, H), dtype=torch.float64, device=cuda) if b is None else b.double().view(R * T, H)
+        for lo in range(0, rows.shape[0], 4096):
+            at = meta[lo:lo + 4096].long()
+            want.index_add_(0, at[:, 0] * T + at[:, 1], y[lo:lo + 4096].double())
+        # at most 9 additions of 2^-24 of sums below 64, and half a step of bfloat16
+        assert bool(((seen[0][0].double().view(R * T, H) - want).abs() <= want.abs() / 256 + 4e-5).all())
