@@ -424,6 +424,36 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
                                int num_experts,
                                void *stream);
 
+/* The same for a caller that knows how many rows are going to be written (a dispatch with the layout of an
+ * earlier one does): the kernel's form is chosen by the rows of a token.  The results do not depend on it, nor
+ * on num_rows being right; -1: not known. */
+int
+nixl_amd_ep_ht_dispatch_rows(void *recv_x,
+                             void *recv_x_scales,
+                             int32_t *recv_topk_idx,
+                             float *recv_topk_weights,
+                             int32_t *recv_src_meta,
+                             const void *x,
+                             const void *x_scales,
+                             const int32_t *topk_idx,
+                             const float *topk_weights,
+                             const uint8_t *is_token_in_rank,
+                             const int *recv_gbl_rank_prefix_sum,
+                             const int *send_head,
+                             const int64_t *recv_row_offset,
+                             int64_t num_rows,
+                             int num_tokens,
+                             int hidden,
+                             int elem_bytes,
+                             int num_scales,
+                             int64_t scale_rank_stride,
+                             int64_t scale_token_stride,
+                             int64_t scale_hidden_stride,
+                             int num_topk,
+                             int num_ranks,
+                             int num_experts,
+                             void *stream);
+
 /*
  * Normal-mode combine.  Replaces ht::combine with one reduction stage
  * (kernels/api.cuh:176-203; combine_token, kernels/nixl_ep_ht.cu:1682-1737):

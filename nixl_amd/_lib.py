@@ -131,6 +131,7 @@ _EP_SIGS = {
     "nixl_amd_ep_ht_notify_dispatch": [c_void_p] * 8 + [c_int] * 5 + [c_void_p],
     "nixl_amd_ep_ht_dispatch": [c_void_p] * 11 + [c_int] * 5 + [c_void_p],
     "nixl_amd_ep_ht_dispatch_scaled": [c_void_p] * 13 + [c_int] * 4 + [c_int64] * 3 + [c_int] * 3 + [c_void_p],
+    "nixl_amd_ep_ht_dispatch_rows": [c_void_p] * 13 + [c_int64] + [c_int] * 4 + [c_int64] * 3 + [c_int] * 3 + [c_void_p],
     "nixl_amd_ep_ht_combine": [c_void_p] * 10 + [c_int] * 4 + [c_void_p],
     "nixl_amd_ep_ht_combine_rows": [c_void_p] * 10 + [c_int64] + [c_int] * 4 + [c_void_p],
     "nixl_amd_ep_router_topk": [c_void_p] * 3 + [c_int] * 3 + [c_void_p],

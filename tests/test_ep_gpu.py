@@ -1464,3 +1464,31 @@ def test_combine_in_every_form(cuda, R, T, H, K):
             want.index_add_(0, at[:, 0] * T + at[:, 1], y[lo:lo + 4096].double())
         # at most 9 additions of 2^-24 of sums below 64, and half a step of bfloat16
         assert bool(((seen[0][0].double().view(R * T, H) - want).abs() <= want.abs() / 256 + 4e-5).all())
+
+
+@pytest.mark.parametrize("K", [3, 8])
+def test_large_dispatch_in_both_forms(cuda, K):
+    """Inputs beyond 128 MiB, of tokens that go to few ranks and to many: every row that is received, with the layout of its own
+    and with a kept one, is its source row, whatever number of rows the caller of the kernel states."""
+    import torch
+    R, T, H, E = 8, 1025, 8192, 64
+    g = torch.Generator(device=cuda).manual_seed(K)
+    topk = torch.topk(torch.rand((R, T, E), generator=g, device=cuda), K, dim=2)[1].to(torch.int32)
+    w = torch.rand((R, T, K), generator=g, device=cuda)
+    buf = Buffer(R, low_latency_mode=False, device=cuda)
+    per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk, E)
+    x = torch.randint(-2**15, 2**15, (R, T, H), generator=g, dtype=torch.int16, device=cuda).view(torch.bfloat16)
+    rows, _, _, _, handle, _ = buf.ht_dispatch(x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=per_expert,
+                                               topk_idx=topk, topk_weights=w)
+    in_rank, prefix, _, meta, head, offset = handle
+    assert rows.shape[0] == int(in_rank.sum())
+    want = x.view(torch.int16)[meta[:, 0].long(), meta[:, 1].long()]
+    assert torch.equal(rows.view(torch.int16), want)
+    assert torch.equal(buf.ht_dispatch(x, handle=handle)[0].view(torch.int16), want)
+    for n in (0, 4 * R * T, 4 * R * T + 1, -1):
+        out = torch.zeros_like(rows)
+        rc = _lib.ep_kernels().nixl_amd_ep_ht_dispatch_rows(out.data_ptr(), None, None, None, None, x.data_ptr(), None, None, None, in_rank.data_ptr(),
+                                                            prefix.data_ptr(), head.data_ptr(), offset.data_ptr(), n, T, H, 2, 0, 0, 0, 0, 0, R, R,
+                                                            torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, _lib.kernels_error()
+        assert torch.equal(out.view(torch.int16), want)
