@@ -996,13 +996,26 @@ round_up_wave(int n) {
     return (n + kWaveSize - 1) / kWaveSize * kWaveSize;
 }
 
+// Workgroup of ll_dispatch_kernel for a row of `lanes` lanes, while nobody has set another: a token's
+// whole row, since every workgroup finds the token's rows again.  Rows of 10 to 15 waves (bf16 from hidden 5120 to below 8192) leave
+// a compute unit's last waves idle that way and go by workgroups of two.  Dispatch, whole rows and workgroups of two waves, us: 32 ranks x 128
+// tokens, top-8, hidden 7168 112 and 106, 6144 94.8 and 93.2, 5120 88.0 and 88.6; top-2 44.2 and 38.5, 39.0 and 37.2, 37.0 and 32.8; 16 x 128,
+// top-4, 31.5 and 27.6, 26.2 and 22.1, 23.1 and 22.9.  Not so rows of 16 waves (hidden 8192, top-2 43.3 and 45.8, 16 x 128 top-4 33.6 and
+// 35.2), of 9 (4608, top-8 70.5 and 75.6: half of the last workgroup is idle), of 8 (4096, 60.8 and 65.9), and fp8 rows (7168, 7 waves, 69.3 and 75.3).
+int
+dispatch_workgroup(int lanes) {
+    constexpr int kPart = 2 * kWaveSize;
+    const int row = round_up_wave(lanes);
+    return row > 512 && row < 1024 && row % kPart == 0 ? kPart : row;
+}
+
 // Largest workgroup (in lanes) of the dispatch and combine kernels; a token whose row needs
 // more lanes is split over several workgroups.
 // Read by every call, set by nixl_amd_ep_ll_set_tuning from any thread: a call sees the old or the
-// new value, never a torn one.  Combine, while nobody has set it (0): a row of more than 512
+// new value, never a torn one; 0: nobody has set it.  Combine then: a row of more than 512
 // lanes is split into two halves (hidden 7168: two workgroups of 448 lanes, 91.6 us against
 // 94.4 for one of 896; 128 and 64 lanes: 93.6-94.4).
-std::atomic<int> g_dispatch_lanes{1024};
+std::atomic<int> g_dispatch_lanes{0};
 std::atomic<int> g_combine_lanes{0};
 
 } // namespace
@@ -1048,7 +1061,7 @@ nixl_amd_ep_ll_set_tuning(int dispatch_lanes, int combine_lanes) {
     if (!ok(dispatch_lanes) || !ok(combine_lanes))
         return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ll_set_tuning: lanes must be 0, -1 or a multiple of 64 in [64, 1024]");
     // -1: back to what the library starts with
-    if (dispatch_lanes) g_dispatch_lanes.store(dispatch_lanes == -1 ? 1024 : dispatch_lanes, std::memory_order_relaxed);
+    if (dispatch_lanes) g_dispatch_lanes.store(dispatch_lanes == -1 ? 0 : dispatch_lanes, std::memory_order_relaxed);
     if (combine_lanes) g_combine_lanes.store(combine_lanes == -1 ? 0 : combine_lanes, std::memory_order_relaxed);
     return NIXL_AMD_OK;
 }
@@ -1188,7 +1201,8 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
         a.use_ue8m0 = c.use_ue8m0;
         a.meta_wgs = (d.E + kDirectExperts - 1) / kDirectExperts;
         const int lanes = c.use_fp8 ? row_lanes<true>(d.H) : row_lanes<false>(d.H);
-        const int most = std::min(kDirectMaxThreads, g_dispatch_lanes.load(std::memory_order_relaxed));
+        const int set = g_dispatch_lanes.load(std::memory_order_relaxed);
+        const int most = set ? std::min(kDirectMaxThreads, set) : kDirectMaxThreads;
         a.parts = (lanes + most - 1) / most;
         const dim3 grid(static_cast<unsigned>(a.meta_wgs + d.R * d.T * a.parts));
         // as many waves as there may be, also where the row needs one: they share the counting (2048
@@ -1290,7 +1304,8 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
     a.recv_scales = c.packed_recv_x_scales;
     a.use_ue8m0 = c.use_ue8m0;
     const int lanes = c.use_fp8 ? row_lanes<true>(d.H) : row_lanes<false>(d.H);
-    const int wg = std::min(round_up_wave(lanes), g_dispatch_lanes.load(std::memory_order_relaxed));
+    const int set = g_dispatch_lanes.load(std::memory_order_relaxed);
+    const int wg = set ? std::min(round_up_wave(lanes), set) : dispatch_workgroup(lanes);
     a.parts = (lanes + wg - 1) / wg;
     const dim3 grid(static_cast<unsigned>(d.R) * d.T * a.parts);
     const dim3 block(wg);

@@ -1492,3 +1492,15 @@ def test_large_dispatch_in_both_forms(cuda, K):
                                                             torch.cuda.current_stream().cuda_stream)
         assert rc == 0, _lib.kernels_error()
         assert torch.equal(out.view(torch.int16), want)
+
+
+@pytest.mark.parametrize("hidden", [4096, 4608, 5120, 5632, 6144, 7168, 8064, 8192])
+def test_ll_dispatch_of_wide_bf16_rows(cuda, hidden):
+    """Rows whose workgroups are split and rows whose are not, in a call that is not one launch, with
+    selections left out: every byte against the oracle."""
+    R, T, K, E, M = 4, 66, 8, 16, 70
+    x, topk, _ = make_world(hidden, R, T, hidden, K, E, drop=0.02, scale=1.0)
+    want = eo.ll_dispatch(bits16(x).reshape(R, T, hidden), topk, E, M, False, fill=0x55)
+    rc, got = raw_ll_dispatch(cuda, x, topk, E, M, False)
+    assert rc == 0, _lib.kernels_error()
+    assert_dispatch_equal(got, want, False)
