@@ -244,7 +244,8 @@ nixl_amd_copy_list_device(const nixl_amd_copy_list_t *list);
  * lengths) and writes the records; the call waits for its verdict and returns
  * NIXL_AMD_ERR_INVALID if a pair is bad.  `n_continued` (may be NULL) receives how many pairs
  * continue the pair before them on both sides: the descriptors an agent that merges
- * neighbours would not have listed (src/core/nixl_agent.cpp:799-857). */
+ * neighbours would not have listed (src/core/nixl_agent.cpp:799-857).  The kernel runs on the
+ * stream that `tuning` names while that is idle (see there), else on one of the library's. */
 int
 nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
                                  const int32_t *src_index,

@@ -246,7 +246,7 @@ copy_piece_kernel(const PieceRec *__restrict__ recs, uint32_t n_recs, uint32_t p
     }
 }
 
-// One wavefront per chunk that crosses descriptor boundaries or is short.
+// One wavefront per chunk of the stream of tiny descriptors.
 template<int UPL, int POL>
 __global__ void __launch_bounds__(kMixedThreads)
 copy_mixed_kernel(MixedArgs a) {
@@ -1406,7 +1406,7 @@ private:
 };
 
 // Byte descriptors of kSplitFromBytes and more (at least two chunks of the largest size besides a
-// first line) are placed when the others are known.  They may join the stream of chunks, and beyond
+// first line) are placed when the others are known.  They may become chunks, and beyond
 // kLongItemsFrom of them the items take four rounds each, as making four times as many costs more
 // than the copy gains (64 MiB in tensors of 1 MiB + 2 B: 24 us to make and 20.6 to copy with short
 // items, 10.7 and 22.0 with long).

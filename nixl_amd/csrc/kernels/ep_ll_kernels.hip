@@ -14,7 +14,7 @@
 //                          indices and weights out as well.  This is the send phase.
 //   1b. ll_arrival_kernel  only for calls with a time-out: the receive side's bounded wait for
 //                          each source rank's bits; a late rank loses its bits and is masked.
-//   2. ll_dispatch_kernel  one workgroup per token reads its bf16 row once and, while the row
+//   2. ll_dispatch_kernel  one workgroup per token (or several, dispatch_workgroup) reads its bf16 row once and, while the row
 //                          travels, counts for each of its K experts the bits in front of its
 //                          own (tokens of lower ranks, then lower tokens of its rank): that is
 //                          its row inside the expert.  It quantises the row in registers and
