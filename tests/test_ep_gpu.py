@@ -1504,3 +1504,49 @@ def test_ll_dispatch_of_wide_bf16_rows(cuda, hidden):
     rc, got = raw_ll_dispatch(cuda, x, topk, E, M, False)
     assert rc == 0, _lib.kernels_error()
     assert_dispatch_equal(got, want, False)
+
+
+@pytest.mark.parametrize("lanes", [64, 128, 192, 1024])
+@pytest.mark.parametrize("hidden", [1152, 5120, 7168])
+def test_ll_repeated_expert_in_rows_of_several_workgroups(cuda, hidden, lanes):
+    """A call with repeats whose bf16 rows are several workgroups of `lanes` lanes, the last of them not full: the first
+    one moves the whole row.  Ragged ranks and left-out selections; every byte against the oracle."""
+    R, T, K, E, M = 4, 130, 5, 16, 150
+    x, topk, _ = make_world(hidden + lanes, R, T, hidden, K, E, drop=0.05)
+    _with_repeats(np.random.default_rng(hidden), topk, 7)
+    nt = np.array([T, T - 1, 1, T // 2], np.int32)
+    want = eo.ll_dispatch(bits16(x), topk, E, M, False, num_tokens=nt, fill=0x55)
+    lib = _lib.ep_kernels()
+    assert lib.nixl_amd_ep_ll_set_tuning(lanes, 0) == 0
+    try:
+        rc, got = raw_ll_dispatch(cuda, x, topk, E, M, False, num_tokens=nt)
+    finally:
+        assert lib.nixl_amd_ep_ll_set_tuning(-1, 0) == 0
+    assert rc == 0, _lib.kernels_error()
+    assert_dispatch_equal(got, want, False)
+
+
+def test_ll_repeated_expert_is_looked_for_once_a_token(cuda):
+    """One repeat in a call makes the search for the rows what takes long.  Workgroups of two waves, seven to a row,
+    must not each do it again (4.8 times the time of one workgroup a row when they did; 1.4 with the first alone)."""
+    R, T, H, K, E = 32, 64, 7168, 8, 256
+    g = torch.Generator(device=cuda).manual_seed(3)
+    x = torch.randn((R, T, H), generator=g, device=cuda).to(torch.bfloat16)
+    topk = torch.topk(torch.rand((R, T, E), generator=g, device=cuda), K)[1].to(torch.int32).contiguous()
+    topk[1, 2, 3] = topk[1, 2, 0]
+    buf, lib = Buffer(R, device=cuda), _lib.ep_kernels()
+    took = {}
+    try:
+        for lanes in (1024, 128, 1024, 128, 1024, 128):
+            assert lib.nixl_amd_ep_ll_set_tuning(lanes, 0) == 0
+            buf.dispatch(x, topk, T, E, use_fp8=False)
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(5):
+                buf.dispatch(x, topk, T, E, use_fp8=False)
+            e1.record()
+            e1.synchronize()
+            took.setdefault(lanes, []).append(e0.elapsed_time(e1))
+    finally:
+        assert lib.nixl_amd_ep_ll_set_tuning(-1, 0) == 0
+    assert min(took[128]) < 2.5 * min(took[1024]), took
