@@ -31,8 +31,8 @@ extern "C" {
 /* Launch-shape knob of the low-latency kernels (no reference counterpart): the largest
  * workgroup, in lanes, of the dispatch and combine kernels; a multiple of 64 in [64, 1024],
  * 0 to leave a value unchanged, or -1 to return to the built-in choice: dispatch takes a
- * workgroup per token, or several of 128 lanes for a row of 640, 768 or 896, combine one per
- * row, or two halves for a row of more than 512 lanes.
+ * workgroup per token, or several of 128 lanes for some rows of 640, 768 or 896, combine one
+ * per row, or two halves for a row of more than 512 lanes.
  * Process-wide; may be called from any thread: a dispatch or
  * combine call that runs at the same time uses the old or the new value. */
 int

@@ -1012,16 +1012,24 @@ round_up_wave(int n) {
 }
 
 // Workgroup of ll_dispatch_kernel for a row of `lanes` lanes, while nobody has set another: a token's
-// whole row, since every workgroup finds the token's rows again.  Rows of 10 to 15 waves (bf16 from hidden 5120 to below 8192) leave
-// a compute unit's last waves idle that way and go by workgroups of two.  Dispatch, whole rows and workgroups of two waves, us: 32 ranks x 128
-// tokens, top-8, hidden 7168 112 and 106, 6144 94.8 and 93.2, 5120 88.0 and 88.6; top-2 44.2 and 38.5, 39.0 and 37.2, 37.0 and 32.8; 16 x 128,
-// top-4, 31.5 and 27.6, 26.2 and 22.1, 23.1 and 22.9.  Not so rows of 16 waves (hidden 8192, top-2 43.3 and 45.8, 16 x 128 top-4 33.6 and
-// 35.2), of 9 (4608, top-8 70.5 and 75.6: half of the last workgroup is idle), of 8 (4096, 60.8 and 65.9), and fp8 rows (7168, 7 waves, 69.3 and 75.3).
+// whole row, since every workgroup finds the token's rows again.  Rows of 10, 12 and 14 waves (bf16, hidden
+// 5120, 6144 and 7168), which leave some of a compute unit's 32 waves idle that way, go by workgroups of two
+// where that was never slower.  With one or two rows a token it is mostly latency: 32 ranks x 128 tokens x 7168 45.3 and
+// 39.5 us, 16 x 128 23.0 and 18.4.  With three or four as long as the call is below four times what the chip holds
+// at once (16 x 128 x 7168 30.6 and 27.5, 32 x 72 x 5120 26.2 and 23.2, but 32 x 87 x 6144 36.0 and 39.9).  Rows of 14 waves again from seven
+// rounds of whole rows on, two to a compute unit (four rows a token 59.2 and 57.5, eight 112 and 105; five 72.1 and 73.4), where many rows a
+// token lose it in larger calls (32 x 256, eight rows, 198 and 204).
 int
-dispatch_workgroup(int lanes) {
-    constexpr int kPart = 2 * kWaveSize;
+dispatch_workgroup(int lanes, const LlDims &d) {
+    constexpr int kPart = 2 * kWaveSize, kWideRow = 14 * kWaveSize;
+    constexpr long long kSmallCall = 30720; // waves
+    constexpr long long kLargeCall = 3584, kVeryLargeCall = 5120; // tokens
     const int row = round_up_wave(lanes);
-    return row > 512 && row < 1024 && row % kPart == 0 ? kPart : row;
+    if (row <= 512 || row >= 1024 || row % kPart) return row;
+    const long long tokens = static_cast<long long>(d.R) * d.T;
+    const bool few = d.K <= 2 || (d.K <= 4 && tokens * (row / kWaveSize) <= kSmallCall);
+    const bool wide = row == kWideRow && tokens > kLargeCall && (d.K <= 4 || (d.K >= 6 && tokens <= kVeryLargeCall));
+    return few || wide ? kPart : row;
 }
 
 // Largest workgroup (in lanes) of the dispatch and combine kernels; a token whose row needs
@@ -1320,7 +1328,7 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
     a.use_ue8m0 = c.use_ue8m0;
     const int lanes = c.use_fp8 ? row_lanes<true>(d.H) : row_lanes<false>(d.H);
     const int set = g_dispatch_lanes.load(std::memory_order_relaxed);
-    const int wg = set ? std::min(round_up_wave(lanes), set) : dispatch_workgroup(lanes);
+    const int wg = set ? std::min(round_up_wave(lanes), set) : dispatch_workgroup(lanes, d);
     a.parts = (lanes + wg - 1) / wg;
     const dim3 grid(static_cast<unsigned>(d.R) * d.T * a.parts);
     const dim3 block(wg);

@@ -1550,3 +1550,18 @@ def test_ll_repeated_expert_is_looked_for_once_a_token(cuda):
     finally:
         assert lib.nixl_amd_ep_ll_set_tuning(-1, 0) == 0
     assert min(took[128]) < 2.5 * min(took[1024]), took
+
+
+@pytest.mark.parametrize("R,T,K", [(16, 66, 2), (16, 34, 4)])
+@pytest.mark.parametrize("hidden", [5120, 6144, 7168])
+def test_ll_dispatch_of_wide_bf16_rows_with_few_selections(cuda, hidden, R, T, K):
+    """Rows that go by workgroups of two waves, whole and with repeats: every byte against the oracle."""
+    E, M = 16, T + 3
+    x, topk, _ = make_world(hidden + K, R, T, hidden, K, E, drop=0.0, scale=1.0)
+    for repeats in (False, True):
+        if repeats:
+            _with_repeats(np.random.default_rng(K), topk, 2, triple=False)
+        want = eo.ll_dispatch(bits16(x).reshape(R, T, hidden), topk, E, M, False, fill=0x55)
+        rc, got = raw_ll_dispatch(cuda, x, topk, E, M, False)
+        assert rc == 0, _lib.kernels_error()
+        assert_dispatch_equal(got, want, False)
