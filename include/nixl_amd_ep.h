@@ -425,9 +425,8 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
                                int num_experts,
                                void *stream);
 
-/* The same for a caller that knows how many rows are going to be written (a dispatch with the layout of an
- * earlier one does): the kernel's form is chosen by the rows of a token.  The results do not depend on it, nor
- * on num_rows being right; -1: not known. */
+/* The same with the number of rows that are going to be written, which is not looked at: the kernel reads it
+ * behind the last rank's offset, where notify left it. */
 int
 nixl_amd_ep_ht_dispatch_rows(void *recv_x,
                              void *recv_x_scales,

@@ -11,7 +11,6 @@
 // HBM traffic: dispatch reads every source row once (2H) and writes it once per destination
 // rank that holds one of its experts; combine reads those rows once and writes 2H per token.
 #include <algorithm>
-#include <cmath>
 #include <cstdint>
 
 #include "common.h"
@@ -563,12 +562,12 @@ next_row(const WaveRows &w, unsigned long long &hits) {
 // again and again takes 44 us with ordinary loads and 54 without.
 //
 // Positions of rows are loaded beside the flags (EAGER) or behind them, which spares the loads of
-// destinations that do not hold the token and is faster for large calls whose tokens go to many: us of 8 x 4096 x 7168 bf16, top-8
-// (5.3 rows a token), eager and not, again and again 513 and 484, behind a 512 MB fill 535 and 505, behind a kernel on the input 485 and
-// 491, passes with combine 985 and 962, with such a kernel in front of each 1109 and 1107; top-6 (4.4) passes 844 and 826, 978 and 967; 8 x 2048 top-8
-// 491 and 481; 16 x 1024 (6.5) 631 and 611.  With few rows it is slower: top-4 (3.3) behind the fill 334 and 347, 8 x 4096 x 4096 top-2 (1.9) passes
-// 268 and 284.  So it is with the scales of fp8 rows in the launch (passes 738 and 769, 808 and 797 behind a kernel on the
-// input), and inputs up to kHtStreamFrom are the same either way (8 x 1024 x 4096 97.2 and 98.0, 8 x 512 x 7168 121.4 and 121.4).
+// destinations that do not hold the token and is faster for large calls whose tokens go to many.  Beside, behind, and
+// by the rows, us a pass of 8 x 4096 x 7168 bf16 top-8 with combine: 1006, 960, 959 with experts anywhere (5.3 rows a token);
+// 713, 714, 713 with those of four ranks a token (3.6 rows), 601, 607, 602 of three, 481, 501, 481 of two; dispatch
+// alone behind a kernel on the input 498, 481, 479 and, of two ranks, 219, 278, 220.  16 x 1024 (6.5 rows) 621, 604, 602.  Beside the
+// flags in any case: the scales of fp8 rows (passes 738 beside, 769 behind) and inputs up to kHtStreamFrom, which are the
+// same either way (8 x 1024 x 4096 97.2 and 98.0).
 constexpr long long kHtStreamFrom = 128ll << 20;
 constexpr int kHtManyRows = 4; // a token
 
@@ -584,7 +583,9 @@ struct HtRows {
     int streamed; // rows are loaded non-temporally
 };
 
-template<bool EAGER>
+// BY_ROWS: the number of rows decides when positions are loaded (else beside the flags).  It lies behind the last
+// rank's offset, is there as early as the flags, and only the host would have to wait for it.
+template<bool BY_ROWS>
 __device__ __forceinline__ void
 dispatch_piece(const HtRows &a, uint32_t piece) {
     const uint32_t token = piece / a.parts, part = piece % a.parts;
@@ -597,8 +598,10 @@ dispatch_piece(const HtRows &a, uint32_t piece) {
         const uint4 *from = reinterpret_cast<const uint4 *>(a.x + static_cast<size_t>(token) * a.d.H) + col;
         v = a.streamed ? ld16_nt(from) : *from;
     }
+    const bool few = !BY_ROWS || a.row_offset[a.d.R] <= static_cast<long long>(kHtManyRows) * a.d.R * a.d.T;
     for (int d0 = 0; d0 < a.d.R; d0 += kWaveSize) {
-        const WaveRows w = wave_rows<EAGER>(a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, r, t, d0);
+        const WaveRows w = few ? wave_rows<true>(a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, r, t, d0) :
+                                 wave_rows<false>(a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, r, t, d0);
         for (unsigned long long hits = w.hits; hits;) {
             const long long row = next_row(w, hits);
             if (active) st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * a.d.H) + col, v);
@@ -791,7 +794,7 @@ constexpr int kHtWaves = kHtThreads / kWaveSize;
 constexpr long long kHtMaxGrid = (1ll << 24) - 1;
 static_assert(kHtThreads == kHtMetaThreads && kHtThreads == kHtScaleThreads);
 
-template<bool VEC, bool SCALES, bool EAGER>
+template<bool VEC, bool SCALES, bool BY_ROWS>
 __global__ void __launch_bounds__(kHtThreads)
 ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint32_t meta_blocks, uint32_t first) {
     uint32_t block = blockIdx.x;
@@ -806,7 +809,7 @@ ht_dispatch_kernel(HtRows a, HtMeta m, HtScales sc, uint32_t scale_blocks, uint3
         meta_block<VEC>(m, a.in_rank, a.prefix, a.send_head, a.row_offset, a.d, first + block);
         return;
     }
-    dispatch_piece<EAGER>(a, (first + block - meta_blocks) * kHtWaves + uniform(threadIdx.x / kWaveSize));
+    dispatch_piece<BY_ROWS>(a, (first + block - meta_blocks) * kHtWaves + uniform(threadIdx.x / kWaveSize));
 }
 
 // From this many ranks on, the metadata has a launch of its own: a workgroup of it finds one token in
@@ -1083,31 +1086,30 @@ nixl_amd_ep_ht_notify_dispatch(const uint8_t *is_token_in_rank,
 }
 
 int
-nixl_amd_ep_ht_dispatch_rows(void *recv_x,
-                             void *recv_x_scales,
-                             int32_t *recv_topk_idx,
-                             float *recv_topk_weights,
-                             int32_t *recv_src_meta,
-                             const void *x,
-                             const void *x_scales,
-                             const int32_t *topk_idx,
-                             const float *topk_weights,
-                             const uint8_t *is_token_in_rank,
-                             const int *recv_gbl_rank_prefix_sum,
-                             const int *send_head,
-                             const int64_t *recv_row_offset,
-                             int64_t num_rows,
-                             int num_tokens,
-                             int hidden,
-                             int elem_bytes,
-                             int num_scales,
-                             int64_t scale_rank_stride,
-                             int64_t scale_token_stride,
-                             int64_t scale_hidden_stride,
-                             int num_topk,
-                             int num_ranks,
-                             int num_experts,
-                             void *stream) {
+nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
+                               void *recv_x_scales,
+                               int32_t *recv_topk_idx,
+                               float *recv_topk_weights,
+                               int32_t *recv_src_meta,
+                               const void *x,
+                               const void *x_scales,
+                               const int32_t *topk_idx,
+                               const float *topk_weights,
+                               const uint8_t *is_token_in_rank,
+                               const int *recv_gbl_rank_prefix_sum,
+                               const int *send_head,
+                               const int64_t *recv_row_offset,
+                               int num_tokens,
+                               int hidden,
+                               int elem_bytes,
+                               int num_scales,
+                               int64_t scale_rank_stride,
+                               int64_t scale_token_stride,
+                               int64_t scale_hidden_stride,
+                               int num_topk,
+                               int num_ranks,
+                               int num_experts,
+                               void *stream) {
     if (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4)
         return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_dispatch: elem_bytes must be 1, 2 or 4");
     if (hidden <= 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "ht_dispatch: hidden must be positive");
@@ -1151,15 +1153,9 @@ nixl_amd_ep_ht_dispatch_rows(void *recv_x,
     const bool vec = num_topk % 4 == 0 && bits % 16 == 0;
     const long long pieces = static_cast<long long>(num_ranks) * num_tokens * parts;
     const long long row_blocks = (pieces + kHtWaves - 1) / kHtWaves;
-    // rows a token: what the caller says, or those of selections that know no favourite ranks
-    const double tokens = static_cast<double>(num_ranks) * num_tokens;
-    const double per_token = num_rows >= 0 ? static_cast<double>(num_rows) / tokens :
-        num_topk > 0                       ? num_ranks * (1.0 - std::pow(1.0 - 1.0 / num_ranks, num_topk)) :
-                                             0.0;
-    const bool behind = !x_scales && rows.streamed && per_token > kHtManyRows;
-    const auto kernel = x_scales ? (vec ? ht_dispatch_kernel<true, true, true> : ht_dispatch_kernel<false, true, true>) :
-        behind                   ? (vec ? ht_dispatch_kernel<true, false, false> : ht_dispatch_kernel<false, false, false>) :
-                                   (vec ? ht_dispatch_kernel<true, false, true> : ht_dispatch_kernel<false, false, true>);
+    const auto kernel = x_scales ? (vec ? ht_dispatch_kernel<true, true, false> : ht_dispatch_kernel<false, true, false>) :
+        rows.streamed            ? (vec ? ht_dispatch_kernel<true, false, true> : ht_dispatch_kernel<false, false, true>) :
+                                   (vec ? ht_dispatch_kernel<true, false, false> : ht_dispatch_kernel<false, false, false>);
     const auto launch = [&](long long n_scale, long long n_meta, long long n_row, long long first) -> int {
         const long long blocks = n_scale + n_meta + n_row;
         if (blocks == 0) return NIXL_AMD_OK;
@@ -1190,34 +1186,35 @@ nixl_amd_ep_ht_dispatch_rows(void *recv_x,
 }
 
 int
-nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
-                               void *recv_x_scales,
-                               int32_t *recv_topk_idx,
-                               float *recv_topk_weights,
-                               int32_t *recv_src_meta,
-                               const void *x,
-                               const void *x_scales,
-                               const int32_t *topk_idx,
-                               const float *topk_weights,
-                               const uint8_t *is_token_in_rank,
-                               const int *recv_gbl_rank_prefix_sum,
-                               const int *send_head,
-                               const int64_t *recv_row_offset,
-                               int num_tokens,
-                               int hidden,
-                               int elem_bytes,
-                               int num_scales,
-                               int64_t scale_rank_stride,
-                               int64_t scale_token_stride,
-                               int64_t scale_hidden_stride,
-                               int num_topk,
-                               int num_ranks,
-                               int num_experts,
-                               void *stream) {
-    return nixl_amd_ep_ht_dispatch_rows(recv_x, recv_x_scales, recv_topk_idx, recv_topk_weights, recv_src_meta, x, x_scales,
-                                        topk_idx, topk_weights, is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
-                                        recv_row_offset, -1, num_tokens, hidden, elem_bytes, num_scales, scale_rank_stride,
-                                        scale_token_stride, scale_hidden_stride, num_topk, num_ranks, num_experts, stream);
+nixl_amd_ep_ht_dispatch_rows(void *recv_x,
+                             void *recv_x_scales,
+                             int32_t *recv_topk_idx,
+                             float *recv_topk_weights,
+                             int32_t *recv_src_meta,
+                             const void *x,
+                             const void *x_scales,
+                             const int32_t *topk_idx,
+                             const float *topk_weights,
+                             const uint8_t *is_token_in_rank,
+                             const int *recv_gbl_rank_prefix_sum,
+                             const int *send_head,
+                             const int64_t *recv_row_offset,
+                             int64_t /*num_rows*/,
+                             int num_tokens,
+                             int hidden,
+                             int elem_bytes,
+                             int num_scales,
+                             int64_t scale_rank_stride,
+                             int64_t scale_token_stride,
+                             int64_t scale_hidden_stride,
+                             int num_topk,
+                             int num_ranks,
+                             int num_experts,
+                             void *stream) {
+    return nixl_amd_ep_ht_dispatch_scaled(recv_x, recv_x_scales, recv_topk_idx, recv_topk_weights, recv_src_meta, x, x_scales,
+                                          topk_idx, topk_weights, is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
+                                          recv_row_offset, num_tokens, hidden, elem_bytes, num_scales, scale_rank_stride,
+                                          scale_token_stride, scale_hidden_stride, num_topk, num_ranks, num_experts, stream);
 }
 
 int

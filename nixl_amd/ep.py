@@ -564,11 +564,11 @@ class Buffer:
                 raise EPError("x_scales must be a float32 or int32 tensor of shape [R, T, num_scales]")
             S = x_scales.shape[2]
 
-        def rows_kernel(recv_x, recv_scales, recv_idx, recv_w, recv_meta, idx, w, in_rank, prefix, send_head, row_offset, n, K, E):
+        def rows_kernel(recv_x, recv_scales, recv_idx, recv_w, recv_meta, idx, w, in_rank, prefix, send_head, row_offset, K, E):
             strides = x_scales.stride() if x_scales is not None else (0, 0, 0)
-            _check(self._k.nixl_amd_ep_ht_dispatch_rows(
+            _check(self._k.nixl_amd_ep_ht_dispatch_scaled(
                 _ptr(recv_x), _ptr(recv_scales), _ptr(recv_idx), _ptr(recv_w), _ptr(recv_meta), _ptr(x), _ptr(x_scales),
-                _ptr(idx), _ptr(w), _ptr(in_rank), _ptr(prefix), _ptr(send_head), _ptr(row_offset), n, T, H,
+                _ptr(idx), _ptr(w), _ptr(in_rank), _ptr(prefix), _ptr(send_head), _ptr(row_offset), T, H,
                 x.element_size(), S, strides[0], strides[1], strides[2], K, R, E, _stream()), "ht_dispatch")
 
         def with_scales(recv_x, recv_scales):
@@ -585,7 +585,7 @@ class Buffer:
             n_rows = recv_src_meta.shape[0]
             recv_x = torch.empty((n_rows, H), dtype=x.dtype, device=dev)
             recv_scales = torch.empty((n_rows, S), dtype=x_scales.dtype, device=dev) if x_scales is not None else None
-            rows_kernel(recv_x, recv_scales, None, None, None, None, None, in_rank, prefix, send_head, row_offset, n_rows, 0, R)
+            rows_kernel(recv_x, recv_scales, None, None, None, None, None, in_rank, prefix, send_head, row_offset, 0, R)
             return with_scales(recv_x, recv_scales), None, None, None, None, self._done(async_finish)
         if num_tokens_per_rank is None or is_token_in_rank is None or num_tokens_per_expert is None:
             raise EPError("ht_dispatch needs either a handle or the tensors of get_dispatch_layout")
@@ -624,7 +624,7 @@ class Buffer:
         recv_topk_weights = torch.empty((rows, K), dtype=torch.float32, device=dev) if K else None
         recv_src_meta = torch.empty((rows, 2), dtype=torch.int32, device=dev)
         rows_kernel(recv_x, recv_scales, recv_topk_idx, recv_topk_weights, recv_src_meta, topk_idx, topk_weights,
-                    is_token_in_rank, prefix, send_head, row_offset, -1 if ahead else rows, K, E)
+                    is_token_in_rank, prefix, send_head, row_offset, K, E)
         if ahead:
             total = self._wait_counts(mapped, R)
             recv_x, recv_src_meta = recv_x[:total], recv_src_meta[:total]

@@ -1565,3 +1565,36 @@ def test_ll_dispatch_of_wide_bf16_rows_with_few_selections(cuda, hidden, R, T, K
         rc, got = raw_ll_dispatch(cuda, x, topk, E, M, False)
         assert rc == 0, _lib.kernels_error()
         assert_dispatch_equal(got, want, False)
+
+
+def test_large_dispatch_to_few_ranks_takes_the_form_for_few_rows(cuda):
+    """Top-8 of experts that all lie on two of eight ranks gathers two rows a token, not the 5.3 of experts anywhere: a
+    dispatch that does not say how many rows there are must not be slower than one that does (1.27 times as long behind a
+    kernel on the input when the number was guessed from top-k)."""
+    R, T, H, K, E = 8, 4096, 7168, 8, 256
+    g = torch.Generator(device=cuda).manual_seed(5)
+    allowed = torch.zeros((R, T, R), dtype=torch.bool, device=cuda)
+    allowed.scatter_(2, torch.topk(torch.rand((R, T, R), generator=g, device=cuda), 2)[1], True)
+    scores = torch.rand((R, T, E), generator=g, device=cuda) + allowed.repeat_interleave(E // R, 2)
+    topk = torch.topk(scores, K)[1].to(torch.int32).contiguous()
+    x = torch.randn((R, T, H), generator=g, device=cuda).to(torch.bfloat16)
+    buf = Buffer(R, low_latency_mode=False, device=cuda)
+    per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk, E)
+    rows, _, _, _, handle, _ = buf.ht_dispatch(x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=per_expert,
+                                               topk_idx=topk, topk_weights=torch.ones((R, T, K), device=cuda))
+    in_rank, prefix, _, _, head, offset = handle
+    n, out, took = rows.shape[0], torch.empty_like(rows), {}
+    assert n <= 2 * R * T  # now and then all eight on one
+    for stated in (n, -1) * 12:
+        x.mul_(1.0)
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        rc = _lib.ep_kernels().nixl_amd_ep_ht_dispatch_rows(out.data_ptr(), None, None, None, None, x.data_ptr(), None, None, None, in_rank.data_ptr(),
+                                                            prefix.data_ptr(), head.data_ptr(), offset.data_ptr(), stated, T, H, 2, 0, 0, 0, 0, K, R, E,
+                                                            torch.cuda.current_stream().cuda_stream)
+        e1.record()
+        e1.synchronize()
+        assert rc == 0, _lib.kernels_error()
+        took.setdefault(stated, []).append(e0.elapsed_time(e1))
+    assert torch.equal(out, rows)
+    assert np.median(took[-1]) < 1.12 * np.median(took[n]), took
