@@ -137,7 +137,7 @@ def measure_ep_traffic_live():
     from nixl_amd import ep_bench
     child = [sys.executable, os.path.abspath(__file__), "--ep-traffic-child"]
     read_classes = {"TCC_EA0_RDREQ_128B_sum": 128, "TCC_EA0_RDREQ_64B_sum": 64, "TCC_EA0_RDREQ_32B_sum": 32}
-    tags = sorted({k for ks in ep_bench.CALL_KERNELS.values() for k in ks})
+    tags = sorted({k for calls in (ep_bench.CALL_KERNELS, ep_bench.CALL_KERNELS_IF_LAUNCHED) for ks in calls.values() for k in ks})
     got = {}
     for run, counters in (("read", list(read_classes)), ("write", ["WRITE_SIZE"])):
         out_dir, found = _counter_run(child, counters, timeout=200)
@@ -151,15 +151,25 @@ def measure_ep_traffic_live():
     if not got["write"][1]["WRITE_SIZE"]:
         return {"error": "the write counter shows nothing for the yardstick"}
     write_scale = (1 << 20) / got["write"][1]["WRITE_SIZE"]
+    return ep_call_traffic(got["read"][0], got["write"][0], read_classes, write_scale)
+
+
+def ep_call_traffic(read, written, read_classes, write_scale):
+    """Bytes of each expert-parallel call from the medians of its kernels ({kernel: {counter: value}}, reads and writes).
+    A kernel that some shapes do without counts where it has samples; a call without samples of one that it
+    cannot do without has no figure and says so, the others keep theirs."""
+    from nixl_amd import ep_bench
     out = {}
     for call, kernels in ep_bench.CALL_KERNELS.items():
+        missing = [k for k in kernels if k not in read or k not in written]
+        if missing:
+            out[call] = {"traffic": None, "traffic_live_error": f"no counter samples of {', '.join(missing)}"}
+            continue
+        also = [k for k in ep_bench.CALL_KERNELS_IF_LAUNCHED.get(call, ()) if k in read and k in written]
         per_kernel = {}
-        for k in kernels:
-            if k not in got["read"][0] or k not in got["write"][0]:
-                return {"error": f"no counter samples of {k}"}
-            read = sum(got["read"][0][k][c] * size for c, size in read_classes.items())
-            written = got["write"][0][k]["WRITE_SIZE"] * write_scale * 1024.0
-            per_kernel[k] = int(round(read + written))
+        for k in (*kernels, *also):
+            per_kernel[k] = int(round(sum(read[k][c] * size for c, size in read_classes.items()) +
+                                      written[k]["WRITE_SIZE"] * write_scale * 1024.0))
         out[call] = {"traffic": sum(per_kernel.values()), "traffic_by_kernel": per_kernel,
                      "traffic_source": "rocprofv3 --pmc over two child runs of this bench invocation (the four expert-parallel "
                                        "calls alone), median per launch summed over the call's kernels: reads = the L2's requests "

@@ -20,9 +20,11 @@ HBM_PEAK_GBPS = 8000.0
 CALL_KERNELS = {
     "ll_dispatch": ("ll_bits_kernel<false", "ll_dispatch_kernel<true", "ll_scales_kernel"),
     "ll_combine": ("ll_combine_kernel<false>",),
-    "ht_dispatch": ("ht_scan_packed_kernel", "ht_prefix_kernel", "ht_dispatch_kernel"),
+    "ht_dispatch": ("ht_scan_packed_kernel", "ht_dispatch_kernel"),
     "ht_combine": ("ht_combine_kernel",),
 }
+# Kernels that a call has at some sizes only: the receive-side counts share the scan's launch up to a number of tokens.
+CALL_KERNELS_IF_LAUNCHED = {"ht_dispatch": ("ht_prefix_kernel",)}
 
 
 def _timed(fn, flush, warmup, iters):

@@ -71,3 +71,38 @@ def test_counter_file_is_read_for_several_kernels_at_once(tmp_path):
             f.write(f'{i},"{k}","{c}",{v}\n')
     medians, yard = bench.counter_medians(str(path), ["A"], ["ll_bits_kernel<false", "ll_dispatch_kernel<true>", "ll_scales_kernel"])
     assert medians == {"ll_bits_kernel<false": {"A": 3.0}, "ll_dispatch_kernel<true>": {"A": 20.0}} and yard == {"A": 8.0}
+
+
+def test_a_kernel_that_is_not_launched_costs_no_call_its_traffic():
+    """The receive-side counts of normal mode share the scan's launch up to a number of tokens, so that their own kernel may have no
+    samples: every call keeps its figure, and a call that lacks one of its kernels is the only one without."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from nixl_amd import ep_bench
+    classes = {"A": 128, "B": 64}
+    names = {k for ks in ep_bench.CALL_KERNELS.values() for k in ks}
+    read = {k: {"A": 10.0, "B": 2.0} for k in names}
+    written = {k: {"WRITE_SIZE": 3.0} for k in names}
+    one = 10 * 128 + 2 * 64 + 3 * 1024 * 2
+    got = bench.ep_call_traffic(read, written, classes, 2.0)
+    assert {c: v["traffic"] for c, v in got.items()} == {c: one * len(ks) for c, ks in ep_bench.CALL_KERNELS.items()}
+    for side, value in ((read, {"A": 1.0, "B": 0.0}), (written, {"WRITE_SIZE": 1.0})):
+        side["ht_prefix_kernel"] = value
+    assert bench.ep_call_traffic(read, written, classes, 2.0)["ht_dispatch"]["traffic"] == 2 * one + 128 + 2048
+    del read["ll_scales_kernel"]
+    got = bench.ep_call_traffic(read, written, classes, 2.0)
+    assert got["ll_dispatch"]["traffic"] is None and "ll_scales_kernel" in got["ll_dispatch"]["traffic_live_error"]
+    assert got["ll_combine"]["traffic"] == one
+
+
+def test_the_kernels_whose_traffic_is_counted_exist():
+    """Every kernel that the traffic figures name is one of the sources' (a renamed one would have no samples), and no
+    name stands for two of a call's kernels."""
+    import re
+    from nixl_amd import ep_bench
+    kernels = os.path.join(ROOT, "nixl_amd", "csrc", "kernels")
+    defined = {name for f in os.listdir(kernels) if f.endswith(".hip")
+               for name in re.findall(r"^(\w+_kernel)\(", open(os.path.join(kernels, f)).read(), re.M)}
+    for calls in (ep_bench.CALL_KERNELS, ep_bench.CALL_KERNELS_IF_LAUNCHED):
+        for names in calls.values():
+            assert all(len([d for d in defined if name.split("<")[0] in d]) == 1 for name in names), names
