@@ -237,10 +237,8 @@ nixlHipEngine::~nixlHipEngine() {
 }
 
 hipStream_t
-nixlHipEngine::pickStream(int device) const {
-    if (useExternalStream_) return externalStream_;
-    const unsigned slot = nextStream_.fetch_add(1, std::memory_order_relaxed) % streamsPerDevice_;
-    const size_t idx = static_cast<size_t>(device) * streamsPerDevice_ + slot;
+nixlHipEngine::pickStream(int device, unsigned turn) const {
+    const size_t idx = static_cast<size_t>(device) * streamsPerDevice_ + turn % streamsPerDevice_;
     std::lock_guard<std::mutex> lock(streamsMutex_);
     if (!streams_[idx]) {
         // Default priority on purpose; non-blocking so that the legacy default stream
@@ -253,11 +251,25 @@ nixlHipEngine::pickStream(int device) const {
 
 bool
 nixlHipEngine::chooseStream(int device, nixlHipReqH &req, nixl_amd_copy_tuning_t &tuning) const {
-    if (!req.stream || req.device != device) req.stream = pickStream(device);
-    req.device = device;
     tuning = tuning_;
-    if (!useExternalStream_) tuning.stream = req.stream;
-    return req.stream || useExternalStream_;
+    if (useExternalStream_) {
+        req.stream = externalStream_;
+        req.device = device;
+        return true;
+    }
+    if (!req.stream || req.device != device) {
+        req.turn = nextStream_.fetch_add(1, std::memory_order_relaxed);
+        req.stream = pickStream(device, req.turn);
+    }
+    req.device = device;
+    tuning.stream = req.stream;
+    return req.stream != nullptr;
+}
+
+void
+nixlHipEngine::returnTurn(const nixlHipReqH &req) const {
+    unsigned behind = req.turn + 1;
+    if (!useExternalStream_) nextStream_.compare_exchange_strong(behind, req.turn, std::memory_order_relaxed);
 }
 
 nixl_amd_hip::WorkerPool *
@@ -744,9 +756,8 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
         }
     }
     if (device < 0) device = first_md->device;
-    // Whole chunks on 128-byte lines are what such plans are made of.  Decided here and not by
-    // the plan's refusal, so that a request which goes on to the descriptor path has taken no
-    // turn on the engine's streams yet.
+    // Whole chunks on 128-byte lines are what such plans are made of.  Decided here, before a buffer
+    // and a stream are taken.
     const uint64_t chunk = 1024u * static_cast<uint64_t>(std::max(tuning_.units_per_lane, 1));
     if ((address_bits & 127u) || len % chunk != 0) return NIXL_ERR_NOT_SUPPORTED;
 
@@ -760,6 +771,7 @@ nixlHipEngine::prepXferIndexed(const nixl_xfer_op_t &operation,
     const int rc = nixl_amd_copy_plan_create_indexed_lists(tables[src].data(), tables[src].size(), index_of[src], flat[src],
                                                            tables[dst].data(), tables[dst].size(), index_of[dst], flat[dst], count, len,
                                                            device, &tuning, &req->plan);
+    if (rc != NIXL_AMD_OK) returnTurn(*req);
     if (rc == NIXL_AMD_ERR_INDEX) {
         NIXL_ERROR << "HIP backend: index outside its prepared list";
         return NIXL_ERR_INVALID_PARAM;
@@ -836,6 +848,7 @@ nixlHipEngine::prepXferListed(const nixl_xfer_op_t &operation,
     if (nixl_amd_copy_plan_create_listed(write ? local : remote, write ? local_indices : remote_indices, write ? remote : local,
                                          write ? remote_indices : local_indices, count, &tuning, &continued,
                                          &req->plan) != NIXL_AMD_OK) {
+        returnTurn(*req);
         NIXL_DEBUG << "HIP backend: " << nixl_amd_last_error();
         return NIXL_ERR_NOT_SUPPORTED;
     }

@@ -74,6 +74,7 @@ class nixlHipReqH : public nixlBackendReqH {
 public:
     nixl_amd_copy_plan_t *plan = nullptr;
     hipStream_t stream = nullptr;
+    unsigned turn = 0; // that `stream` was taken in, if it is the engine's
     int device = 0;
     bool posted = false;
     size_t bytes = 0;
@@ -248,6 +249,10 @@ private:
     // application's is not named: the application may capture it).
     bool
     chooseStream(int device, nixlHipReqH &req, nixl_amd_copy_tuning_t &tuning) const;
+    // Of a request that came to nothing here and may come again as another: its turn is the next
+    // one's, unless some other request has taken one meanwhile.
+    void
+    returnTurn(const nixlHipReqH &req) const;
     // The two passes of prepXfer over a request's descriptor lists (hip_backend.cpp).
     struct blockPass {
         nixl_status_t status;
@@ -284,7 +289,7 @@ private:
                  int &device,
                  size_t &bytes) const;
     hipStream_t
-    pickStream(int device) const;
+    pickStream(int device, unsigned turn) const;
     void
     reapRetired(bool wait) const;
     bool

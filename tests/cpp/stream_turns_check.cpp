@@ -1,5 +1,6 @@
 // The HIP backend deals requests to its streams in turn: one turn a request, also for a request
-// that the indexed entry or the block plan declines and that goes on to the general lowering.
+// that the indexed entry or the block plan declines and that goes on to the general lowering, and
+// none for one that the indexed entry or the one for device-resident lists refuses.
 //
 // usage: stream_turns_check <path to libplugin_HIP.so>; prints "OK" and exits 0 on success.
 #include <dlfcn.h>
@@ -30,7 +31,12 @@ main(int argc, char **argv) {
     using indexed_fn = int (*)(nixlBackendEngine *, int, const nixlStrideDesc *, size_t, const int *, const nixlStrideDesc *, size_t,
                                const int *, size_t, const char *, nixlBackendReqH **);
     auto indexed = reinterpret_cast<indexed_fn>(dlsym(lib, "nixl_hip_prep_xfer_indexed"));
-    REQUIRE(init && indexed);
+    auto prep_list = reinterpret_cast<int (*)(nixlBackendEngine *, const nixlStrideDesc *, size_t, void **)>(dlsym(lib, "nixl_hip_prep_list"));
+    auto release_list = reinterpret_cast<void (*)(void *)>(dlsym(lib, "nixl_hip_release_list"));
+    using listed_fn = int (*)(nixlBackendEngine *, int, const void *, const int *, const void *, const int *, size_t, const char *, size_t *,
+                              size_t *, nixlBackendReqH **);
+    auto listed = reinterpret_cast<listed_fn>(dlsym(lib, "nixl_hip_prep_xfer_listed"));
+    REQUIRE(init && indexed && prep_list && release_list && listed);
     nixlBackendPlugin *plugin = init();
 
     constexpr unsigned n_streams = 3;
@@ -89,6 +95,44 @@ main(int argc, char **argv) {
                         REQUIRE(streams[i] != streams[j]);
                 }
             }
+
+    // Two lists on the device, the second with one entry that is longer: requests that name it are refused.
+    constexpr size_t entries = 1500, piece = 256;
+    const nixlStrideDesc plain(at, piece, 0, md, 2 * piece, entries);
+    nixlStrideDesc odd[2] = {nixlStrideDesc(at + room, piece, 0, md, 2 * piece, entries - 1),
+                             nixlStrideDesc(at + room + (entries - 1) * 2 * piece, 2 * piece, 0, md, 2 * piece, 1)};
+    odd[1].start_idx = entries - 1;
+    void *lists[2] = {nullptr, nullptr};
+    REQUIRE(prep_list(engine, &plain, 1, &lists[0]) == NIXL_SUCCESS && prep_list(engine, odd, 2, &lists[1]) == NIXL_SUCCESS);
+    std::vector<int> good(entries - 1), longer(entries), outside(blocks);
+    std::iota(good.begin(), good.end(), 0);
+    std::iota(longer.begin(), longer.end(), 0);
+    std::iota(outside.begin(), outside.end(), 1);
+    std::vector<hipStream_t> taken;
+    for (unsigned i = 0; i < 2 * n_streams; ++i) {
+        nixlBackendReqH *handle = nullptr;
+        size_t bytes = 0, merged = 0;
+        REQUIRE(listed(engine, NIXL_WRITE, lists[0], longer.data(), lists[1], longer.data(), entries, "turns", &bytes, &merged, &handle) ==
+                NIXL_ERR_NOT_SUPPORTED);
+        const nixlStrideDesc l(at, len, 0, md, len, blocks), r(at + room, len, 0, md, len, blocks);
+        REQUIRE(indexed(engine, NIXL_WRITE, &l, 1, outside.data(), &r, 1, index.data(), blocks, "turns", &handle) == NIXL_ERR_INVALID_PARAM);
+        if (i % 2) {
+            REQUIRE(listed(engine, NIXL_WRITE, lists[0], good.data(), lists[1], good.data(), entries - 1, "turns", &bytes, &merged, &handle) ==
+                    NIXL_SUCCESS);
+            REQUIRE(bytes == (entries - 1) * piece);
+        } else {
+            handle = request(0, blocks, true);
+        }
+        taken.push_back(static_cast<nixlHipReqH *>(handle)->stream);
+        REQUIRE(engine->releaseReqH(handle) == NIXL_SUCCESS);
+    }
+    for (unsigned i = 0; i < n_streams; ++i) {
+        REQUIRE(taken[i] && taken[i] == taken[i + n_streams]);
+        for (unsigned j = 0; j < i; ++j)
+            REQUIRE(taken[i] != taken[j]);
+    }
+    release_list(lists[0]);
+    release_list(lists[1]);
 
     REQUIRE(engine->deregisterMem(md) == NIXL_SUCCESS);
     plugin->destroy_engine(engine);
