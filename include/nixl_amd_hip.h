@@ -244,8 +244,9 @@ nixl_amd_copy_list_device(const nixl_amd_copy_list_t *list);
  * lengths) and writes the records; the call waits for its verdict and returns
  * NIXL_AMD_ERR_INVALID if a pair is bad.  `n_continued` (may be NULL) receives how many pairs
  * continue the pair before them on both sides: the descriptors an agent that merges
- * neighbours would not have listed (src/core/nixl_agent.cpp:799-857).  The kernel runs on the
- * stream that `tuning` names while that is idle (see there), else on one of the library's. */
+ * neighbours would not have listed (src/core/nixl_agent.cpp:799-857).  The kernel runs on a
+ * stream of the library's and has ended when the call returns; the stream that `tuning` names is
+ * not looked at, and the plan can be launched into any capture. */
 int
 nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
                                  const int32_t *src_index,
@@ -255,6 +256,18 @@ nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
                                  const nixl_amd_copy_tuning_t *tuning,
                                  size_t *n_continued,
                                  nixl_amd_copy_plan_t **out);
+
+/* The same for a caller that keeps to what is said of the stream that `tuning` names: while that is
+ * idle the kernel runs there, and the call waits for the verdict alone. */
+int
+nixl_amd_copy_plan_create_listed_on(const nixl_amd_copy_list_t *src,
+                                    const int32_t *src_index,
+                                    const nixl_amd_copy_list_t *dst,
+                                    const int32_t *dst_index,
+                                    size_t n,
+                                    const nixl_amd_copy_tuning_t *tuning,
+                                    size_t *n_continued,
+                                    nixl_amd_copy_plan_t **out);
 
 /* Enqueue the whole plan on `stream`: the per-post work of
  * nixlUcxEngine::postXfer -> sendXferRange (src/plugins/ucx/ucx_backend.cpp:1183-1310).

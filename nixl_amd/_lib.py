@@ -94,10 +94,11 @@ def kernels():
     lib.nixl_amd_copy_list_create.argtypes = [c_void_p, c_size_t, c_int, POINTER(c_void_p)]
     lib.nixl_amd_copy_list_destroy.argtypes = [c_void_p]
     lib.nixl_amd_copy_list_device.argtypes = [c_void_p]
-    lib.nixl_amd_copy_plan_create_listed.argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, POINTER(CopyTuning),
-                                                     POINTER(c_size_t), POINTER(c_void_p)]
+    for fn in ("nixl_amd_copy_plan_create_listed", "nixl_amd_copy_plan_create_listed_on"):
+        getattr(lib, fn).argtypes = [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, POINTER(CopyTuning), POINTER(c_size_t),
+                                     POINTER(c_void_p)]
     for fn in ("nixl_amd_copy_list_create", "nixl_amd_copy_list_destroy", "nixl_amd_copy_list_device",
-               "nixl_amd_copy_plan_create_listed", "nixl_amd_copy_records_begin", "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon",
+               "nixl_amd_copy_plan_create_listed", "nixl_amd_copy_plan_create_listed_on", "nixl_amd_copy_records_begin", "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon",
                "nixl_amd_copy_block_len_fits"):
         getattr(lib, fn).restype = c_int
     lib.nixl_amd_copy_plan_launch.argtypes = [c_void_p, c_void_p]
@@ -163,7 +164,7 @@ def kernel_symbols():
                    "nixl_amd_copy_plan_create_indexed_runs", "nixl_amd_copy_plan_create_indexed_lists", "nixl_amd_copy_records_begin",
                    "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon", "nixl_amd_copy_block_len_fits",
                    "nixl_amd_copy_list_create", "nixl_amd_copy_list_destroy", "nixl_amd_copy_list_device",
-                   "nixl_amd_copy_plan_create_listed",
+                   "nixl_amd_copy_plan_create_listed", "nixl_amd_copy_plan_create_listed_on",
                    "nixl_amd_copy_plan_launch", "nixl_amd_copy_plan_destroy", "nixl_amd_copy_plan_status",
                    "nixl_amd_copy_plan_query", "nixl_amd_copy_plan_time", "nixl_amd_ep_ll_workspace_bytes"] + list(_EP_SIGS))
 

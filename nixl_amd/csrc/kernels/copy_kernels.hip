@@ -2238,21 +2238,23 @@ nixl_amd_copy_list_device(const nixl_amd_copy_list_t *list) {
     return list ? list->device : nixl_amd_fail(NIXL_AMD_ERR_INVALID, "list_device: list is null");
 }
 
-int
-nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
-                                 const int32_t *src_index,
-                                 const nixl_amd_copy_list_t *dst,
-                                 const int32_t *dst_index,
-                                 size_t n,
-                                 const nixl_amd_copy_tuning_t *tuning,
-                                 size_t *n_continued,
-                                 nixl_amd_copy_plan_t **out) {
+static int
+create_listed(const nixl_amd_copy_list_t *src,
+              const int32_t *src_index,
+              const nixl_amd_copy_list_t *dst,
+              const int32_t *dst_index,
+              size_t n,
+              const nixl_amd_copy_tuning_t *tuning,
+              bool on_stream,
+              size_t *n_continued,
+              nixl_amd_copy_plan_t **out) {
     if (!out) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: out is null");
     *out = nullptr;
     if (!src || !dst || !src_index || !dst_index || n == 0) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: null argument");
     if (src->device != dst->device) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create_listed: lists on different devices");
     Tuning t;
     if (const int rc = parse_tuning(tuning, t, "plan_create_listed")) return rc;
+    if (!on_stream) t.stream = nullptr;
     // pieces a descriptor can have: its first line may hold back seven units of the first one
     const size_t max_units = std::min(src->max_len, dst->max_len) / 16u;
     const size_t per_desc = 1 + (max_units + 6) / kPieceUnits;
@@ -2322,10 +2324,12 @@ nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
     if (e == hipSuccess) e = await_verdict(*verdict, up);
     const ListVerdict got = *verdict;
     // The records are complete when the last kernel ends, which comes behind its verdict: a launch
-    // follows on the same stream, or it waits for the event.
+    // follows on the same stream, or waits for the event; a plan that may be launched anywhere, also into a
+    // capture, is complete when the caller has it.
     if (e == hipSuccess && !plan->reserved && !got.bad) {
         e = hipEventCreateWithFlags(&plan->uploaded, hipEventDisableTiming);
         if (e == hipSuccess) e = hipEventRecord(plan->uploaded, up);
+        if (e == hipSuccess && !on_stream) e = settle_upload(plan, true);
     }
     if ((e != hipSuccess || got.bad) && up) (void)hipStreamSynchronize(up); // whatever is queued uses the buffers given back below
     // the verdict is the last thing that is written there, and everything else has been read by then
@@ -2354,6 +2358,30 @@ nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
     if (n_continued) *n_continued = got.continued;
     *out = plan;
     return NIXL_AMD_OK;
+}
+
+int
+nixl_amd_copy_plan_create_listed(const nixl_amd_copy_list_t *src,
+                                 const int32_t *src_index,
+                                 const nixl_amd_copy_list_t *dst,
+                                 const int32_t *dst_index,
+                                 size_t n,
+                                 const nixl_amd_copy_tuning_t *tuning,
+                                 size_t *n_continued,
+                                 nixl_amd_copy_plan_t **out) {
+    return create_listed(src, src_index, dst, dst_index, n, tuning, false, n_continued, out);
+}
+
+int
+nixl_amd_copy_plan_create_listed_on(const nixl_amd_copy_list_t *src,
+                                    const int32_t *src_index,
+                                    const nixl_amd_copy_list_t *dst,
+                                    const int32_t *dst_index,
+                                    size_t n,
+                                    const nixl_amd_copy_tuning_t *tuning,
+                                    size_t *n_continued,
+                                    nixl_amd_copy_plan_t **out) {
+    return create_listed(src, src_index, dst, dst_index, n, tuning, true, n_continued, out);
 }
 
 int

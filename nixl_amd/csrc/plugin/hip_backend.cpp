@@ -845,9 +845,9 @@ nixlHipEngine::prepXferListed(const nixl_xfer_op_t &operation,
     nixl_amd_copy_tuning_t tuning;
     if (!chooseStream(nixl_amd_copy_list_device(local), *req, tuning)) return NIXL_ERR_BACKEND;
     size_t continued = 0;
-    if (nixl_amd_copy_plan_create_listed(write ? local : remote, write ? local_indices : remote_indices, write ? remote : local,
-                                         write ? remote_indices : local_indices, count, &tuning, &continued,
-                                         &req->plan) != NIXL_AMD_OK) {
+    if (nixl_amd_copy_plan_create_listed_on(write ? local : remote, write ? local_indices : remote_indices, write ? remote : local,
+                                            write ? remote_indices : local_indices, count, &tuning, &continued,
+                                            &req->plan) != NIXL_AMD_OK) {
         returnTurn(*req);
         NIXL_DEBUG << "HIP backend: " << nixl_amd_last_error();
         return NIXL_ERR_NOT_SUPPORTED;

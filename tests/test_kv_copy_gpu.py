@@ -1383,6 +1383,60 @@ def test_captured_launches_of_plans_that_name_a_stream(cuda, made):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("mode", ["global", "relaxed"])
+def test_captured_launch_of_a_listed_plan(cuda, mode):
+    """A plan of pairs from device-resident lists is complete when it is made, whatever stream its tuning names: its first launch may
+    go into a capture of that stream, and it can be destroyed while the stream is captured."""
+    import torch
+    n, slot = 3000, 512
+    rng = np.random.default_rng(9)
+    src = torch.randint(0, 256, (n, slot), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros_like(src)
+    lens = rng.choice([128, 256, 4 * 112], n).astype(np.uint32)
+    lib, stream = _lib.kernels(), torch.cuda.Stream()
+    lists = []
+    for t in (src, dst):
+        table = np.zeros(n, dtype=[("addr", "<u8"), ("len", "<u4"), ("continues", "<u4")])
+        table["addr"], table["len"] = t.data_ptr() + np.arange(n, dtype=np.uint64) * np.uint64(slot), lens
+        lists.append(ctypes.c_void_p())
+        assert lib.nixl_amd_copy_list_create(table.ctypes.data, n, 0, ctypes.byref(lists[-1])) == 0, _lib.kernels_error()
+    idx = rng.permutation(n).astype(np.int32)[:2500]
+
+    def make():
+        plan, tuning = ctypes.c_void_p(), _lib.CopyTuning(stream=stream.cuda_stream)
+        assert lib.nixl_amd_copy_plan_create_listed(lists[0], idx.ctypes.data, lists[1], idx.ctypes.data, idx.size, ctypes.byref(tuning), None,
+                                                    ctypes.byref(plan)) == 0, _lib.kernels_error()
+        return plan
+
+    torch.cuda.synchronize()
+    plan, dropped = make(), make()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        graph.capture_begin(capture_error_mode=mode)
+        try:
+            dst.zero_()
+            launched = lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream)
+            why = _lib.kernels_error()
+            destroyed = lib.nixl_amd_copy_plan_destroy(dropped)
+        finally:
+            graph.capture_end()
+    assert launched == 0 and destroyed == 0, why
+    taken = torch.zeros((n, slot), dtype=torch.bool)
+    for i in idx:
+        taken[int(i), :int(lens[i])] = True
+    taken = taken.to(cuda)
+    for _ in range(4):
+        src ^= 0x33
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(dst, torch.where(taken, src, torch.zeros_like(src)))
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+    for one in lists:
+        assert lib.nixl_amd_copy_list_destroy(one) == 0
+    torch.cuda.synchronize()
+
+
 def test_golden_descriptor_list(cuda):
     """Committed vector (tests/golden/kv_descs.npz): mixed aligned / unaligned / empty
     descriptors, destination pre-filled with a canary byte."""
