@@ -19,6 +19,19 @@ class nixlAgent {
 private:
     std::unique_ptr<nixlAgentData> data;
 
+    // makeXferReq over vectors that nobody changes meanwhile (`constant`), or that somebody may.
+    nixl_status_t
+    makeIndexedReq(const nixl_xfer_op_t &operation,
+                   const nixlDlistH *local_side,
+                   const int *local_indices,
+                   size_t local_count,
+                   const nixlDlistH *remote_side,
+                   const int *remote_indices,
+                   size_t remote_count,
+                   bool constant,
+                   nixlXferReqH *&req_hndl,
+                   const nixl_opt_args_t *extra_params) const;
+
 public:
     nixlAgent(const std::string &name, const nixlAgentConfig &cfg);
     ~nixlAgent();
@@ -67,7 +80,8 @@ public:
                 const std::vector<int> &remote_indices,
                 nixlXferReqH *&req_hndl,
                 const nixl_opt_args_t *extra_params = nullptr) const;
-    // The same with the indices where the caller keeps them (no reference counterpart).
+    // The same with the indices where the caller keeps them (no reference counterpart): they are
+    // read, maybe several times, until this returns.
     nixl_status_t
     makeXferReq(const nixl_xfer_op_t &operation,
                 const nixlDlistH *local_side,

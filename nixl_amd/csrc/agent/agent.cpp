@@ -752,11 +752,11 @@ namespace {
 // indices.size().  The scan has no early exit in its inner loop so that it vectorises; it is
 // the only place the index vectors are checked.
 size_t
-firstIndexOutside(const std::vector<int> &indices, size_t flat) {
+firstIndexOutside(const int *indices, size_t count, size_t flat) {
     constexpr size_t kBlock = 4096;
     const unsigned limit = flat > static_cast<size_t>(INT32_MAX) ? static_cast<unsigned>(INT32_MAX) + 1u : static_cast<unsigned>(flat);
-    for (size_t b0 = 0; b0 < indices.size(); b0 += kBlock) {
-        const size_t b1 = std::min(indices.size(), b0 + kBlock);
+    for (size_t b0 = 0; b0 < count; b0 += kBlock) {
+        const size_t b1 = std::min(count, b0 + kBlock);
         unsigned bad = 0;
         for (size_t i = b0; i < b1; ++i)
             bad |= static_cast<unsigned>(static_cast<unsigned>(indices[i]) >= limit); // a negative index wraps to a large one
@@ -764,7 +764,7 @@ firstIndexOutside(const std::vector<int> &indices, size_t flat) {
             for (size_t i = b0; i < b1; ++i)
                 if (static_cast<unsigned>(indices[i]) >= limit) return i;
     }
-    return indices.size();
+    return count;
 }
 
 // Walks a prepared list by flat index.  Consecutive look-ups usually stay inside one run or
@@ -848,19 +848,19 @@ commonBackend(const nixlDlistH &local_side, const nixlDlistH &remote_side, const
 nixl_status_t
 expandIndexPairs(const nixl_stride_dlist_t &lruns,
                  const nixl_stride_dlist_t &rruns,
-                 const std::vector<int> &local_indices,
-                 const std::vector<int> &remote_indices,
+                 const int *local_indices,
+                 const int *remote_indices,
+                 size_t count,
                  bool merge,
                  nixl_meta_dlist_t &initiator,
                  nixl_meta_dlist_t &target,
                  size_t &total_bytes) {
-    const size_t count = local_indices.size();
-    if (const size_t at = firstIndexOutside(local_indices, lruns.flatSize()); at != count) {
+    if (const size_t at = firstIndexOutside(local_indices, count, lruns.flatSize()); at != count) {
         NIXL_ERROR << "makeXferReq: local index " << local_indices[at] << " (position " << at << ") is outside its list of "
                    << lruns.flatSize() << " entries";
         return NIXL_ERR_INVALID_PARAM;
     }
-    if (const size_t at = firstIndexOutside(remote_indices, rruns.flatSize()); at != count) {
+    if (const size_t at = firstIndexOutside(remote_indices, count, rruns.flatSize()); at != count) {
         NIXL_ERROR << "makeXferReq: remote index " << remote_indices[at] << " (position " << at << ") is outside its list of "
                    << rruns.flatSize() << " entries";
         return NIXL_ERR_INVALID_PARAM;
@@ -869,7 +869,7 @@ expandIndexPairs(const nixl_stride_dlist_t &lruns,
     pool.adopt(initiator, count);
     pool.adopt(target, count);
     nixlMetaDesc *const lout = nixlDescStoragePool::data(initiator), *const rout = nixlDescStoragePool::data(target);
-    const int *const lidx = local_indices.data(), *const ridx = remote_indices.data();
+    const int *const lidx = local_indices, *const ridx = remote_indices;
     runCursor lcur(lruns), rcur(rruns);
     size_t made = 0;
     total_bytes = 0;
@@ -923,13 +923,10 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
                        const std::vector<int> &remote_indices,
                        nixlXferReqH *&req_hndl,
                        const nixl_opt_args_t *extra_params) const {
-    return makeXferReq(operation, local_side, local_indices.data(), local_indices.size(), remote_side, remote_indices.data(),
-                       remote_indices.size(), req_hndl, extra_params);
+    return makeIndexedReq(operation, local_side, local_indices.data(), local_indices.size(), remote_side, remote_indices.data(),
+                          remote_indices.size(), true, req_hndl, extra_params);
 }
 
-// reference: src/core/nixl_agent.cpp:696-887
-// A backend that takes index vectors reads every index once and checks what it has read; only the
-// expansion into descriptors, which looks at them twice, works on copies.
 nixl_status_t
 nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
                        const nixlDlistH *local_side,
@@ -940,6 +937,24 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
                        size_t remote_count,
                        nixlXferReqH *&req_hndl,
                        const nixl_opt_args_t *extra_params) const {
+    return makeIndexedReq(operation, local_side, local_indices, local_count, remote_side, remote_indices, remote_count, false,
+                          req_hndl, extra_params);
+}
+
+// reference: src/core/nixl_agent.cpp:696-887
+// A backend that takes index vectors checks what it uses, on a copy or on the device.  The expansion into
+// descriptors checks the vectors and then reads them again: vectors that may change meanwhile are copied for it.
+nixl_status_t
+nixlAgent::makeIndexedReq(const nixl_xfer_op_t &operation,
+                          const nixlDlistH *local_side,
+                          const int *local_indices,
+                          size_t local_count,
+                          const nixlDlistH *remote_side,
+                          const int *remote_indices,
+                          size_t remote_count,
+                          bool constant,
+                          nixlXferReqH *&req_hndl,
+                          const nixl_opt_args_t *extra_params) const {
     req_hndl = nullptr;
     if (!local_side || !remote_side) {
         NIXL_ERROR_FUNC << "local or remote side handle is null";
@@ -1029,8 +1044,13 @@ nixlAgent::makeXferReq(const nixl_xfer_op_t &operation,
     }
     size_t total = 0;
     const auto t_expand = std::chrono::steady_clock::now();
-    const nixl_status_t expanded = expandIndexPairs(lruns, rruns, std::vector<int>(local_indices, local_indices + count),
-                                                    std::vector<int>(remote_indices, remote_indices + count),
+    std::vector<int> copies[2];
+    if (!constant) {
+        copies[0].assign(local_indices, local_indices + count);
+        copies[1].assign(remote_indices, remote_indices + count);
+    }
+    const nixl_status_t expanded = expandIndexPairs(lruns, rruns, constant ? local_indices : copies[0].data(),
+                                                    constant ? remote_indices : copies[1].data(), count,
                                                     !(extra_params && extra_params->skipDescMerge), req->initiatorDescs,
                                                     req->targetDescs, total);
     if (expanded != NIXL_SUCCESS) return expanded;

@@ -321,6 +321,18 @@ def test_agents_used_from_several_threads(oracle_plugin_dir):
     assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
 
 
+def test_index_vectors_are_copied_only_where_they_may_change(oracle_plugin_dir):
+    """tests/cpp/index_vectors_check.cpp: requests by index that a backend takes as descriptors, from std::vectors
+    (read where they are) and from arrays that the caller keeps (copied first)."""
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = os.path.join(root, "tests", "cpp", "_build", "index_vectors_check")
+    if not os.path.exists(exe):
+        pytest.fail(f"{exe} missing: run __graft_entry__.build() first")
+    proc = subprocess.run([exe, oracle_plugin_dir], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
+
+
 def test_notification_ring_of_the_hip_backend_on_the_cpu():
     """tests/cpp/mailbox_check.cpp: the shared-memory ring that carries notifications between
     processes (nixl_amd/csrc/plugin/mailbox.h), fed by four threads and a child process at
