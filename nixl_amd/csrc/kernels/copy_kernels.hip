@@ -15,10 +15,9 @@
 //   no search, no LDS, few registers.  The end of a descriptor that is no whole number of
 //   chunks is one more chunk, which lies over the one before it.
 //   Tiny ones (below 256 B) are concatenated, in request order, into one virtual stream measured
-//   in 16-byte units and cut into such chunks, listed by chunk index in `mixed[]`; the mixed kernel
-//   stages the descriptors a chunk touches (span[m] = {first, last} for the m-th listed chunk; src[j],
-//   dst[j], prefix[j] = first unit of descriptor j, prefix[n] = total) in a per-wave LDS slice and
-//   walks them.
+//   in 16-byte units and cut into such chunks; the mixed kernel stages the descriptors a chunk
+//   touches (span[c] = {first, last}; src[j], dst[j], prefix[j] = first unit of descriptor j,
+//   prefix[n] = total) in a per-wave LDS slice and walks them.
 //   Descriptors that are not 16-byte aligned in src, dst and len are cut into byte-range
 //   work items of at most 4 KiB (16 of many long ones) handled by a third, byte-exact kernel; a
 //   long one whose source and destination lie alike inside their 128-byte lines is chunks as well,
@@ -66,8 +65,7 @@ struct MixedArgs {
     const uint64_t *src; // [n]
     const uint64_t *dst; // [n]
     const uint64_t *prefix; // [n + 1], units
-    const uint2 *span; // [n_mixed], {first desc, last desc} of the m-th mixed chunk
-    const uint32_t *chunks; // [n_mixed] chunk indices
+    const uint2 *span; // [n_mixed], {first desc, last desc} of a chunk
     uint64_t total_units;
     uint32_t n_mixed;
 };
@@ -260,12 +258,11 @@ copy_mixed_kernel(MixedArgs a) {
     const uint32_t n_waves = gridDim.x * kMixedWaves;
 
     for (uint32_t m = uniform(blockIdx.x * kMixedWaves + wave); m < a.n_mixed; m += n_waves) {
-        const uint32_t c = uniform(a.chunks[m]);
         const uint2 sp = a.span[m];
         const uint32_t j0 = uniform(sp.x);
         const uint32_t j1 = uniform(sp.y);
-        const uint64_t u0 = static_cast<uint64_t>(c) * kChunkUnits;
-        const uint64_t remaining = a.total_units - u0; // > 0: the host lists only real chunks
+        const uint64_t u0 = static_cast<uint64_t>(m) * kChunkUnits;
+        const uint64_t remaining = a.total_units - u0; // > 0
         const uint32_t n_units = remaining < kChunkUnits ? static_cast<uint32_t>(remaining) : kChunkUnits;
         const uint32_t nd = j1 - j0 + 1;
 
@@ -1761,7 +1758,6 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
 
     // The stream: descriptors shorter than a chunk.  Every chunk of it remembers the first and the
     // last descriptor that it touches.
-    std::vector<uint32_t> mixed(n_stream);
     std::vector<uint2> span(n_stream);
     for (size_t c = 0, j = 0; c < n_stream; ++c) {
         const uint64_t first = c * chunk_units, last = std::min(units, first + chunk_units) - 1;
@@ -1770,7 +1766,6 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         size_t jl = j;
         while (vprefix[jl + 1] <= last)
             ++jl;
-        mixed[c] = static_cast<uint32_t>(c);
         span[c] = make_uint2(static_cast<uint32_t>(j), static_cast<uint32_t>(jl));
     }
     // Runs of the same whole number of chunks share a record each; else every chunk gets its own,
@@ -1781,7 +1776,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
 
     // ---- one device arena for all plan arrays --------------------------------------
     auto align256 = [](size_t x) { return (x + 255) & ~size_t(255); };
-    const bool need_desc_arrays = !mixed.empty();
+    const bool need_desc_arrays = n_stream != 0;
     // The arena starts with the records the copy kernel reads.  When they are expanded on the
     // device, that stretch is not uploaded: the upload starts behind it, and the runs
     // travel at the arena's end.
@@ -1790,8 +1785,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     const size_t off_dst = off_src + (need_desc_arrays ? align256(nv * 8) : 0);
     const size_t off_prefix = off_dst + (need_desc_arrays ? align256(nv * 8) : 0);
     const size_t off_span = off_prefix + (need_desc_arrays ? align256((nv + 1) * 8) : 0);
-    const size_t off_mixed = off_span + (need_desc_arrays ? align256(span.size() * sizeof(uint2)) : 0);
-    const size_t off_pieces = off_mixed + align256(mixed.size() * sizeof(uint32_t));
+    const size_t off_pieces = off_span + (need_desc_arrays ? align256(span.size() * sizeof(uint2)) : 0);
     const size_t off_items = off_pieces + align256(pieces.n * sizeof(PieceRec));
     const size_t off_runs = off_items + align256(bytes.items.n * sizeof(GenericItem));
     const size_t total = off_runs + (expand ? align256(chunks.runs.size() * sizeof(ChunkRun)) : 0);
@@ -1847,7 +1841,6 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             std::memcpy(host(off_dst), vdst.data(), nv * 8);
             std::memcpy(host(off_prefix), vprefix.data(), (nv + 1) * 8);
             std::memcpy(host(off_span), span.data(), span.size() * sizeof(uint2));
-            std::memcpy(host(off_mixed), mixed.data(), mixed.size() * sizeof(uint32_t));
         }
         if (pieces.n) std::memcpy(host(off_pieces), pieces.at.get(), pieces.n * sizeof(PieceRec));
         if (bytes.items.n) std::memcpy(host(off_items), bytes.items.at.get(), bytes.items.n * sizeof(GenericItem));
@@ -1885,7 +1878,6 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         plan->mixed_args.dst = reinterpret_cast<const uint64_t *>(base + off_dst);
         plan->mixed_args.prefix = reinterpret_cast<const uint64_t *>(base + off_prefix);
         plan->mixed_args.span = reinterpret_cast<const uint2 *>(base + off_span);
-        plan->mixed_args.chunks = reinterpret_cast<const uint32_t *>(base + off_mixed);
         plan->piece_recs = reinterpret_cast<const PieceRec *>(base + off_pieces);
         plan->generic_items = reinterpret_cast<const GenericItem *>(base + off_items);
     }
@@ -1893,7 +1885,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->n_uniform = n_uniform_chunks;
     plan->chunks_per_rec = chunks_per_rec;
     plan->mixed_args.total_units = units;
-    plan->mixed_args.n_mixed = static_cast<uint32_t>(mixed.size());
+    plan->mixed_args.n_mixed = n_stream;
     plan->n_generic = static_cast<uint32_t>(bytes.items.n);
 
     auto wgs_for = [&](uint32_t n_waves, uint32_t waves_per_wg, bool cap) {
