@@ -90,10 +90,13 @@ struct GenericItem {
 };
 
 // 16-byte vector in the global address space, so that accesses compile to
-// global_load/store_dwordx4 rather than flat instructions.
+// global_load/store_dwordx4 rather than flat instructions.  Nothing is said of its alignment: the
+// first and last chunks of odd tensors and the items of the byte path start anywhere.  The
+// hardware takes such addresses, and aligned ones compile to the same instructions.
 using v4u = __attribute__((__vector_size__(4 * sizeof(unsigned)))) unsigned;
-using gv4_ptr = __attribute__((address_space(1))) v4u *;
-using gv4_cptr = const __attribute__((address_space(1))) v4u *;
+using v4u_any = __attribute__((__vector_size__(4 * sizeof(unsigned)), __aligned__(1))) unsigned;
+using gv4_ptr = __attribute__((address_space(1))) v4u_any *;
+using gv4_cptr = const __attribute__((address_space(1))) v4u_any *;
 
 // Cache policy of a plan's loads and stores (tuning field `nontemporal`), measured on MI355X
 // with 16 KiB blocks (TB/s of traffic; sequential = consecutive descriptors adjoin):
@@ -334,11 +337,8 @@ copy_mixed_kernel(MixedArgs a) {
 // number of waves sharing it, not bytes (3000 descriptors of up to 64 KiB, 18 MB: 7 us; with items
 // of 16 KiB whose lanes had one load in flight a 64 KiB descriptor alone was 64 of those trips
 // in a row on four waves).
-using v4u_any = __attribute__((__vector_size__(4 * sizeof(unsigned)), __aligned__(1))) unsigned;
-
 __global__ void __launch_bounds__(kMixedThreads)
 copy_generic_kernel(const GenericItem *items, uint32_t n_items) {
-    using any_cptr = const __attribute__((address_space(1))) v4u_any *;
     using byte_ptr = __attribute__((address_space(1))) uint8_t *;
     using byte_cptr = const __attribute__((address_space(1))) uint8_t *;
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
@@ -368,7 +368,7 @@ copy_generic_kernel(const GenericItem *items, uint32_t n_items) {
             for (int k = 0; k < kGenericLoads; ++k) {
                 const uint32_t at = round + k * kWaveSize + lane;
                 const uint32_t u = min(at < shift ? 0u : at - shift, body - 1);
-                v[k] = *(any_cptr)(src + head + u * 16ull);
+                v[k] = *(gv4_cptr)(src + head + u * 16ull);
             }
 #pragma unroll
             for (int k = 0; k < kGenericLoads; ++k) {
