@@ -45,10 +45,18 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
-def _stream():
-    """The handle of the current device's current stream: 0.1 us, where building the Stream object of
-    torch.cuda.current_stream() takes 2.9 (a small dispatch and combine together: 35 us)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+def _stream_getter():
+    """A function that gives the handle of the current device's current stream.  Building the Stream object of
+    torch.cuda.current_stream() takes 2.9 us (a small dispatch and combine together: 35), asking for the handle 0.1;
+    a torch without the names that this needs, which are not public, builds the object."""
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    handle = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if device is None or handle is None:
+        return lambda: torch.cuda.current_stream().cuda_stream
+    return lambda: handle(device())
+
+
+_stream = _stream_getter()
 
 
 def _check(rc, what):

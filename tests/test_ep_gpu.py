@@ -1598,3 +1598,13 @@ def test_large_dispatch_to_few_ranks_takes_the_form_for_few_rows(cuda):
         took.setdefault(stated, []).append(e0.elapsed_time(e1))
     assert torch.equal(out, rows)
     assert np.median(took[-1]) < 1.12 * np.median(took[n]), took
+
+
+def test_launches_go_to_the_current_stream(cuda):
+    """The stream handle that launches are given is that of torch's current stream, on the default stream and on others."""
+    from nixl_amd import ep
+    assert ep._stream() == torch.cuda.current_stream().cuda_stream
+    for _ in range(2):
+        with torch.cuda.stream(torch.cuda.Stream()) as _, torch.cuda.device(cuda):
+            assert ep._stream() == torch.cuda.current_stream().cuda_stream != 0
+    assert ep._stream() == torch.cuda.current_stream().cuda_stream

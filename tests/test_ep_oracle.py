@@ -600,3 +600,18 @@ def test_normal_mode_config_shims():
         assert ep.Config(24, 6, 256, 6, 128).chunk_sizes == (6, 256, 6, 128)
     finally:
         ep.Buffer.set_num_sms(20)
+
+
+@pytest.mark.parametrize("missing", [None, "_cuda_getDevice", "_cuda_getCurrentRawStream"])
+def test_stream_handle_with_and_without_torchs_private_names(monkeypatch, missing):
+    """A launch's stream handle comes from two functions of torch that are not public; without one of them from the
+    public Stream object."""
+    import types
+    import torch
+    from nixl_amd import ep
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 3, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 1000 + device, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    if missing:
+        monkeypatch.delattr(torch._C, missing)
+    assert ep._stream_getter()() == (77 if missing else 1003)
