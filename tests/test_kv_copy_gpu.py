@@ -1172,11 +1172,18 @@ def test_index_vectors_read_once(cuda, n, consecutive, n_runs):
         agent.close()
 
 
-@pytest.mark.parametrize("cut", ["block", "at_1024", "one", "mixed", "short"])
+def _sent_as_runs(idx):
+    """Whether pairs (i, i) of these indices are sent as runs: stretches of 4096 pairs, at most one run for every eight pairs so far."""
+    breaks = np.concatenate([[True], np.diff(idx) != 1])
+    n_runs = np.cumsum(breaks)
+    return all(n_runs[min(i + 64, idx.size) - 1] <= min(idx.size, (i // 4096 + 1) * 4096) // 8 + 1 for i in range(0, idx.size, 64))
+
+
+@pytest.mark.parametrize("cut", ["block", "at_1024", "one", "mixed", "crowded", "short", "short_in_slices"])
 def test_listed_requests_of_consecutive_entries(cuda, cut):
     """Index pairs that advance by one on both sides, cut into runs of 64, at and around the 1024
-    pairs of a workgroup, not at all, of any length, and so short that the vectors are sent as they
-    are: every byte against the per-descriptor oracle, the descriptors that neighbours merge into
+    pairs of a workgroup, not at all, of any length, so that a workgroup has a run for every pair, and so short that the vectors are sent as they
+    are, in one launch and in two: every byte against the per-descriptor oracle, the descriptors that neighbours merge into
     counted; a run that leaves its list or meets other lengths on its way is refused."""
     import torch
     from nixl_amd.agent import NixlError
@@ -1187,11 +1194,14 @@ def test_listed_requests_of_consecutive_entries(cuda, cut):
     starts = np.concatenate([[0], np.cumsum(lens)])[:-1] + np.repeat(np.arange(n_runs) * 48, per)
     half = int(starts[-1] + lens[-1] + 4096) // 128 * 128 + 128
     so, do = starts, half + starts + 32
-    pairs = {"block": [(64 * i, 64) for i in rng.permutation(n // 64)], "one": [(5, n - 9)],
-             "at_1024": [(0, 1024), (2048, 1023), (6000, 1025), (9000, 1), (10240, 1023), (12000, 1024), (4096, 17)],
-             "mixed": [(int(a), int(b)) for a, b in zip(np.sort(rng.choice(n // 512, 24, replace=False)) * 512, rng.integers(17, 512, 24))],
-             "short": [(12 * i, 12) for i in rng.permutation(n // 12)[:400]]}[cut]
+    pairs = {"block": lambda: [(64 * i, 64) for i in rng.permutation(n // 64)], "one": lambda: [(5, n - 9)],
+             "at_1024": lambda: [(0, 1024), (2048, 1023), (6000, 1025), (9000, 1), (10240, 1023), (12000, 1024), (4096, 17)],
+             "mixed": lambda: [(int(a), int(b)) for a, b in zip(np.sort(rng.choice(n // 512, 24, replace=False)) * 512, rng.integers(17, 512, 24))],
+             "crowded": lambda: [(0, 9216)] + [(11262 - 2 * i, 1) for i in range(1024)] + [(12000, 1100)],
+             "short": lambda: [(7 * i, 3 + i % 5) for i in rng.permutation(n // 7)[:1000]],
+             "short_in_slices": lambda: [(7 * i, 3 + i % 5) for _ in range(8) for i in rng.permutation(n // 7)[:1900]]}[cut]()
     idx = np.concatenate([np.arange(a, a + b) for a, b in pairs]).astype(np.int32)
+    assert _sent_as_runs(idx) == (not cut.startswith("short")) and (idx.size > 65536 + 1024) == (cut == "short_in_slices")
     host = rng.integers(0, 256, 2 * half, dtype=np.uint8)
     mem = torch.from_numpy(host.copy()).to(cuda)
     torch.cuda.synchronize()
