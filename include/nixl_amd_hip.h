@@ -297,10 +297,11 @@ int
 nixl_amd_copy_plan_destroy(nixl_amd_copy_plan_t *plan);
 
 /* Plan facts: total payload bytes, descriptors on the 128-bit paths, descriptors on the
- * byte path, device bytes held by the plan's own arrays, and how the 128-bit work was cut:
- * chunks of the packed stream lying inside one descriptor (uniform) versus chunks crossing
- * descriptor boundaries (mixed), and pieces (one wavefront each) of the descriptors that are
- * short or do not start on a 128-byte line. */
+ * byte path, device bytes held by the plan's own arrays, and how the 128-bit work was cut: all
+ * chunks (vec), the whole ones among them, each a part of one descriptor (uniform), the ends of
+ * aligned descriptors that are no whole number of chunks and the chunks that several tiny
+ * descriptors share (mixed; the two ends of a long odd descriptor are in vec alone), and pieces (one wavefront
+ * each) of the descriptors that are short or do not start on a 128-byte line. */
 typedef struct nixl_amd_copy_plan_info {
     uint64_t payload_bytes;
     uint64_t vec_descs;

@@ -13,7 +13,7 @@
 //   dst address} in `uniform[]`; the uniform kernel reads its record with one scalar load and
 //   issues UPL 128-bit loads and UPL 128-bit stores per lane with wave-uniform base addresses —
 //   no search, no LDS, few registers.  The end of a descriptor that is no whole number of
-//   chunks is one more chunk, which lies over the one before it.
+//   chunks is one more, of as many units as it needs (their number rides in the record's top bytes).
 //   Tiny ones (below 256 B) are concatenated, in request order, into one virtual stream measured
 //   in 16-byte units and cut into such chunks; the mixed kernel stages the descriptors a chunk
 //   touches (span[c] = {first, last}; src[j], dst[j], prefix[j] = first unit of descriptor j,
@@ -60,6 +60,21 @@ struct UniformRec {
     uint64_t src;
     uint64_t dst;
 };
+
+// The record of a chunk that is not whole, the end of a descriptor: its 16-byte units, less one, in the top
+// bytes of the two addresses, and the sign of dst, by which it is known.
+constexpr uint64_t kEndAddress = (1ull << 56) - 1;
+
+__device__ __forceinline__ UniformRec
+end_rec(uint64_t src, uint64_t dst, uint32_t units) {
+    const uint64_t more = units - 1; // < 1024
+    return UniformRec{src | more >> 7 << 56, dst | more << 57 >> 1 | 1ull << 63};
+}
+
+__device__ __forceinline__ uint32_t
+end_units(uint64_t src, uint64_t dst) {
+    return (static_cast<uint32_t>(src >> 56) << 7 | (static_cast<uint32_t>(dst >> 56) & 127u)) + 1u;
+}
 
 struct MixedArgs {
     const uint64_t *src; // [n]
@@ -166,6 +181,16 @@ copy_uniform_kernel(const UniformRec *recs, uint32_t first_chunk, uint32_t n_chu
     const uint64_t s = words[0] + off; // UniformRec::src
     const uint64_t d = words[1] + off; // UniformRec::dst
     v4u v[UPL];
+    if (static_cast<int64_t>(words[1]) < 0) {
+        const uint32_t units = end_units(words[0], words[1]);
+#pragma unroll
+        for (int k = 0; k < UPL; ++k)
+            if (k * kWaveSize + lane < units) v[k] = load16<POL>((s & kEndAddress) + k * (kWaveSize * 16u));
+#pragma unroll
+        for (int k = 0; k < UPL; ++k)
+            if (k * kWaveSize + lane < units) store16<POL>((d & kEndAddress) + k * (kWaveSize * 16u), v[k]);
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < UPL; ++k)
         v[k] = load16<POL>(s + k * (kWaveSize * 16u));
@@ -694,16 +719,15 @@ clear_totals_kernel(ListTotals *totals) {
 }
 
 // A long descriptor as chunks of its own: chunk k starts k chunks behind the place `back` bytes in
-// front of the descriptor, but not before the descriptor and not so late that it would reach
-// beyond it.  With a whole number of chunks and back = 0 that is all there is to it; else the last chunk
-// (and, with a `back` that puts the others on the destination's lines, the first) lies partly over
-// its neighbour, and both write the same bytes there.  So every chunk is whole and belongs to one
-// descriptor, whatever the length, and no descriptor moves another one's chunks off the lines.
-// Cut from one stream of all descriptors, chunks behind one that is no whole number of them started
-// anywhere in a line and those on a border were put together by another kernel: 40 tensors of 1 to
-// 128 MiB in multiples of 16 bytes 393 us, 348 so; 512 of 2 MiB + 16 B to 48 B 397 and 315; 64 of 1 MiB + 16 to 48 B
-// 31.2 and 24.1; 64 165 descriptors of 8 to 64 KiB in multiples of 16 bytes 897 and 805.  Odd tensors, whose ends
-// the byte kernel moved, 358 and 348.  On the grid of whole KiB of the destination they are no faster (351).
+// front of the descriptor.  With a whole number of chunks and back = 0 that is all there is to it; else the
+// last chunk (and, with a `back` that puts the others on the destination's lines, the first) is an end, of as many
+// 16-byte units as its bytes need: less than a unit of it lies over its neighbour, where both write the
+// same bytes (or all that is missing from a chunk, where an address leaves no room for the number of units).  So every chunk belongs to one descriptor, whatever the length, and no descriptor
+// moves another one's chunks off the lines.
+// Cut from one stream of all descriptors, with a whole chunk over its neighbour at each end, and so, us: 512 tensors of 2 MiB + 16 B
+// to 48 B 397, 315 and 314; 60 000 descriptors of 8 to 64 KiB in multiples of 16 bytes, shuffled, 1000, 844 and 838; 65 536 of 8 KiB + 128 B 195, 206
+// and 185; at 16 units a lane 32 768 of 16 KiB + 16 B 253, 412 and 217.  Odd tensors, whose ends the byte kernel moved once,
+// 358, 348 and 348.
 struct ChunkRun {
     uint64_t src, dst, len; // len >= a chunk
     uint32_t first; // chunk of the plan that the run starts with
@@ -714,7 +738,7 @@ struct ChunkRun {
 // table stays in the L2), so that one long run among short ones costs no more than any other;
 // 32 bytes per run cross the bus instead of 16 per chunk.
 __global__ void __launch_bounds__(256)
-expand_runs_kernel(UniformRec *recs, const ChunkRun *runs, uint32_t n_runs, uint32_t n_chunks, uint32_t chunk_bytes) {
+expand_runs_kernel(UniformRec *recs, const ChunkRun *runs, uint32_t n_runs, uint32_t n_chunks, uint32_t chunk_bytes, int ends) {
     for (uint64_t c64 = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; c64 < n_chunks;
          c64 += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
         const uint32_t c = static_cast<uint32_t>(c64);
@@ -726,8 +750,17 @@ expand_runs_kernel(UniformRec *recs, const ChunkRun *runs, uint32_t n_runs, uint
         }
         const ChunkRun run = runs[lo];
         const uint64_t at = static_cast<uint64_t>(c - run.first) * chunk_bytes;
-        const uint64_t off = min(at > run.back ? at - run.back : 0, run.len - chunk_bytes);
-        recs[c] = UniformRec{run.src + off, run.dst + off};
+        const uint64_t left = run.len + run.back - at; // of the run, from this chunk on
+        if (ends && left < chunk_bytes) {
+            const uint32_t units = static_cast<uint32_t>(left + 15u) / 16u;
+            const uint64_t off = run.len - units * 16u;
+            recs[c] = end_rec(run.src + off, run.dst + off, units);
+        } else if (ends && at < run.back) {
+            recs[c] = end_rec(run.src, run.dst, (chunk_bytes - run.back + 15u) / 16u);
+        } else {
+            const uint64_t off = min(at > run.back ? at - run.back : 0, run.len - chunk_bytes);
+            recs[c] = UniformRec{run.src + off, run.dst + off};
+        }
     }
 }
 
@@ -1415,13 +1448,15 @@ struct LongDescs {
 
     const uint64_t chunk_bytes;
     std::vector<ChunkRun> runs;
-    uint64_t n = 0, edges = 0; // chunks, and how many of them lie over their neighbours
-    bool equal = true; // as many chunks in every run, none of them over another
+    uint64_t n = 0, edges = 0; // chunks, and how many of them are ends
+    bool equal = true; // as many chunks in every run, none of them an end
+    uint64_t address_bits = 0;
 
     // len >= chunk_bytes > back, and len + back > chunk_bytes if there is a back
     void
     add(uint64_t src, uint64_t dst, uint64_t len, uint64_t back) {
         const uint64_t reach = len + back;
+        address_bits |= (src + len) | (dst + len);
         equal = equal && reach % chunk_bytes == 0 && back == 0 && (runs.empty() || runs[0].len == len);
         edges += static_cast<uint64_t>(back != 0) + static_cast<uint64_t>(reach % chunk_bytes != 0);
         runs.push_back(ChunkRun{src, dst, len, static_cast<uint32_t>(n), static_cast<uint32_t>(back)});
@@ -1732,8 +1767,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     }
     payload += bytes.payload;
     // A long byte descriptor whose two ends lie at the same place inside their lines (tensors whose
-    // size is no multiple of 16) is chunks but for its two ends, and those are chunks as well that lie
-    // over their neighbours (their lanes' 16 bytes start anywhere).  Without chunks of other
+    // size is no multiple of 16) is chunks, the first and the last of them ends (whose lanes' 16 bytes
+    // start anywhere).  Without chunks of other
     // descriptors and up to kSplitFromTotal (both sides in the 256 MB last-level cache) the byte kernel
     // is as fast or faster: 32 tensors of 1 MiB + 2 B 12.3 us instead of 15.0, 128 of them 36.9 and
     // 45.4; 256 of them 90 us and a plan that takes 25 us to make, instead of 84 and 9.
@@ -1859,7 +1894,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             const uint32_t wgs = static_cast<uint32_t>(std::min<uint64_t>((static_cast<uint64_t>(n_uniform_chunks) + 255) / 256, 1u << 20));
             hipLaunchKernelGGL(expand_runs_kernel, dim3(wgs), dim3(256), 0, up, reinterpret_cast<UniformRec *>(arena + off_uni),
                                reinterpret_cast<const ChunkRun *>(arena + off_runs), static_cast<uint32_t>(chunks.runs.size()),
-                               n_uniform_chunks, static_cast<uint32_t>(chunk_bytes));
+                               n_uniform_chunks, static_cast<uint32_t>(chunk_bytes),
+                               static_cast<int>((chunks.address_bits >> kPieceUnitsShift) == 0));
             e = hipGetLastError();
         }
         if (e == hipSuccess) e = end_build(plan, up, staging, staging_cap);
@@ -1903,7 +1939,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->info.generic_descs = bytes.n;
     plan->info.plan_device_bytes = plan->arena_bytes;
     plan->info.vec_chunks = n_stream + n_uniform_chunks;
-    // chunks that are their descriptor's alone, and those in which something else is written as well
+    // whole chunks, and the ends of aligned descriptors and the chunks of tiny ones
     plan->info.uniform_chunks = static_cast<uint32_t>(chunks.n - chunks.edges);
     plan->info.mixed_chunks = n_stream + static_cast<uint32_t>(n_aligned_edges);
     plan->info.generic_items = plan->n_generic;
