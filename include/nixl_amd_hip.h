@@ -144,7 +144,8 @@ nixl_amd_copy_plan_create_indexed_runs(const nixl_amd_copy_run_t *src_runs,
 
 /* The same for a caller that has not looked at the indices: the two lists have src_entries and
  * dst_entries entries, and an index outside its list is refused (NIXL_AMD_ERR_INDEX).  The
- * arrays are read once, bounds and patterns are found out on the copy that the device reads. */
+ * arrays may be read several times; what is checked is what is used (a copy that the device reads,
+ * or of consecutive indices the first), whatever becomes of them meanwhile. */
 int
 nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
                                         size_t n_src_runs,

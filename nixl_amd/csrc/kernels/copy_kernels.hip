@@ -724,10 +724,10 @@ clear_totals_kernel(ListTotals *totals) {
 // 16-byte units as its bytes need: less than a unit of it lies over its neighbour, where both write the
 // same bytes (or all that is missing from a chunk, where an address leaves no room for the number of units).  So every chunk belongs to one descriptor, whatever the length, and no descriptor
 // moves another one's chunks off the lines.
-// Cut from one stream of all descriptors, with a whole chunk over its neighbour at each end, and so, us: 512 tensors of 2 MiB + 16 B
-// to 48 B 397, 315 and 314; 60 000 descriptors of 8 to 64 KiB in multiples of 16 bytes, shuffled, 1000, 844 and 838; 65 536 of 8 KiB + 128 B 195, 206
-// and 185; at 16 units a lane 32 768 of 16 KiB + 16 B 253, 412 and 217.  Odd tensors, whose ends the byte kernel moved once,
-// 358, 348 and 348.
+// Cut from one stream of all descriptors, with a whole chunk over its neighbour at each end, and so,
+// us: 512 tensors of 2 MiB + 16 B 372, 330 and 328; 60 000 descriptors of 8 to 64 KiB in multiples
+// of 16 bytes, shuffled, 1000, 844 and 838; 65 536 of 8 KiB + 128 B 195, 206 and 185; at 16 units a
+// lane 32 768 of 16 KiB + 16 B 253, 412 and 217.
 struct ChunkRun {
     uint64_t src, dst, len; // len >= a chunk
     uint32_t first; // chunk of the plan that the run starts with
@@ -1767,11 +1767,12 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     }
     payload += bytes.payload;
     // A long byte descriptor whose two ends lie at the same place inside their lines (tensors whose
-    // size is no multiple of 16) is chunks, the first and the last of them ends (whose lanes' 16 bytes
-    // start anywhere).  Without chunks of other
-    // descriptors and up to kSplitFromTotal (both sides in the 256 MB last-level cache) the byte kernel
-    // is as fast or faster: 32 tensors of 1 MiB + 2 B 12.3 us instead of 15.0, 128 of them 36.9 and
-    // 45.4; 256 of them 90 us and a plan that takes 25 us to make, instead of 84 and 9.
+    // size is no multiple of 16) is chunks, the first and the last of them ends (whose lanes' 16
+    // bytes start anywhere).  Alone and up to kSplitFromTotal the byte kernel has the shorter way: its
+    // items are fewer than the chunks' records and need no kernel to write them.  Made, launched and
+    // waited for, by the byte kernel and as chunks, us: 15 tensors of 1 MiB + 2 B 21.2 and 24.0, 15 of 4 MiB
+    // + 6 B 38.0 and 40.9, 126 of 1 MiB + 2 B 63.7 and 60.9, 2031 of 64 KiB + 2 B 74.9 and 76.7; 255 of 1 MiB + 2 B 114 and
+    // 101, 4 of 120 MiB 233 and 174.
     const bool join = whole_chunks || bytes.splittable_total >= kSplitFromTotal;
     if (bytes.long_total - (join ? bytes.splittable_total : 0) > kLongItemsFrom) bytes.reach = kGenericItemBytes;
     const size_t n_aligned_runs = chunks.runs.size(), n_aligned_edges = chunks.edges;

@@ -305,15 +305,13 @@ ht_prefix_kernel(const int *__restrict__ channel_prefix, HtNotifyOut o, int R, i
 }
 
 // The same without a launch of its own, for up to 8 ranks: one more workgroup behind those of the
-// scan counts the flags itself instead of waiting for their counts.  What bounds it is one workgroup's
-// way to flags that another kernel has just written, so every wave has a share of a rank's tokens, eight
-// loads in flight a lane, and counts bytes (eight destinations an addition) that are widened once a
-// step.  Layout, scan and this behind one another, us, against two launches (and the first form, which
-// counted 16-bit fields with half of the waves, up to 32 768 flags): 4 x 333 tokens 8.6 and 11.6 (10.1), 8 x 256 7.9 and
-// 11.1 (9.3), 8 x 512 10.0 and 13.3 (13.0), 8 x 1024 9.6 and 12.7, 8 x 2048 12.1 and 14.8, 8 x 4096 15.0 and 16.0, 8 x 6000
-// 17.5 and 17.3, 8 x 8192 20.0 and 18.6; 4 x 4096 13.1 and 15.7, 4 x 16 384 19.3 and 22.0.  Where a token's flags are
-// no word that one load takes, the line lies lower: 6 x 300 11.5 and 11.6, 6 x 600 14.0 and 12.5, 7 x 400 13.5 and 11.8, 2 x 3000 13.7
-// and 14.2, 2 x 4500 16.2 and 15.5, 1 x 4000 11.2 and 14.1.
+// scan counts the flags itself instead of waiting for their counts.  What bounds it is one
+// workgroup's way to flags that another kernel has just written, so every wave has a share of a
+// rank's tokens, eight loads in flight a lane, and counts bytes (eight destinations an addition)
+// that are widened once a step.  Up to so many tokens that the one workgroup is not slower than the
+// launch (layout, scan and this behind one another, one launch and two, us): 8 x 1024 tokens 9.6 and
+// 12.7, 8 x 4096 15.0 and 16.0, 8 x 6000 17.5 and 17.3; 4 x 16 384 19.3 and 22.0.  Where a token's
+// flags are no word that one load takes: 6 x 300 11.5 and 11.6, 6 x 600 14.0 and 12.5.
 constexpr int kNotifyTokensOf8 = 40960, kNotifyTokensOf4 = 65536; // R * T
 constexpr int kNotifyFlags = 12288; // R * T * R, other numbers of ranks
 constexpr int kNotifyPerLane = 8; // tokens a lane counts at a time, their loads together
@@ -553,21 +551,17 @@ next_row(const WaveRows &w, unsigned long long &hits) {
 // every row of the token.  Bound by the writes, which carry device scope.  Inputs of more than
 // kHtStreamFrom (half the last-level cache) are loaded non-temporally, smaller ones ordinarily:
 // what a large call loads pushes lines out of the cache that the kernel which made the input left
-// there.  8 x 4096 x 7168 bf16 with combine, one pass after another, us a pass with ordinary and with
-// non-temporal loads (and with non-temporal stores as well, before rows and metadata shared a
-// launch): an element-wise kernel on the input in front of every pass 1159 and 1106 (1116), one
-// that writes it from another tensor 1128 and 1118 (1131), a 512 MB fill 1103 and 1068 (1075), nothing
-// 957 and 979 (1012).  Dispatch alone behind the fill 568 and 525 (513), of fp8 rows with scales 305 and
-// 277 (289).  8 x 1024 x 4096 (67 MB) is the same either way behind a producer, and a dispatch
-// again and again takes 44 us with ordinary loads and 54 without.
+// there.  8 x 4096 x 7168 bf16 with combine, ordinary and non-temporal loads, us a pass: behind an
+// element-wise kernel on the input 1159 and 1106, behind a 512 MB fill 1103 and 1068, again and
+// again 957 and 979.  8 x 1024 x 4096 (67 MB) is the same either way behind a producer, and a
+// dispatch again and again takes 44 and 54.
 //
 // Positions of rows are loaded beside the flags (EAGER) or behind them, which spares the loads of
-// destinations that do not hold the token and is faster for large calls whose tokens go to many.  Beside, behind, and
-// by the rows, us a pass of 8 x 4096 x 7168 bf16 top-8 with combine: 1006, 960, 959 with experts anywhere (5.3 rows a token);
-// 713, 714, 713 with those of four ranks a token (3.6 rows), 601, 607, 602 of three, 481, 501, 481 of two; dispatch
-// alone behind a kernel on the input 498, 481, 479 and, of two ranks, 219, 278, 220.  16 x 1024 (6.5 rows) 621, 604, 602.  Beside the
-// flags in any case: the scales of fp8 rows (passes 738 beside, 769 behind) and inputs up to kHtStreamFrom, which are the
-// same either way (8 x 1024 x 4096 97.2 and 98.0).
+// destinations that do not hold the token and is faster for large calls whose tokens go to many.
+// Beside, behind, and by the rows, us a pass of 8 x 4096 x 7168 bf16 top-8 with combine: 1006, 960,
+// 959 with experts anywhere (5.3 rows a token), 713, 714, 713 with those of four ranks a token
+// (3.6 rows), 481, 501, 481 of two.  Beside the flags in any case: the scales of fp8 rows (738
+// beside, 769 behind) and inputs up to kHtStreamFrom, which are the same either way.
 constexpr long long kHtStreamFrom = 128ll << 20;
 constexpr int kHtManyRows = 4; // a token
 
@@ -834,17 +828,15 @@ ht_meta_kernel(HtMeta m,
 
 // ---- combine (combine_token, kernels/nixl_ep_ht.cu:1682-1737) -----------------------------------
 // grid = R*T*parts; a row is H/8 lanes of 16 bytes and a workgroup covers blockDim.x of them,
-// every wave for itself.  Two forms: positions loaded beside the flags (EAGER), which shortens the chain
-// of loads, or behind them, which spares loads.  Which is faster depends on the rows that a token
-// gathers, as long as the call is so large that there are always waves to take over: us a call, eager and not,
-// 2 x 4096 x 7168 (2.0 rows a token) 62 and 72, 4 x 4096 x 7168 (3.6) 165 and 176, 8 x 4096 x 4096 (1.9) 138 and 156, (3.4) 182 and 195,
-// (3.9) 204 and 211, (4.4) 235 and 227, (5.3) 276 and 267, 8 x 4096 x 7168 (3.4) 317 and 337, (3.9) 363 and 363, (4.4) 409 and 397,
-// (5.3) 481 and 464.  Up to kHtCombineEager values the eager one is as fast or faster with any number of rows (8 x 256 x 7168 (5.3) 30.0 and
-// 30.9, 16 x 512 x 4096 (6.8) 84.1 and 84.0).  A call that does not say how many rows there are is eager up to that size.
-// A wave a workgroup, but four where a row is whole workgroups of them and tokens gather few rows: 8 x 4096 x 4096 (1.9) 134 and
-// 138 with one, 4 x 4096 x 4096 (2.8) 79.9 and 81.1, 8 x 4096 x 4096 (3.4) 182.5 and 181.9, (3.9) 208 and 205, 8 x 1024 x 4096 (3.9) 54.8 and
-// 55.3, (4.4) 58.8 and 57.9; with rows of 7168, which leave a fourth of every fourth workgroup idle, 4 x 1024 (1.8) 33.1 and 30.9, 4 x 4096
-// (3.6) 175 and 165.
+// every wave for itself.  Positions are loaded beside the flags (EAGER), which shortens the chain
+// of loads, or behind them, which spares loads and is faster for large calls whose tokens gather
+// more than four rows: 8 x 4096 x 7168, eager and not, 317 and 337 us with 3.4 rows a token, 363
+// and 363 with 3.9, 409 and 397 with 4.4, 481 and 464 with 5.3.  Up to kHtCombineEager values the eager form is
+// as fast or faster with any number (8 x 256 x 7168, 5.3 rows, 30.0 and 30.9), and a call that does
+// not say how many rows there are is eager up to that size.
+// A wave a workgroup, but four where a row is whole workgroups of them and tokens gather few rows:
+// 8 x 4096 x 4096 134 and 138 with one at 1.9 rows, 182.5 and 181.9 at 3.4; rows of 7168, which leave
+// a fourth of every fourth workgroup idle, 175 and 165 (4 x 4096, 3.6 rows).
 constexpr int kHtCombineEagerLanes = 256;
 constexpr long long kHtCombineEager = 1ll << 25;
 constexpr int kHtCombineManyRows = 4, kHtCombineFewRows = 3; // a token; few are as many as are not many in a small call

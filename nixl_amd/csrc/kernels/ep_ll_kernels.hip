@@ -14,10 +14,10 @@
 //                          indices and weights out as well.  This is the send phase.
 //   1b. ll_arrival_kernel  only for calls with a time-out: the receive side's bounded wait for
 //                          each source rank's bits; a late rank loses its bits and is masked.
-//   2. ll_dispatch_kernel  one workgroup per token (or several, dispatch_workgroup) reads its bf16 row once and, while the row
-//                          travels, counts for each of its K experts the bits in front of its
-//                          own (tokens of lower ranks, then lower tokens of its rank): that is
-//                          its row inside the expert.  It quantises the row in registers and
+//   2. ll_dispatch_kernel  one workgroup per token (or several, dispatch_workgroup) reads its
+//                          bf16 row once and, while the row travels, counts for each of its K
+//                          experts the bits in front of its own (tokens of lower ranks, then
+//                          lower tokens of its rank): that is its row inside the expert.  It quantises the row in registers and
 //                          writes it straight to its K final rows of packed_recv_x, plus
 //                          src_info and one row of inverse scales per token.  Workgroup e
 //                          also turns expert e's bits into layout_range, recv_count and the
@@ -1011,14 +1011,16 @@ round_up_wave(int n) {
     return (n + kWaveSize - 1) / kWaveSize * kWaveSize;
 }
 
-// Workgroup of ll_dispatch_kernel for a row of `lanes` lanes, while nobody has set another: a token's
-// whole row, since every workgroup finds the token's rows again.  Rows of 10, 12 and 14 waves (bf16, hidden
-// 5120, 6144 and 7168), which leave some of a compute unit's 32 waves idle that way, go by workgroups of two
-// where that was never slower.  With one or two rows a token it is mostly latency: 32 ranks x 128 tokens x 7168 45.3 and
-// 39.5 us, 16 x 128 23.0 and 18.4.  With three or four as long as the call is below four times what the chip holds
-// at once (16 x 128 x 7168 30.6 and 27.5, 32 x 72 x 5120 26.2 and 23.2, but 32 x 87 x 6144 36.0 and 39.9).  Rows of 14 waves again from seven
-// rounds of whole rows on, two to a compute unit (four rows a token 59.2 and 57.5, eight 112 and 105; five 72.1 and 73.4), where many rows a
-// token lose it in larger calls (32 x 256, eight rows, 198 and 204).
+// Workgroup of ll_dispatch_kernel for a row of `lanes` lanes, while nobody has set another: a
+// token's whole row, since every workgroup finds the token's rows again.  Rows of 10, 12 and 14
+// waves (bf16, hidden 5120, 6144 and 7168), which leave some of a compute unit's 32 waves idle that
+// way, go by workgroups of two where that was never slower.  Whole and so, us:
+// one or two rows a token, mostly latency: 32 ranks x 128 tokens x 7168 45.3 and 39.5;
+// three or four, as long as the call is below four times what the chip holds at once:
+// 16 x 128 x 7168 30.6 and 27.5, 32 x 72 x 5120 26.2 and 23.2, but 32 x 87 x 6144 36.0 and 39.9;
+// rows of 14 waves from seven rounds of whole rows on, two to a compute unit: four rows a token 59.2
+// and 57.5, eight 112 and 105 (five 72.1 and 73.4); in larger calls many rows a token lose it: 32 x
+// 256, eight rows, 198 and 204.
 int
 dispatch_workgroup(int lanes, const LlDims &d) {
     constexpr int kPart = 2 * kWaveSize, kWideRow = 14 * kWaveSize;
