@@ -1696,8 +1696,9 @@ def test_requests_from_several_threads(cuda):
 
 @pytest.mark.parametrize("upl", [4, 8, 16])
 def test_descriptor_ends_cost_what_their_bytes_do(cuda, upl):
-    """Descriptors of 16 bytes more than whole chunks take about as long as whole ones (a second chunk over the first for the 16 bytes
-    took 1.6 and 2.1 times as long at 8 and 16 units a lane), and every byte arrives."""
+    """Descriptors of 16 bytes more than whole chunks take as long as whole ones, at 16 units a lane, where a second wave comes to every
+    one, 1.30 times as long; a second chunk over the first for the 16 bytes took 1.46 times as long at 8 and 2.1 at 16.
+    Every byte arrives."""
     import torch
     n, pitch = 8192, 20480
     src = torch.randint(0, 256, (n, pitch), dtype=torch.uint8, device=cuda)
@@ -1715,7 +1716,7 @@ def test_descriptor_ends_cost_what_their_bytes_do(cuda, upl):
         assert lib.nixl_amd_copy_plan_status(plan, 1) == 0 and lib.nixl_amd_copy_plan_destroy(plan) == 0
         to = torch.from_numpy(((descs[:, 1] - np.uint64(dst.data_ptr())) // np.uint64(pitch)).astype(np.int64)).to(cuda)
         assert torch.equal(dst[to, :size], src[:, :size]) and not bool(dst[:, size:].any())
-    assert took[16400] < 1.35 * took[16384], took
+    assert took[16400] < {4: 1.2, 8: 1.2, 16: 1.6}[upl] * took[16384], took
 
 
 def _time_plan(lib, plan):
