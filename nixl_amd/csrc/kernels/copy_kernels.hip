@@ -61,8 +61,8 @@ struct UniformRec {
     uint64_t dst;
 };
 
-// The record of a chunk that is not whole, the end of a descriptor: its 16-byte units, less one, in the top
-// bytes of the two addresses, and the sign of dst, by which it is known.
+// The record of a chunk that is not whole, the end of a descriptor: its 16-byte units, less one, in
+// the top bytes of the two addresses, and the sign of dst, by which it is known.
 constexpr uint64_t kEndAddress = (1ull << 56) - 1;
 
 __device__ __forceinline__ UniformRec
@@ -719,11 +719,12 @@ clear_totals_kernel(ListTotals *totals) {
 }
 
 // A long descriptor as chunks of its own: chunk k starts k chunks behind the place `back` bytes in
-// front of the descriptor.  With a whole number of chunks and back = 0 that is all there is to it; else the
-// last chunk (and, with a `back` that puts the others on the destination's lines, the first) is an end, of as many
-// 16-byte units as its bytes need: less than a unit of it lies over its neighbour, where both write the
-// same bytes (or all that is missing from a chunk, where an address leaves no room for the number of units).  So every chunk belongs to one descriptor, whatever the length, and no descriptor
-// moves another one's chunks off the lines.
+// front of the descriptor.  With a whole number of chunks and back = 0 that is all there is to it;
+// else the last chunk (and, with a `back` that puts the others on the destination's lines, the
+// first) is an end, of as many 16-byte units as its bytes need: less than a unit of it lies over its
+// neighbour, where both write the same bytes.  (Where an address leaves no room for the number of
+// units, an end is a whole chunk and the rest of it lies there.)  So every chunk belongs to one
+// descriptor, whatever the length, and no descriptor moves another one's chunks off the lines.
 // Cut from one stream of all descriptors, with a whole chunk over its neighbour at each end, and so,
 // us: 512 tensors of 2 MiB + 16 B 372, 330 and 328; 60 000 descriptors of 8 to 64 KiB in multiples
 // of 16 bytes, shuffled, 1000, 844 and 838; 65 536 of 8 KiB + 128 B 195, 206 and 185; at 16 units a
@@ -1770,9 +1771,9 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     // size is no multiple of 16) is chunks, the first and the last of them ends (whose lanes' 16
     // bytes start anywhere).  Alone and up to kSplitFromTotal the byte kernel has the shorter way: its
     // items are fewer than the chunks' records and need no kernel to write them.  Made, launched and
-    // waited for, by the byte kernel and as chunks, us: 15 tensors of 1 MiB + 2 B 21.2 and 24.0, 15 of 4 MiB
-    // + 6 B 38.0 and 40.9, 126 of 1 MiB + 2 B 63.7 and 60.9, 2031 of 64 KiB + 2 B 74.9 and 76.7; 255 of 1 MiB + 2 B 114 and
-    // 101, 4 of 120 MiB 233 and 174.
+    // waited for, by the byte kernel and as chunks, us: 15 tensors of 1 MiB + 2 B 21.2 and 24.0, 15 of
+    // 4 MiB + 6 B 38.0 and 40.9, 126 of 1 MiB + 2 B 63.7 and 60.9, 2031 of 64 KiB + 2 B 74.9 and 76.7; 255
+    // of 1 MiB + 2 B 114 and 101, 4 of 120 MiB 233 and 174.
     const bool join = whole_chunks || bytes.splittable_total >= kSplitFromTotal;
     if (bytes.long_total - (join ? bytes.splittable_total : 0) > kLongItemsFrom) bytes.reach = kGenericItemBytes;
     const size_t n_aligned_runs = chunks.runs.size(), n_aligned_edges = chunks.edges;
