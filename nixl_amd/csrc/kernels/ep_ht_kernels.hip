@@ -837,9 +837,19 @@ ht_meta_kernel(HtMeta m,
 // A wave a workgroup, but four where a row is whole workgroups of them and tokens gather few rows:
 // 8 x 4096 x 4096 134 and 138 with one at 1.9 rows, 182.5 and 181.9 at 3.4; rows of 7168, which leave
 // a fourth of every fourth workgroup idle, 175 and 165 (4 x 4096, 3.6 rows).
+// With many ranks a look-up is many loads, the more so an eager one.  From kHtCombineManyRanks on large
+// calls are eager up to three rows a token (64 x 512 x 4096, 3.9 rows, eager and not 237 and 232), and up to
+// kHtCombineMostRanks, or kHtCombineMostRanksShared where four waves share the look-up (96 x 146 x 7168, 2.0 rows,
+// 142 and 156; 256 x 54 x 7168 282 and 184; 128 x 192 x 4096 142 and 162, 256 x 96 x 4096 226 and 191).
+// From kHtCombineManyRanksSmall on small ones share it if the row is whole workgroups of four waves
+// (four and one: 40 x 194 x 4096, 7.3 rows, 90.2 and 93.6, 96 x 162 x 2048 96.6 and 108.1, 16 x 972 x 2048 82.9 and
+// 82.3; 64 x 69 x 7168 39.8 and 37.1), and above kHtCombineMostRanksShared if it is long
+// (160 x 38 x 5120, 2.0 rows, 64.0 and 70.0, 160 x 77 x 2560 71.4 and 69.4).
 constexpr int kHtCombineEagerLanes = 256;
 constexpr long long kHtCombineEager = 1ll << 25;
 constexpr int kHtCombineManyRows = 4, kHtCombineFewRows = 3; // a token; few are as many as are not many in a small call
+constexpr int kHtCombineManyRanks = 48, kHtCombineManyRanksSmall = 32, kHtCombineMostRanks = 96, kHtCombineMostRanksShared = 128;
+constexpr int kHtCombineLongRow = 512; // lanes
 
 template<bool EAGER>
 __global__ void __launch_bounds__(kHtCombineEagerLanes)
@@ -1257,10 +1267,16 @@ nixl_amd_ep_ht_combine_rows(void *combined_x,
     const HtDims d{num_ranks, num_tokens, hidden, num_topk, num_ranks};
     const long long tokens = static_cast<long long>(num_ranks) * num_tokens;
     const bool large = tokens * hidden > kHtCombineEager;
-    const bool eager = !large || (num_rows >= 0 && num_rows <= kHtCombineManyRows * tokens);
     const int row_lanes = round_up_wave(hidden / 8);
-    const bool four_waves = eager && row_lanes % kHtCombineEagerLanes == 0 && num_rows <= (large ? kHtCombineFewRows : kHtCombineManyRows) * tokens;
-    const int lanes = four_waves ? kHtCombineEagerLanes : kWaveSize, parts = row_lanes / lanes;
+    const bool whole_wgs = row_lanes % kHtCombineEagerLanes == 0;
+    const bool many_ranks = num_ranks >= (large ? kHtCombineManyRanks : kHtCombineManyRanksSmall);
+    const bool eager = !large || (num_rows >= 0 && num_rows <= (many_ranks ? kHtCombineFewRows : kHtCombineManyRows) * tokens &&
+                                  num_ranks <= (whole_wgs ? kHtCombineMostRanksShared : kHtCombineMostRanks));
+    const bool four_waves = !large && many_ranks ?
+        whole_wgs || (num_ranks > kHtCombineMostRanksShared && row_lanes > kHtCombineLongRow) :
+        eager && whole_wgs && num_rows <= (large ? kHtCombineFewRows : kHtCombineManyRows) * tokens;
+    const int most = four_waves ? kHtCombineEagerLanes : kWaveSize;
+    const int parts = (row_lanes + most - 1) / most, lanes = round_up_wave((row_lanes + parts - 1) / parts);
     if (static_cast<long long>(num_ranks) * num_tokens * parts >= (1ll << 31))
         return nixl_amd_fail(NIXL_AMD_ERR_TOO_LARGE, "ht_combine: too many tokens");
     hipLaunchKernelGGL(eager ? ht_combine_kernel<true> : ht_combine_kernel<false>,

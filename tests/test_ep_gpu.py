@@ -1608,3 +1608,65 @@ def test_launches_go_to_the_current_stream(cuda):
         with torch.cuda.stream(torch.cuda.Stream()) as _, torch.cuda.device(cuda):
             assert ep._stream() == torch.cuda.current_stream().cuda_stream != 0
     assert ep._stream() == torch.cuda.current_stream().cuda_stream
+
+
+@pytest.mark.parametrize("R,T,H", [(31, 20, 2048), (32, 20, 2048), (47, 350, 2048), (48, 350, 2048), (64, 9, 2560), (96, 200, 2048), (97, 180, 2048), (97, 350, 1024), (128, 5, 5120),
+                                   (129, 5, 5120), (129, 130, 2048), (130, 9, 512)])
+def test_combine_of_many_ranks_in_every_form(cuda, R, T, H):
+    """Combine on both sides of the numbers of ranks at which its form changes, with rows that are whole workgroups of four waves and not, small calls and
+    large ones, few rows a token and many, the number of rows stated, wrong and not known: the sums are those of the rows, bit for
+    bit the same in every form."""
+    g = torch.Generator(device=cuda).manual_seed(R * 10 + T)
+    lib = _lib.ep_kernels()
+    for K in (2, 6):
+        E = R
+        topk = torch.topk(torch.rand((R, T, E), generator=g, device=cuda), K)[1].to(torch.int32).contiguous()
+        w = torch.rand((R, T, K), generator=g, device=cuda)
+        buf = Buffer(R, low_latency_mode=False, device=cuda)
+        per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk, E)
+        x = torch.zeros((R, T, H), dtype=torch.bfloat16, device=cuda)
+        rows, _, rw, _, handle, _ = buf.ht_dispatch(x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=per_expert,
+                                                    topk_idx=topk, topk_weights=w)
+        y = torch.randn(rows.shape, generator=g, device=cuda).to(torch.bfloat16)
+        in_rank, prefix, _, meta, head, offset = handle
+        want = torch.zeros((R * T, H), dtype=torch.float64, device=cuda)
+        want.index_add_(0, meta[:, 0].long() * T + meta[:, 1].long(), y.double())
+        first = None
+        for stated in (rows.shape[0], -1, 0, 5 * R * T):
+            out, out_w = torch.full((R, T, H), 7, dtype=torch.bfloat16, device=cuda), torch.empty((R, T, K), device=cuda)
+            rc = lib.nixl_amd_ep_ht_combine_rows(out.data_ptr(), out_w.data_ptr(), y.data_ptr(), rw.data_ptr(), None, None, in_rank.data_ptr(),
+                                                 prefix.data_ptr(), head.data_ptr(), offset.data_ptr(), stated, T, H, K, R,
+                                                 torch.cuda.current_stream().cuda_stream)
+            assert rc == 0, _lib.kernels_error()
+            got = (out.view(torch.int16), out_w)
+            first = first or got
+            assert all(torch.equal(a, b) for a, b in zip(got, first))
+        # six additions of 2^-24 of sums below 32, and half a step of bfloat16
+        assert bool(((first[0].view(torch.bfloat16).double().view(R * T, H) - want).abs() <= want.abs() / 256 + 2e-5).all())
+
+
+def test_large_combine_of_many_ranks_does_not_load_every_position(cuda):
+    """256 ranks, two rows a token: looking up the positions at all destinations of every token took 1.5 times as long as at those that hold it. The
+    form that a call takes with the number of rows stated must not be slower than the one that many rows take."""
+    R, T, H, K = 256, 54, 7168, 2
+    g = torch.Generator(device=cuda).manual_seed(8)
+    topk = torch.topk(torch.rand((R, T, R), generator=g, device=cuda), K)[1].to(torch.int32).contiguous()
+    buf = Buffer(R, low_latency_mode=False, device=cuda)
+    per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk, R)
+    x = torch.randn((R, T, H), generator=g, device=cuda).to(torch.bfloat16)
+    rows, _, rw, _, (in_rank, prefix, _, _, head, offset), _ = buf.ht_dispatch(
+        x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=per_expert, topk_idx=topk,
+        topk_weights=torch.ones((R, T, K), device=cuda))
+    out, out_w, took = torch.empty_like(x), torch.empty((R, T, K), device=cuda), {}
+    for stated in (rows.shape[0], 5 * R * T) * 8:
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(3):
+            rc = _lib.ep_kernels().nixl_amd_ep_ht_combine_rows(out.data_ptr(), out_w.data_ptr(), rows.data_ptr(), rw.data_ptr(), None, None,
+                                                               in_rank.data_ptr(), prefix.data_ptr(), head.data_ptr(), offset.data_ptr(), stated,
+                                                               T, H, K, R, torch.cuda.current_stream().cuda_stream)
+        e1.record()
+        e1.synchronize()
+        assert rc == 0, _lib.kernels_error()
+        took.setdefault(stated, []).append(e0.elapsed_time(e1))
+    assert np.median(took[rows.shape[0]]) < 1.2 * np.median(took[5 * R * T]), took
