@@ -277,6 +277,18 @@ nixl_amd_copy_plan_create_listed_on(const nixl_amd_copy_list_t *src,
 int
 nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream);
 
+/* The same for a plan whose destinations are device memory.  Status and destroy then look at a word
+ * in host memory that the launch's last kernel writes instead of at an event behind it, which shows
+ * the end some microseconds sooner.  (A word says nothing of caches over host memory, for which an
+ * event is what releases them.)  Needs nixl_amd_copy_watch_prepare, which allocates the words once a
+ * process; without it, for more than 128 launches in flight on a device, and for a plan whose earlier
+ * launch is still running, an event is recorded as nixl_amd_copy_plan_launch does. */
+int
+nixl_amd_copy_plan_launch_watched(nixl_amd_copy_plan_t *plan, void *stream);
+
+int
+nixl_amd_copy_watch_prepare(void);
+
 /* Whether the plan's launches have completed: NIXL_AMD_OK when all have (or none was made),
  * NIXL_AMD_ERR_BUSY while one still runs (no error text is recorded for that answer: the call
  * is made to be polled), another negative status if a launch failed.  With `wait` non-zero the

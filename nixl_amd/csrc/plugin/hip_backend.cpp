@@ -122,8 +122,7 @@ nixlHipReqH::~nixlHipReqH() {
 }
 
 // NIXL_SUCCESS when nothing of the request is running any more, NIXL_IN_PROG while its posted
-// copy runs, NIXL_ERR_BACKEND if it failed.  The plan itself keeps the event behind its last
-// launch, so a post costs one event record, not two.
+// copy runs, NIXL_ERR_BACKEND if it failed.  The plan itself knows how its last launch is seen to end.
 nixl_status_t
 nixlHipReqH::state(bool wait) const {
     if (!posted) return NIXL_SUCCESS;
@@ -171,6 +170,8 @@ nixlHipEngine::nixlHipEngine(const nixlBackendInitParams *init_params)
         return;
     }
     numDevices_ = n;
+    if (nixl_amd_copy_watch_prepare() != NIXL_AMD_OK) // transfers are seen to end a little later then
+        NIXL_WARN << "HIP backend: " << nixl_amd_last_error();
     streams_.assign(static_cast<size_t>(n) * streamsPerDevice_, nullptr);
     {
         std::lock_guard<std::mutex> lock(g_registryMutex);
@@ -862,8 +863,8 @@ nixlHipEngine::prepXferListed(const nixl_xfer_op_t &operation,
 
 nixl_status_t
 nixlHipEngine::postXfer(const nixl_xfer_op_t &,
-                        const nixl_meta_dlist_t &,
-                        const nixl_meta_dlist_t &,
+                        const nixl_meta_dlist_t &local,
+                        const nixl_meta_dlist_t &remote,
                         const std::string &remote_agent,
                         nixlBackendReqH *&handle,
                         const nixl_opt_b_args_t *opt_args) const {
@@ -878,11 +879,12 @@ nixlHipEngine::postXfer(const nixl_xfer_op_t &,
         deliverPending(req, earlier == NIXL_SUCCESS);
     }
 
-    if (nixl_amd_copy_plan_launch(req->plan, req->stream) != NIXL_AMD_OK) {
+    const bool on_gpu = local.getType() == VRAM_SEG && remote.getType() == VRAM_SEG;
+    if ((on_gpu ? nixl_amd_copy_plan_launch_watched : nixl_amd_copy_plan_launch)(req->plan, req->stream) != NIXL_AMD_OK) {
         NIXL_ERROR << "HIP backend: " << nixl_amd_last_error();
         return NIXL_ERR_BACKEND;
     }
-    req->posted = true; // the launch recorded the plan's event behind its kernels
+    req->posted = true; // and what the plan's status looks at is behind its kernels
     if (opt_args && opt_args->hasNotif) {
         // only now: whoever sees the flag must find the event of THIS post behind it
         std::lock_guard<std::mutex> lock(pendingMutex_);

@@ -1723,3 +1723,71 @@ def _time_plan(lib, plan):
     ms = ctypes.c_float()
     assert lib.nixl_amd_copy_plan_time(plan, None, 10, ctypes.byref(ms)) == 0
     return ms.value
+
+
+@pytest.mark.parametrize("blocks, blk", [(1, 8192), (1, 15 * 1024), (1, 16 * 1024), (1, 17 * 1024), (4, 256 * 1024), (65, 16 * 1024),
+                                         (128, 32 * 1024), (128, 33 * 1024), (129, 8192), (3, 4096), (40, 24)])
+@pytest.mark.parametrize("policy", [0, 1, 3])
+def test_watched_launch_is_done_when_its_bytes_are_there(cuda, blocks, blk, policy):
+    """A launch that is watched by a word says that it is done when its bytes have arrived, again and
+    again: workgroups around the ones that are counted in one group and in several, around the size up to
+    which the copy counts itself, a policy that does not write through, requests of other kernels.  Each
+    look at the bytes follows the word alone, from a stream that is ordered by nothing else."""
+    import torch
+    lib = _lib.kernels()
+    assert lib.nixl_amd_copy_watch_prepare() == 0
+    src = torch.randint(0, 256, (blocks, blk), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros_like(src)
+    stream, look = torch.cuda.Stream(), torch.cuda.Stream()
+    plan = _plan([(src.data_ptr() + i * blk, dst.data_ptr() + i * blk, blk) for i in range(blocks)], (0, policy))
+    for i in range(20):
+        with torch.cuda.stream(look):
+            src += 1
+            dst.zero_()
+        look.synchronize()
+        assert lib.nixl_amd_copy_plan_launch_watched(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+        if i % 2:
+            assert lib.nixl_amd_copy_plan_status(plan, 1) == 0
+        else:
+            while (rc := lib.nixl_amd_copy_plan_status(plan, 0)) == -4:  # NIXL_AMD_ERR_BUSY
+                pass
+            assert rc == 0
+        with torch.cuda.stream(look):
+            assert torch.equal(src, dst), i
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+
+
+def test_watched_launches_beyond_the_words_and_on_two_streams(cuda):
+    """More launches in flight than there are words, a plan launched again while its first launch is
+    still watched (on another stream, ending first), and plans destroyed in between: every status tells the truth."""
+    import torch
+    lib = _lib.kernels()
+    assert lib.nixl_amd_copy_watch_prepare() == 0
+    n, blk = 200, 16 * 1024
+    src = torch.randint(0, 256, (n, blk), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros_like(src)
+    busy = torch.zeros(64 << 20, dtype=torch.float32, device=cuda)
+    slow, fast = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        dst.zero_()
+        torch.cuda.synchronize()
+        plans = [_plan([(src.data_ptr() + i * blk, dst.data_ptr() + i * blk, blk)]) for i in range(n)]
+        with torch.cuda.stream(slow):
+            for _ in range(20):
+                busy.add_(1.0)
+        first = torch.cuda.Event()
+        for p in plans:
+            assert lib.nixl_amd_copy_plan_launch_watched(p, slow.cuda_stream) == 0, _lib.kernels_error()
+            if p is plans[0]:
+                first.record(slow)
+        assert lib.nixl_amd_copy_plan_launch_watched(plans[0], fast.cuda_stream) == 0, _lib.kernels_error()
+        assert lib.nixl_amd_copy_plan_launch(plans[1], fast.cuda_stream) == 0, _lib.kernels_error()
+        fast.synchronize()
+        # the launch on the slow stream is still watched, whatever the other one has done
+        assert lib.nixl_amd_copy_plan_status(plans[0], 0) != 0 or first.query()
+        for p in plans:
+            assert lib.nixl_amd_copy_plan_status(p, 1) == 0
+            assert lib.nixl_amd_copy_plan_destroy(p) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(src, dst)
