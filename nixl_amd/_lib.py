@@ -5,6 +5,7 @@ The libraries are built by ``__graft_entry__.build()`` (``make -C nixl_amd/csrc`
 implementation: a missing library raises ``NativeLibraryMissing``.
 """
 import ctypes
+import importlib.util
 import os
 from ctypes import (POINTER, Structure, c_bool, c_char_p, c_float, c_int, c_int64, c_size_t, c_uint16,
                     c_uint, c_uint32, c_uint64, c_void_p)
@@ -158,6 +159,25 @@ def ep_kernels():
     lib.nixl_amd_ep_ll_workspace_bytes.restype = c_size_t
     _ep = lib
     return lib
+
+
+_host = None
+
+
+def ep_host():
+    """The allocations and launches of the expert-parallel calls (csrc/ep_host), a Python module over torch."""
+    global _host
+    if _host is None:
+        ep_kernels()
+        path = os.path.join(LIB_DIR, "_ep_host.so")
+        if not os.path.exists(path):
+            raise NativeLibraryMissing(f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` first")
+        import torch  # noqa: F401  (the module's symbols are torch's)
+        spec = importlib.util.spec_from_file_location("_ep_host", path)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host
 
 
 def kernel_symbols():

@@ -12,9 +12,7 @@ only owns the memory and the stream; all work is done by the HIP kernels behind
 include/nixl_amd_ep.h, and nothing here falls back to torch ops.
 """
 import ctypes
-import time
 
-import numpy as np
 import torch
 
 from . import _lib
@@ -129,6 +127,7 @@ class Buffer:
         # its receivers wait for, so that their wait runs out (one-shot knob, -1 = off).
         self.withhold_rank = -1
         self._k = _lib.ep_kernels()
+        self._host = _lib.ep_host()
         self.mask_buffer = torch.zeros((self.num_ranks, self.num_ranks), dtype=torch.int32, device=self.device)
         self._mask_active = False
         self._workspace = None
@@ -279,20 +278,6 @@ class Buffer:
             self._mapped_view = self._mapped_tensor.numpy()
         return self._mapped_view
 
-    def _wait_counts(self, mapped, num_ranks):
-        """Polls until the GPU has written every count (reference: csrc/nixl_ep.cpp:779-797,
-        same time-out); returns the total number of rows."""
-        deadline = time.monotonic() + self.cpu_timeout_secs
-        while int(mapped.min()) < 0:
-            if time.monotonic() > deadline:
-                raise EPError("timeout (dispatch CPU): the receive counts never arrived")
-        return int(mapped[:num_ranks].sum(dtype=np.int64))
-
-    def _get_workspace(self, nbytes):
-        if self._workspace is None or self._workspace.numel() < nbytes:
-            self._workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=self.device)
-        return self._workspace
-
     # -- low-latency mode -------------------------------------------------------------------
     def low_latency_dispatch(self, x, topk_idx, num_max_dispatch_tokens_per_rank, num_experts=None,
                              cumulative_local_expert_recv_stats=None, dispatch_wait_recv_cost_stats=None,
@@ -351,27 +336,14 @@ class Buffer:
         if num_experts is None:
             raise EPError("num_experts is required")
         El, N = num_experts // R, R * num_max_dispatch_tokens_per_rank
-        dev = x.device
-        packed_recv_x = torch.empty((R, El, N, H), dtype=torch.float8_e4m3fn if use_fp8 else torch.bfloat16, device=dev)
-        packed_recv_src_info = torch.empty((R, El, N), dtype=torch.int32, device=dev)
-        packed_recv_layout_range = torch.empty((R, El, R), dtype=torch.int64, device=dev)
-        packed_recv_count = torch.empty((R, El), dtype=torch.int32, device=dev)
-        scales = None
-        if use_fp8:
-            if use_ue8m0:
-                scales = torch.empty((R, El, H // 512, N), dtype=torch.int32, device=dev)
-            else:
-                scales = torch.empty((R, El, H // 128, N), dtype=torch.float32, device=dev)
-        row_map = torch.empty((R, T, K), dtype=torch.int32, device=dev)
-        ws_bytes = self._k.nixl_amd_ep_ll_workspace_bytes(R, num_experts, T, K, H)
-        ws = self._get_workspace(ws_bytes)
-        head = (_ptr(packed_recv_x), _ptr(scales), _ptr(packed_recv_src_info), _ptr(packed_recv_layout_range),
-                _ptr(packed_recv_count), self._mask_ptr(), _ptr(stats), _ptr(x))
-        tail = (_ptr(num_tokens_per_rank), T, H, num_max_dispatch_tokens_per_rank, K, R, num_experts, int(use_fp8),
-                int(round_scale), int(use_ue8m0), _ptr(row_map), _ptr(ws), ws.numel(), _stream())
-        topk_weights = None
-        hook = None
         phased = logits is None and (self.timeout_ms is not None or return_recv_hook)
+        (packed_recv_x, scales, packed_recv_src_info, packed_recv_layout_range, packed_recv_count, row_map, topk_idx,
+         topk_weights, ws, rc) = self._host.ll_dispatch(
+            x, topk_idx, logits, self._workspace, stats, num_tokens_per_rank, self._mask_ptr(), El, N, K,
+            num_max_dispatch_tokens_per_rank, num_experts, int(use_fp8), int(round_scale), int(use_ue8m0), int(not phased),
+            _stream())
+        self._workspace = ws
+        hook = None
         if phased:
             if wait_stats is not None and (wait_stats.dtype != torch.int64 or wait_stats.numel() < R):
                 raise EPError("dispatch_wait_recv_cost_stats must hold R int64 values")
@@ -383,8 +355,11 @@ class Buffer:
 
             def issue(phases):
                 return self._k.nixl_amd_ep_ll_dispatch_phased(
-                    *head[:5], mask, _ptr(stats), _ptr(wait_stats), _ptr(x), _ptr(topk_idx), *tail[:-1], phases,
-                    timeout_us, withhold, _stream())
+                    _ptr(packed_recv_x), _ptr(scales), _ptr(packed_recv_src_info), _ptr(packed_recv_layout_range),
+                    _ptr(packed_recv_count), mask, _ptr(stats), _ptr(wait_stats), _ptr(x), _ptr(topk_idx),
+                    _ptr(num_tokens_per_rank), T, H, num_max_dispatch_tokens_per_rank, K, R, num_experts, int(use_fp8),
+                    int(round_scale), int(use_ue8m0), _ptr(row_map), _ptr(ws), ws.numel(), phases, timeout_us, withhold,
+                    _stream())
 
             if return_recv_hook:
                 rc = issue(1)
@@ -398,12 +373,6 @@ class Buffer:
                 check_duplicates = False  # not before the receive phase has run
             else:
                 rc = issue(3)
-        elif logits is None:
-            rc = self._k.nixl_amd_ep_ll_dispatch(*head, _ptr(topk_idx), *tail)
-        else:
-            topk_idx = torch.empty((R, T, K), dtype=topk_idx_t, device=dev)
-            topk_weights = torch.empty((R, T, K), dtype=torch.float32, device=dev)
-            rc = self._k.nixl_amd_ep_ll_route_dispatch(*head, _ptr(logits), _ptr(topk_idx), _ptr(topk_weights), *tail)
         _check(rc, "low_latency_dispatch")
         if check_duplicates:
             self._raise_on_repeats(ws)
@@ -413,7 +382,7 @@ class Buffer:
             event.record()
         handle = DispatchHandle((packed_recv_src_info, packed_recv_layout_range, num_max_dispatch_tokens_per_rank, H))
         handle.row_map = row_map
-        recv = (packed_recv_x, scales.transpose(2, 3)) if use_fp8 else packed_recv_x
+        recv = (packed_recv_x, scales) if use_fp8 else packed_recv_x
         if return_recv_hook and hook is None:
             hook = lambda: None  # noqa: E731  (routing dispatch: issued whole)
         return topk_idx, topk_weights, recv, packed_recv_count, handle, EventOverlap(event), hook
@@ -451,7 +420,6 @@ class Buffer:
             raise EPError("topk_weights must be contiguous float32")
         R, T, K = topk_idx.shape
         num_experts = x.shape[1] * R
-        combined = out if out is not None else torch.empty((R, T, hidden), dtype=torch.bfloat16, device=x.device)
         stats = combine_wait_recv_cost_stats
         if rank_ready is not None:
             if self.timeout_ms is None:
@@ -463,30 +431,32 @@ class Buffer:
             self._mask_active = True
         row_map = getattr(handle, "row_map", None)
 
+        if out is None and (rank_ready is not None or return_recv_hook):
+            out = torch.empty((R, T, hidden), dtype=torch.bfloat16, device=x.device)
+
         def issue():
             if rank_ready is not None:
-                return self._k.nixl_amd_ep_ll_combine_elastic(
-                    _ptr(combined), _ptr(x), _ptr(topk_idx), _ptr(topk_weights), _ptr(src_info), _ptr(layout_range),
+                return out, self._k.nixl_amd_ep_ll_combine_elastic(
+                    _ptr(out), _ptr(x), _ptr(topk_idx), _ptr(topk_weights), _ptr(src_info), _ptr(layout_range),
                     _ptr(self.mask_buffer), _ptr(rank_ready), _ptr(stats), _ptr(num_tokens_per_rank), _ptr(row_map), T,
                     hidden, max_tok, K, R, num_experts, int(use_logfmt), max(int(self.timeout_ms * 1000), 1), _stream())
-            return self._k.nixl_amd_ep_ll_combine(
-                _ptr(combined), _ptr(x), _ptr(topk_idx), _ptr(topk_weights), _ptr(src_info), _ptr(layout_range),
-                self._mask_ptr(), _ptr(num_tokens_per_rank), _ptr(row_map), T, hidden, max_tok, K, R, num_experts,
-                int(use_logfmt), _stream())
+            return self._host.ll_combine(out, x, topk_idx, topk_weights, src_info, layout_range, num_tokens_per_rank, row_map,
+                                         self._mask_ptr(), hidden, max_tok, int(use_logfmt), _stream())
 
         # The send phase of the reference moves the expert outputs to their readers; here they
         # are read where they lie, so with a hook the whole reduction is the receive phase and
         # combined_x is valid once the hook has run (as in the reference).
         hook = None
         if return_recv_hook:
-            hook = lambda: _check(issue(), "low_latency_combine (receive phase)")  # noqa: E731
+            hook = lambda: _check(issue()[1], "low_latency_combine (receive phase)")  # noqa: E731
         else:
-            _check(issue(), "low_latency_combine")
+            out, rc = issue()
+            _check(rc, "low_latency_combine")
         event = None
         if async_finish:
             event = torch.cuda.Event()
             event.record()
-        return combined, EventOverlap(event), hook
+        return out, EventOverlap(event), hook
 
     def combine(self, *args, **kwargs):
         return self.low_latency_combine(*args, **kwargs)
@@ -530,14 +500,11 @@ class Buffer:
         """Reference: buffer.py:278-326, csrc/nixl_ep.cpp:551-613.  topk_idx [R, T, K].
         Returns (num_tokens_per_rank [R, R], num_tokens_per_rdma_rank=None,
         num_tokens_per_expert [R, E], is_token_in_rank [R, T, R] bool, event)."""
-        R, T, K = topk_idx.shape
-        dev = topk_idx.device
+        if topk_idx.dim() != 3:
+            raise ValueError("topk_idx must be a [R, T, K] tensor")
         self._after(previous_event, async_finish, allocate_on_comm_stream)
-        per_rank = torch.empty((R, R), dtype=torch.int32, device=dev)
-        per_expert = torch.empty((R, num_experts), dtype=torch.int32, device=dev)
-        in_rank = torch.empty((R, T, R), dtype=torch.bool, device=dev)
-        _check(self._k.nixl_amd_ep_get_dispatch_layout(_ptr(topk_idx), _ptr(per_rank), _ptr(per_expert), _ptr(in_rank),
-                                                       T, K, R, num_experts, _stream()), "get_dispatch_layout")
+        per_rank, per_expert, in_rank, rc = self._host.layout(topk_idx, num_experts, _stream())
+        _check(rc, "get_dispatch_layout")
         return per_rank, None, per_expert, in_rank, self._done(async_finish)
 
     def ht_dispatch(self, x, handle=None, num_tokens_per_rank=None, num_tokens_per_rdma_rank=None,
@@ -562,7 +529,6 @@ class Buffer:
         if x_scales is None and x.dtype != torch.bfloat16:
             raise EPError("x must be bfloat16 unless it comes with scales, as (x, x_scales)")
         R, T, H = x.shape
-        dev = x.device
         if (H * x.element_size()) % 16:
             raise EPError("a row of x must be a multiple of 16 bytes")  # csrc/nixl_ep.cpp:660
         S = 0
@@ -571,13 +537,6 @@ class Buffer:
             if x_scales.dtype not in (torch.float32, torch.int32) or x_scales.dim() != 3 or tuple(x_scales.shape[:2]) != (R, T):
                 raise EPError("x_scales must be a float32 or int32 tensor of shape [R, T, num_scales]")
             S = x_scales.shape[2]
-
-        def rows_kernel(recv_x, recv_scales, recv_idx, recv_w, recv_meta, idx, w, in_rank, prefix, send_head, row_offset, K, E):
-            strides = x_scales.stride() if x_scales is not None else (0, 0, 0)
-            _check(self._k.nixl_amd_ep_ht_dispatch_scaled(
-                _ptr(recv_x), _ptr(recv_scales), _ptr(recv_idx), _ptr(recv_w), _ptr(recv_meta), _ptr(x), _ptr(x_scales),
-                _ptr(idx), _ptr(w), _ptr(in_rank), _ptr(prefix), _ptr(send_head), _ptr(row_offset), T, H,
-                x.element_size(), S, strides[0], strides[1], strides[2], K, R, E, _stream()), "ht_dispatch")
 
         def with_scales(recv_x, recv_scales):
             return (recv_x, recv_scales) if x_scales is not None else recv_x
@@ -590,10 +549,9 @@ class Buffer:
             in_rank, prefix, _chan, recv_src_meta, send_head, row_offset = handle
             if tuple(in_rank.shape) != (R, T, R):
                 raise EPError("handle does not belong to a dispatch of this shape")
-            n_rows = recv_src_meta.shape[0]
-            recv_x = torch.empty((n_rows, H), dtype=x.dtype, device=dev)
-            recv_scales = torch.empty((n_rows, S), dtype=x_scales.dtype, device=dev) if x_scales is not None else None
-            rows_kernel(recv_x, recv_scales, None, None, None, None, None, in_rank, prefix, send_head, row_offset, 0, R)
+            recv_x, recv_scales, rc = self._host.ht_dispatch_cached(x, x_scales, in_rank, prefix, send_head, row_offset,
+                                                                    recv_src_meta.shape[0], _stream())
+            _check(rc, "ht_dispatch")
             return with_scales(recv_x, recv_scales), None, None, None, None, self._done(async_finish)
         if num_tokens_per_rank is None or is_token_in_rank is None or num_tokens_per_expert is None:
             raise EPError("ht_dispatch needs either a handle or the tensors of get_dispatch_layout")
@@ -604,42 +562,21 @@ class Buffer:
         K = topk_idx.shape[2] if topk_idx is not None else 0
         E = num_tokens_per_expert.shape[1]
         El = E // R
-        prefix = torch.empty((R, R), dtype=torch.int32, device=dev)
-        chan = torch.empty((R, R, num_channels), dtype=torch.int32, device=dev)
-        send_head = torch.empty((R, T, R), dtype=torch.int32, device=dev)
-        row_offset = torch.empty(R + 1, dtype=torch.int64, device=dev)
-        # The counts the host needs go straight to pinned host memory, preset to -1 and polled
-        # below, as in the reference (csrc/nixl_ep.cpp:762-800).
+        # The counts the host needs go straight to pinned host memory, preset to -1 and polled, as
+        # in the reference (csrc/nixl_ep.cpp:762-800).  The reference waits for them before it launches
+        # the rows, because it sizes recv_x from them.  With 288 GB of HBM the receive side can be sized
+        # for the worst case instead (every set entry of is_token_in_rank is one row, so R*T*R rows bound
+        # the total): the row kernels are queued right behind the count kernels, the GPU never idles
+        # through the host round trip, and the host only waits for the counts to cut the views.
         mapped = self._mapped_counts(R + R * El)
-        mapped.fill(-1)
-        recv_counter_ptr = self._mapped_tensor.data_ptr()
-        expert_count_ptr = recv_counter_ptr + 4 * R
-        _check(self._k.nixl_amd_ep_ht_notify_dispatch(_ptr(is_token_in_rank), _ptr(num_tokens_per_expert), _ptr(prefix),
-                                                      expert_count_ptr, _ptr(chan), _ptr(send_head), _ptr(row_offset),
-                                                      recv_counter_ptr, T, R, E, num_channels, expert_alignment,
-                                                      _stream()), "ht_notify_dispatch")
-        # The reference waits here, because it sizes recv_x from the counts.  With 288 GB of
-        # HBM the receive side can be sized for the worst case instead (every set entry of
-        # is_token_in_rank is one row, so R*T*R rows bound the total): the row kernels are
-        # queued right behind the count kernels, the GPU never idles through the host round
-        # trip, and the host only waits for the counts to cut the views.
-        capacity = R * T * R
-        ahead = capacity * (H * x.element_size() + S * 4 + K * 8 + 8) <= self.ht_recv_worst_case_limit
-        rows = capacity if ahead else self._wait_counts(mapped, R)
-        recv_x = torch.empty((rows, H), dtype=x.dtype, device=dev)
-        recv_scales = torch.empty((rows, S), dtype=x_scales.dtype, device=dev) if x_scales is not None else None
-        recv_topk_idx = torch.empty((rows, K), dtype=torch.int32, device=dev) if K else None
-        recv_topk_weights = torch.empty((rows, K), dtype=torch.float32, device=dev) if K else None
-        recv_src_meta = torch.empty((rows, 2), dtype=torch.int32, device=dev)
-        rows_kernel(recv_x, recv_scales, recv_topk_idx, recv_topk_weights, recv_src_meta, topk_idx, topk_weights,
-                    is_token_in_rank, prefix, send_head, row_offset, K, E)
-        if ahead:
-            total = self._wait_counts(mapped, R)
-            recv_x, recv_src_meta = recv_x[:total], recv_src_meta[:total]
-            if recv_scales is not None:
-                recv_scales = recv_scales[:total]
-            if K:
-                recv_topk_idx, recv_topk_weights = recv_topk_idx[:total], recv_topk_weights[:total]
+        ahead = R * T * R * (H * x.element_size() + S * 4 + K * 8 + 8) <= self.ht_recv_worst_case_limit
+        (recv_x, recv_scales, recv_topk_idx, recv_topk_weights, recv_src_meta, prefix, chan, send_head, row_offset,
+         (rc, stage)) = self._host.ht_dispatch(x, x_scales, is_token_in_rank, num_tokens_per_expert, topk_idx, topk_weights,
+                                               self._mapped_tensor, El, num_channels, expert_alignment, int(ahead),
+                                               self.cpu_timeout_secs, _stream())
+        _check(rc, "ht_notify_dispatch" if stage == 1 else "ht_dispatch")
+        if stage == 2:
+            raise EPError("timeout (dispatch CPU): the receive counts never arrived")
         expert_count_list = mapped[R:].reshape(R, El).tolist()
         out_handle = (is_token_in_rank, prefix, chan, recv_src_meta, send_head, row_offset)
         return (with_scales(recv_x, recv_scales), recv_topk_idx, recv_topk_weights, expert_count_list, out_handle,
@@ -653,15 +590,11 @@ class Buffer:
         if self.low_latency_mode:
             raise EPError("ht_combine() requires high-throughput mode (low_latency_mode=False)")
         in_rank, prefix, _chan, _meta, send_head, row_offset = handle
-        R, T, _ = in_rank.shape
-        H = x.shape[1]
-        dev = x.device
+        if in_rank.dim() != 3:
+            raise ValueError("the handle of an ht_dispatch() starts with a [R, T, R] tensor")
         bias_0, bias_1 = (bias if isinstance(bias, (tuple, list)) else (bias, None))
-        K = topk_weights.shape[1] if topk_weights is not None else 0
         self._after(previous_event, async_finish, allocate_on_comm_stream)
-        combined = torch.empty((R, T, H), dtype=torch.bfloat16, device=dev)
-        combined_w = torch.empty((R, T, K), dtype=torch.float32, device=dev) if K else None
-        _check(self._k.nixl_amd_ep_ht_combine_rows(_ptr(combined), _ptr(combined_w), _ptr(x), _ptr(topk_weights),
-                                                   _ptr(bias_0), _ptr(bias_1), _ptr(in_rank), _ptr(prefix), _ptr(send_head),
-                                                   _ptr(row_offset), x.shape[0], T, H, max(K, 1), R, _stream()), "ht_combine")
+        combined, combined_w, rc = self._host.ht_combine(x, topk_weights, bias_0, bias_1, in_rank, prefix, send_head,
+                                                         row_offset, _stream())
+        _check(rc, "ht_combine")
         return combined, combined_w, self._done(async_finish)

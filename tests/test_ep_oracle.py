@@ -615,3 +615,37 @@ def test_stream_handle_with_and_without_torchs_private_names(monkeypatch, missin
     if missing:
         monkeypatch.delattr(torch._C, missing)
     assert ep._stream_getter()() == (77 if missing else 1003)
+
+
+@pytest.mark.parametrize("args, error", [
+    ((), TypeError),  # too few
+    ((1, 8, None), TypeError),  # not a tensor
+    ((torch.zeros(2, 3, 4, dtype=torch.int32), 8.0, None), TypeError),  # a count that is no integer
+    ((torch.zeros(2, 3, 4, dtype=torch.int32), 1 << 40, None), TypeError),  # or more than the entry points take
+    ((torch.zeros(2, 3, 4, dtype=torch.int32), -8, None), RuntimeError),  # a shape that torch refuses
+    ((torch.zeros(2, 3, dtype=torch.int32), 8, None), IndexError),  # a dimension that is not there
+])
+def test_native_host_calls_refuse_what_they_cannot_use(args, error):
+    from nixl_amd import _lib
+    with pytest.raises(error):
+        _lib.ep_host().layout(*args)
+
+
+def test_native_host_calls_hand_back_the_kernels_status_and_the_callers_tensors():
+    """Without a launch the low-latency call only makes its tensors, and a launch that the kernels refuse on the host
+    (five experts on two ranks) comes back as a status, not as an exception."""
+    from nixl_amd import _lib
+    R, T, H, K, E, M = 2, 3, 1024, 2, 4, 5
+    x, topk = torch.zeros(R, T, H, dtype=torch.bfloat16), torch.zeros(R, T, K, dtype=torch.int32)
+    for ue8m0, scales_shape, scales_type in ((0, (R, E // R, R * M, H // 128), torch.float32), (1, (R, E // R, R * M, H // 512), torch.int32)):
+        rows, scales, src, layout, count, row_map, idx, weights, ws, rc = _lib.ep_host().ll_dispatch(
+            x, topk, None, None, None, None, None, E // R, R * M, K, M, E, 1, ue8m0, ue8m0, 0, None)
+        assert rc == 0 and idx is topk and weights is None
+        assert rows.shape == (R, E // R, R * M, H) and rows.dtype == torch.float8_e4m3fn
+        assert scales.shape == scales_shape and scales.dtype == scales_type and scales.stride(2) == 1
+        assert src.shape == (R, E // R, R * M) and layout.shape == (R, E // R, R) and layout.dtype == torch.int64
+        assert count.shape == (R, E // R) and row_map.shape == (R, T, K)
+        assert ws.numel() >= _lib.ep_kernels().nixl_amd_ep_ll_workspace_bytes(R, E, T, K, H)
+        again = _lib.ep_host().ll_dispatch(x, topk, None, ws, None, None, None, E // R, R * M, K, M, E, 0, 0, 0, 0, None)
+        assert again[-2] is ws and again[1] is None and again[0].dtype == torch.bfloat16
+    assert _lib.ep_host().layout(topk, 5, None)[-1] != 0
