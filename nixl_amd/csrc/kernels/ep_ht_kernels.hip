@@ -59,6 +59,7 @@ block_exclusive_scan(V v, V *wave_sums, V &total) {
 // kLayoutWholeFlags a rank: 32 x 768 tokens 5.0 and 5.1 us, 32 x 1024 5.9 and 5.1, 64 x 384 5.5 and 7.0, 64 x 768
 // 8.7 and 8.1, 128 x 384 42 and 37; a single chunk of kLayoutTokens tokens is one workgroup either way, and
 // from 256 ranks on one workgroup a rank fills the chip (256 x 384 121 and 159, 256 x 1024 327 and 592).
+constexpr int kMaxTopk = 16; // check_ht
 constexpr int kLayoutTokens = 256;
 constexpr int kLayoutWhole = 1024;
 constexpr int kLayoutWholeSelections = 4096;
@@ -241,15 +242,21 @@ struct HtNotifyOut {
     int alignment;
 };
 
+__device__ __forceinline__ int
+aligned(int n, int alignment) {
+    return (n + alignment - 1) / alignment * alignment;
+}
+
+// Experts from `first_expert` on: those before it are done.
 template<typename TotalOf>
 __device__ __forceinline__ void
-notify_prefix(const HtNotifyOut &o, int R, int E, const TotalOf &total_of) {
+notify_prefix(const HtNotifyOut &o, int R, int E, int first_expert, const TotalOf &total_of) {
     __shared__ int wave_sums[kScanThreads / kWaveSize];
     const int tid = threadIdx.x;
     // Loads go out eight at a time before anything depends on them: issued one by one, the
     // round trips of this single workgroup add up to most of the kernel's time.
     constexpr int kBatch = 8;
-    for (int e = tid; e < E; e += kScanThreads) {
+    for (int e = first_expert + tid; e < E; e += kScanThreads) {
         int n = 0;
         for (int r0 = 0; r0 < R; r0 += kBatch) {
             int v[kBatch];
@@ -260,7 +267,7 @@ notify_prefix(const HtNotifyOut &o, int R, int E, const TotalOf &total_of) {
             for (int j = 0; j < kBatch; ++j)
                 n += v[j];
         }
-        o.recv_expert_count[e] = (n + o.alignment - 1) / o.alignment * o.alignment;
+        o.recv_expert_count[e] = aligned(n, o.alignment);
     }
     // R <= kScanThreads: thread d owns destination d
     int total = 0;
@@ -283,10 +290,15 @@ notify_prefix(const HtNotifyOut &o, int R, int E, const TotalOf &total_of) {
         // exclusive prefix of the per-destination totals in 64 bits
         long long incl = total;
         const int lane = tid & (kWaveSize - 1), wave = tid / kWaveSize;
-#pragma unroll
-        for (int off = 1; off < kWaveSize; off <<= 1) {
+        if (R <= kWaveSize && wave != 0) return; // the first wave has them all
+        for (int off = 1; off < min(R, kWaveSize); off <<= 1) {
             const long long up = __shfl_up(incl, off);
             if (lane >= off) incl += up;
+        }
+        if (R <= kWaveSize) {
+            if (tid < R) o.row_offset[tid + 1] = incl;
+            if (tid == 0) o.row_offset[0] = 0;
+            return;
         }
         // wave totals fit in 32 bits each only if R * T does; check_ht bounds R * T by 2^30
         if (lane == kWaveSize - 1) wave_sums[wave] = static_cast<int>(incl);
@@ -301,7 +313,7 @@ notify_prefix(const HtNotifyOut &o, int R, int E, const TotalOf &total_of) {
 
 __global__ void __launch_bounds__(kScanThreads)
 ht_prefix_kernel(const int *__restrict__ channel_prefix, HtNotifyOut o, int R, int E, int C) {
-    notify_prefix(o, R, E, [&](int r, int d) { return channel_prefix[(static_cast<size_t>(r) * R + d) * C + (C - 1)]; });
+    notify_prefix(o, R, E, 0, [&](int r, int d) { return channel_prefix[(static_cast<size_t>(r) * R + d) * C + (C - 1)]; });
 }
 
 // The same without a launch of its own, for up to 8 ranks: one more workgroup behind those of the
@@ -329,17 +341,55 @@ token_flags(const uint8_t *flags, int t, int R) {
     return f;
 }
 
+// One in every byte of `flags` that is not zero.
+__device__ __forceinline__ unsigned long long
+byte_flags(unsigned long long flags) {
+    constexpr unsigned long long kLow7 = 0x7f7f7f7f7f7f7f7full, kOnes = 0x0101010101010101ull;
+    return ((((flags & kLow7) + kLow7) | flags) >> 7) & kOnes;
+}
+
+// Four bytes as four 16-bit fields.
+__device__ __forceinline__ unsigned long long
+widen_bytes(uint32_t bytes) {
+    unsigned long long x = bytes;
+    x = (x | x << 16) & 0x0000ffff0000ffffull;
+    return (x | x << 8) & 0x00ff00ff00ff00ffull;
+}
+
+// Hits of this thread's share of the tokens before `base` (a multiple of kScanThreads), four loads in flight.
+template<int RANKS>
+__device__ __forceinline__ PackedCounts
+hits_before(const uint8_t *flags, int base, int R) {
+    constexpr int kBatch = 4;
+    PackedCounts n{0, 0};
+    for (int u0 = 0; u0 < base; u0 += kBatch * kScanThreads) {
+        unsigned long long f[kBatch], sum = 0;
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j)
+            f[j] = u0 + j * kScanThreads < base ? token_flags<RANKS>(flags, u0 + j * kScanThreads + threadIdx.x, R) : 0;
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j)
+            sum += byte_flags(f[j]);
+        n.lo += widen_bytes(static_cast<uint32_t>(sum));
+        n.hi += widen_bytes(static_cast<uint32_t>(sum >> 32));
+    }
+    return n;
+}
+
 // RANKS: the number of ranks, or 0 where it is known at run time only.
 template<int RANKS>
 __device__ __forceinline__ void
 notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int n_ranks, int E) {
     const int R = RANKS ? RANKS : n_ranks;
-    __shared__ int hits[kPackedScanRanks * kPackedScanRanks]; // [source][destination]
     constexpr int kWaves = kScanThreads / kWaveSize, kUnit = kWaveSize * kNotifyPerLane;
-    constexpr unsigned long long kLow7 = 0x7f7f7f7f7f7f7f7full, kOnes = 0x0101010101010101ull, kEven = 0x00ff00ff00ff00ffull;
+    constexpr unsigned long long kEven = 0x00ff00ff00ff00ffull;
     const int tid = threadIdx.x, lane = tid & (kWaveSize - 1), wave = tid / kWaveSize;
-    if (tid < kPackedScanRanks * kPackedScanRanks) hits[tid] = 0;
-    __syncthreads();
+    __shared__ int hits[kWaves][kPackedScanRanks]; // what a wave has counted
+    // the counts of the first experts travel while the flags do
+    int of_rank[kPackedScanRanks];
+#pragma unroll
+    for (int r = 0; r < kPackedScanRanks; ++r)
+        if (r < R && tid < E) of_rank[r] = o.per_expert[static_cast<size_t>(r) * E + tid];
     // as many waves to a rank as there are; a wave adds up what it counts in 16-bit fields (T < 65 536)
     const int per_rank = kWaves / R, r = wave / per_rank;
     if (r < R) {
@@ -354,7 +404,7 @@ notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int n_ran
             }
 #pragma unroll
             for (int j = 0; j < kNotifyPerLane; ++j)
-                sum += ((((f[j] & kLow7) + kLow7) | f[j]) >> 7) & kOnes; // one in every byte that is not zero
+                sum += byte_flags(f[j]);
             even += sum & kEven;
             odd += (sum >> 8) & kEven;
         }
@@ -363,10 +413,22 @@ notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int n_ran
             even += __shfl_xor(even, off);
             odd += __shfl_xor(odd, off);
         }
-        if (lane < R) atomicAdd(&hits[r * kPackedScanRanks + lane], static_cast<int>(((lane & 1 ? odd : even) >> (8 * (lane & 6))) & 0xffffu));
+        if (lane < R) hits[wave][lane] = static_cast<int>(((lane & 1 ? odd : even) >> (8 * (lane & 6))) & 0xffffu);
+    }
+    if (tid < E) {
+        int n = 0;
+#pragma unroll
+        for (int r = 0; r < kPackedScanRanks; ++r)
+            if (r < R) n += of_rank[r];
+        o.recv_expert_count[tid] = aligned(n, o.alignment);
     }
     __syncthreads();
-    notify_prefix(o, R, E, [&](int r, int d) { return hits[r * kPackedScanRanks + d]; });
+    notify_prefix(o, R, E, kScanThreads, [&](int r, int d) {
+        int n = 0;
+        for (int w = 0; w < per_rank; ++w)
+            n += hits[r * per_rank + w][d];
+        return n;
+    });
 }
 
 // NOTIFY: the launch has that workgroup.
@@ -402,15 +464,13 @@ ht_scan_packed_kernel(const uint8_t *__restrict__ in_rank,
     PackedCounts hit{0, 0};
     if (t < T) hit = packed_hits(flags, t, R);
     PackedCounts earlier{0, 0};
-    for (int u = tid; u < base; u += kScanThreads) {
-        const PackedCounts h = packed_hits(flags, u, R);
-        earlier.lo += h.lo;
-        earlier.hi += h.hi;
-    }
+    if (base > 0) {
+        earlier = R == 8 ? hits_before<8>(flags, base, R) : R == 4 ? hits_before<4>(flags, base, R) : hits_before<0>(flags, base, R);
 #pragma unroll
-    for (int off = kWaveSize / 2; off > 0; off >>= 1) {
-        earlier.lo += __shfl_xor(earlier.lo, off);
-        earlier.hi += __shfl_xor(earlier.hi, off);
+        for (int off = kWaveSize / 2; off > 0; off >>= 1) {
+            earlier.lo += __shfl_xor(earlier.lo, off);
+            earlier.hi += __shfl_xor(earlier.hi, off);
+        }
     }
     PackedCounts incl = hit; // inclusive scan inside the wave
 #pragma unroll
@@ -485,6 +545,14 @@ struct HtDims {
     int R, T, H, K, E;
 };
 
+// Rows of the ranks before r in destination dst's segment.  The load is there whatever r is: behind a branch the
+// loads around it wait for it, a trip to memory more in front of every row.
+__device__ __forceinline__ int
+rows_before(const int *prefix, const HtDims &d, int r, int dst) {
+    const int n = prefix[dst * d.R + max(r - 1, 0)];
+    return r == 0 ? 0 : n;
+}
+
 __device__ __forceinline__ long long
 recv_row(const int *prefix, const int *send_head, const long long *row_offset, const HtDims &d, int r, int t, int dst) {
     const int seg = r == 0 ? 0 : prefix[dst * d.R + r - 1];
@@ -519,7 +587,7 @@ wave_rows(const uint8_t *in_rank,
     if (EAGER) {
         if (dst < d.R) {
             const uint8_t flag = in_rank[tok * d.R + dst];
-            const int head = send_head[tok * d.R + dst], seg = r == 0 ? 0 : prefix[dst * d.R + r - 1];
+            const int head = send_head[tok * d.R + dst], seg = rows_before(prefix, d, r, dst);
             const long long lo = row_offset[dst], hi = row_offset[dst + 1];
             row = lo + seg + head;
             hit = flag != 0 && row >= lo && row < hi;
@@ -620,6 +688,26 @@ struct HtMeta {
     const float *topk_weights;
 };
 
+// Up to kMaxTopk values in registers, zeroes where there is nothing to load.
+template<bool VEC, typename One, typename Four>
+struct Few {
+    One one[VEC ? 1 : kMaxTopk];
+    Four four[VEC ? kMaxTopk / 4 : 1];
+
+    __device__ __forceinline__ void
+    load(const One *from, int n) {
+        if constexpr (VEC) {
+#pragma unroll
+            for (int k = 0; k < kMaxTopk; k += 4)
+                four[k / 4] = from && k < n ? *reinterpret_cast<const Four *>(from + k) : Four{};
+        } else {
+#pragma unroll
+            for (int k = 0; k < kMaxTopk; ++k)
+                one[k] = from && k < n ? from[k] : One{};
+        }
+    }
+};
+
 template<bool VEC>
 __device__ __forceinline__ void
 meta_block(const HtMeta &m,
@@ -641,32 +729,41 @@ meta_block(const HtMeta &m,
     if (t >= d.T) return;
     const size_t tok = static_cast<size_t>(r) * d.T + t;
     if (!in_rank[tok * d.R + dst]) return;
+    // the token's selections travel beside its row's position, all of them before one is looked at
+    Few<VEC, int, int4> sel;
+    Few<VEC, float, float4> weight;
+    if (recv_topk_idx) {
+        sel.load(topk_idx + tok * d.K, d.K);
+        weight.load(topk_weights ? topk_weights + tok * d.K : nullptr, d.K);
+    }
     const long long row = recv_row(prefix, send_head, row_offset, d, r, t, dst);
     if (row < row_offset[dst] || row >= row_offset[dst + 1]) return;
-    const int El = d.E / d.R;
+    const int lo = dst * (d.E / d.R), hi = lo + d.E / d.R;
     if (VEC && recv_topk_idx) {
         // four selections a step: 16-byte loads and stores (tok*K and row*K are multiples of 4)
-        const int lo = dst * El, hi = lo + El;
-        for (int k = 0; k < d.K; k += 4) {
-            const int4 sel = *reinterpret_cast<const int4 *>(topk_idx + tok * d.K + k);
-            const bool l0 = sel.x >= lo && sel.x < hi, l1 = sel.y >= lo && sel.y < hi;
-            const bool l2 = sel.z >= lo && sel.z < hi, l3 = sel.w >= lo && sel.w < hi;
+#pragma unroll
+        for (int k = 0; k < kMaxTopk; k += 4) {
+            if (k >= d.K) break;
+            const int4 s = sel.four[k / 4];
+            const bool l0 = s.x >= lo && s.x < hi, l1 = s.y >= lo && s.y < hi;
+            const bool l2 = s.z >= lo && s.z < hi, l3 = s.w >= lo && s.w < hi;
             *reinterpret_cast<int4 *>(recv_topk_idx + row * d.K + k) =
-                make_int4(l0 ? sel.x - lo : -1, l1 ? sel.y - lo : -1, l2 ? sel.z - lo : -1, l3 ? sel.w - lo : -1);
+                make_int4(l0 ? s.x - lo : -1, l1 ? s.y - lo : -1, l2 ? s.z - lo : -1, l3 ? s.w - lo : -1);
             if (recv_topk_weights) {
-                float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (topk_weights) w = *reinterpret_cast<const float4 *>(topk_weights + tok * d.K + k);
+                const float4 w = weight.four[k / 4];
                 *reinterpret_cast<float4 *>(recv_topk_weights + row * d.K + k) =
                     make_float4(l0 ? w.x : 0.f, l1 ? w.y : 0.f, l2 ? w.z : 0.f, l3 ? w.w : 0.f);
             }
         }
-    } else if (recv_topk_idx)
-        for (int k = 0; k < d.K; ++k) {
-            const int sel = topk_idx[tok * d.K + k];
-            const bool local = sel >= dst * El && sel < (dst + 1) * El;
-            recv_topk_idx[row * d.K + k] = local ? sel - dst * El : -1;
-            if (recv_topk_weights) recv_topk_weights[row * d.K + k] = local && topk_weights ? topk_weights[tok * d.K + k] : 0.f;
+    } else if (recv_topk_idx) {
+#pragma unroll
+        for (int k = 0; k < kMaxTopk; ++k) {
+            if (k >= d.K) break;
+            const bool local = sel.one[k] >= lo && sel.one[k] < hi;
+            recv_topk_idx[row * d.K + k] = local ? sel.one[k] - lo : -1;
+            if (recv_topk_weights) recv_topk_weights[row * d.K + k] = local ? weight.one[k] : 0.f;
         }
+    }
     if (recv_src_meta) {
         if (VEC) {
             *reinterpret_cast<int2 *>(recv_src_meta + row * 2) = make_int2(r, t);
@@ -721,13 +818,10 @@ scales_block(const HtScales &a,
     const int t0 = (block % blocks_per_pair) * kHtScaleTokens;
     const int tid = threadIdx.x;
     if (tid < kHtScaleTokens) {
-        const int t = t0 + tid;
-        long long row = -1;
-        if (t < d.T && in_rank[(static_cast<size_t>(r) * d.T + t) * d.R + dst]) {
-            row = recv_row(prefix, send_head, row_offset, d, r, t, dst);
-            if (row < row_offset[dst] || row >= row_offset[dst + 1]) row = -1;
-        }
-        rows[tid] = row;
+        const int t = min(t0 + tid, d.T - 1);
+        const uint8_t flag = in_rank[(static_cast<size_t>(r) * d.T + t) * d.R + dst];
+        const long long row = recv_row(prefix, send_head, row_offset, d, r, t, dst);
+        rows[tid] = flag && t == t0 + tid && row >= row_offset[dst] && row < row_offset[dst + 1] ? row : -1;
     }
     __syncthreads();
     const uint32_t *__restrict__ src = scales + static_cast<long long>(r) * rank_stride;
