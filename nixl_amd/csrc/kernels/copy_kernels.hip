@@ -166,14 +166,15 @@ logical_workgroup(uint32_t n_wgs, bool swizzle) {
 // record array stays small next to the payload.
 template<int UPL, int POL, int WAVES>
 __global__ void __launch_bounds__(kWaveSize *WAVES)
-copy_uniform_kernel(const UniformRec *recs, uint32_t first_chunk, uint32_t n_chunks, uint32_t n_wgs, int swizzle, uint32_t chunks_per_rec) {
+copy_uniform_kernel(const UniformRec *recs, uint32_t first_chunk, uint32_t n_chunks, uint32_t n_wgs, int swizzle, FastDiv chunks_per_rec) {
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
     const uint32_t wave = threadIdx.x / kWaveSize;
     const uint32_t wg = logical_workgroup(n_wgs, swizzle != 0);
     if (wg >= n_wgs || wg * WAVES + wave >= n_chunks) return;
     const uint32_t c = uniform(first_chunk + wg * WAVES + wave); // n_chunks, n_wgs: of this launch
-    const uint32_t r = c / chunks_per_rec;
-    const uint64_t off = static_cast<uint64_t>(c % chunks_per_rec) * (kWaveSize * UPL * 16u) + lane * 16u;
+    uint32_t chunk;
+    const uint32_t r = chunks_per_rec.quotient(c, chunk);
+    const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * UPL * 16u) + lane * 16u;
     // The record is the same for every lane and does not change while the kernel runs: read
     // through the constant address space it comes with ONE scalar load (left as an ordinary
     // global access the compiler makes it a 16-byte vector load by all 64 lanes, followed by
@@ -212,9 +213,10 @@ struct InlineRecs {
 
 template<int POL>
 __global__ void __launch_bounds__(kWaveSize)
-copy_inline_kernel(InlineRecs recs, uint32_t chunks_per_rec) {
-    const uint32_t r = blockIdx.x / chunks_per_rec;
-    const uint64_t off = static_cast<uint64_t>(blockIdx.x % chunks_per_rec) * (kWaveSize * 16u) + threadIdx.x * 16u;
+copy_inline_kernel(InlineRecs recs, FastDiv chunks_per_rec) {
+    uint32_t chunk;
+    const uint32_t r = chunks_per_rec.quotient(blockIdx.x, chunk);
+    const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * 16u) + threadIdx.x * 16u;
     store16<POL>(recs.rec[r].dst + off, load16<POL>(recs.rec[r].src + off));
 }
 
@@ -271,7 +273,7 @@ constexpr int kDoneWaves = 8, kDoneChunks = 2; // chunks a wave
 
 template<int POL>
 __global__ void __launch_bounds__(kWaveSize *kDoneWaves)
-copy_inline_done_kernel(InlineRecs recs, uint32_t chunks_per_rec, uint32_t n_chunks, Done done) {
+copy_inline_done_kernel(InlineRecs recs, FastDiv chunks_per_rec, uint32_t n_chunks, Done done) {
     static_assert(POL == kPolPlainSc1Nt || POL == kPolNtSc1Nt);
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
     const uint32_t first = uniform(blockIdx.x * (kDoneWaves * kDoneChunks) + threadIdx.x / kWaveSize);
@@ -281,8 +283,9 @@ copy_inline_done_kernel(InlineRecs recs, uint32_t chunks_per_rec, uint32_t n_chu
     for (int j = 0; j < kDoneChunks; ++j) {
         const uint32_t c = first + j * kDoneWaves;
         if (c >= n_chunks) continue;
-        const uint32_t r = c / chunks_per_rec;
-        const uint64_t off = static_cast<uint64_t>(c % chunks_per_rec) * (kWaveSize * 16u) + lane * 16u;
+        uint32_t chunk;
+        const uint32_t r = chunks_per_rec.quotient(c, chunk);
+        const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * 16u) + lane * 16u;
         to[j] = recs.rec[r].dst + off;
         v[j] = load16<POL>(recs.rec[r].src + off);
     }
@@ -859,7 +862,7 @@ void
 launch_uniform(int waves, const UniformLaunch &u) {
 #define NIXL_AMD_UNIFORM(WV)                                                                              \
     hipLaunchKernelGGL((copy_uniform_kernel<UPL, POL, WV>), u.grid, dim3(kWaveSize * WV), 0, u.stream, u.recs, \
-                       u.first_chunk, u.n_chunks, u.n_wgs, u.swizzle, u.chunks_per_rec)
+                       u.first_chunk, u.n_chunks, u.n_wgs, u.swizzle, FastDiv(u.chunks_per_rec))
     switch (waves) {
     case 1: NIXL_AMD_UNIFORM(1); break;
     case 2: NIXL_AMD_UNIFORM(2); break;
@@ -2722,7 +2725,7 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
         if (slot >= 0 && through && plan->n_uniform <= kToldChunks) {
             const dim3 grid((plan->n_uniform + kDoneWaves * kDoneChunks - 1) / (kDoneWaves * kDoneChunks));
             const auto launch = [&](auto kernel) {
-                hipLaunchKernelGGL(kernel, grid, dim3(kWaveSize * kDoneWaves), 0, s, *plan->inline_recs, plan->chunks_per_rec,
+                hipLaunchKernelGGL(kernel, grid, dim3(kWaveSize * kDoneWaves), 0, s, *plan->inline_recs, FastDiv(plan->chunks_per_rec),
                                    plan->n_uniform, done);
             };
             if (plan->policy == kPolPlainSc1Nt)
@@ -2733,7 +2736,7 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
         } else {
             with_policy(plan->policy, [&]<int POL>() {
                 hipLaunchKernelGGL(copy_inline_kernel<POL>, dim3(plan->n_uniform), dim3(kWaveSize), 0, s, *plan->inline_recs,
-                                   plan->chunks_per_rec);
+                                   FastDiv(plan->chunks_per_rec));
             });
         }
         if (const hipError_t e = hipGetLastError(); e != hipSuccess) return give_up(e);

@@ -641,7 +641,7 @@ struct HtRows {
     const int *send_head;
     const long long *row_offset;
     HtDims d;
-    int parts;
+    FastDiv parts, tokens; // workgroups a row, tokens a rank
     int streamed; // rows are loaded non-temporally
 };
 
@@ -650,9 +650,10 @@ struct HtRows {
 template<bool BY_ROWS>
 __device__ __forceinline__ void
 dispatch_piece(const HtRows &a, uint32_t piece) {
-    const uint32_t token = piece / a.parts, part = piece % a.parts;
+    uint32_t part, t_of_rank;
+    const uint32_t token = a.parts.quotient(piece, part);
     if (token >= static_cast<uint32_t>(a.d.R) * a.d.T) return;
-    const int r = token / a.d.T, t = token % a.d.T;
+    const int r = a.tokens.quotient(token, t_of_rank), t = t_of_rank;
     const int col = part * kWaveSize + (threadIdx.x & (kWaveSize - 1));
     const bool active = col < a.d.H / 8;
     uint4 v = make_uint4(0, 0, 0, 0);
@@ -958,10 +959,11 @@ ht_combine_kernel(uint16_t *__restrict__ combined,
                   const int *__restrict__ send_head,
                   const long long *__restrict__ row_offset,
                   HtDims d,
-                  int parts) {
+                  FastDiv parts,
+                  FastDiv tokens) {
     const int tid = threadIdx.x;
-    const int token = blockIdx.x / parts, part = blockIdx.x % parts;
-    const int r = token / d.T, t = token % d.T;
+    uint32_t part, t_of_rank;
+    const int token = parts.quotient(blockIdx.x, part), r = tokens.quotient(token, t_of_rank), t = t_of_rank;
     const size_t tok = static_cast<size_t>(r) * d.T + t;
     const int col = part * blockDim.x + tid;
     const bool active = col < d.H / 8;
@@ -1238,7 +1240,7 @@ nixl_amd_ep_ht_dispatch_scaled(void *recv_x,
     const long long *offsets = reinterpret_cast<const long long *>(recv_row_offset);
     const int *prefix = recv_gbl_rank_prefix_sum;
     const HtRows rows{static_cast<uint16_t *>(recv_x), static_cast<const uint16_t *>(x), is_token_in_rank, prefix, send_head, offsets, d,
-                      parts, static_cast<long long>(num_ranks) * num_tokens * d.H * 2 > kHtStreamFrom};
+                      FastDiv(parts), FastDiv(num_tokens), static_cast<long long>(num_ranks) * num_tokens * d.H * 2 > kHtStreamFrom};
     const HtMeta meta{recv_topk_idx, recv_topk_weights, recv_src_meta, topk_idx, topk_weights};
     const HtScales sc{static_cast<uint32_t *>(recv_x_scales), static_cast<const uint32_t *>(x_scales), num_scales,
                       num_scales % 4 == 0 && reinterpret_cast<uintptr_t>(recv_x_scales) % 16 == 0, scale_rank_stride,
@@ -1377,7 +1379,7 @@ nixl_amd_ep_ht_combine_rows(void *combined_x,
                        dim3(static_cast<unsigned>(num_ranks) * num_tokens * parts), dim3(lanes), 0, static_cast<hipStream_t>(stream), static_cast<uint16_t *>(combined_x), combined_topk_weights,
                        static_cast<const uint16_t *>(x), topk_weights, static_cast<const uint16_t *>(bias_0),
                        static_cast<const uint16_t *>(bias_1), is_token_in_rank, recv_gbl_rank_prefix_sum, send_head,
-                       reinterpret_cast<const long long *>(recv_row_offset), d, parts);
+                       reinterpret_cast<const long long *>(recv_row_offset), d, FastDiv(parts), FastDiv(num_tokens));
     HIP_TRY(hipGetLastError());
     return NIXL_AMD_OK;
 }

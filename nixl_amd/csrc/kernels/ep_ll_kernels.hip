@@ -92,6 +92,7 @@ struct BitsArgs {
     const int *mask;
     LlDims d;
     int Wr; // words (groups of 64 tokens) per rank
+    FastDiv wgs_per_rank, topk;
     int stamp; // arrival stamp of this call (0 when nobody checks arrivals)
     int call_id; // never 0; header[3] receives it, and header[2] too if some group holds a repeated expert
     int withhold_rank; // this rank's groups leave their stamp out (its counts "never arrive"), or -1
@@ -110,8 +111,8 @@ ll_bits_kernel(BitsArgs a) {
     __shared__ int sel_i[ROUTE ? kTokens : 1][kMaxTopk];
     const LlDims d = a.d;
     const int tid = threadIdx.x, n_threads = blockDim.x;
-    const int per_rank = a.Wr * (kGroupTokens / kTokens); // workgroups per rank
-    const int r = blockIdx.x / per_rank, t0 = (blockIdx.x % per_rank) * kTokens;
+    uint32_t wg;
+    const int r = a.wgs_per_rank.quotient(blockIdx.x, wg), t0 = wg * kTokens;
     const int nt = a.num_tokens_per_rank ? min(a.num_tokens_per_rank[r], d.T) : d.T;
     for (int e = tid; e < d.E; e += n_threads)
         words[e] = 0ull;
@@ -159,9 +160,10 @@ ll_bits_kernel(BitsArgs a) {
 
     const int32_t *idx = a.topk_idx + (static_cast<size_t>(r) * d.T + t0) * d.K;
     for (int p = tid; p < kTokens * d.K; p += n_threads) {
-        const int j = p / d.K;
+        uint32_t k;
+        const int j = a.topk.quotient(p, k);
         if (t0 + j >= nt) break;
-        const int e = ROUTE ? sel_i[j][p % d.K] : idx[p];
+        const int e = ROUTE ? sel_i[j][k] : idx[p];
         if (e < 0 || e >= d.E || pair_blocked(a.mask, d.R, r, e / d.El)) continue;
         const unsigned long long old = atomicOr(&words[e], 1ull << j);
         if ((old >> j) & 1ull) dup = 1; // the same expert twice in one token's selection
@@ -562,7 +564,8 @@ struct DirectArgs {
     int *rows_out;
     LlDims d;
     int round_scale, use_ue8m0;
-    int parts; // workgroups per token
+    FastDiv parts; // workgroups per token
+    FastDiv tokens; // per rank
     int meta_wgs; // workgroups at the front of the grid that derive the metadata of kDirectExperts experts each
 };
 
@@ -625,7 +628,9 @@ ll_direct_kernel(DirectArgs a) {
     }
     const LlDims d = a.d;
     const int tid = threadIdx.x, wlane = tid & (kWaveSize - 1), wave = tid / kWaveSize, n_waves = blockDim.x / kWaveSize;
-    const int wg = blockIdx.x - a.meta_wgs, token = wg / a.parts, part = wg % a.parts;
+    uint32_t part, t_of_rank;
+    const int token = a.parts.quotient(blockIdx.x - a.meta_wgs, part);
+    a.tokens.quotient(token, t_of_rank);
     int sel = wlane < d.K ? a.topk_idx[static_cast<size_t>(token) * d.K + wlane] : -1;
     const int lane = part * blockDim.x + tid; // lane of the token's row
     const bool active = lane < row_lanes<FP8>(d.H);
@@ -674,7 +679,7 @@ ll_direct_kernel(DirectArgs a) {
             row_of_k[wlane] = row;
             if (part == 0) {
                 if (a.rows_out) a.rows_out[static_cast<size_t>(token) * d.K + wlane] = row;
-                if (row >= 0) a.src_info[row] = token % d.T;
+                if (row >= 0) a.src_info[row] = t_of_rank;
             }
         }
     }
@@ -716,12 +721,12 @@ struct ScalesArgs {
     const long long *layout_range; // [E][R]
     LlDims d;
     int use_ue8m0;
-    int parts; // workgroups per expert; each takes every parts-th tile of 64 rows
+    FastDiv quads; // G / 4
 };
 
 constexpr int kScaleThreads = 256;
 constexpr int kScaleTile = 64; // rows per tile
-constexpr int kScaleParts = 4;
+constexpr int kScaleParts = 4; // workgroups per expert; each takes every kScaleParts-th tile
 
 // dynamic LDS: seg_end[R] ints, then tile[64][C + 1] words (C = G, or G / 4 for exponent
 // bytes), then source[64] ints.
@@ -734,7 +739,7 @@ ll_scales_kernel(ScalesArgs a) {
     int *seg_end = lds; // [R]: end of each source rank's segment
     uint32_t *tile = reinterpret_cast<uint32_t *>(lds + d.R); // [64][C + 1]
     int *source = lds + d.R + kScaleTile * (C + 1); // [64]: r * T + t
-    const int e = blockIdx.x / a.parts, part = blockIdx.x % a.parts, tid = threadIdx.x;
+    const int e = blockIdx.x / kScaleParts, part = blockIdx.x % kScaleParts, tid = threadIdx.x;
     const int *info = a.src_info + static_cast<size_t>(e) * d.N;
 
     // the first tile's source tokens are fetched before it is known how many rows exist (in bounds either way)
@@ -748,7 +753,7 @@ ll_scales_kernel(ScalesArgs a) {
     const int n = seg_end[d.R - 1]; // segments follow each other in rank order
     uint32_t *out = static_cast<uint32_t *>(a.recv_scales) + static_cast<size_t>(e) * C * d.N;
 
-    for (; s0 < n; s0 += a.parts * kScaleTile) {
+    for (; s0 < n; s0 += kScaleParts * kScaleTile) {
         const int rows = min(kScaleTile, n - s0);
         if (tid < rows) {
             if (s0 != part * kScaleTile) t_src = info[s0 + tid];
@@ -766,7 +771,8 @@ ll_scales_kernel(ScalesArgs a) {
         // gather: G / 4 lanes per row, 16 bytes each
         const int quads = G / 4;
         for (int i = tid; i < rows * quads; i += kScaleThreads) {
-            const int row = i / quads, q4 = i % quads;
+            uint32_t q4;
+            const int row = a.quads.quotient(i, q4);
             const float4 v = *reinterpret_cast<const float4 *>(a.token_scales + static_cast<size_t>(source[row]) * G + q4 * 4);
             if (!a.use_ue8m0) {
                 uint32_t *dst = tile + row * (C + 1) + q4 * 4;
@@ -814,7 +820,8 @@ struct CombineArgs {
     const int *num_tokens_per_rank;
     const int *row_map; // optional [R][T][K] from dispatch; replaces the search below
     LlDims d;
-    int parts; // workgroups per token; each covers blockDim.x of the token's H/8 lanes
+    FastDiv parts; // workgroups per token; each covers blockDim.x of the token's H/8 lanes
+    FastDiv tokens; // per rank
 };
 
 // LogFMT-10 as the reference's combine sender encodes a row and its receiver decodes it
@@ -859,8 +866,8 @@ ll_combine_kernel(CombineArgs a) {
     const LlDims d = a.d;
     const int tid = threadIdx.x;
     const int lane = tid & (kWaveSize - 1), wave = tid / kWaveSize, n_waves = blockDim.x / kWaveSize;
-    const int token = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
-    const int r = token / d.T, t = token % d.T;
+    uint32_t part, t_of_rank;
+    const int token = a.parts.quotient(blockIdx.x, part), r = a.tokens.quotient(token, t_of_rank), t = t_of_rank;
     const int nt = a.num_tokens_per_rank ? min(a.num_tokens_per_rank[r], d.T) : d.T;
     if (t >= nt) return;
     const int col = part * blockDim.x + tid; // lane of the token's row
@@ -1228,8 +1235,9 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
         const int lanes = c.use_fp8 ? row_lanes<true>(d.H) : row_lanes<false>(d.H);
         const int set = g_dispatch_lanes.load(std::memory_order_relaxed);
         const int most = set ? std::min(kDirectMaxThreads, set) : kDirectMaxThreads;
-        a.parts = (lanes + most - 1) / most;
-        const dim3 grid(static_cast<unsigned>(a.meta_wgs + d.R * d.T * a.parts));
+        a.parts = FastDiv((lanes + most - 1) / most);
+        a.tokens = FastDiv(d.T);
+        const dim3 grid(static_cast<unsigned>(a.meta_wgs + d.R * d.T * a.parts.divisor));
         // as many waves as there may be, also where the row needs one: they share the counting (2048
         // selections, top-16 of 64 experts, call timed with its host work: hidden 512 bf16 52 us with
         // the row's one wave, 31 with four, 26 with eight; hidden 2048 fp8 37, 32, 27)
@@ -1269,6 +1277,8 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
         b.mask = c.mask_buffer;
         b.d = d;
         b.Wr = Wr;
+        b.wgs_per_rank = FastDiv(Wr * (c.logits ? kGroupTokens / kRouteTokens : 1));
+        b.topk = FastDiv(d.K);
         const size_t lds = static_cast<size_t>(d.E) * sizeof(unsigned long long);
         if (c.logits)
             launch_bits<true>((d.E + kWaveSize - 1) / kWaveSize, dim3(static_cast<unsigned>(groups) * (kGroupTokens / kRouteTokens)), lds,
@@ -1350,10 +1360,10 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
         sa.layout_range = reinterpret_cast<const long long *>(c.packed_recv_layout_range);
         sa.d = d;
         sa.use_ue8m0 = c.use_ue8m0;
-        sa.parts = kScaleParts;
+        sa.quads = FastDiv(d.H / 512);
         const int C = c.use_ue8m0 ? d.H / 512 : d.H / 128;
         const size_t lds = (static_cast<size_t>(d.R) + static_cast<size_t>(kScaleTile) * (C + 1) + kScaleTile) * sizeof(int);
-        hipLaunchKernelGGL(ll_scales_kernel, dim3(static_cast<unsigned>(d.E) * sa.parts), dim3(kScaleThreads), lds, s, sa);
+        hipLaunchKernelGGL(ll_scales_kernel, dim3(static_cast<unsigned>(d.E) * kScaleParts), dim3(kScaleThreads), lds, s, sa);
         HIP_TRY(hipGetLastError());
     }
     return NIXL_AMD_OK;
@@ -1562,8 +1572,9 @@ nixl_amd_ep_ll_combine(void *combined_x,
     // the LogFMT codec's arithmetic wants more workgroups still (hidden 7168: 99.6 us with 192 lanes, 105 with 448)
     if (wg == 0) wg = row_lanes <= 512 ? row_lanes : (use_logfmt ? 192 : round_up_wave((d.H / 8 + 1) / 2));
     wg = std::min(row_lanes, wg);
-    a.parts = (d.H / 8 + wg - 1) / wg;
-    const dim3 grid(static_cast<unsigned>(d.R) * d.T * a.parts);
+    a.parts = FastDiv((d.H / 8 + wg - 1) / wg);
+    a.tokens = FastDiv(d.T);
+    const dim3 grid(static_cast<unsigned>(d.R) * d.T * a.parts.divisor);
     if (use_logfmt)
         hipLaunchKernelGGL(ll_combine_kernel<true>, grid, dim3(wg), 0, static_cast<hipStream_t>(stream), a);
     else
