@@ -1015,10 +1015,10 @@ ht_combine_kernel(uint16_t *__restrict__ combined,
     }
     if (active) {
         uint4 out;
-        out.x = f32_to_bf16(acc[0]) | (f32_to_bf16(acc[1]) << 16);
-        out.y = f32_to_bf16(acc[2]) | (f32_to_bf16(acc[3]) << 16);
-        out.z = f32_to_bf16(acc[4]) | (f32_to_bf16(acc[5]) << 16);
-        out.w = f32_to_bf16(acc[6]) | (f32_to_bf16(acc[7]) << 16);
+        out.x = f32_to_bf16_pair(acc[0], acc[1]);
+        out.y = f32_to_bf16_pair(acc[2], acc[3]);
+        out.z = f32_to_bf16_pair(acc[4], acc[5]);
+        out.w = f32_to_bf16_pair(acc[6], acc[7]);
         st16_nt(reinterpret_cast<uint4 *>(combined + tok * d.H) + col, out);
     }
     if (combined_w && weights) combined_w[tok * d.K + tid] = wsum;

@@ -36,7 +36,8 @@
 //
 // Combine is one launch: one workgroup per token locates its K rows through the dispatch
 // handle, reads them once and accumulates in fp32 with fused multiply-adds in top-k order
-// (kernels/nixl_ep_ll.cu:959-1012).  Traffic per token: read K * 2H, write 2H.
+// (kernels/nixl_ep_ll.cu:959-1012).  A small one is bound by its instructions: 8 x 2 tokens x 7168 4.8 us,
+// 3.9 with rows as 32-bit numbers, absent ones marked in LDS, and the conversion in one instruction.  Traffic per token: read K * 2H, write 2H.
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
@@ -49,8 +50,8 @@
 namespace {
 
 constexpr int kBitsThreads = 256; // index path: two (token, k) entries per thread at top-8
-constexpr int kRouteThreads = 1024; // routing path: 16 waves, a token each
-constexpr int kRouteTokens = 16;
+constexpr int kRouteThreads = 512; // routing path: 8 waves, a token each
+constexpr int kRouteTokens = 8;
 constexpr int kGroupTokens = 64; // tokens per word of the selection bits
 constexpr int kMaxTopk = 16; // reference limit, kernels/nixl_ep_ll.cu:412,421
 constexpr int kRouterMaxPerLane = 16; // E <= 1024 when routing
@@ -99,8 +100,10 @@ struct BitsArgs {
 };
 
 // Index path: grid = R * Wr workgroups, one per word (64 tokens).  Routing path: grid =
-// R * Wr * 4 workgroups, one per quarter word (16 tokens, a wave each), so that the routing
-// runs as wide as a token-per-wave router; a quarter is written as its own 16-bit word.
+// R * Wr * 8 workgroups, one per byte of a word (8 tokens, a wave each).  What bounds the routing is
+// the instructions of its rounds: with 16 waves a workgroup four of them share a SIMD while most of the
+// chip has none (16 x 61 tokens, top-6 of 64 experts, 5.5 us and 4.6 with 8; 8 x 64 top-8 of 256 7.3 and
+// 5.9; 32 x 128, which fills the chip either way, 7.6 and 7.6).
 // Dynamic LDS: E words.
 template<bool ROUTE, int PL>
 __global__ void __launch_bounds__(ROUTE ? kRouteThreads : kBitsThreads)
@@ -108,7 +111,6 @@ ll_bits_kernel(BitsArgs a) {
     constexpr int kTokens = ROUTE ? kRouteTokens : kGroupTokens; // tokens of this workgroup
     extern __shared__ unsigned long long words[]; // [E]
     __shared__ int dup;
-    __shared__ int sel_i[ROUTE ? kTokens : 1][kMaxTopk];
     const LlDims d = a.d;
     const int tid = threadIdx.x, n_threads = blockDim.x;
     uint32_t wg;
@@ -121,16 +123,17 @@ ll_bits_kernel(BitsArgs a) {
     if constexpr (ROUTE) {
         // K rounds of a wave-wide argmax per token; lane l holds experts l, l + 64, ...
         const int lane = tid & (kWaveSize - 1), j = tid / kWaveSize;
-        if (t0 + j < d.T) {
-            const float *row = a.logits + (static_cast<size_t>(r) * d.T + t0 + j) * d.E;
-            float v[PL];
-            unsigned taken = 0;
+        const bool here = t0 + j < d.T;
+        float v[PL];
+        unsigned taken = 0;
 #pragma unroll
-            for (int q = 0; q < PL; ++q) {
-                const int e = q * kWaveSize + lane;
-                v[q] = e < d.E ? row[e] : 0.f;
-                if (e >= d.E) taken |= 1u << q;
-            }
+        for (int q = 0; q < PL; ++q) {
+            const int e = q * kWaveSize + lane;
+            v[q] = here && e < d.E ? a.logits[(static_cast<size_t>(r) * d.T + t0 + j) * d.E + e] : 0.f;
+            if (e >= d.E) taken |= 1u << q;
+        }
+        __syncthreads(); // the words are clear; while the logits travel
+        if (here) {
             float mine = 0.f, first = 0.f; // lane k keeps the k-th selected logit
             int mine_i = 0;
             for (int k = 0; k < d.K; ++k) {
@@ -143,37 +146,38 @@ ll_bits_kernel(BitsArgs a) {
                     mine_i = win;
                 }
             }
-            // softmax over the K selected logits, summed in selection order by lane 0
+            // the wave's own bit of its experts' words: nobody else has to look at what it selected
+            if (lane < d.K && t0 + j < nt && mine_i < d.E && !pair_blocked(a.mask, d.R, r, mine_i / d.El))
+                atomicOr(&words[mine_i], 1ull << j);
+            // softmax over the K selected logits, summed in selection order
             const float ex = lane < d.K ? expf(mine - first) : 0.f;
             float sum = 0.f;
             for (int k = 0; k < d.K; ++k)
-                sum += __shfl(ex, k);
+                sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ex), k));
             if (lane < d.K) {
                 const size_t at = (static_cast<size_t>(r) * d.T + t0 + j) * d.K + lane;
                 a.topk_idx[at] = mine_i;
                 a.topk_weights[at] = ex / sum;
-                sel_i[j][lane] = mine_i;
             }
         }
-    }
-    __syncthreads();
-
-    const int32_t *idx = a.topk_idx + (static_cast<size_t>(r) * d.T + t0) * d.K;
-    for (int p = tid; p < kTokens * d.K; p += n_threads) {
-        uint32_t k;
-        const int j = a.topk.quotient(p, k);
-        if (t0 + j >= nt) break;
-        const int e = ROUTE ? sel_i[j][k] : idx[p];
-        if (e < 0 || e >= d.E || pair_blocked(a.mask, d.R, r, e / d.El)) continue;
-        const unsigned long long old = atomicOr(&words[e], 1ull << j);
-        if ((old >> j) & 1ull) dup = 1; // the same expert twice in one token's selection
+    } else {
+        __syncthreads();
+        const int32_t *idx = a.topk_idx + (static_cast<size_t>(r) * d.T + t0) * d.K;
+        for (int p = tid; p < kTokens * d.K; p += n_threads) {
+            const int j = a.topk.quotient(p);
+            if (t0 + j >= nt) break;
+            const int e = idx[p];
+            if (e < 0 || e >= d.E || pair_blocked(a.mask, d.R, r, e / d.El)) continue;
+            const unsigned long long old = atomicOr(&words[e], 1ull << j);
+            if ((old >> j) & 1ull) dup = 1; // the same expert twice in one token's selection
+        }
     }
     __syncthreads();
     const size_t W = static_cast<size_t>(d.R) * a.Wr;
     if constexpr (ROUTE) {
-        auto *quarters = reinterpret_cast<unsigned short *>(a.bits);
+        auto *eighths = reinterpret_cast<uint8_t *>(a.bits);
         for (int e = tid; e < d.E; e += n_threads)
-            quarters[e * W * (kGroupTokens / kTokens) + blockIdx.x] = static_cast<unsigned short>(words[e]);
+            eighths[e * W * (kGroupTokens / kTokens) + blockIdx.x] = static_cast<uint8_t>(words[e]);
     } else {
         for (int e = tid; e < d.E; e += n_threads)
             a.bits[e * W + blockIdx.x] = words[e];
@@ -421,13 +425,13 @@ scale_word(float scale_inv, bool use_ue8m0) {
     return word;
 }
 
-// Writes a lane's word to its column of `row` = e * N + slot; lanes that hold no word do nothing.
+// Writes a lane's word to its column of row `slot` of expert `e`; lanes that hold no word do nothing.
 __device__ __forceinline__ void
-store_scale(void *recv_scales, const LlDims &d, bool use_ue8m0, int row, int lane, uint32_t word) {
+store_scale(void *recv_scales, const LlDims &d, bool use_ue8m0, int e, int slot, int lane, uint32_t word) {
     const int shift = use_ue8m0 ? 5 : 3; // lanes per word
     if (lane & ((1 << shift) - 1)) return;
-    const int e = row / d.N, columns = d.H / 16 >> shift;
-    static_cast<uint32_t *>(recv_scales)[(static_cast<size_t>(e) * columns + (lane >> shift)) * d.N + (row - e * d.N)] = word;
+    const int columns = d.H / 16 >> shift;
+    static_cast<uint32_t *>(recv_scales)[(static_cast<size_t>(e) * columns + (lane >> shift)) * d.N + slot] = word;
 }
 
 // grid = R*T*parts workgroups.  A lane stores 16 bytes of every row, so that the stores of a
@@ -528,8 +532,10 @@ ll_dispatch_kernel(DispatchArgs a) {
         if (row < 0) continue;
         if (lane == 0) a.src_info[row] = t;
         if (active) st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
-        if constexpr (SCALES)
-            if (active) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, row, lane, word);
+        if constexpr (SCALES) {
+            const int e = __builtin_amdgcn_readlane(sel, k);
+            if (active) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, e, row - e * d.N, lane, word);
+        }
     }
     if constexpr (!FP8) {
         if (!repeats) return;
@@ -547,7 +553,9 @@ ll_dispatch_kernel(DispatchArgs a) {
 // A decode step with few tokens is launches and dependent round trips, not bytes.  While all
 // selections of the world fit in a few KiB, a token's rows can be counted from topk_idx itself:
 // every workgroup scans the selections in front of its own (a ballot and a bit count per
-// selection it looks for), so nothing has to be prepared by a kernel before this one, a repeated
+// selection it looks for), and every wave of it adds up what the waves counted (8 x 2 tokens x 7168
+// 6.2 us where the first wave does so for the others and every scale divides its row by N again,
+// 5.3 so), so nothing has to be prepared by a kernel before this one, a repeated
 // expert needs no special case (every selection counts), and the scales go straight to their
 // column-major places, since there are too few of them for the isolated words to matter.
 // The first workgroups of the grid derive the receive-side metadata from the same scan.
@@ -621,7 +629,6 @@ template<bool FP8, int KP>
 __global__ void __launch_bounds__(kDirectMaxThreads)
 ll_direct_kernel(DirectArgs a) {
     __shared__ int counted[kDirectMaxThreads / kWaveSize][KP];
-    __shared__ int row_of_k[KP];
     if (static_cast<int>(blockIdx.x) < a.meta_wgs) {
         direct_meta(a, blockIdx.x * kDirectExperts);
         return;
@@ -666,31 +673,30 @@ ll_direct_kernel(DirectArgs a) {
             counted[wave][k] = cnt[k];
     float scale_inv = 0.f;
     if constexpr (FP8) raw0 = quantise_group(raw0, raw1, a.round_scale != 0, scale_inv);
-    __syncthreads();
-    if (wave == 0) {
-        // this token's own selections of the same expert come in selection order
-        int slot = 0;
-        for (int k = 0; k < d.K; ++k)
-            slot += k < wlane && __builtin_amdgcn_readlane(sel, k) == sel;
-        if (wlane < d.K) {
-            for (int w = 0; w < n_waves; ++w)
-                slot += counted[w][wlane];
-            const int row = sel != kNone && slot < d.N ? sel * d.N + slot : -1; // beyond N only through repeats: dropped
-            row_of_k[wlane] = row;
-            if (part == 0) {
-                if (a.rows_out) a.rows_out[static_cast<size_t>(token) * d.K + wlane] = row;
-                if (row >= 0) a.src_info[row] = t_of_rank;
-            }
-        }
-    }
-    __syncthreads();
     [[maybe_unused]] uint32_t word = 0;
     if constexpr (FP8) word = scale_word(scale_inv, a.use_ue8m0 != 0);
-    for (int k = 0; k < d.K; ++k) {
-        const int row = row_of_k[k];
-        if (row < 0 || !active) continue;
-        st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
-        if constexpr (FP8) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, row, lane, word);
+    __syncthreads();
+    // Every wave finds the rows for itself, lane k that of selection k: the selections in front of the
+    // token's, and its own of the same expert, which come in selection order.
+    int slot = 0;
+#pragma unroll
+    for (int w = 0; w < kDirectMaxThreads / kWaveSize; ++w)
+        if (w < n_waves) slot += counted[w][wlane & (KP - 1)];
+#pragma unroll
+    for (int k = 0; k < KP; ++k)
+        slot += k < wlane && want[k] == sel;
+    const int row = sel != kNone && slot < d.N ? sel * d.N + slot : -1; // beyond N only through repeats: dropped
+    if (wave == 0 && part == 0 && wlane < d.K) {
+        if (a.rows_out) a.rows_out[static_cast<size_t>(token) * d.K + wlane] = row;
+        if (row >= 0) a.src_info[row] = t_of_rank;
+    }
+    if (!active) return;
+#pragma unroll
+    for (int k = 0; k < KP; ++k) {
+        const int at = __builtin_amdgcn_readlane(row, k); // -1 from K on
+        if (at < 0) continue;
+        st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(at) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
+        if constexpr (FP8) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, want[k], at - want[k] * d.N, lane, word);
     }
 }
 
@@ -871,26 +877,27 @@ ll_combine_kernel(CombineArgs a) {
     const int nt = a.num_tokens_per_rank ? min(a.num_tokens_per_rank[r], d.T) : d.T;
     if (t >= nt) return;
     const int col = part * blockDim.x + tid; // lane of the token's row
-    __shared__ long long row_of_k[kMaxTopk];
-    __shared__ float weight_of_k[kMaxTopk];
+    __shared__ __align__(16) int row_of_k[kMaxTopk]; // -1 from K on
+    __shared__ __align__(16) float weight_of_k[kMaxTopk];
+    if (tid >= d.K && tid < kMaxTopk) row_of_k[tid] = -1;
 
     if (a.row_map) {
         // Rows recorded by dispatch: one load per selection instead of a search.
         if (tid < d.K) {
             const size_t sel = (static_cast<size_t>(r) * d.T + t) * d.K + tid;
-            const int e = a.topk_idx[sel];
-            long long row = a.row_map[sel];
+            int e = a.topk_idx[sel], row = a.row_map[sel];
+            float weight = a.topk_weights[sel];
             if (e < 0 || e >= d.E || pair_blocked(a.mask, d.R, r, e / d.El)) row = -1;
-            if (row >= static_cast<long long>(d.E) * d.N) row = -1; // a foreign handle must not make the kernel fault
+            if (static_cast<unsigned>(row) >= static_cast<unsigned>(d.E) * d.N) row = -1; // a foreign handle must not make the kernel fault
             row_of_k[tid] = row;
-            weight_of_k[tid] = a.topk_weights[sel];
+            weight_of_k[tid] = weight;
         }
     } else
     // Locate the K rows: wave w searches selections w, w + n_waves, ...
     for (int k = wave; k < d.K; k += n_waves) {
         const size_t sel = (static_cast<size_t>(r) * d.T + t) * d.K + k;
         const int e = a.topk_idx[sel];
-        long long row = -1;
+        int row = -1;
         if (e >= 0 && e < d.E && !pair_blocked(a.mask, d.R, r, e / d.El)) {
             const long long lr = a.layout_range[static_cast<size_t>(e) * d.R + r];
             int n = static_cast<int>(lr & 0xffffffffll), begin = static_cast<int>(lr >> 32);
@@ -901,7 +908,7 @@ ll_combine_kernel(CombineArgs a) {
                 const int i = i0 + lane;
                 const bool hit = i < n && seg[i] == t;
                 const unsigned long long m = __ballot(hit);
-                if (m) row = static_cast<long long>(e) * d.N + begin + i0 + (__ffsll(static_cast<long long>(m)) - 1);
+                if (m) row = e * d.N + begin + i0 + (__ffsll(static_cast<long long>(m)) - 1);
             }
         }
         if (lane == 0) {
@@ -917,14 +924,14 @@ ll_combine_kernel(CombineArgs a) {
         uint4 v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const long long row = (k0 + j < d.K) ? row_of_k[k0 + j] : -1;
+            const int row = row_of_k[k0 + j];
             v[j] = make_uint4(0, 0, 0, 0);
             if (row >= 0)
                 v[j] = ld16_nt(reinterpret_cast<const uint4 *>(a.x + static_cast<size_t>(row) * d.H) + col);
         }
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            if (k0 + j >= d.K || row_of_k[k0 + j] < 0) continue;
+            if (row_of_k[k0 + j] < 0) continue;
             const float w = weight_of_k[k0 + j];
             const uint32_t u[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
             if constexpr (LOGFMT) {
@@ -950,10 +957,10 @@ ll_combine_kernel(CombineArgs a) {
         }
     }
     uint4 out;
-    out.x = f32_to_bf16(acc[0]) | (f32_to_bf16(acc[1]) << 16);
-    out.y = f32_to_bf16(acc[2]) | (f32_to_bf16(acc[3]) << 16);
-    out.z = f32_to_bf16(acc[4]) | (f32_to_bf16(acc[5]) << 16);
-    out.w = f32_to_bf16(acc[6]) | (f32_to_bf16(acc[7]) << 16);
+    out.x = f32_to_bf16_pair(acc[0], acc[1]);
+    out.y = f32_to_bf16_pair(acc[2], acc[3]);
+    out.z = f32_to_bf16_pair(acc[4], acc[5]);
+    out.w = f32_to_bf16_pair(acc[6], acc[7]);
     st16_nt(reinterpret_cast<uint4 *>(a.combined + (static_cast<size_t>(r) * d.T + t) * d.H) + col, out);
 }
 

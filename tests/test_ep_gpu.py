@@ -1670,3 +1670,41 @@ def test_large_combine_of_many_ranks_does_not_load_every_position(cuda):
         assert rc == 0, _lib.kernels_error()
         took.setdefault(stated, []).append(e0.elapsed_time(e1))
     assert np.median(took[rows.shape[0]]) < 1.2 * np.median(took[5 * R * T]), took
+
+
+@pytest.mark.parametrize("weight", [1.0, 1.00390625, -0.3])  # the second puts products halfway between two bf16 values
+def test_combine_rounds_every_bf16_value_to_nearest_even(cuda, weight):
+    """One row a token, so that a result is one product rounded once: bit for bit what torch rounds to on the CPU."""
+    H, T, E = 8192, 8, 8
+    buf = Buffer(1, device=cuda)
+    topk = torch.arange(T, dtype=torch.int32, device=cuda).view(1, T, 1)
+    _, _, handle, _, _ = buf.dispatch(torch.zeros(1, T, H, dtype=torch.bfloat16, device=cuda), topk, T, E, use_fp8=False)
+    values = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(T, H)
+    y = torch.zeros(1, E, T, H, dtype=torch.int16)
+    y[0, :, 0] = values  # expert t's first row is token t's
+    w = torch.full((1, T, 1), weight, dtype=torch.float32, device=cuda)
+    got = buf.combine(y.view(torch.bfloat16).to(cuda), topk, w, handle)[0][0].cpu()
+    want = (values.view(torch.bfloat16).float() * weight + 0.0).to(torch.bfloat16)
+    assert torch.equal(got.isnan(), want.isnan())
+    nan = want.isnan()
+    assert torch.equal(got.view(torch.int16)[~nan], want.view(torch.int16)[~nan])
+
+
+@pytest.mark.parametrize("T", [1, 7, 8, 9, 63, 64, 65])
+@pytest.mark.parametrize("E, K", [(32, 2), (192, 8)])
+def test_route_dispatch_is_route_and_dispatch_at_the_edges_of_its_workgroups(cuda, T, E, K):
+    """Eight tokens a workgroup write a byte of their group's word: around the edges of both, with ranks that own fewer."""
+    R, H = 4, 512
+    gen = torch.Generator(device=cuda).manual_seed(T * E + K)
+    x = torch.randn((R, T, H), generator=gen, device=cuda).to(torch.bfloat16)
+    logits = torch.randn((R, T, E), generator=gen, device=cuda)
+    owned = torch.tensor([T, 0, (T + 1) // 2, T - 1], dtype=torch.int32, device=cuda)
+    buf = Buffer(R, device=cuda)
+    idx, weights = buf.route(logits, K)
+    recv, count, handle, _, _ = buf.dispatch(x, idx, T, E, use_fp8=False, num_tokens_per_rank=owned)
+    idx2, weights2, recv2, count2, handle2, _, _ = buf.route_dispatch(x, logits, K, T, use_fp8=False, num_tokens_per_rank=owned)
+    assert torch.equal(idx, idx2) and torch.equal(weights, weights2)
+    assert torch.equal(count, count2) and torch.equal(handle[1], handle2[1]) and torch.equal(handle.row_map, handle2.row_map)
+    assert int(count.sum()) == int(owned.sum()) * K
+    for rows, rows2, src, src2, n in zip(recv.flatten(0, 1), recv2.flatten(0, 1), handle[0].flatten(0, 1), handle2[0].flatten(0, 1), count.flatten()):
+        assert torch.equal(rows[:n], rows2[:n]) and torch.equal(src[:n], src2[:n])
