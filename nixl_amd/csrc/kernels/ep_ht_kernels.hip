@@ -81,11 +81,13 @@ layout_kernel(const int32_t *__restrict__ topk_idx,
               int T,
               int K,
               int R,
-              int E) {
+              int E,
+              FastDiv chunks,
+              FastDiv of_rank) { // experts of a rank
     extern __shared__ int counters[]; // [E] experts, then [R] ranks
-    const int chunks = (T + blockDim.x - 1) / blockDim.x;
-    const int src = blockIdx.x / chunks, El = E / R;
-    const int t = (blockIdx.x % chunks) * blockDim.x + threadIdx.x;
+    uint32_t chunk;
+    const int src = chunks.quotient(blockIdx.x, chunk);
+    const int t = chunk * blockDim.x + threadIdx.x;
     for (int i = threadIdx.x; i < E + R; i += blockDim.x)
         counters[i] = 0;
     __syncthreads();
@@ -101,14 +103,12 @@ layout_kernel(const int32_t *__restrict__ topk_idx,
                 const int e = sel[k];
                 if (e < 0 || e >= E) continue;
                 atomicAdd(&counters[e], 1);
-                mask |= 1ull << (e / El);
+                mask |= 1ull << of_rank.quotient(e);
             }
             if (word_flags) {
-                unsigned long long bytes = 0;
-#pragma unroll
-                for (int d = 0; d < 8; ++d)
-                    bytes |= ((mask >> d) & 1ull) << (8 * d);
-                *reinterpret_cast<unsigned long long *>(flags) = bytes;
+                // bit d to byte d: a copy of the bits in every byte, its own one of them, and that to the last place
+                const unsigned long long own = (mask * 0x0101010101010101ull) & 0x8040201008040201ull;
+                *reinterpret_cast<unsigned long long *>(flags) = ((own + 0x7f7f7f7f7f7f7f7full) >> 7) & 0x0101010101010101ull;
             } else {
                 for (int d = 0; d < R; ++d)
                     flags[d] = static_cast<uint8_t>((mask >> d) & 1ull);
@@ -125,14 +125,14 @@ layout_kernel(const int32_t *__restrict__ topk_idx,
                 const int e = sel[k];
                 if (e < 0 || e >= E) continue;
                 atomicAdd(&counters[e], 1);
-                flags[e / El] = 1;
+                flags[of_rank.quotient(e)] = 1;
             }
             for (int d = 0; d < R; ++d)
                 if (flags[d]) atomicAdd(&counters[E + d], 1);
         }
     }
     __syncthreads();
-    if (chunks == 1) {
+    if (chunks.divisor == 1) {
         for (int i = threadIdx.x; i < E; i += blockDim.x)
             per_expert[static_cast<size_t>(src) * E + i] = counters[i];
         for (int i = threadIdx.x; i < R; i += blockDim.x)
@@ -227,6 +227,16 @@ packed_hits(const uint8_t *flags, int t, int R) {
         }
     }
     return hit;
+}
+
+// Four dwords of two fields each; the upper two only where there are more than four ranks.
+template<typename Op>
+__device__ __forceinline__ PackedCounts
+each_half(const PackedCounts &c, bool upper, const Op &op) {
+    const auto both = [&](unsigned long long x) {
+        return static_cast<unsigned long long>(op(static_cast<uint32_t>(x >> 32))) << 32 | op(static_cast<uint32_t>(x));
+    };
+    return {both(c.lo), upper ? both(c.hi) : 0ull};
 }
 
 // ---- notify, part 2: receive-side prefix over source ranks, aligned per-expert counts
@@ -408,11 +418,9 @@ notify_from_flags(const uint8_t *in_rank, const HtNotifyOut &o, int T, int n_ran
             even += sum & kEven;
             odd += (sum >> 8) & kEven;
         }
-#pragma unroll
-        for (int off = kWaveSize / 2; off > 0; off >>= 1) {
-            even += __shfl_xor(even, off);
-            odd += __shfl_xor(odd, off);
-        }
+        const PackedCounts sums = each_half(PackedCounts{even, odd}, true, wave_sum_dpp);
+        even = sums.lo;
+        odd = sums.hi;
         if (lane < R) hits[wave][lane] = static_cast<int>(((lane & 1 ? odd : even) >> (8 * (lane & 6))) & 0xffffu);
     }
     if (tid < E) {
@@ -466,21 +474,9 @@ ht_scan_packed_kernel(const uint8_t *__restrict__ in_rank,
     PackedCounts earlier{0, 0};
     if (base > 0) {
         earlier = R == 8 ? hits_before<8>(flags, base, R) : R == 4 ? hits_before<4>(flags, base, R) : hits_before<0>(flags, base, R);
-#pragma unroll
-        for (int off = kWaveSize / 2; off > 0; off >>= 1) {
-            earlier.lo += __shfl_xor(earlier.lo, off);
-            earlier.hi += __shfl_xor(earlier.hi, off);
-        }
+        earlier = each_half(earlier, R > 4, wave_sum_dpp);
     }
-    PackedCounts incl = hit; // inclusive scan inside the wave
-#pragma unroll
-    for (int off = 1; off < kWaveSize; off <<= 1) {
-        const unsigned long long ulo = __shfl_up(incl.lo, off), uhi = __shfl_up(incl.hi, off);
-        if (lane >= off) {
-            incl.lo += ulo;
-            incl.hi += uhi;
-        }
-    }
+    PackedCounts incl = each_half(hit, R > 4, wave_scan_dpp); // inside the wave
     if (lane == kWaveSize - 1) wave_sums[wave] = incl;
     if (lane == 0) wave_before[wave] = earlier;
     __syncthreads();
@@ -492,20 +488,8 @@ ht_scan_packed_kernel(const uint8_t *__restrict__ in_rank,
             s = wave_sums[lane];
             e = wave_before[lane];
         }
-        PackedCounts run = s;
-#pragma unroll
-        for (int off = 1; off < kWaves; off <<= 1) {
-            const unsigned long long ulo = __shfl_up(run.lo, off), uhi = __shfl_up(run.hi, off);
-            if (lane >= off) {
-                run.lo += ulo;
-                run.hi += uhi;
-            }
-        }
-#pragma unroll
-        for (int off = kWaves / 2; off > 0; off >>= 1) {
-            e.lo += __shfl_xor(e.lo, off);
-            e.hi += __shfl_xor(e.hi, off);
-        }
+        const PackedCounts run = each_half(s, R > 4, wave_scan_dpp); // lanes beyond the waves add nothing
+        e = each_half(e, R > 4, wave_sum_dpp);
         if (lane < kWaves) wave_sums[lane] = PackedCounts{run.lo - s.lo + e.lo, run.hi - s.hi + e.hi};
         if (lane == kWaves - 1) wave_before[0] = PackedCounts{run.lo + e.lo, run.hi + e.hi};
     }
@@ -1114,7 +1098,7 @@ nixl_amd_ep_get_dispatch_layout(const int32_t *topk_idx,
     if (num_tokens <= kLayoutWhole && num_tokens * num_topk <= kLayoutWholeSelections && flags_fit) {
         hipLaunchKernelGGL(layout_kernel, dim3(static_cast<unsigned>(num_ranks)), dim3(round_up_wave(num_tokens)), lds, s, topk_idx,
                            num_tokens_per_rank, num_tokens_per_expert, is_token_in_rank, num_tokens, num_topk, num_ranks,
-                           num_experts);
+                           num_experts, FastDiv(1), FastDiv(num_experts / num_ranks));
         HIP_TRY(hipGetLastError());
         return NIXL_AMD_OK;
     }
@@ -1127,7 +1111,7 @@ nixl_amd_ep_get_dispatch_layout(const int32_t *topk_idx,
     const long long chunks = (num_tokens + kLayoutTokens - 1) / kLayoutTokens;
     hipLaunchKernelGGL(layout_kernel, dim3(static_cast<unsigned>(num_ranks * chunks)), dim3(kLayoutTokens), lds, s, topk_idx,
                        num_tokens_per_rank, num_tokens_per_expert, is_token_in_rank, num_tokens, num_topk, num_ranks,
-                       num_experts);
+                       num_experts, FastDiv(static_cast<uint32_t>(chunks)), FastDiv(num_experts / num_ranks));
     HIP_TRY(hipGetLastError());
     return NIXL_AMD_OK;
 }
