@@ -331,10 +331,10 @@ ht_prefix_kernel(const int *__restrict__ channel_prefix, HtNotifyOut o, int R, i
 // workgroup's way to flags that another kernel has just written, so every wave has a share of a
 // rank's tokens, eight loads in flight a lane, and counts bytes (eight destinations an addition)
 // that are widened once a step.  Up to so many tokens that the one workgroup is not slower than the
-// launch (layout, scan and this behind one another, one launch and two, us): 8 x 1024 tokens 9.6 and
-// 12.7, 8 x 4096 15.0 and 16.0, 8 x 6000 17.5 and 17.3; 4 x 16 384 19.3 and 22.0.  Where a token's
-// flags are no word that one load takes: 6 x 300 11.5 and 11.6, 6 x 600 14.0 and 12.5.
-constexpr int kNotifyTokensOf8 = 40960, kNotifyTokensOf4 = 65536; // R * T
+// launch (layout, scan and this behind one another, one launch and two, us): 8 x 1024 tokens 8.0 and
+// 10.5, 8 x 5120 13.5 and 14.3, 8 x 6000 14.5 and 13.0; 4 x 12 288 13.9 and 14.6, 4 x 16 384 16.2 and 15.7. Where a
+// token's flags are no word that one load takes: 7 x 250 10.9 and 11.8, 6 x 600 13.3 and 10.2.
+constexpr int kNotifyTokensOf8 = 40960, kNotifyTokensOf4 = 57344; // R * T
 constexpr int kNotifyFlags = 12288; // R * T * R, other numbers of ranks
 constexpr int kNotifyPerLane = 8; // tokens a lane counts at a time, their loads together
 

@@ -1168,11 +1168,14 @@ launch_bits(int per_lane, dim3 grid, size_t lds, hipStream_t s, const BitsArgs &
 }
 
 // Calls that ll_direct_kernel takes: few selections in all, and nothing that only the selection
-// bits know about (masked ranks, ragged ranks, separate phases and their time-outs).  GPU time of
-// a dispatch with hidden 7168, top-8 of 256 experts, fp8, one launch against two (bits and rows,
-// scales written by the rows): 128 selections 6.1 us against 11.5, 2048: 10.2 against 10.9, 4096:
-// 19.5 against 14.2 (every workgroup reads all selections in front of its own).
-constexpr int kDirectSelections = 2048;
+// bits know about (masked ranks, ragged ranks, separate phases and their time-outs).  Dispatches one behind
+// another with hidden 7168, top-8 of 256 experts, fp8, one launch against two (bits and rows,
+// scales written by the rows): 128 selections 4.5 us against 10.4, 2048: 7.9 against 9.9, 3072: 9.9 against 12.1,
+// 4096: 13.8 against 12.8 (every workgroup reads all selections in front of its own).  Beyond 2048 that
+// needs four of a token: top-4 8 x 96 x 4096 7.5 against 9.0, top-16 8 x 24 x 512 10.0 against 12.2, but
+// top-2 8 x 192 x 2048, twice the workgroups, 10.2 against 8.4.  With logits the routing is a launch
+// of its own in front of this one and part of the bits' otherwise.
+constexpr int kDirectSelections = 2048, kDirectSelectionsMany = 3072, kDirectManyTopk = 4;
 // Up to this many words of scales the row kernel writes them itself, one isolated word at a time,
 // which spares the third launch; beyond it ll_scales_kernel moves them through LDS tiles.  Two
 // launches against three: 1024 tokens x top-8 x 56 words (459 thousand) 21.6 us against 26.4, 524
@@ -1181,7 +1184,8 @@ constexpr long long kIsolatedScaleWords = 1 << 19;
 
 bool
 direct_fits(const LlDispatchCall &c, const LlDims &d) {
-    return d.T > 0 && static_cast<long long>(d.R) * d.T * d.K <= kDirectSelections && d.R <= kDirectMaxRanks && !c.mask_buffer &&
+    const int most = d.K >= kDirectManyTopk && !c.logits ? kDirectSelectionsMany : kDirectSelections;
+    return d.T > 0 && static_cast<long long>(d.R) * d.T * d.K <= most && d.R <= kDirectMaxRanks && !c.mask_buffer &&
         !c.num_tokens_per_rank && c.phases == 3 && c.timeout_us == 0;
 }
 

@@ -1708,3 +1708,41 @@ def test_route_dispatch_is_route_and_dispatch_at_the_edges_of_its_workgroups(cud
     assert int(count.sum()) == int(owned.sum()) * K
     for rows, rows2, src, src2, n in zip(recv.flatten(0, 1), recv2.flatten(0, 1), handle[0].flatten(0, 1), handle2[0].flatten(0, 1), count.flatten()):
         assert torch.equal(rows[:n], rows2[:n]) and torch.equal(src[:n], src2[:n])
+
+
+@pytest.mark.parametrize("shape,form", [
+    # 3072 selections of four and more a token take one launch, a token more takes two, and so do 3072 of three a token
+    ((4, 96, 512, 8, 24, 96), "fp8"), ((4, 97, 512, 8, 24, 97), "fp8"), ((8, 96, 1024, 4, 8, 96), "ue8m0"), ((8, 97, 1024, 4, 8, 97), "bf16"),
+    ((2, 96, 8192, 16, 34, 96), "bf16"), ((64, 12, 512, 4, 64, 12), "fp8"), ((8, 128, 512, 3, 24, 128), "fp8"),
+])
+def test_ll_dispatch_forms_at_the_line_of_many_selections_a_token(cuda, shape, form):
+    test_ll_dispatch_forms_by_size(cuda, shape, form)
+
+
+def test_layout_and_notify_of_every_number_of_ranks(cuda):
+    """Both forms of notify (four ranks: the line is at 57 344 tokens) and chunks of 1024 tokens, with empty ranks among
+    the destinations: counts, offsets, positions and prefixes from the flags, on the CPU."""
+    for R, T, K in ((1, 1, 1), (1, 2049, 1), (2, 1023, 2), (3, 1025, 3), (4, 333, 6), (4, 14336, 2), (4, 14337, 2), (5, 64, 4), (6, 65, 5),
+                    (7, 1500, 2), (8, 1024, 4), (8, 3001, 8), (9, 40, 3), (70, 9, 5)):
+        E, C = 4 * R, 10
+        g = torch.Generator().manual_seed(R * T)
+        topk = torch.topk(torch.rand((R, T, E), generator=g), min(K, E))[1].to(torch.int32)
+        topk[:, ::3] = topk[:, ::3] // 8  # repeats, and ranks that get nothing from these tokens
+        buf = Buffer(R, low_latency_mode=False, device=cuda)
+        per_rank, _, per_expert, in_rank, _ = buf.get_dispatch_layout(topk.to(cuda), E)
+        want = torch.zeros((R, T, R), dtype=torch.bool).scatter_(2, (topk // 4).long(), True)
+        assert torch.equal(in_rank.cpu(), want) and torch.equal(per_rank.cpu().long(), want.sum(1))
+        experts = torch.stack([torch.bincount(topk[r].reshape(-1).long(), minlength=E) for r in range(R)])
+        assert torch.equal(per_expert.cpu().long(), experts)
+        x = torch.zeros((R, T, 8), dtype=torch.bfloat16, device=cuda)
+        rows, _, _, counts, handle, _ = buf.ht_dispatch(x, num_tokens_per_rank=per_rank, is_token_in_rank=in_rank, num_tokens_per_expert=per_expert,
+                                                        expert_alignment=4, num_channels=C)
+        _, prefix, chan, _, head, offset = handle
+        total = want.sum(1)  # [source][destination]
+        assert counts == ((experts.sum(0) + 3) // 4 * 4).view(R, 4).tolist() and rows.shape[0] == int(total.sum())
+        assert torch.equal(prefix.cpu().long(), total.t().cumsum(1))
+        assert torch.equal(offset.cpu(), torch.cat([torch.zeros(1, dtype=torch.int64), total.sum(0).cumsum(0)]))
+        up_to = want.cumsum(1)
+        assert torch.equal(head.cpu().long(), torch.where(want, up_to - 1, -1))
+        last = [min((c + 1) * ((T + C - 1) // C), T) - 1 for c in range(C)]
+        assert torch.equal(chan.cpu().long(), up_to[:, last].transpose(1, 2))
