@@ -1791,3 +1791,66 @@ def test_watched_launches_beyond_the_words_and_on_two_streams(cuda):
             assert lib.nixl_amd_copy_plan_destroy(p) == 0
         torch.cuda.synchronize()
         assert torch.equal(src, dst)
+
+
+def test_totals_of_listed_requests_start_at_nothing_every_time(cuda):
+    """Requests against device-resident lists share their totals' memory one after another, and requests of several
+    threads at once: what a request counted (bytes, bad pairs, continued ones) is not there for the next, refused ones
+    included, and every copy moves its own bytes."""
+    import threading
+    import torch
+    lib = _lib.kernels()
+    n, width = 3000, 512
+    src = torch.randint(0, 256, (n, width), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros((4, n, width), dtype=torch.uint8, device=cuda)
+    lists = []
+    lens = 128 + 16 * (np.arange(n) % 17)
+    for base in [src.data_ptr()] + [dst[i].data_ptr() for i in range(4)]:
+        table = np.zeros(n, dtype=np.dtype([("addr", "<u8"), ("len", "<u4"), ("continues", "<u4")]))
+        table["addr"] = base + np.arange(n, dtype=np.uint64) * np.uint64(width)
+        table["len"] = lens
+        lists.append(ctypes.c_void_p())
+        assert lib.nixl_amd_copy_list_create(table.ctypes.data, n, 0, ctypes.byref(lists[-1])) == 0, _lib.kernels_error()
+    torch.cuda.synchronize()
+    failures = []
+
+    def work(thread):
+        rng = np.random.default_rng(thread)
+        for i in range(30):
+            idx = np.sort(rng.choice(n, int(rng.integers(1, n)), replace=False)).astype(np.int32) if i % 2 else \
+                rng.permutation(n)[:int(rng.integers(1, n))].astype(np.int32)
+            other = idx.copy()
+            bad = i % 3 == 0
+            if bad:
+                other[0] = (other[0] + 1) % n  # another length
+            plan, continued = ctypes.c_void_p(), ctypes.c_size_t(99)
+            rc = lib.nixl_amd_copy_plan_create_listed(lists[0], idx.ctypes.data, lists[1 + thread], other.ctypes.data, idx.size, None,
+                                                      ctypes.byref(continued), ctypes.byref(plan))
+            if (rc != 0) != bad:
+                failures.append((thread, i, rc))
+                return
+            if bad:
+                continue
+            info = _lib.CopyPlanInfo()
+            lib.nixl_amd_copy_plan_query(plan, ctypes.byref(info))
+            if info.payload_bytes != lens[idx].sum() or info.vec_descs != idx.size or continued.value != 0:
+                failures.append((thread, i, info.payload_bytes, continued.value))
+            if lib.nixl_amd_copy_plan_launch(plan, None) != 0 or lib.nixl_amd_copy_plan_status(plan, 1) != 0 or lib.nixl_amd_copy_plan_destroy(plan) != 0:
+                failures.append((thread, i, "launch"))
+                return
+            moved[thread, idx] = True
+
+    moved = np.zeros((4, n), dtype=bool)
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
+    torch.cuda.synchronize()
+    inside = torch.arange(width, device=cuda)[None, :] < torch.from_numpy(lens).to(cuda)[:, None]
+    for t in range(4):
+        want = torch.where(inside & torch.from_numpy(moved[t]).to(cuda)[:, None], src, 0)
+        assert torch.equal(dst[t], want)
+    for handle in lists:
+        lib.nixl_amd_copy_list_destroy(handle)
