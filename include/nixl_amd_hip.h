@@ -289,6 +289,16 @@ nixl_amd_copy_plan_launch_watched(nixl_amd_copy_plan_t *plan, void *stream);
 int
 nixl_amd_copy_watch_prepare(void);
 
+/* States (`own` non-zero) that nothing but launches of this library's plans is queued on `stream` of
+ * `device`, or (`own` zero) takes that back, at the latest before the stream is destroyed.  While it
+ * holds, the word of the last watched launch there tells a plan that is made for the stream whether it
+ * is idle (nixl_amd_copy_tuning_t).  The runtime, which answers that for every other stream, calls a
+ * stream busy if it has not been asked since a launch that has no event behind it, and the plan is then
+ * written on a stream of the library's.  NIXL_AMD_ERR_INVALID for the default streams, and without
+ * nixl_amd_copy_watch_prepare. */
+int
+nixl_amd_copy_watch_stream(int device, void *stream, int own);
+
 /* Whether the plan's launches have completed: NIXL_AMD_OK when all have (or none was made),
  * NIXL_AMD_ERR_BUSY while one still runs (no error text is recorded for that answer: the call
  * is made to be polled), another negative status if a launch failed.  With `wait` non-zero the

@@ -104,13 +104,14 @@ def kernels():
         getattr(lib, fn).restype = c_int
     lib.nixl_amd_copy_plan_launch.argtypes = [c_void_p, c_void_p]
     lib.nixl_amd_copy_plan_launch_watched.argtypes = [c_void_p, c_void_p]
+    lib.nixl_amd_copy_watch_stream.argtypes = [c_int, c_void_p, c_int]
     lib.nixl_amd_copy_plan_destroy.argtypes = [c_void_p]
     lib.nixl_amd_copy_plan_status.argtypes = [c_void_p, c_int]
     lib.nixl_amd_copy_plan_status.restype = c_int
     lib.nixl_amd_copy_plan_query.argtypes = [c_void_p, POINTER(CopyPlanInfo)]
     lib.nixl_amd_copy_plan_time.argtypes = [c_void_p, c_void_p, c_int, POINTER(c_float)]
     for fn in ("nixl_amd_copy_plan_create", "nixl_amd_copy_plan_launch", "nixl_amd_copy_plan_launch_watched",
-               "nixl_amd_copy_watch_prepare", "nixl_amd_copy_plan_destroy", "nixl_amd_copy_plan_query",
+               "nixl_amd_copy_watch_prepare", "nixl_amd_copy_watch_stream", "nixl_amd_copy_plan_destroy", "nixl_amd_copy_plan_query",
                "nixl_amd_copy_plan_time"):
         getattr(lib, fn).restype = c_int
     _kernels = lib
@@ -186,7 +187,8 @@ def kernel_symbols():
                    "nixl_amd_copy_plan_create_from_records", "nixl_amd_copy_records_abandon", "nixl_amd_copy_block_len_fits",
                    "nixl_amd_copy_list_create", "nixl_amd_copy_list_destroy", "nixl_amd_copy_list_device",
                    "nixl_amd_copy_plan_create_listed", "nixl_amd_copy_plan_create_listed_on",
-                   "nixl_amd_copy_plan_launch", "nixl_amd_copy_plan_launch_watched", "nixl_amd_copy_watch_prepare", "nixl_amd_copy_plan_destroy", "nixl_amd_copy_plan_status",
+                   "nixl_amd_copy_plan_launch", "nixl_amd_copy_plan_launch_watched", "nixl_amd_copy_watch_prepare",
+                   "nixl_amd_copy_watch_stream", "nixl_amd_copy_plan_destroy", "nixl_amd_copy_plan_status",
                    "nixl_amd_copy_plan_query", "nixl_amd_copy_plan_time", "nixl_amd_ep_ll_workspace_bytes"] + list(_EP_SIGS))
 
 

@@ -1116,8 +1116,6 @@ public:
     static constexpr int kStride = 16; // words: a cache line each
 
     explicit DoneSlots(uint32_t *words) : words_(words) {
-        for (Last &l : last_)
-            l.slot = -1;
         for (int i = kDoneSlots - 1; i >= 0; --i)
             free_.push_back(i);
     }
@@ -1153,31 +1151,34 @@ public:
         return __atomic_load_n(words_ + slot * kStride, __ATOMIC_ACQUIRE) == value;
     }
 
+    // Nothing but launches of plans is queued on `stream`, or (not `own`) that holds no longer.
+    void
+    own_stream(hipStream_t stream, bool own) {
+        std::lock_guard<std::mutex> lock(mutex_);
+        Last *const at = find(stream);
+        if (own && !at)
+            last_.push_back(Last{stream, -1, 0});
+        else if (own)
+            at->slot = -1; // another stream at the address of an earlier one
+        else if (at)
+            last_.erase(last_.begin() + (at - last_.data()));
+    }
+
     // The last launch on `stream` that this library made, if it is watched; slot -1: it is not.
     void
     last_on(hipStream_t stream, int slot, uint32_t value) {
         std::lock_guard<std::mutex> lock(mutex_);
-        Last *at = nullptr;
-        for (Last &l : last_) {
-            if (l.slot >= 0 && l.stream != stream) continue;
-            at = &l;
-            if (l.slot >= 0) break; // the stream's own
-        }
-        if (slot < 0) {
-            if (at) at->slot = -1;
-            return;
-        }
-        if (!at) at = &last_[next_last_++ % kLast];
-        *at = Last{stream, slot, value};
+        if (Last *const at = find(stream)) *at = Last{stream, slot, value};
     }
 
-    // Whether that launch has run: 1, 0, or -1 if nothing is known of one.
+    // Whether a stream that has no other work than plans has run the last of them: 1, 0, or -1 if that is not
+    // known here.
     int
     last_ended(hipStream_t stream) {
         std::lock_guard<std::mutex> lock(mutex_);
-        for (const Last &l : last_)
-            if (l.stream == stream && l.slot >= 0) return l.value != value_[l.slot] || arrived(l.slot, l.value); // a used slot was free again
-        return -1;
+        const Last *const l = find(stream);
+        if (!l || l->slot < 0) return -1;
+        return l->value != value_[l->slot] || arrived(l->slot, l->value); // a used slot was free again
     }
 
 private:
@@ -1186,9 +1187,15 @@ private:
         int slot;
         uint32_t value;
     };
-    static constexpr unsigned kLast = 64;
-    Last last_[kLast] = {};
-    unsigned next_last_ = 0;
+
+    Last *
+    find(hipStream_t stream) {
+        for (Last &l : last_)
+            if (l.stream == stream) return &l;
+        return nullptr;
+    }
+
+    std::vector<Last> last_; // of the streams that were named to own_stream
     uint32_t *const words_;
     uint32_t *counts_ = nullptr;
     std::mutex mutex_;
@@ -1658,8 +1665,8 @@ build_stream(nixl_amd_copy_plan *plan, const Tuning &t, hipStream_t *out) {
         const bool may_ask = hipStreamIsCapturing(t.stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
         // The runtime cannot tell of a launch without an event behind it that it has run: asked for the
         // stream it puts a marker there and finds it busy (a request of 15 250 blocks: 68 us became 103).
-        // A launch that is watched says it itself; what else the caller may have queued behind it costs
-        // this plan time and nothing else.
+        // A launch that is watched says it itself, on a stream that carries nothing else: elsewhere the caller's
+        // own work may lie behind it, and a request that waits for its verdict would wait for that.
         DoneSlots *const slots = done_slots(plan->device);
         const int ended = may_ask && slots ? slots->last_ended(t.stream) : -1;
         if (may_ask && (ended >= 0 ? ended == 1 : hipStreamQuery(t.stream) == hipSuccess)) {
@@ -2722,6 +2729,17 @@ nixl_amd_copy_watch_prepare(void) {
     for (int i = 0; i < n; ++i)
         all[i] = new DoneSlots(words + i * kWords);
     g_done_slots.store(all, std::memory_order_release);
+    return NIXL_AMD_OK;
+}
+
+int
+nixl_amd_copy_watch_stream(int device, void *stream, int own) {
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!s || s == hipStreamLegacy || s == hipStreamPerThread)
+        return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "watch_stream: a default stream is not the caller's alone");
+    DoneSlots *const slots = done_slots(device);
+    if (!slots) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "watch_stream: no words for this device (nixl_amd_copy_watch_prepare)");
+    slots->own_stream(s, own != 0);
     return NIXL_AMD_OK;
 }
 

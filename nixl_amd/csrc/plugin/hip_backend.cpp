@@ -231,7 +231,9 @@ nixlHipEngine::~nixlHipEngine() {
     }
     for (size_t i = 0; i < streams_.size(); ++i) {
         if (!streams_[i]) continue;
-        const DeviceScope on_device(static_cast<int>(i / streamsPerDevice_));
+        const int device = static_cast<int>(i / streamsPerDevice_);
+        const DeviceScope on_device(device);
+        (void)nixl_amd_copy_watch_stream(device, streams_[i], 0);
         (void)hipStreamSynchronize(streams_[i]);
         (void)hipStreamDestroy(streams_[i]);
     }
@@ -246,6 +248,8 @@ nixlHipEngine::pickStream(int device, unsigned turn) const {
         // of the host application does not serialise against transfers.
         if (!hipOk(hipStreamCreateWithFlags(&streams_[idx], hipStreamNonBlocking), "hipStreamCreateWithFlags"))
             streams_[idx] = nullptr;
+        else // whether it is idle is asked of the word of its last transfer, if there are words
+            (void)nixl_amd_copy_watch_stream(device, streams_[idx], 1);
     }
     return streams_[idx];
 }

@@ -1,0 +1,494 @@
+// The host side of copy plans against a HIP runtime made for it: what a plan asks of the runtime, in which
+// order, and what it answers when a launch is late, lost or seen by another thread.  The functions below
+// stand before those of libamdhip64 in the process; no GPU is used.  Memory is the host's, kernels are
+// known by their names, and those that the host waits for do what it waits for.
+//
+// usage: copy_host_check <scenario>; prints "OK" and exits 0 on success.
+#include <hip/hip_runtime_api.h>
+
+#include <atomic>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <deque>
+#include <functional>
+#include <map>
+#include <memory>
+#include <mutex>
+#include <numeric>
+#include <string>
+#include <vector>
+
+#include "nixl_amd_hip.h"
+
+#define REQUIRE(cond)                                                          \
+    do {                                                                       \
+        if (!(cond)) {                                                         \
+            std::fprintf(stderr, "%s:%d: %s failed (%s)\n", __FILE__, __LINE__, #cond, nixl_amd_last_error()); \
+            std::exit(1);                                                      \
+        }                                                                      \
+    } while (0)
+
+namespace {
+
+// ---- streams and events -----------------------------------------------------------------------
+
+// Work runs when it is queued, or, on a stream that is held, when that is let go.
+struct Stream {
+    std::deque<std::function<void()>> work;
+    bool held = false;
+    bool waited_for = false; // by the host
+    std::vector<std::string> kernels; // launched on it
+
+    void
+    queue(std::function<void()> w) {
+        if (held)
+            work.push_back(std::move(w));
+        else
+            w();
+    }
+
+    void
+    let_go() {
+        held = false;
+        for (; !work.empty(); work.pop_front())
+            work.front()();
+    }
+};
+
+struct Event {
+    std::shared_ptr<bool> done = std::make_shared<bool>(true);
+    Stream *on = nullptr;
+};
+
+std::recursive_mutex g_lock;
+
+Stream &
+stream_of(hipStream_t s) {
+    static Stream of_all;
+    static thread_local Stream of_thread;
+    if (!s || s == hipStreamLegacy) return of_all;
+    if (s == hipStreamPerThread) return of_thread;
+    return *reinterpret_cast<Stream *>(s);
+}
+
+Event &
+event_of(hipEvent_t e) {
+    return *reinterpret_cast<Event *>(e);
+}
+
+// ---- kernels ----------------------------------------------------------------------------------
+
+std::map<const void *, std::string> &
+kernel_names() {
+    static std::map<const void *, std::string> names;
+    return names;
+}
+
+std::map<const void *, void *> &
+device_variables() {
+    static std::map<const void *, void *> variables;
+    return variables;
+}
+
+// The arguments of the kernels that the host waits for, as copy_kernels.hip declares them.
+struct Done {
+    uint32_t *counts, *word;
+    uint32_t value;
+};
+
+struct ListTotals {
+    unsigned long long bytes_arrived, extra_continued;
+    uint32_t bad;
+};
+
+struct ListVerdict {
+    unsigned long long bytes;
+    uint32_t bad, continued, extra, there;
+};
+
+struct ListArgs {
+    void *recs;
+    const nixl_amd_copy_list_entry_t *src, *dst;
+    uint32_t n_src, n_dst;
+    const int32_t *src_index, *dst_index;
+    const void *runs;
+    const uint32_t *run_of;
+    uint32_t first_workgroup, n, n_workgroups;
+    ListTotals *totals;
+    ListVerdict *verdict;
+};
+
+std::function<void()>
+work_of(const std::string &kernel, dim3 grid, void **args) {
+    const auto is = [&](const char *name) { return kernel.find(name) != std::string::npos; };
+    if (is("copy_inline_done_kernel")) {
+        const Done done = *static_cast<Done *>(args[3]);
+        return [done] { *done.word = done.value; };
+    }
+    if (is("done_kernel")) {
+        uint32_t *const word = *static_cast<uint32_t **>(args[0]);
+        const uint32_t value = *static_cast<uint32_t *>(args[1]);
+        return [word, value] { *word = value; };
+    }
+    if (is("clear_totals_kernel")) {
+        auto *const totals = *static_cast<ListTotals **>(args[0]);
+        return [totals] { *totals = ListTotals{}; };
+    }
+    if (is("list_records_kernel")) {
+        const ListArgs a = *static_cast<ListArgs *>(args[0]);
+        return [a, grid] {
+            REQUIRE(a.totals->bytes_arrived == 0 || a.first_workgroup != 0); // nothing of an earlier request's
+            a.totals->bytes_arrived += grid.x;
+            if (a.totals->bytes_arrived != a.n_workgroups) return;
+            *a.totals = ListTotals{};
+            a.verdict->bytes = a.n;
+            a.verdict->there = 1;
+        };
+    }
+    return [] {};
+}
+
+// ---- what a scenario looks at -----------------------------------------------------------------
+
+int
+launched(const Stream &s, const char *kernel) {
+    int n = 0;
+    for (const std::string &name : s.kernels)
+        n += name.find(kernel) != std::string::npos;
+    return n;
+}
+
+hipStream_t
+handle(Stream &s) {
+    return reinterpret_cast<hipStream_t>(&s);
+}
+
+nixl_amd_copy_tuning_t
+tuning_for(Stream &s) {
+    nixl_amd_copy_tuning_t t{};
+    t.stream = &s;
+    return t;
+}
+
+// A plan of one block, launched and watched on `s` (it tells its end itself).
+nixl_amd_copy_plan_t *
+block_plan() {
+    alignas(128) static uint8_t from[8192], to[8192];
+    const nixl_amd_copy_desc_t desc{reinterpret_cast<uintptr_t>(from), reinterpret_cast<uintptr_t>(to), sizeof(from)};
+    nixl_amd_copy_plan_t *plan = nullptr;
+    REQUIRE(nixl_amd_copy_plan_create(&desc, 1, 0, nullptr, &plan) == 0);
+    return plan;
+}
+
+// Two lists on the device with entries of equal lengths, and pairs that name them.
+struct Lists {
+    static constexpr size_t kEntries = 2000;
+    std::vector<uint8_t> memory = std::vector<uint8_t>(kEntries * 256);
+    nixl_amd_copy_list_t *src = nullptr, *dst = nullptr;
+    std::vector<int32_t> index = std::vector<int32_t>(kEntries);
+
+    Lists() {
+        std::iota(index.begin(), index.end(), 0);
+        std::vector<nixl_amd_copy_list_entry_t> table(kEntries);
+        for (size_t i = 0; i < kEntries; ++i) {
+            table[i] = {};
+            table[i].addr = reinterpret_cast<uintptr_t>(memory.data()) + i * 256;
+            table[i].len = 256;
+        }
+        REQUIRE(nixl_amd_copy_list_create(table.data(), kEntries, 0, &src) == 0);
+        REQUIRE(nixl_amd_copy_list_create(table.data(), kEntries, 0, &dst) == 0);
+    }
+
+    ~Lists() {
+        (void)nixl_amd_copy_list_destroy(src);
+        (void)nixl_amd_copy_list_destroy(dst);
+    }
+
+    int
+    request(const nixl_amd_copy_tuning_t *tuning, nixl_amd_copy_plan_t **plan) {
+        size_t continued = 0;
+        return nixl_amd_copy_plan_create_listed_on(src, index.data(), dst, index.data(), kEntries, tuning, &continued, plan);
+    }
+};
+
+// ---- scenarios --------------------------------------------------------------------------------
+
+// A caller's stream whose last watched transfer has been seen done and that has other work of the
+// caller's since then: a plan made for it is written elsewhere, and a request against
+// device-resident lists does not wait for that work.  On a stream that the caller keeps for
+// transfers the word answers.
+void
+work_behind_a_watched_launch() {
+    REQUIRE(nixl_amd_copy_watch_prepare() == 0);
+    Lists lists;
+    for (const bool own : {false, true}) {
+        Stream s;
+        if (own) REQUIRE(nixl_amd_copy_watch_stream(0, &s, 1) == 0);
+        const nixl_amd_copy_tuning_t tuning = tuning_for(s);
+        nixl_amd_copy_plan_t *first = block_plan();
+        REQUIRE(nixl_amd_copy_plan_launch_watched(first, &s) == 0);
+        REQUIRE(nixl_amd_copy_plan_status(first, 0) == 0);
+        nixl_amd_copy_plan_t *request = nullptr;
+        if (!own) {
+            s.held = true;
+            s.queue([] {}); // the caller's
+        }
+        REQUIRE(lists.request(&tuning, &request) == 0);
+        REQUIRE(!s.waited_for);
+        REQUIRE(launched(s, "list_records_kernel") == (own ? 1 : 0));
+        s.let_go();
+        REQUIRE(nixl_amd_copy_plan_launch_watched(request, &s) == 0);
+        REQUIRE(nixl_amd_copy_plan_status(request, 1) == 0);
+        REQUIRE(nixl_amd_copy_plan_destroy(request) == 0);
+        REQUIRE(nixl_amd_copy_plan_destroy(first) == 0);
+        if (own) { // and not while that transfer runs, nor when the stream is no longer kept for them
+            s.held = true;
+            first = block_plan();
+            REQUIRE(nixl_amd_copy_plan_launch_watched(first, &s) == 0);
+            REQUIRE(lists.request(&tuning, &request) == 0);
+            REQUIRE(launched(s, "list_records_kernel") == 1);
+            s.let_go();
+            REQUIRE(nixl_amd_copy_plan_status(first, 0) == 0);
+            REQUIRE(nixl_amd_copy_plan_destroy(first) == 0);
+            REQUIRE(nixl_amd_copy_plan_destroy(request) == 0);
+            REQUIRE(nixl_amd_copy_watch_stream(0, &s, 0) == 0);
+            s.held = true;
+            s.queue([] {});
+            REQUIRE(lists.request(&tuning, &request) == 0);
+            REQUIRE(launched(s, "list_records_kernel") == 1 && !s.waited_for);
+            REQUIRE(nixl_amd_copy_plan_destroy(request) == 0);
+            s.let_go();
+        }
+    }
+    for (void *shared : {static_cast<void *>(nullptr), static_cast<void *>(hipStreamLegacy), static_cast<void *>(hipStreamPerThread)})
+        REQUIRE(nixl_amd_copy_watch_stream(0, shared, 1) == NIXL_AMD_ERR_INVALID);
+}
+
+} // namespace
+
+// ---- the runtime ------------------------------------------------------------------------------
+
+#define LOCKED const std::lock_guard<std::recursive_mutex> lock(g_lock)
+
+extern "C" {
+
+void **
+__hipRegisterFatBinary(const void *) {
+    static void *module = nullptr;
+    return &module;
+}
+
+void
+__hipUnregisterFatBinary(void **) {}
+
+void
+__hipRegisterFunction(void **, const void *stub, char *, const char *name, unsigned, void *, void *, void *, void *, int *) {
+    kernel_names()[stub] = name;
+}
+
+void
+__hipRegisterVar(void **, void *symbol, char *, char *, int, size_t size, int, int) {
+    void *p = std::aligned_alloc(128, (size + 127) / 128 * 128);
+    std::memset(p, 0, size);
+    device_variables()[symbol] = p;
+}
+
+struct CallConfiguration {
+    dim3 grid, block;
+    size_t shared;
+    hipStream_t stream;
+};
+static thread_local std::vector<CallConfiguration> g_calls;
+
+hipError_t
+__hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t stream) {
+    g_calls.push_back({grid, block, shared, stream});
+    return hipSuccess;
+}
+
+hipError_t
+__hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *stream) {
+    const CallConfiguration c = g_calls.back();
+    g_calls.pop_back();
+    *grid = c.grid;
+    *block = c.block;
+    *shared = c.shared;
+    *stream = c.stream;
+    return hipSuccess;
+}
+
+hipError_t
+hipLaunchKernel(const void *stub, dim3 grid, dim3, void **args, size_t, hipStream_t stream) {
+    LOCKED;
+    const std::string &name = kernel_names().at(stub);
+    Stream &s = stream_of(stream);
+    s.kernels.push_back(name);
+    s.queue(work_of(name, grid, args));
+    return hipSuccess;
+}
+
+hipError_t
+hipGetSymbolAddress(void **p, const void *symbol) {
+    *p = device_variables().at(symbol);
+    return hipSuccess;
+}
+
+hipError_t
+hipGetDeviceCount(int *n) {
+    *n = 1;
+    return hipSuccess;
+}
+
+hipError_t
+hipGetDevice(int *device) {
+    *device = 0;
+    return hipSuccess;
+}
+
+hipError_t
+hipSetDevice(int) {
+    return hipSuccess;
+}
+
+hipError_t
+hipDeviceGetAttribute(int *value, hipDeviceAttribute_t, int) {
+    *value = 1;
+    return hipSuccess;
+}
+
+hipError_t
+hipGetLastError() {
+    return hipSuccess;
+}
+
+const char *
+hipGetErrorString(hipError_t) {
+    return "an error";
+}
+
+hipError_t
+hipMalloc(void **p, size_t n) {
+    *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
+    return hipSuccess;
+}
+
+hipError_t
+hipHostMalloc(void **p, size_t n, unsigned) {
+    return hipMalloc(p, n);
+}
+
+hipError_t
+hipFree(void *p) {
+    std::free(p);
+    return hipSuccess;
+}
+
+hipError_t
+hipHostFree(void *p) {
+    return hipFree(p);
+}
+
+hipError_t
+hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t stream) {
+    LOCKED;
+    stream_of(stream).queue([=] { std::memcpy(dst, src, n); });
+    return hipSuccess;
+}
+
+hipError_t
+hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
+    *s = handle(*new Stream);
+    return hipSuccess;
+}
+
+hipError_t
+hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) {
+    *status = hipStreamCaptureStatusNone;
+    return hipSuccess;
+}
+
+hipError_t
+hipStreamQuery(hipStream_t stream) {
+    LOCKED;
+    return stream_of(stream).work.empty() ? hipSuccess : hipErrorNotReady;
+}
+
+hipError_t
+hipStreamSynchronize(hipStream_t stream) {
+    LOCKED;
+    Stream &s = stream_of(stream);
+    s.waited_for = true;
+    s.let_go();
+    return hipSuccess;
+}
+
+hipError_t
+hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) {
+    return hipSuccess;
+}
+
+hipError_t
+hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    *e = reinterpret_cast<hipEvent_t>(new Event);
+    return hipSuccess;
+}
+
+hipError_t
+hipEventCreate(hipEvent_t *e) {
+    return hipEventCreateWithFlags(e, 0);
+}
+
+hipError_t
+hipEventDestroy(hipEvent_t e) {
+    delete &event_of(e);
+    return hipSuccess;
+}
+
+hipError_t
+hipEventRecord(hipEvent_t event, hipStream_t stream) {
+    LOCKED;
+    Event &e = event_of(event);
+    e.done = std::make_shared<bool>(false);
+    e.on = &stream_of(stream);
+    e.on->queue([done = e.done] { *done = true; });
+    return hipSuccess;
+}
+
+hipError_t
+hipEventQuery(hipEvent_t event) {
+    LOCKED;
+    const Event &e = event_of(event);
+    return *e.done ? hipSuccess : hipErrorNotReady;
+}
+
+hipError_t
+hipEventSynchronize(hipEvent_t event) {
+    LOCKED;
+    const Event &e = event_of(event);
+    if (!*e.done) {
+        e.on->waited_for = true;
+        e.on->let_go();
+    }
+    return hipSuccess;
+}
+
+hipError_t
+hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
+    *ms = 0.f;
+    return hipSuccess;
+}
+
+} // extern "C"
+
+int
+main(int argc, char **argv) {
+    const std::map<std::string, void (*)()> scenarios{
+        {"work_behind_a_watched_launch", work_behind_a_watched_launch},
+    };
+    REQUIRE(argc == 2 && scenarios.count(argv[1]));
+    scenarios.at(argv[1])();
+    std::printf("OK\n");
+    return 0;
+}

@@ -361,6 +361,19 @@ def test_helper_threads_of_the_hip_backend_on_the_cpu():
     assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
 
 
+@pytest.mark.parametrize("scenario", ["work_behind_a_watched_launch"])
+def test_host_side_of_copy_plans_on_the_cpu(scenario):
+    """tests/cpp/copy_host_check.cpp: what a copy plan asks of the runtime and answers its caller,
+    with a runtime that the program brings itself."""
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = os.path.join(root, "tests", "cpp", "_build", "copy_host_check")
+    if not os.path.exists(exe):
+        pytest.fail(f"{exe} missing: run __graft_entry__.build() first")
+    proc = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
+
+
 def test_list_and_option_helpers_of_the_c_wrapper(two_agents):
     """The descriptor-list, option and stub helpers of the reference's C wrapper
     (src/bindings/rust/wrapper.h:193-201,297-326,457) behave as their names say; the metadata
