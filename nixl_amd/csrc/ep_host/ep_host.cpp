@@ -65,11 +65,15 @@ public:
         return THPVariable_Unpack(o);
     }
 
+    // Whatever stands for an integer in Python: NumPy's integers and tensors of one too.
     int64_t
     integer() {
         PyObject *const o = *next_++;
-        if (!PyLong_Check(o)) throw py_type("an integer");
-        const int64_t v = PyLong_AsLongLong(o);
+        if (!PyIndex_Check(o)) throw py_type("an integer");
+        PyObject *const number = PyNumber_Index(o);
+        if (!number) throw python_error();
+        const int64_t v = PyLong_AsLongLong(number);
+        Py_DECREF(number);
         if (v == -1 && PyErr_Occurred()) throw python_error();
         return v;
     }

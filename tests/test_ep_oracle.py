@@ -631,6 +631,37 @@ def test_native_host_calls_refuse_what_they_cannot_use(args, error):
         _lib.ep_host().layout(*args)
 
 
+class _Count:
+    """An integer of somebody's own."""
+    def __init__(self, n):
+        self.n = n
+
+    def __index__(self):
+        if self.n is None:
+            raise LookupError("no number here")
+        return self.n
+
+
+@pytest.mark.parametrize("five", [5, np.int64(5), np.int32(5), np.uint8(5), torch.tensor(5), _Count(5)])
+def test_native_host_calls_take_whatever_is_an_integer(five):
+    """As every call did that went through ctypes: sizes come from NumPy and tensors, too."""
+    from nixl_amd import _lib
+    topk = torch.zeros(2, 3, 4, dtype=torch.int32)
+    per_rank, per_expert, in_rank, rc = _lib.ep_host().layout(topk, five, None)  # five experts on two ranks: refused on the host
+    assert per_expert.shape == (2, 5) and rc != 0
+    x = torch.zeros(2, 3, 1024, dtype=torch.bfloat16)
+    out = _lib.ep_host().ll_dispatch(x, topk, None, None, None, None, None, five, five, 4, five, 10, 0, 0, 0, 0, None)
+    assert out[0].shape == (2, 5, 5, 1024) and out[-1] == 0
+
+
+@pytest.mark.parametrize("count, error", [(np.float64(5), TypeError), ("5", TypeError), (None, TypeError), (torch.tensor([5, 5]), TypeError),
+                                          (_Count(None), LookupError)])
+def test_native_host_calls_take_nothing_else_for_an_integer(count, error):
+    from nixl_amd import _lib
+    with pytest.raises(error):
+        _lib.ep_host().layout(torch.zeros(2, 3, 4, dtype=torch.int32), count, None)
+
+
 def test_native_host_calls_hand_back_the_kernels_status_and_the_callers_tensors():
     """Without a launch the low-latency call only makes its tensors, and a launch that the kernels refuse on the host
     (five experts on two ranks) comes back as a status, not as an exception."""
