@@ -1366,7 +1366,6 @@ give_back_staging(nixl_amd_copy_plan *plan) {
 // while it may; an error of the stream's, or of a launch that ended without its word.
 static hipError_t
 ask_stream(const nixl_amd_copy_plan *plan) {
-    if (!plan->watched_on) return hipErrorNotReady; // the legacy stream may not be asked while any stream is captured
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     hipError_t e = hipStreamIsCapturing(plan->watched_on, &capture);
     if (e == hipSuccess && capture != hipStreamCaptureStatusNone) return hipErrorNotReady;
@@ -2786,8 +2785,11 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
     }
     // The word this launch is watched by.  A plan whose earlier launch is still being watched takes an
     // event for this one: the two may run on different streams, and end in any order.
+    // The legacy stream takes one, too: how its launch fares may not be asked while any stream is captured, and
+    // without an answer a launch that failed would be waited for without end.
     Done done{};
-    DoneSlots *const slots = watched && capture == hipStreamCaptureStatusNone ? done_slots(plan->device) : nullptr;
+    const bool asked = s && s != hipStreamLegacy;
+    DoneSlots *const slots = watched && asked && capture == hipStreamCaptureStatusNone ? done_slots(plan->device) : nullptr;
     if (slots && plan->slot.load(std::memory_order_relaxed) >= 0) (void)ended(plan, false);
     int slot = slots && plan->slot.load(std::memory_order_relaxed) < 0 ? slots->take(&done) : -1;
     bool told = false; // the copy writes the word itself

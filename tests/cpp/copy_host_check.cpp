@@ -39,6 +39,7 @@ struct Stream {
     std::deque<std::function<void()>> work;
     bool held = false;
     bool waited_for = false; // by the host
+    hipError_t failure = hipSuccess; // what was queued does not run any more
     std::vector<std::string> kernels; // launched on it
 
     void
@@ -51,6 +52,7 @@ struct Stream {
 
     void
     let_go() {
+        if (failure != hipSuccess) return;
         held = false;
         for (; !work.empty(); work.pop_front())
             work.front()();
@@ -266,6 +268,38 @@ work_behind_a_watched_launch() {
         REQUIRE(nixl_amd_copy_watch_stream(0, shared, 1) == NIXL_AMD_ERR_INVALID);
 }
 
+// A watched launch that fails is reported, whatever stream it went to: by a status that is polled
+// (the runtime is asked now and then), and by one that waits.
+void
+launch_fails(hipStream_t stream) {
+    REQUIRE(nixl_amd_copy_watch_prepare() == 0);
+    Stream &s = stream_of(stream);
+    nixl_amd_copy_plan_t *plan = block_plan();
+    s.held = true;
+    REQUIRE(nixl_amd_copy_plan_launch_watched(plan, stream) == 0);
+    for (int i = 0; i < 10000; ++i)
+        REQUIRE(nixl_amd_copy_plan_status(plan, 0) == NIXL_AMD_ERR_BUSY); // it is late, no more
+    s.failure = hipErrorLaunchFailure;
+    int rc = NIXL_AMD_ERR_BUSY;
+    for (int i = 0; i < 10000 && rc == NIXL_AMD_ERR_BUSY; ++i)
+        rc = nixl_amd_copy_plan_status(plan, 0);
+    REQUIRE(rc == NIXL_AMD_ERR_HIP);
+    REQUIRE(nixl_amd_copy_plan_status(plan, 1) == NIXL_AMD_ERR_HIP);
+}
+
+void
+launch_on_a_named_stream_fails() {
+    Stream s;
+    launch_fails(handle(s));
+}
+
+void
+launch_on_the_legacy_stream_fails() {
+    launch_fails(nullptr);
+    stream_of(nullptr) = {};
+    launch_fails(hipStreamLegacy);
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -412,7 +446,9 @@ hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) {
 hipError_t
 hipStreamQuery(hipStream_t stream) {
     LOCKED;
-    return stream_of(stream).work.empty() ? hipSuccess : hipErrorNotReady;
+    const Stream &s = stream_of(stream);
+    if (s.failure != hipSuccess) return s.failure;
+    return s.work.empty() ? hipSuccess : hipErrorNotReady;
 }
 
 hipError_t
@@ -421,7 +457,7 @@ hipStreamSynchronize(hipStream_t stream) {
     Stream &s = stream_of(stream);
     s.waited_for = true;
     s.let_go();
-    return hipSuccess;
+    return s.failure;
 }
 
 hipError_t
@@ -460,18 +496,18 @@ hipError_t
 hipEventQuery(hipEvent_t event) {
     LOCKED;
     const Event &e = event_of(event);
-    return *e.done ? hipSuccess : hipErrorNotReady;
+    if (*e.done) return hipSuccess;
+    return e.on->failure != hipSuccess ? e.on->failure : hipErrorNotReady;
 }
 
 hipError_t
 hipEventSynchronize(hipEvent_t event) {
     LOCKED;
     const Event &e = event_of(event);
-    if (!*e.done) {
-        e.on->waited_for = true;
-        e.on->let_go();
-    }
-    return hipSuccess;
+    if (*e.done) return hipSuccess;
+    e.on->waited_for = true;
+    e.on->let_go();
+    return e.on->failure;
 }
 
 hipError_t
@@ -486,6 +522,8 @@ int
 main(int argc, char **argv) {
     const std::map<std::string, void (*)()> scenarios{
         {"work_behind_a_watched_launch", work_behind_a_watched_launch},
+        {"launch_on_a_named_stream_fails", launch_on_a_named_stream_fails},
+        {"launch_on_the_legacy_stream_fails", launch_on_the_legacy_stream_fails},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
