@@ -282,7 +282,7 @@ nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream);
  * the end some microseconds sooner.  (A word says nothing of caches over host memory, for which an
  * event is what releases them.)  Needs nixl_amd_copy_watch_prepare, which allocates the words once a
  * process; without it, for more than 128 launches in flight on a device, for a plan whose earlier
- * launch is still running, and on the legacy default stream, an event is recorded as
+ * launch is still running, and on the default streams, an event is recorded as
  * nixl_amd_copy_plan_launch does. */
 int
 nixl_amd_copy_plan_launch_watched(nixl_amd_copy_plan_t *plan, void *stream);

@@ -2786,9 +2786,10 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
     // The word this launch is watched by.  A plan whose earlier launch is still being watched takes an
     // event for this one: the two may run on different streams, and end in any order.
     // The legacy stream takes one, too: how its launch fares may not be asked while any stream is captured, and
-    // without an answer a launch that failed would be waited for without end.
+    // without an answer a launch that failed would be waited for without end.  And the per-thread one, which is
+    // another stream in the thread that asks.
     Done done{};
-    const bool asked = s && s != hipStreamLegacy;
+    const bool asked = s && s != hipStreamLegacy && s != hipStreamPerThread;
     DoneSlots *const slots = watched && asked && capture == hipStreamCaptureStatusNone ? done_slots(plan->device) : nullptr;
     if (slots && plan->slot.load(std::memory_order_relaxed) >= 0) (void)ended(plan, false);
     int slot = slots && plan->slot.load(std::memory_order_relaxed) < 0 ? slots->take(&done) : -1;

@@ -18,6 +18,7 @@
 #include <mutex>
 #include <numeric>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "nixl_amd_hip.h"
@@ -300,6 +301,23 @@ launch_on_the_legacy_stream_fails() {
     launch_fails(hipStreamLegacy);
 }
 
+// A watched launch on one thread's per-thread stream, asked for from another thread: late is not failed.
+void
+launch_on_the_stream_of_a_thread() {
+    REQUIRE(nixl_amd_copy_watch_prepare() == 0);
+    Stream &s = stream_of(hipStreamPerThread);
+    nixl_amd_copy_plan_t *plan = block_plan();
+    s.held = true;
+    REQUIRE(nixl_amd_copy_plan_launch_watched(plan, hipStreamPerThread) == 0);
+    std::thread([&] {
+        for (int i = 0; i < 10000; ++i)
+            REQUIRE(nixl_amd_copy_plan_status(plan, 0) == NIXL_AMD_ERR_BUSY);
+    }).join();
+    s.let_go();
+    REQUIRE(nixl_amd_copy_plan_status(plan, 0) == 0);
+    REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -524,6 +542,7 @@ main(int argc, char **argv) {
         {"work_behind_a_watched_launch", work_behind_a_watched_launch},
         {"launch_on_a_named_stream_fails", launch_on_a_named_stream_fails},
         {"launch_on_the_legacy_stream_fails", launch_on_the_legacy_stream_fails},
+        {"launch_on_the_stream_of_a_thread", launch_on_the_stream_of_a_thread},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
