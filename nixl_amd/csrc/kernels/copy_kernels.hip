@@ -1365,15 +1365,17 @@ give_back_staging(nixl_amd_copy_plan *plan) {
 // The word of a launch is long in coming: whether the stream still has it to run.  hipErrorNotReady
 // while it may; an error of the stream's, or of a launch that ended without its word.
 static hipError_t
-ask_stream(const nixl_amd_copy_plan *plan) {
+ask_stream(const nixl_amd_copy_plan *plan, int slot) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     hipError_t e = hipStreamIsCapturing(plan->watched_on, &capture);
     if (e == hipSuccess && capture != hipStreamCaptureStatusNone) return hipErrorNotReady;
     if (e == hipSuccess) e = hipStreamQuery(plan->watched_on);
     if (e != hipSuccess) (void)hipGetLastError();
     if (e == hipErrorNotReady) return e;
-    const int slot = plan->slot.load(std::memory_order_acquire);
-    if (slot < 0 || done_slots(plan->device)->arrived(slot, plan->slot_value)) return hipErrorNotReady; // seen by the next look
+    // Another thread may have seen the end meanwhile and given the slot back, and another launch written its own
+    // value there: only while the slot is the plan's has a word without the plan's value not been written.
+    if (done_slots(plan->device)->arrived(slot, plan->slot_value)) return hipErrorNotReady; // seen by the next look
+    if (plan->slot.load(std::memory_order_acquire) != slot) return hipErrorNotReady;
     return e == hipSuccess ? hipErrorUnknown : e;
 }
 
@@ -1388,7 +1390,7 @@ ended(nixl_amd_copy_plan *plan, bool wait) {
         }
         constexpr uint32_t kAskEvery = 4096;
         if (plan->polls.fetch_add(1, std::memory_order_relaxed) % kAskEvery == kAskEvery - 1) {
-            const hipError_t e = ask_stream(plan);
+            const hipError_t e = ask_stream(plan, slot);
             if (e != hipErrorNotReady) return e;
             if (wait) std::this_thread::yield();
         }

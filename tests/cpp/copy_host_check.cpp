@@ -5,8 +5,9 @@
 //
 // usage: copy_host_check <scenario>; prints "OK" and exits 0 on success.
 #include <hip/hip_runtime_api.h>
+#include <signal.h>
+#include <sys/mman.h>
 
-#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -318,6 +319,50 @@ launch_on_the_stream_of_a_thread() {
     REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
 }
 
+// Two threads ask for one launch, as a progress thread and a caller do.  While the first is about to
+// look at the word after it has asked the stream, the second sees the end and gives the word back, and another
+// launch takes it and ends.  The moment is that of the read itself: the page is taken away when the
+// stream is asked, and the fault is where the second thread runs.
+void (*g_asked)(hipStream_t) = nullptr; // when the runtime is asked for a stream
+uint8_t *g_words = nullptr; // what the words lie in
+size_t g_words_size = 0;
+std::function<void()> g_at_read;
+
+void
+launch_seen_by_two_threads() {
+    REQUIRE(nixl_amd_copy_watch_prepare() == 0 && g_words);
+    static Stream s;
+    static nixl_amd_copy_plan_t *plan = block_plan();
+    static bool reached = false;
+    struct sigaction act{};
+    act.sa_handler = [](int) {
+        REQUIRE(g_at_read && !reached);
+        REQUIRE(mprotect(g_words, g_words_size, PROT_READ | PROT_WRITE) == 0);
+        reached = true;
+        g_at_read();
+    };
+    act.sa_flags = SA_NODEFER;
+    REQUIRE(sigaction(SIGSEGV, &act, nullptr) == 0);
+    g_at_read = [] {
+        std::thread([] {
+            s.let_go();
+            REQUIRE(nixl_amd_copy_plan_status(plan, 0) == 0);
+            nixl_amd_copy_plan_t *other = block_plan();
+            REQUIRE(nixl_amd_copy_plan_launch_watched(other, &s) == 0); // and has run
+        }).join();
+    };
+    g_asked = [](hipStream_t) {
+        g_asked = nullptr;
+        REQUIRE(mprotect(g_words, g_words_size, PROT_NONE) == 0);
+    };
+    s.held = true;
+    REQUIRE(nixl_amd_copy_plan_launch_watched(plan, &s) == 0);
+    int rc = NIXL_AMD_ERR_BUSY;
+    for (int i = 0; i < 10000 && rc == NIXL_AMD_ERR_BUSY; ++i)
+        rc = nixl_amd_copy_plan_status(plan, 0);
+    REQUIRE(reached && rc == 0);
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -427,8 +472,13 @@ hipMalloc(void **p, size_t n) {
 }
 
 hipError_t
-hipHostMalloc(void **p, size_t n, unsigned) {
-    return hipMalloc(p, n);
+hipHostMalloc(void **p, size_t n, unsigned flags) {
+    const hipError_t e = hipMalloc(p, n);
+    if (flags & hipHostMallocPortable) { // the words that launches are watched by
+        g_words = static_cast<uint8_t *>(*p);
+        g_words_size = (n + 4095) / 4096 * 4096;
+    }
+    return e;
 }
 
 hipError_t
@@ -465,6 +515,10 @@ hipError_t
 hipStreamQuery(hipStream_t stream) {
     LOCKED;
     const Stream &s = stream_of(stream);
+    if (g_asked) {
+        g_asked(stream);
+        return hipSuccess; // the launch has just ended
+    }
     if (s.failure != hipSuccess) return s.failure;
     return s.work.empty() ? hipSuccess : hipErrorNotReady;
 }
@@ -543,6 +597,7 @@ main(int argc, char **argv) {
         {"launch_on_a_named_stream_fails", launch_on_a_named_stream_fails},
         {"launch_on_the_legacy_stream_fails", launch_on_the_legacy_stream_fails},
         {"launch_on_the_stream_of_a_thread", launch_on_the_stream_of_a_thread},
+        {"launch_seen_by_two_threads", launch_seen_by_two_threads},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
