@@ -1272,6 +1272,7 @@ struct nixl_amd_copy_plan {
     uint32_t slot_value = 0;
     hipStream_t watched_on = nullptr;
     std::atomic<uint32_t> polls{0};
+    std::atomic<hipError_t> watch_failure{hipSuccess}; // of the watched launch: its word does not come any more
     bool ever_launched = false; // not counting launches into a capture
 
     ~nixl_amd_copy_plan();
@@ -1388,10 +1389,14 @@ ended(nixl_amd_copy_plan *plan, bool wait) {
             if (plan->slot.compare_exchange_strong(slot, -1)) slots.put(slot);
             break;
         }
+        if (const hipError_t e = plan->watch_failure.load(std::memory_order_relaxed); e != hipSuccess) return e;
         constexpr uint32_t kAskEvery = 4096;
         if (plan->polls.fetch_add(1, std::memory_order_relaxed) % kAskEvery == kAskEvery - 1) {
             const hipError_t e = ask_stream(plan, slot);
-            if (e != hipErrorNotReady) return e;
+            if (e != hipErrorNotReady) {
+                plan->watch_failure.store(e, std::memory_order_relaxed);
+                return e;
+            }
             if (wait) std::this_thread::yield();
         }
         if (!wait) return hipErrorNotReady;
@@ -2794,7 +2799,8 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
     const bool asked = s && s != hipStreamLegacy && s != hipStreamPerThread;
     DoneSlots *const slots = watched && asked && capture == hipStreamCaptureStatusNone ? done_slots(plan->device) : nullptr;
     if (slots && plan->slot.load(std::memory_order_relaxed) >= 0) (void)ended(plan, false);
-    int slot = slots && plan->slot.load(std::memory_order_relaxed) < 0 ? slots->take(&done) : -1;
+    const bool failed = plan->watch_failure != hipSuccess;
+    int slot = slots && (failed || plan->slot.load(std::memory_order_relaxed) < 0) ? slots->take(&done) : -1;
     bool told = false; // the copy writes the word itself
     const auto give_up = [&](hipError_t e) {
         if (slot >= 0) slots->put(slot); // nothing that would write its word is queued
@@ -2870,6 +2876,10 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
             slots->put(slot);
             slot = -1;
         }
+    }
+    if (failed && capture == hipStreamCaptureStatusNone) { // this launch is what the status is about from here on
+        plan->slot = -1; // no other launch gets it: who knows whether something still writes there
+        plan->watch_failure.store(hipSuccess);
     }
     if (slot >= 0) {
         plan->slot_value = done.value;

@@ -67,6 +67,7 @@ struct Event {
 };
 
 std::recursive_mutex g_lock;
+hipError_t g_launch_status = hipSuccess; // of a launch that is asked for
 
 Stream &
 stream_of(hipStream_t s) {
@@ -272,7 +273,7 @@ work_behind_a_watched_launch() {
 
 // A watched launch that fails is reported, whatever stream it went to: by a status that is polled
 // (the runtime is asked now and then), and by one that waits.
-void
+nixl_amd_copy_plan_t *
 launch_fails(hipStream_t stream) {
     REQUIRE(nixl_amd_copy_watch_prepare() == 0);
     Stream &s = stream_of(stream);
@@ -287,19 +288,34 @@ launch_fails(hipStream_t stream) {
         rc = nixl_amd_copy_plan_status(plan, 0);
     REQUIRE(rc == NIXL_AMD_ERR_HIP);
     REQUIRE(nixl_amd_copy_plan_status(plan, 1) == NIXL_AMD_ERR_HIP);
+    for (int i = 0; i < 10; ++i)
+        REQUIRE(nixl_amd_copy_plan_status(plan, 0) == NIXL_AMD_ERR_HIP); // and stays so
+    return plan;
 }
 
 void
 launch_on_a_named_stream_fails() {
-    Stream s;
-    launch_fails(handle(s));
+    Stream s, good;
+    nixl_amd_copy_plan_t *plan = launch_fails(handle(s));
+    g_launch_status = hipErrorOutOfMemory; // a launch that is refused changes nothing
+    REQUIRE(nixl_amd_copy_plan_launch_watched(plan, &good) == NIXL_AMD_ERR_HIP);
+    g_launch_status = hipSuccess;
+    REQUIRE(nixl_amd_copy_plan_status(plan, 0) == NIXL_AMD_ERR_HIP);
+    for (const bool watched : {true, false}) { // another launch does
+        REQUIRE((watched ? nixl_amd_copy_plan_launch_watched : nixl_amd_copy_plan_launch)(plan, &good) == 0);
+        REQUIRE(nixl_amd_copy_plan_status(plan, 0) == 0);
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        Stream bad;
+        plan = launch_fails(handle(bad));
+    }
+    REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0); // nothing runs that would read its arrays
 }
 
 void
 launch_on_the_legacy_stream_fails() {
-    launch_fails(nullptr);
+    REQUIRE(nixl_amd_copy_plan_destroy(launch_fails(nullptr)) == 0);
     stream_of(nullptr) = {};
-    launch_fails(hipStreamLegacy);
+    REQUIRE(nixl_amd_copy_plan_destroy(launch_fails(hipStreamLegacy)) == 0);
 }
 
 // A watched launch on one thread's per-thread stream, asked for from another thread: late is not failed.
@@ -419,6 +435,7 @@ __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *
 hipError_t
 hipLaunchKernel(const void *stub, dim3 grid, dim3, void **args, size_t, hipStream_t stream) {
     LOCKED;
+    if (g_launch_status != hipSuccess) return g_launch_status;
     const std::string &name = kernel_names().at(stub);
     Stream &s = stream_of(stream);
     s.kernels.push_back(name);
@@ -457,7 +474,7 @@ hipDeviceGetAttribute(int *value, hipDeviceAttribute_t, int) {
 
 hipError_t
 hipGetLastError() {
-    return hipSuccess;
+    return g_launch_status;
 }
 
 const char *
