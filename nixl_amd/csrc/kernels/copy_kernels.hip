@@ -1088,7 +1088,7 @@ public:
         return totals;
     }
 
-    // Only when its request's verdict is there: what else happened to it nobody knows.
+    // Only when its request's verdict is there, or it has been cleared again.
     void
     put(ListTotals *totals) {
         std::lock_guard<std::mutex> lock(mutex_);
@@ -2632,6 +2632,7 @@ create_listed(const nixl_amd_copy_list_t *src,
     auto *recs = reinterpret_cast<PieceRec *>(static_cast<uint8_t *>(plan->arena) + kRecsAt);
     ListTotals *const slot = e == hipSuccess && device < kMaxDevices ? list_slots(device).take() : nullptr;
     ListTotals *const totals = slot ? slot : static_cast<ListTotals *>(plan->arena);
+    bool queued = false; // something that adds to the totals
     if (e == hipSuccess && !slot) {
         hipLaunchKernelGGL(clear_totals_kernel, dim3(1), dim3(kWaveSize), 0, up, totals);
         e = hipGetLastError();
@@ -2643,6 +2644,7 @@ create_listed(const nixl_amd_copy_list_t *src,
         if (index_runs(src_index, dst_index, n, up_runs, up_run_of)) {
             hipLaunchKernelGGL(list_records_kernel<true>, dim3(workgroups), dim3(kListThreads), 0, up, a);
             e = hipGetLastError();
+            queued = e == hipSuccess;
         } else {
             for (size_t at = 0; at < n && e == hipSuccess; at += kListSlice) {
                 const size_t count = std::min(kListSlice, n - at);
@@ -2652,12 +2654,17 @@ create_listed(const nixl_amd_copy_list_t *src,
                 hipLaunchKernelGGL(list_records_kernel<false>, dim3(static_cast<uint32_t>((count + kListThreads - 1) / kListThreads)),
                                    dim3(kListThreads), 0, up, a);
                 e = hipGetLastError();
+                queued = queued || e == hipSuccess;
             }
         }
     }
     if (e == hipSuccess) e = await_verdict(*verdict, up);
     const ListVerdict got = *verdict;
-    if (slot && e == hipSuccess) list_slots(device).put(slot);
+    if (slot && e != hipSuccess && queued) { // counted in part, or by nobody knows whom
+        hipLaunchKernelGGL(clear_totals_kernel, dim3(1), dim3(kWaveSize), 0, up, totals);
+        queued = hipGetLastError() != hipSuccess || hipStreamSynchronize(up) != hipSuccess;
+    }
+    if (slot && (e == hipSuccess || !queued)) list_slots(device).put(slot);
     // The records are complete when the last kernel ends, which comes behind its verdict: a launch
     // follows on the same stream, or waits for the event; a plan that may be launched anywhere, also into a
     // capture, is complete when the caller has it.

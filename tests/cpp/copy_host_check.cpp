@@ -18,8 +18,10 @@
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <set>
 #include <string>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "nixl_amd_hip.h"
@@ -67,7 +69,10 @@ struct Event {
 };
 
 std::recursive_mutex g_lock;
-hipError_t g_launch_status = hipSuccess; // of a launch that is asked for
+hipError_t g_launch_status = hipSuccess; // of one launch,
+int g_good_launches = 0; // behind so many that are accepted
+void (*g_synchronized)(Stream &) = nullptr; // in front of a wait for a stream
+Stream *g_created = nullptr; // the last stream that the library made
 
 Stream &
 stream_of(hipStream_t s) {
@@ -125,6 +130,8 @@ struct ListArgs {
     ListVerdict *verdict;
 };
 
+std::set<ListTotals *> g_totals; // that requests have counted in
+
 std::function<void()>
 work_of(const std::string &kernel, dim3 grid, void **args) {
     const auto is = [&](const char *name) { return kernel.find(name) != std::string::npos; };
@@ -143,6 +150,7 @@ work_of(const std::string &kernel, dim3 grid, void **args) {
     }
     if (is("list_records_kernel")) {
         const ListArgs a = *static_cast<ListArgs *>(args[0]);
+        g_totals.insert(a.totals);
         return [a, grid] {
             REQUIRE(a.totals->bytes_arrived == 0 || a.first_workgroup != 0); // nothing of an earlier request's
             a.totals->bytes_arrived += grid.x;
@@ -214,7 +222,7 @@ struct Lists {
     int
     request(const nixl_amd_copy_tuning_t *tuning, nixl_amd_copy_plan_t **plan) {
         size_t continued = 0;
-        return nixl_amd_copy_plan_create_listed_on(src, index.data(), dst, index.data(), kEntries, tuning, &continued, plan);
+        return nixl_amd_copy_plan_create_listed_on(src, index.data(), dst, index.data(), index.size(), tuning, &continued, plan);
     }
 };
 
@@ -299,7 +307,6 @@ launch_on_a_named_stream_fails() {
     nixl_amd_copy_plan_t *plan = launch_fails(handle(s));
     g_launch_status = hipErrorOutOfMemory; // a launch that is refused changes nothing
     REQUIRE(nixl_amd_copy_plan_launch_watched(plan, &good) == NIXL_AMD_ERR_HIP);
-    g_launch_status = hipSuccess;
     REQUIRE(nixl_amd_copy_plan_status(plan, 0) == NIXL_AMD_ERR_HIP);
     for (const bool watched : {true, false}) { // another launch does
         REQUIRE((watched ? nixl_amd_copy_plan_launch_watched : nixl_amd_copy_plan_launch)(plan, &good) == 0);
@@ -379,6 +386,65 @@ launch_seen_by_two_threads() {
     REQUIRE(reached && rc == 0);
 }
 
+// 70 requests against device-resident lists that wait for their verdicts at once: each counts in totals of its own
+// that are zero when it starts; 64 find such totals ready, the others clear some.
+void
+many_requests_wait_for_verdicts() {
+    constexpr int kRequests = 70, kReady = 64;
+    Lists lists;
+    nixl_amd_copy_plan_t *plan = nullptr;
+    REQUIRE(lists.request(nullptr, &plan) == 0); // makes the library's stream
+    REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+    static Stream *uploads = nullptr;
+    for (int round = 0; round < 2; ++round) {
+        uploads = g_created;
+        uploads->kernels.clear();
+        uploads->held = true;
+        g_totals.clear();
+        g_synchronized = [](Stream &) {
+            for (int n = 0; n < kRequests; std::this_thread::yield()) {
+                const std::lock_guard<std::recursive_mutex> lock(g_lock);
+                n = launched(*uploads, "list_records_kernel");
+            }
+        };
+        nixl_amd_copy_plan_t *plans[kRequests] = {};
+        std::vector<std::thread> threads;
+        for (nixl_amd_copy_plan_t *&p : plans)
+            threads.emplace_back([&lists, &p] { REQUIRE(lists.request(nullptr, &p) == 0); });
+        for (std::thread &t : threads)
+            t.join();
+        REQUIRE(g_totals.size() == kRequests);
+        REQUIRE(launched(*uploads, "clear_totals_kernel") == kRequests - kReady);
+        for (nixl_amd_copy_plan_t *p : plans)
+            REQUIRE(nixl_amd_copy_plan_destroy(p) == 0);
+        g_synchronized = nullptr;
+    }
+}
+
+// Requests whose launches are refused, the first or a later one, leave their totals to others, at zero.
+void
+refused_launches_keep_no_totals() {
+    Lists lists;
+    nixl_amd_copy_plan_t *plan = nullptr;
+    REQUIRE(lists.request(nullptr, &plan) == 0);
+    REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+    Stream &uploads = *g_created;
+    lists.index.resize(150000); // three launches, as vectors
+    for (size_t i = 0; i < lists.index.size(); ++i)
+        lists.index[i] = static_cast<int32_t>(i * 7919 % Lists::kEntries);
+    for (const int good : {0, 1, 2})
+        for (int i = 0; i < 100; ++i) {
+            g_good_launches = good;
+            g_launch_status = hipErrorOutOfMemory;
+            REQUIRE(lists.request(nullptr, &plan) == NIXL_AMD_ERR_HIP);
+        }
+    uploads.kernels.clear();
+    g_totals.clear();
+    REQUIRE(lists.request(nullptr, &plan) == 0);
+    REQUIRE(launched(uploads, "clear_totals_kernel") == 0);
+    REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -432,10 +498,16 @@ __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *
     return hipSuccess;
 }
 
+static thread_local hipError_t g_last_status = hipSuccess;
+
 hipError_t
 hipLaunchKernel(const void *stub, dim3 grid, dim3, void **args, size_t, hipStream_t stream) {
     LOCKED;
-    if (g_launch_status != hipSuccess) return g_launch_status;
+    g_last_status = g_launch_status != hipSuccess && g_good_launches-- <= 0 ? g_launch_status : hipSuccess;
+    if (g_last_status != hipSuccess) {
+        g_launch_status = hipSuccess; // once
+        return g_last_status;
+    }
     const std::string &name = kernel_names().at(stub);
     Stream &s = stream_of(stream);
     s.kernels.push_back(name);
@@ -474,7 +546,7 @@ hipDeviceGetAttribute(int *value, hipDeviceAttribute_t, int) {
 
 hipError_t
 hipGetLastError() {
-    return g_launch_status;
+    return std::exchange(g_last_status, hipSuccess);
 }
 
 const char *
@@ -485,6 +557,7 @@ hipGetErrorString(hipError_t) {
 hipError_t
 hipMalloc(void **p, size_t n) {
     *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
+    std::memset(*p, 0xa5, n); // nobody may count on zeroes
     return hipSuccess;
 }
 
@@ -518,7 +591,8 @@ hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t 
 
 hipError_t
 hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
-    *s = handle(*new Stream);
+    g_created = new Stream;
+    *s = handle(*g_created);
     return hipSuccess;
 }
 
@@ -542,8 +616,9 @@ hipStreamQuery(hipStream_t stream) {
 
 hipError_t
 hipStreamSynchronize(hipStream_t stream) {
-    LOCKED;
     Stream &s = stream_of(stream);
+    if (g_synchronized) g_synchronized(s);
+    LOCKED;
     s.waited_for = true;
     s.let_go();
     return s.failure;
@@ -615,6 +690,8 @@ main(int argc, char **argv) {
         {"launch_on_the_legacy_stream_fails", launch_on_the_legacy_stream_fails},
         {"launch_on_the_stream_of_a_thread", launch_on_the_stream_of_a_thread},
         {"launch_seen_by_two_threads", launch_seen_by_two_threads},
+        {"many_requests_wait_for_verdicts", many_requests_wait_for_verdicts},
+        {"refused_launches_keep_no_totals", refused_launches_keep_no_totals},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
