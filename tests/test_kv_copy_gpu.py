@@ -1512,6 +1512,19 @@ def test_requests_take_the_streams_in_turn(cuda):
     assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
 
 
+def test_more_listed_requests_at_once_than_totals_are_ready(cuda):
+    """Requests beyond the 64 that find totals ready clear some of their own.  The program is
+    tests/cpp/list_totals_check.cpp."""
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = os.path.join(root, "tests", "cpp", "_build", "list_totals_check")
+    if not os.path.exists(exe):
+        pytest.fail(f"{exe} missing: run __graft_entry__.build() first")
+    proc = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
+
+
 def test_device_memory_view_calls_from_hip(cuda):
     """Memory views and the device-side put / counter add / get-pointer calls over them,
     driven from a HIP program through nixlAgent (tests/cpp/mem_view_device_api.hip; the
