@@ -1782,28 +1782,32 @@ def test_watched_launches_beyond_the_words_and_on_two_streams(cuda):
     busy = torch.zeros(64 << 20, dtype=torch.float32, device=cuda)
     slow, fast = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
+    looked_in_time = 0
     for _ in range(3):
         dst.zero_()
         torch.cuda.synchronize()
         plans = [_plan([(src.data_ptr() + i * blk, dst.data_ptr() + i * blk, blk)]) for i in range(n)]
         with torch.cuda.stream(slow):
-            for _ in range(20):
+            for _ in range(400):  # tens of milliseconds, some times what the launches take
                 busy.add_(1.0)
-        first = torch.cuda.Event()
+        gate = torch.cuda.Event()
+        gate.record(slow)
         for p in plans:
             assert lib.nixl_amd_copy_plan_launch_watched(p, slow.cuda_stream) == 0, _lib.kernels_error()
-            if p is plans[0]:
-                first.record(slow)
         assert lib.nixl_amd_copy_plan_launch_watched(plans[0], fast.cuda_stream) == 0, _lib.kernels_error()
         assert lib.nixl_amd_copy_plan_launch(plans[1], fast.cuda_stream) == 0, _lib.kernels_error()
         fast.synchronize()
         # the launch on the slow stream is still watched, whatever the other one has done
-        assert lib.nixl_amd_copy_plan_status(plans[0], 0) != 0 or first.query()
+        rc = lib.nixl_amd_copy_plan_status(plans[0], 0)
+        if not gate.query():
+            looked_in_time += 1
+            assert rc == -4  # NIXL_AMD_ERR_BUSY
         for p in plans:
             assert lib.nixl_amd_copy_plan_status(p, 1) == 0
             assert lib.nixl_amd_copy_plan_destroy(p) == 0
         torch.cuda.synchronize()
         assert torch.equal(src, dst)
+    assert looked_in_time
 
 
 def test_totals_of_listed_requests_start_at_nothing_every_time(cuda):
