@@ -7,6 +7,7 @@ implementation: a missing library raises ``NativeLibraryMissing``.
 import ctypes
 import importlib.util
 import os
+import sys
 from ctypes import (POINTER, Structure, c_bool, c_char_p, c_float, c_int, c_int64, c_size_t, c_uint16,
                     c_uint, c_uint32, c_uint64, c_void_p)
 
@@ -165,15 +166,27 @@ def ep_kernels():
 _host = None
 
 
+def ep_host_fits():
+    """Whether the module of ep_host() is there and was built for this Python and this torch."""
+    import torch
+    if not os.path.exists(os.path.join(LIB_DIR, "_ep_host.so")):
+        return False
+    try:
+        with open(os.path.join(LIB_DIR, "_ep_host.abi")) as f:
+            return f.read().strip() == f"{sys.implementation.cache_tag} {torch.__version__}"
+    except OSError:
+        return False
+
+
 def ep_host():
     """The allocations and launches of the expert-parallel calls (csrc/ep_host), a Python module over torch."""
     global _host
     if _host is None:
         ep_kernels()
         path = os.path.join(LIB_DIR, "_ep_host.so")
-        if not os.path.exists(path):
-            raise NativeLibraryMissing(f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` first")
-        import torch  # noqa: F401  (the module's symbols are torch's)
+        if not ep_host_fits():  # imports torch, whose symbols the module needs
+            raise NativeLibraryMissing(f"{path} is not built for this Python and torch; "
+                                       "run `python -c 'import __graft_entry__ as g; g.build()'` first")
         spec = importlib.util.spec_from_file_location("_ep_host", path)
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)

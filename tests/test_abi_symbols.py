@@ -111,3 +111,31 @@ def test_product_code_never_reaches_for_the_cpu_oracle():
     for lib in ("libnixl_amd_kernels.so", "libnixl_amd_agent.so", os.path.join("plugins", "libplugin_HIP.so")):
         out = subprocess.run(["readelf", "-d", os.path.join(LIB, lib)], check=True, capture_output=True, text=True).stdout
         assert "oracle" not in out.lower() and "MEMCPY" not in out, lib
+
+
+def test_module_over_torch_is_for_the_python_and_torch_that_load_it(monkeypatch):
+    """A module that was built for another one is not loaded, and is what a new build makes."""
+    import sys
+
+    import torch
+    from nixl_amd import _lib
+    assert _lib.ep_host_fits() and _lib.ep_host()
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    assert not _lib.ep_host_fits()
+    with pytest.raises(_lib.NativeLibraryMissing):
+        _lib.ep_host()
+
+    import __graft_entry__ as g
+    ran = []
+    monkeypatch.setattr(g.subprocess, "run", lambda cmd, **_: ran.append(cmd) or subprocess.CompletedProcess(cmd, 0, "", ""))
+    g._make("oracle")
+    assert f"PYTHON={sys.executable}" in ran[0]
+
+
+def test_libraries_for_cpp_programs_build_without_torch():
+    """`make native` asks no Python for anything."""
+    proc = subprocess.run(["make", "-C", os.path.join(ROOT, "nixl_amd", "csrc"), "-n", "-B", "native", "PYTHON=false"],
+                          capture_output=True, text=True)
+    assert proc.returncode == 0 and "libplugin_HIP.so" in proc.stdout and "-ltorch" not in proc.stdout, proc.stdout + proc.stderr
+    assert "false -c" not in proc.stdout
