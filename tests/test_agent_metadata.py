@@ -376,6 +376,17 @@ def test_host_side_of_copy_plans_on_the_cpu(scenario):
     assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
 
 
+def test_division_by_multiplication_on_the_cpu():
+    """tests/cpp/fast_div_check.hip: the quotients by which the copy and row kernels address memory."""
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = os.path.join(root, "tests", "cpp", "_build", "fast_div_check")
+    if not os.path.exists(exe):
+        pytest.fail(f"{exe} missing: run __graft_entry__.build() first")
+    proc = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
+
+
 def test_list_and_option_helpers_of_the_c_wrapper(two_agents):
     """The descriptor-list, option and stub helpers of the reference's C wrapper
     (src/bindings/rust/wrapper.h:193-201,297-326,457) behave as their names say; the metadata
