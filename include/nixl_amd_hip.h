@@ -277,10 +277,10 @@ nixl_amd_copy_plan_create_listed_on(const nixl_amd_copy_list_t *src,
 int
 nixl_amd_copy_plan_launch(nixl_amd_copy_plan_t *plan, void *stream);
 
-/* The same for a plan whose destinations are device memory.  Status and destroy then look at a word
- * in host memory that the launch's last kernel writes instead of at an event behind it, which shows
- * the end some microseconds sooner.  (A word says nothing of caches over host memory, for which an
- * event is what releases them.)  Needs nixl_amd_copy_watch_prepare, which allocates the words once a
+/* The same for a plan whose destinations are memory of the plan's own device.  Status and destroy then
+ * look at a word in host memory that the launch's last kernel writes instead of at an event behind it,
+ * which shows the end some microseconds sooner.  (A word says nothing of caches over host memory or
+ * another device's, for which an event is what releases them.)  `stream` lives until the end has been seen.  Needs nixl_amd_copy_watch_prepare, which allocates the words once a
  * process; without it, for more than 128 launches in flight on a device, for a plan whose earlier
  * launch is still running, and on the default streams, an event is recorded as
  * nixl_amd_copy_plan_launch does. */

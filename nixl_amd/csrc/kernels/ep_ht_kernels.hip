@@ -332,8 +332,11 @@ ht_prefix_kernel(const int *__restrict__ channel_prefix, HtNotifyOut o, int R, i
 // rank's tokens, eight loads in flight a lane, and counts bytes (eight destinations an addition)
 // that are widened once a step.  Up to so many tokens that the one workgroup is not slower than the
 // launch (layout, scan and this behind one another, one launch and two, us): 8 x 1024 tokens 8.0 and
-// 10.5, 8 x 5120 13.5 and 14.3, 8 x 6000 14.5 and 13.0; 4 x 12 288 13.9 and 14.6, 4 x 16 384 16.2 and 15.7. Where a
-// token's flags are no word that one load takes: 7 x 250 10.9 and 11.8, 6 x 600 13.3 and 10.2.
+// 10.5, 8 x 5120 13.5 and 14.3, 8 x 6000 14.5 and 13.0; 4 x 12 288 13.9 and 14.6, 4 x 16 384 16.2 and 15.7.
+// Where a token's flags are no word that one load takes, the kernels alone are as fast in two launches from some 4000
+// flags on (6 x 200 10.2 and 9.2), but the host has a launch more in front of its wait for the counts: whole passes
+// of layout, dispatch and combine (hidden 2048) take 38.2 and 39.7 for 6 x 200, 38.8 and 39.1 for 6 x 340, 39.1 and
+// 38.2 for 6 x 400; 5 x 491 40.0 and 38.5, 3 x 1365 42.1 and 42.0, 2 x 3072 42.7 and 43.2, 1 x 12 000 51.0 and 52.7.
 constexpr int kNotifyTokensOf8 = 40960, kNotifyTokensOf4 = 57344; // R * T
 constexpr int kNotifyFlags = 12288; // R * T * R, other numbers of ranks
 constexpr int kNotifyPerLane = 8; // tokens a lane counts at a time, their loads together
