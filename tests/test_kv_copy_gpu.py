@@ -1780,8 +1780,24 @@ def test_watched_launches_beyond_the_words_and_on_two_streams(cuda):
     src = torch.randint(0, 256, (n, blk), dtype=torch.uint8, device=cuda)
     dst = torch.zeros_like(src)
     busy = torch.zeros(64 << 20, dtype=torch.float32, device=cuda)
-    slow, fast = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
+
+    def runs_beside(stream, other):
+        """Whether `other` does not wait for `stream`: streams share the few hardware queues of a process."""
+        with torch.cuda.stream(stream):
+            for _ in range(400):  # tens of milliseconds
+                busy.add_(1.0)
+        there, aside = torch.cuda.Event(), torch.cuda.Event()
+        there.record(stream)
+        aside.record(other)
+        while not aside.query() and not there.query():
+            pass
+        beside = not there.query()
+        torch.cuda.synchronize()
+        return beside
+
+    slow = torch.cuda.Stream()
+    fast = next(s for s in [torch.cuda.Stream() for _ in range(16)] if runs_beside(slow, s))
     looked_in_time = 0
     for _ in range(3):
         dst.zero_()
