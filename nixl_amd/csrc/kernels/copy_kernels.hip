@@ -150,6 +150,17 @@ store16(uint64_t addr, const v4u &v) {
         asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(g), "v"(v) : "memory");
 }
 
+// The same for a line that is not written whole, without the streaming hint: such a store goes to memory as
+// a partial write at once, an ordinary one does not (kept plain by the policy that is plain throughout).
+template<int POL>
+__device__ __forceinline__ void
+store16_part(uint64_t addr, const v4u &v) {
+    if constexpr (POL == kPolPlain)
+        store16<POL>(addr, v);
+    else
+        asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"((gv4_ptr)(addr)), "v"(v) : "memory");
+}
+
 // Workgroups are handed to the 8 dies round-robin.  With the swizzle on, die x works
 // through one contiguous eighth of the record array instead of every eighth record.
 __device__ __forceinline__ uint32_t
@@ -335,7 +346,14 @@ copy_piece_kernel(const PieceRec *__restrict__ recs, uint32_t n_recs, uint32_t p
     // so that shift + units <= kPieceUnits), and each store instruction then writes whole
     // lines except at the two ends of the piece.  A line written half by one instruction
     // and half by the next would go out as two partial writes.
+    //
+    // What bounds it is the memory's writes at random places, and of those the partial ones: the lines
+    // at the two ends are stored without the streaming hint.  262 144 descriptors, log-uniform
+    // lengths, us with the hint everywhere and so: 512 B to 4 KiB at 16-byte addresses 206 and 191, 512 B to
+    // 2 KiB 141 and 126, 256 B to 2 KiB 115 and 104; at 64-byte and 128-byte addresses no difference (187 and 186, 178
+    // and 178).  Whole lines without it 258; only what is no whole half of a line without it 208 to 343.
     const uint32_t shift = static_cast<uint32_t>(rec.dst >> 4) & 7u;
+    const uint32_t end = shift + units;
     // Loads are unconditional (a lane outside the piece re-reads its first or last unit) so
     // that all of them are in flight together; only the stores are predicated.
     v4u v[LOADS];
@@ -347,8 +365,12 @@ copy_piece_kernel(const PieceRec *__restrict__ recs, uint32_t n_recs, uint32_t p
     }
 #pragma unroll
     for (int k = 0; k < LOADS; ++k) {
-        const uint32_t at = k * kWaveSize + lane;
-        if (at >= shift && at - shift < units) store16<POL>(rec.dst + (at - shift) * 16ull, v[k]);
+        const uint32_t at = k * kWaveSize + lane, line = at & ~7u; // first unit of the lane's line
+        if (at < shift || at >= end) continue;
+        if (line >= shift && line + 8 <= end)
+            store16<POL>(rec.dst + (at - shift) * 16ull, v[k]);
+        else
+            store16_part<POL>(rec.dst + (at - shift) * 16ull, v[k]);
     }
 }
 

@@ -1485,6 +1485,23 @@ def test_piece_path_line_misaligned_and_split(cuda):
     assert info.uniform_chunks == 32 and info.piece_items == 1
 
 
+@pytest.mark.parametrize("nt", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("waves", [1, 2, 4])
+def test_pieces_that_share_their_first_and_last_lines(cuda, nt, waves):
+    """Pieces whose destinations adjoin at 16-byte addresses: the lines at their ends are written in part by
+    two wavefronts each, every other line whole, at every place inside a line and with every form of stores;
+    the bytes before the first piece and behind the last stay."""
+    import torch
+    units = [16 + (i % 9) for i in range(144)] + [255, 249, 256, 256, 257, 263, 264, 511, 17, 16]
+    lens = [16 * u for u in units]
+    ends = np.cumsum(lens)
+    so = [256 * 48 * i + 16 * (i % 8) for i in range(len(lens))]
+    half = 2 << 20
+    do = [half + 16 + int(e) - n for e, n in zip(ends, lens)]
+    info = _check_against_oracle(torch, cuda, 2 * half, so, do, lens, (1, nt, 0, waves, 0), seed=15)
+    assert info.piece_items >= len(lens) and info.generic_descs == 0 and info.uniform_chunks == 0
+
+
 def test_raw_south_bound_api_from_cpp(cuda):
     """The plugin driven from C++ through nixlBackendEngine alone (no agent): plugin table,
     registerMem / loadLocalMD, prepXfer / postXfer / checkXfer for WRITE and READ, handle
