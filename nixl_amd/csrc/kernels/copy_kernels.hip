@@ -150,8 +150,8 @@ store16(uint64_t addr, const v4u &v) {
         asm volatile("global_store_dwordx4 %0, %1, off sc1 nt\n\ts_nop 1" : : "v"(g), "v"(v) : "memory");
 }
 
-// The same for a line that is not written whole, without the streaming hint: such a store goes to memory as
-// a partial write at once, an ordinary one does not (kept plain by the policy that is plain throughout).
+// The same for a line that is not written whole, without the streaming hint: with it such a store goes to memory
+// as a partial write at once.
 template<int POL>
 __device__ __forceinline__ void
 store16_part(uint64_t addr, const v4u &v) {
@@ -322,6 +322,19 @@ upload_kernel(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t n) 
 // kPieceLoads 128-bit loads in flight per lane, then the stores.  No search and no LDS:
 // the shape for descriptors of a few hundred bytes to a few KiB.
 
+// Cache policy of pieces by the bytes of their request: ordinary loads while what is read and written fits the
+// last-level cache of 256 MiB, non-temporal ones beyond (lines of the destination stay there instead).  One request again and
+// again | three with buffers of their own in turn, us from launch to end, ordinary and non-temporal loads (and
+// non-temporal loads and stores throughout), 512 B to 4 KiB, 1024 pieces 8.8 8.8 (9.2) | 8.8 8.8 (9.2); 8192 10.7 11.8 (13.6) |
+// 12.2 14.0 (13.9); 16 384 14.6 18.3 (20.0) | 17.2 20.3 (20.3); 65 536, 113 MB, 42.4 54.5 (57.9) | 54.4 54.6 (58.6); 131 072, 225 MB,
+// 90.8 99.6 (108) | 106.9 99.4 (108); 512 B to 2 KiB, 131 072, 144 MB, 62.8 67.7 (76.6) | 74.9 67.7 (76.5).
+constexpr uint64_t kPiecesInCache = 112ull << 20;
+
+int
+piece_policy(uint64_t payload) {
+    return payload <= kPiecesInCache ? kPolPlainSc1Nt : kPolNtSc1Nt;
+}
+
 constexpr int kPieceLoads = 4;
 constexpr uint32_t kPieceUnits = kWaveSize * kPieceLoads; // 4 KiB
 
@@ -351,7 +364,7 @@ copy_piece_kernel(const PieceRec *__restrict__ recs, uint32_t n_recs, uint32_t p
     // at the two ends are stored without the streaming hint.  262 144 descriptors, log-uniform
     // lengths, us with the hint everywhere and so: 512 B to 4 KiB at 16-byte addresses 206 and 191, 512 B to
     // 2 KiB 141 and 126, 256 B to 2 KiB 115 and 104; at 64-byte and 128-byte addresses no difference (187 and 186, 178
-    // and 178).  Whole lines without it 258; only what is no whole half of a line without it 208 to 343.
+    // and 178).  Whole lines without it 258; only what is no whole half of a line without it 208.
     const uint32_t shift = static_cast<uint32_t>(rec.dst >> 4) & 7u;
     const uint32_t end = shift + units;
     // Loads are unconditional (a lane outside the piece re-reads its first or last unit) so
@@ -1251,7 +1264,7 @@ struct nixl_amd_copy_plan {
     int device = 0;
     int upl = 1;
     int policy = kPolNtSc1Nt;
-    int piece_policy = kPolNtNt; // pieces of a few hundred bytes to 4 KiB: 225 us for the 262 144-descriptor stress, against 239 (4) and 285 (3)
+    int piece_policy = kPolNtSc1Nt; // piece_policy()
     int waves = 1;
     int swizzle = 0;
     uint32_t max_wgs = 0;
@@ -2175,7 +2188,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         nt = (pairs == 0 || 2 * regular >= pairs) ? kPolNtSc1Nt : kPolPlainSc1Nt;
     }
     plan->policy = nt;
-    if (tuning && tuning->nontemporal) plan->piece_policy = tuning->nontemporal;
+    plan->piece_policy = tuning && tuning->nontemporal ? tuning->nontemporal : piece_policy(payload);
     plan->waves = waves;
     plan->swizzle = swizzle;
     plan->max_wgs = max_wgs;
@@ -2645,7 +2658,6 @@ create_listed(const nixl_amd_copy_list_t *src,
     plan->swizzle = t.swizzle;
     plan->max_wgs = t.max_wgs;
     plan->policy = t.nt ? t.nt : kPolNtSc1Nt;
-    if (t.nt) plan->piece_policy = t.nt;
     // one arena: the totals, then the records
     constexpr size_t kRecsAt = 256;
     hipStream_t up = nullptr;
@@ -2714,6 +2726,7 @@ create_listed(const nixl_amd_copy_list_t *src,
     plan->arena_bytes = kRecsAt + (n + got.extra) * sizeof(PieceRec);
     plan->piece_recs = recs;
     plan->n_pieces = static_cast<uint32_t>(n + got.extra);
+    plan->piece_policy = t.nt ? t.nt : piece_policy(got.bytes);
     plan->info.payload_bytes = got.bytes;
     plan->info.vec_descs = n;
     plan->info.plan_device_bytes = plan->arena_bytes;
