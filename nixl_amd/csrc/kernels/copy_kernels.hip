@@ -662,9 +662,10 @@ index_records_runs_kernel(UniformRec *recs, IndexVector src_index, IndexVector d
 //
 // The verdict reaches the host through pinned memory, written by the workgroup that finishes last;
 // the host waits for it, because a bad pair must fail the request.  A workgroup adds to the totals
-// with two atomics (all dies add to one line).  Kernel time: 65 536 pairs as vectors 22.5 us with an
-// atomic for every descriptor of several pieces and four a workgroup of 256 pairs, 19.2 now; as
-// runs of 64 pairs 9.9, and 262 144 pairs 14.8 (as vectors in four launches 77).
+// with two atomics (all dies add to one line), and nothing in front of the verdict writes a cache back: a
+// device-scope fence around the additions did, for records that only the next kernel reads.  Kernel time, with such
+// fences and sums over a wave through LDS, and without: runs of 64 pairs, 1024 pairs 8.0 and 6.4 us, 16 384 9.9 and
+// 8.1, 65 536 10.9 and 8.7, 262 144 15.5 and 13.8; vectors, 1024 pairs 6.8 and 5.3, 65 536 19.2 and 18.1.
 struct IndexRun {
     uint32_t first; // pair the run starts with; it ends where the next one starts
     uint32_t src, dst; // indices of that pair
@@ -724,8 +725,8 @@ template<bool RUNS>
 __global__ void __launch_bounds__(kListThreads)
 list_records_kernel(ListArgs a) {
     constexpr int kWaves = kListThreads / kWaveSize;
-    __shared__ unsigned long long wave_bytes[kWaves];
-    __shared__ uint32_t wave_bad[kWaves], wave_continued[kWaves], wave_extra[kWaves], extra_at;
+    static_assert(kListThreads * kListMaxBytes <= 0xffffffffu);
+    __shared__ uint32_t wave_bytes[kWaves], wave_bad[kWaves], wave_continued[kWaves], wave_extra[kWaves], extra_at;
     __shared__ IndexRun runs[RUNS ? kListThreads + 1 : 1];
     __shared__ uint2 last[RUNS ? 1 : kWaves];
     const uint32_t workgroup = a.first_workgroup + blockIdx.x, i = workgroup * kListThreads + threadIdx.x;
@@ -780,16 +781,10 @@ list_records_kernel(ListArgs a) {
     const uint32_t mine = (more + kPieceUnits - 1) / kPieceUnits; // records beyond the first
     if (good) a.recs[i] = PieceRec{s.addr, d.addr | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
 
+    // sums over a workgroup fit 32 bits: at most kListMaxBytes a pair
     const uint32_t n_bad = __popcll(__ballot(here && !good));
     const uint32_t n_continued = __popcll(__ballot(good && follows && s.continues && d.continues));
-    unsigned long long bytes = good ? s.len : 0;
-    uint32_t incl = mine;
-#pragma unroll
-    for (int off = 1; off < kWaveSize; off <<= 1) {
-        bytes += __shfl_xor(bytes, off);
-        const uint32_t up = __shfl_up(incl, off);
-        if (lane >= off) incl += up;
-    }
+    const uint32_t bytes = wave_sum_dpp(good ? s.len : 0), incl = wave_scan_dpp(mine);
     if (lane == kWaveSize - 1) {
         wave_bytes[wave] = bytes;
         wave_bad[wave] = n_bad;
@@ -797,44 +792,40 @@ list_records_kernel(ListArgs a) {
         wave_extra[wave] = incl;
     }
     __syncthreads();
+    uint32_t sum = 0, b = 0; // of the workgroup, in the first wave
     if (wave == 0) {
-        unsigned long long sum = lane < kWaves ? wave_bytes[lane] : 0;
-        uint32_t b = lane < kWaves ? wave_bad[lane] : 0, c = lane < kWaves ? wave_continued[lane] : 0;
-        const uint32_t x = lane < kWaves ? wave_extra[lane] : 0;
-        uint32_t run = x;
-#pragma unroll
-        for (int off = 1; off < kWaves; off <<= 1) {
-            sum += __shfl_xor(sum, off);
-            b += __shfl_xor(b, off);
-            c += __shfl_xor(c, off);
-            const uint32_t up = __shfl_up(run, off);
-            if (lane >= off) run += up;
-        }
+        sum = wave_sum_dpp(lane < kWaves ? wave_bytes[lane] : 0);
+        b = wave_sum_dpp(lane < kWaves ? wave_bad[lane] : 0);
+        const uint32_t c = wave_sum_dpp(lane < kWaves ? wave_continued[lane] : 0);
+        const uint32_t x = lane < kWaves ? wave_extra[lane] : 0, run = wave_scan_dpp(x);
         if (lane < kWaves) wave_extra[lane] = run - x; // records of the waves before
-        const uint32_t extra = __shfl(run, kWaves - 1);
-        if (lane == 0) {
-            const unsigned long long packed = extra | static_cast<unsigned long long>(c) << 32;
-            if (packed) extra_at = static_cast<uint32_t>(atomicAdd(&a.totals->extra_continued, packed));
+        if (lane == kWaves - 1) {
+            const unsigned long long packed = run | static_cast<unsigned long long>(c) << 32;
             if (b) atomicAdd(&a.totals->bad, b);
-            __threadfence();
-            const unsigned long long before = atomicAdd(&a.totals->bytes_arrived, sum | 1ull << kListBytesBits);
-            if (before >> kListBytesBits == a.n_workgroups - 1) {
-                __threadfence();
-                const unsigned long long both = __hip_atomic_load(&a.totals->extra_continued, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                const uint32_t bad = __hip_atomic_load(&a.totals->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&a.totals->bytes_arrived, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&a.totals->extra_continued, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&a.totals->bad, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __threadfence();
-                a.verdict->bytes = (before & ((1ull << kListBytesBits) - 1)) + sum;
-                a.verdict->bad = bad;
-                a.verdict->continued = static_cast<uint32_t>(both >> 32);
-                a.verdict->extra = static_cast<uint32_t>(both);
-                __hip_atomic_store(&a.verdict->there, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
+            if (packed) extra_at = static_cast<uint32_t>(atomicAdd(&a.totals->extra_continued, packed));
         }
     }
     __syncthreads();
+    if (threadIdx.x == kWaves - 1) {
+        // The verdict waits for nothing but additions, which are done where all dies see them: no cache is written
+        // back for it (the records are for the kernel behind this one).
+        const auto settle = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+        settle(); // this workgroup's additions
+        const unsigned long long before = __hip_atomic_fetch_add(&a.totals->bytes_arrived, sum | 1ull << kListBytesBits,
+                                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before >> kListBytesBits == a.n_workgroups - 1) {
+            const unsigned long long both = __hip_atomic_exchange(&a.totals->extra_continued, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint32_t bad = __hip_atomic_exchange(&a.totals->bad, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&a.totals->bytes_arrived, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const auto tell = [](auto *where, auto what) { __hip_atomic_store(where, what, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+            tell(&a.verdict->bytes, (before & ((1ull << kListBytesBits) - 1)) + sum);
+            tell(&a.verdict->bad, bad);
+            tell(&a.verdict->continued, static_cast<uint32_t>(both >> 32));
+            tell(&a.verdict->extra, static_cast<uint32_t>(both));
+            settle(); // the totals are zero, the words in front of the last one there
+            tell(&a.verdict->there, 1u);
+        }
+    }
     if (!more) return;
     uint32_t at = a.n + extra_at + wave_extra[wave] + (incl - mine);
     for (uint32_t first = count; more; first += count, more -= count) {

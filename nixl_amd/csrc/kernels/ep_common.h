@@ -139,30 +139,6 @@ wave_reduce_dpp(int x, Op op) {
     return __builtin_amdgcn_readlane(x, kEpWaveSize - 1);
 }
 
-// Sum of one 32-bit value per lane over the wave, or of 16-bit fields that do not overflow: in every lane.
-__device__ __forceinline__ uint32_t
-wave_sum_dpp(uint32_t x) {
-    x += __builtin_amdgcn_update_dpp(0u, x, 0xb1, 0xf, 0xf, false); // quad_perm [1,0,3,2]
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x4e, 0xf, 0xf, false); // quad_perm [2,3,0,1]
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x124, 0xf, 0xf, false); // row_ror 4
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x128, 0xf, 0xf, false); // row_ror 8
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x142, 0xa, 0xf, false); // row_bcast 15 into rows 1 and 3
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x143, 0xc, 0xf, false); // row_bcast 31 into rows 2 and 3
-    return __builtin_amdgcn_readlane(x, kEpWaveSize - 1);
-}
-
-// The same up to and with each lane.
-__device__ __forceinline__ uint32_t
-wave_scan_dpp(uint32_t x) {
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x111, 0xf, 0xf, false); // row_shr 1
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x112, 0xf, 0xf, false); // row_shr 2
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x114, 0xf, 0xf, false); // row_shr 4
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x118, 0xf, 0xf, false); // row_shr 8
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x142, 0xa, 0xf, false); // row_bcast 15 into rows 1 and 3
-    x += __builtin_amdgcn_update_dpp(0u, x, 0x143, 0xc, 0xf, false); // row_bcast 31 into rows 2 and 3
-    return x;
-}
-
 // Order-preserving map of a float onto a signed integer (negative floats reversed), so that
 // integer max is float max; -0.0 and +0.0 stay distinct neighbours, which the tie rule of the
 // values below undoes by comparing the floats themselves.
