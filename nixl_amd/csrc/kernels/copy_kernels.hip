@@ -122,8 +122,21 @@ using gv4_cptr = const __attribute__((address_space(1))) v4u_any *;
 //   3  plain loads, sc1 nt stores       6.65       6.07         5.90          5.31
 //   4  nt loads,    sc1 nt stores       6.71       6.35         5.80          5.15
 // "sc1 nt" is a streaming store with device scope.  A plan whose destinations adjoin or
-// advance by a constant step takes 4, any other plan 3.
+// advance by a constant step takes 4, any other plan 3; and 3 any plan whose payload is read and
+// written inside the last-level cache of 256 MiB (copy_policy).  Policies 4 and 3 there, us from launch to
+// end, three requests with buffers of their own in turn (and one again and again):
+//                16 MiB       32 MiB       64 MiB       96 MiB       112 MiB      128 MiB
+//   seq->seq     12.5 12.2    18.0 16.8    27.9 25.5    37.6 38.0    42.5 43.4    47.4 48.5 (48.0 42.9)
+//   random->seq  12.9 12.2    19.0 17.0    29.6 27.8    40.2 38.1    45.5 45.2    50.8 51.6 (50.7 44.6)
+//   seq->random  13.2 12.4    19.8 17.2    31.9 26.7    45.0 44.2    51.2 51.0    56.9 56.3 (56.7 45.6)
 constexpr int kPolNtNt = 1, kPolPlain = 2, kPolPlainSc1Nt = 3, kPolNtSc1Nt = 4;
+constexpr uint64_t kInLastLevelCache = 112ull << 20; // of payload
+
+// `regular`: destinations adjoin, advance by a constant step or are sorted, or the copy does not depend on it.
+constexpr int
+copy_policy(uint64_t payload, bool regular) {
+    return regular && payload > kInLastLevelCache ? kPolNtSc1Nt : kPolPlainSc1Nt;
+}
 
 template<int POL>
 __device__ __forceinline__ v4u
@@ -322,19 +335,11 @@ upload_kernel(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t n) 
 // kPieceLoads 128-bit loads in flight per lane, then the stores.  No search and no LDS:
 // the shape for descriptors of a few hundred bytes to a few KiB.
 
-// Cache policy of pieces by the bytes of their request: ordinary loads while what is read and written fits the
-// last-level cache of 256 MiB, non-temporal ones beyond (lines of the destination stay there instead).  One request again and
+// Loads of pieces are ordinary or non-temporal by the bytes of their request alone.  One request again and
 // again | three with buffers of their own in turn, us from launch to end, ordinary and non-temporal loads (and
 // non-temporal loads and stores throughout), 512 B to 4 KiB, 1024 pieces 8.8 8.8 (9.2) | 8.8 8.8 (9.2); 8192 10.7 11.8 (13.6) |
 // 12.2 14.0 (13.9); 16 384 14.6 18.3 (20.0) | 17.2 20.3 (20.3); 65 536, 113 MB, 42.4 54.5 (57.9) | 54.4 54.6 (58.6); 131 072, 225 MB,
 // 90.8 99.6 (108) | 106.9 99.4 (108); 512 B to 2 KiB, 131 072, 144 MB, 62.8 67.7 (76.6) | 74.9 67.7 (76.5).
-constexpr uint64_t kPiecesInCache = 112ull << 20;
-
-int
-piece_policy(uint64_t payload) {
-    return payload <= kPiecesInCache ? kPolPlainSc1Nt : kPolNtSc1Nt;
-}
-
 constexpr int kPieceLoads = 4;
 constexpr uint32_t kPieceUnits = kWaveSize * kPieceLoads; // 4 KiB
 
@@ -1255,7 +1260,7 @@ struct nixl_amd_copy_plan {
     int device = 0;
     int upl = 1;
     int policy = kPolNtSc1Nt;
-    int piece_policy = kPolNtSc1Nt; // piece_policy()
+    int piece_policy = kPolNtSc1Nt;
     int waves = 1;
     int swizzle = 0;
     uint32_t max_wgs = 0;
@@ -1923,7 +1928,7 @@ build_block_plan(int device, const Tuning &t, void *staging, size_t staging_cap,
     const bool scattered = !(steps == 0 || 2 * regular >= steps);
     // a scatter out of consecutive memory is put into ascending destination order, window by window
     const bool sort = scattered && t.sort_scatter != 2 && 2 * src_follows >= steps && n_recs >= kSortWindow;
-    plan->policy = t.nt ? t.nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
+    plan->policy = t.nt ? t.nt : copy_policy(n_recs * len, !scattered || sort);
     if (fits_inline(n_recs, len, t)) {
         plan->inline_recs = std::make_unique<InlineRecs>();
         std::memcpy(plan->inline_recs->rec, recs, bytes);
@@ -2176,10 +2181,10 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             prev_dst = descs[i].dst;
             prev_end = descs[i].dst + descs[i].len;
         }
-        nt = (pairs == 0 || 2 * regular >= pairs) ? kPolNtSc1Nt : kPolPlainSc1Nt;
+        nt = copy_policy(payload, pairs == 0 || 2 * regular >= pairs);
     }
     plan->policy = nt;
-    plan->piece_policy = tuning && tuning->nontemporal ? tuning->nontemporal : piece_policy(payload);
+    plan->piece_policy = tuning && tuning->nontemporal ? tuning->nontemporal : copy_policy(payload, true);
     plan->waves = waves;
     plan->swizzle = swizzle;
     plan->max_wgs = max_wgs;
@@ -2442,7 +2447,7 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
     plan->upl = upl;
     plan->waves = waves;
     plan->swizzle = swizzle;
-    plan->policy = nt ? nt : ((!scattered || sort) ? kPolNtSc1Nt : kPolPlainSc1Nt);
+    plan->policy = nt ? nt : copy_policy(n * len, !scattered || sort);
     if (inlined) {
         const auto address = [](const nixl_amd_copy_run_t *runs, size_t n_runs, uint64_t index) {
             const auto *run = std::upper_bound(runs, runs + n_runs, index, [](uint64_t i, const nixl_amd_copy_run_t &r) { return i < r.first_index; }) - 1;
@@ -2717,7 +2722,7 @@ create_listed(const nixl_amd_copy_list_t *src,
     plan->arena_bytes = kRecsAt + (n + got.extra) * sizeof(PieceRec);
     plan->piece_recs = recs;
     plan->n_pieces = static_cast<uint32_t>(n + got.extra);
-    plan->piece_policy = t.nt ? t.nt : piece_policy(got.bytes);
+    plan->piece_policy = t.nt ? t.nt : copy_policy(got.bytes, true);
     plan->info.payload_bytes = got.bytes;
     plan->info.vec_descs = n;
     plan->info.plan_device_bytes = plan->arena_bytes;
