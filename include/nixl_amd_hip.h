@@ -51,13 +51,15 @@ typedef struct nixl_amd_copy_tuning {
     int units_per_lane; /* 16-byte units one lane moves per chunk: 1, 2, 4, 8 or 16 */
     int nontemporal; /* cache policy: 1 = non-temporal loads and stores, 2 = plain, 3 = plain loads and
                       * streaming device-scope stores, 4 = non-temporal loads and streaming
-                      * device-scope stores; 0 = 4 if the destinations of consecutive
-                      * descriptors adjoin or advance by a constant step, else 3 */
+                      * device-scope stores; 0 = 4 if the request is longer than the last-level cache can
+                      * hold and the destinations of consecutive descriptors adjoin or advance by a
+                      * constant step, else 3 */
     int max_workgroups; /* grid cap of the mixed and byte-path kernels; waves loop beyond it */
     int waves_per_workgroup; /* uniform-chunk kernel: 1, 2, 4, 8 or 16 */
     int xcd_swizzle; /* 1 = each accelerator die walks a contiguous slice of the chunk list, 2 = off */
     int sort_scatter; /* a plan that scatters consecutive memory over irregular destinations has its records put
-                       * into ascending destination order inside windows of 1024 (on the device): 1 = on, 2 = off */
+                       * into ascending destination order inside windows of 1024 (on the device): 1 = on, 2 = off,
+                       * 0 = on for requests of more than 512 MiB */
     /* The HIP stream the plan will be launched on, or NULL.  While that stream is idle the
      * kernels that write the plan's arrays are queued on it, so that a launch needs no wait; the
      * stream must then outlive the plan, and while it is under capture the plan can be launched

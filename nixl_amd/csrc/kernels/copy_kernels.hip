@@ -1662,6 +1662,21 @@ block_len_fits(uint64_t len, const Tuning &t) {
     return len >= 8192 && len % chunk_bytes == 0;
 }
 
+// Whether a plan that scatters `n` equal blocks out of consecutive memory has its records sorted, unless the caller
+// says so or not (tuning field `sort_scatter`).  Sorted, the writes find DRAM pages open; but sorting takes 4 us more in
+// front of the copy, and the loads of unsorted records are ordinary ones.  Requests made, moved and waited for, three
+// with pools of their own in turn, sorted and not, us: blocks of 8 KiB, 38 MB 32.1 and 27.5, 118 MB 60.6 and 55.8, 354 MB 141 and
+// 138, 590 MB 225 and 222; of 9 KiB 18 MB 25.7 and 21.2, 225 MB 98.9 and 94.3, 562 MB 225 and 217; of 16 KiB 34 MB 30.1 and
+// 25.6, 168 MB 74.3 and 71.5, 420 MB 157 and 156, 629 MB 226.9 and 229.1, 1049 MB 370.4 and 373.0; of 64 KiB 67 MB 38.8 and 34.2,
+// 537 MB 183 and 182, 839 MB 275 and 274.
+constexpr uint64_t kSortScatterFrom = 512ull << 20;
+
+static bool
+sort_pays(int sort_scatter, size_t n, uint64_t len) {
+    if (sort_scatter == 2 || n < kSortWindow) return false;
+    return sort_scatter == 1 || n * len > kSortScatterFrom;
+}
+
 // Whether a plan of `n` equal blocks can carry its records as kernel arguments: few enough, and
 // the launch shape the inline kernel has.
 static bool
@@ -1927,7 +1942,7 @@ build_block_plan(int device, const Tuning &t, void *staging, size_t staging_cap,
     // cache policy by destination pattern, as in the general lowering
     const bool scattered = !(steps == 0 || 2 * regular >= steps);
     // a scatter out of consecutive memory is put into ascending destination order, window by window
-    const bool sort = scattered && t.sort_scatter != 2 && 2 * src_follows >= steps && n_recs >= kSortWindow;
+    const bool sort = scattered && sort_pays(t.sort_scatter, n_recs, len) && 2 * src_follows >= steps;
     plan->policy = t.nt ? t.nt : copy_policy(n_recs * len, !scattered || sort);
     if (fits_inline(n_recs, len, t)) {
         plan->inline_recs = std::make_unique<InlineRecs>();
@@ -2167,8 +2182,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->upl = upl;
     if (nt == 0) {
         // Destinations that adjoin (a gather into staging, one long copy) or advance by a
-        // constant step (the same block of every layer of a pool) take non-temporal loads;
-        // destinations without such a pattern (a scatter over a pool) take plain loads.
+        // constant step (the same block of every layer of a pool) take non-temporal loads where they
+        // are long; destinations without such a pattern (a scatter over a pool) take plain loads.
         uint64_t pairs = 0, regular = 0, prev_dst = 0, prev_end = 0, prev_step = 0;
         for (size_t i = 0; i < n; ++i) {
             if (descs[i].len == 0) continue;
@@ -2436,7 +2451,7 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         return nixl_amd_fail(NIXL_AMD_ERR_INDEX, "plan_create_indexed: an index names no entry of its list");
     }
     const bool scattered = !(n == 1 || 2 * static_cast<uint64_t>(dst_facts.regular) >= n - 1);
-    const bool sort = scattered && sort_scatter != 2 && src_all_dense && 2 * static_cast<uint64_t>(src_facts.ones) >= n - 1 && n >= kSortWindow;
+    const bool sort = scattered && sort_pays(sort_scatter, n, len) && src_all_dense && 2 * static_cast<uint64_t>(src_facts.ones) >= n - 1;
     if (tables && !inlined) {
         auto *up_runs = reinterpret_cast<nixl_amd_copy_run_t *>(static_cast<uint8_t *>(staging) + table_at);
         std::memcpy(up_runs, src_runs, n_src_runs * sizeof(nixl_amd_copy_run_t));

@@ -113,6 +113,39 @@ def test_scatter_of_consecutive_memory_matches_oracle(cuda, n, sort_scatter):
     assert info.uniform_chunks == n * (blk // 1024) and info.mixed_chunks == 0 and info.piece_items == 0
 
 
+@pytest.mark.parametrize("n", [1023, 1024, 1025, 3000])
+@pytest.mark.parametrize("form", ["descriptors", "strides", "runs"])
+def test_scatter_sorted_because_the_caller_says_so(cuda, form, n):
+    """sort_scatter=1 at the edges of the sorting windows and far below the bytes from which a request is sorted
+    by itself: equal blocks out of consecutive memory, from descriptors and from index vectors (whose records a kernel
+    sorts as it makes them), one destination run and two."""
+    import torch
+    lib = _lib.kernels()
+    rng = np.random.default_rng(n)
+    blk, pool = 8192, n + 13
+    half = n * blk
+    perm = rng.permutation(pool)[:n].astype(np.int32)
+    so, do = np.arange(n) * blk, half + perm.astype(np.int64) * blk
+    if form == "descriptors":
+        _check_against_oracle(torch, cuda, half + pool * blk, so, do, [blk] * n, (0, 0, 0, 0, 0, 1), seed=n)
+        return
+    host = rng.integers(0, 256, half + pool * blk, dtype=np.uint8)
+    dev = torch.from_numpy(host.copy()).to(cuda)
+    base = dev.data_ptr()
+    tuning = _lib.CopyTuning(0, 0, 0, 0, 0, 1)
+    flat = np.arange(n, dtype=np.int32)
+    src = (_lib.CopyRun * 1)(_lib.CopyRun(base, blk, 0, n))
+    cut = pool if form == "strides" else 7
+    dst = (_lib.CopyRun * 2)(_lib.CopyRun(base + half, blk, 0, cut), _lib.CopyRun(base + half + cut * blk, blk, cut, pool - cut))
+    plan = ctypes.c_void_p()
+    rc = lib.nixl_amd_copy_plan_create_indexed_runs(src, 1, flat.ctypes.data, dst, 1 if form == "strides" else 2, perm.ctypes.data, n, blk, 0,
+                                                    ctypes.byref(tuning), ctypes.byref(plan))
+    assert rc == 0, _lib.kernels_error()
+    _run_plan(torch, plan)
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+    assert np.array_equal(dev.cpu().numpy(), ko.copy_descs(host, so, do, [blk] * n))
+
+
 def test_ragged_small_descriptors_match_oracle(cuda):
     # BASELINE config 3 in miniature: sizes log-uniform in [512, 4096] rounded to 16.
     import torch
