@@ -114,6 +114,16 @@ st16_stream(void *p, const uint4 &x) {
                  : "memory");
 }
 
+// The same without the streaming hint: lines stay in the last-level cache as far as there is room.
+__device__ __forceinline__ void
+st16_through(void *p, const uint4 &x) {
+    const ep_v4u v = {x.x, x.y, x.z, x.w};
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1"
+                 :
+                 : "v"((__attribute__((address_space(1))) ep_v4u *)(reinterpret_cast<uintptr_t>(p))), "v"(v)
+                 : "memory");
+}
+
 // ---- wave-wide reductions on the DPP data path ------------------------------------------------
 
 constexpr int kEpWaveSize = 64;

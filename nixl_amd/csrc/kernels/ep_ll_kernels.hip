@@ -434,13 +434,37 @@ store_scale(void *recv_scales, const LlDims &d, bool use_ue8m0, int e, int slot,
     static_cast<uint32_t *>(recv_scales)[(static_cast<size_t>(e) * columns + (lane >> shift)) * d.N + slot] = word;
 }
 
+// Rows of up to so many bytes in all are stored without the streaming hint: they stay in the last-level cache of 256 MiB,
+// where the experts read them, and are not in the way of the next rows' stores.  With the hint and without, us, the
+// same three calls in turn (their input written just before; the cache full of another buffer's writes), means of two processes:
+//   16 x 61 x 2560, top-6, bf16, 30 MB   9.1  8.3   (9.1  8.5;   8.9  8.6)
+//   32 x 64 x 5120, top-8, fp8, 84 MB    24.2 21.8  (23.1 19.9;  24.5 21.8)
+//   32 x 128 x 2560, top-6, bf16, 126 MB 30.9 28.2  (28.2 23.4;  31.1 29.3)
+//   32 x 128 x 5120, top-8, fp8, 168 MB  46.7 40.4  (40.1 35.1;  46.9 42.1)
+//   32 x 128 x 7168, top-8, fp8, 235 MB  53.6 49.6  (46.3 45.8;  54.2 56.1)
+//   16 x 128 x 7168, top-8, bf16, 235 MB 45.5 45.0  (39.5 40.1;  45.9 47.6)
+//   32 x 128 x 7168, top-8, bf16, 470 MB 95.0 95.6  (79.0 84.0, both with ordinary loads)
+// Whole passes with combine: 73 and 68, 64 and 59, 125 and 116 (the second to fourth), 32 x 128 x 4096, top-8, fp8, 134 MB 95.6 and
+// 92.9; those of 235 MB differ by less than what they do with the place of their buffers (152 to 162).
+constexpr long long kKeptRowBytes = 176ll << 20;
+
+template<bool KEEP>
+__device__ __forceinline__ void
+store_row(void *p, const uint4 &v) {
+    if constexpr (KEEP)
+        st16_through(p, v);
+    else
+        st16_stream(p, v);
+}
+
 // grid = R*T*parts workgroups.  A lane stores 16 bytes of every row, so that the stores of a
 // wave are whole lines: a row is H/16 lanes of 16 channels as fp8 (a 128-channel scale group is
 // 8 neighbouring lanes) and H/8 lanes of 8 channels as bf16; a workgroup covers blockDim.x of
 // them (a multiple of 64).  (With 16 channels a lane for bf16 too, every store instruction left
 // half of each line to the next one: 976 tokens x 2560, top-6, took 31 us instead of 7.)
 // SCALES: the scales are written here (kIsolatedScaleWords), not by ll_scales_kernel.
-template<bool FP8, bool SCALES>
+// KEEP: rows without the streaming hint (kKeptRowBytes).
+template<bool FP8, bool SCALES, bool KEEP>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8)))
 ll_dispatch_kernel(DispatchArgs a) {
     const LlDims d = a.d;
@@ -531,7 +555,7 @@ ll_dispatch_kernel(DispatchArgs a) {
         const int row = row_of_k[k];
         if (row < 0) continue;
         if (lane == 0) a.src_info[row] = t;
-        if (active) st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
+        if (active) store_row<KEEP>(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
         if constexpr (SCALES) {
             const int e = __builtin_amdgcn_readlane(sel, k);
             if (active) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, e, row - e * d.N, lane, word);
@@ -543,7 +567,7 @@ ll_dispatch_kernel(DispatchArgs a) {
             load_row<FP8>(a.x + (static_cast<size_t>(r) * d.T + t) * d.H, at, raw0, raw1);
             for (int k = 0; k < d.K; ++k)
                 if (const int row = row_of_k[k]; row >= 0)
-                    st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * 2) + at, raw0);
+                    store_row<KEEP>(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(row) * d.H * 2) + at, raw0);
         }
     }
 }
@@ -695,7 +719,7 @@ ll_direct_kernel(DirectArgs a) {
     for (int k = 0; k < KP; ++k) {
         const int at = __builtin_amdgcn_readlane(row, k); // -1 from K on
         if (at < 0) continue;
-        st16_stream(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(at) * d.H * (FP8 ? 1 : 2)) + lane, raw0);
+        st16_through(reinterpret_cast<uint4 *>(a.recv_x + static_cast<size_t>(at) * d.H * (FP8 ? 1 : 2)) + lane, raw0); // few rows: kKeptRowBytes
         if constexpr (FP8) store_scale(a.recv_scales, d, a.use_ue8m0 != 0, want[k], at - want[k] * d.N, lane, word);
     }
 }
@@ -1355,12 +1379,18 @@ ll_dispatch_impl(const char *who, const LlDispatchCall &c) {
     a.parts = (lanes + wg - 1) / wg;
     const dim3 grid(static_cast<unsigned>(d.R) * d.T * a.parts);
     const dim3 block(wg);
-    if (scales_here)
-        hipLaunchKernelGGL((ll_dispatch_kernel<true, true>), grid, block, 0, s, a);
-    else if (c.use_fp8)
-        hipLaunchKernelGGL((ll_dispatch_kernel<true, false>), grid, block, 0, s, a);
+    const auto launch = [&]<bool KEEP>() {
+        if (scales_here)
+            hipLaunchKernelGGL((ll_dispatch_kernel<true, true, KEEP>), grid, block, 0, s, a);
+        else if (c.use_fp8)
+            hipLaunchKernelGGL((ll_dispatch_kernel<true, false, KEEP>), grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL((ll_dispatch_kernel<false, false, KEEP>), grid, block, 0, s, a);
+    };
+    if (static_cast<long long>(d.R) * d.T * d.K * d.H * (c.use_fp8 ? 1 : 2) <= kKeptRowBytes)
+        launch.template operator()<true>();
     else
-        hipLaunchKernelGGL((ll_dispatch_kernel<false, false>), grid, block, 0, s, a);
+        launch.template operator()<false>();
     HIP_TRY(hipGetLastError());
 
     if (c.use_fp8 && !scales_here) {
