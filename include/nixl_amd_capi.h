@@ -177,6 +177,13 @@ nixl_capi_status_t nixl_capi_xfer_dlist_add_descs(nixl_capi_xfer_dlist_t dlist,
                                                   const uint64_t *dev_ids,
                                                   size_t n);
 
+/* A list of n descriptors made at once from {address, length, device id} triples that lie behind one
+ * another; they are copied.  triples may be NULL if n is 0. */
+nixl_capi_status_t nixl_capi_create_xfer_dlist_of(nixl_capi_mem_type_t mem_type,
+                                                  const uint64_t *triples,
+                                                  size_t n,
+                                                  nixl_capi_xfer_dlist_t *dlist);
+
 /* Number of descriptors the backend received after index expansion and merging
  * (nixlXferTelemetry::descCount, src/api/cpp/nixl_types.h:283-287); no telemetry needed. */
 nixl_capi_status_t nixl_capi_xfer_req_desc_count(nixl_capi_xfer_req_t req, size_t *count, size_t *bytes);

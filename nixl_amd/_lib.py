@@ -243,6 +243,7 @@ _CAPI_SIGS = {
     "nixl_capi_destroy_xfer_dlist": [c_void_p],
     "nixl_capi_xfer_dlist_add_desc": [c_void_p, c_uint64, c_size_t, c_uint64],
     "nixl_capi_xfer_dlist_add_descs": [c_void_p, c_void_p, c_void_p, c_void_p, c_size_t],
+    "nixl_capi_create_xfer_dlist_of": [c_int, c_void_p, c_size_t, POINTER(c_void_p)],
     "nixl_capi_xfer_dlist_desc_count": [c_void_p, POINTER(c_size_t)],
     "nixl_capi_xfer_dlist_clear": [c_void_p],
     "nixl_capi_create_reg_dlist": [c_int, POINTER(c_void_p)],

@@ -116,16 +116,12 @@ class nixl_xfer_dlist:
         self.mem = mem
         self.triples = triples
         h = ctypes.c_void_p()
-        _check("create_xfer_dlist", self._lib.nixl_capi_create_xfer_dlist(mem, ctypes.byref(h)))
+        rows = np.ascontiguousarray(triples, dtype=np.uint64)
+        if rows.shape[1] != 3:
+            rows = np.ascontiguousarray(rows[:, :3])
+        _check("create_xfer_dlist", self._lib.nixl_capi_create_xfer_dlist_of(
+            mem, rows.__array_interface__["data"][0], rows.shape[0], ctypes.byref(h)))
         self._h = h
-        n = triples.shape[0]
-        if n:
-            addrs = np.ascontiguousarray(triples[:, 0])
-            lens = np.ascontiguousarray(triples[:, 1])
-            devs = np.ascontiguousarray(triples[:, 2])
-            _check("xfer_dlist_add_descs",
-                   self._lib.nixl_capi_xfer_dlist_add_descs(h, addrs.ctypes.data, lens.ctypes.data,
-                                                            devs.ctypes.data, n))
 
     def descCount(self):
         return int(self.triples.shape[0])

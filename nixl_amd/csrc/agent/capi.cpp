@@ -1,11 +1,15 @@
 // extern "C" façade over nixlAgent (declared in include/nixl_amd_capi.h).
 #include "nixl_amd_capi.h"
 
+#include <climits>
+#include <cstddef>
 #include <cstdlib>
 #include <cstring>
 #include <exception>
 #include <iterator>
+#include <memory>
 #include <thread>
+#include <type_traits>
 
 #include "agent_impl.h"
 
@@ -260,6 +264,22 @@ nixl_capi_xfer_dlist_add_descs(nixl_capi_xfer_dlist_t dlist,
         dlist->dlist->emplace(static_cast<uintptr_t>(addrs[i]), static_cast<size_t>(lens[i]),
                               dev_ids ? dev_ids[i] : uint64_t{0});
     return NIXL_CAPI_SUCCESS;
+}
+
+nixl_capi_status_t
+nixl_capi_create_xfer_dlist_of(nixl_capi_mem_type_t mem_type, const uint64_t *triples, size_t n, nixl_capi_xfer_dlist_t *dlist) {
+    static_assert(sizeof(nixlBasicDesc) == 3 * sizeof(uint64_t) && offsetof(nixlBasicDesc, addr) == 0 &&
+                  offsetof(nixlBasicDesc, len) == 8 && offsetof(nixlBasicDesc, devId) == 16 &&
+                  std::is_trivially_copyable_v<nixlBasicDesc>);
+    if (!dlist || mem_type >= NIXL_CAPI_MEM_UNKNOWN || (n && !triples) || n > static_cast<size_t>(INT_MAX))
+        return NIXL_CAPI_ERROR_INVALID_PARAM;
+    return guarded([&] {
+        auto list = std::make_unique<nixl_xfer_dlist_t>(memOf(mem_type), static_cast<int>(n));
+        if (n) std::memcpy(static_cast<void *>(&(*list)[0]), triples, n * sizeof(nixlBasicDesc));
+        *dlist = new nixl_capi_xfer_dlist_s{list.get()};
+        list.release();
+        return NIXL_CAPI_SUCCESS;
+    });
 }
 
 nixl_capi_status_t

@@ -1761,27 +1761,57 @@ generic_item(uint64_t src, uint64_t dst, uint64_t len) {
 // them is written, without a check for each and without touching memory that is not needed.
 template<typename Rec>
 struct Records {
-    std::unique_ptr<Rec[]> at;
+    Rec *at = nullptr;
     size_t n = 0, cap = 0;
 
     Rec *
     room(size_t more, size_t expected) {
         if (cap - n < more) grow(more + expected);
-        return at.get() + n;
+        return at + n;
     }
 
     void
     end_at(const Rec *end) {
-        n = static_cast<size_t>(end - at.get());
+        n = static_cast<size_t>(end - at);
+    }
+
+    // Memory of somebody else's for the first records, left again when they are more.
+    void
+    lend(void *memory, size_t bytes) {
+        at = static_cast<Rec *>(memory);
+        cap = bytes / sizeof(Rec);
     }
 
 private:
+    std::unique_ptr<Rec[]> own_;
+
     __attribute__((noinline)) void
     grow(size_t more) {
         cap = std::max(2 * cap, n + more);
         std::unique_ptr<Rec[]> grown(new Rec[cap]);
-        if (n) std::memcpy(grown.get(), at.get(), n * sizeof(Rec));
-        at = std::move(grown);
+        if (n) std::memcpy(grown.get(), at, n * sizeof(Rec));
+        own_ = std::move(grown);
+        at = own_.get();
+    }
+};
+
+// A pinned upload buffer that goes back to its cache if nothing takes it over.
+struct Staging {
+    const int device;
+    void *at = nullptr;
+    size_t cap = 0;
+
+    explicit Staging(int d) : device(d) {}
+    ~Staging() {
+        if (at) upload_cache().put(device, at, cap);
+    }
+    Staging(const Staging &) = delete;
+    Staging &
+    operator=(const Staging &) = delete;
+
+    hipError_t
+    get(size_t bytes) {
+        return upload_cache().get(device, bytes, &at, &cap);
     }
 };
 
@@ -1818,6 +1848,8 @@ struct LongDescs {
 // the others: in one loop, with items appended one by one to a vector, making a plan took 106 us for
 // 14 394 descriptors of up to 16 KiB and 24 for 3000 of up to 64 KiB (54 and 18 so), and code
 // for items inlined there cost aligned descriptors 0.6 ns each (50 000 of 512 B: 203 us, 166 so).
+// Items are written to the buffer that is uploaded, in front of everything else in it (a request of 2000 descriptors of
+// 32 to 64 KiB made in 35 us with a copy of them, 27.8 so; of 3000 of up to 64 KiB 28.1 and 26.7).
 struct ByteDescs {
     Records<GenericItem> items;
     std::vector<uint32_t> longs;
@@ -1849,11 +1881,21 @@ struct ByteDescs {
         items.end_at(cut(items.room(len / reach + 2, longs.size()), src, dst, len, reach));
     }
 
+    // Items of one short descriptor at most, and of short ones among descs[i .. end) together.
+    static constexpr size_t kMost = kSplitFromBytes / kGenericRound + 2;
+
+    static size_t
+    most(const nixl_amd_copy_desc_t *descs, size_t i, size_t end) {
+        size_t rounds = 0;
+        for (size_t j = i; j < end; ++j)
+            rounds += descs[j].len < kSplitFromBytes ? descs[j].len / kGenericRound : 0;
+        return rounds + 2 * (end - i);
+    }
+
     // Takes descriptors from `i` on until one that is aligned or that plan_create refuses; returns
     // where it stopped.
     __attribute__((noinline)) size_t
     take(const nixl_amd_copy_desc_t *descs, size_t i, size_t end) {
-        constexpr size_t kMost = kSplitFromBytes / kGenericRound + 2; // items of one descriptor
         GenericItem *at = nullptr, *limit = nullptr;
         uint64_t taken = 0, bytes = 0;
         for (; i < end; ++i) {
@@ -1874,7 +1916,7 @@ struct ByteDescs {
             if (static_cast<size_t>(limit - at) < kMost) {
                 if (at) items.end_at(at);
                 at = items.room(kMost, 2 * (end - i));
-                limit = items.at.get() + items.cap;
+                limit = items.at + items.cap;
             }
             at = cut(at, d.src, d.dst, d.len, kGenericRound);
         }
@@ -2069,6 +2111,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     uint64_t units = 0, payload = 0, n_piece_descs = 0;
     LongDescs chunks(chunk_bytes);
     ByteDescs bytes;
+    Staging buffer(device); // what is uploaded; items are written there at once
     bool whole_chunks = false; // there are chunks of some aligned descriptor whatever becomes of those
     for (size_t i = 0; i < n; ++i) {
         const nixl_amd_copy_desc_t &d = descs[i];
@@ -2080,6 +2123,15 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         if (((d.src | d.dst | d.len) & 15u) != 0) {
             if (((d.src + d.len) | (d.dst + d.len)) >> kPieceUnitsShift)
                 return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create: address beyond 2^56");
+            if (!bytes.items.at) {
+                constexpr size_t kMostAhead = 64u << 20;
+                const size_t ahead = (ByteDescs::most(descs, i, n) + ByteDescs::kMost) * sizeof(GenericItem);
+                reap_uploads(device);
+                if (ahead <= kMostAhead && buffer.get(ahead) == hipSuccess)
+                    bytes.items.lend(buffer.at, buffer.cap);
+                else
+                    (void)hipGetLastError();
+            }
             i = bytes.take(descs, i, n) - 1; // this one, and the ones behind it as far as they are like it
             continue;
         }
@@ -2163,19 +2215,17 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     // ---- one device arena for all plan arrays --------------------------------------
     auto align256 = [](size_t x) { return (x + 255) & ~size_t(255); };
     const bool need_desc_arrays = n_stream != 0;
-    // The arena starts with the records the copy kernel reads.  When they are expanded on the
-    // device, that stretch is not uploaded: the upload starts behind it, and the runs
-    // travel at the arena's end.
-    const size_t off_uni = 0;
-    const size_t off_src = off_uni + align256(n_uniform_recs * sizeof(UniformRec));
+    // The arena ends with the records of chunks.  When they are expanded on the device, that stretch is not uploaded.
+    const size_t off_items = 0;
+    const size_t off_src = off_items + align256(bytes.items.n * sizeof(GenericItem));
     const size_t off_dst = off_src + (need_desc_arrays ? align256(nv * 8) : 0);
     const size_t off_prefix = off_dst + (need_desc_arrays ? align256(nv * 8) : 0);
     const size_t off_span = off_prefix + (need_desc_arrays ? align256((nv + 1) * 8) : 0);
     const size_t off_pieces = off_span + (need_desc_arrays ? align256(span.size() * sizeof(uint2)) : 0);
-    const size_t off_items = off_pieces + align256(pieces.n * sizeof(PieceRec));
-    const size_t off_runs = off_items + align256(bytes.items.n * sizeof(GenericItem));
-    const size_t total = off_runs + (expand ? align256(chunks.runs.size() * sizeof(ChunkRun)) : 0);
-    const size_t upload_from = expand ? off_src : 0;
+    const size_t off_runs = off_pieces + align256(pieces.n * sizeof(PieceRec));
+    const size_t off_uni = off_runs + (expand ? align256(chunks.runs.size() * sizeof(ChunkRun)) : 0);
+    const size_t total = off_uni + align256(n_uniform_recs * sizeof(UniformRec));
+    const size_t uploaded = expand ? off_uni : total;
 
     auto *plan = new nixl_amd_copy_plan();
     plan->device = device;
@@ -2185,7 +2235,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         // constant step (the same block of every layer of a pool) take non-temporal loads where they
         // are long; destinations without such a pattern (a scatter over a pool) take plain loads.
         uint64_t pairs = 0, regular = 0, prev_dst = 0, prev_end = 0, prev_step = 0;
-        for (size_t i = 0; i < n; ++i) {
+        const bool matters = copy_policy(payload, true) != copy_policy(payload, false);
+        for (size_t i = 0; matters && i < n; ++i) {
             if (descs[i].len == 0) continue;
             if (prev_end) {
                 const uint64_t step = descs[i].dst - prev_dst;
@@ -2205,16 +2256,21 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     plan->max_wgs = max_wgs;
 
     if (total > 0) {
-        void *staging = nullptr;
-        size_t staging_cap = 0;
-        reap_uploads(device);
-        hipError_t e = upload_cache().get(device, std::max<size_t>(total - upload_from, 256), &staging, &staging_cap);
-        if (e != hipSuccess) {
-            delete plan;
-            return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
+        Staging larger(device);
+        hipError_t e = hipSuccess;
+        if (buffer.cap < std::max<size_t>(uploaded, 256)) {
+            reap_uploads(device);
+            e = larger.get(std::max<size_t>(uploaded, 256));
+            if (e != hipSuccess) {
+                delete plan;
+                return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
+            }
         }
-        // the pinned buffer mirrors the arena from upload_from on
-        const auto host = [&](size_t arena_offset) { return static_cast<uint8_t *>(staging) + (arena_offset - upload_from); };
+        // the pinned buffer mirrors the arena; this function or the plan gives it back from here on
+        Staging &from = larger.at ? larger : buffer;
+        void *const staging = from.at;
+        const size_t staging_cap = from.cap;
+        const auto host = [&](size_t arena_offset) { return static_cast<uint8_t *>(staging) + arena_offset; };
         if (expand) {
             std::memcpy(host(off_runs), chunks.runs.data(), chunks.runs.size() * sizeof(ChunkRun));
         } else {
@@ -2228,8 +2284,9 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
             std::memcpy(host(off_prefix), vprefix.data(), (nv + 1) * 8);
             std::memcpy(host(off_span), span.data(), span.size() * sizeof(uint2));
         }
-        if (pieces.n) std::memcpy(host(off_pieces), pieces.at.get(), pieces.n * sizeof(PieceRec));
-        if (bytes.items.n) std::memcpy(host(off_items), bytes.items.at.get(), bytes.items.n * sizeof(GenericItem));
+        if (pieces.n) std::memcpy(host(off_pieces), pieces.at, pieces.n * sizeof(PieceRec));
+        if (bytes.items.n && bytes.items.at != staging) std::memcpy(host(off_items), bytes.items.at, bytes.items.n * sizeof(GenericItem));
+        from.at = nullptr;
         e = arena_cache().get(device, total, &plan->arena, &plan->arena_cap);
         if (e != hipSuccess) {
             upload_cache().put(device, staging, staging_cap);
@@ -2239,8 +2296,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         hipStream_t up = nullptr;
         e = build_stream(plan, t, &up);
         auto *arena = static_cast<uint8_t *>(plan->arena);
-        if (e == hipSuccess && total > upload_from)
-            e = upload(up, arena + upload_from, staging, total - upload_from);
+        if (e == hipSuccess) e = upload(up, arena, staging, uploaded);
         if (e == hipSuccess && expand) {
             const uint32_t wgs = static_cast<uint32_t>(std::min<uint64_t>((static_cast<uint64_t>(n_uniform_chunks) + 255) / 256, 1u << 20));
             hipLaunchKernelGGL(expand_runs_kernel, dim3(wgs), dim3(256), 0, up, reinterpret_cast<UniformRec *>(arena + off_uni),

@@ -397,9 +397,10 @@ nixlHipEngine::lowerGeneral(bool write,
                             size_t &bytes) const {
     const int n = local.descCount();
     const nixlHipMD *prev_lmd = nullptr, *prev_rmd = nullptr;
-    for (int i = 0; i < n; ++i) {
-        const nixlMetaDesc &l = local[i];
-        const nixlMetaDesc &r = remote[i];
+    const nixlMetaDesc *const L = &local[0], *const R = &remote[0];
+    for (int i = 0; i < n;) {
+        const nixlMetaDesc &l = L[i];
+        const nixlMetaDesc &r = R[i];
         if (l.len != r.len) {
             NIXL_ERROR << "HIP backend: length mismatch at descriptor " << i;
             return NIXL_ERR_INVALID_PARAM;
@@ -424,11 +425,24 @@ nixlHipEngine::lowerGeneral(bool write,
                 return NIXL_ERR_NOT_SUPPORTED;
             }
         }
-        const uintptr_t la = lmd->here(l.addr), ra = rmd->here(r.addr); // a peer's region may be mapped elsewhere here
-        lowered[i].src = write ? la : ra;
-        lowered[i].dst = write ? ra : la;
-        lowered[i].len = l.len;
-        bytes += l.len;
+        // The pairs of the same two regions behind this one (this one again first): their bounds stay in registers and
+        // their checks are looked at once.  A pair that fails one ends the stretch and is found again above.
+        const nixlBackendMD *const lkey = l.metadataP, *const rkey = r.metadataP;
+        const uintptr_t lbase = lmd->addr, rbase = rmd->addr;
+        const size_t lspan = lmd->len, rspan = rmd->len;
+        // a peer's region may be mapped elsewhere here; the direction decides which side is read
+        const uintptr_t to_src = static_cast<uintptr_t>(write ? lmd->delta : rmd->delta);
+        const uintptr_t to_dst = static_cast<uintptr_t>(write ? rmd->delta : lmd->delta);
+        for (; i < n; ++i) {
+            const nixlMetaDesc &lj = L[i], &rj = R[i];
+            const size_t len = lj.len;
+            const size_t bad = static_cast<size_t>(lj.metadataP != lkey) | static_cast<size_t>(rj.metadataP != rkey) |
+                static_cast<size_t>(len != rj.len) | static_cast<size_t>(len > lspan) | static_cast<size_t>(len > rspan) |
+                static_cast<size_t>(lj.addr - lbase > lspan - len) | static_cast<size_t>(rj.addr - rbase > rspan - len);
+            if (bad) break;
+            lowered[i] = nixl_amd_copy_desc_t{(write ? lj.addr : rj.addr) + to_src, (write ? rj.addr : lj.addr) + to_dst, len};
+            bytes += len;
+        }
     }
     if (device < 0) device = static_cast<const nixlHipMD *>(local[0].metadataP)->device;
     return NIXL_SUCCESS;

@@ -146,6 +146,32 @@ def test_scatter_sorted_because_the_caller_says_so(cuda, form, n):
     assert np.array_equal(dev.cpu().numpy(), ko.copy_descs(host, so, do, [blk] * n))
 
 
+@pytest.mark.parametrize("op", ["WRITE", "READ"])
+@pytest.mark.parametrize("stretch", [1, 2, 63, 400])
+def test_explicit_lists_over_changing_regions(hip_agent, cuda, op, stretch):
+    """Byte descriptors whose regions change after every `stretch` of them, on one side or the other."""
+    import torch
+    rng = np.random.default_rng(stretch)
+    n = 400
+    bufs = [torch.from_numpy(rng.integers(0, 256, 1 << 19, dtype=np.uint8)).to(cuda) for _ in range(4)]
+    hip_agent.register_memory(bufs)
+    lens = rng.integers(1, 600, n)
+    offs = np.arange(n) * 1200 + rng.integers(0, 600, n)
+    of_src, of_dst = (np.arange(n) // stretch) % 2, 2 + (np.arange(n) // (2 * stretch)) % 2
+    src = np.array([bufs[b].data_ptr() + o for b, o in zip(of_src, offs)], np.uint64)
+    dst = np.array([bufs[b].data_ptr() + o + 3 for b, o in zip(of_dst, offs)], np.uint64)
+    want = [b.cpu().numpy().copy() for b in bufs]
+    for s, d, o, l in zip(of_src, of_dst, offs, lens):
+        want[d][o + 3:o + 3 + l] = want[s][o:o + l]
+    local, remote = (src, dst) if op == "WRITE" else (dst, src)
+    lists = [hip_agent.get_xfer_descs(np.stack([a, lens.astype(np.uint64), np.zeros(n, np.uint64)], 1), "VRAM") for a in (local, remote)]
+    req = hip_agent.initialize_xfer(op, *lists, "agent")
+    _wait(hip_agent, req)
+    for b, w in zip(bufs, want):
+        assert np.array_equal(b.cpu().numpy(), w)
+    req.release()
+
+
 def test_ragged_small_descriptors_match_oracle(cuda):
     # BASELINE config 3 in miniature: sizes log-uniform in [512, 4096] rounded to 16.
     import torch

@@ -314,6 +314,56 @@ def test_sorted_region_list_matches_reference_expectations():
     assert proc.returncode == 0 and proc.stdout.strip() == "OK", proc.stdout + proc.stderr
 
 
+def test_regions_that_cover_the_descriptors_of_a_list():
+    """tests/cpp/covering_regions_check.cpp: the region every descriptor is resolved to, whatever the order of
+    the list and however regions overlap, against the two searches written out."""
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    exe = os.path.join(root, "tests", "cpp", "_build", "covering_regions_check")
+    if not os.path.exists(exe):
+        pytest.fail(f"{exe} missing: run __graft_entry__.build() first")
+    proc = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert proc.returncode == 0 and proc.stdout.strip().endswith("OK"), proc.stdout + proc.stderr
+
+
+@pytest.mark.parametrize("n", [1, 2, 700])
+@pytest.mark.parametrize("form", ["rows", "columns", "strided", "int64", "list", "four columns"])
+def test_lists_from_any_layout_of_triples(cpu_agent, form, n):
+    """Explicit lists from arrays of any order, stride and integer type move the bytes that they name."""
+    rng = np.random.default_rng(n)
+    src, dst = rng.integers(0, 256, 64 * n, dtype=np.uint8), np.zeros(64 * n, dtype=np.uint8)
+    cpu_agent.register_memory(np.array([[b.ctypes.data, b.nbytes, 0] for b in (src, dst)], dtype=np.uint64), "DRAM")
+    offs, lens = 64 * rng.permutation(n) + rng.integers(0, 32, n), rng.integers(1, 32, n)
+
+    def rows(buf):
+        t = np.stack([buf.ctypes.data + offs, lens, np.zeros_like(lens)], 1).astype(np.uint64)
+        if form == "columns":
+            return np.asfortranarray(t)
+        if form == "strided":
+            return np.repeat(t, 2, 0)[::2]
+        if form == "int64":
+            return t.astype(np.int64)
+        return [tuple(int(v) for v in r) for r in t] if form == "list" else t
+
+    if form == "four columns":
+        wide = [np.concatenate([rows(b), np.ones((n, 1), np.uint64)], 1) for b in (src, dst)]
+        local, remote = (ag.nixl_xfer_dlist(w, 0) for w in wide)
+    else:
+        local, remote = (cpu_agent.get_xfer_descs(rows(b), "DRAM") for b in (src, dst))
+    assert local.descCount() == n
+    req = cpu_agent.initialize_xfer("WRITE", local, remote, cpu_agent.name)
+    state = cpu_agent.transfer(req)
+    while state == "PROC":
+        state = cpu_agent.check_xfer_state(req)
+    assert state == "DONE"
+    want = np.zeros_like(dst)
+    for o, l in zip(offs, lens):
+        want[o:o + l] = src[o:o + l]
+    assert np.array_equal(dst, want)
+    req.release()
+
+
 def test_api_behaviour_of_the_reference_python_tests(cpu_agent, oracle_plugin_dir):
     """Cases of the reference's test/python/test_nixl_api.py that concern one agent:
     empty name (:90-93), unknown operation (:135-142), unknown plugin name gives empty
