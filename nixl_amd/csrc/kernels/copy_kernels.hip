@@ -667,10 +667,11 @@ index_records_runs_kernel(UniformRec *recs, IndexVector src_index, IndexVector d
 //
 // The verdict reaches the host through pinned memory, written by the workgroup that finishes last;
 // the host waits for it, because a bad pair must fail the request.  A workgroup adds to the totals
-// with two atomics (all dies add to one line), and nothing in front of the verdict writes a cache back: a
+// with two atomics, on two lines (an addition to a line takes 11 ns behind another one, and there are 256 workgroups in
+// 262 144 pairs: 13.8 us with one line, 11.2 with two), and nothing in front of the verdict writes a cache back: a
 // device-scope fence around the additions did, for records that only the next kernel reads.  Kernel time, with such
-// fences and sums over a wave through LDS, and without: runs of 64 pairs, 1024 pairs 8.0 and 6.4 us, 16 384 9.9 and
-// 8.1, 65 536 10.9 and 8.7, 262 144 15.5 and 13.8; vectors, 1024 pairs 6.8 and 5.3, 65 536 19.2 and 18.1.
+// fences, sums over a wave through LDS and one line, and now: runs of 64 pairs, 1024 pairs 8.0 and 6.4 us, 16 384 9.9 and
+// 8.1, 65 536 10.9 and 8.7, 262 144 15.5 and 11.2; vectors, 1024 pairs 6.8 and 5.3, 65 536 19.2 and 18.1.
 struct IndexRun {
     uint32_t first; // pair the run starts with; it ends where the next one starts
     uint32_t src, dst; // indices of that pair
@@ -685,7 +686,7 @@ struct ListTotals {
     unsigned long long bytes_arrived; // bytes of the good pairs | workgroups that have added theirs << kListBytesBits
     // records beyond the first of their pair | pairs that continue the pair before them inside one
     // dense run on both sides << 32
-    unsigned long long extra_continued;
+    alignas(128) unsigned long long extra_continued; // on a line of its own: additions to one line wait for each other
     uint32_t bad; // pairs that name no entry or join entries of different lengths
 };
 
@@ -2727,6 +2728,7 @@ create_listed(const nixl_amd_copy_list_t *src,
     plan->policy = t.nt ? t.nt : kPolNtSc1Nt;
     // one arena: the totals, then the records
     constexpr size_t kRecsAt = 256;
+    static_assert(sizeof(ListTotals) <= kRecsAt);
     hipStream_t up = nullptr;
     e = arena_cache().get(device, kRecsAt + n * per_desc * sizeof(PieceRec), &plan->arena, &plan->arena_cap);
     if (e == hipSuccess) e = build_stream(plan, t, &up);
