@@ -38,6 +38,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #if defined(__x86_64__)
@@ -233,15 +234,50 @@ constexpr uint32_t kInlineRecs = 128;
 
 struct InlineRecs {
     UniformRec rec[kInlineRecs];
+
+    __device__ __forceinline__ UniformRec
+    at(uint32_t r) const {
+        return rec[r];
+    }
 };
 
-template<int POL>
+// A request of some more, by index into two lists of one stride each: what travels is the indices, and every wave
+// makes its record of them.  A vector that is consecutive is its first index.  Requests made, moved and waited for, us, with
+// records that a kernel makes in front of the copy and so, blocks of 8 KiB gathered: 192 17.4 and 14.8, 512 17.6 and 14.9, 896
+// 18.8 and 15.5; scattered 896 17.9 and 15.5.  896 words are 3.5 of the 4 KiB that a launch can carry; 16-bit indices
+// would make twice as many blocks fit, of pools with few entries.
+constexpr uint32_t kInlineIndices = 896;
+
+struct InlineIndices {
+    struct Side {
+        uint64_t base, stride;
+        uint32_t first; // index, of a consecutive vector
+        uint32_t listed; // ~0 where the vector is in `index`, from `place` on, 0 where it is consecutive (and `place` 0)
+        uint32_t place;
+    };
+
+    Side src, dst;
+    int32_t index[kInlineIndices];
+
+    __device__ __forceinline__ UniformRec
+    at(uint32_t r) const { // r < n <= kInlineIndices
+        const auto address = [&](const Side &s) {
+            // no branch, so that the words of both sides are loaded together and behind nothing but the sides
+            const uint32_t word = static_cast<uint32_t>(index[s.place + r]);
+            return s.base + ((word & s.listed) | ((s.first + r) & ~s.listed)) * s.stride;
+        };
+        return UniformRec{address(src), address(dst)};
+    }
+};
+
+template<int POL, typename Recs>
 __global__ void __launch_bounds__(kWaveSize)
-copy_inline_kernel(InlineRecs recs, FastDiv chunks_per_rec) {
+copy_inline_kernel(Recs recs, FastDiv chunks_per_rec) {
     uint32_t chunk;
     const uint32_t r = chunks_per_rec.quotient(blockIdx.x, chunk);
     const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * 16u) + threadIdx.x * 16u;
-    store16<POL>(recs.rec[r].dst + off, load16<POL>(recs.rec[r].src + off));
+    const UniformRec rec = recs.at(r);
+    store16<POL>(rec.dst + off, load16<POL>(rec.src + off));
 }
 
 // ---- the end of a launch as a word in host memory ----------------------------------------------
@@ -295,9 +331,9 @@ done_kernel(uint32_t *word, uint32_t value) {
 // (device scope): their completion is what s_waitcnt waits for, no cache has to be written back.
 constexpr int kDoneWaves = 8, kDoneChunks = 2; // chunks a wave
 
-template<int POL>
+template<int POL, typename Recs>
 __global__ void __launch_bounds__(kWaveSize *kDoneWaves)
-copy_inline_done_kernel(InlineRecs recs, FastDiv chunks_per_rec, uint32_t n_chunks, Done done) {
+copy_inline_done_kernel(Recs recs, FastDiv chunks_per_rec, uint32_t n_chunks, Done done) {
     static_assert(POL == kPolPlainSc1Nt || POL == kPolNtSc1Nt);
     const uint32_t lane = threadIdx.x & (kWaveSize - 1);
     const uint32_t first = uniform(blockIdx.x * (kDoneWaves * kDoneChunks) + threadIdx.x / kWaveSize);
@@ -310,8 +346,9 @@ copy_inline_done_kernel(InlineRecs recs, FastDiv chunks_per_rec, uint32_t n_chun
         uint32_t chunk;
         const uint32_t r = chunks_per_rec.quotient(c, chunk);
         const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * 16u) + lane * 16u;
-        to[j] = recs.rec[r].dst + off;
-        v[j] = load16<POL>(recs.rec[r].src + off);
+        const UniformRec rec = recs.at(r);
+        to[j] = rec.dst + off;
+        v[j] = load16<POL>(rec.src + off);
     }
 #pragma unroll
     for (int j = 0; j < kDoneChunks; ++j)
@@ -1274,6 +1311,7 @@ struct nixl_amd_copy_plan {
     uint32_t chunks_per_rec = 1;
     uint32_t uniform_wgs = 0;
     std::unique_ptr<InlineRecs> inline_recs; // instead of uniform_recs: a plan of a few blocks, nothing on the device
+    std::unique_ptr<InlineIndices> inline_indices; // or of some more
     MixedArgs mixed_args{};
     uint32_t mixed_wgs = 0;
     const PieceRec *piece_recs = nullptr;
@@ -1681,8 +1719,8 @@ sort_pays(int sort_scatter, size_t n, uint64_t len) {
 // Whether a plan of `n` equal blocks can carry its records as kernel arguments: few enough, and
 // the launch shape the inline kernel has.
 static bool
-fits_inline(size_t n, uint64_t len, const Tuning &t) {
-    return n <= kInlineRecs && t.upl == 1 && t.waves == 1 && !t.swizzle && n * (len / (kWaveSize * 16u)) <= kMaxGrid;
+fits_inline(size_t n, uint64_t len, const Tuning &t, size_t most = kInlineRecs) {
+    return n <= most && t.upl == 1 && t.waves == 1 && !t.swizzle && n * (len / (kWaveSize * 16u)) <= kMaxGrid;
 }
 
 // The members a plan of `n_recs` equal blocks has wherever its records are.
@@ -2483,24 +2521,28 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
     // The records of a few blocks are made right here instead.
     const size_t index_bytes = n * sizeof(int32_t);
     const bool inlined = fits_inline(n, len, t);
-    int32_t few[2 * kInlineRecs];
+    const bool tables = n_src_runs > 1 || n_dst_runs > 1;
+    const bool some = !inlined && !tables && fits_inline(n, len, t, kInlineIndices); // their indices may travel as arguments
+    int32_t few[2 * kInlineIndices];
     void *staging = nullptr;
     size_t staging_cap = 0;
-    const bool tables = n_src_runs > 1 || n_dst_runs > 1;
     const size_t table_at = (2 * index_bytes + 15) & ~size_t(15); // the run tables follow the index vectors
     const size_t table_bytes = tables ? (n_src_runs + n_dst_runs) * sizeof(nixl_amd_copy_run_t) : 0;
     hipError_t e = hipSuccess;
-    if (!inlined) {
+    const auto take_staging = [&] {
         reap_uploads(device);
         e = upload_cache().get(device, table_at + table_bytes, &staging, &staging_cap);
-        if (e != hipSuccess)
-            return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
-    }
+        return e == hipSuccess ?
+            NIXL_AMD_OK :
+            nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("hipHostMalloc(plan upload buffer): ") + hipGetErrorString(e));
+    };
+    if (!inlined && !some)
+        if (const int rc = take_staging()) return rc;
     // One pass over each vector on its way there: bounds, and the patterns that decide cache policy and
     // record order.  A request of 65 536 blocks made, one of whose vectors is consecutive: 51 us with a
     // pass each for a copy, bounds, the pinned copy and the pattern, 23 in one, 16 with the consecutive
     // one left where it is.
-    int32_t *const si = inlined ? few : static_cast<int32_t *>(staging), *const di = si + n;
+    int32_t *si = staging ? static_cast<int32_t *>(staging) : few, *di = si + n;
     const IndexFacts src_facts = take_indices(src_index, n, si, src_all_dense, inlined),
                      dst_facts = take_indices(dst_index, n, di, dst_all_dense, inlined);
     if (src_facts.highest >= src_entries || dst_facts.highest >= dst_entries) {
@@ -2533,13 +2575,42 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         *out = plan;
         return NIXL_AMD_OK;
     }
+    const bool src_follows = src_facts.ones == n - 1, dst_follows = dst_facts.ones == n - 1;
+    if (some) {
+        const size_t words = (src_follows ? 0 : n) + (dst_follows ? 0 : n);
+        if (words <= kInlineIndices) {
+            std::unique_ptr<InlineIndices> in(new InlineIndices); // not cleared
+            uint32_t place = 0;
+            const auto side = [&](const nixl_amd_copy_run_t &run, const int32_t *index, bool follows) {
+                InlineIndices::Side s{run.base, run.stride, static_cast<uint32_t>(index[0]), follows ? 0 : ~0u, follows ? 0 : place};
+                if (!follows) {
+                    std::memcpy(in->index + place, index, index_bytes);
+                    place += static_cast<uint32_t>(n);
+                }
+                return s;
+            };
+            in->src = side(src_runs[0], si, src_follows);
+            in->dst = side(dst_runs[0], di, dst_follows);
+            plan->inline_indices = std::move(in);
+            describe_blocks(*plan, t, n, len, n);
+            *out = plan;
+            return NIXL_AMD_OK;
+        }
+        if (const int rc = take_staging()) {
+            delete plan;
+            return rc;
+        }
+        std::memcpy(staging, few, 2 * index_bytes);
+        si = static_cast<int32_t *>(staging);
+        di = si + n;
+    }
     const size_t rec_bytes = n * sizeof(UniformRec);
     hipStream_t up = nullptr;
     e = arena_cache().get(device, rec_bytes, &plan->arena, &plan->arena_cap);
     if (e == hipSuccess) e = build_stream(plan, t, &up);
     auto *recs = static_cast<UniformRec *>(plan->arena);
     if (e == hipSuccess) {
-        const IndexVector src_at{src_facts.ones == n - 1 ? nullptr : si, si[0]}, dst_at{dst_facts.ones == n - 1 ? nullptr : di, di[0]};
+        const IndexVector src_at{src_follows ? nullptr : si, si[0]}, dst_at{dst_follows ? nullptr : di, di[0]};
         const auto launch = [&]<bool SORTED>() {
             const dim3 block(kIndexThreads<SORTED>), grid(static_cast<uint32_t>((n + block.x - 1) / block.x));
             if (tables) {
@@ -2917,7 +2988,8 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
         if (slot >= 0) slots->put(slot); // nothing that would write its word is queued
         return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("plan_launch: ") + hipGetErrorString(e));
     };
-    if (plan->inline_recs) {
+    const auto launch_inline = [&](const auto &recs) {
+        using Recs = std::decay_t<decltype(recs)>;
         // The line between the two forms (above): at 4 MiB, 256 workgroups to be counted, 11.0 us and 11.3
         // with a kernel behind, the median of both 10.5; at 8 MiB 11.8 both, the median 11.5 and 10.8.
         constexpr uint32_t kToldChunks = 4096;
@@ -2925,21 +2997,26 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
         if (slot >= 0 && through && plan->n_uniform <= kToldChunks) {
             const dim3 grid((plan->n_uniform + kDoneWaves * kDoneChunks - 1) / (kDoneWaves * kDoneChunks));
             const auto launch = [&](auto kernel) {
-                hipLaunchKernelGGL(kernel, grid, dim3(kWaveSize * kDoneWaves), 0, s, *plan->inline_recs, FastDiv(plan->chunks_per_rec),
+                hipLaunchKernelGGL(kernel, grid, dim3(kWaveSize * kDoneWaves), 0, s, recs, FastDiv(plan->chunks_per_rec),
                                    plan->n_uniform, done);
             };
             if (plan->policy == kPolPlainSc1Nt)
-                launch(copy_inline_done_kernel<kPolPlainSc1Nt>);
+                launch(copy_inline_done_kernel<kPolPlainSc1Nt, Recs>);
             else
-                launch(copy_inline_done_kernel<kPolNtSc1Nt>);
+                launch(copy_inline_done_kernel<kPolNtSc1Nt, Recs>);
             told = true;
         } else {
             with_policy(plan->policy, [&]<int POL>() {
-                hipLaunchKernelGGL(copy_inline_kernel<POL>, dim3(plan->n_uniform), dim3(kWaveSize), 0, s, *plan->inline_recs,
+                hipLaunchKernelGGL((copy_inline_kernel<POL, Recs>), dim3(plan->n_uniform), dim3(kWaveSize), 0, s, recs,
                                    FastDiv(plan->chunks_per_rec));
             });
         }
-        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return give_up(e);
+        return hipGetLastError();
+    };
+    if (plan->inline_recs) {
+        if (const hipError_t e = launch_inline(*plan->inline_recs); e != hipSuccess) return give_up(e);
+    } else if (plan->inline_indices) {
+        if (const hipError_t e = launch_inline(*plan->inline_indices); e != hipSuccess) return give_up(e);
     } else if (plan->uniform_wgs) {
         // One launch per kMaxGrid workgroups.  With the die swizzle each launch's grid is
         // rounded up to a multiple of 8 so that every die owns an equally long slice; surplus

@@ -537,6 +537,66 @@ def test_index_vectors_into_lists_of_several_runs(hip_agent, cuda):
         h.release()
 
 
+@pytest.mark.parametrize("n", [128, 129, 448, 449, 896, 897])
+@pytest.mark.parametrize("listed", ["source", "destination", "both", "neither"])
+@pytest.mark.parametrize("chunks, policy", [(1, 0), (3, 2), (9, 0)])
+def test_requests_whose_indices_travel_as_arguments(cuda, n, listed, chunks, policy):
+    """Requests by index into two strided lists, around the numbers of blocks and of index words that a launch carries:
+    vectors that are consecutive from somewhere in their list and vectors in any order, strides longer than
+    a block, copies that count their own workgroups and longer ones; watched, launched again on new bytes, and
+    replayed from a graph."""
+    import torch
+    lib = _lib.kernels()
+    assert lib.nixl_amd_copy_watch_prepare() == 0
+    rng = np.random.default_rng(n)
+    blk, entries, first = 1024 * chunks, n + 61, 17
+    s_stride, d_stride = blk, blk + 384
+    src = torch.from_numpy(rng.integers(0, 256, entries * s_stride, dtype=np.uint8)).to(cuda)
+    dst = torch.zeros(entries * d_stride, dtype=torch.uint8, device=cuda)
+    assert src.data_ptr() % 128 == 0 and dst.data_ptr() % 128 == 0
+
+    def vector(in_order):
+        return np.arange(first, first + n, dtype=np.int32) if in_order else rng.permutation(entries)[:n].astype(np.int32)
+
+    si, di = vector(listed not in ("source", "both")), vector(listed not in ("destination", "both"))
+    run = lambda t, stride: (_lib.CopyRun * 1)(_lib.CopyRun(t.data_ptr(), stride, 0, entries))  # noqa: E731
+    tuning, plan = _lib.CopyTuning(0, policy), ctypes.c_void_p()
+    given = si.copy(), di.copy()
+    assert lib.nixl_amd_copy_plan_create_indexed_runs(run(src, s_stride), 1, given[0].ctypes.data, run(dst, d_stride), 1, given[1].ctypes.data,
+                                                      n, blk, 0, ctypes.byref(tuning), ctypes.byref(plan)) == 0, _lib.kernels_error()
+    for g in given:
+        g.fill(0)  # the plan keeps nothing of the caller's vectors
+    info = _lib.CopyPlanInfo()
+    assert lib.nixl_amd_copy_plan_query(plan, ctypes.byref(info)) == 0
+    assert info.payload_bytes == n * blk and info.uniform_chunks == n * chunks
+    words = n * {"both": 2, "neither": 0}.get(listed, 1)
+    assert (info.plan_device_bytes == 0) == (n <= 128 or (n <= 896 and words <= 896))
+
+    def check(what):
+        want = np.zeros(entries * d_stride, dtype=np.uint8)
+        host = src.cpu().numpy()
+        for i, j in zip(si, di):
+            want[j * d_stride:j * d_stride + blk] = host[i * s_stride:i * s_stride + blk]
+        assert np.array_equal(dst.cpu().numpy(), want), what
+        src.add_(1)
+        dst.zero_()
+        torch.cuda.synchronize()
+
+    stream = torch.cuda.Stream()
+    for i in range(3):
+        assert lib.nixl_amd_copy_plan_launch_watched(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+        assert lib.nixl_amd_copy_plan_status(plan, 1) == 0
+        check(f"launch {i}")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        assert lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        check(f"replay {i}")
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+
+
 def test_run_tables_through_the_kernel_library(cuda):
     """nixl_amd_copy_plan_create_indexed_runs called directly: three source runs with
     different strides, two destination runs, 5000 random blocks (more than one bisection
