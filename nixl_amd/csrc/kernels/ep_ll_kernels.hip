@@ -742,7 +742,9 @@ launch_direct(const DirectArgs &a, dim3 grid, dim3 block, hipStream_t s) {
 // workgroup takes 64 consecutive rows of one expert, finds their source tokens (src_info
 // has the token, the segment the row lies in has the rank), gathers the tokens' scale rows
 // (contiguous, 16 bytes per lane) into LDS and writes them out along the row index, 16 bytes
-// per lane.
+// per lane.  What bounds it is that chain, and the lines it leaves to be written back at its end: with
+// ordinary and with non-temporal stores 32 x 64 x 5120 top-8 6.4 and 5.2 us, 16 x 128 x 7168 7.7 and 5.9, 32 x 128 x 7168 7.6
+// and 6.4 (with device scope 8.5, 10.3 and 9.3).
 
 struct ScalesArgs {
     void *recv_scales; // [E][G][N] float, or [E][G/4][N] words of four exponent bytes
@@ -825,8 +827,7 @@ ll_scales_kernel(ScalesArgs a) {
             uint32_t *dst = out + static_cast<size_t>(c) * d.N + s0 + r4;
             const uint32_t v0 = tile[r4 * (C + 1) + c];
             if (wide && r4 + 3 < rows) {
-                *reinterpret_cast<uint4 *>(dst) =
-                    make_uint4(v0, tile[(r4 + 1) * (C + 1) + c], tile[(r4 + 2) * (C + 1) + c], tile[(r4 + 3) * (C + 1) + c]);
+                st16_nt(dst, make_uint4(v0, tile[(r4 + 1) * (C + 1) + c], tile[(r4 + 2) * (C + 1) + c], tile[(r4 + 3) * (C + 1) + c]));
             } else {
                 dst[0] = v0;
                 for (int k = 1; k < 4 && r4 + k < rows; ++k)
@@ -1201,9 +1202,10 @@ launch_bits(int per_lane, dim3 grid, size_t lds, hipStream_t s, const BitsArgs &
 // of its own in front of this one and part of the bits' otherwise.
 constexpr int kDirectSelections = 2048, kDirectSelectionsMany = 3072, kDirectManyTopk = 4;
 // Up to this many words of scales the row kernel writes them itself, one isolated word at a time,
-// which spares the third launch; beyond it ll_scales_kernel moves them through LDS tiles.  Two
-// launches against three: 1024 tokens x top-8 x 56 words (459 thousand) 21.6 us against 26.4, 524
-// thousand 25.9 against 26.5, 917 thousand 44.8 against 44.3, 1.8 million 86.3 against 71.1.
+// which spares the third launch; beyond it ll_scales_kernel moves them through LDS tiles.  Passes with
+// combine, two launches against three: 179 thousand (8 x 50 x 7168, top-8) 23.6 us against 26.7, 358
+// thousand 38.0 against 41.1, 459 thousand 45.0 against 47.0, 487 thousand 52.1 against 51.8, 524 thousand (32 x 128 x 2048)
+// 52.5 against 51.9; dispatch alone there 26.2 against 27.2, of 1.8 million 86.3 against 71.1.
 constexpr long long kIsolatedScaleWords = 1 << 19;
 
 bool
