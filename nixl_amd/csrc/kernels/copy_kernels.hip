@@ -175,6 +175,19 @@ store16_part(uint64_t addr, const v4u &v) {
         asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"((gv4_ptr)(addr)), "v"(v) : "memory");
 }
 
+// Stores 16 bytes that the kernel behind this one reads, through the die's cache as it goes: what a
+// kernel leaves in there is written back when it ends, in front of the next one's start.  Requests of
+// 1280, 4096 and 3904 blocks by index, launch to end: 18.6 -> 18.3 us, 26.0 -> 25.6 and 26.9 -> 26.4.  Non-temporal
+// stores send the records to memory and the next kernel there for them: 19.0, 26.4 and 27.1.
+template<class T>
+__device__ __forceinline__ void
+store_ahead(T *at, const T &x) {
+    static_assert(sizeof(T) == 16);
+    v4u v;
+    __builtin_memcpy(&v, &x, 16);
+    store16_part<kPolPlainSc1Nt>(reinterpret_cast<uint64_t>(at), v);
+}
+
 // Workgroups are handed to the 8 dies round-robin.  With the swizzle on, die x works
 // through one contiguous eighth of the record array instead of every eighth record.
 __device__ __forceinline__ uint32_t
@@ -365,7 +378,7 @@ copy_inline_done_kernel(Recs recs, FastDiv chunks_per_rec, uint32_t n_chunks, Do
 __global__ void __launch_bounds__(256)
 upload_kernel(uint4 *__restrict__ dst, const uint4 *__restrict__ src, size_t n) {
     for (size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += static_cast<size_t>(gridDim.x) * blockDim.x)
-        dst[i] = src[i];
+        store_ahead(dst + i, src[i]);
 }
 
 // One wavefront per piece: the descriptor's own {src, dst, units} record, up to
@@ -613,7 +626,7 @@ __global__ void __launch_bounds__(kSortWindow)
 sort_records_kernel(UniformRec *recs, uint32_t n) {
     const uint32_t i = blockIdx.x * kSortWindow + threadIdx.x;
     const UniformRec sorted = sort_window(i < n ? recs[i] : UniformRec{}, i < n);
-    if (i < n) recs[i] = sorted;
+    if (i < n) store_ahead(recs + i, sorted);
 }
 
 // Records of an indexed plan: block i goes from src_base + src_index[i] * src_stride to
@@ -643,7 +656,7 @@ index_records_kernel(UniformRec *recs, IndexVector src_index, IndexVector dst_in
     UniformRec rec{};
     if (i < n) rec = UniformRec{src_base + index_at(src_index, i) * src_stride, dst_base + index_at(dst_index, i) * dst_stride};
     if constexpr (SORTED) rec = sort_window(rec, i < n);
-    if (i < n) recs[i] = rec;
+    if (i < n) store_ahead(recs + i, rec);
 }
 
 // The same for lists of several runs (a pool registered as several regions): index i of a
@@ -686,7 +699,7 @@ index_records_runs_kernel(UniformRec *recs, IndexVector src_index, IndexVector d
         rec = UniformRec{run_address(first[0], base[0], stride[0], n_src, index_at(src_index, i)),
                          run_address(first[1], base[1], stride[1], n_dst, index_at(dst_index, i))};
     if constexpr (SORTED) rec = sort_window(rec, i < n);
-    if (i < n) recs[i] = rec;
+    if (i < n) store_ahead(recs + i, rec);
 }
 
 // Records of a listed plan: pair i joins entry src_index[i] of one prepared list with entry
@@ -822,7 +835,7 @@ list_records_kernel(ListArgs a) {
     const uint32_t units = s.len / 16u, head = kPieceUnits - (static_cast<uint32_t>(d.addr >> 4) & 7u);
     uint32_t count = min(units, head), more = good ? units - count : 0;
     const uint32_t mine = (more + kPieceUnits - 1) / kPieceUnits; // records beyond the first
-    if (good) a.recs[i] = PieceRec{s.addr, d.addr | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
+    if (good) store_ahead(a.recs + i, PieceRec{s.addr, d.addr | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)});
 
     // sums over a workgroup fit 32 bits: at most kListMaxBytes a pair
     const uint32_t n_bad = __popcll(__ballot(here && !good));
@@ -873,8 +886,8 @@ list_records_kernel(ListArgs a) {
     uint32_t at = a.n + extra_at + wave_extra[wave] + (incl - mine);
     for (uint32_t first = count; more; first += count, more -= count) {
         count = min(more, kPieceUnits);
-        a.recs[at++] =
-            PieceRec{s.addr + first * 16ull, (d.addr + first * 16ull) | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)};
+        store_ahead(a.recs + at++,
+                    PieceRec{s.addr + first * 16ull, (d.addr + first * 16ull) | (static_cast<uint64_t>(count - 1) << kPieceUnitsShift)});
     }
 }
 
@@ -920,12 +933,12 @@ expand_runs_kernel(UniformRec *recs, const ChunkRun *runs, uint32_t n_runs, uint
         if (ends && left < chunk_bytes) {
             const uint32_t units = static_cast<uint32_t>(left + 15u) / 16u;
             const uint64_t off = run.len - units * 16u;
-            recs[c] = end_rec(run.src + off, run.dst + off, units);
+            store_ahead(recs + c, end_rec(run.src + off, run.dst + off, units));
         } else if (ends && at < run.back) {
-            recs[c] = end_rec(run.src, run.dst, (chunk_bytes - run.back + 15u) / 16u);
+            store_ahead(recs + c, end_rec(run.src, run.dst, (chunk_bytes - run.back + 15u) / 16u));
         } else {
             const uint64_t off = min(at > run.back ? at - run.back : 0, run.len - chunk_bytes);
-            recs[c] = UniformRec{run.src + off, run.dst + off};
+            store_ahead(recs + c, UniformRec{run.src + off, run.dst + off});
         }
     }
 }
