@@ -283,6 +283,53 @@ struct InlineIndices {
     }
 };
 
+// A request by index of any length whose vectors repeat themselves: the blocks of some sequences in every layer of
+// a cache, listed layer by layer or block by block.  Seen as a grid, rows of equal length, index (row, column)
+// of a listed side is an id of the column and `step` times the row, or an id of the row and `step` times the
+// column; a side that is not listed is consecutive.  The ids, counted from the smallest one of a side, take 16 bits.
+// No records are made and nothing is uploaded.  Requests made, moved and waited for, us, with records and so: 900 blocks of 1 KiB 15.0 and
+// 12.4, 65 520 44.0 and 31.9; of 4 KiB 2048 15.9 and 14.5, 8192 22.8 and 19.3, 32 768 60.2 and 53.5, 131 072 204 and 181; 15 250 of 9 KiB 62.4
+// and 58.5; 8192 of 16 KiB 54.5 and 51.9, 65 520 341 and 333; 2048 of 128 KiB 92.4 and 90.0.  What it costs the host to see
+// that indices are no grid is 0.1 to 0.3 us.
+constexpr uint32_t kGridIds = 1792;
+constexpr uint32_t kMaxGridRows = 65535; // the second dimension of a launch
+
+struct GridIndices {
+    struct Side {
+        uint64_t base, stride;
+        uint32_t first; // index, of a consecutive vector; what ids are counted from
+        uint32_t step;
+        uint32_t listed; // ~0 where the ids are in `ids`, from `place` on, 0 where the vector is consecutive (and `place` 0)
+        uint32_t place;
+    };
+
+    Side src, dst;
+    FastDiv row_length;
+    uint32_t by_column; // whose ids are listed: ~0 those of the columns, 0 those of the rows
+    alignas(4) uint16_t ids[kGridIds];
+
+    __device__ __forceinline__ UniformRec
+    at(uint32_t r) const {
+        uint32_t column;
+        const uint32_t row = row_length.quotient(r, column);
+        return at(row, column, r);
+    }
+
+    __device__ __forceinline__ UniformRec
+    at(uint32_t row, uint32_t column, uint32_t r) const {
+        const uint32_t named = (column & by_column) | (row & ~by_column), other = row ^ column ^ named; // named < kGridIds
+        const auto address = [&](const Side &s) {
+            // no branch, as above
+            const uint32_t i = s.place + named;
+            uint32_t two; // by a scalar load, which a word alone can have
+            __builtin_memcpy(&two, ids + (i & ~1u), sizeof(two));
+            const uint32_t id = (two >> (i % 2 * 16)) & 0xffffu;
+            return s.base + (s.first + ((id + other * s.step) & s.listed) + (r & ~s.listed)) * s.stride;
+        };
+        return UniformRec{address(src), address(dst)};
+    }
+};
+
 template<int POL, typename Recs>
 __global__ void __launch_bounds__(kWaveSize)
 copy_inline_kernel(Recs recs, FastDiv chunks_per_rec) {
@@ -290,6 +337,18 @@ copy_inline_kernel(Recs recs, FastDiv chunks_per_rec) {
     const uint32_t r = chunks_per_rec.quotient(blockIdx.x, chunk);
     const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * 16u) + threadIdx.x * 16u;
     const UniformRec rec = recs.at(r);
+    store16<POL>(rec.dst + off, load16<POL>(rec.src + off));
+}
+
+// Of such a request of many blocks: a row of the launch a row of the grid, so that a wave divides once (36 600 blocks of 9 KiB 121.5 -> 118.4
+// us; with a third dimension instead of the other division, so few workgroups a row, 142.9).
+template<int POL>
+__global__ void __launch_bounds__(kWaveSize)
+copy_grid_kernel(GridIndices grid, FastDiv chunks_per_rec) {
+    uint32_t chunk;
+    const uint32_t column = chunks_per_rec.quotient(blockIdx.x, chunk);
+    const uint64_t off = static_cast<uint64_t>(chunk) * (kWaveSize * 16u) + threadIdx.x * 16u;
+    const UniformRec rec = grid.at(blockIdx.y, column, blockIdx.y * grid.row_length.divisor + column);
     store16<POL>(rec.dst + off, load16<POL>(rec.src + off));
 }
 
@@ -1325,6 +1384,7 @@ struct nixl_amd_copy_plan {
     uint32_t uniform_wgs = 0;
     std::unique_ptr<InlineRecs> inline_recs; // instead of uniform_recs: a plan of a few blocks, nothing on the device
     std::unique_ptr<InlineIndices> inline_indices; // or of some more
+    std::unique_ptr<GridIndices> inline_grid; // or whose indices repeat themselves
     MixedArgs mixed_args{};
     uint32_t mixed_wgs = 0;
     const PieceRec *piece_recs = nullptr;
@@ -1618,6 +1678,177 @@ take_indices(const int32_t *from, size_t n, int32_t *to, bool dense, bool whole)
         study_indices(v, i, end, dense, f);
     }
     return f;
+}
+
+// Whether `n` indices, in rows of `length`, are a grid (GridIndices): listed by column every row is the one before it `step`
+// further on, listed by row every row ascends by `step`.
+static __attribute__((always_inline)) inline bool
+is_grid(const uint32_t *v, size_t n, uint32_t length, bool by_column, uint32_t step) {
+    if (by_column) {
+        for (size_t at = length; at < n;) {
+            const size_t end = std::min<size_t>(n, at + 1024);
+            uint32_t off = 0;
+            for (; at < end; ++at)
+                off |= (v[at] - v[at - length]) ^ step;
+            if (off) return false;
+        }
+        return true;
+    }
+    // no other steps than those from a row to the next: counted there first, then in all, which vectorises
+    size_t between = 0;
+    for (size_t at = length; at < n; at += length)
+        between += v[at] - v[at - 1] != step;
+    for (size_t at = 1; at < n;) {
+        const size_t end = std::min<size_t>(n, at + 1024);
+        uint32_t others = 0;
+        for (; at < end; ++at)
+            others += v[at] - v[at - 1] != step;
+        if (others > between) return false;
+        between -= others;
+    }
+    return between == 0;
+}
+
+// A grid listed by row has rows of at least kMinGridRow, which are looked at one by one, and is left to records of its own
+// where these are faster. Blocks that are neighbours in their list, us with records and as a grid: 12 288 of 8 KiB in rows of 16
+// 43.9 and 39.8, 14 336 48.0 and 49.5, 16 384 55.5 and 57.1 (of 4 KiB 32.3 and 33.5), 32 768 in rows of 32 97.4 and 99.7. Others: a
+// GiB in rows of 1092 of 16 KiB 364 and 357, of 546 of 32 KiB 353 and 357, of 273 of 64 KiB 334 and 340, of 136 of 128 KiB 322 and 330;
+// half a GiB of 64 KiB 171.5 and 171.4, of 128 KiB 168.4 and 168.7, of 256 KiB 169.7 and 167.9.
+constexpr size_t kMinGridRow = 8, kMaxConsecutive = 12288;
+constexpr uint64_t kMaxRowBlock = 16384, kMaxRowBytes = 512ull << 20;
+
+struct GridShape {
+    uint32_t length = 0; // of a row; 0: no grid
+    bool by_column;
+};
+
+// The shape of `n` >= 4 indices: rows as long as they ascend evenly from the start, or the first length at which
+// they start again as they started, as far on as the last row is from the one before it.  Few lengths are looked at
+// in full.
+static __attribute__((always_inline)) inline GridShape
+find_grid(const uint32_t *v, size_t n, bool by_row) {
+    const uint32_t step = v[1] - v[0];
+    size_t length = 2;
+    while (length < n && v[length] - v[length - 1] == step)
+        ++length;
+    if (step == 1 && n > kMaxConsecutive) by_row = false;
+    if (by_row && length >= kMinGridRow && n % length == 0 && n / length <= kGridIds && is_grid(v, n, static_cast<uint32_t>(length), false, step))
+        return {static_cast<uint32_t>(length), false};
+    constexpr size_t kStretch = 64;
+    int looks = 8;
+    for (size_t from = 2; from <= std::min<size_t>(n / 2, kGridIds); from += kStretch) {
+        const size_t end = std::min(from + kStretch, std::min<size_t>(n / 2, kGridIds) + 1);
+        uint32_t any = 0;
+        const auto may = [&](size_t i) { // i + 1 <= n / 2 + 1 < n
+            return static_cast<uint32_t>(v[i + 1] - v[i] == step) & static_cast<uint32_t>(v[n - 1] - v[n - 1 - i] == v[i] - v[0]);
+        };
+        for (size_t i = from; i < end; ++i)
+            any |= may(i);
+        if (!any) continue;
+        for (size_t i = from; i < end; ++i) {
+            if (!may(i) || n % i != 0) continue;
+            if (is_grid(v, n, static_cast<uint32_t>(i), true, v[i] - v[0])) return {static_cast<uint32_t>(i), true};
+            if (--looks == 0) return {};
+        }
+    }
+    return {};
+}
+
+// The ids of a side, `apart` from each other in `v`, counted from the smallest one (`lowest`, the largest one being `last`), or false if
+// they don't fit 16 bits.
+static __attribute__((always_inline)) inline bool
+take_ids(const uint32_t *v, size_t n_ids, size_t apart, uint16_t *to, uint32_t &lowest, uint32_t &last) {
+    uint32_t id[kGridIds]; // read once, whatever becomes of the caller's array
+    for (size_t i = 0; i < n_ids; ++i)
+        id[i] = v[i * apart];
+    uint32_t low = UINT32_MAX, high = 0;
+    for (size_t i = 0; i < n_ids; ++i) {
+        low = std::min(low, id[i]);
+        high = std::max(high, id[i]);
+    }
+    lowest = low;
+    last = high;
+    if (high - low > 0xffffu) return false;
+    for (size_t i = 0; i < n_ids; ++i)
+        to[i] = static_cast<uint16_t>(id[i] - low);
+    return true;
+}
+
+#if defined(__x86_64__)
+__attribute__((target("avx2"))) static bool
+take_ids_avx2(const uint32_t *v, size_t n_ids, size_t apart, uint16_t *to, uint32_t &lowest, uint32_t &last) {
+    return take_ids(v, n_ids, apart, to, lowest, last);
+}
+
+__attribute__((target("avx2"))) static GridShape
+find_grid_avx2(const uint32_t *v, size_t n, bool by_row) {
+    return find_grid(v, n, by_row);
+}
+
+__attribute__((target("avx2"))) static bool
+is_grid_avx2(const uint32_t *v, size_t n, uint32_t length, bool by_column, uint32_t step) {
+    return is_grid(v, n, length, by_column, step);
+}
+#endif
+
+// The indices of a request as a grid, if both vectors are consecutive or grids of one shape, one of them listed.  What
+// the kernel reads are the ids and steps taken here, and those are what is held against the lists' lengths:
+// a request that this turns away is looked at as any other, and told what is wrong with it.
+static std::unique_ptr<GridIndices>
+take_grid(const nixl_amd_copy_run_t &src_run, const int32_t *src_index, uint64_t src_entries, const nixl_amd_copy_run_t &dst_run,
+          const int32_t *dst_index, uint64_t dst_entries, size_t n, uint64_t len) {
+#if defined(__x86_64__)
+    const bool wide = __builtin_cpu_supports("avx2");
+    const auto find = wide ? find_grid_avx2 : [](const uint32_t *v, size_t of, bool by_row) { return find_grid(v, of, by_row); };
+    const auto is = wide ? is_grid_avx2 : [](const uint32_t *v, size_t of, uint32_t length, bool by_column, uint32_t step) {
+        return is_grid(v, of, length, by_column, step);
+    };
+    const auto take = wide ? take_ids_avx2 : [](const uint32_t *v, size_t n_ids, size_t apart, uint16_t *to, uint32_t &lowest, uint32_t &last) {
+        return take_ids(v, n_ids, apart, to, lowest, last);
+    };
+    const auto count = wide ? count_consecutive_avx2 : [](const uint32_t *v, uint32_t first, size_t of) { return count_consecutive(v, first, of); };
+#else
+    const auto find = find_grid;
+    const auto is = is_grid;
+    const auto take = take_ids;
+    const auto count = count_consecutive;
+#endif
+    const uint32_t *v[2] = {reinterpret_cast<const uint32_t *>(src_index), reinterpret_cast<const uint32_t *>(dst_index)};
+    const nixl_amd_copy_run_t *run[2] = {&src_run, &dst_run};
+    const uint64_t entries[2] = {src_entries, dst_entries};
+    // which are listed is guessed from their start: the shape of one that is decides more cheaply than all of one that is not
+    const auto looks_listed = [&](int side) { return count(v[side], v[side][0], std::min<size_t>(n, 1024)) < std::min<size_t>(n, 1024); };
+    const bool listed[2] = {looks_listed(0), looks_listed(1)};
+    if (!listed[0] && !listed[1]) return nullptr;
+    const GridShape shape = find(v[listed[0] ? 0 : 1], n, len <= kMaxRowBlock || n * len <= kMaxRowBytes);
+    if (shape.length == 0) return nullptr;
+    const size_t rows = n / shape.length, n_ids = shape.by_column ? shape.length : rows, others = shape.by_column ? rows : shape.length;
+    if (rows > kMaxGridRows) return nullptr;
+    std::unique_ptr<GridIndices> g(new GridIndices); // not cleared
+    g->row_length = FastDiv(shape.length);
+    g->by_column = shape.by_column ? ~0u : 0;
+    size_t place = 0;
+    for (int side = 0; side < 2; ++side) {
+        GridIndices::Side &s = side ? g->dst : g->src;
+        s = {run[side]->base, run[side]->stride, v[side][0], 0, 0, 0};
+        uint64_t highest = static_cast<uint64_t>(s.first) + (n - 1);
+        if (listed[side]) {
+            s.step = shape.by_column ? v[side][shape.length] - v[side][0] : v[side][1] - v[side][0];
+            if (place + n_ids > kGridIds || s.step > INT32_MAX) return nullptr;
+            if (side == 1 && listed[0] && !is(v[1], n, shape.length, shape.by_column, s.step)) return nullptr;
+            uint32_t lowest, last;
+            if (!take(v[side], n_ids, shape.by_column ? 1 : shape.length, g->ids + place, lowest, last)) return nullptr;
+            s.first = lowest;
+            s.listed = ~0u;
+            s.place = static_cast<uint32_t>(place);
+            place += n_ids;
+            highest = static_cast<uint64_t>(last) + static_cast<uint64_t>(others - 1) * s.step;
+        } else if (count(v[side], s.first, n) < n) {
+            return nullptr;
+        }
+        if (highest > INT32_MAX || highest >= entries[side]) return nullptr;
+    }
+    return g;
 }
 
 // Requests of at least so many pairs a run are sent as runs.  Making a request of 65 536 and of 262 144
@@ -2537,6 +2768,42 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
     const bool tables = n_src_runs > 1 || n_dst_runs > 1;
     const bool some = !inlined && !tables && fits_inline(n, len, t, kInlineIndices); // their indices may travel as arguments
     int32_t few[2 * kInlineIndices];
+    const auto is_scattered = [](const IndexFacts &dst, size_t of) { return !(of == 1 || 2 * static_cast<uint64_t>(dst.regular) >= of - 1); };
+    const auto is_sorted = [&](bool scattered, const IndexFacts &src, size_t of) {
+        return scattered && sort_pays(sort_scatter, n, len) && src_all_dense && 2 * static_cast<uint64_t>(src.ones) >= of - 1;
+    };
+    const auto new_plan = [&](bool scattered, bool sort) {
+        auto *plan = new nixl_amd_copy_plan();
+        plan->device = device;
+        plan->upl = upl;
+        plan->waves = waves;
+        plan->swizzle = swizzle;
+        plan->policy = nt ? nt : copy_policy(n * len, !scattered || sort);
+        return plan;
+    };
+    // More indices than an inline plan lists, but a grid.  It repeats itself, so its start says for all of it how regular it is.
+    const auto grid_plan = [&](size_t of, const auto &facts) { // of the first `of` indices of both sides
+        const auto sorted = [&] { // by the kernel that makes its records
+            const auto [src, dst] = facts();
+            return is_sorted(is_scattered(dst, of), src, of);
+        };
+        if (sort_pays(sort_scatter, n, len) && sorted()) return false;
+        auto grid = take_grid(src_runs[0], src_index, src_entries, dst_runs[0], dst_index, dst_entries, n, len);
+        if (!grid) return false;
+        auto *plan = new_plan(is_scattered(facts().second, of), false);
+        plan->inline_grid = std::move(grid);
+        describe_blocks(*plan, t, n, len, n);
+        *out = plan;
+        return true;
+    };
+    if (!inlined && !some && !tables && fits_inline(n, len, t, n)) {
+        const size_t start = std::size(few) / 2;
+        if (grid_plan(start, [&] {
+                return std::pair(take_indices(src_index, start, few, src_all_dense, true),
+                                 take_indices(dst_index, start, few + start, dst_all_dense, true));
+            }))
+            return NIXL_AMD_OK;
+    }
     void *staging = nullptr;
     size_t staging_cap = 0;
     const size_t table_at = (2 * index_bytes + 15) & ~size_t(15); // the run tables follow the index vectors
@@ -2562,19 +2829,13 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         if (staging) upload_cache().put(device, staging, staging_cap);
         return nixl_amd_fail(NIXL_AMD_ERR_INDEX, "plan_create_indexed: an index names no entry of its list");
     }
-    const bool scattered = !(n == 1 || 2 * static_cast<uint64_t>(dst_facts.regular) >= n - 1);
-    const bool sort = scattered && sort_pays(sort_scatter, n, len) && src_all_dense && 2 * static_cast<uint64_t>(src_facts.ones) >= n - 1;
+    const bool scattered = is_scattered(dst_facts, n), sort = is_sorted(scattered, src_facts, n);
     if (tables && !inlined) {
         auto *up_runs = reinterpret_cast<nixl_amd_copy_run_t *>(static_cast<uint8_t *>(staging) + table_at);
         std::memcpy(up_runs, src_runs, n_src_runs * sizeof(nixl_amd_copy_run_t));
         std::memcpy(up_runs + n_src_runs, dst_runs, n_dst_runs * sizeof(nixl_amd_copy_run_t));
     }
-    auto *plan = new nixl_amd_copy_plan();
-    plan->device = device;
-    plan->upl = upl;
-    plan->waves = waves;
-    plan->swizzle = swizzle;
-    plan->policy = nt ? nt : copy_policy(n * len, !scattered || sort);
+    auto *plan = new_plan(scattered, sort);
     if (inlined) {
         const auto address = [](const nixl_amd_copy_run_t *runs, size_t n_runs, uint64_t index) {
             const auto *run = std::upper_bound(runs, runs + n_runs, index, [](uint64_t i, const nixl_amd_copy_run_t &r) { return i < r.first_index; }) - 1;
@@ -2607,6 +2868,10 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
             plan->inline_indices = std::move(in);
             describe_blocks(*plan, t, n, len, n);
             *out = plan;
+            return NIXL_AMD_OK;
+        }
+        if (grid_plan(n, [&] { return std::pair(src_facts, dst_facts); })) {
+            delete plan;
             return NIXL_AMD_OK;
         }
         if (const int rc = take_staging()) {
@@ -3020,8 +3285,14 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
             told = true;
         } else {
             with_policy(plan->policy, [&]<int POL>() {
-                hipLaunchKernelGGL((copy_inline_kernel<POL, Recs>), dim3(plan->n_uniform), dim3(kWaveSize), 0, s, recs,
-                                   FastDiv(plan->chunks_per_rec));
+                if constexpr (std::is_same_v<Recs, GridIndices>) {
+                    const uint32_t length = recs.row_length.divisor, rows = plan->n_uniform / plan->chunks_per_rec / length;
+                    hipLaunchKernelGGL(copy_grid_kernel<POL>, dim3(plan->chunks_per_rec * length, rows), dim3(kWaveSize), 0, s, recs,
+                                       FastDiv(plan->chunks_per_rec));
+                } else {
+                    hipLaunchKernelGGL((copy_inline_kernel<POL, Recs>), dim3(plan->n_uniform), dim3(kWaveSize), 0, s, recs,
+                                       FastDiv(plan->chunks_per_rec));
+                }
             });
         }
         return hipGetLastError();
@@ -3030,6 +3301,8 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
         if (const hipError_t e = launch_inline(*plan->inline_recs); e != hipSuccess) return give_up(e);
     } else if (plan->inline_indices) {
         if (const hipError_t e = launch_inline(*plan->inline_indices); e != hipSuccess) return give_up(e);
+    } else if (plan->inline_grid) {
+        if (const hipError_t e = launch_inline(*plan->inline_grid); e != hipSuccess) return give_up(e);
     } else if (plan->uniform_wgs) {
         // One launch per kMaxGrid workgroups.  With the die swizzle each launch's grid is
         // rounded up to a multiple of 8 so that every die owns an equally long slice; surplus

@@ -21,6 +21,7 @@
 #include <set>
 #include <string>
 #include <thread>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -132,9 +133,32 @@ struct ListArgs {
 
 std::set<ListTotals *> g_totals; // that requests have counted in
 
+// Of the copies whose indices repeat themselves.
+struct GridIndices {
+    struct Side {
+        uint64_t base, stride;
+        uint32_t first, step, listed, place;
+    } src, dst;
+    uint32_t row_length[4]; // the number itself, and how to divide by it
+    uint32_t by_column, ids[1792 / 2];
+
+    uint64_t
+    address(const Side &s, uint32_t r) const {
+        const uint32_t row = r / row_length[0], column = r % row_length[0];
+        if (!s.listed) return s.base + static_cast<uint64_t>(s.first + r) * s.stride;
+        const uint32_t i = s.place + (by_column ? column : row);
+        REQUIRE(i < 1792);
+        const uint32_t id = i % 2 ? ids[i / 2] >> 16 : ids[i / 2] & 0xffffu;
+        return s.base + static_cast<uint64_t>(s.first + id + (by_column ? row : column) * s.step) * s.stride;
+    }
+};
+
+std::unique_ptr<GridIndices> g_grid; // of the last such launch
+
 std::function<void()>
 work_of(const std::string &kernel, dim3 grid, void **args) {
     const auto is = [&](const char *name) { return kernel.find(name) != std::string::npos; };
+    if (is("GridIndices")) g_grid = std::make_unique<GridIndices>(*static_cast<GridIndices *>(args[0]));
     if (is("copy_inline_done_kernel")) {
         const Done done = *static_cast<Done *>(args[3]);
         return [done] { *done.word = done.value; };
@@ -277,6 +301,94 @@ work_behind_a_watched_launch() {
     }
     for (void *shared : {static_cast<void *>(nullptr), static_cast<void *>(hipStreamLegacy), static_cast<void *>(hipStreamPerThread)})
         REQUIRE(nixl_amd_copy_watch_stream(0, shared, 1) == NIXL_AMD_ERR_INVALID);
+}
+
+// Requests by index whose vectors repeat themselves, listed by column or by row, on one side or both, and such with
+// one index changed: the addresses that a copy is told are those of the indices, and what it is told so or by records.
+void
+indices_that_repeat_themselves() {
+    constexpr uint64_t kLen = 1024;
+    constexpr uintptr_t kSrc = 1ull << 40, kDst = 1ull << 41;
+    uint32_t seed = 1;
+    const auto random = [&](uint32_t below) { return ((seed = seed * 1664525u + 1013904223u) >> 8) % below; };
+    Stream s;
+    const auto made = [&](const std::vector<int32_t> &src, const std::vector<int32_t> &dst, uint64_t entries, int sort = 0, uint64_t len = 1024) {
+        const nixl_amd_copy_run_t src_run{kSrc, kLen, 0, entries}, dst_run{kDst, 2 * kLen, 0, entries};
+        nixl_amd_copy_tuning_t tuning = tuning_for(s);
+        tuning.sort_scatter = sort;
+        nixl_amd_copy_plan_t *plan = nullptr;
+        const int rc = nixl_amd_copy_plan_create_indexed_lists(&src_run, 1, src.data(), entries, &dst_run, 1, dst.data(), entries, src.size(), len,
+                                                               0, &tuning, &plan);
+        if (rc) return rc;
+        g_grid.reset();
+        REQUIRE(nixl_amd_copy_plan_launch(plan, &s) == 0);
+        REQUIRE(nixl_amd_copy_plan_status(plan, 1) == 0);
+        if (g_grid)
+            for (uint32_t r = 0; r < src.size(); ++r) {
+                REQUIRE(g_grid->address(g_grid->src, r) == kSrc + static_cast<uint64_t>(src[r]) * kLen);
+                REQUIRE(g_grid->address(g_grid->dst, r) == kDst + static_cast<uint64_t>(dst[r]) * 2 * kLen);
+            }
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        return 0;
+    };
+    const uint32_t shapes[][2] = {{225, 4}, {64, 15}, {130, 7}, {130, 8}, {900, 17}, {3, 65535}, {3, 65536}, {3, 299}, {3, 300}, {250, 61}, {896, 2}, {897, 2}, {1791, 3}, {1792, 3}, {1793, 3}, {7, 1000}, {150, 3}};
+    for (const auto &[n_ids, others] : shapes)
+        for (const bool by_column : {true, false})
+            for (const int sides : {1, 2, 3}) // listed: the source, the destination, both
+                for (const uint32_t range : {3000u, 65536u, 65537u}) {
+                    const size_t n = static_cast<size_t>(n_ids) * others;
+                    if (static_cast<uint64_t>(range + 150) * others > INT32_MAX) continue;
+                    std::vector<int32_t> v[2];
+                    uint64_t entries = 0;
+                    for (int side = 0; side < 2; ++side) {
+                        std::vector<uint32_t> ids(n_ids);
+                        for (uint32_t &id : ids)
+                            id = random(range);
+                        ids[0] = 5; // neither even steps, nor all from one id on
+                        ids[1] = 0;
+                        ids[2] = range - 1;
+                        const uint32_t step = range + random(100), first = random(50);
+                        v[side].resize(n);
+                        for (size_t r = 0; r < n; ++r) {
+                            const size_t length = by_column ? n_ids : others, row = r / length, column = r % length;
+                            v[side][r] = static_cast<int32_t>(!(sides >> side & 1) ? first + r :
+                                                              by_column            ? first + ids[column] + row * step :
+                                                                                     first + ids[row] + column * step);
+                            entries = std::max(entries, static_cast<uint64_t>(v[side][r]) + 1);
+                        }
+                    }
+                    const bool fits = range <= 65536 && n_ids * (sides == 3 ? 2 : 1) <= 1792 && (by_column ? others <= 65535 : others >= 8), few = n <= 896 && sides != 3;
+                    REQUIRE(made(v[0], v[1], entries) == 0);
+                    REQUIRE((g_grid != nullptr) == (fits && !few && n > 448));
+                    REQUIRE(made(v[0], v[1], entries - 1) == NIXL_AMD_ERR_INDEX);
+                    for (const size_t at : {size_t(0), size_t(n_ids), n / 2, n - 1}) // one that breaks it
+                        for (int side = 0; side < 2; ++side) {
+                            auto changed = v[side];
+                            std::swap(changed, v[side]);
+                            v[side][at] ^= 1;
+                            REQUIRE(made(v[0], v[1], entries + 1) == 0);
+                            REQUIRE(g_grid == nullptr);
+                            v[side][at] = -1;
+                            REQUIRE(made(v[0], v[1], entries) == NIXL_AMD_ERR_INDEX);
+                            v[side] = changed;
+                        }
+                    s.kernels.clear();
+                    REQUIRE(made(v[0], v[1], entries, 1) == 0); // what is to be sorted has records
+                    const bool sorted = launched(s, "index_records_kernelILb1E") != 0;
+                    REQUIRE(!sorted || !g_grid);
+                    if (n >= 1024 && sides == 2 && by_column) REQUIRE(sorted);
+                }
+    // listed by row, large blocks of more than half a GiB and many that are neighbours have records
+    for (const auto &[rows, length, step, len, grid] : std::vector<std::tuple<int, int, int, uint64_t, bool>>{
+             {256, 128, 700, 16384, true}, {256, 128, 700, 17408, false}, {64, 512, 700, 16384, true}, {64, 512, 700, 32768, false},
+             {32, 512, 700, 32768, true}, {768, 16, 1, 8192, true}, {769, 16, 1, 8192, false}}) {
+        std::vector<int32_t> listed(static_cast<size_t>(rows) * length), flat(listed.size());
+        std::iota(flat.begin(), flat.end(), 0);
+        for (size_t r = 0; r < listed.size(); ++r) // every other place, in an order of its own
+            listed[r] = static_cast<int32_t>((r / length * 5 % rows) * (step == 1 ? 2 * length : 2) + r % length * step);
+        REQUIRE(made(listed, flat, 1u << 30, 0, len) == 0);
+        REQUIRE((g_grid != nullptr) == grid);
+    }
 }
 
 // A watched launch that fails is reported, whatever stream it went to: by a status that is polled
@@ -686,6 +798,7 @@ int
 main(int argc, char **argv) {
     const std::map<std::string, void (*)()> scenarios{
         {"work_behind_a_watched_launch", work_behind_a_watched_launch},
+        {"indices_that_repeat_themselves", indices_that_repeat_themselves},
         {"launch_on_a_named_stream_fails", launch_on_a_named_stream_fails},
         {"launch_on_the_legacy_stream_fails", launch_on_the_legacy_stream_fails},
         {"launch_on_the_stream_of_a_thread", launch_on_the_stream_of_a_thread},

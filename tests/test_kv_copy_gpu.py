@@ -597,6 +597,69 @@ def test_requests_whose_indices_travel_as_arguments(cuda, n, listed, chunks, pol
     assert lib.nixl_amd_copy_plan_destroy(plan) == 0
 
 
+@pytest.mark.parametrize("by_column", [True, False])
+@pytest.mark.parametrize("listed", ["source", "destination", "both"])
+@pytest.mark.parametrize("n_ids, others, chunks, policy", [(225, 4, 1, 0), (299, 3, 5, 1), (64, 61, 2, 0), (130, 7, 1, 0), (130, 8, 3, 0), (3, 700, 1, 2), (896, 2, 3, 0), (896, 17, 1, 0), (1792, 16, 1, 0),
+                                                           (1793, 16, 1, 0)])
+def test_requests_whose_indices_repeat_themselves(cuda, n_ids, others, chunks, policy, listed, by_column):
+    """Requests by index whose vectors are the same blocks in every layer, listed layer by layer or block by block, around the
+    number of blocks that a launch carries, for copies that count their own workgroups and longer ones: launched,
+    launched again on new bytes, and replayed from a graph."""
+    import torch
+    lib = _lib.kernels()
+    assert lib.nixl_amd_copy_watch_prepare() == 0
+    rng = np.random.default_rng(n_ids)
+    n, blk, pool = n_ids * others, 1024 * chunks, n_ids + 37
+    entries = pool * others + 5
+    s_stride, d_stride = blk, blk + 128
+
+    def vector(is_listed):
+        if not is_listed:
+            return np.arange(3, 3 + n, dtype=np.int32)
+        ids = rng.permutation(pool)[:n_ids]
+        at = np.arange(others)[:, None] * pool + ids[None, :] + 2
+        return np.ascontiguousarray((at if by_column else at.T).reshape(-1), dtype=np.int32)
+
+    si, di = vector(listed != "destination"), vector(listed != "source")
+    src = torch.from_numpy(rng.integers(0, 256, entries * s_stride, dtype=np.uint8)).to(cuda)
+    dst = torch.zeros(entries * d_stride, dtype=torch.uint8, device=cuda)
+    assert src.data_ptr() % 128 == 0 and dst.data_ptr() % 128 == 0
+    run = lambda t, stride: (_lib.CopyRun * 1)(_lib.CopyRun(t.data_ptr(), stride, 0, entries))  # noqa: E731
+    tuning, plan = _lib.CopyTuning(0, policy), ctypes.c_void_p()
+    given = si.copy(), di.copy()
+    assert lib.nixl_amd_copy_plan_create_indexed_runs(run(src, s_stride), 1, given[0].ctypes.data, run(dst, d_stride), 1, given[1].ctypes.data,
+                                                      n, blk, 0, ctypes.byref(tuning), ctypes.byref(plan)) == 0, _lib.kernels_error()
+    for g in given:
+        g.fill(0)  # the plan keeps nothing of the caller's vectors
+    info = _lib.CopyPlanInfo()
+    assert lib.nixl_amd_copy_plan_query(plan, ctypes.byref(info)) == 0
+    assert info.payload_bytes == n * blk and info.uniform_chunks == n * chunks
+    assert (info.plan_device_bytes == 0) == (n_ids * (2 if listed == "both" else 1) <= 1792 and (by_column or others >= 8))
+
+    def check(what):
+        rows = dst.cpu().numpy().reshape(entries, d_stride)
+        want = np.zeros_like(rows)
+        want[di, :blk] = src.cpu().numpy().reshape(entries, s_stride)[si]
+        assert np.array_equal(rows, want), what
+        src.add_(1)
+        dst.zero_()
+        torch.cuda.synchronize()
+
+    stream = torch.cuda.Stream()
+    for i in range(3):
+        assert lib.nixl_amd_copy_plan_launch_watched(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+        assert lib.nixl_amd_copy_plan_status(plan, 1) == 0
+        check(f"launch {i}")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        assert lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        check(f"replay {i}")
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+
+
 def test_run_tables_through_the_kernel_library(cuda):
     """nixl_amd_copy_plan_create_indexed_runs called directly: three source runs with
     different strides, two destination runs, 5000 random blocks (more than one bisection
