@@ -1954,6 +1954,11 @@ block_len_fits(uint64_t len, const Tuning &t) {
 // 537 MB 183 and 182, 839 MB 275 and 274.
 constexpr uint64_t kSortScatterFrom = 512ull << 20;
 
+// Scatters that are grids listed by column (GridIndices) are sorted if their blocks are as large as this. Sorted and as a grid, us, 734 MB of
+// 2 KiB 347 and 281, 940 MB of 4 KiB 382 and 347, 786 MB of 8 KiB 294 and 286, 562 and 956 MB of 9 KiB 245 and 221, 376 and 355, 1180 MB of 12 KiB
+// 443 and 438, 787 MB of 14 KiB 309 and 293; of 16 KiB 629 MB 241 and 244, 839 MB 314 and 324, 1074 MB 385 and 418; 1468 MB of 32 KiB 505 and 537.
+constexpr uint64_t kSortGridBlock = 16384;
+
 static bool
 sort_pays(int sort_scatter, size_t n, uint64_t len) {
     if (sort_scatter == 2 || n < kSortWindow) return false;
@@ -2787,7 +2792,7 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
             const auto [src, dst] = facts();
             return is_sorted(is_scattered(dst, of), src, of);
         };
-        if (sort_pays(sort_scatter, n, len) && sorted()) return false;
+        if ((sort_scatter == 1 || len >= kSortGridBlock) && sort_pays(sort_scatter, n, len) && sorted()) return false;
         auto grid = take_grid(src_runs[0], src_index, src_entries, dst_runs[0], dst_index, dst_entries, n, len);
         if (!grid) return false;
         auto *plan = new_plan(is_scattered(facts().second, of), false);

@@ -389,6 +389,17 @@ indices_that_repeat_themselves() {
         REQUIRE(made(listed, flat, 1u << 30, 0, len) == 0);
         REQUIRE((g_grid != nullptr) == grid);
     }
+    // a scatter of more than half a GiB is sorted if its blocks are large
+    std::vector<int32_t> by_column(700 * 64), flat(by_column.size());
+    std::iota(flat.begin(), flat.end(), 0);
+    for (size_t r = 0; r < by_column.size(); ++r)
+        by_column[r] = static_cast<int32_t>((r % 700) * (r % 700) % 701 + r / 700 * 800);
+    for (const uint64_t len : {11264u, 12288u, 15360u, 16384u}) {
+        s.kernels.clear();
+        REQUIRE(made(flat, by_column, 1u << 30, 0, len) == 0);
+        REQUIRE((g_grid != nullptr) == (len < 16384));
+        REQUIRE((launched(s, "index_records_kernelILb1E") != 0) == (len >= 16384));
+    }
 }
 
 // A watched launch that fails is reported, whatever stream it went to: by a status that is polled
