@@ -307,13 +307,12 @@ work_behind_a_watched_launch() {
 // one index changed: the addresses that a copy is told are those of the indices, and what it is told so or by records.
 void
 indices_that_repeat_themselves() {
-    constexpr uint64_t kLen = 1024;
     constexpr uintptr_t kSrc = 1ull << 40, kDst = 1ull << 41;
     uint32_t seed = 1;
     const auto random = [&](uint32_t below) { return ((seed = seed * 1664525u + 1013904223u) >> 8) % below; };
     Stream s;
     const auto made = [&](const std::vector<int32_t> &src, const std::vector<int32_t> &dst, uint64_t entries, int sort = 0, uint64_t len = 1024) {
-        const nixl_amd_copy_run_t src_run{kSrc, kLen, 0, entries}, dst_run{kDst, 2 * kLen, 0, entries};
+        const nixl_amd_copy_run_t src_run{kSrc, len, 0, entries}, dst_run{kDst, 2 * len, 0, entries};
         nixl_amd_copy_tuning_t tuning = tuning_for(s);
         tuning.sort_scatter = sort;
         nixl_amd_copy_plan_t *plan = nullptr;
@@ -325,8 +324,8 @@ indices_that_repeat_themselves() {
         REQUIRE(nixl_amd_copy_plan_status(plan, 1) == 0);
         if (g_grid)
             for (uint32_t r = 0; r < src.size(); ++r) {
-                REQUIRE(g_grid->address(g_grid->src, r) == kSrc + static_cast<uint64_t>(src[r]) * kLen);
-                REQUIRE(g_grid->address(g_grid->dst, r) == kDst + static_cast<uint64_t>(dst[r]) * 2 * kLen);
+                REQUIRE(g_grid->address(g_grid->src, r) == kSrc + static_cast<uint64_t>(src[r]) * len);
+                REQUIRE(g_grid->address(g_grid->dst, r) == kDst + static_cast<uint64_t>(dst[r]) * 2 * len);
             }
         REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
         return 0;
