@@ -41,36 +41,37 @@ HBM_PEAK_GBPS = 8000.0  # MI355X published HBM3E peak, decimal GB/s
 # reports null.
 _KV_PROFILE = "profiles/copy_uniform_kernel_kv_llama3_16KiB_32KiB.txt (rocprofv3 --pmc runs of this file, not this run)"
 MEASURED_TRAFFIC = {
-    (1024, 8192, 16384): {"bytes": 2155883520, "source": _KV_PROFILE},
-    (1024, 8192, 32768): {"bytes": 4303367616, "source": _KV_PROFILE},
-    ("small", 262144): {"bytes": 938782368,
+    (1024, 8192, 16384): {"bytes": 2151697050, "source": _KV_PROFILE},
+    (1024, 8192, 32768): {"bytes": 4299181107, "source": _KV_PROFILE},
+    ("small", 262144): {"bytes": 936329216,
                         "source": "profiles/copy_piece_kernel_small_descriptor_stress_262144x512B-4KiB.txt (rocprofv3 --pmc runs of "
                                   "this file, not this run)"},
 }
 
 
-def counter_samples(csv_path, counters, kernel_tag="copy_uniform_kernel", yardstick_tag="CUDAFunctorOnSelf_add<int>"):
+def counter_samples(csv_path, counters, kernel_tags=("copy_uniform_kernel", "copy_grid_kernel"), yardstick_tag="CUDAFunctorOnSelf_add<int>"):
     """Reads a rocprofv3 counter_collection.csv (one row per dispatch and counter: Kernel_Name,
-    Counter_Name, Counter_Value).  Returns ({counter: median over the kernel's dispatches},
-    {counter: largest value over the yardstick's dispatches}, number of kernel dispatches), or
-    None when either has no sample of some counter."""
+    Counter_Name, Counter_Value).  Returns ({counter: median over the kernel's dispatches, the mean of these
+    where several kernels have some (a step's gather and its scatter)}, {counter: largest value over the
+    yardstick's dispatches}, number of kernel dispatches), or None when either has no sample of some counter."""
     import csv
     import statistics
-    kernel = {c: [] for c in counters}
+    kernel = {c: {} for c in counters}
     yard = {c: [] for c in counters}
     with open(csv_path, newline="") as f:
         for row in csv.DictReader(f):
             c, name = row.get("Counter_Name"), row.get("Kernel_Name", "")
             if c not in kernel:
                 continue
-            if kernel_tag in name:
-                kernel[c].append(float(row["Counter_Value"]))
+            tag = next((t for t in kernel_tags if t in name), None)
+            if tag:
+                kernel[c].setdefault(tag, []).append(float(row["Counter_Value"]))
             elif yardstick_tag in name:
                 yard[c].append(float(row["Counter_Value"]))
     if any(not kernel[c] or not yard[c] for c in counters):
         return None
-    return ({c: statistics.median(kernel[c]) for c in counters}, {c: max(yard[c]) for c in counters},
-            len(kernel[counters[0]]))
+    return ({c: statistics.mean(statistics.median(v) for v in kernel[c].values()) for c in counters}, {c: max(yard[c]) for c in counters},
+            sum(len(v) for v in kernel[counters[0]].values()))
 
 
 def counter_medians(csv_path, counters, tags, yardstick_tag="CUDAFunctorOnSelf_add<int>"):
@@ -530,7 +531,7 @@ def run_kv(args, blk, order, steps, warmup, fresh_requests=4, sorted_ids=False, 
                      "frac": round(achieved / HBM_PEAK_GBPS, 4),
                      "traffic": traffic["bytes"] if traffic else None,
                      "traffic_source": traffic["source"] if traffic else None,
-                     "kernel": "copy_uniform_kernel<1,policy,1>",
+                     "kernel": "copy_grid_kernel<policy>, copy_uniform_kernel<1,policy,1> where records are sorted",
                      "avg_launch_ms": round(avg_launch_ms, 4),
                      "min_launch_ms": round(float(np.min(kernel_ms)), 4),
                      "p99_launch_ms": round(float(np.percentile(kernel_ms, 99)), 4),
@@ -648,9 +649,9 @@ def run_concurrent_requests(args, blk, counts=(1, 2, 4), steps=10, warmup=3):
 def run_counter_sequence(args, blk, repeats=6):
     """A fixed sequence of launches for hardware-counter runs (rocprofv3 --pmc ... -- python3
     bench.py --counter-sequence), so that counters can be told apart per access pattern although
-    the kernel is the same: copy_uniform_kernel `repeats` times each as (1) gather and (2)
-    scatter of config 2 listed layer by layer, (3) gather and (4) scatter listed block by block,
-    (5) one contiguous descriptor of the same payload; then the small-descriptor stress
+    the kernel is the same: `repeats` times each (1) gather and (2)
+    scatter of config 2 listed layer by layer, (3) gather and (4) scatter listed block by block (copy_uniform_kernel in (2),
+    copy_grid_kernel in the others), (5) one contiguous descriptor of the same payload (copy_inline_kernel); then the small-descriptor stress
     (copy_piece_kernel) and the expert-parallel dispatch and combine of both modes, whose
     kernels have names of their own.  Prints the order as one JSON line; times nothing."""
     import torch
@@ -709,7 +710,7 @@ def run_counter_sequence(args, blk, repeats=6):
     run_small_descriptors(steps=repeats, warmup=1)
     from nixl_amd import ep_bench
     ep_bench.run_traffic_child(repeats=repeats, normal_mode=True)
-    print(json.dumps({"copy_uniform_kernel_launches": order, "descriptor_bytes": blk, "repeats": repeats}))
+    print(json.dumps({"copy_kernel_launches": order, "descriptor_bytes": blk, "repeats": repeats}))
 
 
 def run_prep_breakdown_child(args, blk):
