@@ -59,7 +59,8 @@ typedef struct nixl_amd_copy_tuning {
     int xcd_swizzle; /* 1 = each accelerator die walks a contiguous slice of the chunk list, 2 = off */
     int sort_scatter; /* a plan that scatters consecutive memory over irregular destinations has its records put
                        * into ascending destination order inside windows of 1024 (on the device): 1 = on, 2 = off,
-                       * 0 = on for requests of more than 512 MiB */
+                       * 0 = on for requests of more than 512 MiB, unless they are by index, of blocks below 16 KiB and
+                       * their indices repeat themselves (such a request has no records) */
     /* The HIP stream the plan will be launched on, or NULL.  While that stream is idle the
      * kernels that write the plan's arrays are queued on it, so that a launch needs no wait; the
      * stream must then outlive the plan, and while it is under capture the plan can be launched
