@@ -116,11 +116,14 @@ class nixl_xfer_dlist:
         self.mem = mem
         self.triples = triples
         h = ctypes.c_void_p()
+        n = triples.shape[0]
         rows = np.ascontiguousarray(triples, dtype=np.uint64)
-        if rows.shape[1] != 3:
-            rows = np.ascontiguousarray(rows[:, :3])
+        if rows.shape != (n, 3):
+            rows = np.stack([rows[:, 0], rows[:, 1], rows[:, 2]], 1)
+            if rows.size != 3 * n:  # 24 bytes a row are read
+                raise IndexError("a descriptor list takes one address, length and device id a row")
         _check("create_xfer_dlist", self._lib.nixl_capi_create_xfer_dlist_of(
-            mem, rows.__array_interface__["data"][0], rows.shape[0], ctypes.byref(h)))
+            mem, rows.__array_interface__["data"][0], n, ctypes.byref(h)))
         self._h = h
 
     def descCount(self):

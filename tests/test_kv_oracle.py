@@ -364,6 +364,16 @@ def test_lists_from_any_layout_of_triples(cpu_agent, form, n):
     req.release()
 
 
+@pytest.mark.parametrize("shape", [(4,), (4, 0), (4, 2), (4, 3, 0), (4, 3, 2), (4, 4, 2), (4, 2, 3)])
+def test_lists_are_not_made_of_rows_that_are_no_triples(shape):
+    """A list made directly takes three columns of one value a row, and reads nothing behind them."""
+    with pytest.raises(IndexError):
+        ag.nixl_xfer_dlist(np.ones(shape, dtype=np.uint64), 0)
+    with pytest.raises(AttributeError):
+        ag.nixl_xfer_dlist([(1, 2, 0)], 0)
+    assert ag.nixl_xfer_dlist(np.ones((4, 3, 1), dtype=np.uint64), 0).descCount() == 4
+
+
 def test_api_behaviour_of_the_reference_python_tests(cpu_agent, oracle_plugin_dir):
     """Cases of the reference's test/python/test_nixl_api.py that concern one agent:
     empty name (:90-93), unknown operation (:135-142), unknown plugin name gives empty
