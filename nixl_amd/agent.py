@@ -118,7 +118,7 @@ class nixl_xfer_dlist:
         h = ctypes.c_void_p()
         n = triples.shape[0]
         rows = np.ascontiguousarray(triples, dtype=np.uint64)
-        if rows.shape != (n, 3):
+        if n and rows.shape != (n, 3):
             rows = np.stack([rows[:, 0], rows[:, 1], rows[:, 2]], 1)
             if rows.size != 3 * n:  # 24 bytes a row are read
                 raise IndexError("a descriptor list takes one address, length and device id a row")

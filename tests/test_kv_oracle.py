@@ -374,6 +374,11 @@ def test_lists_are_not_made_of_rows_that_are_no_triples(shape):
     assert ag.nixl_xfer_dlist(np.ones((4, 3, 1), dtype=np.uint64), 0).descCount() == 4
 
 
+@pytest.mark.parametrize("empty", [np.zeros(0), np.zeros(0, np.uint64), np.zeros((0, 2), np.uint64), np.zeros((0, 3), np.uint64)])
+def test_lists_of_no_descriptors_from_any_empty_array(empty):
+    assert ag.nixl_xfer_dlist(empty, 0).descCount() == 0
+
+
 def test_api_behaviour_of_the_reference_python_tests(cpu_agent, oracle_plugin_dir):
     """Cases of the reference's test/python/test_nixl_api.py that concern one agent:
     empty name (:90-93), unknown operation (:135-142), unknown plugin name gives empty
