@@ -1093,7 +1093,8 @@ class BlockCache {
 public:
     explicit BlockCache(bool pinned) : pinned_(pinned) {}
 
-    // A block of at least `bytes` on `device` (ignored for pinned memory); `cap` receives its size.
+    // A block of at least `bytes` on `device` (ignored for pinned memory); `cap` receives its size.  Both are left as
+    // they are if there is none.
     hipError_t
     get(int device, size_t bytes, void **out, size_t *cap) {
         size_t size = 4096;
@@ -1110,8 +1111,12 @@ public:
                     return hipSuccess;
                 }
         }
+        void *ptr = nullptr;
+        const hipError_t e = pinned_ ? hipHostMalloc(&ptr, size, hipHostMallocDefault) : hipMalloc(&ptr, size);
+        if (e != hipSuccess) return e;
+        *out = ptr;
         *cap = size;
-        return pinned_ ? hipHostMalloc(out, size, hipHostMallocDefault) : hipMalloc(out, size);
+        return hipSuccess;
     }
 
     // The block just given back is the likeliest to be asked for again (the next request of the

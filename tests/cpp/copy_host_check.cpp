@@ -72,6 +72,7 @@ struct Event {
 std::recursive_mutex g_lock;
 hipError_t g_launch_status = hipSuccess; // of one launch,
 int g_good_launches = 0; // behind so many that are accepted
+int g_refused_pinned = 0; // allocations of pinned memory that fail from here on
 void (*g_synchronized)(Stream &) = nullptr; // in front of a wait for a stream
 Stream *g_created = nullptr; // the last stream that the library made
 
@@ -567,6 +568,29 @@ refused_launches_keep_no_totals() {
     REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
 }
 
+// A request of byte descriptors while pinned memory is short: what cannot be had ahead is asked for again
+// when its size is known, and if it cannot be had then either the request is refused.
+void
+pinned_memory_is_short() {
+    Stream s;
+    const nixl_amd_copy_tuning_t tuning = tuning_for(s);
+    size_t n = 100;
+    for (const int refused : {1, 2, 0, 1, 2, 0}) {
+        std::vector<nixl_amd_copy_desc_t> descs(n *= 4); // longer than what earlier requests gave back
+        for (size_t i = 0; i < n; ++i)
+            descs[i] = {(1ull << 40) + i * 64 + 1, (1ull << 41) + i * 64, 33};
+        g_refused_pinned = refused;
+        nixl_amd_copy_plan_t *plan = nullptr;
+        const int rc = nixl_amd_copy_plan_create(descs.data(), n, 0, &tuning, &plan);
+        REQUIRE(rc == (refused == 2 ? NIXL_AMD_ERR_HIP : NIXL_AMD_OK) && g_refused_pinned == 0);
+        const hipError_t left = hipGetLastError();
+        if (rc) continue;
+        REQUIRE(left == hipSuccess); // for the caller's next call
+        REQUIRE(nixl_amd_copy_plan_launch(plan, &s) == 0);
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+    }
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -685,6 +709,10 @@ hipMalloc(void **p, size_t n) {
 
 hipError_t
 hipHostMalloc(void **p, size_t n, unsigned flags) {
+    if (g_refused_pinned > 0) {
+        --g_refused_pinned;
+        return g_last_status = hipErrorOutOfMemory;
+    }
     const hipError_t e = hipMalloc(p, n);
     if (flags & hipHostMallocPortable) { // the words that launches are watched by
         g_words = static_cast<uint8_t *>(*p);
@@ -815,6 +843,7 @@ main(int argc, char **argv) {
         {"launch_seen_by_two_threads", launch_seen_by_two_threads},
         {"many_requests_wait_for_verdicts", many_requests_wait_for_verdicts},
         {"refused_launches_keep_no_totals", refused_launches_keep_no_totals},
+        {"pinned_memory_is_short", pinned_memory_is_short},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
