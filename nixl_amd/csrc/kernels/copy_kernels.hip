@@ -2405,6 +2405,7 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
     LongDescs chunks(chunk_bytes);
     ByteDescs bytes;
     Staging buffer(device); // what is uploaded; items are written there at once
+    bool asked_ahead = false; // for that buffer: once, as it takes a look at the whole list
     bool whole_chunks = false; // there are chunks of some aligned descriptor whatever becomes of those
     for (size_t i = 0; i < n; ++i) {
         const nixl_amd_copy_desc_t &d = descs[i];
@@ -2416,7 +2417,8 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         if (((d.src | d.dst | d.len) & 15u) != 0) {
             if (((d.src + d.len) | (d.dst + d.len)) >> kPieceUnitsShift)
                 return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create: address beyond 2^56");
-            if (!bytes.items.at) {
+            if (!asked_ahead) {
+                asked_ahead = true;
                 constexpr size_t kMostAhead = 64u << 20;
                 const size_t ahead = (ByteDescs::most(descs, i, n) + ByteDescs::kMost) * sizeof(GenericItem);
                 reap_uploads(device);

@@ -73,6 +73,7 @@ std::recursive_mutex g_lock;
 hipError_t g_launch_status = hipSuccess; // of one launch,
 int g_good_launches = 0; // behind so many that are accepted
 int g_refused_pinned = 0; // allocations of pinned memory that fail from here on
+std::vector<size_t> g_pinned; // those asked for
 void (*g_synchronized)(Stream &) = nullptr; // in front of a wait for a stream
 Stream *g_created = nullptr; // the last stream that the library made
 
@@ -591,6 +592,25 @@ pinned_memory_is_short() {
     }
 }
 
+// What cannot be had ahead is not asked for ahead again in the same request.
+void
+pinned_memory_is_asked_for_once() {
+    Stream s;
+    const nixl_amd_copy_tuning_t tuning = tuning_for(s);
+    std::vector<nixl_amd_copy_desc_t> descs;
+    for (size_t i = 0; i < 64; ++i) {
+        descs.push_back({(1ull << 40) + i * (2ull << 20) + 1, (1ull << 41) + i * (2ull << 20), (1 << 20) + 2});
+        descs.push_back({(3ull << 40) + i * 4096, (4ull << 40) + i * 4096, 640});
+    }
+    nixl_amd_copy_plan_t *plan = nullptr;
+    g_refused_pinned = 1000;
+    g_pinned.clear();
+    REQUIRE(nixl_amd_copy_plan_create(descs.data(), descs.size(), 0, &tuning, &plan) == NIXL_AMD_ERR_HIP);
+    REQUIRE(g_pinned.size() <= 2);
+    g_refused_pinned = 0;
+    (void)hipGetLastError();
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -709,6 +729,8 @@ hipMalloc(void **p, size_t n) {
 
 hipError_t
 hipHostMalloc(void **p, size_t n, unsigned flags) {
+    LOCKED;
+    g_pinned.push_back(n);
     if (g_refused_pinned > 0) {
         --g_refused_pinned;
         return g_last_status = hipErrorOutOfMemory;
@@ -844,6 +866,7 @@ main(int argc, char **argv) {
         {"many_requests_wait_for_verdicts", many_requests_wait_for_verdicts},
         {"refused_launches_keep_no_totals", refused_launches_keep_no_totals},
         {"pinned_memory_is_short", pinned_memory_is_short},
+        {"pinned_memory_is_asked_for_once", pinned_memory_is_asked_for_once},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
