@@ -2174,15 +2174,25 @@ struct ByteDescs {
         items.end_at(cut(items.room(len / reach + 2, longs.size()), src, dst, len, reach));
     }
 
-    // Items of one short descriptor at most, and of short ones among descs[i .. end) together.
+    // Items of one short descriptor at most.
     static constexpr size_t kMost = kSplitFromBytes / kGenericRound + 2;
 
+    // Bytes to have ahead for the items of short descriptors among descs[i .. end), or 0 if they are too many.  The
+    // lengths alone decide while they ask for little (3000 descriptors 1.4 us, 2.4 with a look at what is
+    // aligned); beyond that only what has items counts.
     static size_t
-    most(const nixl_amd_copy_desc_t *descs, size_t i, size_t end) {
-        size_t rounds = 0;
+    ahead(const nixl_amd_copy_desc_t *descs, size_t i, size_t end) {
+        constexpr size_t kLittle = 512u << 10, kTooMany = 64u << 20;
+        const auto bytes = [](size_t n_items) { return (n_items + kMost) * sizeof(GenericItem); };
+        size_t items = 2 * (end - i);
         for (size_t j = i; j < end; ++j)
-            rounds += descs[j].len < kSplitFromBytes ? descs[j].len / kGenericRound : 0;
-        return rounds + 2 * (end - i);
+            items += descs[j].len < kSplitFromBytes ? descs[j].len / kGenericRound : 0;
+        if (bytes(items) <= kLittle) return bytes(items);
+        items = 0;
+        for (size_t j = i; j < end; ++j)
+            if (((descs[j].src | descs[j].dst | descs[j].len) & 15u) != 0 && descs[j].len < kSplitFromBytes)
+                items += descs[j].len / kGenericRound + 2;
+        return bytes(items) <= kTooMany ? bytes(items) : 0;
     }
 
     // Takes descriptors from `i` on until one that is aligned or that plan_create refuses; returns
@@ -2419,13 +2429,14 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
                 return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_create: address beyond 2^56");
             if (!asked_ahead) {
                 asked_ahead = true;
-                constexpr size_t kMostAhead = 64u << 20;
-                const size_t ahead = (ByteDescs::most(descs, i, n) + ByteDescs::kMost) * sizeof(GenericItem);
+                const size_t ahead = ByteDescs::ahead(descs, i, n);
                 reap_uploads(device);
-                if (ahead <= kMostAhead && buffer.get(ahead) == hipSuccess)
-                    bytes.items.lend(buffer.at, buffer.cap);
-                else
-                    (void)hipGetLastError();
+                if (ahead != 0) {
+                    if (buffer.get(ahead) == hipSuccess)
+                        bytes.items.lend(buffer.at, buffer.cap);
+                    else
+                        (void)hipGetLastError();
+                }
             }
             i = bytes.take(descs, i, n) - 1; // this one, and the ones behind it as far as they are like it
             continue;

@@ -611,6 +611,29 @@ pinned_memory_is_asked_for_once() {
     (void)hipGetLastError();
 }
 
+// What byte descriptors are written to ahead is as long as they need, whatever else is in the list.
+void
+pinned_memory_is_for_byte_descriptors() {
+    Stream s;
+    const nixl_amd_copy_tuning_t tuning = tuning_for(s);
+    constexpr size_t kDescs = 100000;
+    std::vector<nixl_amd_copy_desc_t> descs;
+    for (size_t i = 0; i < kDescs; ++i) // a record of 16 bytes for each
+        descs.push_back({(1ull << 40) + i * 4096, (2ull << 40) + i * 4096, 640});
+    for (size_t i = 0; i < kDescs; i += 100) // and an item of 24 for some
+        descs[i] = {(3ull << 40) + i * 64 + 1, (4ull << 40) + i * 64, 33};
+    for (const size_t n : {size_t(50), kDescs}) {
+        nixl_amd_copy_plan_t *plan = nullptr;
+        g_pinned.clear();
+        REQUIRE(nixl_amd_copy_plan_create(descs.data(), n, 0, &tuning, &plan) == 0);
+        nixl_amd_copy_plan_info_t info{};
+        REQUIRE(nixl_amd_copy_plan_query(plan, &info) == 0);
+        for (const size_t size : g_pinned)
+            REQUIRE(size <= std::max<size_t>(512 << 10, 2 * info.plan_device_bytes));
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+    }
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -867,6 +890,7 @@ main(int argc, char **argv) {
         {"refused_launches_keep_no_totals", refused_launches_keep_no_totals},
         {"pinned_memory_is_short", pinned_memory_is_short},
         {"pinned_memory_is_asked_for_once", pinned_memory_is_asked_for_once},
+        {"pinned_memory_is_for_byte_descriptors", pinned_memory_is_for_byte_descriptors},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
