@@ -112,9 +112,11 @@ struct Done {
 };
 
 struct ListTotals {
-    unsigned long long bytes_arrived, extra_continued;
+    unsigned long long bytes_arrived;
+    alignas(128) unsigned long long extra_continued;
     uint32_t bad;
 };
+static_assert(sizeof(ListTotals) == 256);
 
 struct ListVerdict {
     unsigned long long bytes;
@@ -178,9 +180,13 @@ work_of(const std::string &kernel, dim3 grid, void **args) {
         const ListArgs a = *static_cast<ListArgs *>(args[0]);
         g_totals.insert(a.totals);
         return [a, grid] {
-            REQUIRE(a.totals->bytes_arrived == 0 || a.first_workgroup != 0); // nothing of an earlier request's
-            a.totals->bytes_arrived += grid.x;
-            if (a.totals->bytes_arrived != a.n_workgroups) return;
+            ListTotals &t = *a.totals;
+            if (a.first_workgroup == 0) REQUIRE(t.bytes_arrived == 0 && t.extra_continued == 0 && t.bad == 0); // nothing of an earlier request's
+            t.bytes_arrived += grid.x;
+            t.extra_continued += 3 * grid.x;
+            t.bad += 7 * grid.x;
+            if (t.bytes_arrived != a.n_workgroups) return;
+            REQUIRE(t.extra_continued == 3 * a.n_workgroups && t.bad == 7 * a.n_workgroups);
             *a.totals = ListTotals{};
             a.verdict->bytes = a.n;
             a.verdict->there = 1;
