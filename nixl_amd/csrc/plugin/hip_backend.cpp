@@ -396,7 +396,6 @@ nixlHipEngine::lowerGeneral(bool write,
                             int &device,
                             size_t &bytes) const {
     const int n = local.descCount();
-    const nixlHipMD *prev_lmd = nullptr, *prev_rmd = nullptr;
     const nixlMetaDesc *const L = &local[0], *const R = &remote[0];
     for (int i = 0; i < n;) {
         const nixlMetaDesc &l = L[i];
@@ -413,11 +412,7 @@ nixlHipEngine::lowerGeneral(bool write,
         }
         // The kernel runs on the device that owns the VRAM side(s); two VRAM regions on
         // different devices would need peer mappings, which this backend does not set up.
-        // Checked once per pair of regions: consecutive descriptors mostly share theirs.
-        const bool same_regions = (lmd == prev_lmd && rmd == prev_rmd);
-        prev_lmd = lmd;
-        prev_rmd = rmd;
-        if (!same_regions) for (const nixlHipMD *md : {lmd, rmd}) {
+        for (const nixlHipMD *md : {lmd, rmd}) {
             if (md->mem != VRAM_SEG) continue;
             if (device < 0) device = md->device;
             if (md->device != device) {
@@ -425,7 +420,7 @@ nixlHipEngine::lowerGeneral(bool write,
                 return NIXL_ERR_NOT_SUPPORTED;
             }
         }
-        // The pairs of the same two regions behind this one (this one again first): their bounds stay in registers and
+        // A stretch of pairs of these two regions (consecutive ones mostly are), this one again first: their bounds stay in registers and
         // their checks are looked at once.  A pair that fails one ends the stretch and is found again above.
         const nixlBackendMD *const lkey = l.metadataP, *const rkey = r.metadataP;
         const uintptr_t lbase = lmd->addr, rbase = rmd->addr;
