@@ -124,19 +124,26 @@ using gv4_cptr = const __attribute__((address_space(1))) v4u_any *;
 //   4  nt loads,    sc1 nt stores       6.71       6.35         5.80          5.15
 // "sc1 nt" is a streaming store with device scope.  A plan whose destinations adjoin or
 // advance by a constant step takes 4, any other plan 3; and 3 any plan whose payload is read and
-// written inside the last-level cache of 256 MiB (copy_policy).  Policies 4 and 3 there, us from launch to
-// end, three requests with buffers of their own in turn (and one again and again):
-//                16 MiB       32 MiB       64 MiB       96 MiB       112 MiB      128 MiB
-//   seq->seq     12.5 12.2    18.0 16.8    27.9 25.5    37.6 38.0    42.5 43.4    47.4 48.5 (48.0 42.9)
-//   random->seq  12.9 12.2    19.0 17.0    29.6 27.8    40.2 38.1    45.5 45.2    50.8 51.6 (50.7 44.6)
-//   seq->random  13.2 12.4    19.8 17.2    31.9 26.7    45.0 44.2    51.2 51.0    56.9 56.3 (56.7 45.6)
+// written inside the last-level cache of 256 MiB (copy_policy): up to 112 MiB, and up to 88 where sources follow
+// one another.  Policies 4 and 3 there, us from launch to end, three requests with buffers of their own in turn (and one
+// again and again):
+//                                     64 MiB       88 MiB       96 MiB       104 MiB      112 MiB
+//   one descriptor                    28.0 25.9    35.1 33.5    37.6 38.6    39.9 41.1    42.5 43.6 (42.3 38.9)
+//   16 KiB, both sides following      28.5 25.9    36.3 35.7    39.0 39.4    41.2 41.9    43.9 44.3 (43.9 39.7)
+//   16 KiB, destinations a step on    28.2 26.0    36.9 37.1    38.4 39.2    41.5 42.1    44.0 44.8 (43.9 39.7)
+//   16 KiB gathered                   30.2 28.1    38.3 36.9    41.2 39.2    43.7 42.2    46.2 45.8 (46.1 40.6)
+//   1 MiB gathered                                 37.8 36.4    40.2 39.1    43.0 42.0    45.2 44.1 (44.6 41.2)
+//   2 KiB gathered (pieces)                        40.5 35.9    42.9 42.4    45.9 45.4    49.7 49.3 (49.5 42.0)
+//   16 KiB scattered                  32.1 26.5    40.7 37.0    43.7 43.0    46.6 46.1    49.1 49.1 (49.3 40.0)
+// 16 KiB gathered 128 MiB 51.5 and 51.9 (51.1 45.3), 144 MiB 56.9 and 58.5.  At 16 and 32 MiB 3 is 0.3 to 2.6 faster.
 constexpr int kPolNtNt = 1, kPolPlain = 2, kPolPlainSc1Nt = 3, kPolNtSc1Nt = 4;
-constexpr uint64_t kInLastLevelCache = 112ull << 20; // of payload
+constexpr uint64_t kInLastLevelCache = 112ull << 20, kFollowingInLastLevelCache = 88ull << 20; // of payload
 
 // `regular`: destinations adjoin, advance by a constant step or are sorted, or the copy does not depend on it.
+// `following`: so do sources adjoin.
 constexpr int
-copy_policy(uint64_t payload, bool regular) {
-    return regular && payload > kInLastLevelCache ? kPolNtSc1Nt : kPolPlainSc1Nt;
+copy_policy(uint64_t payload, bool regular, bool following) {
+    return regular && payload > (following ? kFollowingInLastLevelCache : kInLastLevelCache) ? kPolNtSc1Nt : kPolPlainSc1Nt;
 }
 
 template<int POL>
@@ -2288,7 +2295,7 @@ build_block_plan(int device, const Tuning &t, void *staging, size_t staging_cap,
     const bool scattered = !(steps == 0 || 2 * regular >= steps);
     // a scatter out of consecutive memory is put into ascending destination order, window by window
     const bool sort = scattered && sort_pays(t.sort_scatter, n_recs, len) && 2 * src_follows >= steps;
-    plan->policy = t.nt ? t.nt : copy_policy(n_recs * len, !scattered || sort);
+    plan->policy = t.nt ? t.nt : copy_policy(n_recs * len, !scattered || sort, 2 * src_follows >= steps);
     if (fits_inline(n_recs, len, t)) {
         plan->inline_recs = std::make_unique<InlineRecs>();
         std::memcpy(plan->inline_recs->rec, recs, bytes);
@@ -2540,23 +2547,25 @@ nixl_amd_copy_plan_create(const nixl_amd_copy_desc_t *descs,
         // Destinations that adjoin (a gather into staging, one long copy) or advance by a
         // constant step (the same block of every layer of a pool) take non-temporal loads where they
         // are long; destinations without such a pattern (a scatter over a pool) take plain loads.
-        uint64_t pairs = 0, regular = 0, prev_dst = 0, prev_end = 0, prev_step = 0;
-        const bool matters = copy_policy(payload, true) != copy_policy(payload, false);
+        uint64_t pairs = 0, regular = 0, following = 0, prev_dst = 0, prev_end = 0, prev_step = 0, prev_src_end = 0;
+        const bool matters = copy_policy(payload, true, true) != copy_policy(payload, false, false);
         for (size_t i = 0; matters && i < n; ++i) {
             if (descs[i].len == 0) continue;
             if (prev_end) {
                 const uint64_t step = descs[i].dst - prev_dst;
                 ++pairs;
                 regular += (descs[i].dst == prev_end || step == prev_step);
+                following += descs[i].src == prev_src_end;
                 prev_step = step;
             }
             prev_dst = descs[i].dst;
             prev_end = descs[i].dst + descs[i].len;
+            prev_src_end = descs[i].src + descs[i].len;
         }
-        nt = copy_policy(payload, pairs == 0 || 2 * regular >= pairs);
+        nt = copy_policy(payload, 2 * regular >= pairs, 2 * following >= pairs);
     }
     plan->policy = nt;
-    plan->piece_policy = tuning && tuning->nontemporal ? tuning->nontemporal : copy_policy(payload, true);
+    plan->piece_policy = tuning && tuning->nontemporal ? tuning->nontemporal : copy_policy(payload, true, false);
     plan->waves = waves;
     plan->swizzle = swizzle;
     plan->max_wgs = max_wgs;
@@ -2792,16 +2801,17 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
     const bool some = !inlined && !tables && fits_inline(n, len, t, kInlineIndices); // their indices may travel as arguments
     int32_t few[2 * kInlineIndices];
     const auto is_scattered = [](const IndexFacts &dst, size_t of) { return !(of == 1 || 2 * static_cast<uint64_t>(dst.regular) >= of - 1); };
+    const auto follows = [&](const IndexFacts &src, size_t of) { return src_all_dense && 2 * static_cast<uint64_t>(src.ones) >= of - 1; };
     const auto is_sorted = [&](bool scattered, const IndexFacts &src, size_t of) {
-        return scattered && sort_pays(sort_scatter, n, len) && src_all_dense && 2 * static_cast<uint64_t>(src.ones) >= of - 1;
+        return scattered && sort_pays(sort_scatter, n, len) && follows(src, of);
     };
-    const auto new_plan = [&](bool scattered, bool sort) {
+    const auto new_plan = [&](bool scattered, bool sort, bool following) {
         auto *plan = new nixl_amd_copy_plan();
         plan->device = device;
         plan->upl = upl;
         plan->waves = waves;
         plan->swizzle = swizzle;
-        plan->policy = nt ? nt : copy_policy(n * len, !scattered || sort);
+        plan->policy = nt ? nt : copy_policy(n * len, !scattered || sort, following);
         return plan;
     };
     // More indices than an inline plan lists, but a grid.  It repeats itself, so its start says for all of it how regular it is.
@@ -2813,7 +2823,8 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         if ((sort_scatter == 1 || len >= kSortGridBlock) && sort_pays(sort_scatter, n, len) && sorted()) return false;
         auto grid = take_grid(src_runs[0], src_index, src_entries, dst_runs[0], dst_index, dst_entries, n, len);
         if (!grid) return false;
-        auto *plan = new_plan(is_scattered(facts().second, of), false);
+        const auto [src, dst] = facts();
+        auto *plan = new_plan(is_scattered(dst, of), false, follows(src, of));
         plan->inline_grid = std::move(grid);
         describe_blocks(*plan, t, n, len, n);
         *out = plan;
@@ -2858,7 +2869,7 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         std::memcpy(up_runs, src_runs, n_src_runs * sizeof(nixl_amd_copy_run_t));
         std::memcpy(up_runs + n_src_runs, dst_runs, n_dst_runs * sizeof(nixl_amd_copy_run_t));
     }
-    auto *plan = new_plan(scattered, sort);
+    auto *plan = new_plan(scattered, sort, follows(src_facts, n));
     if (inlined) {
         const auto address = [](const nixl_amd_copy_run_t *runs, size_t n_runs, uint64_t index) {
             const auto *run = std::upper_bound(runs, runs + n_runs, index, [](uint64_t i, const nixl_amd_copy_run_t &r) { return i < r.first_index; }) - 1;
@@ -3167,7 +3178,7 @@ create_listed(const nixl_amd_copy_list_t *src,
     plan->arena_bytes = kRecsAt + (n + got.extra) * sizeof(PieceRec);
     plan->piece_recs = recs;
     plan->n_pieces = static_cast<uint32_t>(n + got.extra);
-    plan->piece_policy = t.nt ? t.nt : copy_policy(got.bytes, true);
+    plan->piece_policy = t.nt ? t.nt : copy_policy(got.bytes, true, false);
     plan->info.payload_bytes = got.bytes;
     plan->info.vec_descs = n;
     plan->info.plan_device_bytes = plan->arena_bytes;

@@ -640,6 +640,53 @@ pinned_memory_is_for_byte_descriptors() {
     }
 }
 
+// Loads through the last-level cache (policy 3) or past it (4): where sources follow one another and destinations are
+// regular from 88 MiB of payload on past it, otherwise from 112.
+void
+loads_through_the_last_level_cache() {
+    Stream s;
+    const nixl_amd_copy_tuning_t tuning = tuning_for(s);
+    constexpr uint64_t kSrc = 1ull << 40, kDst = 1ull << 41, kMiB = 1 << 20;
+    const auto policy = [&](nixl_amd_copy_plan_t *plan) {
+        s.kernels.clear();
+        REQUIRE(nixl_amd_copy_plan_launch(plan, &s) == 0);
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        REQUIRE(s.kernels.size() == 1);
+        const std::string &name = s.kernels[0];
+        for (const char *kernel : {"copy_inline_kernelILi", "copy_grid_kernelILi", "copy_piece_kernelILi", "copy_uniform_kernelILi1ELi"})
+            if (const size_t at = name.find(kernel); at != std::string::npos) return name[at + std::strlen(kernel)] - '0';
+        return 0;
+    };
+    const auto of = [&](const std::vector<nixl_amd_copy_desc_t> &descs) {
+        nixl_amd_copy_plan_t *plan = nullptr;
+        REQUIRE(nixl_amd_copy_plan_create(descs.data(), descs.size(), 0, &tuning, &plan) == 0);
+        return policy(plan);
+    };
+    enum { kOne, kFollowing, kApart, kGathered, kScattered, kStrided };
+    for (const uint64_t mib : {64, 88, 92, 112, 116, 200})
+        for (const uint64_t len : {uint64_t(2048), uint64_t(16384), kMiB, kMiB + 1024})
+            for (const int shape : {kOne, kFollowing, kApart, kGathered, kScattered, kStrided}) {
+                const uint64_t n = shape == kOne ? 1 : mib * kMiB / len, each = shape == kOne ? mib * kMiB : len;
+                const auto place = [&](uint64_t i, bool any, uint64_t step) { return (any ? i * 7919 % n * 3 + i % 2 : i) * step; };
+                std::vector<nixl_amd_copy_desc_t> descs(n);
+                for (uint64_t i = 0; i < n; ++i)
+                    descs[i] = {kSrc + place(i, shape == kApart || shape == kGathered, each),
+                                kDst + place(i, shape == kApart || shape == kScattered, shape == kStrided ? 3 * each : each), each};
+                const bool past = shape <= kFollowing || shape == kStrided ? mib > 88 && (len != 2048 || shape == kOne || mib > 112) : shape == kGathered ? mib > 112 : len == 2048 && mib > 112;
+                REQUIRE(of(descs) == (past ? 4 : 3));
+                if (each % 1024 != 0 || len == 2048 || len > 16384 || shape == kOne) continue;
+                std::vector<int32_t> src(n), dst(n); // the same by index
+                for (uint64_t i = 0; i < n; ++i) {
+                    src[i] = static_cast<int32_t>((descs[i].src - kSrc) / each);
+                    dst[i] = static_cast<int32_t>((descs[i].dst - kDst) / each);
+                }
+                const nixl_amd_copy_run_t from{kSrc, each, 0, 4 * n}, to{kDst, each, 0, 4 * n};
+                nixl_amd_copy_plan_t *plan = nullptr;
+                REQUIRE(nixl_amd_copy_plan_create_indexed_lists(&from, 1, src.data(), 4 * n, &to, 1, dst.data(), 4 * n, n, each, 0, &tuning, &plan) == 0);
+                REQUIRE(policy(plan) == (past ? 4 : 3));
+            }
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -897,6 +944,7 @@ main(int argc, char **argv) {
         {"pinned_memory_is_short", pinned_memory_is_short},
         {"pinned_memory_is_asked_for_once", pinned_memory_is_asked_for_once},
         {"pinned_memory_is_for_byte_descriptors", pinned_memory_is_for_byte_descriptors},
+        {"loads_through_the_last_level_cache", loads_through_the_last_level_cache},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();
