@@ -66,7 +66,8 @@ typedef struct nixl_amd_copy_tuning {
      * stream must then outlive the plan, and while it is under capture the plan can be launched
      * on it only after nixl_amd_copy_plan_status has seen an earlier launch complete
      * (NIXL_AMD_ERR_INVALID otherwise; the capture goes on).  NULL, a busy stream or one under
-     * capture: they run on a stream of the library's. */
+     * capture: they run on a stream of the library's.  A plan by index that was made without arrays gets
+     * some when it is launched on this stream again and again, in front of one of those launches. */
     void *stream;
 } nixl_amd_copy_tuning_t;
 

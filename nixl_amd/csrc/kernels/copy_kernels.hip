@@ -725,6 +725,17 @@ index_records_kernel(UniformRec *recs, IndexVector src_index, IndexVector dst_in
     if (i < n) store_ahead(recs + i, rec);
 }
 
+// Records of a plan whose waves made their own so far (InlineIndices, GridIndices; later_records).
+template<bool SORTED, typename Recs>
+__global__ void __launch_bounds__(kIndexThreads<SORTED>)
+later_records_kernel(UniformRec *recs, Recs from, uint32_t n) {
+    const uint32_t i = blockIdx.x * kIndexThreads<SORTED> + threadIdx.x;
+    UniformRec rec{};
+    if (i < n) rec = from.at(i);
+    if constexpr (SORTED) rec = sort_window(rec, i < n);
+    if (i < n) store_ahead(recs + i, rec);
+}
+
 // The same for lists of several runs (a pool registered as several regions): index i of a
 // list lies in the run r with first[r] <= i < first[r + 1], at base[r] + (i - first[r]) *
 // stride[r].  The run tables (at most kMaxIndexRuns entries a side) are staged in LDS and
@@ -1397,6 +1408,13 @@ struct nixl_amd_copy_plan {
     std::unique_ptr<InlineRecs> inline_recs; // instead of uniform_recs: a plan of a few blocks, nothing on the device
     std::unique_ptr<InlineIndices> inline_indices; // or of some more
     std::unique_ptr<GridIndices> inline_grid; // or whose indices repeat themselves
+    // Records all the same, for its launches on the stream it was made for, from one of these on (later_records).
+    hipStream_t home = nullptr;
+    uint32_t launches_at_home = 0;
+    bool sort_later = false;
+    int later_policy = kPolNtSc1Nt;
+    void *later = nullptr;
+    size_t later_cap = 0;
     MixedArgs mixed_args{};
     uint32_t mixed_wgs = 0;
     const PieceRec *piece_recs = nullptr;
@@ -1970,6 +1988,11 @@ constexpr uint64_t kSortScatterFrom = 512ull << 20;
 // 2 KiB 347 and 281, 940 MB of 4 KiB 382 and 347, 786 MB of 8 KiB 294 and 286, 562 and 956 MB of 9 KiB 245 and 221, 376 and 355, 1180 MB of 12 KiB
 // 443 and 438, 787 MB of 14 KiB 309 and 293; of 16 KiB 629 MB 241 and 244, 839 MB 314 and 324, 1074 MB 385 and 418; 1468 MB of 32 KiB 505 and 537.
 constexpr uint64_t kSortGridBlock = 16384;
+
+// Of those that are left as they are, the ones of more than this are sorted when they get records (later_records). Up to
+// it, unsorted records are loaded ordinarily and find what is in the last-level cache: 128 MiB of 16 KiB
+// launched again and again 50.8 sorted and 45.8 not, three with pools of their own in turn 50.7 and 52.0; of 64 KiB 48.9 and 43.9, 48.9 and 49.7.
+constexpr uint64_t kSortLaterFrom = 256ull << 20;
 
 static bool
 sort_pays(int sort_scatter, size_t n, uint64_t len) {
@@ -2814,6 +2837,10 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         plan->policy = nt ? nt : copy_policy(n * len, !scattered || sort, following);
         return plan;
     };
+    const auto keep_home = [&](nixl_amd_copy_plan &plan) { // of a plan without records, which may get some
+        plan.home = t.stream == hipStreamLegacy || t.stream == hipStreamPerThread ? nullptr : t.stream;
+        plan.later_policy = nt == 0 && plan.sort_later ? copy_policy(n * len, true, true) : plan.policy;
+    };
     // More indices than an inline plan lists, but a grid.  It repeats itself, so its start says for all of it how regular it is.
     const auto grid_plan = [&](size_t of, const auto &facts) { // of the first `of` indices of both sides
         const auto sorted = [&] { // by the kernel that makes its records
@@ -2824,7 +2851,10 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
         auto grid = take_grid(src_runs[0], src_index, src_entries, dst_runs[0], dst_index, dst_entries, n, len);
         if (!grid) return false;
         const auto [src, dst] = facts();
-        auto *plan = new_plan(is_scattered(dst, of), false, follows(src, of));
+        const bool scattered = is_scattered(dst, of), following = follows(src, of);
+        auto *plan = new_plan(scattered, false, following);
+        plan->sort_later = grid->by_column && len >= kSortGridBlock && n * len > kSortLaterFrom && sort_scatter == 0 && scattered && following;
+        keep_home(*plan);
         plan->inline_grid = std::move(grid);
         describe_blocks(*plan, t, n, len, n);
         *out = plan;
@@ -2899,6 +2929,7 @@ nixl_amd_copy_plan_create_indexed_lists(const nixl_amd_copy_run_t *src_runs,
             };
             in->src = side(src_runs[0], si, src_follows);
             in->dst = side(dst_runs[0], di, dst_follows);
+            keep_home(*plan);
             plan->inline_indices = std::move(in);
             describe_blocks(*plan, t, n, len, n);
             *out = plan;
@@ -3243,6 +3274,54 @@ nixl_amd_copy_watch_stream(int device, void *stream, int own) {
     return NIXL_AMD_OK;
 }
 
+// The records of a plan that was made without any (InlineIndices, GridIndices), or null if this launch is to go without.
+// Making records costs a request that is launched once more than it gives, but one that is launched again and again
+// pays for their lack every time: a wave finds its addresses by one more division and multiplication, a launch
+// carries 3.7 KiB, and a scatter is not sorted.  Without and with, launch to end, us: 300 blocks of 8 KiB 10.4 and
+// 9.5; gathers of grids 4096 of 1 KiB 10.8 and 9.6, 8192 of 16 KiB 51.0 and 50.0, 28 672 157.4 and 155.8; scatters listed by column
+// 14 560 of 9 KiB 55.7 and 52.8, 50 944 176 and 166, 28 672 of 16 KiB 172 and 163, 32 640 196 and 182.5, 8160 of 64 KiB 181 and 172.  Hence
+// the sixteenth launch on the stream that the plan was made for makes them, in front of its copy.  Only launches on
+// that stream, which are behind their making, use them, and none into a capture, whose graph may be replayed
+// anywhere: other launches go without, as before.
+constexpr uint32_t kRecordsAt = 16;
+
+static const UniformRec *
+later_records(nixl_amd_copy_plan *plan, hipStream_t s, bool captured, bool *made) {
+    if (!s || s != plan->home || captured) return nullptr;
+    if (plan->later) return static_cast<const UniformRec *>(plan->later);
+    if (plan->launches_at_home >= kRecordsAt || ++plan->launches_at_home < kRecordsAt) return nullptr; // tried once
+    const uint32_t n = plan->n_uniform / plan->chunks_per_rec;
+    const size_t bytes = static_cast<size_t>(n) * sizeof(UniformRec);
+    // Another stream may be under a capture that allocations in any thread would end, but for those of a thread in this mode.
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+    const hipError_t had = arena_cache().get(plan->device, bytes, &plan->later, &plan->later_cap);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (had != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    auto *recs = static_cast<UniformRec *>(plan->later);
+    const auto launch = [&]<bool SORTED>(const auto &from) {
+        hipLaunchKernelGGL((later_records_kernel<SORTED, std::decay_t<decltype(from)>>), dim3((n + kIndexThreads<SORTED> - 1) / kIndexThreads<SORTED>),
+                           dim3(kIndexThreads<SORTED>), 0, s, recs, from, n);
+    };
+    if (plan->inline_indices)
+        launch.template operator()<false>(*plan->inline_indices);
+    else if (plan->sort_later)
+        launch.template operator()<true>(*plan->inline_grid);
+    else
+        launch.template operator()<false>(*plan->inline_grid);
+    if (hipGetLastError() != hipSuccess) { // nothing is queued
+        arena_cache().put(plan->device, plan->later, plan->later_cap);
+        plan->later = nullptr;
+        return nullptr;
+    }
+    plan->info.plan_device_bytes = bytes;
+    *made = true;
+    return recs;
+}
+
 static int
 launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
     if (!plan) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_launch: plan is null");
@@ -3296,7 +3375,10 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
     const bool failed = plan->watch_failure != hipSuccess;
     int slot = slots && (failed || plan->slot.load(std::memory_order_relaxed) < 0) ? slots->take(&done) : -1;
     bool told = false; // the copy writes the word itself
+    bool made = false;
+    const UniformRec *const later = later_records(plan, s, capture != hipStreamCaptureStatusNone, &made);
     const auto give_up = [&](hipError_t e) {
+        if (made) (void)hipStreamSynchronize(s); // no launch that destroying the plan would wait for is behind the records
         if (slot >= 0) slots->put(slot); // nothing that would write its word is queued
         return nixl_amd_fail(NIXL_AMD_ERR_HIP, std::string("plan_launch: ") + hipGetErrorString(e));
     };
@@ -3333,9 +3415,9 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
     };
     if (plan->inline_recs) {
         if (const hipError_t e = launch_inline(*plan->inline_recs); e != hipSuccess) return give_up(e);
-    } else if (plan->inline_indices) {
+    } else if (plan->inline_indices && !later) {
         if (const hipError_t e = launch_inline(*plan->inline_indices); e != hipSuccess) return give_up(e);
-    } else if (plan->inline_grid) {
+    } else if (plan->inline_grid && !later) {
         if (const hipError_t e = launch_inline(*plan->inline_grid); e != hipSuccess) return give_up(e);
     } else if (plan->uniform_wgs) {
         // One launch per kMaxGrid workgroups.  With the die swizzle each launch's grid is
@@ -3345,7 +3427,7 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
         for (uint64_t wg64 = 0; wg64 < plan->uniform_wgs; wg64 += kMaxGrid) {
             const uint32_t wg0 = static_cast<uint32_t>(wg64);
             UniformLaunch u{};
-            u.recs = plan->uniform_recs;
+            u.recs = later ? later : plan->uniform_recs;
             u.first_chunk = wg0 * waves;
             u.n_chunks = plan->n_uniform - u.first_chunk;
             u.n_wgs = std::min(kMaxGrid, plan->uniform_wgs - wg0);
@@ -3353,7 +3435,7 @@ launch_plan(nixl_amd_copy_plan_t *plan, void *stream, bool watched) {
             u.swizzle = plan->swizzle;
             u.grid = dim3(plan->swizzle ? ((u.n_wgs + kNumXcd - 1) / kNumXcd) * kNumXcd : u.n_wgs);
             u.stream = s;
-            with_policy(plan->policy, [&]<int POL>() { launch_uniform_upl<POL>(plan->upl, plan->waves, u); });
+            with_policy(later ? plan->later_policy : plan->policy, [&]<int POL>() { launch_uniform_upl<POL>(plan->upl, plan->waves, u); });
             if (const hipError_t e = hipGetLastError(); e != hipSuccess) return give_up(e);
         }
     }
@@ -3456,6 +3538,7 @@ nixl_amd_copy_plan_destroy(nixl_amd_copy_plan_t *plan) {
     if (plan->ev1) (void)hipEventDestroy(plan->ev1);
     give_back_staging(plan);
     if (plan->arena) arena_cache().put(plan->device, plan->arena, plan->arena_cap);
+    if (plan->later) arena_cache().put(plan->device, plan->later, plan->later_cap);
     delete plan;
     return NIXL_AMD_OK;
 }

@@ -74,6 +74,9 @@ hipError_t g_launch_status = hipSuccess; // of one launch,
 int g_good_launches = 0; // behind so many that are accepted
 int g_refused_pinned = 0; // allocations of pinned memory that fail from here on
 std::vector<size_t> g_pinned; // those asked for
+int g_refused_device = 0; // allocations of device memory that fail from here on
+bool g_only_relaxed = false; // such allocations would end another stream's capture
+thread_local hipStreamCaptureMode t_mode = hipStreamCaptureModeGlobal;
 void (*g_synchronized)(Stream &) = nullptr; // in front of a wait for a stream
 Stream *g_created = nullptr; // the last stream that the library made
 
@@ -687,6 +690,119 @@ loads_through_the_last_level_cache() {
             }
 }
 
+// A request without records that is launched again and again on the stream it was made for: the sixteenth launch makes some, in
+// front of its copy, and launches on that stream use them; others, and all where there can be none, go without.
+void
+records_for_many_launches() {
+    constexpr uintptr_t kSrc = 1ull << 40, kDst = 1ull << 41;
+    REQUIRE(nixl_amd_copy_watch_prepare() == 0);
+    const auto made = [&](size_t n, bool grid, bool scatter, uint64_t len, void *stream) {
+        std::vector<int32_t> listed(n), flat(n);
+        std::iota(flat.begin(), flat.end(), 0);
+        const size_t ids = grid ? 1000 : n;
+        for (size_t i = 0; i < n; ++i)
+            listed[i] = static_cast<int32_t>((i % ids) * (i % ids) * 31 % 65521 + i / ids * 65521); // no even steps
+        const nixl_amd_copy_run_t src{kSrc, len, 0, 1u << 30}, dst{kDst, len, 0, 1u << 30};
+        nixl_amd_copy_tuning_t tuning{};
+        tuning.stream = stream;
+        nixl_amd_copy_plan_t *plan = nullptr;
+        REQUIRE(nixl_amd_copy_plan_create_indexed_lists(&src, 1, (scatter ? flat : listed).data(), 1u << 30, &dst, 1, (scatter ? listed : flat).data(),
+                                                        1u << 30, n, len, 0, &tuning, &plan) == 0);
+        return plan;
+    };
+    const auto launch = [&](nixl_amd_copy_plan_t *plan, Stream &s, bool ok = true) { // the kernels of one launch
+        s.kernels.clear();
+        REQUIRE((nixl_amd_copy_plan_launch_watched(plan, &s) == 0) == ok);
+        REQUIRE(nixl_amd_copy_plan_status(plan, 1) == 0);
+        return s.kernels;
+    };
+    const auto has = [](const std::vector<std::string> &kernels, size_t i, const char *name) { return i < kernels.size() && kernels[i].find(name) != std::string::npos; };
+    const auto device_bytes = [](nixl_amd_copy_plan_t *plan) {
+        nixl_amd_copy_plan_info_t info{};
+        REQUIRE(nixl_amd_copy_plan_query(plan, &info) == 0);
+        return info.plan_device_bytes;
+    };
+    struct Case {
+        size_t n;
+        bool grid, scatter;
+        uint64_t len;
+        const char *records; // kernel
+        char policy; // of the copy from then on
+    };
+    for (const Case &c : {Case{600, false, false, 8192, "ILb0ENS_13InlineIndicesE", '3'}, {2000, true, false, 1024, "ILb0ENS_11GridIndicesE", '3'},
+                          {16000, true, true, 16384, "ILb0ENS_11GridIndicesE", '3'}, {17000, true, true, 16384, "ILb1ENS_11GridIndicesE", '4'},
+                          {32000, true, true, 15360, "ILb0ENS_11GridIndicesE", '3'}, {17000, true, false, 16384, "ILb0ENS_11GridIndicesE", '4'}}) {
+        Stream home, other;
+        nixl_amd_copy_plan_t *plan = made(c.n, c.grid, c.scatter, c.len, &home);
+        REQUIRE(device_bytes(plan) == 0);
+        const auto without = [&](const std::vector<std::string> &kernels) { return has(kernels, 0, c.grid ? "GridIndices" : "InlineIndices") && !has(kernels, 0, "later_records"); };
+        for (int i = 1; i <= 15; ++i) {
+            REQUIRE(without(launch(plan, home)));
+            REQUIRE(without(launch(plan, other)));
+        }
+        REQUIRE(without(launch(plan, other)) && device_bytes(plan) == 0);
+        g_only_relaxed = true;
+        auto kernels = launch(plan, home);
+        g_only_relaxed = false;
+        const auto with = [&](size_t at) { return has(kernels, at, "copy_uniform_kernelILi1E") && has(kernels, at, (std::string("ILi1ELi") + c.policy + "E").c_str()); };
+        REQUIRE(has(kernels, 0, "later_records_kernel") && has(kernels, 0, c.records) && with(1));
+        REQUIRE(device_bytes(plan) == c.n * 16);
+        for (int i = 0; i < 20; ++i) {
+            kernels = launch(plan, home);
+            REQUIRE(with(0));
+            REQUIRE(without(launch(plan, other)));
+        }
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        // no memory, or no launch of the kernel that makes them: not tried again
+        for (const bool memory : {true, false}) {
+            plan = made(c.n, c.grid, c.scatter, c.len, &home);
+            for (int i = 0; i < 15; ++i)
+                (void)launch(plan, home);
+            std::vector<nixl_amd_copy_plan_t *> takers; // of the memory that plans gave back
+            if (memory)
+                for (int i = 0; i < 4; ++i) {
+                    takers.push_back(made(c.n, c.grid, c.scatter, c.len, &other));
+                    for (int j = 0; j < 16; ++j)
+                        (void)launch(takers.back(), other);
+                }
+            if (memory)
+                g_refused_device = 1;
+            else
+                g_launch_status = hipErrorOutOfMemory, g_good_launches = 0;
+            REQUIRE(without(launch(plan, home)) && device_bytes(plan) == 0);
+            REQUIRE(g_refused_device == 0 && g_launch_status == hipSuccess && hipGetLastError() == hipSuccess);
+            for (int i = 0; i < 40; ++i)
+                REQUIRE(without(launch(plan, home)));
+            for (nixl_amd_copy_plan_t *taker : takers)
+                REQUIRE(nixl_amd_copy_plan_destroy(taker) == 0);
+            REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        }
+        // the copy behind them fails: nothing of theirs runs when the plan may be destroyed
+        plan = made(c.n, c.grid, c.scatter, c.len, &home);
+        for (int i = 0; i < 15; ++i)
+            (void)launch(plan, home);
+        home.waited_for = false;
+        g_launch_status = hipErrorOutOfMemory;
+        g_good_launches = 1;
+        home.held = true;
+        REQUIRE(nixl_amd_copy_plan_launch_watched(plan, &home) == NIXL_AMD_ERR_HIP);
+        REQUIRE(home.waited_for && home.work.empty());
+        kernels = launch(plan, home);
+        REQUIRE(with(0));
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        // made for no stream, or for one that is not the same in every thread
+        for (void *stream : {static_cast<void *>(nullptr), static_cast<void *>(hipStreamPerThread), static_cast<void *>(hipStreamLegacy)}) {
+            plan = made(c.n, c.grid, c.scatter, c.len, stream);
+            for (int i = 0; i < 40; ++i) {
+                REQUIRE(nixl_amd_copy_plan_launch(plan, stream) == 0);
+                REQUIRE(without(launch(plan, home)));
+            }
+            REQUIRE(device_bytes(plan) == 0);
+            REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
+        }
+    }
+}
+
 } // namespace
 
 // ---- the runtime ------------------------------------------------------------------------------
@@ -797,7 +913,19 @@ hipGetErrorString(hipError_t) {
 }
 
 hipError_t
+hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *mode) {
+    std::swap(*mode, t_mode);
+    return hipSuccess;
+}
+
+hipError_t
 hipMalloc(void **p, size_t n) {
+    LOCKED;
+    REQUIRE(!g_only_relaxed || t_mode == hipStreamCaptureModeRelaxed);
+    if (g_refused_device > 0) {
+        --g_refused_device;
+        return g_last_status = hipErrorOutOfMemory;
+    }
     *p = std::aligned_alloc(4096, (n + 4095) / 4096 * 4096);
     std::memset(*p, 0xa5, n); // nobody may count on zeroes
     return hipSuccess;
@@ -945,6 +1073,7 @@ main(int argc, char **argv) {
         {"pinned_memory_is_asked_for_once", pinned_memory_is_asked_for_once},
         {"pinned_memory_is_for_byte_descriptors", pinned_memory_is_for_byte_descriptors},
         {"loads_through_the_last_level_cache", loads_through_the_last_level_cache},
+        {"records_for_many_launches", records_for_many_launches},
     };
     REQUIRE(argc == 2 && scenarios.count(argv[1]));
     scenarios.at(argv[1])();

@@ -365,7 +365,8 @@ def test_helper_threads_of_the_hip_backend_on_the_cpu():
                                       "launch_on_the_stream_of_a_thread", "launch_seen_by_two_threads",
                                       "refused_launches_keep_no_totals", "many_requests_wait_for_verdicts", "indices_that_repeat_themselves",
                                       "pinned_memory_is_short", "pinned_memory_is_asked_for_once",
-                                      "pinned_memory_is_for_byte_descriptors", "loads_through_the_last_level_cache"])
+                                      "pinned_memory_is_for_byte_descriptors", "loads_through_the_last_level_cache",
+                                      "records_for_many_launches"])
 def test_host_side_of_copy_plans_on_the_cpu(scenario):
     """tests/cpp/copy_host_check.cpp: what a copy plan asks of the runtime and answers its caller,
     with a runtime that the program brings itself."""

@@ -660,6 +660,94 @@ def test_requests_whose_indices_repeat_themselves(cuda, n_ids, others, chunks, p
     assert lib.nixl_amd_copy_plan_destroy(plan) == 0
 
 
+@pytest.mark.parametrize("n_ids, others, listed, scatter, by_column, kib", [
+    (600, 1, "some", False, True, 8), (897, 3, "grid", False, True, 1), (250, 61, "grid", True, True, 9), (130, 17, "grid", False, False, 16),
+    (300, 65, "grid", True, True, 16)])
+def test_requests_without_records_that_are_launched_again_and_again(cuda, n_ids, others, listed, scatter, by_column, kib):
+    """The sixteenth launch on the stream of a request makes its records (the last form's sorted), here while another stream is
+    under capture.  The launches before it, that one and those behind it move the same bytes, on that stream, on another
+    one, and from graphs captured before and after it."""
+    import torch
+    lib = _lib.kernels()
+    assert lib.nixl_amd_copy_watch_prepare() == 0
+    rng = np.random.default_rng(n_ids)
+    n, blk, pool = n_ids * others, 1024 * kib, n_ids + 37
+    entries = pool * others
+    ids = rng.permutation(pool)[:n_ids]
+    at = np.arange(others)[:, None] * pool + ids[None, :]
+    v = np.ascontiguousarray((at if by_column else at.T).reshape(-1), dtype=np.int32)
+    flat = np.arange(n, dtype=np.int32)
+    si, di = (flat, v) if scatter else (v, flat)
+    src = torch.randint(0, 256, ((n if scatter else entries), blk), dtype=torch.uint8, device=cuda)
+    dst = torch.zeros(((entries if scatter else n), blk), dtype=torch.uint8, device=cuda)
+    index = torch.from_numpy(v.astype(np.int64)).to(cuda)
+    run = lambda t: (_lib.CopyRun * 1)(_lib.CopyRun(t.data_ptr(), blk, 0, t.shape[0]))  # noqa: E731
+    home, other, captured = (torch.cuda.Stream() for _ in range(3))
+    tuning, plan = _lib.CopyTuning(), ctypes.c_void_p()
+    tuning.stream = home.cuda_stream
+    assert lib.nixl_amd_copy_plan_create_indexed_runs(run(src), 1, si.ctypes.data, run(dst), 1, di.ctypes.data, n, blk, 0, ctypes.byref(tuning),
+                                                      ctypes.byref(plan)) == 0, _lib.kernels_error()
+
+    def device_bytes():
+        info = _lib.CopyPlanInfo()
+        assert lib.nixl_amd_copy_plan_query(plan, ctypes.byref(info)) == 0
+        return info.plan_device_bytes
+
+    def check(what):
+        torch.cuda.synchronize()
+        want = torch.zeros_like(dst)
+        if scatter:
+            want[index] = src
+        else:
+            want.copy_(src[index])
+        assert torch.equal(dst, want), what
+        src.add_(1)
+        dst.zero_()
+        torch.cuda.synchronize()
+
+    def launch(stream):
+        assert lib.nixl_amd_copy_plan_launch_watched(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+        assert lib.nixl_amd_copy_plan_status(plan, 1) == 0
+
+    def graph_of(stream):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            assert lib.nixl_amd_copy_plan_launch(plan, stream.cuda_stream) == 0, _lib.kernels_error()
+        return graph
+
+    torch.cuda.synchronize()
+    launch(home)
+    check("first")
+    before = graph_of(home)
+    for _ in range(14):
+        launch(home)
+    check("before records")
+    assert device_bytes() == 0
+    x = torch.ones(1000, device=cuda)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=captured):
+        y = x + 1
+        assert lib.nixl_amd_copy_plan_launch_watched(plan, home.cuda_stream) == 0, _lib.kernels_error()
+        y += x
+    assert lib.nixl_amd_copy_plan_status(plan, 1) == 0
+    assert device_bytes() == 16 * n
+    check("the launch that makes them")
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, torch.full_like(y, 3))
+    after = graph_of(home)
+    for i in range(3):
+        launch(home)
+        check(f"with records {i}")
+        launch(other)
+        check(f"elsewhere {i}")
+        for name, g in (("before", before), ("after", after)):
+            g.replay()
+            check(f"graph {name} {i}")
+    assert lib.nixl_amd_copy_plan_destroy(plan) == 0
+
+
 def test_run_tables_through_the_kernel_library(cuda):
     """nixl_amd_copy_plan_create_indexed_runs called directly: three source runs with
     different strides, two destination runs, 5000 random blocks (more than one bisection
