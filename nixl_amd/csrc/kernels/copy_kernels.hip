@@ -185,7 +185,8 @@ store16_part(uint64_t addr, const v4u &v) {
 // Stores 16 bytes that the kernel behind this one reads, through the die's cache as it goes: what a
 // kernel leaves in there is written back when it ends, in front of the next one's start.  Requests of
 // 1280, 4096 and 3904 blocks by index, launch to end: 18.6 -> 18.3 us, 26.0 -> 25.6 and 26.9 -> 26.4.  Non-temporal
-// stores send the records to memory and the next kernel there for them: 19.0, 26.4 and 27.1.
+// stores send the records to memory and the next kernel there for them: 19.0, 26.4 and 27.1.  (The kernel that uploads the
+// 108 KB of items of 3000 byte descriptors takes 4.8 either way.)
 template<class T>
 __device__ __forceinline__ void
 store_ahead(T *at, const T &x) {
@@ -725,7 +726,8 @@ index_records_kernel(UniformRec *recs, IndexVector src_index, IndexVector dst_in
     if (i < n) store_ahead(recs + i, rec);
 }
 
-// Records of a plan whose waves made their own so far (InlineIndices, GridIndices; later_records).
+// Records of a plan whose waves made their own so far (InlineIndices, GridIndices; later_records).  A launch and its chain of
+// loads: 300 listed blocks 2.2 us, a grid of 4096 2.8, of 131 072 3.1; sorted 32 640 8.6.
 template<bool SORTED, typename Recs>
 __global__ void __launch_bounds__(kIndexThreads<SORTED>)
 later_records_kernel(UniformRec *recs, Recs from, uint32_t n) {
@@ -794,11 +796,11 @@ index_records_runs_kernel(UniformRec *recs, IndexVector src_index, IndexVector d
 //
 // The verdict reaches the host through pinned memory, written by the workgroup that finishes last;
 // the host waits for it, because a bad pair must fail the request.  A workgroup adds to the totals
-// with two atomics, on two lines (an addition to a line takes 11 ns behind another one, and there are 256 workgroups in
-// 262 144 pairs: 13.8 us with one line, 11.2 with two), and nothing in front of the verdict writes a cache back: a
-// device-scope fence around the additions did, for records that only the next kernel reads.  Kernel time, with such
-// fences, sums over a wave through LDS and one line, and now: runs of 64 pairs, 1024 pairs 8.0 and 6.4 us, 16 384 9.9 and
-// 8.1, 65 536 10.9 and 8.7, 262 144 15.5 and 11.2; vectors, 1024 pairs 6.8 and 5.3, 65 536 19.2 and 18.1.
+// with two atomics, on two lines, and nothing in front of the verdict writes a cache back: a device-scope fence around the
+// additions did, for records that only the next kernel reads.  Kernel time, medians under the profiler, with such fences,
+// sums over a wave through LDS and one line; without them and with sums between lanes; and with two lines: runs of 64 pairs, 1024 pairs 9.3, 8.0 and
+// 8.0 us, 16 384 9.6, 8.4 and 8.4, 65 536 10.3, 8.8 and 8.7, 262 144 13.8, 10.4 and 9.9; vectors, 1024 pairs 9.4, 8.6 and 8.4, 16 384 11.4,
+// 10.2 and 10.3, 65 536 18.5, 17.1 and 17.4.
 struct IndexRun {
     uint32_t first; // pair the run starts with; it ends where the next one starts
     uint32_t src, dst; // indices of that pair
@@ -1739,11 +1741,13 @@ is_grid(const uint32_t *v, size_t n, uint32_t length, bool by_column, uint32_t s
     return between == 0;
 }
 
-// A grid listed by row has rows of at least kMinGridRow, which are looked at one by one, and is left to records of its own
-// where these are faster. Blocks that are neighbours in their list, us with records and as a grid: 12 288 of 8 KiB in rows of 16
-// 43.9 and 39.8, 14 336 48.0 and 49.5, 16 384 55.5 and 57.1 (of 4 KiB 32.3 and 33.5), 32 768 in rows of 32 97.4 and 99.7. Others: a
-// GiB in rows of 1092 of 16 KiB 364 and 357, of 546 of 32 KiB 353 and 357, of 273 of 64 KiB 334 and 340, of 136 of 128 KiB 322 and 330;
-// half a GiB of 64 KiB 171.5 and 171.4, of 128 KiB 168.4 and 168.7, of 256 KiB 169.7 and 167.9.
+// A grid listed by row has rows of at least kMinGridRow, which are looked at one by one.  Rows that are neighbours in their list have
+// records of their own beyond kMaxConsecutive blocks, and blocks larger than kMaxRowBlock beyond kMaxRowBytes.  These lines were drawn
+// where records had been measured faster, and that did not hold: passes of gathers through an agent, with records and as a grid on
+// either side of the lines, us: 14 336 neighbours of 8 KiB in rows of 16 53.3 and 49.2, 16 384 59.5 and 55.1, 32 768 of 2 KiB in rows of 32 41.2 and
+// 34.4, 16 384 of 16 KiB 98.5 and 94.8, rows in ascending order 59.2 and 59.2; scatters 54.9 and 50.8, 60.0 and 55.1, 41.8 and 35.2, 98.3 and 94.4;
+// blocks of 24 KiB, 600 MiB, 216.6 and 212.5, of 32 KiB, 640 MiB, 229.9 and 225.8, 1024 MiB 355.7 and 354.4, of 64 KiB, 800 MiB, 278.2 and 276.0, of 256 KiB, 960 MiB,
+// 312.6 and 311.7.  Neither blocks nor bytes nor rows decide: nowhere are records faster by more than runs differ.
 constexpr size_t kMinGridRow = 8, kMaxConsecutive = 12288;
 constexpr uint64_t kMaxRowBlock = 16384, kMaxRowBytes = 512ull << 20;
 
