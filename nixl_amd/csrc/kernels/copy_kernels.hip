@@ -1417,6 +1417,7 @@ struct nixl_amd_copy_plan {
     int later_policy = kPolNtSc1Nt;
     void *later = nullptr;
     size_t later_cap = 0;
+    std::atomic<size_t> later_bytes{0}; // in use: the plan may be queried from any thread
     MixedArgs mixed_args{};
     uint32_t mixed_wgs = 0;
     const PieceRec *piece_recs = nullptr;
@@ -3321,7 +3322,7 @@ later_records(nixl_amd_copy_plan *plan, hipStream_t s, bool captured, bool *made
         plan->later = nullptr;
         return nullptr;
     }
-    plan->info.plan_device_bytes = bytes;
+    plan->later_bytes.store(bytes, std::memory_order_relaxed);
     *made = true;
     return recs;
 }
@@ -3551,6 +3552,7 @@ int
 nixl_amd_copy_plan_query(const nixl_amd_copy_plan_t *plan, nixl_amd_copy_plan_info_t *info) {
     if (!plan || !info) return nixl_amd_fail(NIXL_AMD_ERR_INVALID, "plan_query: null argument");
     *info = plan->info;
+    info->plan_device_bytes += plan->later_bytes.load(std::memory_order_relaxed);
     return NIXL_AMD_OK;
 }
 
