@@ -3317,7 +3317,8 @@ later_records(nixl_amd_copy_plan *plan, hipStream_t s, bool captured, bool *made
         launch.template operator()<true>(*plan->inline_grid);
     else
         launch.template operator()<false>(*plan->inline_grid);
-    if (hipGetLastError() != hipSuccess) { // nothing is queued
+    if (hipGetLastError() != hipSuccess) {
+        (void)hipStreamSynchronize(s); // unless the error is an earlier one's, and they are being made
         arena_cache().put(plan->device, plan->later, plan->later_cap);
         plan->later = nullptr;
         return nullptr;

@@ -777,6 +777,21 @@ records_for_many_launches() {
                 REQUIRE(nixl_amd_copy_plan_destroy(taker) == 0);
             REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
         }
+        // an error that somebody else left behind is taken for theirs: they are waited for before their memory goes back
+        plan = made(c.n, c.grid, c.scatter, c.len, &home);
+        for (int i = 0; i < 15; ++i)
+            (void)launch(plan, home);
+        g_refused_device = 1;
+        void *none = nullptr;
+        REQUIRE(hipMalloc(&none, 1) != hipSuccess);
+        home.waited_for = false;
+        home.held = true;
+        home.kernels.clear();
+        REQUIRE(nixl_amd_copy_plan_launch_watched(plan, &home) == 0);
+        REQUIRE(has(home.kernels, 0, "later_records_kernel") && home.waited_for);
+        REQUIRE(nixl_amd_copy_plan_status(plan, 1) == 0);
+        REQUIRE(without(launch(plan, home)) && device_bytes(plan) == 0);
+        REQUIRE(nixl_amd_copy_plan_destroy(plan) == 0);
         // the copy behind them fails: nothing of theirs runs when the plan may be destroyed
         plan = made(c.n, c.grid, c.scatter, c.len, &home);
         for (int i = 0; i < 15; ++i)
@@ -861,9 +876,8 @@ static thread_local hipError_t g_last_status = hipSuccess;
 hipError_t
 hipLaunchKernel(const void *stub, dim3 grid, dim3, void **args, size_t, hipStream_t stream) {
     LOCKED;
-    g_last_status = g_launch_status != hipSuccess && g_good_launches-- <= 0 ? g_launch_status : hipSuccess;
-    if (g_last_status != hipSuccess) {
-        g_launch_status = hipSuccess; // once
+    if (g_launch_status != hipSuccess && g_good_launches-- <= 0) {
+        g_last_status = std::exchange(g_launch_status, hipSuccess); // once
         return g_last_status;
     }
     const std::string &name = kernel_names().at(stub);
